@@ -76,7 +76,7 @@ def build() -> str:
     """Compile the library in-tree with the Makefile beside the sources (cross-compiles without a GPU)."""
     import subprocess
 
-    subprocess.run(["make", "-C", _CSRC, "-B", "-j8", "libmi355_qlinear.so"], check=True)
+    subprocess.run(["make", "-C", _CSRC, "-B", "-j8", "all"], check=True)
     return LIB_PATH
 
 

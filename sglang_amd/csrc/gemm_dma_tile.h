@@ -1,0 +1,394 @@
+// The mid-M tile of the FP8 and INT8 GEMMs for gfx950: (64 or 128) tokens x (256, 192 or 128) channels, 8 waves (two per
+// SIMD), S LDS stages filled by direct-to-LDS loads, operand fragments read one K block AHEAD of their multiplication.
+//
+// What bounds a short tile is the chain of one K block: after the block's barrier every wave reads its operand fragments
+// from LDS (96-128 KB over the workgroup, ~450 cycles at the LDS's rate) and only then multiplies them (256-512 cycles of
+// matrix pipe per SIMD); with eight waves in lockstep the two never overlap.  Here a wave holds two sets of fragments: while
+// it multiplies block k out of one, it reads block k + 1 from LDS into the other, so the LDS and the matrix pipe work at the
+// same time inside every wave and nothing but the barrier itself separates two blocks' multiplications.  The stage that
+// held block k is free as soon as its fragments are in registers, so S stages keep S - 1 blocks in flight from memory as
+// before.  Registers: 64 accumulators + 2 x 64 fragments for 128 x 256 (INT8 and FP8 alike), two waves per SIMD.
+//
+// Instructions written by hand, because the compiler's own waits cover every load it knows about:
+//   * per block every wave issues exactly LOADS loads (tile rows plus, where the K loop applies scales, the token scales),
+//     so "block k + 1 has landed" is the constant s_waitcnt vmcnt((S - 2) * LOADS) until the last S blocks, which issue
+//     nothing and count down;
+//   * s_waitcnt lgkmcnt(0) in front of the barrier: the fragments of block k have left its stage;
+//   * nothing else in the loop counts in vmcnt (weight-block scales come by scalar loads).
+// Requires K % 128 == 0, 16-byte aligned rows and row offsets below 4 GiB; AR_F32 / AR_UE8M0 also token scales laid out
+// M-major with a pitch that is a multiple of four words.
+#pragma once
+
+#include "gemm_common.h"
+
+namespace mi355 {
+namespace {
+
+// What the K loop does with a product block.
+enum Arith {
+  AR_F32,    // FP8, fp32 scales: acc += product * (token scale * weight-block scale)
+  AR_UE8M0,  // FP8, packed exponents on both operands: the MFMA applies them and accumulates in place
+  AR_UNIT,   // FP8, no scales in the loop: accumulates in place; one scale per token and channel in the epilogue
+  AR_INT8,   // INT8: accumulates in place (int32); scales and bias in the epilogue
+};
+
+constexpr int T_THREADS = 512;
+
+typedef __attribute__((address_space(3))) void* lptr_t;
+typedef const __attribute__((address_space(3))) uint8_t* lds_cptr;
+typedef const __attribute__((address_space(4))) float* cfloat_ptr;
+
+struct Frag {
+  u32x4 lo, hi;
+};
+__device__ __forceinline__ v8i as_v8i(const Frag& f) {
+  return v8i{(int)f.lo.x, (int)f.lo.y, (int)f.lo.z, (int)f.lo.w, (int)f.hi.x, (int)f.hi.y, (int)f.hi.z, (int)f.hi.w};
+}
+__device__ __forceinline__ v4i as_v4i(const u32x4& x) { return v4i{(int)x.x, (int)x.y, (int)x.z, (int)x.w}; }
+__device__ __forceinline__ u32x4 lds16(lds_cptr p, int imm) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(p + imm);
+}
+__device__ __forceinline__ float lds_f32(lds_cptr p, int imm) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) float*>(p + imm);
+}
+
+template <Arith AR, int BM, int BN>
+struct TileShape {
+  static_assert((BM == 64 || BM == 128) && (BN == 128 || BN == 192 || BN == 256), "tile");
+  static constexpr bool SCALED = AR == AR_F32 || AR == AR_UE8M0;
+  static constexpr int MT = BM / 32, NT = BN / 64, STEPS = MT * NT;   // a wave owns BM / 2 tokens x BN / 4 channels
+  static constexpr int ROW_LOADS = (BM + BN) / 64;                    // a wave fills 8 rows per load
+  static constexpr int LOADS = ROW_LOADS + (SCALED ? 1 : 0);
+  // A wave's channels are BN / 4 consecutive ones inside one 128-channel scale block, except for BN = 192, where 48
+  // consecutive channels could straddle two blocks: there the wave's channel tile i is channels 64 i + 16 wave .. + 15, so that
+  // tile i of every wave lies in the block of channel n0 + 64 i.
+  static constexpr bool INTERLEAVED = BN == 192;
+  static constexpr int SB = INTERLEAVED ? NT : 1;
+  static constexpr int W_STRIDE = INTERLEAVED ? 64 * 128 : 16 * 128;  // bytes between a wave's consecutive channel tiles in a stage
+  static constexpr int STAGE_BYTES = (BM + BN) * KSTEP;
+  static_assert(LOADS <= STEPS, "one load per step");
+  __device__ static int channel(int wave_n, int i) { return INTERLEAVED ? i * 64 + wave_n * 16 : wave_n * (BN / 4) + i * 16; }
+};
+
+// One BM x BN output tile at (m0, n0), K blocks of split `split`, by the whole workgroup.
+// AR_UE8M0: p.sa / p.sb point to packed exponent words: token word (m, kw) at sa[kw * sa_sk + m], channel word (n, kw) at
+// sb[kw * sb_sk + n * sb_sn], byte kb & 3 of word kb >> 2 belongs to K block kb.
+template <Arith AR, int BM, int BN, bool SPLIT, int S>
+__device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, int split) {
+  using T = TileShape<AR, BM, BN>;
+  static_assert(S >= 3 && S * (T::STAGE_BYTES + BM * 4) <= 160 * 1024, "the stages must fit the CU's LDS");
+  constexpr int MT = T::MT, NT = T::NT, SB = T::SB, LOADS = T::LOADS, WM = BM / 2;
+  using AccT = typename std::conditional<AR == AR_INT8, int, float>::type;
+  typedef AccT acc4 __attribute__((ext_vector_type(4)));
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_m = wave >> 2, wave_n = wave & 3;
+  const int l16 = lane & 15, q = lane >> 4;
+  const int kb_begin = split * p.kb_per_split;
+  const int nkb = min(p.kb_total, kb_begin + p.kb_per_split) - kb_begin;
+  const int kb_last = kb_begin + nkb - 1;
+
+  // the stages: tile rows (0..BM-1 tokens, then channels) and the tile's BM token scales
+  __shared__ __attribute__((aligned(1024))) uint8_t t_stage[S * T::STAGE_BYTES];
+  __shared__ __attribute__((aligned(256))) float t_scale[S * BM];
+
+  // ---- loader: lane's byte offset from the matrix base for each of its rows (rows clamped); lands swizzled by (row & 7)
+  uint32_t goff[T::ROW_LOADS];
+  {
+    const int lrow = lane >> 3;
+    const int chunk_byte = ((lane & 7) ^ lrow) * 16;
+#pragma unroll
+    for (int i = 0; i < T::ROW_LOADS; ++i) {
+      const int row = i * 64 + wave * 8 + lrow;
+      goff[i] = row < BM ? (uint32_t)((int64_t)min(m0 + row, p.M - 1) * p.lda + chunk_byte)
+                         : (uint32_t)((int64_t)min(n0 + row - BM, p.N - 1) * p.ldb + chunk_byte);
+    }
+  }
+  // every wave fetches BM / 8 token scales per K block, four per lane; quads past M refetch the last valid one
+  const uint32_t sa_off = (uint32_t)min(m0 + wave * (BM / 8) + (lane & (BM / 32 - 1)) * 4, (p.M - 1) & ~3) * 4u;
+  // Load number i of K block kb (< ROW_LOADS: tile rows; then the token scales) into stage `st`.  The statements write m0; it
+  // cannot be listed as a clobber (the compiler reserves the register), and no compiler-managed use of m0 lies between them
+  // and the next statement that sets it.
+  auto issue = [&](int i, int st, int kb) {
+    kb = min(kb, kb_last);
+    if (i < T::ROW_LOADS) {
+      const uint8_t* base = (i < BM / 64 ? p.a : p.b) + (uint64_t)kb * KSTEP;  // wave-uniform
+      asm volatile("" : "+s"(base));
+      const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_stage + (uint32_t)(st * T::STAGE_BYTES + (i * 64 + wave * 8) * KSTEP);
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
+    } else if constexpr (T::SCALED) {
+      // BM / 32 lanes fetch 16 bytes each (a 4-byte-per-lane load in this stream costs far more than its size).  exec is
+      // narrowed and restored inside the statement.  Packed exponents: one row of words per four K blocks, fetched again for
+      // each of the four (the load count per K block stays constant).
+      const float* sbase = p.sa + (int64_t)(AR == AR_UE8M0 ? kb >> 2 : kb) * p.sa_sk;  // wave-uniform
+      asm volatile("" : "+s"(sbase));
+      const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_scale + (uint32_t)(st * BM + wave * (BM / 8)) * 4u;
+      uint64_t saved;
+      if constexpr (BM == 128)
+        asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, 0xf\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, %0"
+                     : "=&s"(saved) : "v"(sa_off), "s"(sbase), "s"(lds_addr) : "memory");
+      else
+        asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, 0x3\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, %0"
+                     : "=&s"(saved) : "v"(sa_off), "s"(sbase), "s"(lds_addr) : "memory");
+    }
+  };
+
+  // ---- fragment addresses inside a stage.  Lane quarter q takes the 16-byte chunks q and q + 4 of a row (full LDS rate).
+  uint32_t tok_off[2], ch_off[2];
+  {
+    const int trow = wave_m * WM + l16, crow = BM + T::channel(wave_n, 0) + l16;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      tok_off[h] = trow * KSTEP + (((q + 4 * h) ^ (trow & 7)) << 4);
+      ch_off[h] = crow * KSTEP + (((q + 4 * h) ^ (crow & 7)) << 4);
+    }
+  }
+  const uint32_t sc_off = (wave_m * WM + l16) * 4;
+  cfloat_ptr sb_ptr[SB];  // the wave's (channel tile's) row of weight-block scales
+  if constexpr (T::SCALED) {
+#pragma unroll
+    for (int b = 0; b < SB; ++b) {
+      const int first = min(n0 + T::channel(wave_n, b), p.N - 1);
+      sb_ptr[b] = (cfloat_ptr)(p.sb + (int64_t)__builtin_amdgcn_readfirstlane(AR == AR_UE8M0 ? first : first / 128) * p.sb_sn);
+    }
+  }
+  float sbv[SB];  // scales (words) of the block to be multiplied next
+  auto load_sb = [&](int kb) {
+    if constexpr (T::SCALED) {
+      kb = min(kb, kb_last);
+#pragma unroll
+      for (int b = 0; b < SB; ++b) sbv[b] = sb_ptr[b][(int64_t)(AR == AR_UE8M0 ? kb >> 2 : kb) * p.sb_sk];
+    }
+  };
+
+  acc4 acc[NT][MT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = acc4{0, 0, 0, 0};
+
+  // two sets of fragments and token scales
+  Frag w[2][NT], tok[2][MT];
+  float tsc[2][MT];
+  constexpr int READS = 2 * (NT + MT);
+  // read number r of a block out of stage `st` into set `set`: token tile 0, the channel tiles, the other token tiles
+  auto read = [&](int r, int set, lds_cptr st, lds_cptr sc) {
+    const int f = r >> 1, h = r & 1;
+    if (f >= 1 && f <= NT) {
+      const u32x4 v = lds16(st + ch_off[h], (f - 1) * T::W_STRIDE);
+      if (h == 0) w[set][f - 1].lo = v;
+      else w[set][f - 1].hi = v;
+    } else {
+      const int j = f == 0 ? 0 : f - NT;
+      const u32x4 v = lds16(st + tok_off[h], j * 2048);
+      if (h == 0) tok[set][j].lo = v;
+      else tok[set][j].hi = v;
+      if (T::SCALED && h == 1) tsc[set][j] = lds_f32(sc + sc_off, j * 64);
+    }
+  };
+  auto stage_at = [&](int st) { return (lds_cptr)t_stage + st * T::STAGE_BYTES; };
+  auto scales_at = [&](int st) { return (lds_cptr) reinterpret_cast<uint8_t*>(t_scale) + st * BM * 4; };
+
+  v4f pend = v4f{0.f, 0.f, 0.f, 0.f};  // AR_F32: the product of the previous step, whose promotion runs behind this step's MFMA
+  float pend_scale = 0.f;
+
+  // Multiplies block k out of set CUR while reading block k + 1 (in stage st_next) into the other set and, with FILL, issuing
+  // block k + S into st_fill, the stage block k has just left.
+  auto block = [&](auto cur_c, auto fill_c, int k, int st_next, int st_fill) {
+    constexpr int CUR = decltype(cur_c)::value, NXT = 1 - CUR;
+    constexpr bool FILL = decltype(fill_c)::value;
+    const int kb = kb_begin + k;
+    const lds_cptr nst = stage_at(st_next), nsc = scales_at(st_next);
+    float sc[MT][SB];
+    int w_exp[SB];
+    if constexpr (AR == AR_F32) {
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int b = 0; b < SB; ++b) sc[j][b] = tsc[CUR][j] * sbv[b];
+    } else if constexpr (AR == AR_UE8M0) {
+      const int shift = (kb & 3) * 8;
+#pragma unroll
+      for (int b = 0; b < SB; ++b) w_exp[b] = in_vgpr((int)(__float_as_uint(sbv[b]) >> shift));
+#pragma unroll
+      for (int j = 0; j < MT; ++j) sc[j][0] = __uint_as_float(__float_as_uint(tsc[CUR][j]) >> shift);
+    }
+    load_sb(kb + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // the reads go out over the first three quarters of the steps, so that the last ones have returned at the barrier
+    constexpr int PER = (READS * 4 + T::STEPS * 3 - 1) / (T::STEPS * 3);
+    v4f part[2];
+#pragma unroll
+    for (int t = 0; t < T::STEPS; ++t) {
+      const int j = t / NT, i = t % NT;
+      if constexpr (AR == AR_F32) {
+        part[t & 1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(w[CUR][i]), as_v8i(tok[CUR][j]), v4f{0.f, 0.f, 0.f, 0.f},
+                                                                       0, 0, 0, 0, 0, 0);
+      } else if constexpr (AR == AR_UE8M0) {
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(w[CUR][i]), as_v8i(tok[CUR][j]), acc[i][j], 0, 0, 0,
+                                                                     w_exp[SB > 1 ? i : 0], 0, (int)__float_as_uint(sc[j][0]));
+      } else if constexpr (AR == AR_UNIT) {
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(w[CUR][i]), as_v8i(tok[CUR][j]), acc[i][j], 0, 0, 0, 0, 0, 0);
+      } else {
+        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(as_v4i(w[CUR][i].lo), as_v4i(tok[CUR][j].lo), acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(as_v4i(w[CUR][i].hi), as_v4i(tok[CUR][j].hi), acc[i][j], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the MFMA goes first; the rest of the step runs in its shadow
+#pragma unroll
+      for (int r = t * PER; r < (t + 1) * PER; ++r)
+        if (r < READS) read(r, NXT, nst, nsc);
+      if (FILL && t < LOADS) issue(t, st_fill, kb + S);
+      if constexpr (AR == AR_F32) {
+        if (t == 0) {  // the last product of the previous block
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[NT - 1][MT - 1][v] = fmaf(pend[v], pend_scale, acc[NT - 1][MT - 1][v]);
+        } else {
+          const int pj = (t - 1) / NT, pi = (t - 1) % NT;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[pi][pj][v] = fmaf(part[(t - 1) & 1][v], sc[pj][SB > 1 ? pi : 0], acc[pi][pj][v]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (AR == AR_F32) pend = part[(T::STEPS - 1) & 1], pend_scale = sc[MT - 1][SB > 1 ? NT - 1 : 0];
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  // everything but the YOUNGER youngest loads has landed, the wave's LDS reads have returned; then the workgroup barrier
+#define MI355_TILE_BARRIER(YOUNGER) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(YOUNGER) : "memory")
+
+  // ---- prologue: blocks 0 .. S-1 (clamped) into the stages, the fragments of block 0 into set 0
+#pragma unroll
+  for (int b = 0; b < S; ++b)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) issue(i, b, kb_begin + b);
+  load_sb(kb_begin);
+  MI355_TILE_BARRIER((S - 1) * LOADS);
+#pragma unroll
+  for (int r = 0; r < READS; ++r) read(r, 0, stage_at(0), scales_at(0));
+
+  // ---- blocks that still request one S further on
+  const int nmain = max(nkb - S, 0);
+  int st = 0;  // stage of block k
+  auto next_stage = [](int s) { return s + 1 == S ? 0 : s + 1; };
+  int k = 0;
+  for (; k + 1 < nmain; k += 2) {
+    const int st1 = next_stage(st), st2 = next_stage(st1);
+    MI355_TILE_BARRIER((S - 2) * LOADS);
+    block(C0{}, std::true_type{}, k, st1, st);
+    MI355_TILE_BARRIER((S - 2) * LOADS);
+    block(C1{}, std::true_type{}, k + 1, st2, st1);
+    st = st2;
+  }
+  if (k < nmain) {  // an odd one: the next block's fragments move to set 0
+    const int st1 = next_stage(st);
+    MI355_TILE_BARRIER((S - 2) * LOADS);
+    block(C0{}, std::true_type{}, k, st1, st);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) w[0][i] = w[1][i];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) tok[0][j] = tok[1][j], tsc[0][j] = tsc[1][j];
+    st = st1;
+    ++k;
+  }
+  // ---- the last blocks (up to S): nothing is requested any more, the number of loads in flight counts down.  The last one
+  //      reads a stage for nobody.
+#pragma unroll
+  for (int u = 0; u < S; ++u) {
+    if (u < nkb - nmain) {
+      const int st1 = next_stage(st);
+      MI355_TILE_BARRIER((u < S - 2 ? S - 2 - u : 0) * LOADS);
+      if (u & 1) block(C1{}, std::false_type{}, k + u, st1, 0);
+      else block(C0{}, std::false_type{}, k + u, st1, 0);
+      st = st1;
+    }
+  }
+  if constexpr (AR == AR_F32) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[NT - 1][MT - 1][v] = fmaf(pend[v], pend_scale, acc[NT - 1][MT - 1][v]);
+  }
+#undef MI355_TILE_BARRIER
+
+  // ---- epilogue: lane holds channels n .. n + 3 of token m for each of its MFMA tiles
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const int m = m0 + wave_m * WM + j * 16 + l16;
+      if (m >= p.M) continue;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int n = n0 + T::channel(wave_n, i) + 4 * q;
+        if (n >= p.N) continue;  // (N % 4 == 0: all four are in)
+        *reinterpret_cast<acc4*>(reinterpret_cast<AccT*>(p.ws) + ((int64_t)split * p.M + m) * p.N + n) = acc[i][j];
+      }
+    }
+  } else {
+    if constexpr (AR == AR_INT8) {
+      if (p.out_dtype == MI355_I32) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          const int m = m0 + wave_m * WM + j * 16 + l16;
+          if (m >= p.M) continue;
+#pragma unroll
+          for (int i = 0; i < NT; ++i) {
+            const int n = n0 + T::channel(wave_n, i) + 4 * q;
+            int* o = reinterpret_cast<int*>(p.out) + (int64_t)m * p.ldo + n;
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              if (n + v < p.N) o[v] = acc[i][j][v];
+          }
+        }
+        return;
+      }
+    }
+    // Whole rows through LDS where the output allows it: stored straight from registers a wave instruction writes sixteen
+    // separate 32-byte pieces.
+    const bool staged = (p.out_dtype == MI355_BF16 || p.out_dtype == MI355_F16) && (p.ldo & 7) == 0 &&
+                        (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && n0 + BN <= p.N;
+    const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
+    static_assert(BM * BN * 2 <= S * T::STAGE_BYTES, "the output tile fits the stages");
+    if (staged) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every load has landed: the stages are free
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const int row = wave_m * WM + j * 16 + l16;
+      const int m = m0 + row;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int col = T::channel(wave_n, i) + 4 * q;
+        const int n = n0 + col;
+        float r[4];
+        if constexpr (AR == AR_INT8) int8_epilogue(p, m, n, acc[i][j], r);
+        else {
+          r[0] = acc[i][j][0], r[1] = acc[i][j][1], r[2] = acc[i][j][2], r[3] = acc[i][j][3];
+          fp8_epilogue(p, m, n, r);
+        }
+        if (staged) {
+          *reinterpret_cast<u32x2*>(t_stage + row * (BN * 2) + (((col >> 3) ^ (row & 7)) << 4) + ((col >> 2) & 1) * 8) =
+              u32x2{pack2_16(p.out_dtype, r[0], r[1]), pack2_16(p.out_dtype, r[2], r[3])};
+        } else if (m < p.M && n < p.N) {
+          store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, min(4, p.N - n), vec_ok);
+        }
+      }
+    }
+    if (staged) {
+      __syncthreads();
+      constexpr int CHUNKS = BN / 8;  // 16-byte pieces of a row
+#pragma unroll 4
+      for (int c = tid; c < BM * CHUNKS; c += T_THREADS) {
+        const int row = c / CHUNKS, chunk = c % CHUNKS;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(t_stage + row * (BN * 2) + ((chunk ^ (row & 7)) << 4));
+        if (m0 + row < p.M)
+          *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.out) + (int64_t)(m0 + row) * p.ldo + n0 + chunk * 8) = v;
+      }
+    }
+  }
+}
+
+// Stages per tile shape.  A 64 x 128 tile's three stages take 73.5 KB, so two such workgroups share a CU and keep four blocks
+// in flight between them; where a launch has at most one workgroup per CU it runs six stages instead.  64 x 192 and
+// 128 x 128 tiles (32 KB a stage) have the CU to themselves either way: four stages.
+constexpr int stages_of(int bm, int bn, bool own_cu) { return bm + bn == 192 ? (own_cu ? 6 : 3) : bm + bn == 256 ? 4 : 3; }
+
+}  // namespace
+}  // namespace mi355

@@ -11,7 +11,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from . import _lib, ops
+from . import _lib, _native, ops
 from .sgl_kernel import sgl_per_token_group_quant_8bit
 
 fp8_dtype = torch.float8_e4m3fn
@@ -74,6 +74,10 @@ def _per_token_group_quant_8bit_raw(
     ``s`` up to a power of two and repacks the fp32 scales with DeepGEMM's
     ``transform_sf_into_required_layout``; here the kernel writes that packed int32 layout
     directly (four exponent bytes per word, words column-major and padded to 4 rows)."""
+    out = _native.try_group_quant(x, group_size, eps, dtype, column_major_scales, scale_tma_aligned or scale_ue8m0, scale_ue8m0,
+                                  True, False)
+    if out is not None:
+        return out
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
 
@@ -198,6 +202,12 @@ def sglang_per_token_group_quant_fp8(
     enable_v2: Optional[bool] = None,
 ):
     """fp8_kernel.py:477-527: allocate outputs, then ``sgl_per_token_group_quant_8bit``."""
+    if enable_v2 is None:
+        enable_v2 = _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
+    if not fuse_silu_and_mul and masked_m is None:
+        out = _native.try_group_quant(x, group_size, eps, fp8_dtype, column_major_scales, scale_tma_aligned, scale_ue8m0, False, enable_v2)
+        if out is not None:
+            return out
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
 

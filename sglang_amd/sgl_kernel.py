@@ -3,19 +3,13 @@
 ``torch.ops.sgl_kernel.<op>.default`` exactly like the reference's wrappers do."""
 from __future__ import annotations
 
-import os
 from typing import Optional
 
 import torch
 
-from . import ops
+from . import _native, ops
 
 ops.register()
-
-
-def _get_bool_env_var(name: str, default: str = "false") -> bool:
-    # same truth values as sglang.srt.utils.get_bool_env_var
-    return os.getenv(name, default).lower() in ("true", "1")
 
 
 def int8_scaled_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
@@ -69,7 +63,7 @@ def sgl_per_token_group_quant_8bit(
     enable_v2: Optional[bool] = None,
 ) -> None:
     if enable_v2 is None:
-        enable_v2 = _get_bool_env_var("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
+        enable_v2 = _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
 
     if enable_v2:
         return torch.ops.sgl_kernel.sgl_per_token_group_quant_8bit_v2.default(
