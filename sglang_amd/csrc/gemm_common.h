@@ -27,7 +27,7 @@ struct GemmParams {
   const float* sb;
   const void* bias;        // optional [N] in the output dtype (INT8 GEMM; per-channel FP8 epilogue)
   const float* col_scale;  // FP8 only, optional [N]: per-channel scale applied in the epilogue (fp8_scaled_mm)
-  const float* row_scale;  // FP8 two-phase kernel in its epilogue-scaled mode only: per-token scale [M]
+  const float* row_scale;  // FP8 two-phase and mid-M kernels in their epilogue-scaled mode (no scales in the K loop): per-token scale [M]
   const void* x16;         // FP8 decode kernel only, optional: unquantized tokens [M, K] (x_dtype, row stride ldx elements);
   int64_t ldx;             // when set, the kernel quantizes them per 1 x 128 group itself and ignores a / sa
   int x_dtype;
@@ -128,40 +128,6 @@ __device__ __forceinline__ void store_out4(void* out, int out_dtype, int64_t off
 }
 
 
-// ---- 256 x 256 output tile of 16-bit elements through LDS.
-// A lane's accumulators are four consecutive channels of one token: stored straight from registers, a wave instruction
-// writes 16 or 32 separate 32-byte pieces, and a tile takes ~12 us.  Instead every wave writes its results into a
-// [256 tokens][512 bytes] image of the tile in LDS (16-byte chunks XOR-swizzled with the row so that neither side has
-// bank conflicts), and after a barrier each wave stores 32 whole rows, two rows of 512 contiguous bytes per instruction.
-constexpr int OUT_TILE_BYTES = 256 * 512;
-
-__device__ __forceinline__ uint32_t pack2_16(int out_dtype, float lo, float hi) {
-  return out_dtype == MI355_BF16 ? pack_bf16x2(lo, hi) : pack_f16x2(lo, hi);
-}
-// four consecutive channels starting at tile column `col` (a multiple of 4) of tile row `row`
-__device__ __forceinline__ void out_tile_put4(uint8_t* tile, int row, int col, int out_dtype, const float* r) {
-  const int chunk = col >> 3, half = (col >> 2) & 1;
-  *reinterpret_cast<u32x2*>(tile + row * 512 + ((chunk ^ (row & 7)) << 4) + half * 8) =
-      u32x2{pack2_16(out_dtype, r[0], r[1]), pack2_16(out_dtype, r[2], r[3])};
-}
-// Called by all 512 threads after a barrier that follows the last out_tile_put4.  Needs ldo % 8 == 0, a 16-byte aligned
-// output base and n0 + 256 <= N; rows at or past M are skipped.
-__device__ __forceinline__ void out_tile_store(const uint8_t* tile, void* out, int64_t ldo, int m0, int n0, int M) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int chunk = lane & 31;
-  uint16_t* o = reinterpret_cast<uint16_t*>(out);
-#pragma unroll 4
-  for (int it = 0; it < 16; ++it) {
-    const int row = wave * 32 + it * 2 + (lane >> 5);
-    const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * 512 + ((chunk ^ (row & 7)) << 4));
-    if (m0 + row < M) *reinterpret_cast<u32x4*>(o + (int64_t)(m0 + row) * ldo + n0 + chunk * 8) = v;
-  }
-}
-__device__ __forceinline__ bool out_tile_ok(const void* out, int64_t ldo, int out_dtype, int n0, int N) {
-  return (out_dtype == MI355_BF16 || out_dtype == MI355_F16) && (ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
-         n0 + 256 <= N;
-}
-
 // Optional per-channel epilogue of the FP8 kernels: r[v] = col_scale[n + v] * r[v] + bias[n + v] for the four consecutive
 // channels n .. n + 3 (channels at or past N repeat the last one; they are never stored).
 __device__ __forceinline__ void fp8_channel_epilogue(const GemmParams& p, int n, float* r) {
@@ -184,6 +150,153 @@ __device__ __forceinline__ void fp8_channel_epilogue(const GemmParams& p, int n,
       const uint32_t h = b[min(n + v, p.N - 1)];
       r[v] += (p.out_dtype == MI355_BF16) ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
     }
+  }
+}
+
+// What an epilogue needs of four consecutive channels n .. n + 3 (channels at or past N repeat the last one; they are never
+// stored): a scale each and a bias each, fetched with one 16- and one 8-byte load where alignment allows.
+struct ChannelTerms {
+  float scale[4], bias[4];
+};
+__device__ __forceinline__ ChannelTerms load_channel_terms(const GemmParams& p, const float* scales, int n) {
+  ChannelTerms c;
+  const uint16_t* b = reinterpret_cast<const uint16_t*>(p.bias);
+  const bool whole = n + 4 <= p.N;
+  if (scales == nullptr) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c.scale[v] = 1.f;
+  } else if (whole && (reinterpret_cast<uintptr_t>(scales + n) & 15) == 0) {
+    const v4f t = *reinterpret_cast<const v4f*>(scales + n);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c.scale[v] = t[v];
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c.scale[v] = scales[min(n + v, p.N - 1)];
+  }
+  if (b == nullptr) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c.bias[v] = 0.f;
+  } else {
+    uint32_t h[4];
+    if (whole && (reinterpret_cast<uintptr_t>(b + n) & 7) == 0) {
+      const u32x2 t = *reinterpret_cast<const u32x2*>(b + n);
+      h[0] = t.x & 0xffffu, h[1] = t.x >> 16, h[2] = t.y & 0xffffu, h[3] = t.y >> 16;
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) h[v] = b[min(n + v, p.N - 1)];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c.bias[v] = p.out_dtype == MI355_BF16 ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]);
+  }
+  return c;
+}
+// INT8: f32(acc) * (channel scale * token scale) + bias, each step rounded.
+__device__ __forceinline__ void int8_apply_terms(const GemmParams& p, const ChannelTerms& c, float token_scale, const int* acc, float* r) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    r[v] = mul_rn((float)acc[v], mul_rn(c.scale[v], token_scale));
+    if (p.bias) r[v] = add_rn(r[v], c.bias[v]);
+  }
+}
+// FP8: token scale * (channel scale * r) + bias, each step rounded; scales that the call does not have are left out.
+__device__ __forceinline__ void fp8_apply_terms(const GemmParams& p, const ChannelTerms& c, float token_scale, float* r) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    if (p.col_scale) r[v] = mul_rn(c.scale[v], r[v]);
+    if (p.row_scale) r[v] = mul_rn(token_scale, r[v]);
+    if (p.bias) r[v] = add_rn(r[v], c.bias[v]);
+  }
+}
+
+// ---- output tile of 16-bit elements through LDS.
+// A lane's accumulators are four consecutive channels of one token: stored straight from registers, a wave instruction
+// writes 16 or 32 separate 32-byte pieces, and a 256 x 256 tile takes ~12 us.  Instead every wave writes its results into a
+// [tokens][BN] image of the tile in LDS (16-byte chunks XOR-swizzled with the row so that neither side has bank conflicts),
+// and after a barrier the workgroup stores whole rows.
+//
+// The conversion is one straight-line copy per output type and with / without bias, chosen once per tile.  With these
+// choices inside the loop over the accumulators (unrolled, since registers cannot be indexed) every tile ran through
+// hundreds of branches and several times the code: 9500 cycles against 1100 for a 128 x 256 tile.
+enum OutScale {
+  OUT_PLAIN,    // no scales left to apply
+  OUT_ROW_COL,  // FP8: row_scale[m] * (col_scale[n] * r)
+  OUT_INT8,     // INT8: f32(acc) * (sb[n] * sa[m])
+};
+template <OutScale OS>
+__device__ __forceinline__ const float* out_channel_scales(const GemmParams& p) { return OS == OUT_INT8 ? p.sb : p.col_scale; }
+template <OutScale OS>
+__device__ __forceinline__ bool out_tile_ok(const GemmParams& p) {
+  return (p.out_dtype == MI355_BF16 || p.out_dtype == MI355_F16) && (p.ldo & 7) == 0 && (p.N & 7) == 0 &&
+         (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0 &&
+         (OS == OUT_PLAIN ? p.col_scale == nullptr : (reinterpret_cast<uintptr_t>(out_channel_scales<OS>(p)) & 15) == 0);
+}
+// The wave's accumulators into the image: acc[i][j][0..3] are channels n0 + channel(i) + 4 q .. + 3 of token m0 + row0 + 16 j.
+template <OutScale OS, int BN, int NT, int MT, class Acc, class Channel>
+__device__ __forceinline__ void out_tile_put(const GemmParams& p, uint8_t* tile, int m0, int n0, int row0, int q, const Acc& acc,
+                                             Channel channel) {
+  uint8_t* put[NT];  // address of the lane's piece of token tile 0; (row & 7) does not depend on the token tile
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const int col = channel(i) + 4 * q;
+    put[i] = tile + row0 * (BN * 2) + (((col >> 3) ^ (row0 & 7)) << 4) + ((col >> 2) & 1) * 8;
+  }
+  auto emit = [&](auto bf16_c, auto bias_c) {
+    constexpr bool BF16 = decltype(bf16_c)::value, BIAS = decltype(bias_c)::value;
+    const float* row_scales = OS == OUT_INT8 ? p.sa : p.row_scale;
+    float token_scale[MT];
+    if constexpr (OS != OUT_PLAIN) {
+#pragma unroll
+      for (int j = 0; j < MT; ++j) token_scale[j] = row_scales[min(m0 + row0 + j * 16, p.M - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int n = min(n0 + channel(i) + 4 * q, p.N - 4);  // (channels past N are never stored)
+      v4f cs = {1.f, 1.f, 1.f, 1.f};
+      u32x2 hb = {0u, 0u};
+      if constexpr (OS != OUT_PLAIN) cs = *reinterpret_cast<const v4f*>(out_channel_scales<OS>(p) + n);
+      if constexpr (BIAS) hb = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.bias) + n);
+      const uint32_t h[4] = {hb.x & 0xffffu, hb.x >> 16, hb.y & 0xffffu, hb.y >> 16};
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        float r[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          // separately rounded steps: neither contract allows a fused multiply-add
+          if constexpr (OS == OUT_INT8) r[v] = mul_rn((float)acc[i][j][v], mul_rn(cs[v], token_scale[j]));
+          else if constexpr (OS == OUT_ROW_COL) r[v] = mul_rn(token_scale[j], mul_rn(cs[v], acc[i][j][v]));
+          else r[v] = acc[i][j][v];
+          if constexpr (BIAS) r[v] = add_rn(r[v], BF16 ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]));
+        }
+        *reinterpret_cast<u32x2*>(put[i] + j * 16 * (BN * 2)) =
+            BF16 ? u32x2{pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])} : u32x2{pack_f16x2(r[0], r[1]), pack_f16x2(r[2], r[3])};
+      }
+    }
+  };
+  if (p.out_dtype == MI355_BF16) {
+    if (p.bias) emit(std::true_type{}, std::true_type{});
+    else emit(std::true_type{}, std::false_type{});
+  } else {
+    if (p.bias) emit(std::false_type{}, std::true_type{});
+    else emit(std::false_type{}, std::false_type{});
+  }
+}
+// Called by all 512 threads after a barrier that follows the last out_tile_put; rows at or past M and channels at or past N
+// are skipped (N is a multiple of 8, see out_tile_ok).
+template <int BM, int BN>
+__device__ __forceinline__ void out_tile_store(const GemmParams& p, const uint8_t* tile, int m0, int n0) {
+  constexpr int CHUNKS = BN / 8, PIECES = (BM * CHUNKS + 511) / 512;  // 16-byte pieces of a row, pieces per thread
+  const int tid = threadIdx.x;
+  u32x4 v[PIECES];
+#pragma unroll
+  for (int e = 0; e < PIECES; ++e) {
+    const int c = min(e * 512 + tid, BM * CHUNKS - 1), row = c / CHUNKS, chunk = c % CHUNKS;
+    v[e] = *reinterpret_cast<const u32x4*>(tile + row * (BN * 2) + ((chunk ^ (row & 7)) << 4));
+  }
+#pragma unroll
+  for (int e = 0; e < PIECES; ++e) {
+    const int c = e * 512 + tid, row = c / CHUNKS, chunk = c % CHUNKS;
+    if (c < BM * CHUNKS && m0 + row < p.M && n0 + chunk * 8 < p.N)
+      *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.out) + (int64_t)(m0 + row) * p.ldo + n0 + chunk * 8) = v[e];
   }
 }
 
@@ -232,6 +345,12 @@ int launch_fp8_pp_rowcol(GemmParams& p, hipStream_t stream, const char* what);
 // Mid-M blockwise FP8 GEMM (64/128 x 256 tile, 8 waves, three LDS stages, hand-issued direct-to-LDS loads);
 // gemm_fp8_dma3.hip.  Needs 16-byte aligned rows, K % 128 == 0, row offsets below 4 GiB.  dma3_plan() gives the split it
 // wants; the caller sets p.splits, p.kb_per_split and p.ws accordingly.
+// The tile shapes it is built with, tokens x channels.
+struct TileSize {
+  int bm, bn;
+};
+constexpr TileSize MID_TILES[] = {{64, 128}, {96, 128}, {128, 128}, {160, 128}, {192, 128}, {256, 128}, {64, 192},
+                                  {96, 192}, {128, 192}, {160, 192}, {64, 256}, {96, 256}, {128, 256}};
 struct Dma3Plan {
   int bm, bn, splits, kb_per_split;  // bn: 256, 192 (FP8 only) or 128, whichever models fastest
   double efficiency;  // modelled fraction of the streaming time that is useful (balance, partial sums, pipeline fill)
@@ -243,6 +362,8 @@ int launch_fp8_dma3(GemmParams& p, int bm, int bn, hipStream_t stream, const cha
 // The same for packed UE8M0 scales on both operands (p.sa / p.sb point to the words, p.sa_sk / p.sb_sn / p.sb_sk are word
 // strides; token words M-major with a pitch that is a multiple of four words), applied by the MFMA.
 int launch_fp8_dma3_ue8m0(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
+// The same with one scale per token (p.row_scale) and per channel (p.col_scale) applied in the epilogue; no scales in the K loop.
+int launch_fp8_dma3_unit(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
 // One-call linear at decode sizes on this kernel: a producer wave quantizes the unquantized tokens (p.x16, M <= 16) block by block.
 int launch_fp8_dma3_quant(GemmParams& p, int bn, hipStream_t stream, const char* what);
 

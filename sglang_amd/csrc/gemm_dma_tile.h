@@ -1,4 +1,4 @@
-// The mid-M tile of the FP8 and INT8 GEMMs for gfx950: (64 or 128) tokens x (256, 192 or 128) channels, 8 waves (two per
+// The mid-M tile of the FP8 and INT8 GEMMs for gfx950: 64 .. 256 tokens x 256, 192 or 128 channels, 8 waves (two per
 // SIMD), S LDS stages filled by direct-to-LDS loads, operand fragments read one K block AHEAD of their multiplication.
 //
 // What bounds a short tile is the chain of one K block: after the block's barrier every wave reads its operand fragments
@@ -18,6 +18,8 @@
 // Requires K % 128 == 0, 16-byte aligned rows and row offsets below 4 GiB; AR_F32 / AR_UE8M0 also token scales laid out
 // M-major with a pitch that is a multiple of four words.
 #pragma once
+
+#include <utility>
 
 #include "gemm_common.h"
 
@@ -54,20 +56,24 @@ __device__ __forceinline__ float lds_f32(lds_cptr p, int imm) {
 
 template <Arith AR, int BM, int BN>
 struct TileShape {
-  static_assert((BM == 64 || BM == 128) && (BN == 128 || BN == 192 || BN == 256), "tile");
+  static_assert(BM % 32 == 0 && (BN == 128 || BN == 192 || BN == 256), "tile");
   static constexpr bool SCALED = AR == AR_F32 || AR == AR_UE8M0;
-  static constexpr int MT = BM / 32, NT = BN / 64, STEPS = MT * NT;   // a wave owns BM / 2 tokens x BN / 4 channels
-  static constexpr int ROW_LOADS = (BM + BN) / 64;                    // a wave fills 8 rows per load
+  // eight waves: two rows of four, or four rows of two where the tile is taller than wide (fewer fragments per product)
+  static constexpr int WAVES_M = BM >= 192 && BM % 64 == 0 && BN == 128 ? 4 : 2, WAVES_N = 8 / WAVES_M;
+  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
+  static constexpr int MT = WM / 16, NT = WN / 16, STEPS = MT * NT;   // 16 x 16 tiles of a wave
+  static_assert(WM % 16 == 0 && WN % 16 == 0, "whole MFMA tiles");
+  static constexpr int GROUPS = (BM + BN) / 8;                        // a load fills 8 rows of a stage
+  static constexpr int ROW_LOADS = (GROUPS + 7) / 8;                  // per wave and stage; the last may repeat a row group
   static constexpr int LOADS = ROW_LOADS + (SCALED ? 1 : 0);
-  // A wave's channels are BN / 4 consecutive ones inside one 128-channel scale block, except for BN = 192, where 48
-  // consecutive channels could straddle two blocks: there the wave's channel tile i is channels 64 i + 16 wave .. + 15, so that
-  // tile i of every wave lies in the block of channel n0 + 64 i.
+  // A wave's channels are WN consecutive ones inside one 128-channel scale block, except for BN = 192, where 48 consecutive
+  // channels could straddle two blocks: there the wave's channel tile i is channels 64 i + 16 wave .. + 15, so that tile i of
+  // every wave lies in the block of channel n0 + 64 i.
   static constexpr bool INTERLEAVED = BN == 192;
   static constexpr int SB = INTERLEAVED ? NT : 1;
   static constexpr int W_STRIDE = INTERLEAVED ? 64 * 128 : 16 * 128;  // bytes between a wave's consecutive channel tiles in a stage
   static constexpr int STAGE_BYTES = (BM + BN) * KSTEP;
-  static_assert(LOADS <= STEPS, "one load per step");
-  __device__ static int channel(int wave_n, int i) { return INTERLEAVED ? i * 64 + wave_n * 16 : wave_n * (BN / 4) + i * 16; }
+  __device__ static int channel(int wave_n, int i) { return INTERLEAVED ? i * 64 + wave_n * 16 : wave_n * WN + i * 16; }
 };
 
 // One BM x BN output tile at (m0, n0), K blocks of split `split`, by the whole workgroup.
@@ -77,13 +83,13 @@ template <Arith AR, int BM, int BN, bool SPLIT, int S>
 __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, int split) {
   using T = TileShape<AR, BM, BN>;
   static_assert(S >= 3 && S * (T::STAGE_BYTES + BM * 4) <= 160 * 1024, "the stages must fit the CU's LDS");
-  constexpr int MT = T::MT, NT = T::NT, SB = T::SB, LOADS = T::LOADS, WM = BM / 2;
+  constexpr int MT = T::MT, NT = T::NT, SB = T::SB, LOADS = T::LOADS, WM = T::WM;
   using AccT = typename std::conditional<AR == AR_INT8, int, float>::type;
   typedef AccT acc4 __attribute__((ext_vector_type(4)));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave_m = wave >> 2, wave_n = wave & 3;
+  const int wave_m = wave / T::WAVES_N, wave_n = wave % T::WAVES_N;
   const int l16 = lane & 15, q = lane >> 4;
   const int kb_begin = split * p.kb_per_split;
   const int nkb = min(p.kb_total, kb_begin + p.kb_per_split) - kb_begin;
@@ -100,22 +106,28 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
     const int chunk_byte = ((lane & 7) ^ lrow) * 16;
 #pragma unroll
     for (int i = 0; i < T::ROW_LOADS; ++i) {
-      const int row = i * 64 + wave * 8 + lrow;
+      const int row = min(i * 8 + wave, T::GROUPS - 1) * 8 + lrow;
       goff[i] = row < BM ? (uint32_t)((int64_t)min(m0 + row, p.M - 1) * p.lda + chunk_byte)
                          : (uint32_t)((int64_t)min(n0 + row - BM, p.N - 1) * p.ldb + chunk_byte);
     }
   }
+  const int last_group = __builtin_amdgcn_readfirstlane(min((T::ROW_LOADS - 1) * 8 + wave, T::GROUPS - 1));
+  // matrix of the wave's row group in the load that covers both kinds of rows (BM not a multiple of 64)
+  const bool mixed_tokens = __builtin_amdgcn_readfirstlane(BM / 64 * 8 + wave < BM / 8);
+  const uint8_t* mixed_base = mixed_tokens ? p.a : p.b;
   // every wave fetches BM / 8 token scales per K block, four per lane; quads past M refetch the last valid one
-  const uint32_t sa_off = (uint32_t)min(m0 + wave * (BM / 8) + (lane & (BM / 32 - 1)) * 4, (p.M - 1) & ~3) * 4u;
+  const uint32_t sa_off = (uint32_t)min(m0 + wave * (BM / 8) + min(lane, BM / 32 - 1) * 4, (p.M - 1) & ~3) * 4u;
   // Load number i of K block kb (< ROW_LOADS: tile rows; then the token scales) into stage `st`.  The statements write m0; it
   // cannot be listed as a clobber (the compiler reserves the register), and no compiler-managed use of m0 lies between them
   // and the next statement that sets it.
   auto issue = [&](int i, int st, int kb) {
     kb = min(kb, kb_last);
     if (i < T::ROW_LOADS) {
-      const uint8_t* base = (i < BM / 64 ? p.a : p.b) + (uint64_t)kb * KSTEP;  // wave-uniform
+      // wave-uniform: the row group (the last load's may be one another wave fetches too) and its matrix
+      const int group = i * 8 + 8 <= T::GROUPS ? i * 8 + wave : last_group;
+      const uint8_t* base = (i * 8 + 8 <= BM / 8 ? p.a : i * 8 >= BM / 8 ? p.b : mixed_base) + (uint64_t)kb * KSTEP;
       asm volatile("" : "+s"(base));
-      const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_stage + (uint32_t)(st * T::STAGE_BYTES + (i * 64 + wave * 8) * KSTEP);
+      const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_stage + (uint32_t)(st * T::STAGE_BYTES + group * 8 * KSTEP);
       asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
     } else if constexpr (T::SCALED) {
       // BM / 32 lanes fetch 16 bytes each (a 4-byte-per-lane load in this stream costs far more than its size).  exec is
@@ -125,12 +137,8 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
       asm volatile("" : "+s"(sbase));
       const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_scale + (uint32_t)(st * BM + wave * (BM / 8)) * 4u;
       uint64_t saved;
-      if constexpr (BM == 128)
-        asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, 0xf\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, %0"
-                     : "=&s"(saved) : "v"(sa_off), "s"(sbase), "s"(lds_addr) : "memory");
-      else
-        asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, 0x3\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, %0"
-                     : "=&s"(saved) : "v"(sa_off), "s"(sbase), "s"(lds_addr) : "memory");
+      asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, %4\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, %0"
+                   : "=&s"(saved) : "v"(sa_off), "s"(sbase), "s"(lds_addr), "n"((1 << (BM / 32)) - 1) : "memory");
     }
   };
 
@@ -190,8 +198,15 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
   auto stage_at = [&](int st) { return (lds_cptr)t_stage + st * T::STAGE_BYTES; };
   auto scales_at = [&](int st) { return (lds_cptr) reinterpret_cast<uint8_t*>(t_scale) + st * BM * 4; };
 
-  v4f pend = v4f{0.f, 0.f, 0.f, 0.f};  // AR_F32: the product of the previous step, whose promotion runs behind this step's MFMA
-  float pend_scale = 0.f;
+  // AR_F32: a product is promoted (acc += product * scale) behind the second MFMA after its own, where its result needs no wait
+  // states any more; the last two products of a block are promoted in the next one.
+  v4f pend[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+  float pend_scale[2] = {0.f, 0.f};
+  auto promote = [&](int t, const v4f& product, float scale) {
+    const int j = t / NT, i = t % NT;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(product[v], scale, acc[i][j][v]);
+  };
 
   // Multiplies block k out of set CUR while reading block k + 1 (in stage st_next) into the other set and, with FILL, issuing
   // block k + S into st_fill, the stage block k has just left.
@@ -214,16 +229,18 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
 #pragma unroll
       for (int j = 0; j < MT; ++j) sc[j][0] = __uint_as_float(__float_as_uint(tsc[CUR][j]) >> shift);
     }
+    __builtin_amdgcn_sched_barrier(0);  // the waits for this block's scales come before the scalar load of the next one's
     load_sb(kb + 1);
     __builtin_amdgcn_sched_barrier(0);
     // the reads go out over the first three quarters of the steps, so that the last ones have returned at the barrier
+    constexpr int LPS = (LOADS + T::STEPS - 1) / T::STEPS;  // loads per step
     constexpr int PER = (READS * 4 + T::STEPS * 3 - 1) / (T::STEPS * 3);
-    v4f part[2];
+    v4f part[3];
 #pragma unroll
     for (int t = 0; t < T::STEPS; ++t) {
       const int j = t / NT, i = t % NT;
       if constexpr (AR == AR_F32) {
-        part[t & 1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(w[CUR][i]), as_v8i(tok[CUR][j]), v4f{0.f, 0.f, 0.f, 0.f},
+        part[t % 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(w[CUR][i]), as_v8i(tok[CUR][j]), v4f{0.f, 0.f, 0.f, 0.f},
                                                                        0, 0, 0, 0, 0, 0);
       } else if constexpr (AR == AR_UE8M0) {
         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(w[CUR][i]), as_v8i(tok[CUR][j]), acc[i][j], 0, 0, 0,
@@ -238,20 +255,19 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
 #pragma unroll
       for (int r = t * PER; r < (t + 1) * PER; ++r)
         if (r < READS) read(r, NXT, nst, nsc);
-      if (FILL && t < LOADS) issue(t, st_fill, kb + S);
+#pragma unroll
+      for (int l = t * LPS; l < (t + 1) * LPS; ++l)
+        if (FILL && l < LOADS) issue(l, st_fill, kb + S);
       if constexpr (AR == AR_F32) {
-        if (t == 0) {  // the last product of the previous block
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[NT - 1][MT - 1][v] = fmaf(pend[v], pend_scale, acc[NT - 1][MT - 1][v]);
-        } else {
-          const int pj = (t - 1) / NT, pi = (t - 1) % NT;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[pi][pj][v] = fmaf(part[(t - 1) & 1][v], sc[pj][SB > 1 ? pi : 0], acc[pi][pj][v]);
-        }
+        if (t < 2) promote(T::STEPS - 2 + t, pend[t], pend_scale[t]);
+        else promote(t - 2, part[(t - 2) % 3], sc[(t - 2) / NT][SB > 1 ? (t - 2) % NT : 0]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (AR == AR_F32) pend = part[(T::STEPS - 1) & 1], pend_scale = sc[MT - 1][SB > 1 ? NT - 1 : 0];
+    if constexpr (AR == AR_F32) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) pend[e] = part[(T::STEPS - 2 + e) % 3], pend_scale[e] = sc[MT - 1][SB > 1 ? NT - 2 + e : 0];
+    }
   };
   using C0 = std::integral_constant<int, 0>;
   using C1 = std::integral_constant<int, 1>;
@@ -304,11 +320,9 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
       st = st1;
     }
   }
-  if constexpr (AR == AR_F32) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[NT - 1][MT - 1][v] = fmaf(pend[v], pend_scale, acc[NT - 1][MT - 1][v]);
-  }
+  if constexpr (AR == AR_F32) promote(T::STEPS - 2, pend[0], pend_scale[0]), promote(T::STEPS - 1, pend[1], pend_scale[1]);
 #undef MI355_TILE_BARRIER
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // refetches of a K shorter than the pipeline must not outlive the workgroup's LDS
 
   // ---- epilogue: lane holds channels n .. n + 3 of token m for each of its MFMA tiles
   if constexpr (SPLIT) {
@@ -342,53 +356,83 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
         return;
       }
     }
-    // Whole rows through LDS where the output allows it: stored straight from registers a wave instruction writes sixteen
-    // separate 32-byte pieces.
-    const bool staged = (p.out_dtype == MI355_BF16 || p.out_dtype == MI355_F16) && (p.ldo & 7) == 0 &&
-                        (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && n0 + BN <= p.N;
-    const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
+    constexpr OutScale OS = AR == AR_INT8 ? OUT_INT8 : AR == AR_UNIT ? OUT_ROW_COL : OUT_PLAIN;
     static_assert(BM * BN * 2 <= S * T::STAGE_BYTES, "the output tile fits the stages");
-    if (staged) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every load has landed: the stages are free
-#pragma unroll
-    for (int j = 0; j < MT; ++j) {
-      const int row = wave_m * WM + j * 16 + l16;
-      const int m = m0 + row;
+    const int row0 = wave_m * WM + l16;
+    if (out_tile_ok<OS>(p)) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave's loads have landed: the stages are free
+      out_tile_put<OS, BN, NT, MT>(p, t_stage, m0, n0, row0, q, acc, [&](int i) { return T::channel(wave_n, i); });
+      __syncthreads();
+      out_tile_store<BM, BN>(p, t_stage, m0, n0);
+    } else {
+      const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
+      const float* row_scales = AR == AR_INT8 ? p.sa : p.row_scale;
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
-        const int col = T::channel(wave_n, i) + 4 * q;
-        const int n = n0 + col;
-        float r[4];
-        if constexpr (AR == AR_INT8) int8_epilogue(p, m, n, acc[i][j], r);
-        else {
-          r[0] = acc[i][j][0], r[1] = acc[i][j][1], r[2] = acc[i][j][2], r[3] = acc[i][j][3];
-          fp8_epilogue(p, m, n, r);
-        }
-        if (staged) {
-          *reinterpret_cast<u32x2*>(t_stage + row * (BN * 2) + (((col >> 3) ^ (row & 7)) << 4) + ((col >> 2) & 1) * 8) =
-              u32x2{pack2_16(p.out_dtype, r[0], r[1]), pack2_16(p.out_dtype, r[2], r[3])};
-        } else if (m < p.M && n < p.N) {
+        const int n = n0 + T::channel(wave_n, i) + 4 * q;
+        const ChannelTerms c = load_channel_terms(p, out_channel_scales<OS>(p), n);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          const int m = m0 + row0 + j * 16;
+          if (m >= p.M || n >= p.N) continue;
+          const float token_scale = row_scales ? row_scales[m] : 1.f;
+          float r[4];
+          if constexpr (AR == AR_INT8) {
+            const int a4[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            int8_apply_terms(p, c, token_scale, a4, r);
+          } else {
+            r[0] = acc[i][j][0], r[1] = acc[i][j][1], r[2] = acc[i][j][2], r[3] = acc[i][j][3];
+            fp8_apply_terms(p, c, token_scale, r);
+          }
           store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, min(4, p.N - n), vec_ok);
         }
-      }
-    }
-    if (staged) {
-      __syncthreads();
-      constexpr int CHUNKS = BN / 8;  // 16-byte pieces of a row
-#pragma unroll 4
-      for (int c = tid; c < BM * CHUNKS; c += T_THREADS) {
-        const int row = c / CHUNKS, chunk = c % CHUNKS;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(t_stage + row * (BN * 2) + ((chunk ^ (row & 7)) << 4));
-        if (m0 + row < p.M)
-          *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.out) + (int64_t)(m0 + row) * p.ldo + n0 + chunk * 8) = v;
       }
     }
   }
 }
 
-// Stages per tile shape.  A 64 x 128 tile's three stages take 73.5 KB, so two such workgroups share a CU and keep four blocks
-// in flight between them; where a launch has at most one workgroup per CU it runs six stages instead.  64 x 192 and
-// 128 x 128 tiles (32 KB a stage) have the CU to themselves either way: four stages.
-constexpr int stages_of(int bm, int bn, bool own_cu) { return bm + bn == 192 ? (own_cu ? 6 : 3) : bm + bn == 256 ? 4 : 3; }
+// Stages per tile shape: as many as the LDS holds, up to six.  A 64 x 128 tile's three stages take 73.5 KB, so two such
+// workgroups share a CU and keep four blocks in flight between them; where a launch has at most one workgroup per CU it runs
+// six stages instead.
+constexpr int stages_of(int bm, int bn, bool own_cu) {
+  return bm + bn == 192 ? (own_cu ? 6 : 3) : bm + bn == 224 ? 5 : bm + bn <= 288 ? 4 : 3;
+}
+
+template <Arith AR, int BM, int BN, bool SPLIT, int S>
+__global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + BN == 192 && S == 3 ? 4 : 2))) void gemm_dma_kernel(const GemmParams p) {
+  const TileCoord tc = tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n);
+  dma_tile<AR, BM, BN, SPLIT, S>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
+}
+
+template <Arith AR, int BM, int BN>
+int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
+  p.tiles_m = (p.M + BM - 1) / BM;
+  p.tiles_n = (p.N + BN - 1) / BN;
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
+  constexpr int OWN = stages_of(BM, BN, true), SHARED = stages_of(BM, BN, false);
+  if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) {
+    if (p.splits > 1) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, true, SHARED>), grid, dim3(T_THREADS), 0, stream, p);
+    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, false, SHARED>), grid, dim3(T_THREADS), 0, stream, p);
+  } else {
+    if (p.splits > 1) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, true, OWN>), grid, dim3(T_THREADS), 0, stream, p);
+    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, false, OWN>), grid, dim3(T_THREADS), 0, stream, p);
+  }
+  return check_launch(what);
+}
+
+// The tile shapes that are built (MID_TILES in gemm_common.h), by height and width.
+template <Arith AR, size_t... I>
+int launch_dma_tile_of(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what, std::index_sequence<I...>) {
+  int rc = MI355_ERR_UNSUPPORTED;
+  bool found = false;
+  ((found = found || (bm == MID_TILES[I].bm && bn == MID_TILES[I].bn && (rc = launch_dma_tile<AR, MID_TILES[I].bm, MID_TILES[I].bn>(p, stream, what), true))), ...);
+  if (!found) set_error("%s: no %d x %d tile is built", what, bm, bn);
+  return rc;
+}
+template <Arith AR>
+int launch_dma_tile_of(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what) {
+  return launch_dma_tile_of<AR>(p, bm, bn, stream, what, std::make_index_sequence<sizeof(MID_TILES) / sizeof(MID_TILES[0])>{});
+}
 
 }  // namespace
 }  // namespace mi355

@@ -51,7 +51,7 @@ constexpr int G_STAGE = G_ROWS * KSTEP;
 __shared__ __attribute__((aligned(1024))) uint8_t g_stages[2 * G_STAGE];
 #define g_stage0 (g_stages)
 #define g_stage1 (g_stages + G_STAGE)
-static_assert(2 * G_STAGE >= OUT_TILE_BYTES, "the output tile is staged in the two input stages");
+static_assert(2 * G_STAGE >= G_BM * G_BN * 2, "the output tile is staged in the two input stages");
 // token scales: four stages (block b in stage b % 4) of 256 floats
 __shared__ __attribute__((aligned(256))) float g_scale[4 * G_BM];
 
@@ -248,38 +248,6 @@ __device__ __forceinline__ void compute_ue8m0(const Frag (&w)[G_NT], const Frag 
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// r[v] = row_scale[m] * (col_scale[n + v] * r[v]) + bias[n + v], each step rounded (the order of fp8_scaled_mm's epilogue,
-// sgl-kernel/csrc/gemm/fp8_gemm_kernel.cu:529-547); channels at or past N repeat the last one and are never stored.
-__device__ __forceinline__ void row_col_epilogue(const GemmParams& p, int m, int n, float* r) {
-  const float rs = p.row_scale[min(m, p.M - 1)];
-  const uint16_t* b = reinterpret_cast<const uint16_t*>(p.bias);
-  float cs[4], bv[4] = {0.f, 0.f, 0.f, 0.f};
-  if (n + 4 <= p.N && (reinterpret_cast<uintptr_t>(p.col_scale + n) & 15) == 0 &&
-      (p.bias == nullptr || (reinterpret_cast<uintptr_t>(b + n) & 7) == 0)) {
-    // one 16-byte and one 8-byte load instead of eight scattered ones
-    const v4f c = *reinterpret_cast<const v4f*>(p.col_scale + n);
-    cs[0] = c[0], cs[1] = c[1], cs[2] = c[2], cs[3] = c[3];
-    if (p.bias) {
-      const u32x2 hb = *reinterpret_cast<const u32x2*>(b + n);
-      const uint32_t h[4] = {hb.x & 0xffffu, hb.x >> 16, hb.y & 0xffffu, hb.y >> 16};
-#pragma unroll
-      for (int v = 0; v < 4; ++v) bv[v] = (p.out_dtype == MI355_BF16) ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]);
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int nn = min(n + v, p.N - 1);
-      cs[v] = p.col_scale[nn];
-      if (p.bias) bv[v] = (p.out_dtype == MI355_BF16) ? bf16_bits_to_f32(b[nn]) : f16_bits_to_f32(b[nn]);
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const float t = mul_rn(rs, mul_rn(cs[v], r[v]));
-    r[v] = p.bias ? add_rn(t, bv[v]) : t;
-  }
-}
-
 // SM, where the scales are applied:
 //   SM_BLOCK_F32  fp32 scales per K block, by promotion FMAs (the blockwise GEMM of the reference);
 //   SM_UE8M0      p.sa / p.sb point to packed exponent words (int32): token word (m, kw) at sa[kw * sa_sk + m], channel word
@@ -403,31 +371,26 @@ __device__ __forceinline__ void pp_tile(const GemmParams& p, const int m0, const
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- epilogue: lane holds channels n .. n+3 of token m
-  if (out_tile_ok(p.out, p.ldo, p.out_dtype, n0, p.N)) {
+  constexpr OutScale OS = SM == SM_EPILOGUE ? OUT_ROW_COL : OUT_PLAIN;
+  const int row0 = grp * G_WM + l16;
+  auto channel = [&](int i) { return wave_n * G_WN + i * 16; };
+  if (out_tile_ok<OS>(p)) {
     asm volatile("s_barrier" ::: "memory");  // every wave's stray loads have landed: the stages are free
-#pragma unroll
-    for (int j = 0; j < G_MT; ++j)
-#pragma unroll
-      for (int i = 0; i < G_NT; ++i) {
-        if constexpr (SM == SM_EPILOGUE) row_col_epilogue(p, m0 + grp * G_WM + j * 16 + l16, n0 + wave_n * G_WN + i * 16 + 4 * q, acc[i][j]);
-        else fp8_channel_epilogue(p, n0 + wave_n * G_WN + i * 16 + 4 * q, acc[i][j]);
-        out_tile_put4(g_stages, grp * G_WM + j * 16 + l16, wave_n * G_WN + i * 16 + 4 * q, p.out_dtype, acc[i][j]);
-      }
+    out_tile_put<OS, G_BN, G_NT, G_MT>(p, g_stages, m0, n0, row0, q, acc, channel);
     __syncthreads();
-    out_tile_store(g_stages, p.out, p.ldo, m0, n0, p.M);
+    out_tile_store<G_BM, G_BN>(p, g_stages, m0, n0);
     return;
   }
   const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
 #pragma unroll
-  for (int j = 0; j < G_MT; ++j) {
-    const int m = m0 + grp * G_WM + j * 16 + l16;
-    if (m >= p.M) continue;
+  for (int i = 0; i < G_NT; ++i) {
+    const int n = n0 + channel(i) + 4 * q;
+    const ChannelTerms c = load_channel_terms(p, p.col_scale, n);
 #pragma unroll
-    for (int i = 0; i < G_NT; ++i) {
-      const int n = n0 + wave_n * G_WN + i * 16 + 4 * q;
-      if (n >= p.N) continue;
-      if constexpr (SM == SM_EPILOGUE) row_col_epilogue(p, m, n, acc[i][j]);
-      else fp8_channel_epilogue(p, n, acc[i][j]);
+    for (int j = 0; j < G_MT; ++j) {
+      const int m = m0 + row0 + j * 16;
+      if (m >= p.M || n >= p.N) continue;
+      fp8_apply_terms(p, c, p.row_scale ? p.row_scale[m] : 1.f, acc[i][j]);
       store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, acc[i][j], min(4, p.N - n), vec_ok);
     }
   }

@@ -35,7 +35,7 @@ constexpr int J_SET_A = 6, J_SET_B = 2;
 __shared__ __attribute__((aligned(1024))) uint8_t j_stages[2 * J_STAGE];
 #define j_stage0 (j_stages)
 #define j_stage1 (j_stages + J_STAGE)
-static_assert(2 * J_STAGE >= OUT_TILE_BYTES, "the output tile is staged in the two input stages");
+static_assert(2 * J_STAGE >= J_BM * J_BN * 2, "the output tile is staged in the two input stages");
 
 typedef __attribute__((address_space(3))) void* lptr_t;
 typedef const __attribute__((address_space(3))) uint8_t* lds_cptr;
@@ -195,40 +195,11 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp_kernel(const GemmParam
   // ---- epilogue: lane holds, for token m = 16 j + l16 of the wave's rows, channels 16 i + 4 q + (0..3) of its columns
   const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
   const bool raw = p.out_dtype == MI355_I32;
-  if (out_tile_ok(p.out, p.ldo, p.out_dtype, n0, p.N) && (reinterpret_cast<uintptr_t>(p.sb) & 15) == 0 &&
-      (p.bias == nullptr || (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0)) {
-    // full tile: channel scales and bias by 16- and 8-byte loads, results through LDS, whole rows to memory
+  if (out_tile_ok<OUT_INT8>(p)) {
     asm volatile("s_barrier" ::: "memory");  // every wave's stray loads have landed: the stages are free
-    float sa_j[J_MT];
-#pragma unroll
-    for (int j = 0; j < J_MT; ++j) sa_j[j] = p.sa[min(m0 + grp * J_WM + j * 16 + l16, p.M - 1)];
-#pragma unroll
-    for (int i = 0; i < J_NT; ++i) {
-      {
-        const int col = wave_n * J_WN + i * 16 + 4 * q;
-        const v4f sbv = *reinterpret_cast<const v4f*>(p.sb + n0 + col);
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
-          const u32x2 hb = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.bias) + n0 + col);
-          const uint32_t h[4] = {hb.x & 0xffffu, hb.x >> 16, hb.y & 0xffffu, hb.y >> 16};
-#pragma unroll
-          for (int v = 0; v < 4; ++v) bv[v] = (p.out_dtype == MI355_BF16) ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]);
-        }
-#pragma unroll
-        for (int j = 0; j < J_MT; ++j) {
-          float r[4];
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            float x = mul_rn((float)acc[i][j][v], mul_rn(sbv[v], sa_j[j]));
-            if (p.bias) x = add_rn(x, bv[v]);
-            r[v] = x;
-          }
-          out_tile_put4(j_stages, grp * J_WM + j * 16 + l16, col, p.out_dtype, r);
-        }
-      }
-    }
+    out_tile_put<OUT_INT8, J_BN, J_NT, J_MT>(p, j_stages, m0, n0, grp * J_WM + l16, q, acc, [&](int i) { return wave_n * J_WN + i * 16; });
     __syncthreads();
-    out_tile_store(j_stages, p.out, p.ldo, m0, n0, p.M);
+    out_tile_store<J_BM, J_BN>(p, j_stages, m0, n0);
     return;
   }
 #pragma unroll

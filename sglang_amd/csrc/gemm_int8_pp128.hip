@@ -99,20 +99,6 @@ __device__ __forceinline__ void compute(const v4i (&w)[J_NT][2], const v4i (&t)[
       for (int i = 0; i < J_NT; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[i][h], t[j][h], acc[i][j], 0, 0, 0);
 }
 
-// 128-row output tile through LDS (rows of 512 bytes, chunks swizzled as out_tile_put4 writes them): every wave stores 16
-// whole rows, two per instruction.  Needs ldo % 8 == 0, a 16-byte aligned output base and n0 + 256 <= N.
-__device__ __forceinline__ void out_tile128_store(const uint8_t* tile, void* out, int64_t ldo, int m0, int n0, int M) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int chunk = lane & 31;
-  uint16_t* o = reinterpret_cast<uint16_t*>(out);
-#pragma unroll 4
-  for (int it = 0; it < 8; ++it) {
-    const int row = wave * 16 + it * 2 + (lane >> 5);
-    const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * 512 + ((chunk ^ (row & 7)) << 4));
-    if (m0 + row < M) *reinterpret_cast<u32x4*>(o + (int64_t)(m0 + row) * ldo + n0 + chunk * 8) = v;
-  }
-}
-
 template <bool SPLIT>
 __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmParams p) {
   const int tid = threadIdx.x;
@@ -213,40 +199,11 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmPa
   }
   const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
   const bool raw = p.out_dtype == MI355_I32;
-  if (out_tile_ok(p.out, p.ldo, p.out_dtype, n0, p.N) && (reinterpret_cast<uintptr_t>(p.sb) & 15) == 0 &&
-      (p.bias == nullptr || (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0)) {
-    // full tile: channel scales and bias by 16- and 8-byte loads, results through LDS, whole rows to memory
+  if (out_tile_ok<OUT_INT8>(p)) {
     asm volatile("s_barrier" ::: "memory");  // every wave's stray loads have landed: the stages are free
-    float sa_j[J_MT];
-#pragma unroll
-    for (int j = 0; j < J_MT; ++j) sa_j[j] = p.sa[min(m0 + grp * J_WM + j * 16 + l16, p.M - 1)];
-#pragma unroll
-    for (int i = 0; i < J_NT; ++i) {
-      {
-        const int col = wave_n * J_WN + i * 16 + 4 * q;
-        const v4f sbv = *reinterpret_cast<const v4f*>(p.sb + n0 + col);
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
-          const u32x2 hb = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.bias) + n0 + col);
-          const uint32_t h[4] = {hb.x & 0xffffu, hb.x >> 16, hb.y & 0xffffu, hb.y >> 16};
-#pragma unroll
-          for (int v = 0; v < 4; ++v) bv[v] = (p.out_dtype == MI355_BF16) ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]);
-        }
-#pragma unroll
-        for (int j = 0; j < J_MT; ++j) {
-          float r[4];
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            float x = mul_rn((float)acc[i][j][v], mul_rn(sbv[v], sa_j[j]));
-            if (p.bias) x = add_rn(x, bv[v]);
-            r[v] = x;
-          }
-          out_tile_put4(j_stages, grp * J_WM + j * 16 + l16, col, p.out_dtype, r);
-        }
-      }
-    }
+    out_tile_put<OUT_INT8, J_BN, J_NT, J_MT>(p, j_stages, m0, n0, grp * J_WM + l16, q, acc, [&](int i) { return wave_n * J_WN + i * 16; });
     __syncthreads();
-    out_tile128_store(j_stages, p.out, p.ldo, m0, n0, p.M);
+    out_tile_store<J_BM, J_BN>(p, j_stages, m0, n0);
     return;
   }
 #pragma unroll

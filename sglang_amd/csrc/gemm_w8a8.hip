@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmParams p) 
         if (k0 + j < p.splits) s[0] += t[j][0], s[1] += t[j][1], s[2] += t[j][2], s[3] += t[j][3];
     }
     float r[4] = {s[0], s[1], s[2], s[3]};
-    fp8_channel_epilogue(p, n, r);
+    fp8_apply_terms(p, load_channel_terms(p, p.col_scale, n), p.row_scale ? p.row_scale[m] : 1.f, r);
     const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
     store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, 4, vec_ok);
   } else {
@@ -570,7 +570,7 @@ bool route_wants_m_major_scales(bool is_fp8, const Route& r) {
 // partial sums (after it).
 size_t route_workspace_need(bool is_fp8, const Route& r, const GemmParams& p) {
   size_t need = r.splits > 1 ? (size_t)r.splits * (size_t)p.M * (size_t)p.N * 4u : 0;
-  if (!p.ue8m0 && route_wants_m_major_scales(is_fp8, r) && !fp8_scales_conform(p)) need += scale_relayout_bytes(p.M, p.K);
+  if (!p.ue8m0 && !p.row_scale && route_wants_m_major_scales(is_fp8, r) && !fp8_scales_conform(p)) need += scale_relayout_bytes(p.M, p.K);
   return need;
 }
 
@@ -594,7 +594,7 @@ int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipSt
                   "%s: workspace must be 16-byte aligned", what);
     p.ws = workspace;
   }
-  if (!p.ue8m0 && route_wants_m_major_scales(IS_FP8, r) && !fp8_scales_conform(p)) {
+  if (!p.ue8m0 && !p.row_scale && route_wants_m_major_scales(IS_FP8, r) && !fp8_scales_conform(p)) {
     float* dst = static_cast<float*>(workspace);
     const int64_t ld = (p.M + 3) & ~3;
     hipLaunchKernelGGL(relayout_scales_kernel, dim3((unsigned)((p.M + 31) / 32), (unsigned)((p.kb_total + 31) / 32)), dim3(256), 0,
@@ -619,7 +619,7 @@ int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipSt
       }
       break;
     case RK_DMA3:
-      if constexpr (IS_FP8) rc = p.ue8m0 ? launch_fp8_dma3_ue8m0(p, r.bm, r.bn, stream, what) : launch_fp8_dma3(p, r.bm, r.bn, stream, what);
+      if constexpr (IS_FP8) rc = p.ue8m0 ? launch_fp8_dma3_ue8m0(p, r.bm, r.bn, stream, what) : p.row_scale ? launch_fp8_dma3_unit(p, r.bm, r.bn, stream, what) : launch_fp8_dma3(p, r.bm, r.bn, stream, what);
       else rc = launch_int8_dma3(p, r.bm, r.bn, stream, what);
       break;
     case RK_PINGPONG: return IS_FP8 ? launch_fp8_pp(p, stream, what) : launch_int8_pp(p, stream, what);
@@ -983,6 +983,7 @@ extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa
   p.bias = bias;
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
   const Route r = choose_route(true, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  if (r.kernel == RK_DMA3) p.row_scale = sa;  // mid M: no scales in the K loop, both in the epilogue (or the reduce)
   if (r.kernel == RK_PINGPONG && K % KSTEP == 0) {
     // large M: accumulate in the MFMA with unit scales, apply both scales once in the epilogue (the reference's order)
     p.row_scale = sa;
