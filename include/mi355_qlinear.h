@@ -333,6 +333,11 @@ int mi355_block_dequant_fp8(const void* q, const float* s, void* out, int out_dt
  */
 int mi355_silu_mul_group_quant_fp8(const void* x, int x_dtype, void* q, void* s_words, int64_t E, int64_t T, int64_t H,
                                    const int32_t* masked_m, int64_t s_expert_stride, int64_t s_k_stride, void* stream);
+/* The same, and codes and scale words of tokens t >= masked_m[e] are written as zeros: what the reference's
+ * _per_token_group_quant_8bit_fuse_silu_and_mul (python/sglang/srt/layers/quantization/fp8_kernel.py:325-397) returns, whose
+ * outputs start as zeros. */
+int mi355_silu_mul_group_quant_fp8_zero_rest(const void* x, int x_dtype, void* q, void* s_words, int64_t E, int64_t T, int64_t H,
+                                             const int32_t* masked_m, int64_t s_expert_stride, int64_t s_k_stride, void* stream);
 
 /*
  * Per-tensor FP8 activation quantization: ONE fp32 scale for the whole tensor, q = e4m3fn(clamp(x * (1 / scale))).

@@ -50,6 +50,7 @@ EXPORTS = (
     "mi355_row_group_quant_fp8",
     "mi355_per_tensor_quant_fp8",
     "mi355_silu_mul_group_quant_fp8",
+    "mi355_silu_mul_group_quant_fp8_zero_rest",
     "mi355_block_cast_to_fp8",
     "mi355_block_dequant_fp8",
     "mi355_fp8_scaled_mm_workspace_bytes",
@@ -141,8 +142,9 @@ def lib() -> ctypes.CDLL:
     L.mi355_row_group_quant_fp8.restype = i32
     L.mi355_per_tensor_quant_fp8.argtypes = [vp, i32, vp, vp, i64, i32, vp, i64, vp]
     L.mi355_per_tensor_quant_fp8.restype = i32
-    L.mi355_silu_mul_group_quant_fp8.argtypes = [vp, i32, vp, vp, i64, i64, i64, vp, i64, i64, vp]
-    L.mi355_silu_mul_group_quant_fp8.restype = i32
+    for fn in (L.mi355_silu_mul_group_quant_fp8, L.mi355_silu_mul_group_quant_fp8_zero_rest):
+        fn.argtypes = [vp, i32, vp, vp, i64, i64, i64, vp, i64, i64, vp]
+        fn.restype = i32
     L.mi355_block_cast_to_fp8.argtypes = [vp, i32, vp, vp, i64, i64, vp]
     L.mi355_block_cast_to_fp8.restype = i32
     L.mi355_block_dequant_fp8.argtypes = [vp, vp, vp, i32, i64, i64, vp]

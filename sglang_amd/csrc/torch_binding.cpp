@@ -756,6 +756,29 @@ std::optional<Quantized> try_group_quant(const Tensor& x, int64_t group, double 
   return r;
 }
 
+// fp8_kernel._per_token_group_quant_8bit_fuse_silu_and_mul: x [T, 2H], or [E, T, 2H] with masked_m; rows past masked_m are zeros
+std::optional<Quantized> try_silu_quant(const Tensor& x, const OptTensor& masked_m) {
+  const bool masked = given(masked_m);
+  if (!x.is_cuda() || x.dim() != (masked ? 3 : 2) || !x.is_contiguous() || x.numel() == 0 || !is_16bit(x.scalar_type())) return std::nullopt;
+  const int64_t E = masked ? x.size(0) : 1, T = x.size(-2), H = x.size(-1) / 2;
+  if (x.size(-1) % 256 != 0) return std::nullopt;
+  if (masked && !(masked_m->is_cuda() && masked_m->scalar_type() == ScalarType::Int && masked_m->numel() == E && masked_m->is_contiguous()))
+    return std::nullopt;
+  const int64_t words = (H / 128 + 3) / 4, pitch = (T + 3) / 4 * 4;
+  Quantized r;
+  if (masked) {
+    r.q = new_tensor({E, T, H}, FP8, x);
+    r.s = new_tensor({E, words, pitch}, ScalarType::Int, x).as_strided({E, T, words}, {words * pitch, 1, pitch});
+  } else {
+    r.q = new_tensor({T, H}, FP8, x);
+    r.s = new_tensor({words, pitch}, ScalarType::Int, x).as_strided({T, words}, {1, pitch});
+  }
+  check(mi355_silu_mul_group_quant_fp8_zero_rest(x.const_data_ptr(), dtype_code(x.scalar_type()), r.q.data_ptr(), r.s.data_ptr(), E, T, H,
+                                                 static_cast<const int32_t*>(data_or_null(masked_m)), masked ? words * pitch : 0, pitch,
+                                                 current_stream()));
+  return r;
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(sgl_kernel, CUDA, m) {
@@ -931,6 +954,7 @@ PyMethodDef METHODS[] = {
     TRY("try_int8_linear", try_int8_linear, -1),
     TRY("try_token_linear", try_token_linear, -1),
     TRY("try_group_quant", try_group_quant, -1),
+    TRY("try_silu_quant", try_silu_quant, -1),
     {"env_flag", &env_flag, METH_O, nullptr},
     {"set_error_class", &set_error_class, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},

@@ -146,6 +146,10 @@ def _per_token_group_quant_8bit_fuse_silu_and_mul(
     assert scale_tma_aligned
     assert scale_ue8m0
     assert group_size == 128
+    if dst_dtype == fp8_dtype:
+        out = _native.try_silu_quant(x, masked_m)
+        if out is not None:
+            return out
     out_shape = (*x.shape[:-1], x.shape[-1] // 2)
     output = torch.zeros(out_shape, device=x.device, dtype=dst_dtype)
     output_scale = create_per_token_group_quant_fp8_output_scale(
@@ -204,7 +208,12 @@ def sglang_per_token_group_quant_fp8(
     """fp8_kernel.py:477-527: allocate outputs, then ``sgl_per_token_group_quant_8bit``."""
     if enable_v2 is None:
         enable_v2 = _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
-    if not fuse_silu_and_mul and masked_m is None:
+    if fuse_silu_and_mul:
+        if (enable_v2 and group_size == 128 and abs(1e-10 - eps) < 1e-13 and column_major_scales and scale_tma_aligned and scale_ue8m0):
+            out = _native.try_silu_quant(x, masked_m)
+            if out is not None:
+                return out
+    elif masked_m is None:
         out = _native.try_group_quant(x, group_size, eps, fp8_dtype, column_major_scales, scale_tma_aligned, scale_ue8m0, False, enable_v2)
         if out is not None:
             return out
