@@ -374,11 +374,12 @@ int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const flo
  *          GEMM and `output += bias`.  The activation is quantized with q = x / s (s = max(amax, 1e-10) / 448) into the
  *          workspace, with M-major scales, and the bias is added in fp32 in the GEMM epilogue (the reference adds it
  *          after rounding the GEMM result to the output type).  At decode sizes (M <= 16, 16-bit x, N % 128 == 0) there
- *          is no quantizer launch where that is the faster way: the GEMM kernel quantizes the tokens itself (the streaming
- *          kernel in its prologue, the mid-M kernel by producer waves), with the same arithmetic, and the result is
- *          bit-identical to the two-step sequence.
+ *          is no quantizer launch where that is the faster way: the GEMM kernel quantizes the tokens itself (the wave-split
+ *          and streaming kernels in their prologues, the mid-M kernel by producer waves), with the same arithmetic; the result
+ *          is bit-identical to the two-step sequence where the GEMM alone takes the same kernel.
  *          mi355_fp8_block_linear_plan (host only, dense 16-byte aligned operands assumed) writes the GEMM's plan in the
- *          format of mi355_fp8_blockwise_mm_plan followed by quantizer=fused|launch.
+ *          format of mi355_fp8_blockwise_mm_plan followed by quantizer=fused|launch, and by wavesplit_waves=W where the
+ *          wave-split kernel with W waves and its own quantizer runs in place of that plan.
  *   x [M, K] contiguous F32/F16/BF16, K % 128 == 0; w [N, K] e4m3fn row stride ldw; w_scale element (nb, kb) at
  *   w_scale[nb * ws_sn + kb * ws_sk]; bias NULL or [N] in the output dtype; out [M, N] BF16/F16 row stride ldo.
  *   workspace: mi355_fp8_block_linear_workspace_bytes(M, N, K) bytes, 256-byte aligned.
@@ -389,7 +390,7 @@ int mi355_fp8_block_linear(const void* x, int x_dtype, const void* w, const floa
                            int64_t ldo, void* workspace, size_t workspace_bytes, void* stream);
 /* The same with the quantizer's arithmetic chosen: MI355_QUANT_DIV as above (fp8_utils.py:201-203, the M-major-scale path),
  * MI355_QUANT_RCP for q = x * (1 / s), which is what triton_w8a8_block_fp8_linear's quantizer computes (fp8_utils.py:293-295,
- * fp8_kernel.py:156-158).  Either way the result is bit-identical to that wrapper's quantizer followed by the blockwise GEMM. */
+ * fp8_kernel.py:156-158).  Codes and scales are bit-identical to that wrapper's quantizer either way. */
 int mi355_fp8_block_linear_mode(const void* x, int x_dtype, int quant_mode, const void* w, const float* w_scale, int64_t ws_sn,
                                 int64_t ws_sk, const void* bias, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
                                 int64_t ldw, int64_t ldo, void* workspace, size_t workspace_bytes, void* stream);

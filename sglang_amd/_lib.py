@@ -200,7 +200,8 @@ def gemm_plan(kind: str, M: int, N: int, K: int, aligned: bool = True) -> dict:
 
 def block_linear_plan(M: int, N: int, K: int) -> dict:
     """Plan of the one-call block-FP8 linear: `gemm_plan`'s keys plus "quantizer": "fused" (the GEMM kernel quantizes the
-    tokens in its prologue) or "launch" (a quantizer launch in front of the GEMM)."""
+    tokens in its prologue) or "launch" (a quantizer launch in front of the GEMM); with "wavesplit_waves" where the wave-split
+    kernel of that many waves, with its own quantizer, runs instead."""
     buf = ctypes.create_string_buffer(256)
     check(lib().mi355_fp8_block_linear_plan(M, N, K, buf, len(buf)))
     out = {}

@@ -442,6 +442,11 @@ bool wavesplit_two_tiles(bool is_fp8, int64_t M, int64_t N, int64_t K);  // 32 c
 bool wavesplit_supported(int64_t M, int64_t N, int64_t K);
 int launch_fp8_wavesplit(GemmParams& p, hipStream_t stream, const char* what);
 int launch_int8_wavesplit(GemmParams& p, hipStream_t stream, const char* what);
+// The same with a quantizer for the tokens inside (p.x16 / p.ldx / p.x_dtype, p.x_by_reciprocal; p.a and p.sa are not read):
+// no quantizer launch.  For few tokens, see wavesplit_quant_fits.
+enum class WavesplitQuant { BLOCK_F32, BLOCK_UE8M0, TOKEN_FP8, TOKEN_INT8 };
+bool wavesplit_quant_fits(int64_t M, int64_t K);
+int launch_wavesplit_quant(GemmParams& p, WavesplitQuant kind, hipStream_t stream, const char* what);
 // The FP8 kernel with packed power-of-two scales on both operands, applied by the MFMA (p.sa / p.sb point to the words,
 // p.sa_sk / p.sb_sn / p.sb_sk are word strides; see decode_wavesplit_kernel).
 int launch_fp8_wavesplit_ue8m0(GemmParams& p, hipStream_t stream, const char* what);

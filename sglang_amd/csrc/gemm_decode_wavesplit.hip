@@ -33,19 +33,78 @@ __device__ __forceinline__ v8i as_v8i(const Frag& f) {
   return v8i{(int)f.lo.x, (int)f.lo.y, (int)f.lo.z, (int)f.lo.w, (int)f.hi.x, (int)f.hi.y, (int)f.hi.z, (int)f.hi.w};
 }
 
+// Where the tokens come from.
+enum TokenQuant {
+  TQ_NONE,   // codes p.a and scales p.sa
+  TQ_GROUP,  // unquantized (p.x16): quantized here per 1 x 128 group, fp32 scales, or exponents where UE8M0
+  TQ_ROW,    // unquantized: quantized here per token
+};
+// Fused quantizer (TQ_GROUP / TQ_ROW): before its K loop the workgroup quantizes ALL of the M x K tokens into LDS, with the
+// arithmetic of the quantizer kernels, and takes its token fragments from there.  Every workgroup repeats that work, so it
+// pays for few tokens only: at most WS_QUANT_VECTORS 16-byte pieces per thread (K = 7168 with eight waves: five tokens), about
+// 1 us, most of it under the latency of the weight blocks requested just before; the launch it replaces costs 2.4 us on the
+// GPU and 2.7 us on the host.
+constexpr int WS_QUANT_VECTORS = 10;
+
+__host__ __device__ constexpr int ws_scale_bytes(bool per_group, int M, int kb_total) { return ((per_group ? M * kb_total * 4 : 64) + 15) & ~15; }
+
+template <bool F8>
+__device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, int x_dtype, float mul) {  // per_token_quant.hip, emit_vector
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu);
+    f[2 * i + 1] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16);
+  }
+  uint32_t out[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if constexpr (F8) {
+      float t[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) t[b] = fmaxf(fminf(f[4 * j + b] * mul, 448.0f), -448.0f);
+      int c = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
+      out[j] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c, true);
+    } else {
+      out[j] = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) out[j] |= ((uint32_t)(int)roundf(f[4 * j + b] * mul) & 0xffu) << (8 * b);
+    }
+  }
+  return u32x2{out[0], out[1]};
+}
+__device__ __forceinline__ float amax8(const u32x4& raw, int x_dtype) {
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m = fmaxf(m, fabsf(x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu)));
+    m = fmaxf(m, fabsf(x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16)));
+  }
+  return m;
+}
+
 // UE8M0 (FP8 only): p.sa / p.sb point to 32-bit words of four exponent bytes (token words M-major: word (kb >> 2) * sa_sk + m;
 // weight words one row per weight row: (kb >> 2) * sb_sk + n * sb_sn, constant over a 128-row block) and the MFMA applies
 // them itself (v_mfma_scale_f32_16x16x128_f8f6f4: the weight row's byte with the A operand, the token's with the B
 // operand), accumulating in place: no scale arithmetic, no expansion of the exponents to fp32 in front of the GEMM.
 // CT: MFMA channel tiles per workgroup (16 or 32 channels).  With two, a block's token fragment is fetched once for both:
 // the tokens' share of what a workgroup pulls from L2 halves, which matters from about five tokens on.
-template <bool IS_FP8, int W, int KBW, bool UE8M0 = false, int CT = 1>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 ? 4 : 5))) void decode_wavesplit_kernel(const GemmParams p) {
+template <bool IS_FP8, int W, int KBW, bool UE8M0 = false, int CT = 1, TokenQuant TQ = TQ_NONE, int NV = 2>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu((CT == 2 ? 4 : 5) - (TQ != TQ_NONE)))) void decode_wavesplit_kernel(const GemmParams p) {
   static_assert(IS_FP8 || !UE8M0, "exponent scales belong to the FP8 path");
   static_assert(CT == 1 || CT == 2, "one or two channel tiles");
   using AccT = typename std::conditional<IS_FP8, float, int>::type;
   typedef AccT acc4 __attribute__((ext_vector_type(4)));
   __shared__ acc4 red[W][CT][64];
+  __shared__ float row_max[TQ == TQ_ROW ? 16 : 1];
+  // fused quantizer: the token scales (one per token, or per token and K block), then the codes, rows 16 bytes longer than K so
+  // that a fragment's rows do not share banks
+  extern __shared__ __attribute__((aligned(16))) uint8_t ws_dynamic[];
+  float* token_scale = reinterpret_cast<float*>(ws_dynamic);
+  const int code_pitch = p.K + 16;
+  uint8_t* codes = ws_dynamic + ws_scale_bytes(TQ == TQ_GROUP, p.M, p.kb_total);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, q = lane >> 4;
@@ -54,7 +113,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
   // operand layout of the 16 x 16 x 128 MFMA: lane (row l16, quarter q) holds bytes [16 q, +16) and [64 + 16 q, +16) of the row's block
   const uint8_t* wrow = p.b + (int64_t)(n0 + l16) * p.ldb + q * 16;
   const uint8_t* trow = p.a + (int64_t)tok * p.lda + q * 16;
-  const float* sa_row = IS_FP8 ? p.sa + (int64_t)tok * p.sa_sm : nullptr;
+  const float* sa_row = IS_FP8 && TQ == TQ_NONE ? p.sa + (int64_t)tok * p.sa_sm : nullptr;
   // wave-uniform, read through the constant address space: scalar loads, which the vector-memory counter does not see
   const cfloat_ptr sb_row = (cfloat_ptr)(IS_FP8 ? p.sb + (int64_t)(UE8M0 ? n0 : (n0 >> 7)) * p.sb_sn : nullptr);
 
@@ -69,12 +128,28 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
   // "everything but the newest block" and the ring runs empty once per turn.  A slot's registers are outputs of its request
   // and in-out operands of its wait, so no compiler-generated instruction touches them in between; vector loads complete in
   // order, so "at most (KBW - 1) blocks' loads outstanding" means the oldest slot has landed.
-  constexpr int LOADS = 2 * CT + 2 + (IS_FP8 ? 1 : 0);  // per block: the halves of the weight and token fragments, the token scale (word)
+  // loads per block: the halves of the weight and token fragments, the token scale (word); fused: of the weight only
+  constexpr int LOADS = TQ != TQ_NONE ? 2 * CT : 2 * CT + 2 + (IS_FP8 ? 1 : 0);
   Frag wf[KBW][CT], tf[KBW];
   float sav[KBW], sbv[KBW];
   auto request = [&](int j, int i) {
     const int kc = min(i * W + wave, p.kb_total - 1);  // wave-uniform
     const uint8_t* wp = wrow + (int64_t)kc * KSTEP;
+    if constexpr (TQ != TQ_NONE) {
+      asm volatile("global_load_dwordx4 %0, %2, off\n\tglobal_load_dwordx4 %1, %2, off offset:64"
+                   : "=&v"(wf[j][0].lo), "=&v"(wf[j][0].hi)
+                   : "v"(wp)
+                   : "memory");
+      if constexpr (CT == 2) {
+        const uint8_t* wp1 = wp + 16 * p.ldb;
+        asm volatile("global_load_dwordx4 %0, %2, off\n\tglobal_load_dwordx4 %1, %2, off offset:64"
+                     : "=&v"(wf[j][1].lo), "=&v"(wf[j][1].hi)
+                     : "v"(wp1)
+                     : "memory");
+      }
+      if constexpr (IS_FP8 && TQ == TQ_GROUP) sbv[j] = sb_row[(int64_t)(UE8M0 ? (kc >> 2) : kc) * p.sb_sk];
+      return;
+    }
     const uint8_t* tp = trow + (int64_t)kc * KSTEP;
     asm volatile(
         "global_load_dwordx4 %0, %4, off\n\tglobal_load_dwordx4 %1, %4, off offset:64\n\t"
@@ -99,7 +174,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
   // waits until at most `behind` blocks requested after slot j's are still outstanding: slot j has landed
   auto await = [&](int j, int behind) {  // `behind` is a constant at every call; the switch folds away
 #define MI355_WS_AWAIT(NBLK)                                                                                                     \
-  if constexpr (IS_FP8 && CT == 2)                                                                                               \
+  if constexpr (TQ != TQ_NONE && CT == 2)                                                                                        \
+    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(wf[j][0].lo), "+v"(wf[j][0].hi), "+v"(wf[j][1].lo), "+v"(wf[j][1].hi) : "n"((NBLK)*LOADS)); \
+  else if constexpr (TQ != TQ_NONE)                                                                                              \
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(wf[j][0].lo), "+v"(wf[j][0].hi) : "n"((NBLK)*LOADS));                               \
+  else if constexpr (IS_FP8 && CT == 2)                                                                                               \
     asm volatile("s_waitcnt vmcnt(%7)" : "+v"(wf[j][0].lo), "+v"(wf[j][0].hi), "+v"(wf[j][1].lo), "+v"(wf[j][1].hi), "+v"(tf[j].lo), "+v"(tf[j].hi), "+v"(sav[j]) : "n"((NBLK)*LOADS)); \
   else if constexpr (IS_FP8)                                                                                                     \
     asm volatile("s_waitcnt vmcnt(%5)" : "+v"(wf[j][0].lo), "+v"(wf[j][0].hi), "+v"(tf[j].lo), "+v"(tf[j].hi), "+v"(sav[j]) : "n"((NBLK)*LOADS)); \
@@ -118,7 +197,23 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
   auto multiply = [&](int j, int i) {
     const int kb = i * W + wave;
     const bool valid = kb < p.kb_total;
-    if constexpr (UE8M0) {
+    if constexpr (TQ != TQ_NONE) {  // the block's token fragment and scale out of LDS
+      const int kc = min(kb, p.kb_total - 1);
+      const uint8_t* src = codes + tok * code_pitch + kc * KSTEP + q * 16;
+      tf[j].lo = *reinterpret_cast<const u32x4*>(src);
+      tf[j].hi = *reinterpret_cast<const u32x4*>(src + 64);
+      if constexpr (TQ == TQ_GROUP) sav[j] = token_scale[tok * p.kb_total + kc];
+      else if constexpr (IS_FP8) sav[j] = token_scale[tok], sbv[j] = 1.0f;
+    }
+    if constexpr (UE8M0 && TQ != TQ_NONE) {
+      const int ea = in_vgpr((int)((__float_as_uint(sbv[j]) >> (8 * (min(kb, p.kb_total - 1) & 3))) & 0xffu)), eb = (int)__float_as_uint(sav[j]);
+      const u32x4 z = {0u, 0u, 0u, 0u};
+      Frag t = tf[j];
+      if (!valid) t.lo = z, t.hi = z;
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        acc[c] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(wf[j][c]), as_v8i(t), acc[c], 0, 0, 0, ea, 0, eb);
+    } else if constexpr (UE8M0) {
       const int shift = 8 * (min(kb, p.kb_total - 1) & 3);
       const int ea = in_vgpr((int)((__float_as_uint(sbv[j]) >> shift) & 0xffu)), eb = (int)((__float_as_uint(sav[j]) >> shift) & 0xffu);
       const u32x4 z = {0u, 0u, 0u, 0u};
@@ -150,8 +245,94 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
     }
   };
   const int blocks = (p.kb_total + W * KBW - 1) / (W * KBW) * KBW;  // per wave, padded to whole turns of the ring
+  if constexpr (TQ == TQ_NONE) {
 #pragma unroll
-  for (int j = 0; j < KBW; ++j) request(j, j);
+    for (int j = 0; j < KBW; ++j) request(j, j);
+  } else {
+    // ---- the tokens, quantized into LDS.  Piece c (16 bytes of input, 8 values) of the M x K / 8 goes to thread c % (64 W); 16
+    //      consecutive pieces are a group, in the 16 lanes of a DPP row.  The raw values are requested first, then the first
+    //      weight blocks, so that these are in flight while the tokens are quantized.
+    constexpr int NT = 64 * W;
+    const int per_row = p.K >> 3, total = p.M * per_row;
+    const uint16_t* x = reinterpret_cast<const uint16_t*>(p.x16);
+    // (NV pieces per thread, all of them always requested: a load under a condition could leave the compiler a copy to make
+    // while it is in flight; pieces past the end repeat the last one and are dropped)
+    u32x4 raw[NV];
+    int at[NV];  // the piece's row in the high half, its place in the row in the low one
+    auto row_of = [&](int i) { return at[i] >> 16; };
+    auto col_of = [&](int i) { return at[i] & 0xffff; };
+    int r = 0, c = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      while (c >= per_row && r < p.M) c -= per_row, ++r;
+      at[i] = (r << 16) | (c & 0xffff);
+      const uint16_t* src = x + (int64_t)min(r, p.M - 1) * p.ldx + (r < p.M ? c : per_row - 1) * 8;
+      asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(raw[i]) : "v"(src) : "memory");
+      c += NT;
+    }
+    if constexpr (TQ == TQ_ROW) {
+      if (threadIdx.x < 16) reinterpret_cast<uint32_t*>(row_max)[threadIdx.x] = __float_as_uint(IS_FP8 ? 0.f : 1e-10f);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+#pragma unroll
+    for (int j = 0; j < KBW; ++j) request(j, j);
+    // the raw values have landed, the weight blocks may be in flight
+    static_assert(NV == 2 || NV == 4 || NV == WS_QUANT_VECTORS, "the wait names every piece");
+    if constexpr (NV == 2)
+      asm volatile("s_waitcnt vmcnt(%2)" : "+v"(raw[0]), "+v"(raw[1]) : "n"(KBW * LOADS));
+    else if constexpr (NV == 4)
+      asm volatile("s_waitcnt vmcnt(%4)" : "+v"(raw[0]), "+v"(raw[1]), "+v"(raw[2]), "+v"(raw[3]) : "n"(KBW * LOADS));
+    else
+      asm volatile("s_waitcnt vmcnt(%10)"
+                   : "+v"(raw[0]), "+v"(raw[1]), "+v"(raw[2]), "+v"(raw[3]), "+v"(raw[4]), "+v"(raw[5]), "+v"(raw[6]), "+v"(raw[7]),
+                     "+v"(raw[8]), "+v"(raw[9])
+                   : "n"(KBW * LOADS));
+    if constexpr (TQ == TQ_ROW) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        if (i * NT < total) {
+          const float m = row16_max(amax8(raw[i], p.x_dtype));
+          if ((lane & 15) == 0 && row_of(i) < p.M) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (threadIdx.x < 16) {
+        const float m = row_max[threadIdx.x];
+        token_scale[threadIdx.x] = IS_FP8 ? m / 448.0f : m / 127.0f;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      __builtin_amdgcn_sched_barrier(0);  // one piece's arithmetic at a time: no register may be spilled while loads are in flight
+      if (i * NT < total) {
+        u32x2 q8;
+        if constexpr (TQ == TQ_ROW) {
+          const float m = row_max[min(row_of(i), 15)];
+          float mul;
+          if constexpr (IS_FP8) {
+            const float sc = m / 448.0f;
+            mul = sc == 0.f ? 0.f : 1.0f / sc;
+          } else {
+            mul = 127.0f / m;
+          }
+          q8 = codes_of_row<IS_FP8>(raw[i], p.x_dtype, mul);
+        } else if constexpr (UE8M0) {
+          // q = x * 2^-e with e = ceil(log2(max(amax, 1e-10) / 448)): group_quant.hip, MUL with packed exponents
+          const float m = row16_max(fmaxf(amax8(raw[i], p.x_dtype), 1e-10f));
+          const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
+          const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
+          q8 = codes_of_row<true>(raw[i], p.x_dtype, __uint_as_float((uint32_t)(127 - e) << 23));
+          if ((lane & 15) == 0 && row_of(i) < p.M) reinterpret_cast<uint32_t*>(token_scale)[row_of(i) * p.kb_total + (col_of(i) >> 4)] = (uint32_t)(e + 127);
+        } else {
+          float sc;
+          q8 = quantize_group_lane(raw[i], p.x_dtype, p.x_by_reciprocal != 0, sc);
+          if ((lane & 15) == 0 && row_of(i) < p.M) token_scale[row_of(i) * p.kb_total + (col_of(i) >> 4)] = sc;
+        }
+        if (row_of(i) < p.M) *reinterpret_cast<u32x2*>(codes + row_of(i) * code_pitch + col_of(i) * 8) = q8;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
   // the fences keep the order "await and multiply slot j, request it again"
   int i0 = 0;
   for (; i0 + KBW < blocks; i0 += KBW) {
@@ -211,7 +392,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
 #pragma unroll
       for (int v = 0; v < 4; ++v) o[v] = acc[c][v];
     } else {
-      const float sa_m = p.sa[l16];
+      const float sa_m = TQ == TQ_NONE ? p.sa[l16] : token_scale[l16];
       float r4[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -228,21 +409,30 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(CT == 2 
   }
 }
 
-template <bool IS_FP8, int W, int KBW, bool UE8M0 = false, int CT = 1>
+template <bool IS_FP8, int W, int KBW, bool UE8M0 = false, int CT = 1, TokenQuant TQ = TQ_NONE>
 int launch_variant(const GemmParams& p, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT>), dim3((unsigned)(p.N / (16 * CT))), dim3(64 * W), 0, stream, p);
+  const dim3 grid((unsigned)(p.N / (16 * CT))), block(64 * W);
+  if constexpr (TQ == TQ_NONE) {
+    hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT>), grid, block, 0, stream, p);
+  } else {
+    const size_t lds = (size_t)ws_scale_bytes(TQ == TQ_GROUP, p.M, p.kb_total) + (size_t)p.M * (p.K + 16);
+    const int64_t pieces = (int64_t)p.M * p.K / 8;  // over 64 W threads, 2, 4 or WS_QUANT_VECTORS each
+    if (pieces <= 2 * 64 * W) hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, 2>), grid, block, lds, stream, p);
+    else if (pieces <= 4 * 64 * W) hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, 4>), grid, block, lds, stream, p);
+    else hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, WS_QUANT_VECTORS>), grid, block, lds, stream, p);
+  }
   return check_launch(what);
 }
 
-template <bool IS_FP8, bool UE8M0 = false>
+template <bool IS_FP8, bool UE8M0 = false, TokenQuant TQ = TQ_NONE>
 int launch_wavesplit(GemmParams& p, hipStream_t stream, const char* what) {
   p.splits = 1;
   p.tiles_m = 1;
   p.tiles_n = p.N / 16;
   const WavesplitShape s = wavesplit_shape(p.K);
   if (wavesplit_two_tiles(IS_FP8, p.M, p.N, p.K))
-    return s.waves == 4 ? launch_variant<IS_FP8, 4, 4, UE8M0, 2>(p, stream, what) : launch_variant<IS_FP8, 8, 4, UE8M0, 2>(p, stream, what);
-  return s.waves == 4 ? launch_variant<IS_FP8, 4, 4, UE8M0>(p, stream, what) : launch_variant<IS_FP8, 8, 4, UE8M0>(p, stream, what);
+    return s.waves == 4 ? launch_variant<IS_FP8, 4, 4, UE8M0, 2, TQ>(p, stream, what) : launch_variant<IS_FP8, 8, 4, UE8M0, 2, TQ>(p, stream, what);
+  return s.waves == 4 ? launch_variant<IS_FP8, 4, 4, UE8M0, 1, TQ>(p, stream, what) : launch_variant<IS_FP8, 8, 4, UE8M0, 1, TQ>(p, stream, what);
 }
 
 }  // namespace
@@ -271,5 +461,20 @@ bool wavesplit_supported(int64_t M, int64_t N, int64_t K) { return M >= 1 && M <
 int launch_fp8_wavesplit(GemmParams& p, hipStream_t stream, const char* what) { return launch_wavesplit<true>(p, stream, what); }
 int launch_int8_wavesplit(GemmParams& p, hipStream_t stream, const char* what) { return launch_wavesplit<false>(p, stream, what); }
 int launch_fp8_wavesplit_ue8m0(GemmParams& p, hipStream_t stream, const char* what) { return launch_wavesplit<true, true>(p, stream, what); }
+
+// Unquantized tokens (p.x16, p.ldx, p.x_dtype; 16-byte aligned rows): quantized in the kernel.
+bool wavesplit_quant_fits(int64_t M, int64_t K) { return M * K <= (int64_t)wavesplit_shape(K).waves * 64 * WS_QUANT_VECTORS * 8; }
+int launch_wavesplit_quant(GemmParams& p, WavesplitQuant kind, hipStream_t stream, const char* what) {
+  if (p.x16 == nullptr || p.M > 16 || !wavesplit_quant_fits(p.M, p.K)) {
+    set_error("%s: the fused quantizer of the wave-split kernel takes few unquantized tokens", what);
+    return MI355_ERR_UNSUPPORTED;
+  }
+  switch (kind) {
+    case WavesplitQuant::BLOCK_F32: return launch_wavesplit<true, false, TQ_GROUP>(p, stream, what);
+    case WavesplitQuant::BLOCK_UE8M0: return launch_wavesplit<true, true, TQ_GROUP>(p, stream, what);
+    case WavesplitQuant::TOKEN_FP8: return launch_wavesplit<true, false, TQ_ROW>(p, stream, what);
+    default: return launch_wavesplit<false, false, TQ_ROW>(p, stream, what);
+  }
+}
 
 }  // namespace mi355

@@ -1018,6 +1018,44 @@ Route linear_producer_route(int64_t M, int64_t N, int64_t K, int64_t ldw) {
   return plain;
 }
 
+// The wave-split kernel quantizing the tokens itself (one launch) against the alternatives: a quantizer launch in front of the
+// GEMM's own plan, or, for the fp32-scaled block linear, the streaming or producer-wave kernel with its quantizer.  Every
+// workgroup quantizes all tokens, v = M K / 8 / threads pieces of 8 values per thread, so what it costs grows with v and with
+// the waves a SIMD has to run, x = v * max(1, workgroups * waves / 1024); what it saves is a launch, about 3.6 us.  GPU time of
+// one call in us, alternative / this:
+//   block  7168->576 M=1 9.3/5.8, 4 10.1/9.2;  7168->2048 M=1 8.7/6.7, 3 9.1/9.2, 4 9.3/10.0;  2048->7168 M=1 8.7/5.2, 8 10.6/8.1;
+//          4096->28672 M=1 28.0/22.2, 4 29.7/25.3, 5 29.6/31.6;  7168->36864 M=1 48.4/44.9, 2 48.4/47.5, 3 48.4/58.9
+//   UE8M0  4096->6144 M=1 10.3/7.3, 8 11.7/11.2, 10 11.9/12.4;  1536->24576 M=1 12.2/9.1, 12 13.6/12.3
+//   INT8   4096->6144 M=1 11.5/7.8, 5 12.2/11.8, 6 12.4/12.7;  2048->7168 M=5 8.8/8.3, 8 9.2/10.2;  4096->28672 M=2 25.7/23.2,
+//          3 25.8/27.0;  14336->4096 M=1 16.0/14.0
+//   token  4096->6144 M=1 11.1/7.7, 5 11.8/11.0;  2048->7168 M=6 8.1/7.8, 8 8.3/8.7;  7168->36864 M=2 53.1/48.8
+// The sums of FP8 products are those of the quantizer and GEMM entry points bit for bit only where the GEMM takes this kernel
+// too, so the per-token and packed-scale linears, which promise that, take it only there; the block linear promises the
+// tolerance at decode sizes; INT8 sums are exact.
+bool wavesplit_quant_preferred(WavesplitQuant kind, int64_t M, int64_t N, int64_t K, int64_t ldw) {
+  const bool is_fp8 = kind != WavesplitQuant::TOKEN_INT8;
+  if (!wavesplit_supported(M, N, K) || !wavesplit_quant_fits(M, K) || N * ldw >= (1ll << 32)) return false;
+  const double kb = (double)(K / KSTEP), waves = wavesplit_shape(K).waves;
+  const bool plain_wavesplit = choose_route(is_fp8, M, N, K, K, ldw, true).kernel == RK_WAVESPLIT;
+  if ((kind == WavesplitQuant::BLOCK_UE8M0 || kind == WavesplitQuant::TOKEN_FP8) && !plain_wavesplit) return false;
+  if (kb < route_constants().wavesplit_min_kblocks && (is_fp8 || N / 16 > 512)) return false;  // a block per wave: 512->32768 8.2 against 10.5
+  const double v = (double)(M * K) / (8.0 * 64.0 * waves);
+  const double workgroups = (double)N / (wavesplit_two_tiles(is_fp8, M, N, K) ? 32.0 : 16.0);
+  const double x = v * std::max(1.0, workgroups * waves / 1024.0);
+  if (v <= 4.0) return x <= 32.0;
+  const bool per_row = kind == WavesplitQuant::TOKEN_FP8 || kind == WavesplitQuant::TOKEN_INT8;
+  if (kind == WavesplitQuant::BLOCK_F32 && decode_supported(M, N, K) && kb > 40.0) return false;  // the streaming kernel's prologue quantizes less per workgroup
+  return x <= (waves == 4.0 ? (per_row ? 9.0 : 24.0) : (per_row ? 15.0 : 17.0));
+}
+bool wavesplit_quant_operands(const void* x, int x_dtype, const void* w, int64_t ldw) {
+  return x_dtype != MI355_F32 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
+}
+int run_wavesplit_quant(GemmParams& p, WavesplitQuant kind, const void* x, int x_dtype, void* stream, const char* what) {
+  p.x16 = x, p.ldx = p.K, p.x_dtype = x_dtype;
+  p.kb_total = p.K / KSTEP, p.splits = 1, p.kb_per_split = p.kb_total;
+  return launch_wavesplit_quant(p, kind, static_cast<hipStream_t>(stream), what);
+}
+
 bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
   const int plain = choose_route(true, M, N, K, K, ldw, true).kernel;
   if (plain == RK_DMA3) return false;  // the mid-M kernel at decode sizes beats the streaming kernel by more than a launch
@@ -1060,9 +1098,18 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   float* sa = reinterpret_cast<float*>(q + q_bytes);
   const int64_t pitch = (M + 3) & ~3ll;
   const size_t sa_bytes = align256((size_t)pitch * (size_t)(K / KSTEP) * 4u);
-  // Decode sizes: the GEMM kernel quantizes the tokens of each K range itself (same arithmetic), no quantizer launch -
-  // except where a quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
+  // Decode sizes: the GEMM kernel quantizes the tokens itself (same arithmetic), no quantizer launch - except where a
+  // quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
   const bool ptr_ok = x_dtype != MI355_F32 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
+  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, ldw)) {
+    GemmParams p;
+    bool empty;
+    const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, pitch, ws_sn, ws_sk, ldo, p, empty);
+    if (rc != MI355_OK || empty) return rc;
+    p.bias = bias;
+    p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
+    return run_wavesplit_quant(p, WavesplitQuant::BLOCK_F32, x, x_dtype, stream, what);
+  }
   if (ptr_ok && M <= 16) {
     const Route plain = linear_producer_route(M, N, K, ldw);
     if (plain.kernel == RK_DMA3) {  // one round of unsplit 64-token tiles: producer waves of that kernel quantize the tokens
@@ -1126,9 +1173,12 @@ extern "C" int mi355_fp8_block_linear_plan(int64_t M, int64_t N, int64_t K, char
   const bool producer = M <= 16 && plain.kernel == RK_DMA3;  // the mid-M kernel's producer waves quantize
   const bool fused = producer || (choose_route(true, M, N, K, K, K, true, true).kernel == RK_DECODE && fused_quant_preferred(M, N, K, K));
   const Route r = producer ? plain : choose_route(true, M, N, K, K, K, true, fused);
-  const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d quantizer=%s",
+  const bool wavesplit = wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, K);
+  char instead[32] = "";
+  if (wavesplit) snprintf(instead, sizeof instead, " wavesplit_waves=%d", wavesplit_shape(K).waves);
+  const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d quantizer=%s%s",
                          ROUTE_NAMES[r.kernel], r.bm, r.bn, r.splits, r.kb_per_split, r.groups_per_wg, (int)r.aligned,
-                         route_stages(true, r, M, N), fused ? "fused" : "launch");
+                         route_stages(true, r, M, N), fused ? "fused" : "launch", instead);
   MI355_REQUIRE(n > 0 && (size_t)n < buf_len, MI355_ERR_INVALID_ARGUMENT, "%s: buffer of %zu bytes is too small", what, buf_len);
   return MI355_OK;
 }
@@ -1193,8 +1243,6 @@ extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, cons
   const size_t q_bytes = align256((size_t)M * (size_t)K);
   float* sa = reinterpret_cast<float*>(q + q_bytes);
   const size_t sa_bytes = align256((size_t)M * 4u);
-  const int rc = mi355_per_token_quant_int8(x, x_dtype, q, sa, M, K, stream);
-  if (rc != MI355_OK) return rc;
   GemmParams p{};
   p.a = q;
   p.b = static_cast<const uint8_t*>(w);
@@ -1202,6 +1250,10 @@ extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, cons
   p.M = (int)M, p.N = (int)N, p.K = (int)K;
   p.lda = K, p.ldb = ldw, p.ldo = ldo;
   p.out_dtype = out_dtype;
+  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::TOKEN_INT8, M, N, K, ldw))
+    return run_wavesplit_quant(p, WavesplitQuant::TOKEN_INT8, x, x_dtype, stream, what);
+  const int rc = mi355_per_token_quant_int8(x, x_dtype, q, sa, M, K, stream);
+  if (rc != MI355_OK) return rc;
   return run_gemm<false>(p, q + q_bytes + sa_bytes, workspace_bytes_given - q_bytes - sa_bytes, static_cast<hipStream_t>(stream), what);
 }
 
@@ -1232,6 +1284,15 @@ extern "C" int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void
   const size_t q_bytes = align256((size_t)M * (size_t)K);
   float* sa = reinterpret_cast<float*>(q + q_bytes);
   const size_t sa_bytes = align256((size_t)M * 4u);
+  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::TOKEN_FP8, M, N, K, ldw)) {
+    GemmParams p;
+    bool empty;
+    // (the block scales are not read in this mode; they only have to satisfy the checks)
+    const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, 0, 0, 0, ldo, p, empty);
+    if (rc != MI355_OK || empty) return rc;
+    p.col_scale = w_scale, p.bias = bias;
+    return run_wavesplit_quant(p, WavesplitQuant::TOKEN_FP8, x, x_dtype, stream, what);
+  }
   const int rc = mi355_per_token_quant_fp8(x, x_dtype, q, sa, M, K, stream);
   if (rc != MI355_OK) return rc;
   return mi355_fp8_scaled_mm(q, w, sa, w_scale, bias, out, out_dtype, M, N, K, K, ldw, ldo, q + q_bytes + sa_bytes,
@@ -1269,6 +1330,15 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
   void* sa_words = q + q_bytes;
   const int64_t pitch = (M + 3) & ~3ll;
   const size_t sa_bytes = align256((size_t)pitch * (size_t)((K / KSTEP + 3) / 4) * 4u);
+  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw)) {
+    GemmParams p;
+    bool empty;
+    const float* words = static_cast<const float*>(sb_words);  // (strides of the packed words stand in for fp32 ones)
+    const int rc = fp8_mm_params(what, x, w, words, words, out, out_dtype, M, N, K, K, ldw, 1, pitch, sb_sn, sb_sk, ldo, p, empty);
+    if (rc != MI355_OK || empty) return rc;
+    p.bias = bias;
+    return run_wavesplit_quant(p, WavesplitQuant::BLOCK_UE8M0, x, x_dtype, stream, what);
+  }
   // q = x * (448 / amax) with the scale rounded up to a power of two: per_token_group_quant_8bit_v2.cu:77-78 with scale_ue8m0
   const int rc = mi355_group_quant_8bit(x, x_dtype, q, MI355_FP8_E4M3FN, sa_words, M, K, KSTEP, 1e-10f, -448.0f, 448.0f,
                                         MI355_QUANT_MUL, MI355_SCALE_UE8M0_PACKED, 0.0f, 1, pitch, stream);

@@ -1,0 +1,55 @@
+"""One-call linears whose wave-split decode kernel quantizes the tokens itself: at the steps of the pieces a thread quantizes
+(2, 4, 10), four and eight waves, one and two channel tiles, K blocks that do not fill the waves' turns, and just past the
+limit, where a quantizer launch stands in front of the GEMM again."""
+import pytest
+import torch
+
+from fp8_tolerance import check_fp8_gemm
+from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
+
+pytestmark = pytest.mark.gpu
+
+# pieces of 8 values per thread: M K / (8 * 64 * waves)
+SHAPES = [(1, 4096, 1152), (8, 144, 2048), (16, 4096, 1152), (2, 576, 4096), (3, 1040, 2176), (4, 512, 4096), (5, 512, 4096),
+          (10, 6144, 4096), (11, 512, 4096), (1, 512, 8320), (1, 272, 20480), (2, 40960, 4096), (5, 576, 7168)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fused_quantizer_of_the_wavesplit_kernel(gpu, oracle, M, N, K, dtype):
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import per_token_group_quant_fp8, sglang_per_token_group_quant_fp8, sglang_per_token_quant_fp8, w8a8_block_fp8_matmul
+    from sglang_amd.fp8_utils import requant_weight_ue8m0
+    from sglang_amd.int8_kernel import per_token_quant_int8
+
+    plan = _lib.block_linear_plan(M, N, K)
+    print(f"case M={M} N={N} K={K} {plan}", flush=True)
+    bits = lambda t: t.view(torch.int16)
+    x = make_activation(M, K, seed=M + N, dtype=dtype)
+    x[0, :128] = 0
+    if M > 2:
+        x[M - 1] = 0  # a token of zeros
+    xg = x.to(gpu)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).to(dtype).to(gpu)
+    w_q, w_s = make_fp8_weight(N, K, seed=K)
+    wg, sg = w_q.to(gpu), w_s.to(gpu)
+    for by_reciprocal in (False, True):
+        out = ops.block_fp8_linear(xg, wg, sg, None, dtype, by_reciprocal=by_reciprocal)
+        q, s = per_token_group_quant_fp8(xg, 128, column_major_scales=not by_reciprocal)
+        two = w8a8_block_fp8_matmul(q, wg, s, sg, [128, 128], dtype)
+        if "wavesplit_waves" in plan and _lib.gemm_plan("fp8", M, N, K)["kernel"] == "decode_wavesplit":
+            assert torch.equal(bits(out), bits(two))
+        if N <= 1040:
+            xq, xs = oracle.group_quant(x, 128, mode="rcp" if by_reciprocal else "div")
+            ref, mag = oracle.fp8_blockwise_mm(xq, w_q, xs, w_s, torch.float32, want_abs=True)
+            check_fp8_gemm(out, ref, mag, "block")
+    w2, words = requant_weight_ue8m0(wg, sg, [128, 128])
+    q, s = sglang_per_token_group_quant_fp8(xg, 128, column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=True)
+    assert torch.equal(bits(ops.block_fp8_linear_ue8m0(xg, w2, words, bias, dtype)), bits(ops.fp8_blockwise_mm_ue8m0(q, w2, s, words, dtype, bias)))
+    scale = torch.rand(N, generator=torch.Generator().manual_seed(K)).to(gpu) * 0.01 + 1e-3
+    q, s = sglang_per_token_quant_fp8(xg)
+    assert torch.equal(bits(ops.fp8_per_token_linear(xg, wg.t(), scale, bias, dtype)), bits(ops.fp8_scaled_mm(q, wg.t(), s, scale, dtype, bias)))
+    i_q, i_s = make_int8_weight(N, K, seed=K)
+    q, s = per_token_quant_int8(xg)
+    iw, isc = i_q.to(gpu).t(), i_s.to(gpu)
+    assert torch.equal(bits(ops.int8_linear(xg, iw, isc, bias, dtype)), bits(ops.int8_scaled_mm(q, iw, s, isc, dtype, bias)))
