@@ -1,0 +1,142 @@
+// Tokens quantized inside a GEMM kernel at decode sizes: the whole workgroup quantizes ALL of the M x K tokens into LDS before
+// its K loop, with the arithmetic of the quantizer kernels, and takes its token fragments from there.
+#pragma once
+
+#include "gemm_common.h"
+
+namespace mi355 {
+namespace {
+
+// Where the tokens come from.
+enum TokenQuant {
+  TQ_NONE,   // codes p.a and scales p.sa
+  TQ_GROUP,  // unquantized (p.x16): quantized here per 1 x 128 group, fp32 scales, or exponents where UE8M0
+  TQ_ROW,    // unquantized: quantized here per token
+};
+// Every workgroup repeats the quantizer's work, so it pays for few tokens only: at most WS_QUANT_VECTORS 16-byte pieces per
+// thread (K = 7168 with eight waves: five tokens), about 1 us, most of it under the latency of the weight blocks requested just
+// before; the launch it replaces costs 2.4 us on the GPU and 2.7 us on the host.
+constexpr int WS_QUANT_VECTORS = 10;
+
+__host__ __device__ constexpr int ws_scale_bytes(bool per_group, int M, int kb_total) { return ((per_group ? M * kb_total * 4 : 64) + 15) & ~15; }
+
+template <bool F8>
+__device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, int x_dtype, float mul) {  // per_token_quant.hip, emit_vector
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu);
+    f[2 * i + 1] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16);
+  }
+  uint32_t out[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if constexpr (F8) {
+      float t[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) t[b] = fmaxf(fminf(f[4 * j + b] * mul, 448.0f), -448.0f);
+      int c = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
+      out[j] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c, true);
+    } else {
+      out[j] = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) out[j] |= ((uint32_t)(int)roundf(f[4 * j + b] * mul) & 0xffu) << (8 * b);
+    }
+  }
+  return u32x2{out[0], out[1]};
+}
+__device__ __forceinline__ float amax8(const u32x4& raw, int x_dtype) {
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m = fmaxf(m, fabsf(x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu)));
+    m = fmaxf(m, fabsf(x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16)));
+  }
+  return m;
+}
+
+
+// Piece c (16 bytes of input, 8 values) of the M x K / 8 goes to thread c % NT; 16 consecutive pieces are a group, in the 16 lanes
+// of a DPP row.  Codes go to codes[row * (K + 16) + k] (rows 16 bytes longer than K, so that a fragment's rows do not share banks),
+// scales to token_scale (one per token, or per token and K block: row * kb_total + kb; exponents for UE8M0).  `request` is called
+// behind the loads of the raw values: it requests the first weight blocks and waits until only those are outstanding.  Ends with
+// a barrier that does not wait for them.
+template <bool IS_FP8, bool UE8M0, TokenQuant TQ, int NV, int NT, class Request>
+__device__ __forceinline__ void quantize_tokens(const GemmParams& p, uint8_t* codes, float* token_scale, float* row_max, Request request) {
+  const int lane = threadIdx.x & 63, code_pitch = p.K + 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int per_row = p.K >> 3, total = p.M * per_row;
+  const uint16_t* x = reinterpret_cast<const uint16_t*>(p.x16);
+  // (NV pieces per thread, all of them always requested: a load under a condition could leave the compiler a copy to make
+  // while it is in flight; pieces past the end repeat the last one and are dropped)
+  u32x4 raw[NV];
+  int at[NV];  // the piece's row in the high half, its place in the row in the low one
+  auto row_of = [&](int i) { return at[i] >> 16; };
+  auto col_of = [&](int i) { return at[i] & 0xffff; };
+  int r = 0, c = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    while (c >= per_row && r < p.M) c -= per_row, ++r;
+    at[i] = (r << 16) | (c & 0xffff);
+    const uint16_t* src = x + (int64_t)min(r, p.M - 1) * p.ldx + (r < p.M ? c : per_row - 1) * 8;
+    asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(raw[i]) : "v"(src) : "memory");
+    c += NT;
+  }
+  if constexpr (TQ == TQ_ROW) {
+    if (threadIdx.x < 16) reinterpret_cast<uint32_t*>(row_max)[threadIdx.x] = __float_as_uint(IS_FP8 ? 0.f : 1e-10f);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  request();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));  // landed
+  if constexpr (TQ == TQ_ROW) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if (i * NT + wave * 64 < total) {
+        const float m = row16_max(amax8(raw[i], p.x_dtype));
+        if ((lane & 15) == 0 && row_of(i) < p.M) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (threadIdx.x < 16) {
+      const float m = row_max[threadIdx.x];
+      token_scale[threadIdx.x] = IS_FP8 ? m / 448.0f : m / 127.0f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    __builtin_amdgcn_sched_barrier(0);  // one piece's arithmetic at a time: no register may be spilled while loads are in flight
+    if (i * NT + wave * 64 < total) {
+      u32x2 q8;
+      if constexpr (TQ == TQ_ROW) {
+        const float m = row_max[min(row_of(i), 15)];
+        float mul;
+        if constexpr (IS_FP8) {
+          const float sc = m / 448.0f;
+          mul = sc == 0.f ? 0.f : 1.0f / sc;
+        } else {
+          mul = 127.0f / m;
+        }
+        q8 = codes_of_row<IS_FP8>(raw[i], p.x_dtype, mul);
+      } else if constexpr (UE8M0) {
+        // q = x * 2^-e with e = ceil(log2(max(amax, 1e-10) / 448)): group_quant.hip, MUL with packed exponents
+        const float m = row16_max(fmaxf(amax8(raw[i], p.x_dtype), 1e-10f));
+        const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
+        const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
+        q8 = codes_of_row<true>(raw[i], p.x_dtype, __uint_as_float((uint32_t)(127 - e) << 23));
+        if ((lane & 15) == 0 && row_of(i) < p.M) reinterpret_cast<uint32_t*>(token_scale)[row_of(i) * p.kb_total + (col_of(i) >> 4)] = (uint32_t)(e + 127);
+      } else {
+        float sc;
+        q8 = quantize_group_lane(raw[i], p.x_dtype, p.x_by_reciprocal != 0, sc);
+        if ((lane & 15) == 0 && row_of(i) < p.M) token_scale[row_of(i) * p.kb_total + (col_of(i) >> 4)] = sc;
+      }
+      if (row_of(i) < p.M) *reinterpret_cast<u32x2*>(codes + row_of(i) * code_pitch + col_of(i) * 8) = q8;
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+}  // namespace
+}  // namespace mi355

@@ -23,6 +23,7 @@
 #include <mutex>
 
 #include "gemm_common.h"
+#include "tile_choice.h"
 
 namespace mi355 {
 namespace {
@@ -345,6 +346,7 @@ Plan make_plan(int64_t M, int64_t N, int64_t K) {
 }
 
 size_t scale_relayout_bytes(int64_t M, int64_t K);
+int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K);
 
 // Upper bound over the kernels a shape may be routed to (the choice also depends on pointer alignment, which is not
 // known here).
@@ -361,6 +363,11 @@ size_t workspace_bytes(int64_t M, int64_t N, int64_t K, bool is_fp8) {
     const int ds = decode_splits(M, N, K);
     const size_t dneed = ds > 1 ? (size_t)ds * (size_t)M * (size_t)N * 4u : 0;
     if (dneed > need) need = dneed;
+  }
+  if (M > 16 && K % KSTEP == 0) {
+    const int splits = is_fp8 ? std::max(run_splits(GK_F32, M, N, K), run_splits(GK_UNIT, M, N, K)) : run_splits(GK_INT8, M, N, K);
+    const size_t rneed = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * 4u : 0;
+    if (rneed > need) need = rneed;
   }
   if (is_fp8 && (M > 16 || (double)M >= route_constants().decode_dma3_min_tokens)) need += scale_relayout_bytes(M, K);  // the direct-to-LDS kernels may have to re-lay the token scales out
   return need;
@@ -401,8 +408,8 @@ int launch_tile(GemmParams& p, bool aligned, hipStream_t stream, const char* wha
 
 // Which kernel serves a problem, with which tiling.  One function decides for the launcher and for the plan query, so
 // what the query reports is what runs.
-enum RouteKernel { RK_DECODE = 0, RK_DMA3, RK_PINGPONG, RK_PIPELINED, RK_GENERIC, RK_WAVESPLIT, RK_PP128 };
-const char* const ROUTE_NAMES[] = {"decode", "dma3", "pingpong", "pipelined", "generic", "decode_wavesplit", "pingpong128"};
+enum RouteKernel { RK_DECODE = 0, RK_DMA3, RK_PINGPONG, RK_PIPELINED, RK_GENERIC, RK_WAVESPLIT, RK_PP128, RK_WAVESPLIT_TILE };
+const char* const ROUTE_NAMES[] = {"decode", "dma3", "pingpong", "pipelined", "generic", "decode_wavesplit", "pingpong128", "wavesplit_tile"};
 
 struct Route {
   int kernel;
@@ -529,6 +536,65 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
   return r;
 }
 
+const RouteConstants g_route_defaults{};
+thread_local const RouteConstants* g_route_override = nullptr;  // set while a perturbed plan is queried
+
+// The route that runs: choose_route's, or the tile that models faster (tile_choice.h).
+Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
+  Route r = choose_route(kind != GK_INT8, M, N, K, lda, ldb, aligned);
+  if (!aligned || M * lda >= (1ll << 32) || N * ldb >= (1ll << 32)) return r;
+  TileChoice c{TF_NONE, 0, 0, 1, 0.0};
+  if (K % KSTEP != 0) {
+    if (kind == GK_UNIT || kind == GK_INT8) c = choose_ragged_tile(M, N, K);
+  } else if (M <= 16) {
+    c = choose_decode_tile(kind, M, N, K);
+  } else {
+    TileChoice base{TF_NONE, r.bm, r.bn, r.splits, 0.0};
+    if (r.kernel == RK_DMA3 || (r.kernel == RK_PP128 && r.splits == 1)) base.family = TF_DMA;
+    if (r.kernel == RK_PINGPONG) base.family = TF_TWO_PHASE;
+    c = choose_mid_tile(kind, M, N, K, base);
+  }
+  if (c.family == TF_NONE) return r;
+  r.kernel = c.family == TF_DMA ? RK_DMA3 : c.family == TF_WAVESPLIT ? RK_WAVESPLIT_TILE : RK_PINGPONG;
+  r.bm = c.bm, r.bn = c.bn, r.splits = c.splits, r.groups_per_wg = 0;
+  const int64_t kb = (K + KSTEP - 1) / KSTEP;
+  r.kb_per_split = (int)((kb + c.splits - 1) / c.splits);
+  return r;
+}
+// A model evaluation takes some 10 us, so each thread keeps the routes of the shapes it met last.
+Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
+  struct Entry {
+    int64_t M, N, K, lda, ldb;
+    int kind;  // -1: empty
+    bool aligned;
+    Route route;
+  };
+  constexpr int ENTRIES = 256;
+  struct Table {
+    Entry e[ENTRIES];
+    Table() {
+      for (Entry& x : e) x.kind = -1;
+    }
+  };
+  if (&route_constants() != &g_route_defaults) return uncached_run_route(kind, M, N, K, lda, ldb, aligned);
+  static thread_local Table table;
+  uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull) ^ (uint64_t)kind * 0x27d4eb2f165667c5ull;
+  Entry& e = table.e[(h ^ (h >> 29)) >> 20 & (ENTRIES - 1)];
+  if (e.kind != (int)kind || e.M != M || e.N != N || e.K != K || e.lda != lda || e.ldb != ldb || e.aligned != aligned) {
+    e.route = uncached_run_route(kind, M, N, K, lda, ldb, aligned);
+    e.kind = (int)kind, e.M = M, e.N = N, e.K = K, e.lda = lda, e.ldb = ldb, e.aligned = aligned;
+  }
+  return e.route;
+}
+int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K) { return run_route(kind, M, N, K, K, K, true).splits; }
+bool same_route(const Route& a, const Route& b) { return a.kernel == b.kernel && a.bm == b.bm && a.bn == b.bn && a.splits == b.splits; }
+// " run_bm=.. run_bn=.. run_splits=.. run_wavesplit=0|1" where another tile runs than the plan names
+void describe_run(char* buf, size_t len, const Route& plan, const Route& run) {
+  buf[0] = 0;
+  if (!same_route(plan, run))
+    snprintf(buf, len, " run_bm=%d run_bn=%d run_splits=%d run_wavesplit=%d", run.bm, run.bn, run.splits, (int)(run.kernel == RK_WAVESPLIT_TILE));
+}
+
 // out[kb * ld_out + m] = sa[m * sa_sm + kb * sa_sk]: token scales re-laid out M-major with a row pitch that is a multiple
 // of four floats.  One 32 x 32 tile per workgroup through LDS, so that reads and writes are both contiguous for either
 // input layout.
@@ -580,10 +646,12 @@ bool operands_aligned(const GemmParams& p) {
 }
 
 template <bool IS_FP8>
-int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipStream_t stream, const char* what) {
+int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_given, hipStream_t stream, const char* what) {
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
   const bool aligned = operands_aligned(p);
-  const Route r = choose_route(IS_FP8, p.M, p.N, p.K, p.lda, p.ldb, aligned, p.x16 != nullptr);
+  const bool wide_scales = (r.kernel == RK_WAVESPLIT_TILE) && p.sa_sm * (int64_t)p.M >= (1ll << 30);  // 32-bit byte offsets
+  if (!p.ue8m0 && !p.row_scale && (wide_scales || route_workspace_need(IS_FP8, r, p) > workspace_bytes_given))  // (a workspace for the plan's own splits)
+    r = choose_route(IS_FP8, p.M, p.N, p.K, p.lda, p.ldb, aligned, p.x16 != nullptr);
   p.splits = r.splits;
   p.kb_per_split = r.kb_per_split;
   const size_t need = route_workspace_need(IS_FP8, r, p);
@@ -610,6 +678,10 @@ int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipSt
       rc = IS_FP8 ? launch_fp8_decode(p, r.groups_per_wg, stream, what) : launch_int8_decode(p, r.groups_per_wg, stream, what);
       break;
     case RK_WAVESPLIT: return IS_FP8 ? launch_fp8_wavesplit(p, stream, what) : launch_int8_wavesplit(p, stream, what);
+    case RK_WAVESPLIT_TILE:
+      if constexpr (IS_FP8)
+        return p.ue8m0 ? launch_fp8_wavesplit_tile_ue8m0(p, r.bm, r.bn, stream, what) : p.row_scale ? launch_fp8_wavesplit_tile_unit(p, r.bm, r.bn, stream, what) : launch_fp8_wavesplit_tile(p, r.bm, r.bn, stream, what);
+      else return launch_int8_wavesplit_tile(p, r.bm, r.bn, stream, what);
     case RK_PP128:
       if constexpr (IS_FP8) {
         set_error("%s: the 128-token two-phase kernel is built for INT8", what);
@@ -640,9 +712,16 @@ int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipSt
   return check_launch(what);
 }
 
-// ---- the constants table: defaults, the per-thread override of a perturbed plan query, names
-const RouteConstants g_route_defaults{};
-thread_local const RouteConstants* g_route_override = nullptr;
+template <bool IS_FP8>
+int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipStream_t stream, const char* what) {
+  const bool aligned = operands_aligned(p);
+  const GemmKind kind = !IS_FP8 ? GK_INT8 : p.ue8m0 ? GK_UE8M0 : p.row_scale ? GK_UNIT : GK_F32;
+  const Route r = p.x16 != nullptr ? choose_route(IS_FP8, p.M, p.N, p.K, p.lda, p.ldb, aligned, true)
+                                   : run_route(kind, p.M, p.N, p.K, p.lda, p.ldb, aligned);
+  return run_gemm<IS_FP8>(p, r, workspace, workspace_bytes_given, stream, what);
+}
+
+// ---- names of the constants table
 const char* const ROUTE_CONSTANT_NAMES[ROUTE_CONSTANT_COUNT] = {
     "pp_fp8_us_per_kblock", "pp_int8_us_per_kblock", "pp_us_per_tile", "dma3_hbm_bytes_per_us",
     "dma3_tile_us[fp8][128x256]", "dma3_tile_us[fp8][64x256]", "dma3_tile_us[fp8][128x128]", "dma3_tile_us[fp8][64x128]",
@@ -675,9 +754,11 @@ int describe_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int aligned, ch
   MI355_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31),
                 MI355_ERR_INVALID_ARGUMENT, "%s: shape out of range", what);
   const Route r = choose_route(is_fp8, M, N, K, K, K, aligned != 0 && K % 16 == 0);
-  const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d",
+  char run[96];
+  describe_run(run, sizeof run, r, run_route(is_fp8 ? GK_F32 : GK_INT8, M, N, K, K, K, r.aligned));
+  const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d%s",
                          ROUTE_NAMES[r.kernel], r.bm, r.bn, r.splits, r.kb_per_split, r.groups_per_wg, (int)r.aligned,
-                         route_stages(is_fp8, r, M, N));
+                         route_stages(is_fp8, r, M, N), run);
   MI355_REQUIRE(n > 0 && (size_t)n < buf_len, MI355_ERR_INVALID_ARGUMENT, "%s: buffer of %zu bytes is too small", what,
                 buf_len);
   return MI355_OK;
@@ -871,7 +952,7 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
   p.bias = bias;
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
-  const Route r = choose_route(true, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  const Route r = run_route(GK_UE8M0, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
   const bool words_conform = (sa_sk & 3) == 0 && sa_sk >= ((M + 3) & ~3ll) && (reinterpret_cast<uintptr_t>(sa_words) & 15) == 0;
   if (r.kernel == RK_PINGPONG && K % KSTEP == 0 && words_conform) {
     // the MFMA applies both exponents itself: no scale arithmetic at all
@@ -882,11 +963,11 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
     // decode sizes on the wave-split kernel: the same, one launch, no workspace
     return launch_fp8_wavesplit_ue8m0(p, st, what);
   }
-  if ((r.kernel == RK_DMA3 && K % KSTEP == 0 && words_conform) || r.kernel == RK_DECODE) {
+  if ((r.kernel == RK_DMA3 && K % KSTEP == 0 && words_conform) || r.kernel == RK_DECODE || r.kernel == RK_WAVESPLIT_TILE) {
     // mid-M and streaming decode: the same kernels with the exponents applied by the MFMA; the workspace only holds
     // split-K partial sums (the decode kernel reads the words with ordinary loads: any pitch will do)
     p.ue8m0 = 1;
-    return run_gemm<true>(p, workspace, workspace_bytes_given, st, what);
+    return run_gemm<true>(p, r, workspace, workspace_bytes_given, st, what);
   }
   // every other shape: exponents to fp32 scales in the head of the workspace (tokens M-major, weights one row per
   // 128-channel block, read from the block's first channel), then the fp32-scale kernels
@@ -937,7 +1018,8 @@ extern "C" int mi355_fp8_blockwise_mm_noalloc(const void* a, const void* b, cons
   int rc = fp8_mm_params(what, a, b, sa, sb, out, out_dtype, M, N, K, lda, ldb, sa_sm, sa_sk, sb_sn, sb_sk, ldo, p, empty);
   if (rc != MI355_OK || empty) return rc;
   // the same plan the launcher will make: how many partial-sum bytes it needs
-  const Route r = choose_route(true, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  Route r = run_route(GK_F32, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  if (route_workspace_need(true, r, p) > NOALLOC_SCRATCH_BYTES) r = choose_route(true, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
   const size_t need = route_workspace_need(true, r, p);
   MI355_REQUIRE(need <= NOALLOC_SCRATCH_BYTES, MI355_ERR_WORKSPACE,
                 "%s: M=%lld N=%lld K=%lld needs %zu bytes of scratch (split-K partial sums), the built-in scratch holds %zu; use "
@@ -949,7 +1031,7 @@ extern "C" int mi355_fp8_blockwise_mm_noalloc(const void* a, const void* b, cons
     if (rc != MI355_OK) return rc;
   }
   // every partial sum that the reduce kernel reads is written by this call first, so nothing has to be cleared
-  return run_gemm<true>(p, ws, need > 0 ? NOALLOC_SCRATCH_BYTES : 0, static_cast<hipStream_t>(stream), what);
+  return run_gemm<true>(p, r, ws, need > 0 ? NOALLOC_SCRATCH_BYTES : 0, static_cast<hipStream_t>(stream), what);
 }
 
 extern "C" int mi355_qlinear_init(void) {
@@ -982,8 +1064,8 @@ extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa
   p.col_scale = sb;
   p.bias = bias;
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
-  const Route r = choose_route(true, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
-  if (r.kernel == RK_DMA3) p.row_scale = sa;  // mid M: no scales in the K loop, both in the epilogue (or the reduce)
+  const Route r = run_route(GK_UNIT, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  if (r.kernel == RK_DMA3 || r.kernel == RK_WAVESPLIT_TILE) p.row_scale = sa;  // no scales in the K loop, both in the epilogue (or the reduce)
   if (r.kernel == RK_PINGPONG && K % KSTEP == 0) {
     // large M: accumulate in the MFMA with unit scales, apply both scales once in the epilogue (the reference's order)
     p.row_scale = sa;
@@ -992,7 +1074,7 @@ extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa
     p.splits = 1, p.kb_per_split = p.kb_total;
     return launch_fp8_pp_rowcol(p, static_cast<hipStream_t>(stream), what);
   }
-  return run_gemm<true>(p, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
+  return run_gemm<true>(p, r, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
 }
 
 namespace {
@@ -1036,7 +1118,10 @@ bool wavesplit_quant_preferred(WavesplitQuant kind, int64_t M, int64_t N, int64_
   const bool is_fp8 = kind != WavesplitQuant::TOKEN_INT8;
   if (!wavesplit_supported(M, N, K) || !wavesplit_quant_fits(M, K) || N * ldw >= (1ll << 32)) return false;
   const double kb = (double)(K / KSTEP), waves = wavesplit_shape(K).waves;
-  const bool plain_wavesplit = choose_route(is_fp8, M, N, K, K, ldw, true).kernel == RK_WAVESPLIT;
+  const GemmKind gemm = kind == WavesplitQuant::BLOCK_F32 ? GK_F32 : kind == WavesplitQuant::BLOCK_UE8M0 ? GK_UE8M0 : is_fp8 ? GK_UNIT : GK_INT8;
+  const int plain = run_route(gemm, M, N, K, K, ldw, true).kernel;
+  if (plain == RK_WAVESPLIT_TILE) return false;
+  const bool plain_wavesplit = plain == RK_WAVESPLIT;
   if ((kind == WavesplitQuant::BLOCK_UE8M0 || kind == WavesplitQuant::TOKEN_FP8) && !plain_wavesplit) return false;
   if (kb < route_constants().wavesplit_min_kblocks && (is_fp8 || N / 16 > 512)) return false;  // a block per wave: 512->32768 8.2 against 10.5
   const double v = (double)(M * K) / (8.0 * 64.0 * waves);
@@ -1049,6 +1134,24 @@ bool wavesplit_quant_preferred(WavesplitQuant kind, int64_t M, int64_t N, int64_
 }
 bool wavesplit_quant_operands(const void* x, int x_dtype, const void* w, int64_t ldw) {
   return x_dtype != MI355_F32 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
+}
+// The wave-split tile quantizing the tokens itself, where the GEMM takes that tile (same sums, bit for bit): the launch saved
+// against the quantizer's work in every workgroup, v pieces per thread and round.
+bool tile_quant_preferred(const Route& run, int64_t M, int64_t N, int64_t K) {
+  if (run.kernel != RK_WAVESPLIT_TILE || M > 16 || K % KSTEP != 0) return false;
+  const int64_t pieces = M * K / 8, threads = 512, rounds = (N + (int64_t)run.bn * NUM_CUS - 1) / ((int64_t)run.bn * NUM_CUS);
+  return pieces <= 10 * threads && pieces * rounds <= 10 * threads;
+}
+int run_tile_quant(GemmParams& p, WavesplitQuant kind, const Route& run, const void* x, int x_dtype, void* stream, const char* what) {
+  p.x16 = x, p.ldx = p.K, p.x_dtype = x_dtype;
+  p.kb_total = p.K / KSTEP;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  switch (kind) {
+    case WavesplitQuant::BLOCK_F32: return launch_fp8_wavesplit_tile_quant(p, run.bn, st, what);
+    case WavesplitQuant::BLOCK_UE8M0: return launch_fp8_wavesplit_tile_ue8m0_quant(p, run.bn, st, what);
+    case WavesplitQuant::TOKEN_FP8: return launch_fp8_wavesplit_tile_unit_quant(p, run.bn, st, what);
+    default: return launch_int8_wavesplit_tile_quant(p, run.bn, st, what);
+  }
 }
 int run_wavesplit_quant(GemmParams& p, WavesplitQuant kind, const void* x, int x_dtype, void* stream, const char* what) {
   p.x16 = x, p.ldx = p.K, p.x_dtype = x_dtype;
@@ -1101,16 +1204,21 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   // Decode sizes: the GEMM kernel quantizes the tokens itself (same arithmetic), no quantizer launch - except where a
   // quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
   const bool ptr_ok = x_dtype != MI355_F32 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
-  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, ldw)) {
+  const bool w_aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
+  const Route run = run_route(GK_F32, M, N, K, K, ldw, w_aligned);
+  const bool tile = M <= 16 && run.kernel == RK_WAVESPLIT_TILE;  // faster than the kernels below also behind a quantizer launch
+  const bool tile_quant = tile && wavesplit_quant_operands(x, x_dtype, w, ldw) && tile_quant_preferred(run, M, N, K);
+  if (tile_quant || (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, ldw))) {
     GemmParams p;
     bool empty;
     const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, pitch, ws_sn, ws_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
     p.bias = bias;
     p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
+    if (tile_quant) return run_tile_quant(p, WavesplitQuant::BLOCK_F32, run, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::BLOCK_F32, x, x_dtype, stream, what);
   }
-  if (ptr_ok && M <= 16) {
+  if (ptr_ok && M <= 16 && !tile) {
     const Route plain = linear_producer_route(M, N, K, ldw);
     if (plain.kernel == RK_DMA3) {  // one round of unsplit 64-token tiles: producer waves of that kernel quantize the tokens
       GemmParams p;
@@ -1123,7 +1231,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
       return launch_fp8_dma3_quant(p, plain.bn, static_cast<hipStream_t>(stream), what);
     }
   }
-  if (ptr_ok && choose_route(true, M, N, K, K, ldw, true, true).kernel == RK_DECODE && fused_quant_preferred(M, N, K, ldw)) {
+  if (ptr_ok && !tile && choose_route(true, M, N, K, K, ldw, true, true).kernel == RK_DECODE && fused_quant_preferred(M, N, K, ldw)) {
     GemmParams p;
     bool empty;
     // a / sa are not read by the kernel in this mode; they only have to satisfy the checks
@@ -1174,7 +1282,8 @@ extern "C" int mi355_fp8_block_linear_plan(int64_t M, int64_t N, int64_t K, char
   const bool fused = producer || (choose_route(true, M, N, K, K, K, true, true).kernel == RK_DECODE && fused_quant_preferred(M, N, K, K));
   const Route r = producer ? plain : choose_route(true, M, N, K, K, K, true, fused);
   const bool wavesplit = wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, K);
-  char instead[32] = "";
+  char instead[96] = "";
+  describe_run(instead, sizeof instead, choose_route(true, M, N, K, K, K, true), run_route(GK_F32, M, N, K, K, K, true));
   if (wavesplit) snprintf(instead, sizeof instead, " wavesplit_waves=%d", wavesplit_shape(K).waves);
   const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d quantizer=%s%s",
                          ROUTE_NAMES[r.kernel], r.bm, r.bn, r.splits, r.kb_per_split, r.groups_per_wg, (int)r.aligned,
@@ -1250,7 +1359,10 @@ extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, cons
   p.M = (int)M, p.N = (int)N, p.K = (int)K;
   p.lda = K, p.ldb = ldw, p.ldo = ldo;
   p.out_dtype = out_dtype;
-  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::TOKEN_INT8, M, N, K, ldw))
+  const bool fusable = wavesplit_quant_operands(x, x_dtype, w, ldw);
+  const Route run = run_route(GK_INT8, M, N, K, K, ldw, fusable && K % 16 == 0);
+  if (fusable && tile_quant_preferred(run, M, N, K)) return run_tile_quant(p, WavesplitQuant::TOKEN_INT8, run, x, x_dtype, stream, what);
+  if (fusable && wavesplit_quant_preferred(WavesplitQuant::TOKEN_INT8, M, N, K, ldw))
     return run_wavesplit_quant(p, WavesplitQuant::TOKEN_INT8, x, x_dtype, stream, what);
   const int rc = mi355_per_token_quant_int8(x, x_dtype, q, sa, M, K, stream);
   if (rc != MI355_OK) return rc;
@@ -1284,13 +1396,17 @@ extern "C" int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void
   const size_t q_bytes = align256((size_t)M * (size_t)K);
   float* sa = reinterpret_cast<float*>(q + q_bytes);
   const size_t sa_bytes = align256((size_t)M * 4u);
-  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::TOKEN_FP8, M, N, K, ldw)) {
+  const bool fusable = wavesplit_quant_operands(x, x_dtype, w, ldw);
+  const Route run = run_route(GK_UNIT, M, N, K, K, ldw, fusable && K % 16 == 0);
+  const bool tile_quant = fusable && tile_quant_preferred(run, M, N, K);
+  if (tile_quant || (fusable && wavesplit_quant_preferred(WavesplitQuant::TOKEN_FP8, M, N, K, ldw))) {
     GemmParams p;
     bool empty;
     // (the block scales are not read in this mode; they only have to satisfy the checks)
     const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, 0, 0, 0, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
     p.col_scale = w_scale, p.bias = bias;
+    if (tile_quant) return run_tile_quant(p, WavesplitQuant::TOKEN_FP8, run, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::TOKEN_FP8, x, x_dtype, stream, what);
   }
   const int rc = mi355_per_token_quant_fp8(x, x_dtype, q, sa, M, K, stream);
@@ -1330,13 +1446,17 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
   void* sa_words = q + q_bytes;
   const int64_t pitch = (M + 3) & ~3ll;
   const size_t sa_bytes = align256((size_t)pitch * (size_t)((K / KSTEP + 3) / 4) * 4u);
-  if (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw)) {
+  const bool fusable = wavesplit_quant_operands(x, x_dtype, w, ldw);
+  const Route run = run_route(GK_UE8M0, M, N, K, K, ldw, fusable);
+  const bool tile_quant = fusable && tile_quant_preferred(run, M, N, K);
+  if (tile_quant || (fusable && wavesplit_quant_preferred(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw))) {
     GemmParams p;
     bool empty;
     const float* words = static_cast<const float*>(sb_words);  // (strides of the packed words stand in for fp32 ones)
     const int rc = fp8_mm_params(what, x, w, words, words, out, out_dtype, M, N, K, K, ldw, 1, pitch, sb_sn, sb_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
     p.bias = bias;
+    if (tile_quant) return run_tile_quant(p, WavesplitQuant::BLOCK_UE8M0, run, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::BLOCK_UE8M0, x, x_dtype, stream, what);
   }
   // q = x * (448 / amax) with the scale rounded up to a power of two: per_token_group_quant_8bit_v2.cu:77-78 with scale_ue8m0

@@ -1,0 +1,297 @@
+// A small output tile of the FP8 and INT8 GEMMs for gfx950, K split over the waves of the workgroup: 16 MT tokens x 16 CT
+// channels, eight waves, each with its own ring of LDS slots filled by direct-to-LDS loads, no barrier in the K loop.
+//
+// For few tokens, or a small weight, the tile of gemm_dma_tile.h has too few workgroups to fill the chip, and each of them is one
+// serial chain of K blocks (load, barrier, LDS, multiply), about 0.3 us a block; splitting K over workgroups fills the chip but
+// costs fp32 partial tiles and a second launch.  Here a workgroup's waves take K blocks w, w + 8, ... each on its own, and the
+// eight partial tiles meet in LDS once at the end: K / 1024 steps deep, one launch, as many workgroups as small tiles give.
+//
+// What bounds it is what a CU pulls out of L2, (16 MT + 16 CT) x 128 bytes per K block: 40 to 55 bytes a cycle, against a peak of
+// 61.  The loads must take whole 128-byte lines: fetched straight into registers in the MFMA's layout (16 rows x 64 bytes per
+// instruction, neighbouring lanes in different rows), the same bytes came at 16 a cycle whatever the number of waves, which is what
+// bounded an earlier form of this tile and bounds the decode kernel (gemm_decode_wavesplit.hip).
+// GPU time of one GEMM in us, before (the better of the mid-M tile, split or not, and the decode kernels) / this:
+//   K = 7168 -> N = 576: 1 token 6.8 / 5.1, 64 9.6 / 5.6, 320 12.4 / 7.6;  K = 4096 -> N = 6144: 8 8.6 / 6.0, 64 13.0 / 7.7
+//   K = 7168 -> N = 2048: 160 14.1 / 8.8;  K = 2048 -> N = 2048: 64 8.4 / 4.3;  K = 2560 -> N = 512: 45 9.3 / 4.4
+// Releasing the token rows of a slot before the weight rows are read (a finer ring) measured the same.
+//
+// Registers stay low (34 - 190); the LDS holds one workgroup per CU.  A wave's loads per K block are constant, so "slot landed" is
+// a counted wait; the slot is refilled as soon as its fragments are in registers.
+// Any M and N; K % 128 == 0 for AR_F32 and AR_UE8M0, K % 16 == 0 otherwise (the tokens' tail is zeroed, the weight's repeats valid
+// bytes of the same row); 16-byte aligned rows, row offsets below 4 GiB; any strides of the token scales.
+#pragma once
+
+#include "gemm_dma_tile.h"
+#include "gemm_token_quant.h"
+
+namespace mi355 {
+namespace {
+
+// Eight waves: with four, K = 7168 takes twice the steps; sixteen would halve the slots.
+constexpr int WST_WAVES = 8;
+
+// TQ: the tokens arrive unquantized (MT = 1 only); their codes take WST_CODE_BYTES of the LDS and the slots hold weight rows only.
+constexpr int WST_CODE_BYTES = 64 * WST_WAVES * WS_QUANT_VECTORS * 8 + 16 * 16;  // M (K + 16) for as many pieces as there may be
+constexpr int WST_SCALE_BYTES = WST_CODE_BYTES / KSTEP * 4;
+template <Arith AR, int MT, int CT, TokenQuant TQ>
+struct WavesplitTile {
+  static constexpr bool SCALED = (AR == AR_F32 || AR == AR_UE8M0) && TQ == TQ_NONE;  // token scales in the slots
+  static constexpr int BM = 16 * MT, BN = 16 * CT, TOKENS = TQ == TQ_NONE ? BM : 0;
+  static constexpr int SLOT_BYTES = (TOKENS + BN) * KSTEP + (SCALED ? BM * 4 : 0);
+  static constexpr int RING_LIMIT = 160 * 1024 - (TQ == TQ_NONE ? 0 : WST_CODE_BYTES + WST_SCALE_BYTES + 64);
+  static constexpr int FIT = RING_LIMIT / (WST_WAVES * SLOT_BYTES), R = FIT > 4 ? 4 : FIT;
+  static_assert(R >= 1, "a slot per wave");
+  static constexpr int ROW_LOADS = (TOKENS + BN) / 8, LOADS = ROW_LOADS + (SCALED ? 1 : 0);
+};
+
+template <int N>
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// waits until at most the loads of the `blocks` youngest requests are outstanding
+template <int LOADS>
+__device__ __forceinline__ void wait_blocks(int blocks) {
+  if (blocks >= 4) wait_loads<4 * LOADS>();
+  else if (blocks == 3) wait_loads<3 * LOADS>();
+  else if (blocks == 2) wait_loads<2 * LOADS>();
+  else if (blocks == 1) wait_loads<LOADS>();
+  else wait_loads<0>();
+}
+
+template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2>
+__global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void wavesplit_tile_kernel(const GemmParams p) {
+  using T = WavesplitTile<AR, MT, CT, TQ>;
+  static_assert(TQ == TQ_NONE || MT == 1, "the fused quantizer is for 16 tokens at most");
+  constexpr int R = T::R, LOADS = T::LOADS, BM = T::BM, BN = T::BN, W = WST_WAVES;
+  using AccT = typename std::conditional<AR == AR_INT8, int, float>::type;
+  typedef AccT acc4 __attribute__((ext_vector_type(4)));
+  constexpr int RING_BYTES = W * R * T::SLOT_BYTES, RED_BYTES = W * MT * CT * 64 * 16;
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[RING_BYTES > RED_BYTES ? RING_BYTES : RED_BYTES];
+  __shared__ __attribute__((aligned(16))) uint8_t codes[TQ == TQ_NONE ? 16 : WST_CODE_BYTES];
+  __shared__ float token_scale[TQ == TQ_NONE ? 1 : WST_SCALE_BYTES / 4];
+  __shared__ float row_max[TQ == TQ_ROW ? 16 : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, q = lane >> 4;
+  // consecutive workgroups of an XCD take the token tiles of the same channels
+  int bid = blockIdx.x;
+  const int per_xcd = (int)gridDim.x >> 3;
+  if (bid < per_xcd * 8) bid = (bid & 7) * per_xcd + (bid >> 3);
+  const int m0 = (bid % p.tiles_m) * BM, n0 = (bid / p.tiles_m) * BN;
+
+  // loader: a load fills 8 rows of a slot, lane = row lane >> 3, 16-byte chunk lane & 7; chunks land swizzled by (row & 7)
+  uint32_t goff[T::ROW_LOADS];
+  const int chunk = (lane & 7) ^ (lane >> 3);
+#pragma unroll
+  for (int i = 0; i < T::ROW_LOADS; ++i) {
+    const int row = i * 8 + (lane >> 3);
+    goff[i] = i * 8 < T::TOKENS ? (uint32_t)((int64_t)min(m0 + row, p.M - 1) * p.lda + chunk * 16)
+                         : (uint32_t)((int64_t)min(n0 + row - T::TOKENS, p.N - 1) * p.ldb + chunk * 16);
+  }
+  const uint32_t soff = T::SCALED ? (uint32_t)((int64_t)min(m0 + min(lane, BM - 1), p.M - 1) * p.sa_sm * 4) : 0u;
+  const int last = p.kb_total - 1;
+  const int tail = p.K - last * KSTEP;  // bytes of the last K block
+  const uint32_t my_ring = (uint32_t)(uintptr_t)(lptr_t)ring + (uint32_t)(wave * R * T::SLOT_BYTES);
+  auto issue = [&](int slot, int kb) {
+    const uint8_t *wb = p.b + (int64_t)kb * KSTEP, *tb = p.a + (int64_t)kb * KSTEP;
+    uint32_t lds = my_ring + (uint32_t)(slot * T::SLOT_BYTES);
+    uint32_t back = 0;  // chunks past the row's end repeat its last one
+    if constexpr (AR == AR_UNIT || AR == AR_INT8) back = kb == last ? (uint32_t)(max(chunk - (tail / 16 - 1), 0) * 16) : 0u;
+    asm volatile("" : "+s"(wb), "+s"(tb), "+s"(lds));
+#pragma unroll
+    for (int i = 0; i < T::ROW_LOADS; ++i)
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i] - back), "s"(i * 8 < T::TOKENS ? tb : wb), "s"(lds + i * 1024)
+                   : "memory");
+    if constexpr (T::SCALED) {
+      const float* sbase = p.sa + (int64_t)(AR == AR_UE8M0 ? kb >> 2 : kb) * p.sa_sk;
+      asm volatile("" : "+s"(sbase));
+      uint64_t saved;
+      asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, %4\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b64 exec, %0"
+                   : "=&s"(saved) : "v"(soff), "s"(sbase), "s"(lds + T::ROW_LOADS * 1024), "s"(BM == 64 ? ~0ull : (1ull << (BM & 63)) - 1) : "memory");
+    }
+  };
+
+  constexpr bool SCALES = AR == AR_F32 || AR == AR_UE8M0;
+  const cfloat_ptr sb_row = (cfloat_ptr)(SCALES ? p.sb + (int64_t)(AR == AR_UE8M0 ? n0 : (n0 >> 7)) * p.sb_sn : nullptr);
+  acc4 acc[CT][MT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[c][t] = acc4{0, 0, 0, 0};
+  const uint32_t lo = l16 * KSTEP + ((q ^ (l16 & 7)) << 4), hi = l16 * KSTEP + (((q + 4) ^ (l16 & 7)) << 4);
+
+  const int blocks = wave <= last ? (last - wave) / W + 1 : 0;  // K blocks wave, wave + W, ...
+  auto request_first = [&] {
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      if (j < blocks) issue(j, wave + j * W);
+  };
+  if constexpr (TQ == TQ_NONE) {
+    request_first();
+  } else {
+    quantize_tokens<AR != AR_INT8, AR == AR_UE8M0, TQ, NV, 64 * W>(p, codes, token_scale, row_max, [&] {
+      request_first();
+      wait_blocks<LOADS>(min(blocks, R));
+    });
+  }
+  int slot = 0;
+  for (int i = 0; i < blocks; ++i) {
+    const int kb = wave + i * W;
+    float sb = 0.f;
+    if constexpr (SCALES) sb = sb_row[(int64_t)(AR == AR_UE8M0 ? kb >> 2 : kb) * p.sb_sk];
+    wait_blocks<LOADS>(min(blocks - 1 - i, R - 1));
+    const lds_cptr st = (lds_cptr)ring + (wave * R + slot) * T::SLOT_BYTES;
+    Frag tf[MT], wf[CT];
+    float ts[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      if constexpr (TQ == TQ_NONE) {
+        tf[t].lo = lds16(st + lo, t * 2048), tf[t].hi = lds16(st + hi, t * 2048);
+      } else {
+        const uint8_t* src = codes + min(l16, p.M - 1) * (p.K + 16) + kb * KSTEP + q * 16;
+        tf[t].lo = *reinterpret_cast<const u32x4*>(src), tf[t].hi = *reinterpret_cast<const u32x4*>(src + 64);
+        if constexpr (TQ == TQ_GROUP) ts[t] = token_scale[min(l16, p.M - 1) * p.kb_total + kb];
+      }
+      if constexpr (T::SCALED) ts[t] = lds_f32(st + (T::ROW_LOADS * 1024) + l16 * 4, t * 64);
+    }
+#pragma unroll
+    for (int c = 0; c < CT; ++c) wf[c].lo = lds16(st + lo, (T::TOKENS / 16 + c) * 2048), wf[c].hi = lds16(st + hi, (T::TOKENS / 16 + c) * 2048);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + R < blocks) issue(slot, kb + R * W);
+    slot = slot + 1 == R ? 0 : slot + 1;
+    if constexpr ((AR == AR_UNIT || AR == AR_INT8) && TQ == TQ_NONE) {
+      const int valid = kb == last ? tail : KSTEP;
+      const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        if (16 * q >= valid) tf[t].lo = z;
+        if (64 + 16 * q >= valid) tf[t].hi = z;
+      }
+    }
+    if constexpr (AR == AR_F32) {
+      v4f part[CT * MT];
+#pragma unroll
+      for (int s = 0; s < CT * MT; ++s)
+        part[s] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(wf[s % CT]), as_v8i(tf[s / CT]), v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const float sc = ts[t] * sb;
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[c][t][v] = fmaf(part[t * CT + c][v], sc, acc[c][t][v]);
+      }
+    } else if constexpr (AR == AR_UE8M0) {
+      const int shift = (kb & 3) * 8;
+      const int ew = in_vgpr((int)((__float_as_uint(sb) >> shift) & 0xffu));
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int et = (int)(__float_as_uint(ts[t]) >> (TQ == TQ_NONE ? shift : 0));
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+          acc[c][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(wf[c]), as_v8i(tf[t]), acc[c][t], 0, 0, 0, ew, 0, et);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          if constexpr (AR == AR_UNIT) {
+            acc[c][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(as_v8i(wf[c]), as_v8i(tf[t]), acc[c][t], 0, 0, 0, 0, 0, 0);
+          } else {
+            acc[c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(as_v4i(wf[c].lo), as_v4i(tf[t].lo), acc[c][t], 0, 0, 0);
+            acc[c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(as_v4i(wf[c].hi), as_v4i(tf[t].hi), acc[c][t], 0, 0, 0);
+          }
+        }
+    }
+  }
+
+  // ---- add the W partial tiles in wave order, 16 x 16 tile t of them by wave t % W, and store
+  __syncthreads();  // the rings are free
+  acc4* red = reinterpret_cast<acc4*>(ring);
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) red[(wave * MT * CT + c * MT + t) * 64 + lane] = acc[c][t];
+  __syncthreads();
+  const bool vec_ok = (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+#pragma unroll
+  for (int e = wave; e < CT * MT; e += W) {
+    acc4 s = red[e * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+      const acc4 x = red[(w * MT * CT + e) * 64 + lane];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s[v] += x[v];
+    }
+    // lane holds channels n .. n + 3 of token m
+    const int m = m0 + 16 * (e % MT) + l16, n = n0 + 16 * (e / MT) + 4 * q;
+    if (m >= p.M || n >= p.N) continue;
+    if constexpr (AR == AR_INT8) {
+      if (p.out_dtype == MI355_I32) {
+        int* o = reinterpret_cast<int*>(p.out) + (int64_t)m * p.ldo + n;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (n + v < p.N) o[v] = s[v];
+        continue;
+      }
+    }
+    const ChannelTerms ct = load_channel_terms(p, AR == AR_INT8 ? p.sb : p.col_scale, n);
+    float r[4];
+    if constexpr (AR == AR_INT8) {
+      const int a4[4] = {s[0], s[1], s[2], s[3]};
+      int8_apply_terms(p, ct, TQ == TQ_NONE ? p.sa[m] : token_scale[m], a4, r);
+    } else {
+      r[0] = s[0], r[1] = s[1], r[2] = s[2], r[3] = s[3];
+      fp8_apply_terms(p, ct, TQ == TQ_ROW ? token_scale[m] : p.row_scale ? p.row_scale[m] : 1.f, r);
+    }
+    store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, min(4, p.N - n), vec_ok);
+  }
+}
+
+template <Arith AR, int MT, int CT>
+int launch_wavesplit_tile_inst(GemmParams& p, hipStream_t stream, const char* what) {
+  p.tiles_m = (p.M + 16 * MT - 1) / (16 * MT), p.tiles_n = (p.N + 16 * CT - 1) / (16 * CT);
+  p.splits = 1;
+  hipLaunchKernelGGL((wavesplit_tile_kernel<AR, MT, CT>), dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(64 * WST_WAVES), 0, stream, p);
+  return check_launch(what);
+}
+template <Arith AR, size_t... I>
+int launch_wavesplit_tile_of(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what, std::index_sequence<I...>) {
+  int rc = MI355_ERR_UNSUPPORTED;
+  bool found = false;
+  ((found = found || (bm == WAVESPLIT_TILES[I].bm && bn == WAVESPLIT_TILES[I].bn &&
+                      (rc = launch_wavesplit_tile_inst<AR, WAVESPLIT_TILES[I].bm / 16, WAVESPLIT_TILES[I].bn / 16>(p, stream, what), true))), ...);
+  if (!found) set_error("%s: no wave-split %d x %d tile is built", what, bm, bn);
+  return rc;
+}
+template <Arith AR>
+int launch_wavesplit_tile_of(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what) {
+  return launch_wavesplit_tile_of<AR>(p, bm, bn, stream, what, std::make_index_sequence<sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0])>{});
+}
+
+// The same with the tokens quantized in the kernel (p.x16 / p.ldx / p.x_dtype; p.a and p.sa are not read).
+template <Arith AR, TokenQuant TQ, int CT>
+int launch_wavesplit_tile_quant_inst(GemmParams& p, hipStream_t stream, const char* what) {
+  p.tiles_m = 1, p.tiles_n = (p.N + 16 * CT - 1) / (16 * CT);
+  p.splits = 1;
+  const dim3 grid((unsigned)p.tiles_n), block(64 * WST_WAVES);
+  const int64_t pieces = (int64_t)p.M * p.K / 8;
+  if (pieces <= 2 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 2>), grid, block, 0, stream, p);
+  else if (pieces <= 4 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 4>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, WS_QUANT_VECTORS>), grid, block, 0, stream, p);
+  return check_launch(what);
+}
+template <Arith AR, TokenQuant TQ>
+int launch_wavesplit_tile_quant(GemmParams& p, int bn, hipStream_t stream, const char* what) {
+  if (p.x16 == nullptr || p.M > 16 || p.K % KSTEP != 0 || (int64_t)p.M * p.K > 64 * WST_WAVES * WS_QUANT_VECTORS * 8) {
+    set_error("%s: the fused quantizer of the wave-split tile takes few unquantized tokens", what);
+    return MI355_ERR_UNSUPPORTED;
+  }
+  if (TQ == TQ_ROW && AR != AR_INT8) p.row_scale = p.col_scale;  // (there is one: it lies in LDS)
+  return bn == 16 ? launch_wavesplit_tile_quant_inst<AR, TQ, 1>(p, stream, what)
+       : bn == 32 ? launch_wavesplit_tile_quant_inst<AR, TQ, 2>(p, stream, what)
+                  : launch_wavesplit_tile_quant_inst<AR, TQ, 4>(p, stream, what);
+}
+
+}  // namespace
+}  // namespace mi355

@@ -1,0 +1,171 @@
+// Which tile a GEMM runs on, by modelled time: the mid-M tiles (gemm_dma_tile.h) with or without split K, the small wave-split
+// tiles (gemm_wavesplit_tile.h) and the 256 x 256 two-phase tile, next to what the route of the constants table names.
+//
+// The model was fitted to 60 000 timings of forced tiles (14 to 37 layers of K = 256 .. 18432 by N = 192 .. 36864, 1 to 4096
+// tokens, all tiles and splits, weights rotated out of the caches, and results too where they are large): 4 % root mean square for
+// the mid-M tiles, 6 % for the wave-split ones; its choice is 1.5 to 2 % slower than the best measured tile on average (geometric
+// mean over 2100 shapes), where the constants table alone was 16 to 25 % slower.
+#pragma once
+
+#include <cmath>
+
+#include "gemm_common.h"
+
+namespace mi355 {
+namespace {
+
+enum GemmKind { GK_F32, GK_UE8M0, GK_UNIT, GK_INT8 };  // FP8 with block scales, with exponents, with epilogue scales; INT8
+enum TileFamily { TF_NONE, TF_DMA, TF_WAVESPLIT, TF_TWO_PHASE };
+
+struct TileChoice {
+  int family, bm, bn, splits;
+  double us;
+};
+
+struct TileTimes {
+  // mid-M tile: launch + rounds of one workgroup per CU (64 x 128: two where there are more workgroups than CUs, each then
+  // `shared` times slower per block), each tile[i] + K blocks * block[i] * (1 + busy * fill); against the stream of both
+  // operands at `stream` TB/s plus the result; a split adds its launch and its partial sums
+  double launch, busy, split_us, split_us_per_mb, stream, stream_us, shared, result_us_per_mb;
+  double tile[13], block[13];  // in the order of MID_TILES
+  double pp_tile, pp_block, pp_busy, pp_store;  // 256 x 256; pp_store: a full round's result on its way to memory
+  // wave-split tile: rounds of ws_tile + KB of operands * (ws_kb + ws_kb_busy * fill) + kilo-elements of the tile * ws_result,
+  // together with the weight stream (ws_norm: how far the two overlap)
+  double ws_launch, ws_tile, ws_kb, ws_kb_busy, ws_stream, ws_stream_us, ws_result, ws_norm;
+};
+constexpr TileTimes SCALED_TIMES = {
+    1.93, 0.586, 4.31, 0.217, 4.18, -4.54, 1.808, 0.421,
+    {2.33, 2.83, 3.02, 3.40, 3.53, 4.64, 2.57, 3.31, 3.96, 4.32, 2.64, 3.53, 4.44},
+    {0.219, 0.277, 0.317, 0.385, 0.419, 0.533, 0.288, 0.363, 0.441, 0.532, 0.334, 0.445, 0.535},
+    7.88, 0.567, 1.70, 12.5,
+    2.74, 1.041, 0.00591, 0.00334, 5.49, -3.81, 0.253, 1.511};
+constexpr TileTimes PLAIN_TIMES = {
+    1.77, 0.777, 3.81, 0.251, 4.55, -2.24, 1.871, 0.402,
+    {2.21, 2.72, 3.03, 3.17, 3.76, 4.72, 2.48, 3.12, 3.83, 4.14, 2.81, 3.80, 4.64},
+    {0.165, 0.205, 0.240, 0.295, 0.333, 0.432, 0.224, 0.271, 0.339, 0.420, 0.278, 0.347, 0.431},
+    8.48, 0.511, 1.70, 10.8,
+    2.71, 1.017, 0.00609, 0.00343, 5.07, -4.41, 0.282, 1.673};
+static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above follow MID_TILES");
+
+double norm_of(double a, double b, double n) { return b <= 0.1 ? a : std::pow(std::pow(a, n) + std::pow(b, n), 1.0 / n); }
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// full rounds of `slots` workgroups and a partly filled one
+template <class Round>
+double rounds_of(int64_t workgroups, int64_t slots, Round round) {
+  const int64_t full = workgroups / slots, rest = workgroups % slots;
+  return (double)full * round(1.0) + (rest ? round((double)rest / (double)slots) : 0.0);
+}
+
+double dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, int splits) {
+  const int bm = MID_TILES[i].bm, bn = MID_TILES[i].bn;
+  const int64_t kb = ceil_div(K, KSTEP), wg = ceil_div(M, bm) * ceil_div(N, bn) * splits;
+  const double blocks = (double)ceil_div(kb, splits);
+  const bool two = bm + bn == 192 && wg > NUM_CUS;
+  const double us = t.launch + rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) {
+                      return t.tile[i] + blocks * t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill);
+                    });
+  const double mn = (double)M * (double)N * 1e-6;
+  const double stream = ((double)N + (double)M) * (double)K * 1e-6 / t.stream + mn * 2.0 * t.result_us_per_mb + t.stream_us;
+  return norm_of(us, stream, 6.0) + (splits > 1 ? t.split_us + t.split_us_per_mb * splits * mn * 4.0 : 0.0);
+}
+double two_phase_us(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  const double blocks = (double)ceil_div(K, KSTEP);
+  return t.launch + rounds_of(ceil_div(M, 256) * ceil_div(N, 256), NUM_CUS, [&](double fill) {
+           return norm_of(t.pp_tile + blocks * t.pp_block * (1.0 + t.pp_busy * fill), t.pp_store * fill, 6.0);
+         });
+}
+double wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K) {
+  const int bm = WAVESPLIT_TILES[i].bm, bn = WAVESPLIT_TILES[i].bn;
+  const double kbytes = (double)(bm + bn) * (double)K * 1e-3;
+  const double us = t.ws_launch + rounds_of(ceil_div(M, bm) * ceil_div(N, bn), NUM_CUS, [&](double fill) {
+                      return t.ws_tile + kbytes * (t.ws_kb + t.ws_kb_busy * fill) + (double)(bm * bn) / 1024.0 * t.ws_result;
+                    });
+  return norm_of(us, (double)N * (double)K * 1e-6 / t.ws_stream + t.ws_stream_us, t.ws_norm);
+}
+
+TileChoice best_wavesplit_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+  constexpr int COUNT = sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0]);
+  for (int i = 0; i < COUNT; ++i) {
+    const double us = wavesplit_tile_us(t, i, M, N, K);
+    if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
+  }
+  return best;
+}
+TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+  const int64_t kb = ceil_div(K, KSTEP);
+  for (int i = 0; i < 13; ++i) {
+    const int64_t tiles = ceil_div(M, MID_TILES[i].bm) * ceil_div(N, MID_TILES[i].bn);
+    int previous = 0;
+    for (int want = 1; want <= 16; ++want) {
+      const int per = (int)ceil_div(kb, want), splits = (int)ceil_div(kb, per);
+      if (splits > 1 && (N % 4 != 0 || per < 4 || tiles * splits > 560 || tiles > 200)) break;
+      if (splits == previous) continue;
+      previous = splits;
+      const double us = dma_tile_us(t, i, M, N, K, splits);
+      if (us < best.us) best = {TF_DMA, MID_TILES[i].bm, MID_TILES[i].bn, splits, us};
+    }
+  }
+  return best;
+}
+
+// More than 16 tokens, K % 128 == 0, aligned operands: the fastest tile, or TF_NONE where `base`, what the route names (a mid-M
+// tile or the two-phase tile), models within 5 % of it (the two-phase tile 10 %): below that the model does not order two tiles.
+TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base) {
+  const TileTimes& t = kind == GK_F32 || kind == GK_UE8M0 ? SCALED_TIMES : PLAIN_TIMES;
+  TileChoice best = best_dma_tile(t, M, N, K);
+  if (N * K <= 100000000) {  // (a larger weight streams better through the wide tiles: K = 4096 -> N = 28672 at 48 tokens 27.2 against 33.6 us)
+    const TileChoice ws = best_wavesplit_tile(t, M, N, K);
+    if (ws.us < best.us) best = ws;
+  }
+  if (M > 128) {
+    const double us = two_phase_us(t, M, N, K);
+    if (us < best.us) best = {TF_TWO_PHASE, 256, 256, 1, us};
+  }
+  double base_us = 1e30;
+  if (base.family == TF_TWO_PHASE) base_us = two_phase_us(t, M, N, K);
+  if (base.family == TF_DMA)
+    for (int i = 0; i < 13; ++i)
+      if (MID_TILES[i].bm == base.bm && MID_TILES[i].bn == base.bn) base_us = dma_tile_us(t, i, M, N, K, base.splits);
+  // (bound by a large weight's stream, the model knows little of how many CUs it takes: K = 10880 -> N = 16896 at 36 tokens, 132
+  // unsplit tiles instead of 198 split ones, 54.8 against 48.3 us)
+  const double margin = base.family == TF_TWO_PHASE ? 0.90 : M <= 64 && N * K > 100000000 ? 0.85 : 0.95;
+  return best.us < margin * base_us ? best : TileChoice{TF_NONE, 0, 0, 1, 0.0};
+}
+
+// K not a multiple of 128 (scales in the epilogue only): the wave-split tile against the generic kernel, which takes at least
+// twice as long as the mid-M tile would (K = 5920 -> N = 8320 at 90 tokens INT8: 42 against 18 us); not for the largest weights,
+// which the tile fetches once per 64 tokens (K = 16016 -> N = 26880 at 256 tokens 320 against 260 us).
+TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
+  const TileChoice ws = best_wavesplit_tile(PLAIN_TIMES, M, N, K);
+  return N * K <= 100000000 && ws.us < 2.0 * best_dma_tile(PLAIN_TIMES, M, N, K).us ? ws : TileChoice{TF_NONE, 0, 0, 1, 0.0};
+}
+
+// Up to 16 tokens: the wave-split tile against the streaming and the register wave-split kernel.  It wins wherever K has more
+// than 16 blocks and the weight is not one of the largest (us, the other / the tile, one token and 16; FP8):
+//   K = 7168: N = 576 6.8/5.1, 9.4/5.6;  2048 6.9/5.2, 8.8/6.5;  K = 14336: N = 512 9.9/6.8, 8.0/6.8;  K = 5120: N = 10240 16.0/10.2, 13.9/10.5
+//   K = 18432: N = 896 12.4/7.7, 11.6/9.4;  7168 23.3/23.1, 28.1/25.0;  K = 4096: N = 6144 7.5/6.3, 9.7/6.2;  28672 22.9/24.7, 26.1/25.5
+// because its operands come in whole 128-byte lines: 16 rows x 64 bytes per instruction, which is what the MFMA's layout asks
+// for when loaded straight into registers, pass through a CU's cache at 16 bytes a cycle, whole lines at 61.
+// With fewer K blocks both are bound by the launch (K = 2048 -> N = 2048 4.3 / 4.4) except where there are many channels
+// (K = 1024 -> N = 12288 5.8/4.8, 8.0/4.9; but 512 -> 32768 5.9/6.8, 1536 -> 24576 9.3/9.6).
+TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+  const int64_t kb = ceil_div(K, KSTEP), weight = N * K;
+  // (the largest weights: the register kernel's single-tile stream is as fast for few tokens, unless it pads K to whole turns of 32 blocks)
+  const bool padded = kb <= 64 && (kb + 31) / 32 * 32 * 4 > kb * 5;
+  const int64_t most = M > (kind == GK_F32 ? 6 : 8) || kb > 64 || padded ? 140000000 : 100000000;
+  const bool take = kb > 16 ? weight <= most : kb >= 8 && N >= 7168 && weight <= 20000000 && M > 8;
+  if (!take) return TileChoice{TF_NONE, 0, 0, 1, 0.0};
+  const TileTimes& t = kind == GK_F32 || kind == GK_UE8M0 ? SCALED_TIMES : PLAIN_TIMES;
+  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+  for (int i = 0; i < 3; ++i) {
+    static_assert(WAVESPLIT_TILES[2].bm == 16, "the 16-token tiles come first");
+    const double us = wavesplit_tile_us(t, i, M, N, K);
+    if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
+  }
+  return best;
+}
+
+}  // namespace
+}  // namespace mi355
