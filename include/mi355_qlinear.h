@@ -36,6 +36,10 @@ enum {
   MI355_I32 = 5
 };
 
+/* Or-ed into out_dtype of the block-FP8 linears: the bias is added to the result rounded to the output type, as a separate
+ * `output += bias` does (fp8_utils.py:208-209), bit for bit; without it the bias is added in fp32 before the only rounding. */
+enum { MI355_BIAS_ON_ROUNDED = 0x100 };
+
 /* How the group quantizer scales an element once the group's amax is known. */
 enum {
   MI355_QUANT_DIV = 0, /* s = amax / qmax;          q = x / s           (per_token_group_quant_8bit.cu:86,:110) */
@@ -373,7 +377,7 @@ int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const flo
  *          (python/sglang/srt/layers/quantization/fp8_utils.py:184-214, :281-301): per_token_group_quant_fp8, the blockwise
  *          GEMM and `output += bias`.  The activation is quantized with q = x / s (s = max(amax, 1e-10) / 448) into the
  *          workspace, with M-major scales, and the bias is added in fp32 in the GEMM epilogue (the reference adds it
- *          after rounding the GEMM result to the output type).  At decode sizes (M <= 16, 16-bit x, N % 128 == 0) there
+ *          after rounding the GEMM result to the output type: MI355_BIAS_ON_ROUNDED).  At decode sizes (M <= 16, 16-bit x, N % 128 == 0) there
  *          is no quantizer launch where that is the faster way: the GEMM kernel quantizes the tokens itself (the wave-split
  *          and streaming kernels in their prologues, the mid-M kernel by producer waves), with the same arithmetic; the result
  *          is bit-identical to the two-step sequence where the GEMM alone takes the same kernel.

@@ -26,6 +26,7 @@ struct GemmParams {
   const float* sa;
   const float* sb;
   const void* bias;        // optional [N] in the output dtype (INT8 GEMM; per-channel FP8 epilogue)
+  int bias_rounded;        // FP8 only: the result is rounded to the output dtype before the bias is added (`out += bias`)
   const float* col_scale;  // FP8 only, optional [N]: per-channel scale applied in the epilogue (fp8_scaled_mm)
   const float* row_scale;  // FP8 two-phase and mid-M kernels in their epilogue-scaled mode (no scales in the K loop): per-token scale [M]
   const void* x16;         // FP8 decode kernel only, optional: unquantized tokens [M, K] (x_dtype, row stride ldx elements);
@@ -128,6 +129,22 @@ __device__ __forceinline__ void store_out4(void* out, int out_dtype, int64_t off
 }
 
 
+// Four results rounded to the 16-bit output dtype, for a bias that is added to the rounded result.
+template <bool BF16>
+__device__ __forceinline__ void round_to_16_bits(float* r) {
+#pragma unroll
+  for (int v = 0; v < 4; v += 2) {
+    const uint32_t w = BF16 ? pack_bf16x2(r[v], r[v + 1]) : pack_f16x2(r[v], r[v + 1]);
+    r[v] = BF16 ? __uint_as_float(w << 16) : f16_bits_to_f32(w & 0xffffu);
+    r[v + 1] = BF16 ? __uint_as_float(w & 0xffff0000u) : f16_bits_to_f32(w >> 16);
+  }
+}
+__device__ __forceinline__ void round_before_bias(const GemmParams& p, float* r) {
+  if (!p.bias_rounded) return;
+  if (p.out_dtype == MI355_BF16) round_to_16_bits<true>(r);
+  else round_to_16_bits<false>(r);
+}
+
 // Optional per-channel epilogue of the FP8 kernels: r[v] = col_scale[n + v] * r[v] + bias[n + v] for the four consecutive
 // channels n .. n + 3 (channels at or past N repeat the last one; they are never stored).
 __device__ __forceinline__ void fp8_channel_epilogue(const GemmParams& p, int n, float* r) {
@@ -144,6 +161,7 @@ __device__ __forceinline__ void fp8_channel_epilogue(const GemmParams& p, int n,
     }
   }
   if (p.bias) {
+    round_before_bias(p, r);
     const uint16_t* b = reinterpret_cast<const uint16_t*>(p.bias);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -204,7 +222,11 @@ __device__ __forceinline__ void fp8_apply_terms(const GemmParams& p, const Chann
   for (int v = 0; v < 4; ++v) {
     if (p.col_scale) r[v] = mul_rn(c.scale[v], r[v]);
     if (p.row_scale) r[v] = mul_rn(token_scale, r[v]);
-    if (p.bias) r[v] = add_rn(r[v], c.bias[v]);
+  }
+  if (p.bias) {
+    round_before_bias(p, r);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) r[v] = add_rn(r[v], c.bias[v]);
   }
 }
 
@@ -241,7 +263,7 @@ __device__ __forceinline__ void out_tile_put(const GemmParams& p, uint8_t* tile,
     put[i] = tile + row0 * (BN * 2) + (((col >> 3) ^ (row0 & 7)) << 4) + ((col >> 2) & 1) * 8;
   }
   auto emit = [&](auto bf16_c, auto bias_c) {
-    constexpr bool BF16 = decltype(bf16_c)::value, BIAS = decltype(bias_c)::value;
+    constexpr bool BF16 = decltype(bf16_c)::value, BIAS = decltype(bias_c)::value != 0, ROUNDED = decltype(bias_c)::value == 2;
     const float* row_scales = OS == OUT_INT8 ? p.sa : p.row_scale;
     float token_scale[MT];
     if constexpr (OS != OUT_PLAIN) {
@@ -265,19 +287,27 @@ __device__ __forceinline__ void out_tile_put(const GemmParams& p, uint8_t* tile,
           if constexpr (OS == OUT_INT8) r[v] = mul_rn((float)acc[i][j][v], mul_rn(cs[v], token_scale[j]));
           else if constexpr (OS == OUT_ROW_COL) r[v] = mul_rn(token_scale[j], mul_rn(cs[v], acc[i][j][v]));
           else r[v] = acc[i][j][v];
-          if constexpr (BIAS) r[v] = add_rn(r[v], BF16 ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]));
         }
+        if constexpr (ROUNDED) round_to_16_bits<BF16>(r);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if constexpr (BIAS) r[v] = add_rn(r[v], BF16 ? bf16_bits_to_f32(h[v]) : f16_bits_to_f32(h[v]));
         *reinterpret_cast<u32x2*>(put[i] + j * 16 * (BN * 2)) =
             BF16 ? u32x2{pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])} : u32x2{pack_f16x2(r[0], r[1]), pack_f16x2(r[2], r[3])};
       }
     }
   };
+  using NoBias = std::integral_constant<int, 0>;
+  using Bias = std::integral_constant<int, 1>;
+  using BiasOnRounded = std::integral_constant<int, OS == OUT_PLAIN ? 2 : 1>;  // (block scales only)
   if (p.out_dtype == MI355_BF16) {
-    if (p.bias) emit(std::true_type{}, std::true_type{});
-    else emit(std::true_type{}, std::false_type{});
+    if (OS == OUT_PLAIN && p.bias_rounded && p.bias) emit(std::true_type{}, BiasOnRounded{});
+    else if (p.bias) emit(std::true_type{}, Bias{});
+    else emit(std::true_type{}, NoBias{});
   } else {
-    if (p.bias) emit(std::false_type{}, std::true_type{});
-    else emit(std::false_type{}, std::false_type{});
+    if (OS == OUT_PLAIN && p.bias_rounded && p.bias) emit(std::false_type{}, BiasOnRounded{});
+    else if (p.bias) emit(std::false_type{}, Bias{});
+    else emit(std::false_type{}, NoBias{});
   }
 }
 // Called by all 512 threads after a barrier that follows the last out_tile_put; rows at or past M and channels at or past N

@@ -939,6 +939,8 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
                                             int64_t ldb, int64_t sa_sk, int64_t sb_sn, int64_t sb_sk, int64_t ldo,
                                             void* workspace, size_t workspace_bytes_given, void* stream) {
   const char* what = "mi355_fp8_blockwise_mm_ue8m0";
+  const int bias_rounded = (out_dtype & MI355_BIAS_ON_ROUNDED) != 0;
+  out_dtype &= ~MI355_BIAS_ON_ROUNDED;
   GemmParams p;
   bool empty;
   // strides of the packed words stand in for the fp32 scale strides of the shared argument check
@@ -949,7 +951,7 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
                 MI355_ERR_INVALID_ARGUMENT, "%s: scale words must be 4-byte aligned", what);
   MI355_REQUIRE(bias == nullptr || out_dtype != MI355_F32, MI355_ERR_INVALID_ARGUMENT,
                 "%s: a bias needs a 16-bit output type (it has the output's type)", what);
-  p.bias = bias;
+  p.bias = bias, p.bias_rounded = bias_rounded;
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
   const Route r = run_route(GK_UE8M0, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
@@ -1181,6 +1183,8 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
                  int64_t ws_sk, const void* bias, void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw,
                  int64_t ldo, void* workspace, size_t workspace_bytes_given, void* stream) {
   clear_error();
+  const int bias_rounded = (out_dtype & MI355_BIAS_ON_ROUNDED) != 0;
+  out_dtype &= ~MI355_BIAS_ON_ROUNDED;
   MI355_REQUIRE(quant_mode == MI355_QUANT_DIV || quant_mode == MI355_QUANT_RCP, MI355_ERR_INVALID_ARGUMENT,
                 "%s: quant_mode must be MI355_QUANT_DIV or MI355_QUANT_RCP", what);
   MI355_REQUIRE(M >= 0 && N >= 0 && K >= 0, MI355_ERR_INVALID_ARGUMENT, "%s: negative shape", what);
@@ -1213,7 +1217,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
     bool empty;
     const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, pitch, ws_sn, ws_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
-    p.bias = bias;
+    p.bias = bias, p.bias_rounded = bias_rounded;
     p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
     if (tile_quant) return run_tile_quant(p, WavesplitQuant::BLOCK_F32, run, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::BLOCK_F32, x, x_dtype, stream, what);
@@ -1225,7 +1229,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
       bool empty;
       const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, (M + 3) & ~3ll, ws_sn, ws_sk, ldo, p, empty);
       if (rc != MI355_OK || empty) return rc;
-      p.bias = bias;
+      p.bias = bias, p.bias_rounded = bias_rounded;
       p.x16 = x, p.ldx = K, p.x_dtype = x_dtype, p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
       p.kb_total = K / KSTEP, p.splits = 1, p.kb_per_split = p.kb_total;
       return launch_fp8_dma3_quant(p, plain.bn, static_cast<hipStream_t>(stream), what);
@@ -1237,7 +1241,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
     // a / sa are not read by the kernel in this mode; they only have to satisfy the checks
     int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, (M + 3) & ~3ll, ws_sn, ws_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
-    p.bias = bias;
+    p.bias = bias, p.bias_rounded = bias_rounded;
     p.x16 = x, p.ldx = K, p.x_dtype = x_dtype, p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
     return run_gemm<true>(p, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
   }
@@ -1250,7 +1254,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   bool empty;
   rc = fp8_mm_params(what, q, w, sa, w_scale, out, out_dtype, M, N, K, K, ldw, 1, pitch, ws_sn, ws_sk, ldo, p, empty);
   if (rc != MI355_OK || empty) return rc;
-  p.bias = bias;
+  p.bias = bias, p.bias_rounded = bias_rounded;
   return run_gemm<true>(p, q + q_bytes + sa_bytes, workspace_bytes_given - q_bytes - sa_bytes, static_cast<hipStream_t>(stream), what);
 }
 }  // namespace
@@ -1428,6 +1432,8 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
                                             void* stream) {
   const char* what = "mi355_fp8_block_linear_ue8m0";
   clear_error();
+  const int bias_rounded = (out_dtype & MI355_BIAS_ON_ROUNDED) != 0;
+  out_dtype &= ~MI355_BIAS_ON_ROUNDED;
   MI355_REQUIRE(M >= 0 && N >= 0 && K >= 0, MI355_ERR_INVALID_ARGUMENT, "%s: negative shape", what);
   MI355_REQUIRE(out_dtype == MI355_BF16 || out_dtype == MI355_F16, MI355_ERR_INVALID_ARGUMENT,
                 "%s: out_dtype must be bfloat16 or float16", what);
@@ -1455,7 +1461,7 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
     const float* words = static_cast<const float*>(sb_words);  // (strides of the packed words stand in for fp32 ones)
     const int rc = fp8_mm_params(what, x, w, words, words, out, out_dtype, M, N, K, K, ldw, 1, pitch, sb_sn, sb_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
-    p.bias = bias;
+    p.bias = bias, p.bias_rounded = bias_rounded;
     if (tile_quant) return run_tile_quant(p, WavesplitQuant::BLOCK_UE8M0, run, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::BLOCK_UE8M0, x, x_dtype, stream, what);
   }
@@ -1463,7 +1469,7 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
   const int rc = mi355_group_quant_8bit(x, x_dtype, q, MI355_FP8_E4M3FN, sa_words, M, K, KSTEP, 1e-10f, -448.0f, 448.0f,
                                         MI355_QUANT_MUL, MI355_SCALE_UE8M0_PACKED, 0.0f, 1, pitch, stream);
   if (rc != MI355_OK) return rc;
-  return mi355_fp8_blockwise_mm_ue8m0(q, w, sa_words, sb_words, bias, out, out_dtype, M, N, K, K, ldw, pitch, sb_sn, sb_sk, ldo,
+  return mi355_fp8_blockwise_mm_ue8m0(q, w, sa_words, sb_words, bias, out, out_dtype | (bias_rounded ? MI355_BIAS_ON_ROUNDED : 0), M, N, K, K, ldw, pitch, sb_sn, sb_sk, ldo,
                                       q + q_bytes + sa_bytes, workspace_bytes_given - q_bytes - sa_bytes, stream);
 }
 

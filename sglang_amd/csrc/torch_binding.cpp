@@ -16,6 +16,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/Allocator.h>
+#include <c10/core/GradMode.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/Dtype.h>
@@ -515,18 +516,18 @@ void check_bias(const OptTensor& bias, int64_t N, ScalarType out_dtype, const ch
 
 // The launches without checks: `x` holds M rows of K values, `out` M rows of N.
 void launch_block_linear(const Tensor& x, const Tensor& w, const Tensor& ws, const void* bias, const Tensor& out, int64_t M, int64_t N,
-                         int64_t K, bool by_reciprocal) {
+                         int64_t K, bool by_reciprocal, int bias_flag = 0) {
   const Workspace mem(mi355_fp8_block_linear_workspace_bytes(M, N, K));
   check(mi355_fp8_block_linear_mode(x.const_data_ptr(), dtype_code(x.scalar_type()), by_reciprocal ? MI355_QUANT_RCP : MI355_QUANT_DIV,
                                     w.const_data_ptr(), static_cast<const float*>(ws.const_data_ptr()), ws.stride(0), ws.stride(1), bias,
-                                    out.data_ptr(), dtype_code(out.scalar_type()), M, N, K, w.stride(0), N, mem.ptr(), mem.bytes,
+                                    out.data_ptr(), dtype_code(out.scalar_type()) | bias_flag, M, N, K, w.stride(0), N, mem.ptr(), mem.bytes,
                                     current_stream()));
 }
 void launch_block_linear_ue8m0(const Tensor& x, const Tensor& w, const Tensor& words, const void* bias, const Tensor& out, int64_t M,
-                               int64_t N, int64_t K) {
+                               int64_t N, int64_t K, int bias_flag = 0) {
   const Workspace mem(mi355_fp8_block_linear_ue8m0_workspace_bytes(M, N, K));
   check(mi355_fp8_block_linear_ue8m0(x.const_data_ptr(), dtype_code(x.scalar_type()), w.const_data_ptr(), words.const_data_ptr(),
-                                     words.stride(0), words.stride(1), bias, out.data_ptr(), dtype_code(out.scalar_type()), M, N, K,
+                                     words.stride(0), words.stride(1), bias, out.data_ptr(), dtype_code(out.scalar_type()) | bias_flag, M, N, K,
                                      w.stride(0), N, mem.ptr(), mem.bytes, current_stream()));
 }
 void launch_per_token_linear(const Tensor& x, const Tensor& w_kn, const Tensor& ws, const void* bias, const Tensor& out, int64_t M,
@@ -639,6 +640,12 @@ bool plain_epilogue_bias(const OptTensor& bias, ScalarType dtype, int64_t N) {
   return !given(bias) || (bias->is_cuda() && bias->scalar_type() == dtype && bias->is_contiguous() && bias->numel() == N);
 }
 
+// `output += bias` in the GEMM's epilogue (same bits, no pass over the output) where nothing about it is unusual
+bool fused_bias(const OptTensor& bias, const Tensor& out, int64_t N) {
+  return given(bias) && bias->dim() == 1 && bias->numel() == N && bias->is_contiguous() && bias->scalar_type() == out.scalar_type() &&
+         bias->device() == out.device() && !(bias->requires_grad() && c10::GradMode::is_enabled());
+}
+
 // fp8_utils.triton_w8a8_block_fp8_linear / cutlass_w8a8_block_fp8_linear_with_fallback: the latter's `x / s` quantizer for
 // N a multiple of 128, else the former's `x * (1 / s)`; the bias is added to the rounded output.
 std::optional<Tensor> try_block_linear(const Tensor& x, const Tensor& w, const Tensor& ws, const OptTensor& bias, bool triton) {
@@ -649,8 +656,9 @@ std::optional<Tensor> try_block_linear(const Tensor& x, const Tensor& w, const T
   if (ws.scalar_type() != ScalarType::Float || !ws.is_cuda() || ws.dim() != 2 || ws.size(0) != (N + 127) / 128 || ws.size(1) != K / 128)
     return std::nullopt;
   Tensor out = new_output(x, N);
-  launch_block_linear(x, w, ws, nullptr, out, M, N, K, triton || N % 128 != 0);
-  if (given(bias)) out.add_(*bias);
+  const bool fused = fused_bias(bias, out, N);
+  launch_block_linear(x, w, ws, fused ? bias->const_data_ptr() : nullptr, out, M, N, K, triton || N % 128 != 0, MI355_BIAS_ON_ROUNDED);
+  if (given(bias) && !fused) out.add_(*bias);
   return out;
 }
 
@@ -663,8 +671,9 @@ std::optional<Tensor> try_block_linear_ue8m0(const Tensor& x, const Tensor& w, c
   if (words.scalar_type() != ScalarType::Int || !words.is_cuda() || words.dim() != 2 || words.size(0) != N || words.size(1) < (K / 128 + 3) / 4)
     return std::nullopt;
   Tensor out = new_output(x, N);
-  launch_block_linear_ue8m0(x, w, words, nullptr, out, M, N, K);
-  if (given(bias)) out.add_(*bias);
+  const bool fused = fused_bias(bias, out, N);
+  launch_block_linear_ue8m0(x, w, words, fused ? bias->const_data_ptr() : nullptr, out, M, N, K, MI355_BIAS_ON_ROUNDED);
+  if (given(bias) && !fused) out.add_(*bias);
   return out;
 }
 
