@@ -102,11 +102,12 @@ __device__ __forceinline__ float clamp448(float v) { return fmaxf(fminf(v, 448.0
 // order - with streaming loads: what the first pass left in the caches is then still there when the second arrives
 // (both passes: 108 -> 96 us on 235 MB of bf16; with a grid-stride second pass 102 us, with streaming loads in the
 // FIRST pass 106 us, walking the ranges backwards 99 us).
-template <int DT>
-__global__ __launch_bounds__(ABSMAX_THREADS) void per_tensor_quant_kernel(const void* x, uint8_t* q, const float* scale, int64_t n,
+// A static scale has no first pass: then the ranges are those of launch_static below, and a small tensor's codes are stored so
+// that the GEMM behind finds them in the caches.
+template <int DT, int T, int U, bool STREAM>
+__global__ __launch_bounds__(T) void per_tensor_quant_kernel(const void* x, uint8_t* q, const float* scale, int64_t n,
                                                                           float* scale_rows, int64_t rows) {
   constexpr int VEC = (DT == MI355_F32) ? 4 : 8;
-  constexpr int U = ABSMAX_UNROLL, T = ABSMAX_THREADS;
   const int64_t gid = (int64_t)blockIdx.x * T + threadIdx.x, stride = (int64_t)gridDim.x * T;
   const float s = *scale;
   const float inv = 1.0f / s;
@@ -124,7 +125,9 @@ __global__ __launch_bounds__(ABSMAX_THREADS) void per_tensor_quant_kernel(const 
       c = __builtin_amdgcn_cvt_pk_fp8_f32(clamp448(f[4 * j + 2] * inv), clamp448(f[4 * j + 3] * inv), c, true);
       w[j] = (uint32_t)c;
     }
-    if constexpr (VEC == 8)
+    if constexpr (VEC == 8 && !STREAM)
+      *reinterpret_cast<u32x2*>(q + v * VEC) = u32x2{w[0], w[1]};
+    else if constexpr (VEC == 8)
       __builtin_nontemporal_store(u32x2{w[0], w[1]}, reinterpret_cast<u32x2*>(q + v * VEC));
     else
       *reinterpret_cast<uint32_t*>(q + v * VEC) = w[0];
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(ABSMAX_THREADS) void per_tensor_quant_kernel(const 
   const int64_t per = (nvec + gridDim.x - 1) / gridDim.x;
   const int64_t begin = (int64_t)blockIdx.x * per, end = min(nvec, begin + per);
   int64_t v = begin + threadIdx.x;
-  for (; v + (U - 1) * T < end; v += U * T) {  // eight loads in flight per thread
+  for (; v + (U - 1) * T < end; v += U * T) {  // U loads in flight per thread
     u32x4 r[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) r[u] = __builtin_nontemporal_load(src + v + u * T);
@@ -146,14 +149,27 @@ __global__ __launch_bounds__(ABSMAX_THREADS) void per_tensor_quant_kernel(const 
   }
 }
 
+// Static scale: bound by latency up to a few MB, so as many small workgroups as there are - one vector per thread until every CU
+// has its waves, then four - instead of the 1024 threads x 8 vectors that suit two passes (238 x 4480 fp16: 17 workgroups, 6.1 us;
+// 521 now, 3.3 us; 763 x 6144 10.9 -> 4.6 us).
+template <int DT>
+void launch_static(const void* x, uint8_t* q, float* scale, int64_t n, float* scale_rows, int64_t rows, hipStream_t st) {
+  const int64_t nvec = n / ((DT == MI355_F32) ? 4 : 8);
+  if (nvec <= 256 * 2048)
+    hipLaunchKernelGGL((per_tensor_quant_kernel<DT, 256, 1, false>), dim3((unsigned)std::max<int64_t>(1, (nvec + 255) / 256)), dim3(256), 0, st, x, q, scale, n, scale_rows, rows);
+  else
+    hipLaunchKernelGGL((per_tensor_quant_kernel<DT, 256, 4, true>), dim3((unsigned)std::min<int64_t>((nvec + 1023) / 1024, 1 << 20)), dim3(256), 0, st, x, q, scale, n, scale_rows, rows);
+}
+
 template <int DT>
 void launch_both(const void* x, uint8_t* q, float* scale, int64_t n, bool is_static, float* scale_rows, int64_t rows,
                  hipStream_t st) {
   // both passes use the same grid, so that a workgroup of the second pass re-reads what its namesake of the first pass read
+  if (is_static) return launch_static<DT>(x, q, scale, n, scale_rows, rows, st);
   const int64_t per_wg = (int64_t)ABSMAX_THREADS * ABSMAX_UNROLL * ((DT == MI355_F32) ? 4 : 8);
   const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + per_wg - 1) / per_wg, ABSMAX_MAX_WGS));
-  if (!is_static) hipLaunchKernelGGL(per_tensor_absmax_kernel<DT>, dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, scale, n);
-  hipLaunchKernelGGL(per_tensor_quant_kernel<DT>, dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, q, scale, n, scale_rows, rows);
+  hipLaunchKernelGGL(per_tensor_absmax_kernel<DT>, dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, scale, n);
+  hipLaunchKernelGGL((per_tensor_quant_kernel<DT, ABSMAX_THREADS, ABSMAX_UNROLL, true>), dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, q, scale, n, scale_rows, rows);
 }
 
 }  // namespace

@@ -11,11 +11,9 @@
 //         scale = max(absmax, eps) / 448 and either q = e4m3fn(clamp(x * (1 / scale))), the arithmetic of the Triton kernel
 //         python/sglang/srt/layers/quantization/fp8_kernel.py:122-161, or q = e4m3fn(clamp(x / scale)) with a true
 //         division, the arithmetic of sgl-kernel/csrc/gemm/per_token_group_quant_8bit.cu:25-114.
-// Rows of up to 8192 two-byte elements stay in registers between the two phases; longer rows are
-// re-read (from L2).
-// Two-byte inputs with rows of at most 8192 elements (every hidden size of the benchmark models) take a second kernel: one
-// WAVE per row, four rows per workgroup, the row in registers (up to 16 x 16 bytes per lane), no LDS and no barrier -
-// 16384 workgroups of one short row each spend a visible share of their life starting up and at the barrier.
+// Two-byte inputs: rows of up to 24576 elements stay in registers between the two phases (per_token_quant_row_kernel; thousands of
+// short rows, and the mode with row sums up to 8192 elements, one WAVE per row, four rows per workgroup, no LDS and no barrier).
+// Other rows take per_token_quant_kernel, which reads again (from L2) what its registers do not hold.
 #include "common.h"
 
 namespace mi355 {
@@ -166,6 +164,44 @@ __global__ __launch_bounds__(256) void per_token_quant_wave_kernel(const void* x
   }
 }
 
+// One workgroup of T threads per row, the row in registers: NV vectors of eight two-byte elements per thread (K <= 8 * T * NV), all
+// requested before the first is looked at.
+template <int DT, bool FP8_OUT, int T, int NV>
+__global__ __launch_bounds__(T) void per_token_quant_row_kernel(const void* x, int8_t* q, float* s, int64_t K) {
+  static_assert(DT != MI355_F32, "two-byte inputs");
+  __shared__ float wave_max[T / 64];
+  const int64_t row = blockIdx.x;
+  const int nvec = (int)(K / 8);
+  const u32x4* src = reinterpret_cast<const u32x4*>(x) + row * nvec;
+  u32x4 keep[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = threadIdx.x + T * i;
+    keep[i] = (v < nvec) ? __builtin_nontemporal_load(src + v) : u32x4{0, 0, 0, 0};
+  }
+  float amax = FP8_OUT ? 0.f : 1e-10f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[8];
+    unpack16<DT>(keep[i], f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(f[j]));
+  }
+  amax = wave_allreduce_max(amax);
+  if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) amax = fmaxf(amax, wave_max[w]);
+  float mul;
+  const float scale = row_scale<FP8_OUT>(amax, mul);
+  if (threadIdx.x == 0) s[row] = scale;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = threadIdx.x + T * i;
+    if (v < nvec) emit_vector<DT, FP8_OUT, false>(keep[i], mul, q + row * K + (int64_t)v * 8);
+  }
+}
+
 // ROW_GROUP (FP8 only): the row is one quantization group: absmax floored at eps; DIVIDE: elements are divided by the
 // scale instead of multiplied by its reciprocal.
 template <int DT, bool FP8_OUT, bool ROW_GROUP = false, bool DIVIDE = false, bool SUM = false>
@@ -256,6 +292,33 @@ int per_token_quant(const char* what, const void* x, int x_dtype, void* q, float
   MI355_REQUIRE(M < (1ll << 31), MI355_ERR_INVALID_ARGUMENT, "%s: too many rows", what);
   hipStream_t st = static_cast<hipStream_t>(stream);
   int8_t* qq = static_cast<int8_t*>(q);
+  if constexpr (!ROW_GROUP && !SUM) {
+    // Rows in the registers of one workgroup: with few rows as many threads as a row has vectors (latency), with many rows more
+    // vectors per thread (fewer barriers).  us before / now, FP8 and INT8:  160 x 7168 4.6 / 2.9, 5.6 / 3.1;  512 x 4096 3.9 / 3.0,
+    // 4.5 / 3.1;  2048 x 14336 16.7 / 15.9, 18.2 / 16.5;  4096 x 18432 55 / 37 (rows beyond 8192 elements used to be read twice).
+    // Thousands of rows of up to 4096 elements stay with the wave per row (4096 x 4096 INT8 10.6 against 10.8).
+    if (x_dtype != MI355_F32 && K <= 8 * 512 * 6 && !(M > 3072 && K <= 4096)) {
+#define MI355_ROWS(T, NV)                                                                                                              \
+  {                                                                                                                                    \
+    if (x_dtype == MI355_BF16) hipLaunchKernelGGL((per_token_quant_row_kernel<MI355_BF16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K); \
+    else hipLaunchKernelGGL((per_token_quant_row_kernel<MI355_F16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K);  \
+  }
+      const bool few = M <= 640;
+      if (K <= 2048) {
+        if (few) MI355_ROWS(256, 1) else MI355_ROWS(128, 2)
+      } else if (K <= 4096) {
+        if (few) MI355_ROWS(512, 1) else MI355_ROWS(128, 4)
+      } else if (K <= 8192) {
+        if (few) MI355_ROWS(512, 2) else MI355_ROWS(256, 4)
+      } else if (K <= 16384) {
+        MI355_ROWS(512, 4)
+      } else {
+        MI355_ROWS(512, 6)
+      }
+#undef MI355_ROWS
+      return check_launch(what);
+    }
+  }
   if (!ROW_GROUP && x_dtype != MI355_F32 && K <= 8192) {  // one wave per row
     const dim3 grid((unsigned)((M + 3) / 4));
     const int nv = (int)((K / 8 + 63) / 64);
