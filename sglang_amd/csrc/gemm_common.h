@@ -442,7 +442,7 @@ __device__ __forceinline__ bool grouped_tile_of_block(const GroupedParams& gp, G
   p.M = __builtin_amdgcn_readfirstlane(rec.z);
   return true;
 }
-int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, hipStream_t stream, const char* what);  // gemm_fp8_dma3.hip; bm: 64 or 128
+int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, hipStream_t stream, const char* what);  // gemm_fp8_dma3.hip; 64 or 128 x 128 or 256
 int launch_fp8_grouped_pp(GroupedParams& gp, hipStream_t stream, const char* what);            // gemm_fp8_pp.hip: 256-row tiles
 int launch_int8_dma3(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);  // gemm_int8_dma3.hip: same tiling, int8 MFMA, int32 partials
 

@@ -287,12 +287,12 @@ __global__ __launch_bounds__(T_THREADS + 64 * T_PW) void fp8_gemm_dma3_q_kernel(
 
 // Grouped problems (see GroupedParams): the workgroup's token tile comes from the table the plan kernel wrote, the
 // operand bases move to that tile's expert, and the ordinary tile runs.
-template <int BM>
-__global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void fp8_grouped_dma3_kernel(const GroupedParams gp) {
+template <int BM, int BN, int S>
+__global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + BN == 192 && S == 3 ? 4 : 2))) void fp8_grouped_dma_kernel(const GroupedParams gp) {
   GemmParams p;
   int m0, tile_n;
   if (!grouped_tile_of_block(gp, p, m0, tile_n)) return;  // the whole workgroup leaves before any barrier
-  dma_tile<AR_F32, BM, T_BN, false, 3>(p, m0, tile_n * T_BN, 0);
+  dma_tile<AR_F32, BM, BN, false, S>(p, m0, tile_n * BN, 0);
 }
 
 }  // namespace
@@ -385,14 +385,16 @@ Dma3Plan dma3_plan(int64_t M, int64_t N, int64_t K, bool is_int8) {
   return pl;
 }
 
-int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, hipStream_t stream, const char* what) {
-  gp.g.tiles_n = (gp.g.N + T_BN - 1) / T_BN;
+int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, hipStream_t stream, const char* what) {
+  gp.g.tiles_n = (gp.g.N + bn - 1) / bn;
   gp.g.splits = 1, gp.g.kb_per_split = gp.g.kb_total;
   const dim3 grid((unsigned)(gp.max_tiles_m * gp.g.tiles_n));
-  if (bm == 64)
-    hipLaunchKernelGGL(fp8_grouped_dma3_kernel<64>, grid, dim3(T_THREADS), 0, stream, gp);
-  else
-    hipLaunchKernelGGL(fp8_grouped_dma3_kernel<128>, grid, dim3(T_THREADS), 0, stream, gp);
+  const dim3 block(T_THREADS);
+  if (bm == 64 && bn == 128 && few) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, true)>), grid, block, 0, stream, gp);
+  else if (bm == 64 && bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, false)>), grid, block, 0, stream, gp);
+  else if (bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 128, stages_of(128, 128, true)>), grid, block, 0, stream, gp);
+  else if (bm == 64) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 256, stages_of(64, 256, true)>), grid, block, 0, stream, gp);
+  else hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 256, stages_of(128, 256, true)>), grid, block, 0, stream, gp);
   return check_launch(what);
 }
 

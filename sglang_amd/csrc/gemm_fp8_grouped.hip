@@ -6,19 +6,19 @@
 // expert_offsets[e] .. + problem_sizes[e][0], multiplies them with its own weight b[e] [N, K] (128 x 128 block scales
 // scales_b[e] [N / 128, K / 128]) and writes the same rows of out [total_m, N].  problem_sizes and expert_offsets live
 // on the device (they come out of the routing kernel), so the tile schedule is built on the device too:
-//   1. grouped_plan_kernel  - one workgroup; prefix sums over the experts' tile counts turn the problem sizes into one
+//   1. grouped_prepare_kernel - one workgroup turns the problem sizes, by prefix sums over the experts' tile counts, into one
 //      record per token tile (expert, rows, position) in two tables, 256-row tiles and 64/128-row tiles, each headed by
 //      its number of records; sizes are clamped into the stacked matrix, so inconsistent routing data cannot make a later kernel read
-//      or write out of bounds;
-//   2. grouped_relayout_scales_kernel - token scales re-laid out M-major (what the direct-to-LDS GEMMs read with 16-byte
-//      loads), every expert padded to start on a whole quad of rows;
-//   3. fp8_grouped_pp_kernel (gemm_fp8_pp.hip), the two-phase 256 x 256 tile kernel, over the first table, then
-//      fp8_grouped_dma3_kernel (gemm_fp8_dma3.hip), the three-stage (64 or 128) x 256 tile kernel, over the second:
+//      or write out of bounds.  The other workgroups re-lay the token scales out M-major (what the direct-to-LDS GEMMs read with
+//      16-byte loads), every expert padded to start on a whole quad of rows; they find the experts of their 32 rows themselves and
+//      wait for nobody (two launches, one after the other, took 9.6 us with the gap between them, this one 5);
+//   2. fp8_grouped_pp_kernel (gemm_fp8_pp.hip), the two-phase 256 x 256 tile kernel, over the first table, then
+//      fp8_grouped_dma_kernel (gemm_fp8_dma3.hip), the mid-M tile of 64 or 128 tokens x 128 or 256 channels, over the second:
 //      one workgroup per (token tile, channel tile).  The first launch is left out when no expert can have more than
-//      128 rows.
+//      128 rows, and where small tiles alone model faster (grouped_run): then every row goes to the second table.
 // Where the reference takes device arrays of per-expert pointers, strides and scale layouts as scratch that its own
 // set-up kernel fills, this interface takes the base pointers and strides and keeps its scratch in the workspace.
-#include "gemm_common.h"
+#include "tile_choice.h"
 
 namespace mi355 {
 namespace {
@@ -35,27 +35,31 @@ struct ExpertTiles {
   int row0, rows, big, small, small_first;  // tiles of each kind; first row (inside the expert) of the small tiles
 };
 __device__ __forceinline__ ExpertTiles expert_tiles(const int32_t* problem_sizes, const int32_t* expert_offsets, int e, int E,
-                                                    int total_m, int bm) {
+                                                    int total_m, int bm, bool use_big) {
   ExpertTiles t{0, 0, 0, 0, 0};
   if (e >= E) return t;
   t.row0 = min(max(expert_offsets[e], 0), total_m);
   t.rows = min(max(problem_sizes[3 * e], 0), total_m - t.row0);
-  t.big = t.rows / BIG;
+  t.big = use_big ? t.rows / BIG : 0;
   const int rest = t.rows - t.big * BIG;
-  if (rest > 128) t.big += 1;
+  if (use_big && rest > 128) t.big += 1;
   else t.small = (rest + bm - 1) / bm;
   t.small_first = t.big * BIG;
   return t;
 }
 
-__global__ __launch_bounds__(256) void grouped_plan_kernel(const int32_t* problem_sizes, const int32_t* expert_offsets, int E,
-                                                           int total_m, int bm, v4i* big_tiles, int max_big, v4i* small_tiles,
-                                                           int max_small) {
+struct GroupedTables {
+  int E, total_m, bm, use_big, max_big, max_small;
+  v4i *big_tiles, *small_tiles;
+};
+__device__ void grouped_plan(const int32_t* problem_sizes, const int32_t* expert_offsets, const GroupedTables& g) {
+  const int E = g.E, bm = g.bm, max_big = g.max_big, max_small = g.max_small;
+  v4i *big_tiles = g.big_tiles, *small_tiles = g.small_tiles;
   __shared__ int scan_b[256], scan_s[256];
   int base_b = 0, base_s = 0;
   for (int c = 0; c < E; c += 256) {
     const int e = c + (int)threadIdx.x;
-    const ExpertTiles t = expert_tiles(problem_sizes, expert_offsets, e, E, total_m, bm);
+    const ExpertTiles t = expert_tiles(problem_sizes, expert_offsets, e, E, g.total_m, bm, g.use_big);
     scan_b[threadIdx.x] = t.big, scan_s[threadIdx.x] = t.small;
     __syncthreads();
     for (int d = 1; d < 256; d <<= 1) {  // inclusive prefix sums
@@ -80,31 +84,48 @@ __global__ __launch_bounds__(256) void grouped_plan_kernel(const int32_t* proble
   }
 }
 
-// out[kb * pitch + col(e) + m] = sa[(row0 + m) * sa_sm + kb * sa_sk], col(e) = ((row0 + 3) & ~3) + 4 * e.
-// Up to 128 rows x 32 K blocks per workgroup, through LDS so that both sides are contiguous.  blockIdx.x walks the two
-// halves of every 256-row tile record, then the small tile records.
-__global__ __launch_bounds__(256) void grouped_relayout_scales_kernel(const float* sa, int64_t sa_sm, int64_t sa_sk, float* out,
-                                                                      int64_t pitch, int KB, int bm, const v4i* big_tiles,
-                                                                      int max_big, const v4i* small_tiles) {
-  __shared__ float tile[32][129];
-  const bool is_big = (int)blockIdx.x < 2 * max_big;
-  const int idx = is_big ? (int)(blockIdx.x >> 1) : (int)blockIdx.x - 2 * max_big;
-  const v4i* table = is_big ? big_tiles : small_tiles;
-  if (idx >= table[0].x) return;
-  const v4i rec = table[1 + idx];
-  const int first = rec.w + (is_big ? (int)(blockIdx.x & 1) * 128 : 0);  // first row, inside the expert
-  const int rows = min(is_big ? 128 : bm, rec.z - first);
-  if (rows <= 0) return;
-  const int k0 = blockIdx.y * 32;
+// Workgroup (x, y) < (chunks, K blocks / 32): out[kb * pitch + col(e) + m] = sa[(row0 + m) * sa_sm + kb * sa_sk] for 32 stacked rows x 32
+// K blocks, col(e) = ((row0 + 3) & ~3) + 4 * e, through LDS so that both sides are contiguous.  The last x: the tables.
+constexpr int CHUNK = 32;
+__global__ __launch_bounds__(256) void grouped_prepare_kernel(const int32_t* problem_sizes, const int32_t* expert_offsets, GroupedTables g,
+                                                              const float* sa, int64_t sa_sm, int64_t sa_sk, float* out, int64_t pitch, int KB) {
+  if (blockIdx.x == gridDim.x - 1) {
+    if (blockIdx.y == 0) grouped_plan(problem_sizes, expert_offsets, g);
+    return;
+  }
+  __shared__ float tile[32][CHUNK + 1];
+  __shared__ int owners[CHUNK], column[CHUNK];  // per row of the chunk: how many experts of the batch own it, and the row's column
+  const int r0 = blockIdx.x * CHUNK, r1 = min(r0 + CHUNK, g.total_m), k0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const float* src = sa + (int64_t)(rec.y + first) * sa_sm;
-  if (k0 + tx < KB)
-    for (int r = ty; r < rows; r += 8) tile[tx][r] = src[(int64_t)r * sa_sm + (int64_t)(k0 + tx) * sa_sk];
-  __syncthreads();
-  float* dst = out + ((rec.y + 3) & ~3) + 4 * rec.x + first;
-  for (int i = threadIdx.x; i < 32 * 128; i += 256) {
-    const int kk = i >> 7, m = i & 127;
-    if (m < rows && k0 + kk < KB) dst[(int64_t)(k0 + kk) * pitch + m] = tile[kk][m];
+  const bool k_fast = sa_sk < sa_sm;
+#pragma unroll
+  for (int i = ty; i < 32; i += 8) {
+    const int m = k_fast ? i : tx, kb = k_fast ? tx : i;
+    if (r0 + m < r1 && k0 + kb < KB) tile[kb][m] = sa[(int64_t)(r0 + m) * sa_sm + (int64_t)(k0 + kb) * sa_sk];
+  }
+  auto store = [&](int m, int col) {
+    for (int kb = ty; kb < 32; kb += 8)
+      if (k0 + kb < KB) out[(int64_t)(k0 + kb) * pitch + col] = tile[kb][m];
+  };
+  for (int c = 0; c < g.E; c += 256) {
+    if (threadIdx.x < CHUNK) owners[threadIdx.x] = 0;
+    __syncthreads();
+    const int e = c + (int)threadIdx.x;
+    const ExpertTiles t = expert_tiles(problem_sizes, expert_offsets, e, g.E, g.total_m, g.bm, false);
+    const int lo = max(t.row0, r0), hi = min(t.row0 + t.rows, r1), shift = ((t.row0 + 3) & ~3) + 4 * e - t.row0;
+    int shared_rows = 0;
+    if (e < g.E)
+      for (int m = lo; m < hi; ++m) shared_rows |= atomicAdd(&owners[m - r0], 1), column[m - r0] = shift + m;
+    if (__syncthreads_or(shared_rows) == 0) {  // every row has one owner at most: all rows at once
+      if (owners[tx]) store(tx, column[tx]);
+    } else {  // inconsistent offsets: expert by expert
+      for (int i = 0; i < 256 && c + i < g.E; ++i) {
+        const ExpertTiles o = expert_tiles(problem_sizes, expert_offsets, c + i, g.E, g.total_m, g.bm, false);
+        const int m = r0 + tx;
+        if (m >= o.row0 && m < min(o.row0 + o.rows, r1)) store(tx, ((o.row0 + 3) & ~3) + 4 * (c + i) + m - o.row0);
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -112,7 +133,7 @@ struct GroupedPlan {
   int bm;                  // height of the small tiles
   int max_big, max_small;  // upper bounds on the number of tile records of each kind
   int64_t pitch;           // floats per K block in the re-laid-out token scales
-  size_t big_bytes, small_bytes, scale_bytes;
+  size_t big_bytes, scale_bytes;
 };
 
 GroupedPlan grouped_plan(int64_t E, int64_t total_m, int64_t K) {
@@ -125,9 +146,51 @@ GroupedPlan grouped_plan(int64_t E, int64_t total_m, int64_t K) {
   // align4(rows) past it: one more quad of slack keeps that inside the row (and inside the workspace for the last row)
   pl.pitch = ((total_m + 3) & ~3ll) + 4 * E + 4;
   pl.big_bytes = align256((size_t)(pl.max_big + 1) * sizeof(v4i));  // record 0 holds the count
-  pl.small_bytes = align256((size_t)(pl.max_small + 1) * sizeof(v4i));
   pl.scale_bytes = align256((size_t)pl.pitch * (size_t)((K + KSTEP - 1) / KSTEP) * 4u);
   return pl;
+}
+
+// What runs: with or without the 256-row tiles, and the shape of the small ones.
+struct GroupedRun {
+  bool use_big;
+  int bm, bn, max_big, max_small;
+  bool few;  // at most a workgroup per CU is expected
+};
+
+size_t grouped_small_bytes(const GroupedRun& r) { return align256((size_t)(r.max_small + 1) * sizeof(v4i)); }
+
+// Small tiles alone against 256-row tiles plus small ones, by the tile times of the dense GEMM for evenly spread rows; the second
+// launch costs about 4 us, also when no expert fills a 256-row tile.  Measured (whole
+// call, us, always with 256-row tiles / as chosen): 32 experts, 5392 rows, K = 896 -> N = 384 34.2 / 13.8;  8, 396, 1024 -> 1024
+// 17.0 / 12.3;  64, 7112, 1408 -> 1792 78.7 / 62.9;  8, 26, 6144 -> 384 29.7 / 21.5.
+GroupedRun grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, const GroupedPlan& pl) {
+  const TileTimes& t = SCALED_TIMES;
+  const int64_t active = std::min(E, total_m), rows = ceil_div(total_m, active), kb = ceil_div(K, KSTEP);
+  auto small_us = [&](int bm, int bn, int64_t tiles_m, int64_t* workgroups) {
+    int i = 0;
+    while (MID_TILES[i].bm != bm || MID_TILES[i].bn != bn) ++i;
+    const int64_t wg = tiles_m * ceil_div(N, bn);
+    const bool two = bm + bn == 192 && wg > NUM_CUS;
+    if (workgroups) *workgroups = wg;
+    return rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) { return t.tile[i] + (double)kb * t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill); });
+  };
+  // the weights of every active expert stream from memory once whatever the tiles
+  const double stream = (double)active * (double)N * (double)K * 1e-6 / 5.0;
+  const int64_t big = rows / BIG + (rows % BIG > 128), rest = rows % BIG > 128 ? 0 : rows % BIG;
+  double best = std::max(small_us(pl.bm, 256, active * ceil_div(rest, pl.bm), nullptr) + rounds_of(active * big * ceil_div(N, 256), NUM_CUS, [&](double fill) {
+                           return t.pp_tile + (double)kb * t.pp_block * (1.0 + t.pp_busy * fill);
+                         }), stream) + (pl.max_big > 0 ? 4.0 : 0.0);
+  GroupedRun r{pl.max_big > 0, pl.bm, 256, pl.max_big, pl.max_small, false};
+  for (int bm = 64; bm <= 128; bm += 64)
+    for (int bn = 256; bn >= 128; bn -= 128) {
+      int64_t wg = 0;
+      const double us = std::max(small_us(bm, bn, active * ceil_div(rows, bm), &wg), stream);
+      if (us < 0.95 * best) {
+        best = us;
+        r = GroupedRun{false, bm, bn, 0, (int)std::min<int64_t>(total_m, total_m / bm + E), wg <= NUM_CUS};
+      }
+    }
+  return r;
 }
 
 }  // namespace
@@ -139,7 +202,7 @@ extern "C" size_t mi355_fp8_blockwise_scaled_grouped_mm_workspace_bytes(int64_t 
                                                                         int64_t K) {
   if (num_experts <= 0 || total_m <= 0 || N <= 0 || K <= 0) return 0;
   const GroupedPlan pl = grouped_plan(num_experts, total_m, K);
-  return pl.big_bytes + pl.small_bytes + pl.scale_bytes;
+  return pl.big_bytes + grouped_small_bytes(grouped_run(num_experts, total_m, N, K, pl)) + pl.scale_bytes;
 }
 
 extern "C" int mi355_fp8_blockwise_scaled_grouped_mm_plan(int64_t num_experts, int64_t total_m, int64_t N, int64_t K, char* buf,
@@ -179,9 +242,11 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
                     total_m * lda < (1ll << 32) && N * ldb < (1ll << 32),
                 MI355_ERR_INVALID_ARGUMENT, "%s: dimensions out of range (row offsets must stay below 4 GiB)", what);
   const GroupedPlan pl = grouped_plan(num_experts, total_m, K);
-  MI355_REQUIRE(((int64_t)pl.max_big + pl.max_small) * ((N + 255) / 256) < (1ll << 31), MI355_ERR_INVALID_ARGUMENT,
+  const GroupedRun run = grouped_run(num_experts, total_m, N, K, pl);
+  const size_t small_bytes = grouped_small_bytes(run);
+  MI355_REQUIRE(((int64_t)run.max_big + run.max_small) * ((N + run.bn - 1) / run.bn) < (1ll << 31), MI355_ERR_INVALID_ARGUMENT,
                 "%s: too many tiles", what);
-  const size_t need = pl.big_bytes + pl.small_bytes + pl.scale_bytes;
+  const size_t need = pl.big_bytes + small_bytes + pl.scale_bytes;
   MI355_REQUIRE(workspace && workspace_bytes >= need, MI355_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", what,
                 need, workspace_bytes);
   MI355_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, MI355_ERR_INVALID_ARGUMENT,
@@ -191,15 +256,12 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
   uint8_t* wsp = static_cast<uint8_t*>(workspace);
   v4i* big_tiles = reinterpret_cast<v4i*>(wsp);
   v4i* small_tiles = reinterpret_cast<v4i*>(wsp + pl.big_bytes);
-  float* sa_mm = reinterpret_cast<float*>(wsp + pl.big_bytes + pl.small_bytes);
+  float* sa_mm = reinterpret_cast<float*>(wsp + pl.big_bytes + small_bytes);
   const int KB = (int)(K / KSTEP);
-  hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(256), 0, st, problem_sizes, expert_offsets, (int)num_experts, (int)total_m,
-                     pl.bm, big_tiles, pl.max_big, small_tiles, pl.max_small);
+  const GroupedTables tables{(int)num_experts, (int)total_m, run.bm, (int)run.use_big, run.max_big, run.max_small, big_tiles, small_tiles};
+  hipLaunchKernelGGL(grouped_prepare_kernel, dim3((unsigned)((total_m + CHUNK - 1) / CHUNK + 1), (unsigned)((KB + 31) / 32)), dim3(256), 0, st,
+                     problem_sizes, expert_offsets, tables, scales_a, sa_sm, sa_sk, sa_mm, pl.pitch, KB);
   int rc = check_launch(what);
-  if (rc != MI355_OK) return rc;
-  hipLaunchKernelGGL(grouped_relayout_scales_kernel, dim3((unsigned)(2 * pl.max_big + pl.max_small), (unsigned)((KB + 31) / 32)),
-                     dim3(256), 0, st, scales_a, sa_sm, sa_sk, sa_mm, pl.pitch, KB, pl.bm, big_tiles, pl.max_big, small_tiles);
-  rc = check_launch(what);
   if (rc != MI355_OK) return rc;
 
   GroupedParams gp{};
@@ -214,11 +276,11 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
   gp.b_expert_stride = b_expert_stride;
   gp.sb_expert_stride = sb_expert_stride;
   gp.out_elem = 2;
-  if (pl.max_big > 0) {
-    gp.tiles = big_tiles, gp.max_tiles_m = pl.max_big;
+  if (run.use_big) {
+    gp.tiles = big_tiles, gp.max_tiles_m = run.max_big;
     rc = launch_fp8_grouped_pp(gp, st, what);
     if (rc != MI355_OK) return rc;
   }
-  gp.tiles = small_tiles, gp.max_tiles_m = pl.max_small;
-  return launch_fp8_grouped_dma3(gp, pl.bm, st, what);
+  gp.tiles = small_tiles, gp.max_tiles_m = run.max_small;
+  return launch_fp8_grouped_dma3(gp, run.bm, run.bn, run.few, st, what);
 }

@@ -403,7 +403,7 @@ __global__ __launch_bounds__(G_THREADS) void fp8_gemm_pp_kernel(const GemmParams
 }
 
 // Grouped problems (see GroupedParams): the workgroup's token tile comes from the table the plan kernel wrote, the
-// operand bases move to that tile's expert.  Workgroup order as in fp8_grouped_dma3_kernel.
+// operand bases move to that tile's expert.  Workgroup order as in fp8_grouped_dma_kernel.
 __global__ __launch_bounds__(G_THREADS) void fp8_grouped_pp_kernel(const GroupedParams gp) {
   GemmParams p;
   int m0, tile_n;
