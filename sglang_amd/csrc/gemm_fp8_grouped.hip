@@ -185,7 +185,7 @@ GroupedRun grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, const G
     for (int bn = 256; bn >= 128; bn -= 128) {
       int64_t wg = 0;
       const double us = std::max(small_us(bm, bn, active * ceil_div(rows, bm), &wg), stream);
-      if (us < 0.95 * best) {
+      if (us < 0.95 * best || us + 3.0 < best) {  // (bound by the weights' stream either way: the launch alone decides)
         best = us;
         r = GroupedRun{false, bm, bn, 0, (int)std::min<int64_t>(total_m, total_m / bm + E), wg <= NUM_CUS};
       }
