@@ -15,15 +15,23 @@
 // computed at build time by gen_silu_table.cpp with one fixed sequence of individually rounded fp32 operations - the
 // definition the CPU oracle restates, so results are reproducible bit for bit (the reference uses its GPU's approximate
 // exp intrinsic and compares its kernels with a tolerance) - and are part of the code object: nothing is initialised at
-// run time.  Two forms, chosen by the number of groups (SQ_SMALL_GROUPS):
-//   * many: 256 workgroups of 1024 threads (one per CU), each with its table copied into LDS (128 of the CU's 160 KB);
-//   * few: the copy alone would take longer than the work: 256-thread workgroups that look up in the table where it lies.
+// run time.  Three forms, chosen by type and number of groups (SQ_NEAR_GROUPS):
+//   * ST_WHOLE: 256 workgroups of 1024 threads (one per CU), each with the table copied into LDS (128 of the CU's 160 KB);
+//   * ST_NEAR: the copy takes longer than the work where there is little of it, and sixteen waves a CU keep too few loads in
+//     flight.  256-thread workgroups with the entries of ordinary bfloat16 magnitudes only (12 KB); a lane with any other gate
+//     (zero, huge, infinite, NaN) looks its eight up in the table where it lies.  Costs two more operations a value, which is
+//     why the largest inputs take ST_WHOLE;
+//   * ST_IN_PLACE: float16 (the same magnitudes would be 76 KB), few groups: every value is looked up where the table lies.
 // A 16-lane row of a wave takes a group (8 values per lane: one 16-byte load of gate, one of up, eight lookups, one 8-byte
 // store), the loads of the next two groups are requested before the current one is processed.  4 B in and 1 B out per value.
 //
 // Rows in use are dealt out over the whole launch: every workgroup scans the experts' row counts (they are on the device) and
 // walks the list of used rows of all experts with the grid's stride.  With a fixed share of the workgroups per expert the
 // fullest expert set the time: 32 experts of 256 rows, half of them used on average, took 17.8 us, the fills 5.5 + 1.8 more.
+// The expert of a row is found by bisection of the prefix sums: stepping through them one by one, 256 experts of 16 rows took
+// 22.9 us (now 8.9), 256 of 64 rows 49.6 (26.4); 32 of 256 rows 16.0 (12.6 with the near gates in LDS).
+#include <algorithm>
+
 #include "common.h"
 
 namespace mi355 {
@@ -31,10 +39,16 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __attribute__((aligned(16))) const uint16_t g_silu_table[2][65536] = {
 #include "silu_table.inc"
 };
+
+enum SiluTable { ST_IN_PLACE, ST_NEAR, ST_WHOLE };
+// The entries of ST_NEAR: bfloat16 gates of 2^-16 <= |gate| < 2^8.  Both signs of a magnitude lie next to each other, so that entry
+// r - 2 NEAR_FIRST holds the gate whose bits rotated left by one are r, and one comparison tells whether it is there.
+constexpr int NEAR_FIRST = 0x3780, NEAR_COUNT = 24 * 128;
 
 // round a float to T and back
 template <int DT>
@@ -69,9 +83,13 @@ struct SiluQuantParams {
 };
 
 constexpr int SQ_MAX_EXPERTS = 1024;           // per launch: the scan of their row counts is one value per thread, at most four
-// Up to here the looked-up table stays where it lies.  Measured, us a call, in place / in LDS: 24000 groups 6.8 / 8.3, 65536
-// 13.3 / 11.0; masked with about half of the rows in use 32768 7.1 / 10.3, 65536 9.9 / 12.9, 131072 17.8 / 15.6, 262144 30.6 / 23.4.
-constexpr int64_t SQ_SMALL_GROUPS = 49152, SQ_SMALL_GROUPS_MASKED = 98304;
+// Which table, by the number of groups.  Measured, us a call (H = 2048, masked with about half of the rows in use), bfloat16,
+// near gates / whole table: 8192 groups 4.2 / 5.5, 32768 7.0 / 8.1, 48000 9.4 / 9.8, 65536 11.6 / 11.2, 524288 63.7 / 61.1;
+// masked 65536 8.2 / 11.0, 131072 12.6 / 14.9, 524288 44.0 / 45.9.  float16, in place / whole table: 11200 5.5 / 5.6,
+// 16384 6.4 / 5.9, 65536 18.9 / 11.2; masked 32768 8.1 / 9.4, 65536 13.2 / 11.0, 131072 20.3 / 15.1.
+constexpr int64_t SQ_NEAR_GROUPS = 49152, SQ_NEAR_GROUPS_MASKED = 524288;
+constexpr int64_t SQ_IN_PLACE_GROUPS = 12288, SQ_IN_PLACE_GROUPS_MASKED = 32768;
+constexpr int SQ_NEAR_WORKGROUPS = 6 * 256;  // six fit a CU by their registers
 
 // Row counts of the experts as prefix sums in LDS: pre[e] = used rows of experts < e, pre[E] = all of them.
 template <int THREADS>
@@ -109,10 +127,24 @@ struct GroupLoads {
   u32x4 gate, up;
 };
 
-// group c of the used rows; `e` walks forward with c
+// the first expert >= e whose end lies behind `at`; there is one
+template <class End>
+__device__ __forceinline__ int expert_of(int e, int E, int64_t at, End end) {
+  if (at < end(e)) return e;
+  int last = E - 1;
+  ++e;
+  while (e < last) {
+    const int mid = (e + last) >> 1;
+    if (at < end(mid)) last = mid;
+    else e = mid + 1;
+  }
+  return e;
+}
+
+// group c of the used rows; `e` moves forward with c
 __device__ __forceinline__ GroupAt locate(const SiluQuantParams& p, const int* pre, uint32_t c, int& e) {
   const int row = (int)fastdiv(c, p.div_gpr);
-  while (row >= pre[e + 1]) ++e;
+  e = expert_of(e, p.E, row, [&](int i) { return pre[i + 1]; });
   return GroupAt{e, row - pre[e], (int)(c - (uint32_t)row * p.gpr)};
 }
 // its gate and up (16 bytes each per lane)
@@ -123,19 +155,41 @@ __device__ __forceinline__ void fetch_group(const SiluQuantParams& p, const Grou
   l.up = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + p.H) + lane);
 }
 
-template <int DT>
+// T(silu(gate)) of a lane's eight gates
+template <int DT, SiluTable TABLE>
+__device__ __forceinline__ void look_up(const uint16_t* tbl, const uint32_t (&gate)[4], uint32_t (&silu)[8]) {
+  if constexpr (TABLE == ST_NEAR) {
+    u16x2 at[4], most = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u16x2 bits = __builtin_bit_cast(u16x2, gate[j]);
+      at[j] = ((bits << (uint16_t)1) | (bits >> (uint16_t)15)) - (uint16_t)(2 * NEAR_FIRST);
+      most = __builtin_elementwise_max(most, at[j]);
+    }
+    if (max((int)most.x, (int)most.y) < 2 * NEAR_COUNT) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) silu[j] = tbl[at[j >> 1][j & 1]];
+      return;
+    }
+    tbl = g_silu_table[DT == MI355_BF16 ? 0 : 1];
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) silu[j] = tbl[(j & 1) ? (gate[j >> 1] >> 16) : (gate[j >> 1] & 0xffffu)];
+}
+
+template <int DT, SiluTable TABLE>
 __device__ __forceinline__ void quant_group(const SiluQuantParams& p, const uint16_t* tbl, const GroupAt& g, const GroupLoads& cur) {
   const int lane = threadIdx.x & 15;
   const uint32_t wg[4] = {cur.gate.x, cur.gate.y, cur.gate.z, cur.gate.w};
   const uint32_t wu[4] = {cur.up.x, cur.up.y, cur.up.z, cur.up.w};
+  uint32_t silu[8];
+  look_up<DT, TABLE>(tbl, wg, silu);
   float v[8];
   float amax = 1e-10f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const uint32_t gb = (j & 1) ? (wg[j >> 1] >> 16) : (wg[j >> 1] & 0xffffu);
     const uint32_t ub = (j & 1) ? (wu[j >> 1] >> 16) : (wu[j >> 1] & 0xffffu);
-    const float sl = t_bits_to_f32<DT>(tbl[gb]);                    // T(silu(gate))
-    v[j] = round_to_t<DT>(mul_rn(sl, t_bits_to_f32<DT>(ub)));       // the product of two T values is exact in fp32
+    v[j] = round_to_t<DT>(mul_rn(t_bits_to_f32<DT>(silu[j]), t_bits_to_f32<DT>(ub)));  // the product of two T values is exact in fp32
     amax = fmaxf(amax, fabsf(v[j]));
   }
   amax = row16_max(amax);
@@ -159,17 +213,28 @@ __device__ __forceinline__ void quant_group(const SiluQuantParams& p, const uint
   }
 }
 
-template <int DT, bool LDS_TABLE>
-__global__ __launch_bounds__(LDS_TABLE ? 1024 : 256) void silu_mul_quant_kernel(const SiluQuantParams p) {
-  constexpr int THREADS = LDS_TABLE ? 1024 : 256;
-  __shared__ __attribute__((aligned(16))) uint16_t lds_table[LDS_TABLE ? 65536 : 1];
+template <int DT, SiluTable TABLE>
+__global__ __launch_bounds__(TABLE == ST_WHOLE ? 1024 : 256) void silu_mul_quant_kernel(const SiluQuantParams p) {
+  constexpr int THREADS = TABLE == ST_WHOLE ? 1024 : 256;
+  constexpr int ENTRIES = TABLE == ST_WHOLE ? 65536 : TABLE == ST_NEAR ? 2 * NEAR_COUNT : 8;
+  static_assert(TABLE != ST_NEAR || DT == MI355_BF16, "the near gates are bfloat16");
+  __shared__ __attribute__((aligned(16))) uint16_t lds_table[ENTRIES];
   __shared__ int pre[SQ_MAX_EXPERTS + 1];
   const uint16_t* tbl = g_silu_table[DT == MI355_BF16 ? 0 : 1];
-  constexpr int PIECES = 65536 * 2 / 16 / 1024;  // of the table, per thread: requested first, put into LDS last
-  u32x4 piece[LDS_TABLE ? PIECES : 1];
-  if constexpr (LDS_TABLE) {
+  const u32x4* entries = reinterpret_cast<const u32x4*>(tbl);
+  // of the table, per thread: requested first, put into LDS last
+  constexpr int NEAR_PIECES = NEAR_COUNT / 8, NEAR_EACH = (NEAR_PIECES + THREADS - 1) / THREADS;
+  constexpr int PIECES = TABLE == ST_WHOLE ? 65536 / 8 / THREADS : TABLE == ST_NEAR ? 2 * NEAR_EACH : 1;
+  u32x4 piece[PIECES];
+  if constexpr (TABLE == ST_WHOLE) {
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) piece[i] = reinterpret_cast<const u32x4*>(tbl)[i * THREADS + threadIdx.x];
+    for (int i = 0; i < PIECES; ++i) piece[i] = entries[i * THREADS + threadIdx.x];
+  } else if constexpr (TABLE == ST_NEAR) {
+#pragma unroll
+    for (int i = 0; i < NEAR_EACH; ++i) {
+      const int at = NEAR_FIRST / 8 + min(i * THREADS + (int)threadIdx.x, NEAR_PIECES - 1);
+      piece[2 * i] = entries[at], piece[2 * i + 1] = entries[0x8000 / 8 + at];
+    }
   }
   scan_rows<THREADS>(p, pre);
   const uint32_t groups = (uint32_t)pre[p.E] * p.gpr;
@@ -179,9 +244,19 @@ __global__ __launch_bounds__(LDS_TABLE ? 1024 : 256) void silu_mul_quant_kernel(
   GroupAt at{0, 0, 0}, at1{0, 0, 0}, at2{0, 0, 0};
   GroupLoads cur, nxt, nxt2;
   if (c < groups) at = locate(p, pre, c, e), fetch_group(p, at, cur);
-  if constexpr (LDS_TABLE) {
+  if constexpr (TABLE == ST_WHOLE) {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) reinterpret_cast<u32x4*>(lds_table)[i * THREADS + threadIdx.x] = piece[i];
+  } else if constexpr (TABLE == ST_NEAR) {
+#pragma unroll
+    for (int i = 0; i < NEAR_EACH; ++i) {
+      u32x4* to = reinterpret_cast<u32x4*>(lds_table) + 2 * min(i * THREADS + (int)threadIdx.x, NEAR_PIECES - 1);
+      const u32x4 pos = piece[2 * i], neg = piece[2 * i + 1];
+      const u32x4 even = (pos & 0xffffu) | (neg << 16), odd = (pos >> 16) | (neg & 0xffff0000u);
+      to[0] = u32x4{even.x, odd.x, even.y, odd.y}, to[1] = u32x4{even.z, odd.z, even.w, odd.w};
+    }
+  }
+  if constexpr (TABLE != ST_IN_PLACE) {
     __syncthreads();
     tbl = lds_table;
   }
@@ -189,7 +264,7 @@ __global__ __launch_bounds__(LDS_TABLE ? 1024 : 256) void silu_mul_quant_kernel(
   for (; c < groups; c += stride) {
     // two groups ahead: three 32-byte requests per lane in flight
     if (c + 2 * stride < groups) at2 = locate(p, pre, c + 2 * stride, e), fetch_group(p, at2, nxt2);
-    quant_group<DT>(p, tbl, at, cur);
+    quant_group<DT, TABLE>(p, tbl, at, cur);
     cur = nxt, nxt = nxt2;
     at = at1, at1 = at2;
   }
@@ -199,7 +274,7 @@ __global__ __launch_bounds__(LDS_TABLE ? 1024 : 256) void silu_mul_quant_kernel(
   const int64_t dead = (int64_t)p.E * p.T - pre[p.E];
   int ez = 0;
   for (int64_t d = (int64_t)blockIdx.x * (THREADS / 64) + (threadIdx.x >> 6); d < dead; d += (int64_t)gridDim.x * (THREADS / 64)) {
-    while (d >= (int64_t)(ez + 1) * p.T - pre[ez + 1]) ++ez;
+    ez = expert_of(ez, p.E, d, [&](int i) { return (int64_t)(i + 1) * p.T - pre[i + 1]; });
     const int64_t t = pre[ez + 1] - pre[ez] + (d - ((int64_t)ez * p.T - pre[ez]));
     uint8_t* row = p.q + ((int64_t)ez * p.T + t) * p.H;
     for (int64_t i = lane * 8; i < p.H; i += 64 * 8) __builtin_nontemporal_store(u32x2{0u, 0u}, reinterpret_cast<u32x2*>(row + i));
@@ -233,13 +308,16 @@ int silu_mul_group_quant(const char* what, const void* x, int x_dtype, void* q, 
     p.zero_rest = zero_rest;
     const int64_t groups = p.E * T * gpr;
     MI355_REQUIRE(groups < (1ll << 30), MI355_ERR_INVALID_ARGUMENT, "%s: too many groups", what);
-    if (groups <= (masked_m ? SQ_SMALL_GROUPS_MASKED : SQ_SMALL_GROUPS)) {
-      const dim3 grid((unsigned)((groups + 15) / 16));
-      if (x_dtype == MI355_BF16) hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_BF16, false>), grid, dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_F16, false>), grid, dim3(256), 0, st, p);
+    const bool bf16 = x_dtype == MI355_BF16;
+    if (bf16 && groups <= (masked_m ? SQ_NEAR_GROUPS_MASKED : SQ_NEAR_GROUPS)) {
+      const dim3 grid((unsigned)std::min<int64_t>((groups + 15) / 16, SQ_NEAR_WORKGROUPS));
+      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_BF16, ST_NEAR>), grid, dim3(256), 0, st, p);
+    } else if (bf16) {
+      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_BF16, ST_WHOLE>), dim3(256), dim3(1024), 0, st, p);
+    } else if (groups <= (masked_m ? SQ_IN_PLACE_GROUPS_MASKED : SQ_IN_PLACE_GROUPS)) {
+      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_F16, ST_IN_PLACE>), dim3((unsigned)((groups + 15) / 16)), dim3(256), 0, st, p);
     } else {
-      if (x_dtype == MI355_BF16) hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_BF16, true>), dim3(256), dim3(1024), 0, st, p);
-      else hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_F16, true>), dim3(256), dim3(1024), 0, st, p);
+      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_F16, ST_WHOLE>), dim3(256), dim3(1024), 0, st, p);
     }
     const int rc = check_launch(what);
     if (rc != MI355_OK) return rc;
