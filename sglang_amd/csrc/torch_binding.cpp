@@ -10,13 +10,16 @@
 //   * the operators: argument checks with the conditions and wording of the reference's host functions (cited at each),
 //     allocation, one C-ABI call.  They throw; the GIL is not held while they run.
 //   * the linear methods' fast paths (try_*): whole forward passes of fp8_utils / w8a8_int8 for the operands those meet in
-//     use.  They return None for anything else and the Python function goes its long way, which raises the errors.
+//     use.  They return None for anything else, and where a mode, a tracer or a functional transform listens at the dispatcher;
+//     the Python function then goes its long way, which calls the operators and raises the errors.
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/Allocator.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/Dtype.h>
@@ -897,8 +900,27 @@ bool is_pair_of_128(PyObject* o) {
   return true;
 }
 
-// The fast path FN, tried only for plain tensors (a subclass may mean something else by an operation) and, where BLOCK is an
-// argument's index, for 128 x 128 blocks; that argument is not handed on.
+// Whether an operator called on `t` here and now would end in the CUDA kernel itself.  A fast path launches kernels without
+// the dispatcher, so whoever listens there would see its allocations and not what fills them: modes, tracers and functional
+// wrappers (vmap, grad) announce themselves in the thread's or the tensor's key set, function modes in a state of their own.
+// Autograd and autocast keys may be set: the operators have no formula for either, and the calls record nothing with them.
+bool plain_dispatch(const Tensor& t) {
+  using c10::DispatchKey;
+  constexpr c10::DispatchKeySet direct({DispatchKey::Dense, DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView,
+                                        DispatchKey::AutogradFunctionality, DispatchKey::AutocastCUDA, DispatchKey::AutocastCPU});
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  const c10::DispatchKeySet keys = ((t.key_set() | tls.included_) - tls.excluded_) - direct;
+  return (keys.raw_repr() & ~c10::full_backend_mask) == 0 && !at::impl::torch_function_mode_enabled();
+}
+
+PyObject* plain_dispatch_py(PyObject*, PyObject* t) {
+  HANDLE_TH_ERRORS
+  return PyBool_FromLong(plain_dispatch(as_tensor(t)));
+  END_HANDLE_TH_ERRORS
+}
+
+// The fast path FN, tried only for plain tensors (a subclass may mean something else by an operation), only where nobody looks
+// on (plain_dispatch) and, where BLOCK is an argument's index, for 128 x 128 blocks; that argument is not handed on.
 template <auto FN, int BLOCK> struct Try;
 template <class R, class... A, R (*FN)(A...), int BLOCK> struct Try<FN, BLOCK> {
   static constexpr Py_ssize_t COUNT = (Py_ssize_t)sizeof...(A) + (BLOCK >= 0 ? 1 : 0);
@@ -912,7 +934,7 @@ template <class R, class... A, R (*FN)(A...), int BLOCK> struct Try<FN, BLOCK> {
         if (!is_pair_of_128(args[i])) Py_RETURN_NONE;
         continue;
       }
-      if (THPVariable_Check(args[i]) && !THPVariable_CheckExact(args[i])) Py_RETURN_NONE;
+      if (THPVariable_Check(args[i]) && !(THPVariable_CheckExact(args[i]) && plain_dispatch(THPVariable_Unpack(args[i])))) Py_RETURN_NONE;
       rest[at++] = args[i];
     }
     return Call<FN>::py(self, rest, (Py_ssize_t)sizeof...(A));
@@ -964,6 +986,7 @@ PyMethodDef METHODS[] = {
     TRY("try_token_linear", try_token_linear, -1),
     TRY("try_group_quant", try_group_quant, -1),
     TRY("try_silu_quant", try_silu_quant, -1),
+    {"plain_dispatch", &plain_dispatch_py, METH_O, nullptr},
     {"env_flag", &env_flag, METH_O, nullptr},
     {"set_error_class", &set_error_class, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},

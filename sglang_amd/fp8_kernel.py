@@ -10,9 +10,10 @@ from __future__ import annotations
 from typing import List, Optional, Tuple
 
 import torch
+from torch.compiler import is_compiling
 
 from . import _lib, _native, ops
-from .sgl_kernel import sgl_per_token_group_quant_8bit
+from .sgl_kernel import _v2_by_environment, sgl_per_token_group_quant_8bit
 
 fp8_dtype = torch.float8_e4m3fn
 fp8_max = torch.finfo(fp8_dtype).max
@@ -74,10 +75,11 @@ def _per_token_group_quant_8bit_raw(
     ``s`` up to a power of two and repacks the fp32 scales with DeepGEMM's
     ``transform_sf_into_required_layout``; here the kernel writes that packed int32 layout
     directly (four exponent bytes per word, words column-major and padded to 4 rows)."""
-    out = _native.try_group_quant(x, group_size, eps, dtype, column_major_scales, scale_tma_aligned or scale_ue8m0, scale_ue8m0,
-                                  True, False)
-    if out is not None:
-        return out
+    if not is_compiling():
+        out = _native.try_group_quant(x, group_size, eps, dtype, column_major_scales, scale_tma_aligned or scale_ue8m0, scale_ue8m0,
+                                      True, False)
+        if out is not None:
+            return out
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
 
@@ -146,7 +148,7 @@ def _per_token_group_quant_8bit_fuse_silu_and_mul(
     assert scale_tma_aligned
     assert scale_ue8m0
     assert group_size == 128
-    if dst_dtype == fp8_dtype:
+    if dst_dtype == fp8_dtype and not is_compiling():
         out = _native.try_silu_quant(x, masked_m)
         if out is not None:
             return out
@@ -207,8 +209,10 @@ def sglang_per_token_group_quant_fp8(
 ):
     """fp8_kernel.py:477-527: allocate outputs, then ``sgl_per_token_group_quant_8bit``."""
     if enable_v2 is None:
-        enable_v2 = _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
-    if fuse_silu_and_mul:
+        enable_v2 = _v2_by_environment()
+    if is_compiling():
+        pass
+    elif fuse_silu_and_mul:
         if (enable_v2 and group_size == 128 and abs(1e-10 - eps) < 1e-13 and column_major_scales and scale_tma_aligned and scale_ue8m0):
             out = _native.try_silu_quant(x, masked_m)
             if out is not None:

@@ -13,7 +13,9 @@ The two block-FP8 wrappers are different computations and are kept different her
 both add the bias to the rounded 16-bit output (a second rounding), as the reference does.
 The linear methods first offer their operands to a native fast path (`_native.try_*`: the whole forward pass in one call for
 plain contiguous 16-bit activations and the weight layouts of a loaded checkpoint, about 4 us of host time); it declines
-anything else, and the Python below computes it, or raises.
+anything else, among it every call that somebody looks at through PyTorch's dispatcher (dispatch and function modes, tracing,
+vmap), and the Python below computes it, or raises.  Under `torch.compile` and export it is not asked: its tracer cannot
+follow a C function.
 `fused_w8a8_block_fp8_linear` is this library's own one-call variant (`mi355_fp8_block_linear`: codes and scales live
 only in the call's workspace, bias added in fp32 before the single rounding); it is an opt-in, not what the reference's
 names resolve to, because its outputs may differ from theirs in the last bit when a bias is present.
@@ -24,6 +26,7 @@ import functools
 from typing import Callable, List, Optional
 
 import torch
+from torch.compiler import is_compiling
 
 from . import _lib, _native, ops
 from .fp8_kernel import (
@@ -76,9 +79,10 @@ def triton_w8a8_block_fp8_linear(
 ) -> torch.Tensor:
     """fp8_utils.py:281-301: row-major-scale quantizer (`x * (1 / s)`), the ragged-shape matmul, bias on the rounded output."""
     assert input_scale is None
-    output = _native.try_block_linear(input, weight, block_size, weight_scale, bias, True)
-    if output is not None:
-        return output
+    if not is_compiling():
+        output = _native.try_block_linear(input, weight, block_size, weight_scale, bias, True)
+        if output is not None:
+            return output
     input_2d = input.view(-1, input.shape[-1])
     output_shape = [*input.shape[:-1], weight.shape[0]]
 
@@ -102,9 +106,10 @@ def cutlass_w8a8_block_fp8_linear_with_fallback(
     """fp8_utils.py:184-214: M-major-scale quantizer (`x / s`), `fp8_blockwise_scaled_mm` on the transposed views, bias on
     the rounded output; shapes with N or K not a multiple of 128 go to the Triton wrapper."""
     assert input_scale is None
-    output = _native.try_block_linear(input, weight, block_size, weight_scale, bias, False)
-    if output is not None:
-        return output
+    if not is_compiling():
+        output = _native.try_block_linear(input, weight, block_size, weight_scale, bias, False)
+        if output is not None:
+            return output
 
     shape_supported = weight.shape[0] % 128 == 0 and weight.shape[1] % 128 == 0
     if not shape_supported:
@@ -175,9 +180,10 @@ def deepgemm_w8a8_block_fp8_linear_with_fallback(
     assert input_scale is None
     if weight_scale.dtype != torch.int32 or input.dtype != torch.bfloat16 or weight.shape[1] % 128 != 0:
         return triton_w8a8_block_fp8_linear(input, weight, block_size, weight_scale, input_scale, bias)
-    out = _native.try_block_linear_ue8m0(input, weight, block_size, weight_scale, bias)
-    if out is not None:
-        return out
+    if not is_compiling():
+        out = _native.try_block_linear_ue8m0(input, weight, block_size, weight_scale, bias)
+        if out is not None:
+            return out
     from .fp8_kernel import sglang_per_token_group_quant_fp8
 
     K = input.shape[-1]
@@ -217,7 +223,7 @@ def apply_fp8_linear(
     default; a static per-tensor `input_scale` is repeated per token (:748-753); with `compressed_tensor_quant` the
     quantizer is `scaled_fp8_quant` (:598-603), whose per-tensor scale is repeated likewise for the GEMM.
     `input_scale_ub` is accepted and unused, as in the reference (:570 is its only mention there)."""
-    if not compressed_tensor_quant:
+    if not compressed_tensor_quant and not is_compiling():
         out = _native.try_token_linear(input, weight, weight_scale, input_scale, bias)
         if out is not None:
             return out

@@ -3,13 +3,22 @@
 ``torch.ops.sgl_kernel.<op>.default`` exactly like the reference's wrappers do."""
 from __future__ import annotations
 
+import os
 from typing import Optional
 
 import torch
+from torch.compiler import is_compiling
 
 from . import _native, ops
 
 ops.register()
+
+
+def _v2_by_environment() -> bool:
+    """SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2 with the truth values of sglang.srt.utils.get_bool_env_var."""
+    if is_compiling():  # (the tracer can follow this, and not a C function)
+        return os.getenv("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2", "false").lower() in ("true", "1")
+    return _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
 
 
 def int8_scaled_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
@@ -63,7 +72,7 @@ def sgl_per_token_group_quant_8bit(
     enable_v2: Optional[bool] = None,
 ) -> None:
     if enable_v2 is None:
-        enable_v2 = _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
+        enable_v2 = _v2_by_environment()
 
     if enable_v2:
         return torch.ops.sgl_kernel.sgl_per_token_group_quant_8bit_v2.default(
