@@ -211,9 +211,11 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm_plan(int64_t num_experts, i
   clear_error();
   MI355_REQUIRE(buf && buf_len > 0, MI355_ERR_INVALID_ARGUMENT, "%s: no buffer", what);
   MI355_REQUIRE(num_experts > 0 && total_m > 0 && N > 0 && K > 0, MI355_ERR_INVALID_ARGUMENT, "%s: empty problem", what);
-  const GroupedPlan pl = grouped_plan(num_experts, total_m, K);
-  snprintf(buf, buf_len, "kernel=grouped_pingpong+grouped_dma3 small_tile=%dx256 max_big_tiles=%d max_small_tiles=%d tiles_n=%lld",
-           pl.bm, pl.max_big, pl.max_small, (long long)((N + 255) / 256));
+  const GroupedRun run = grouped_run(num_experts, total_m, N, K, grouped_plan(num_experts, total_m, K));
+  const int n = snprintf(buf, buf_len, "kernel=%s small_tile=%dx%d max_big_tiles=%d max_small_tiles=%d tiles_n=%lld",
+                         run.use_big ? "grouped_pingpong+grouped_dma3" : "grouped_dma3", run.bm, run.bn, run.max_big, run.max_small,
+                         (long long)ceil_div(N, run.bn));
+  MI355_REQUIRE(n > 0 && (size_t)n < buf_len, MI355_ERR_INVALID_ARGUMENT, "%s: buffer of %zu bytes is too small", what, buf_len);
   return MI355_OK;
 }
 

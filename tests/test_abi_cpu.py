@@ -130,10 +130,10 @@ def test_newer_entry_points_validate_before_any_device_work():
     assert G(None, None, None, None, None, _lib.BF16, None, None, 0, 0, 128, 128, *tail, None, 0, None) == 0
     W = L.mi355_fp8_blockwise_scaled_grouped_mm_workspace_bytes
     assert W(0, 8, 128, 128) == 0 and W(2, 8, 128, 128) % 256 == 0 and W(256, 32768, 512, 7168) > W(256, 256, 512, 7168) > 0
-    plan = _lib.grouped_gemm_plan(256, 32768, 512, 7168)
-    assert plan["small_tile"] == "128x256" and plan["max_big_tiles"] == 32768 // 129 and plan["max_small_tiles"] == 256
-    assert _lib.grouped_gemm_plan(256, 256, 512, 7168) == {
-        "kernel": "grouped_pingpong+grouped_dma3", "small_tile": "64x256", "max_big_tiles": 1, "max_small_tiles": 256, "tiles_n": 2}
+    assert _lib.grouped_gemm_plan(16, 8192, 4096, 7168) == {
+        "kernel": "grouped_pingpong+grouped_dma3", "small_tile": "128x256", "max_big_tiles": 8192 // 129, "max_small_tiles": 16, "tiles_n": 16}
+    assert _lib.grouped_gemm_plan(256, 256, 512, 7168) == {  # one row per expert: small tiles alone
+        "kernel": "grouped_dma3", "small_tile": "64x256", "max_big_tiles": 0, "max_small_tiles": 256, "tiles_n": 2}
 
 
 def test_operator_schemas_are_the_reference_ones():

@@ -166,8 +166,8 @@ def test_workspace_covers_the_plan(kind, M, N, K):
 def test_grouped_plan_bounds_hold_for_any_routing():
     """The grouped GEMM sizes its tile tables and grids on the host from (experts, stacked rows) alone, while the real
     tile counts come from row counts that only exist on the device.  Replay the device rule here (256-row tiles; a rest of
-    129..255 rows is one more; a rest of 1..128 rows becomes small tiles of the height the plan names) for random and
-    adversarial routings: the host bounds must never be exceeded."""
+    129..255 rows is one more; a rest of 1..128 rows becomes small tiles of the height the plan names; small tiles for every row
+    where the plan has no 256-row launch) for random and adversarial routings: the host bounds must never be exceeded."""
     import random
 
     from sglang_amd import _lib
@@ -187,22 +187,26 @@ def test_grouped_plan_bounds_hold_for_any_routing():
             sizes = [rnd.choice([1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 384, 385]) for _ in range(E)]
         cases.append(sizes)
     cases += [[128] * 256, [129] * 256, [1] * 256, [64] * 300, [65] * 300, [385] * 16, [0] * 8 + [1]]
+    kernels = set()
     for sizes in cases:
         E, total = len(sizes), sum(sizes)
         if total == 0:
             continue
-        plan = _lib.grouped_gemm_plan(E, total, 512, 1024)
-        bm = int(plan["small_tile"].split("x")[0])
-        big = small = 0
-        for rows in sizes:
-            b, rest = divmod(rows, 256)
-            if rest > 128:
-                b += 1
-            else:
-                small += -(-rest // bm)
-            big += b
-        assert big <= plan["max_big_tiles"], (sizes[:8], big, plan)
-        assert small <= plan["max_small_tiles"], (sizes[:8], small, plan)
+        for N, K in ((512, 1024), (4096, 7168)):
+            plan = _lib.grouped_gemm_plan(E, total, N, K)
+            bm = int(plan["small_tile"].split("x")[0])
+            two_kinds = "pingpong" in plan["kernel"]
+            kernels.add(plan["kernel"])
+            big = small = 0
+            for rows in sizes:
+                b, rest = divmod(rows, 256) if two_kinds else (0, rows)
+                if two_kinds and rest > 128:
+                    b += 1
+                else:
+                    small += -(-rest // bm)
+                big += b
+            assert big <= plan["max_big_tiles"], (sizes[:8], big, plan)
+            assert small <= plan["max_small_tiles"], (sizes[:8], small, plan)
         # the re-laid-out scale columns: expert e starts at align4(row0) + 4 e and is read in whole quads
         pitch = (total + 3) // 4 * 4 + 4 * E + 4
         row0 = 0
@@ -210,6 +214,7 @@ def test_grouped_plan_bounds_hold_for_any_routing():
             if rows:
                 assert (row0 + 3) // 4 * 4 + 4 * e + (rows + 3) // 4 * 4 <= pitch
             row0 += rows
+    assert len(kernels) == 2
 
 
 def test_mid_m_plans_are_consistent():
