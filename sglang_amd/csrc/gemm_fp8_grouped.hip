@@ -26,9 +26,10 @@ namespace {
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Tile heights.  An expert's rows are cut into 256-row tiles for the two-phase kernel; what is left (fewer than 256 rows)
-// becomes one more 256-row tile when it is more than 128 rows, otherwise 64- or 128-row tiles for the three-stage kernel
-// (one height per call, chosen on the host from the average rows per expert).  Measured on the dense kernels: per output
-// element a 128-row tile costs 1.5x and a 64-row tile 2.3x of a 256-row tile when both are bound by the matrix pipe.
+// becomes one more 256-row tile when it is more than 128 rows, otherwise a 128-row tile for the mid-M kernel; where small
+// tiles run alone, all rows are cut into tiles of one height, 64 or 128 (chosen on the host from the average rows per
+// expert).  Measured on the dense kernels: per output element a 128-row tile costs 1.5x and a 64-row tile 2.3x of a
+// 256-row tile when both are bound by the matrix pipe.
 constexpr int BIG = 256;
 
 struct ExpertTiles {
@@ -130,18 +131,14 @@ __global__ __launch_bounds__(256) void grouped_prepare_kernel(const int32_t* pro
 }
 
 struct GroupedPlan {
-  int bm;                  // height of the small tiles
-  int max_big, max_small;  // upper bounds on the number of tile records of each kind
+  int max_big;             // upper bound on the number of 256-row tiles
   int64_t pitch;           // floats per K block in the re-laid-out token scales
   size_t big_bytes, scale_bytes;
 };
 
 GroupedPlan grouped_plan(int64_t E, int64_t total_m, int64_t K) {
   GroupedPlan pl;
-  pl.bm = total_m > 64 * E ? 128 : 64;  // by the average rows per expert; the sizes themselves are on the device
-  pl.max_big = (int)(total_m / 129);    // every 256-row tile covers more than 128 rows
-  // an expert leaves at most 128 rows to small tiles, and every small tile covers at least one row
-  pl.max_small = (int)std::min<int64_t>(total_m, E * (128 / pl.bm));
+  pl.max_big = (int)(total_m / 129);  // every 256-row tile covers more than 128 rows
   // the last expert's column is at most align4(total_m) - rows + 4 (E - 1) + 3, and the GEMM reads whole quads up to
   // align4(rows) past it: one more quad of slack keeps that inside the row (and inside the workspace for the last row)
   pl.pitch = ((total_m + 3) & ~3ll) + 4 * E + 4;
@@ -159,38 +156,107 @@ struct GroupedRun {
 
 size_t grouped_small_bytes(const GroupedRun& r) { return align256((size_t)(r.max_small + 1) * sizeof(v4i)); }
 
-// Small tiles alone against 256-row tiles plus small ones, by the tile times of the dense GEMM for evenly spread rows; the second
-// launch costs about 4 us, also when no expert fills a 256-row tile.  Measured (whole
-// call, us, always with 256-row tiles / as chosen): 32 experts, 5392 rows, K = 896 -> N = 384 34.2 / 13.8;  8, 396, 1024 -> 1024
-// 17.0 / 12.3;  64, 7112, 1408 -> 1792 78.7 / 62.9;  8, 26, 6144 -> 384 29.7 / 21.5.
-GroupedRun grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, const GroupedPlan& pl) {
-  const TileTimes& t = SCALED_TIMES;
-  const int64_t active = std::min(E, total_m), rows = ceil_div(total_m, active), kb = ceil_div(K, KSTEP);
-  auto small_us = [&](int bm, int bn, int64_t tiles_m, int64_t* workgroups) {
-    int i = 0;
-    while (MID_TILES[i].bm != bm || MID_TILES[i].bn != bn) ++i;
-    const int64_t wg = tiles_m * ceil_div(N, bn);
-    const bool two = bm + bn == 192 && wg > NUM_CUS;
-    if (workgroups) *workgroups = wg;
-    return rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) { return t.tile[i] + (double)kb * t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill); });
-  };
-  // the weights of every active expert stream from memory once whatever the tiles
-  const double stream = (double)active * (double)N * (double)K * 1e-6 / 5.0;
-  const int64_t big = rows / BIG + (rows % BIG > 128), rest = rows % BIG > 128 ? 0 : rows % BIG;
-  double best = std::max(small_us(pl.bm, 256, active * ceil_div(rest, pl.bm), nullptr) + rounds_of(active * big * ceil_div(N, 256), NUM_CUS, [&](double fill) {
-                           return t.pp_tile + (double)kb * t.pp_block * (1.0 + t.pp_busy * fill);
-                         }), stream) + (pl.max_big > 0 ? 4.0 : 0.0);
-  GroupedRun r{pl.max_big > 0, pl.bm, 256, pl.max_big, pl.max_small, false};
-  for (int bm = 64; bm <= 128; bm += 64)
-    for (int bn = 256; bn >= 128; bn -= 128) {
-      int64_t wg = 0;
-      const double us = std::max(small_us(bm, bn, active * ceil_div(rows, bm), &wg), stream);
-      if (us < 0.95 * best || us + 3.0 < best) {  // (bound by the weights' stream either way: the launch alone decides)
-        best = us;
-        r = GroupedRun{false, bm, bn, 0, (int)std::min<int64_t>(total_m, total_m / bm + E), wg <= NUM_CUS};
-      }
+// Which tiles a call runs: 256-row tiles with small ones for the rests, or small tiles of one of four shapes alone, by modelled time.
+// What separates them is how often an expert's weight is fetched, once per token tile, against the rows that tiles pad; the
+// routing itself is on the device, so the rows of the experts are taken to spread evenly over 0.25 .. 1.75 of their average.
+//
+// Per tiling, us: rounds of one workgroup per CU (64 x 128: two), each tile + K blocks * block * (1 + BUSY * fill); the stream, the
+// weights of the experts that have rows at `stream` TB/s, REFETCH more for every further tile of an expert, and the tokens and the
+// result; both joined by the 3/2 norm, plus CALL for the preparation and the ends, and BIG_LAUNCH where there are two GEMM launches.
+// Fitted to the five tilings of 240 problems (8 .. 256 experts, 8 .. 40000 rows, K = 512 .. 7168, N = 256 .. 7168; all experts equal,
+// and popularities of 0.25 .. 1.25): 4.4 % root mean square.  What it chooses takes 1.023 of the best tiling's time (geometric mean),
+// at most 1.04 of what the maximum of tile time and stream chose, which took 1.057: bound by the stream all tilings looked equal to
+// that one, and it fetched the weights of 65 .. 128 rows twice.  Whole call, us, that rule / this one: 256 experts of 128 rows,
+// K = 7168 -> N = 512 278 / 242;  32 of 128, 7168 -> 4096 254 / 208;  64 of 96, 7168 -> 2048 247 / 200;  32 of 160, 2048 -> 7168
+// 194 / 153;  256 of 4, 7168 -> 512 172 / 172;  half of all rows on one expert, 64 of 128, 7168 -> 2048 259 / 265.  Few experts with
+// exactly equal rows lose by the assumed spread what uneven ones gain: 8 of 256, 4096 -> 3584 50 / 65 if equal, 76 / 69 if not;
+// 16 of 160, 7168 -> 4096 128 / 149 and 167 / 151.
+struct GroupedTile {
+  int bm, bn;
+  double tile, block, stream;
+};
+constexpr GroupedTile BIG_TILE = {256, 256, 4.70, 0.929, 7.02};
+constexpr GroupedTile SMALL_TILES[] = {{64, 256, 1.32, 0.447, 7.01}, {128, 256, 2.96, 0.626, 7.99}, {128, 128, 2.34, 0.392, 8.34}, {64, 128, 1.12, 0.306, 7.53}};
+
+struct GroupedTimes {
+  static constexpr double BUSY = 0.19, SHARED = 1.64, REFETCH = 0.185, CALL = 7.5, BIG_LAUNCH = 1.8, TOKENS = 3.0;
+  static constexpr int SPREAD = 8;
+  int64_t active, total_m, N, K, kb;
+  int64_t rows_of[SPREAD];  // of an expert in each eighth of the active ones
+
+  GroupedTimes(int64_t E, int64_t total_m_, int64_t N_, int64_t K_) : active(std::min(E, total_m_)), total_m(total_m_), N(N_), K(K_), kb(ceil_div(K_, KSTEP)) {
+    for (int j = 0; j < SPREAD; ++j) {
+      const double share = active == 1 ? 1.0 : 0.25 + (j + 0.5) * 1.5 / SPREAD;
+      rows_of[j] = std::max<int64_t>(1, (int64_t)std::ceil((double)total_m / (double)active * share - 1e-9));
     }
+  }
+  template <class Tiles>
+  double tiles(Tiles of) const {
+    int64_t n = 0;
+    for (int64_t rows : rows_of) n += of(rows);
+    return (double)n * (double)active / SPREAD;
+  }
+  // where experts take more than one tile the number of workgroups is only about right, and the last round with it
+  double rounds(const GroupedTile& t, double token_tiles, bool about) const {
+    const double workgroups = token_tiles * (double)ceil_div(N, t.bn);
+    const bool two = t.bm + t.bn == 192 && workgroups > NUM_CUS;
+    const double slots = two ? 2.0 * NUM_CUS : NUM_CUS;
+    const auto exact = [&](double wg) {
+      const auto round = [&](double fill) { return t.tile + (double)kb * t.block * (two ? SHARED : 1.0) * (1.0 + BUSY * fill); };
+      const double full = std::floor(wg / slots), rest = wg / slots - full;
+      return full * round(1.0) + (rest > 1e-9 ? round(rest) : 0.0);
+    };
+    return about ? (exact(0.94 * workgroups) + exact(workgroups) + exact(1.06 * workgroups)) / 3.0 : exact(workgroups);
+  }
+  double us(double tile_us, double token_tiles, double rate) const {
+    const double stream = (double)active * (double)N * (double)K * 1e-6 / rate * (1.0 + REFETCH * (token_tiles / (double)active - 1.0)) +
+                          (double)total_m * (double)(K + 2 * N) * 1e-6 / TOKENS;
+    const double norm = std::cbrt(tile_us * std::sqrt(tile_us) + stream * std::sqrt(stream));
+    return CALL + norm * norm;
+  }
+  double small(const GroupedTile& t) const {
+    const double n = tiles([&](int64_t rows) { return ceil_div(rows, t.bm); });
+    return us(rounds(t, n, n > (double)active), n, t.stream);
+  }
+  double big() const {
+    const GroupedTile& rest_tile = SMALL_TILES[1];
+    const double nb = tiles([&](int64_t rows) { return rows / BIG + (rows % BIG > 128); });
+    const double ns = tiles([&](int64_t rows) { return rows % BIG > 128 ? 0 : ceil_div(rows % BIG, rest_tile.bm); });
+    const bool about = nb + ns > (double)active;
+    return us(rounds(BIG_TILE, nb, about) + rounds(rest_tile, ns, about), nb + ns, BIG_TILE.stream) + BIG_LAUNCH;
+  }
+};
+
+GroupedRun choose_grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, const GroupedPlan& pl) {
+  const GroupedTimes times(E, total_m, N, K);
+  const auto alone = [&](const GroupedTile& t) {
+    const int64_t workgroups = times.active * ceil_div(ceil_div(total_m, times.active), t.bm) * ceil_div(N, t.bn);
+    return GroupedRun{false, t.bm, t.bn, 0, (int)std::min<int64_t>(total_m, total_m / t.bm + E), workgroups <= NUM_CUS};
+  };
+  GroupedRun r = alone(SMALL_TILES[0]);
+  double best = times.small(SMALL_TILES[0]);
+  // (another tiling only for 5 %: below that the model does not order two)
+  if (pl.max_big > 0 && total_m > 64 * E) {
+    const double us = times.big();
+    // (an expert leaves at most 128 rows to the small tiles, one tile, and a tile covers at least one row)
+    if (us < 0.95 * best) best = us, r = GroupedRun{true, 128, 256, pl.max_big, (int)std::min(total_m, E), false};
+  }
+  for (int i = 1; i < 4; ++i) {
+    const double us = times.small(SMALL_TILES[i]);
+    if (us < 0.95 * best) best = us, r = alone(SMALL_TILES[i]);
+  }
   return r;
+}
+// The choice takes 1.3 us; a call asks twice, for its workspace and for its launches, so a thread keeps the last one.
+GroupedRun grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, const GroupedPlan& pl) {
+  struct Last {
+    int64_t E, total_m, N, K;
+    GroupedRun run;
+  };
+  static thread_local Last last{};  // (no call has zero experts)
+  if (last.E != E || last.total_m != total_m || last.N != N || last.K != K)
+    last = Last{E, total_m, N, K, choose_grouped_run(E, total_m, N, K, pl)};
+  return last.run;
 }
 
 }  // namespace

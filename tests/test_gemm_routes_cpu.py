@@ -217,6 +217,21 @@ def test_grouped_plan_bounds_hold_for_any_routing():
     assert len(kernels) == 2
 
 
+@pytest.mark.parametrize("E,N,K", [(256, 512, 7168), (32, 4096, 7168), (64, 2048, 7168), (128, 1536, 2048)])
+def test_grouped_plan_fetches_each_weight_once(E, N, K):
+    """Calls bound by the stream of the experts' weights: experts of up to 128 rows get one token tile each (two of 64 rows
+    fetch the weight twice: 32 experts of 128 rows, 7168 -> 4096, 254 against 208 us), and no 256-row launch stands in front where
+    an expert has a few rows (256 of 4 rows: 174 against 172 us)."""
+    from sglang_amd import _lib
+
+    for rows in (1, 4, 16, 32):
+        p = _lib.grouped_gemm_plan(E, E * rows, N, K)
+        assert p["kernel"] == "grouped_dma3", (rows, p)
+    for rows in (72, 96, 112, 128):
+        p = _lib.grouped_gemm_plan(E, E * rows, N, K)
+        assert p["small_tile"] == "128x256", (rows, p)
+
+
 def test_mid_m_plans_are_consistent():
     """Whatever the time model picks, a split must give every K range some work and the ranges must cover K."""
     from sglang_amd import _lib

@@ -27,6 +27,32 @@ def test_grouped(gpu, oracle, name, sizes, N, K, m_major):
     _verify(oracle, out, a, w, sa, sw, sizes, offsets, name)
 
 
+# experts (uneven: some without a row, one with many), stacked rows, N, K -> what has to run
+FORMS = [(40, 1240, 2056, 128, "grouped_dma3", "64x256"), (16, 16, 64, 384, "grouped_dma3", "64x128"),
+         (40, 29, 2056, 128, "grouped_dma3", "64x128"),  # (more workgroups than CUs: two share one)
+         (24, 1233, 2056, 384, "grouped_dma3", "128x256"), (16, 2075, 2056, 384, "grouped_dma3", "128x256"),
+         (1, 1695, 2056, 640, "grouped_dma3", "128x128"), (24, 3078, 768, 2048, "grouped_dma3", "128x128"),
+         (2, 5548, 2056, 384, "grouped_pingpong+grouped_dma3", "128x256")]
+
+
+@pytest.mark.parametrize("E,rows,N,K,kernel,tile", FORMS)
+def test_every_tiling(gpu, oracle, E, rows, N, K, kernel, tile):
+    from sglang_amd import _lib
+
+    plan = _lib.grouped_gemm_plan(E, rows, N, K)
+    print(f"case {E} {rows} {N} {K} {plan}", flush=True)
+    assert (plan["kernel"], plan["small_tile"]) == (kernel, tile)
+    g = torch.Generator().manual_seed(E + rows)
+    weight = torch.rand(E, generator=g) + 0.1
+    weight[E // 2] += E / 4
+    if E > 2:
+        weight[1] = 0
+    sizes = torch.bincount(torch.multinomial(weight, rows, replacement=True, generator=g), minlength=E).tolist()
+    a, w, sa, sw, offsets, T = _problem(sizes, N, K, rows + N)
+    out = _call(gpu, a, w, sa, sw, sizes, offsets, torch.bfloat16)
+    _verify(oracle, out, a, w, sa, sw, sizes, offsets, f"{E} {rows}")
+
+
 def test_experts_that_share_rows(gpu, oracle):
     """Overlapping offsets: every expert still multiplies the rows it names with its own weight; rows named twice hold the result of
     one of them."""
