@@ -245,22 +245,26 @@ int mi355_int8_scaled_mm(const void* a, const void* b, const float* sa, const fl
                          void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * Host-only query: which kernel and tiling mi355_fp8_blockwise_mm / mi355_int8_scaled_mm would run for a shape.
+ * Host-only query: which kernel and tiling the GEMM entry points would run for a shape (with a workspace of the size that
+ * their queries name and, for UE8M0, token words of a conforming pitch and base).
  * Stands in for the reference's shape dispatchers, which are compile-time ladders nobody can ask
  * (sgl-kernel/csrc/gemm/fp8_blockwise_gemm_kernel.cu:181-195, sgl-kernel/csrc/gemm/int8_gemm_kernel.cu:603-661);
  * here the choice is observable so that tests can prove every kernel variant is reached.
  *   aligned  nonzero if both operand base pointers and row strides are multiples of 16 bytes (rows are assumed dense)
  *   buf      receives a NUL-terminated "key=value ..." line:
- *            kernel=decode|decode_wavesplit|dma3|pingpong|pingpong128|pipelined|generic bm= bn= splits= kb_per_split=
- *            groups_per_wg= aligned= stages=   (stages: LDS stages of the mid-M kernel's pipeline, 0 for the other kernels)
+ *            kernel=decode|decode_wavesplit|wavesplit_tile|dma3|pingpong|pingpong128|pipelined|generic bm= bn= splits=
+ *            kb_per_split= groups_per_wg= aligned= stages=   (stages: LDS stages of the mid-M kernel's pipeline, 0 for the
+ *            other kernels) and for UE8M0 exponents=mfma|unpacked (unpacked: a launch in front expands them to fp32 scales)
  * Launches nothing and touches no device state.
  */
 int mi355_fp8_blockwise_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len);
+int mi355_fp8_blockwise_mm_ue8m0_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len);
+int mi355_fp8_scaled_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len);
 int mi355_int8_scaled_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len);
 
 /*
- * Host-only: the measured constants of the dispatcher's time models (sglang_amd/csrc/route_constants.h holds the table and
- * where each number comes from) and the plan a shape would get with ONE constant multiplied by `factor`.  No counterpart
+ * Host-only: the measured constants of the dispatcher's time models (sglang_amd/csrc/route_constants.h and tile_choice.h hold
+ * the tables and where each number comes from) and the plan a shape would get with ONE constant multiplied by `factor`.  No counterpart
  * in the reference, whose dispatch ladders hold their thresholds inline (fp8_blockwise_gemm_kernel.cu:181-195,
  * int8_gemm_kernel.cu:603-661); here a test perturbs every constant by +-10 % and checks that the benchmark shapes stay on
  * their kernels.  The perturbed copy is local to the calling thread and gone when the call returns.
@@ -380,11 +384,11 @@ int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const flo
  *          workspace, with M-major scales, and the bias is added in fp32 in the GEMM epilogue (the reference adds it
  *          after rounding the GEMM result to the output type: MI355_BIAS_ON_ROUNDED).  At decode sizes (M <= 16, 16-bit x, N % 128 == 0) there
  *          is no quantizer launch where that is the faster way: the GEMM kernel quantizes the tokens itself (the wave-split
- *          and streaming kernels in their prologues, the mid-M kernel by producer waves), with the same arithmetic; the result
- *          is bit-identical to the two-step sequence where the GEMM alone takes the same kernel.
- *          mi355_fp8_block_linear_plan (host only, dense 16-byte aligned operands assumed) writes the GEMM's plan in the
- *          format of mi355_fp8_blockwise_mm_plan followed by quantizer=fused|launch, and by wavesplit_waves=W where the
- *          wave-split kernel with W waves and its own quantizer runs in place of that plan.
+ *          kernel, the wave-split tile and the streaming kernel in their prologues, the mid-M kernel by producer waves), with
+ *          the same arithmetic; the result is bit-identical to the two-step sequence where the GEMM alone takes the same
+ *          kernel, that is where mi355_fp8_block_linear_plan without its last key equals mi355_fp8_blockwise_mm_plan.
+ *          mi355_fp8_block_linear_plan (host only, dense 16-byte aligned operands and 16-bit x assumed) writes the GEMM that
+ *          runs in the format of mi355_fp8_blockwise_mm_plan followed by quantizer=fused|launch.
  *   x [M, K] contiguous F32/F16/BF16, K % 128 == 0; w [N, K] e4m3fn row stride ldw; w_scale element (nb, kb) at
  *   w_scale[nb * ws_sn + kb * ws_sk]; bias NULL or [N] in the output dtype; out [M, N] BF16/F16 row stride ldo.
  *   workspace: mi355_fp8_block_linear_workspace_bytes(M, N, K) bytes, 256-byte aligned.
@@ -412,6 +416,7 @@ int mi355_fp8_block_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, size
  *   workspace: mi355_int8_linear_workspace_bytes(M, N, K) bytes, 256-byte aligned.
  */
 size_t mi355_int8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mi355_int8_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len); /* as mi355_fp8_block_linear_plan */
 int mi355_int8_linear(const void* x, int x_dtype, const void* w, const float* w_scale, const void* bias, void* out, int out_dtype,
                       int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo, void* workspace, size_t workspace_bytes,
                       void* stream);
@@ -426,6 +431,7 @@ int mi355_int8_linear(const void* x, int x_dtype, const void* w, const float* w_
  *   workspace: mi355_fp8_per_token_linear_workspace_bytes(M, N, K) bytes, 256-byte aligned.
  */
 size_t mi355_fp8_per_token_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mi355_fp8_per_token_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len); /* as mi355_fp8_block_linear_plan */
 int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void* w, const float* w_scale, const void* bias, void* out,
                                int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo, void* workspace,
                                size_t workspace_bytes, void* stream);
@@ -443,6 +449,7 @@ int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void* w, const 
  *   workspace: mi355_fp8_block_linear_ue8m0_workspace_bytes(M, N, K) bytes, 256-byte aligned.
  */
 size_t mi355_fp8_block_linear_ue8m0_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mi355_fp8_block_linear_ue8m0_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len); /* as mi355_fp8_block_linear_plan */
 int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const void* w, const void* sb_words, int64_t sb_sn, int64_t sb_sk,
                                  const void* bias, void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw,
                                  int64_t ldo, void* workspace, size_t workspace_bytes, void* stream);

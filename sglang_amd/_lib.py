@@ -39,7 +39,12 @@ EXPORTS = (
     "mi355_int8_scaled_mm",
     "mi355_fp8_blockwise_mm_plan",
     "mi355_fp8_block_linear_plan",
+    "mi355_fp8_blockwise_mm_ue8m0_plan",
+    "mi355_fp8_scaled_mm_plan",
     "mi355_int8_scaled_mm_plan",
+    "mi355_fp8_block_linear_ue8m0_plan",
+    "mi355_fp8_per_token_linear_plan",
+    "mi355_int8_linear_plan",
     "mi355_route_constant_count",
     "mi355_route_constant_name",
     "mi355_route_constant_value",
@@ -127,11 +132,13 @@ def lib() -> ctypes.CDLL:
     L.mi355_int8_scaled_mm_workspace_bytes.restype = sz
     L.mi355_int8_scaled_mm.argtypes = [vp, vp, vp, vp, vp, vp, i32] + [i64] * 6 + [vp, sz, vp]
     L.mi355_int8_scaled_mm.restype = i32
-    for fn in (L.mi355_fp8_blockwise_mm_plan, L.mi355_int8_scaled_mm_plan):
+    for fn in (L.mi355_fp8_blockwise_mm_plan, L.mi355_fp8_blockwise_mm_ue8m0_plan, L.mi355_fp8_scaled_mm_plan, L.mi355_int8_scaled_mm_plan):
         fn.argtypes = [i64, i64, i64, i32, ctypes.c_char_p, sz]
         fn.restype = i32
-    L.mi355_fp8_block_linear_plan.argtypes = [i64, i64, i64, ctypes.c_char_p, sz]
-    L.mi355_fp8_block_linear_plan.restype = i32
+    for fn in (L.mi355_fp8_block_linear_plan, L.mi355_fp8_block_linear_ue8m0_plan, L.mi355_fp8_per_token_linear_plan,
+               L.mi355_int8_linear_plan):
+        fn.argtypes = [i64, i64, i64, ctypes.c_char_p, sz]
+        fn.restype = i32
     L.mi355_per_token_quant_int8.argtypes = [vp, i32, vp, vp, i64, i64, vp]
     L.mi355_per_token_quant_int8.restype = i32
     L.mi355_per_token_quant_int8_sum.argtypes = [vp, i32, vp, vp, vp, i64, i64, vp]
@@ -185,30 +192,38 @@ def lib() -> ctypes.CDLL:
     return L
 
 
+def _parse(line: bytes) -> dict:
+    items = (item.split("=") for item in line.decode().split())
+    return {k: v if k in ("kernel", "quantizer", "exponents", "small_tile") else int(v) for k, v in items}
+
+
 def gemm_plan(kind: str, M: int, N: int, K: int, aligned: bool = True) -> dict:
-    """Kernel and tiling the library would use for an FP8 (`kind` "fp8") or INT8 ("int8") GEMM of this shape:
-    {"kernel": str, "bm": int, "bn": int, "splits": int, "kb_per_split": int, "groups_per_wg": int, "aligned": int, "stages": int}."""
-    fn = {"fp8": lib().mi355_fp8_blockwise_mm_plan, "int8": lib().mi355_int8_scaled_mm_plan}[kind]
+    """Kernel and tiling that an FP8 (`kind` "fp8": block scales, "fp8_ue8m0": packed exponents, "fp8_scaled": one scale per token
+    and channel) or INT8 ("int8") GEMM of this shape runs: {"kernel": str, "bm": int, "bn": int, "splits": int,
+    "kb_per_split": int, "groups_per_wg": int, "aligned": int, "stages": int}, and "exponents": "mfma" | "unpacked" for
+    "fp8_ue8m0"."""
+    L = lib()
+    fn = {"fp8": L.mi355_fp8_blockwise_mm_plan, "fp8_ue8m0": L.mi355_fp8_blockwise_mm_ue8m0_plan, "fp8_scaled": L.mi355_fp8_scaled_mm_plan,
+          "int8": L.mi355_int8_scaled_mm_plan}[kind]
     buf = ctypes.create_string_buffer(256)
     check(fn(M, N, K, int(aligned), buf, len(buf)))
-    out = {}
-    for item in buf.value.decode().split():
-        k, v = item.split("=")
-        out[k] = v if k == "kernel" else int(v)
-    return out
+    return _parse(buf.value)
+
+
+def linear_plan(kind: str, M: int, N: int, K: int) -> dict:
+    """What a one-call linear (`kind` "block", "ue8m0", "token_fp8" or "int8") of 16-bit tokens runs: `gemm_plan`'s keys for its
+    GEMM plus "quantizer": "fused" (the GEMM kernel quantizes the tokens itself) or "launch" (a quantizer launch in front)."""
+    L = lib()
+    fn = {"block": L.mi355_fp8_block_linear_plan, "ue8m0": L.mi355_fp8_block_linear_ue8m0_plan,
+          "token_fp8": L.mi355_fp8_per_token_linear_plan, "int8": L.mi355_int8_linear_plan}[kind]
+    buf = ctypes.create_string_buffer(256)
+    check(fn(M, N, K, buf, len(buf)))
+    return _parse(buf.value)
 
 
 def block_linear_plan(M: int, N: int, K: int) -> dict:
-    """Plan of the one-call block-FP8 linear: `gemm_plan`'s keys plus "quantizer": "fused" (the GEMM kernel quantizes the
-    tokens in its prologue) or "launch" (a quantizer launch in front of the GEMM); with "wavesplit_waves" where the wave-split
-    kernel of that many waves, with its own quantizer, runs instead."""
-    buf = ctypes.create_string_buffer(256)
-    check(lib().mi355_fp8_block_linear_plan(M, N, K, buf, len(buf)))
-    out = {}
-    for item in buf.value.decode().split():
-        k, v = item.split("=")
-        out[k] = v if k in ("kernel", "quantizer") else int(v)
-    return out
+    """`linear_plan` of the block-FP8 linear."""
+    return linear_plan("block", M, N, K)
 
 
 def route_constants() -> dict:
@@ -221,11 +236,7 @@ def gemm_plan_perturbed(kind: str, M: int, N: int, K: int, constant: int, factor
     """`gemm_plan` with the `constant`-th entry of the dispatcher's constants table multiplied by `factor`."""
     buf = ctypes.create_string_buffer(256)
     check(lib().mi355_gemm_plan_perturbed(int(kind == "fp8"), M, N, K, int(aligned), constant, factor, buf, len(buf)))
-    out = {}
-    for item in buf.value.decode().split():
-        k, v = item.split("=")
-        out[k] = v if k == "kernel" else int(v)
-    return out
+    return _parse(buf.value)
 
 
 def grouped_gemm_plan(num_experts: int, total_m: int, N: int, K: int) -> dict:
@@ -233,11 +244,7 @@ def grouped_gemm_plan(num_experts: int, total_m: int, N: int, K: int) -> dict:
     "grouped_dma3", "small_tile": "<64|128>x<128|256>", "max_big_tiles": int, "max_small_tiles": int, "tiles_n": int}."""
     buf = ctypes.create_string_buffer(256)
     check(lib().mi355_fp8_blockwise_scaled_grouped_mm_plan(num_experts, total_m, N, K, buf, len(buf)))
-    out = {}
-    for item in buf.value.decode().split():
-        k, v = item.split("=")
-        out[k] = v if k in ("kernel", "small_tile") else int(v)
-    return out
+    return _parse(buf.value)
 
 
 def check(status: int) -> None:

@@ -20,6 +20,8 @@ constexpr int GROUP_M = 8;    // M-tiles per group in the tile order
 
 constexpr int NUM_CUS = 256;
 
+constexpr int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 struct GemmParams {
   const uint8_t* a;  // tokens   [M, K], row stride lda
   const uint8_t* b;  // channels [N, K], row stride ldb

@@ -18,7 +18,9 @@
 //      128 rows, and where small tiles alone model faster (grouped_run): then every row goes to the second table.
 // Where the reference takes device arrays of per-expert pointers, strides and scale layouts as scratch that its own
 // set-up kernel fills, this interface takes the base pointers and strides and keeps its scratch in the workspace.
-#include "tile_choice.h"
+#include <cmath>
+
+#include "gemm_common.h"
 
 namespace mi355 {
 namespace {

@@ -21,6 +21,8 @@
 //   * workgroups are renumbered so that each of the 8 XCDs (own L2) works on a contiguous, M-grouped
 //     patch of output tiles.
 #include <mutex>
+#include <string>
+#include <vector>
 
 #include "gemm_common.h"
 #include "tile_choice.h"
@@ -406,8 +408,8 @@ int launch_tile(GemmParams& p, bool aligned, hipStream_t stream, const char* wha
                : launch_tile_inst<IS_FP8, BM, BN, WGM, WGN, false, false>(p, grid, lds, stream, what);
 }
 
-// Which kernel serves a problem, with which tiling.  One function decides for the launcher and for the plan query, so
-// what the query reports is what runs.
+// Which kernel serves a problem, with which tiling.  run_route decides for the launchers and for the plan queries (choose_linear
+// for the one-call linears), so what a query reports is what runs.
 enum RouteKernel { RK_DECODE = 0, RK_DMA3, RK_PINGPONG, RK_PIPELINED, RK_GENERIC, RK_WAVESPLIT, RK_PP128, RK_WAVESPLIT_TILE };
 const char* const ROUTE_NAMES[] = {"decode", "dma3", "pingpong", "pipelined", "generic", "decode_wavesplit", "pingpong128", "wavesplit_tile"};
 
@@ -445,6 +447,7 @@ int decode_dma3_channel_tile(bool is_fp8, int64_t N) {
   return bn;
 }
 
+// The route by the constants table; run_route below runs it or a tile that models faster.
 // `aligned`: both operand base pointers and row strides are multiples of 16 bytes and K % 16 == 0.
 // `fused_quant`: the tokens arrive unquantized and the kernel is to quantize them itself, which only the streaming
 // decode kernel can.
@@ -536,8 +539,15 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
   return r;
 }
 
-const RouteConstants g_route_defaults{};
-thread_local const RouteConstants* g_route_override = nullptr;  // set while a perturbed plan is queried
+// Both tables, an array of doubles as far as the queries of single constants go.
+struct DispatchConstants {
+  RouteConstants route;
+  TileModel tiles;
+};
+constexpr int CONSTANT_COUNT = ROUTE_CONSTANT_COUNT + TILE_CONSTANT_COUNT;
+static_assert(sizeof(DispatchConstants) == CONSTANT_COUNT * sizeof(double), "the tables are read as an array of doubles");
+const DispatchConstants g_defaults{};
+thread_local const DispatchConstants* g_override = nullptr;  // set while a perturbed plan is queried
 
 // The route that runs: choose_route's, or the tile that models faster (tile_choice.h).
 Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
@@ -576,7 +586,7 @@ Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int
       for (Entry& x : e) x.kind = -1;
     }
   };
-  if (&route_constants() != &g_route_defaults) return uncached_run_route(kind, M, N, K, lda, ldb, aligned);
+  if (g_override != nullptr) return uncached_run_route(kind, M, N, K, lda, ldb, aligned);
   static thread_local Table table;
   uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull) ^ (uint64_t)kind * 0x27d4eb2f165667c5ull;
   Entry& e = table.e[(h ^ (h >> 29)) >> 20 & (ENTRIES - 1)];
@@ -587,13 +597,6 @@ Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int
   return e.route;
 }
 int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K) { return run_route(kind, M, N, K, K, K, true).splits; }
-bool same_route(const Route& a, const Route& b) { return a.kernel == b.kernel && a.bm == b.bm && a.bn == b.bn && a.splits == b.splits; }
-// " run_bm=.. run_bn=.. run_splits=.. run_wavesplit=0|1" where another tile runs than the plan names
-void describe_run(char* buf, size_t len, const Route& plan, const Route& run) {
-  buf[0] = 0;
-  if (!same_route(plan, run))
-    snprintf(buf, len, " run_bm=%d run_bn=%d run_splits=%d run_wavesplit=%d", run.bm, run.bn, run.splits, (int)(run.kernel == RK_WAVESPLIT_TILE));
-}
 
 // out[kb * ld_out + m] = sa[m * sa_sm + kb * sa_sk]: token scales re-laid out M-major with a row pitch that is a multiple
 // of four floats.  One 32 x 32 tile per workgroup through LDS, so that reads and writes are both contiguous for either
@@ -741,55 +744,95 @@ const char* const ROUTE_CONSTANT_NAMES[ROUTE_CONSTANT_COUNT] = {
     "decode_dma3_min_workgroups",
     "linear_producer_min_decode_splits", "fused_quant_long_k_blocks", "fused_quant_short_k_blocks", "fused_quant_short_k_max_tokens"};
 
+// UE8M0: the kernels in which the MFMA applies the exponents; the others take them as fp32 scales, unpacked by a launch in front.
+bool applies_exponents(const Route& r, int64_t K) {
+  return ((r.kernel == RK_PINGPONG || r.kernel == RK_DMA3 || r.kernel == RK_WAVESPLIT) && K % KSTEP == 0) || r.kernel == RK_DECODE ||
+         r.kernel == RK_WAVESPLIT_TILE;
+}
+
+// in the order of TileModel
+std::vector<std::string> tile_constant_names() {
+  std::vector<std::string> names;
+  const auto add = [&](const std::string& prefix, std::initializer_list<const char*> fields) {
+    for (const char* f : fields) names.push_back(prefix + f);
+  };
+  for (const char* times : {"scaled.", "plain."}) {
+    add(times, {"launch", "busy", "split_us", "split_us_per_mb", "stream", "stream_us", "shared", "result_us_per_mb"});
+    for (const char* what : {"tile", "block"})
+      for (const TileSize& t : MID_TILES) names.push_back(std::string(times) + what + "[" + std::to_string(t.bm) + "x" + std::to_string(t.bn) + "]");
+    add(times, {"pp_tile", "pp_block", "pp_busy", "pp_store", "ws_launch", "ws_tile", "ws_kb", "ws_kb_busy", "ws_stream", "ws_stream_us",
+                "ws_result", "ws_norm"});
+  }
+  add("limits.", {"margin", "two_phase_margin", "large_weight_margin", "large_weight_max_tokens", "mid_wavesplit_max_weight", "ragged_max_weight",
+                  "ragged_max_factor", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
+                  "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
+                  "decode_short_max_weight", "decode_short_min_tokens"});
+  names.resize(TILE_CONSTANT_COUNT);
+  return names;
+}
+
 // LDS stages of the mid-M kernel's pipeline for this plan (0 for the other kernels, whose depth is fixed).
-int route_stages(bool is_fp8, const Route& r, int64_t M, int64_t N) {
+int route_stages(const Route& r, int64_t M, int64_t N) {
   if (r.kernel != RK_DMA3) return 0;
   const int64_t workgroups = ((M + r.bm - 1) / r.bm) * ((N + r.bn - 1) / r.bn) * r.splits;
   return dma3_stages(r.bm, r.bn, workgroups);  // the INT8 kernel of the same structure follows the same rule
 }
 
-int describe_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len, const char* what) {
+int check_query(int64_t M, int64_t N, int64_t K, const char* buf, size_t buf_len, const char* what) {
   clear_error();
   MI355_REQUIRE(buf != nullptr && buf_len > 0, MI355_ERR_INVALID_ARGUMENT, "%s: no buffer", what);
   MI355_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31),
                 MI355_ERR_INVALID_ARGUMENT, "%s: shape out of range", what);
-  const Route r = choose_route(is_fp8, M, N, K, K, K, aligned != 0 && K % 16 == 0);
-  char run[96];
-  describe_run(run, sizeof run, r, run_route(is_fp8 ? GK_F32 : GK_INT8, M, N, K, K, K, r.aligned));
+  return MI355_OK;
+}
+int write_route(const Route& r, int64_t M, int64_t N, const char* more, char* buf, size_t buf_len, const char* what) {
   const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d%s",
                          ROUTE_NAMES[r.kernel], r.bm, r.bn, r.splits, r.kb_per_split, r.groups_per_wg, (int)r.aligned,
-                         route_stages(is_fp8, r, M, N), run);
+                         route_stages(r, M, N), more);
   MI355_REQUIRE(n > 0 && (size_t)n < buf_len, MI355_ERR_INVALID_ARGUMENT, "%s: buffer of %zu bytes is too small", what,
                 buf_len);
   return MI355_OK;
 }
+int describe_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len, const char* what) {
+  const int rc = check_query(M, N, K, buf, buf_len, what);
+  if (rc != MI355_OK) return rc;
+  const bool ok = aligned != 0 && K % 16 == 0;
+  const Route r = run_route(kind, M, N, K, K, K, ok);
+  if (kind == GK_UE8M0 && !applies_exponents(r, K))
+    return write_route(run_route(GK_F32, M, N, K, K, K, ok), M, N, " exponents=unpacked", buf, buf_len, what);
+  return write_route(r, M, N, kind == GK_UE8M0 ? " exponents=mfma" : "", buf, buf_len, what);
+}
 
 }  // namespace
 
-const RouteConstants& route_constants() { return g_route_override ? *g_route_override : g_route_defaults; }
+const RouteConstants& route_constants() { return (g_override ? g_override : &g_defaults)->route; }
+const TileModel& tile_model() { return (g_override ? g_override : &g_defaults)->tiles; }
 const char* route_constant_name(int index) {
-  return index >= 0 && index < ROUTE_CONSTANT_COUNT ? ROUTE_CONSTANT_NAMES[index] : nullptr;
+  if (index < 0 || index >= CONSTANT_COUNT) return nullptr;
+  if (index < ROUTE_CONSTANT_COUNT) return ROUTE_CONSTANT_NAMES[index];
+  static const std::vector<std::string> names = tile_constant_names();
+  return names[index - ROUTE_CONSTANT_COUNT].c_str();
 }
 }  // namespace mi355
 
 using namespace mi355;
 
-extern "C" int mi355_route_constant_count(void) { return ROUTE_CONSTANT_COUNT; }
+extern "C" int mi355_route_constant_count(void) { return CONSTANT_COUNT; }
 extern "C" const char* mi355_route_constant_name(int index) { return route_constant_name(index); }
 extern "C" double mi355_route_constant_value(int index) {
-  return index >= 0 && index < ROUTE_CONSTANT_COUNT ? reinterpret_cast<const double*>(&g_route_defaults)[index] : 0.0;
+  return index >= 0 && index < CONSTANT_COUNT ? reinterpret_cast<const double*>(&g_defaults)[index] : 0.0;
 }
 extern "C" int mi355_gemm_plan_perturbed(int is_fp8, int64_t M, int64_t N, int64_t K, int aligned, int constant_index, double factor,
                                          char* buf, size_t buf_len) {
   const char* what = "mi355_gemm_plan_perturbed";
   clear_error();
-  MI355_REQUIRE(constant_index >= 0 && constant_index < ROUTE_CONSTANT_COUNT && factor > 0.0, MI355_ERR_INVALID_ARGUMENT,
-                "%s: constant index 0..%d and a positive factor", what, ROUTE_CONSTANT_COUNT - 1);
-  RouteConstants rc = g_route_defaults;
-  reinterpret_cast<double*>(&rc)[constant_index] *= factor;
-  g_route_override = &rc;
-  const int status = describe_route(is_fp8 != 0, M, N, K, aligned, buf, buf_len, what);
-  g_route_override = nullptr;
+  MI355_REQUIRE(constant_index >= 0 && constant_index < CONSTANT_COUNT && factor > 0.0, MI355_ERR_INVALID_ARGUMENT,
+                "%s: constant index 0..%d and a positive factor", what, CONSTANT_COUNT - 1);
+  DispatchConstants perturbed = g_defaults;
+  reinterpret_cast<double*>(&perturbed)[constant_index] *= factor;
+  g_override = &perturbed;
+  const int status = describe_route(is_fp8 ? GK_F32 : GK_INT8, M, N, K, aligned, buf, buf_len, what);
+  g_override = nullptr;
   return status;
 }
 
@@ -956,18 +999,14 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
   const Route r = run_route(GK_UE8M0, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
   const bool words_conform = (sa_sk & 3) == 0 && sa_sk >= ((M + 3) & ~3ll) && (reinterpret_cast<uintptr_t>(sa_words) & 15) == 0;
-  if (r.kernel == RK_PINGPONG && K % KSTEP == 0 && words_conform) {
-    // the MFMA applies both exponents itself: no scale arithmetic at all
-    p.splits = 1, p.kb_per_split = p.kb_total;
-    return launch_fp8_pp_ue8m0(p, st, what);
-  }
-  if (r.kernel == RK_WAVESPLIT && K % KSTEP == 0) {
-    // decode sizes on the wave-split kernel: the same, one launch, no workspace
-    return launch_fp8_wavesplit_ue8m0(p, st, what);
-  }
-  if ((r.kernel == RK_DMA3 && K % KSTEP == 0 && words_conform) || r.kernel == RK_DECODE || r.kernel == RK_WAVESPLIT_TILE) {
-    // mid-M and streaming decode: the same kernels with the exponents applied by the MFMA; the workspace only holds
-    // split-K partial sums (the decode kernel reads the words with ordinary loads: any pitch will do)
+  const bool wants_conforming = r.kernel == RK_PINGPONG || r.kernel == RK_DMA3;  // (the decode kernels read the words with ordinary loads: any pitch will do)
+  if (applies_exponents(r, K) && (words_conform || !wants_conforming)) {
+    // the MFMA applies both exponents itself: no scale arithmetic at all, and the workspace only holds split-K partial sums
+    if (r.kernel == RK_PINGPONG) {
+      p.splits = 1, p.kb_per_split = p.kb_total;
+      return launch_fp8_pp_ue8m0(p, st, what);
+    }
+    if (r.kernel == RK_WAVESPLIT) return launch_fp8_wavesplit_ue8m0(p, st, what);
     p.ue8m0 = 1;
     return run_gemm<true>(p, r, workspace, workspace_bytes_given, st, what);
   }
@@ -1098,7 +1137,7 @@ Route linear_producer_route(int64_t M, int64_t N, int64_t K, int64_t ldw) {
   const bool few_tokens = (double)M < rc.decode_dma3_min_tokens &&
                           choose_route(true, (int64_t)rc.decode_dma3_min_tokens, N, K, K, ldw, true).kernel == RK_DMA3;
   const bool many_ranges = decode_supported(M, N, K) && (double)decode_splits(M, N, K) >= rc.linear_producer_min_decode_splits;
-  if (few_tokens || many_ranges) plain.kernel = RK_DMA3, plain.bm = 64, plain.bn = bn, plain.splits = 1, plain.kb_per_split = (int)(K / KSTEP);
+  if (few_tokens || many_ranges) plain.kernel = RK_DMA3, plain.bm = 64, plain.bn = bn, plain.splits = 1, plain.kb_per_split = (int)(K / KSTEP), plain.groups_per_wg = 0;
   return plain;
 }
 
@@ -1144,6 +1183,45 @@ bool tile_quant_preferred(const Route& run, int64_t M, int64_t N, int64_t K) {
   const int64_t pieces = M * K / 8, threads = 512, rounds = (N + (int64_t)run.bn * NUM_CUS - 1) / ((int64_t)run.bn * NUM_CUS);
   return pieces <= 10 * threads && pieces * rounds <= 10 * threads;
 }
+bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
+  const int plain = choose_route(true, M, N, K, K, ldw, true).kernel;
+  if (plain == RK_DMA3) return false;  // the mid-M kernel at decode sizes beats the streaming kernel by more than a launch
+  if (plain != RK_WAVESPLIT) return true;
+  const RouteConstants& rc = route_constants();
+  const double kb = (double)(K / KSTEP);
+  if (kb > rc.fused_quant_long_k_blocks) return false;
+  return !(kb <= rc.fused_quant_short_k_blocks && (double)M > rc.fused_quant_short_k_max_tokens);
+}
+
+// What a one-call linear does: quantize inside the GEMM kernel, in one of four ways, or by a launch in front of the GEMM.  One
+// function decides for the entry points and for the plan queries.  `gemm` is the GEMM that runs; q_ok: the fused quantizers can
+// read the operands (wavesplit_quant_operands), w_aligned: the weight's base and row stride are multiples of 16 bytes.
+enum LinearMode { LM_LAUNCH, LM_TILE, LM_WAVESPLIT, LM_PRODUCER, LM_STREAMING };
+struct LinearRoute {
+  LinearMode mode;
+  Route gemm;
+};
+LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K, int64_t ldw, bool q_ok, bool w_aligned) {
+  const GemmKind kind = quant == WavesplitQuant::BLOCK_F32 ? GK_F32 : quant == WavesplitQuant::BLOCK_UE8M0 ? GK_UE8M0 : quant == WavesplitQuant::TOKEN_FP8 ? GK_UNIT : GK_INT8;
+  const Route run = run_route(kind, M, N, K, K, ldw, w_aligned && K % 16 == 0);
+  if (!q_ok) return {LM_LAUNCH, run};
+  if (tile_quant_preferred(run, M, N, K)) return {LM_TILE, run};
+  if (wavesplit_quant_preferred(quant, M, N, K, ldw)) {
+    Route r{};
+    r.kernel = RK_WAVESPLIT, r.bm = 16, r.bn = wavesplit_two_tiles(quant != WavesplitQuant::TOKEN_INT8, M, N, K) ? 32 : 16, r.splits = 1;
+    r.kb_per_split = (int)(K / KSTEP), r.groups_per_wg = wavesplit_shape(K).waves, r.aligned = true;
+    return {LM_WAVESPLIT, r};
+  }
+  // the block linear's other decode kernels; the wave-split tile is faster than they are also behind a quantizer launch
+  if (quant != WavesplitQuant::BLOCK_F32 || (M <= 16 && run.kernel == RK_WAVESPLIT_TILE)) return {LM_LAUNCH, run};
+  if (M <= 16) {
+    const Route r = linear_producer_route(M, N, K, ldw);
+    if (r.kernel == RK_DMA3) return {LM_PRODUCER, r};  // one round of unsplit 64-token tiles: producer waves of that kernel quantize the tokens
+  }
+  const Route r = choose_route(true, M, N, K, K, ldw, true, true);
+  if (r.kernel == RK_DECODE && fused_quant_preferred(M, N, K, ldw)) return {LM_STREAMING, r};
+  return {LM_LAUNCH, run};
+}
 int run_tile_quant(GemmParams& p, WavesplitQuant kind, const Route& run, const void* x, int x_dtype, void* stream, const char* what) {
   p.x16 = x, p.ldx = p.K, p.x_dtype = x_dtype;
   p.kb_total = p.K / KSTEP;
@@ -1161,15 +1239,6 @@ int run_wavesplit_quant(GemmParams& p, WavesplitQuant kind, const void* x, int x
   return launch_wavesplit_quant(p, kind, static_cast<hipStream_t>(stream), what);
 }
 
-bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
-  const int plain = choose_route(true, M, N, K, K, ldw, true).kernel;
-  if (plain == RK_DMA3) return false;  // the mid-M kernel at decode sizes beats the streaming kernel by more than a launch
-  if (plain != RK_WAVESPLIT) return true;
-  const RouteConstants& rc = route_constants();
-  const double kb = (double)(K / KSTEP);
-  if (kb > rc.fused_quant_long_k_blocks) return false;
-  return !(kb <= rc.fused_quant_short_k_blocks && (double)M > rc.fused_quant_short_k_max_tokens);
-}
 }  // namespace
 
 extern "C" size_t mi355_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -1207,43 +1276,21 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   const size_t sa_bytes = align256((size_t)pitch * (size_t)(K / KSTEP) * 4u);
   // Decode sizes: the GEMM kernel quantizes the tokens itself (same arithmetic), no quantizer launch - except where a
   // quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
-  const bool ptr_ok = x_dtype != MI355_F32 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
   const bool w_aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
-  const Route run = run_route(GK_F32, M, N, K, K, ldw, w_aligned);
-  const bool tile = M <= 16 && run.kernel == RK_WAVESPLIT_TILE;  // faster than the kernels below also behind a quantizer launch
-  const bool tile_quant = tile && wavesplit_quant_operands(x, x_dtype, w, ldw) && tile_quant_preferred(run, M, N, K);
-  if (tile_quant || (wavesplit_quant_operands(x, x_dtype, w, ldw) && wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, ldw))) {
+  const LinearRoute linear = choose_linear(WavesplitQuant::BLOCK_F32, M, N, K, ldw, wavesplit_quant_operands(x, x_dtype, w, ldw), w_aligned);
+  if (linear.mode != LM_LAUNCH) {
     GemmParams p;
     bool empty;
+    // (a / sa are not read by the kernels in these modes; they only have to satisfy the checks)
     const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, pitch, ws_sn, ws_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
     p.bias = bias, p.bias_rounded = bias_rounded;
-    p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
-    if (tile_quant) return run_tile_quant(p, WavesplitQuant::BLOCK_F32, run, x, x_dtype, stream, what);
-    return run_wavesplit_quant(p, WavesplitQuant::BLOCK_F32, x, x_dtype, stream, what);
-  }
-  if (ptr_ok && M <= 16 && !tile) {
-    const Route plain = linear_producer_route(M, N, K, ldw);
-    if (plain.kernel == RK_DMA3) {  // one round of unsplit 64-token tiles: producer waves of that kernel quantize the tokens
-      GemmParams p;
-      bool empty;
-      const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, (M + 3) & ~3ll, ws_sn, ws_sk, ldo, p, empty);
-      if (rc != MI355_OK || empty) return rc;
-      p.bias = bias, p.bias_rounded = bias_rounded;
-      p.x16 = x, p.ldx = K, p.x_dtype = x_dtype, p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
-      p.kb_total = K / KSTEP, p.splits = 1, p.kb_per_split = p.kb_total;
-      return launch_fp8_dma3_quant(p, plain.bn, static_cast<hipStream_t>(stream), what);
-    }
-  }
-  if (ptr_ok && !tile && choose_route(true, M, N, K, K, ldw, true, true).kernel == RK_DECODE && fused_quant_preferred(M, N, K, ldw)) {
-    GemmParams p;
-    bool empty;
-    // a / sa are not read by the kernel in this mode; they only have to satisfy the checks
-    int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, (M + 3) & ~3ll, ws_sn, ws_sk, ldo, p, empty);
-    if (rc != MI355_OK || empty) return rc;
-    p.bias = bias, p.bias_rounded = bias_rounded;
     p.x16 = x, p.ldx = K, p.x_dtype = x_dtype, p.x_by_reciprocal = quant_mode == MI355_QUANT_RCP;
-    return run_gemm<true>(p, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
+    if (linear.mode == LM_TILE) return run_tile_quant(p, WavesplitQuant::BLOCK_F32, linear.gemm, x, x_dtype, stream, what);
+    if (linear.mode == LM_WAVESPLIT) return run_wavesplit_quant(p, WavesplitQuant::BLOCK_F32, x, x_dtype, stream, what);
+    if (linear.mode == LM_STREAMING) return run_gemm<true>(p, linear.gemm, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
+    p.kb_total = K / KSTEP, p.splits = 1, p.kb_per_split = p.kb_total;
+    return launch_fp8_dma3_quant(p, linear.gemm.bn, static_cast<hipStream_t>(stream), what);
   }
   // quantize with q = x / s, the arithmetic of the reference's column-major path (fp8_kernel.py:164-212 via fp8_utils.py:201-203),
   // or with q = x * (1 / s), that of its row-major path (fp8_kernel.py:156-158); the scale layout here is the library's own
@@ -1275,25 +1322,28 @@ extern "C" int mi355_fp8_block_linear_mode(const void* x, int x_dtype, int quant
                       K, ldw, ldo, workspace, workspace_bytes_given, stream);
 }
 
+namespace {
+int describe_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len, const char* what) {
+  int rc = check_query(M, N, K, buf, buf_len, what);
+  if (rc != MI355_OK) return rc;
+  const bool block = quant == WavesplitQuant::BLOCK_F32 || quant == WavesplitQuant::BLOCK_UE8M0;
+  MI355_REQUIRE(K % (block ? KSTEP : 8) == 0, MI355_ERR_INVALID_ARGUMENT, "%s: K must be a multiple of %d", what, block ? KSTEP : 8);
+  const LinearRoute r = choose_linear(quant, M, N, K, K, K % 16 == 0, K % 16 == 0);
+  return write_route(r.gemm, M, N, r.mode == LM_LAUNCH ? " quantizer=launch" : " quantizer=fused", buf, buf_len, what);
+}
+}  // namespace
+
 extern "C" int mi355_fp8_block_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len) {
-  const char* what = "mi355_fp8_block_linear_plan";
-  clear_error();
-  MI355_REQUIRE(buf != nullptr && buf_len > 0, MI355_ERR_INVALID_ARGUMENT, "%s: no buffer", what);
-  MI355_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) && K % KSTEP == 0,
-                MI355_ERR_INVALID_ARGUMENT, "%s: shape out of range (K must be a multiple of 128)", what);
-  const Route plain = linear_producer_route(M, N, K, K);
-  const bool producer = M <= 16 && plain.kernel == RK_DMA3;  // the mid-M kernel's producer waves quantize
-  const bool fused = producer || (choose_route(true, M, N, K, K, K, true, true).kernel == RK_DECODE && fused_quant_preferred(M, N, K, K));
-  const Route r = producer ? plain : choose_route(true, M, N, K, K, K, true, fused);
-  const bool wavesplit = wavesplit_quant_preferred(WavesplitQuant::BLOCK_F32, M, N, K, K);
-  char instead[96] = "";
-  describe_run(instead, sizeof instead, choose_route(true, M, N, K, K, K, true), run_route(GK_F32, M, N, K, K, K, true));
-  if (wavesplit) snprintf(instead, sizeof instead, " wavesplit_waves=%d", wavesplit_shape(K).waves);
-  const int n = snprintf(buf, buf_len, "kernel=%s bm=%d bn=%d splits=%d kb_per_split=%d groups_per_wg=%d aligned=%d stages=%d quantizer=%s%s",
-                         ROUTE_NAMES[r.kernel], r.bm, r.bn, r.splits, r.kb_per_split, r.groups_per_wg, (int)r.aligned,
-                         route_stages(true, r, M, N), fused ? "fused" : "launch", instead);
-  MI355_REQUIRE(n > 0 && (size_t)n < buf_len, MI355_ERR_INVALID_ARGUMENT, "%s: buffer of %zu bytes is too small", what, buf_len);
-  return MI355_OK;
+  return describe_linear(WavesplitQuant::BLOCK_F32, M, N, K, buf, buf_len, "mi355_fp8_block_linear_plan");
+}
+extern "C" int mi355_fp8_block_linear_ue8m0_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len) {
+  return describe_linear(WavesplitQuant::BLOCK_UE8M0, M, N, K, buf, buf_len, "mi355_fp8_block_linear_ue8m0_plan");
+}
+extern "C" int mi355_fp8_per_token_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len) {
+  return describe_linear(WavesplitQuant::TOKEN_FP8, M, N, K, buf, buf_len, "mi355_fp8_per_token_linear_plan");
+}
+extern "C" int mi355_int8_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, size_t buf_len) {
+  return describe_linear(WavesplitQuant::TOKEN_INT8, M, N, K, buf, buf_len, "mi355_int8_linear_plan");
 }
 
 extern "C" size_t mi355_int8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -1363,11 +1413,10 @@ extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, cons
   p.M = (int)M, p.N = (int)N, p.K = (int)K;
   p.lda = K, p.ldb = ldw, p.ldo = ldo;
   p.out_dtype = out_dtype;
-  const bool fusable = wavesplit_quant_operands(x, x_dtype, w, ldw);
-  const Route run = run_route(GK_INT8, M, N, K, K, ldw, fusable && K % 16 == 0);
-  if (fusable && tile_quant_preferred(run, M, N, K)) return run_tile_quant(p, WavesplitQuant::TOKEN_INT8, run, x, x_dtype, stream, what);
-  if (fusable && wavesplit_quant_preferred(WavesplitQuant::TOKEN_INT8, M, N, K, ldw))
-    return run_wavesplit_quant(p, WavesplitQuant::TOKEN_INT8, x, x_dtype, stream, what);
+  const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);
+  const LinearRoute linear = choose_linear(WavesplitQuant::TOKEN_INT8, M, N, K, ldw, q_ok, q_ok);
+  if (linear.mode == LM_TILE) return run_tile_quant(p, WavesplitQuant::TOKEN_INT8, linear.gemm, x, x_dtype, stream, what);
+  if (linear.mode == LM_WAVESPLIT) return run_wavesplit_quant(p, WavesplitQuant::TOKEN_INT8, x, x_dtype, stream, what);
   const int rc = mi355_per_token_quant_int8(x, x_dtype, q, sa, M, K, stream);
   if (rc != MI355_OK) return rc;
   return run_gemm<false>(p, q + q_bytes + sa_bytes, workspace_bytes_given - q_bytes - sa_bytes, static_cast<hipStream_t>(stream), what);
@@ -1400,17 +1449,16 @@ extern "C" int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void
   const size_t q_bytes = align256((size_t)M * (size_t)K);
   float* sa = reinterpret_cast<float*>(q + q_bytes);
   const size_t sa_bytes = align256((size_t)M * 4u);
-  const bool fusable = wavesplit_quant_operands(x, x_dtype, w, ldw);
-  const Route run = run_route(GK_UNIT, M, N, K, K, ldw, fusable && K % 16 == 0);
-  const bool tile_quant = fusable && tile_quant_preferred(run, M, N, K);
-  if (tile_quant || (fusable && wavesplit_quant_preferred(WavesplitQuant::TOKEN_FP8, M, N, K, ldw))) {
+  const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);
+  const LinearRoute linear = choose_linear(WavesplitQuant::TOKEN_FP8, M, N, K, ldw, q_ok, q_ok);
+  if (linear.mode != LM_LAUNCH) {
     GemmParams p;
     bool empty;
     // (the block scales are not read in this mode; they only have to satisfy the checks)
     const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, 0, 0, 0, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
     p.col_scale = w_scale, p.bias = bias;
-    if (tile_quant) return run_tile_quant(p, WavesplitQuant::TOKEN_FP8, run, x, x_dtype, stream, what);
+    if (linear.mode == LM_TILE) return run_tile_quant(p, WavesplitQuant::TOKEN_FP8, linear.gemm, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::TOKEN_FP8, x, x_dtype, stream, what);
   }
   const int rc = mi355_per_token_quant_fp8(x, x_dtype, q, sa, M, K, stream);
@@ -1452,17 +1500,16 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
   void* sa_words = q + q_bytes;
   const int64_t pitch = (M + 3) & ~3ll;
   const size_t sa_bytes = align256((size_t)pitch * (size_t)((K / KSTEP + 3) / 4) * 4u);
-  const bool fusable = wavesplit_quant_operands(x, x_dtype, w, ldw);
-  const Route run = run_route(GK_UE8M0, M, N, K, K, ldw, fusable);
-  const bool tile_quant = fusable && tile_quant_preferred(run, M, N, K);
-  if (tile_quant || (fusable && wavesplit_quant_preferred(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw))) {
+  const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);
+  const LinearRoute linear = choose_linear(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw, q_ok, q_ok);
+  if (linear.mode != LM_LAUNCH) {
     GemmParams p;
     bool empty;
     const float* words = static_cast<const float*>(sb_words);  // (strides of the packed words stand in for fp32 ones)
     const int rc = fp8_mm_params(what, x, w, words, words, out, out_dtype, M, N, K, K, ldw, 1, pitch, sb_sn, sb_sk, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
     p.bias = bias, p.bias_rounded = bias_rounded;
-    if (tile_quant) return run_tile_quant(p, WavesplitQuant::BLOCK_UE8M0, run, x, x_dtype, stream, what);
+    if (linear.mode == LM_TILE) return run_tile_quant(p, WavesplitQuant::BLOCK_UE8M0, linear.gemm, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::BLOCK_UE8M0, x, x_dtype, stream, what);
   }
   // q = x * (448 / amax) with the scale rounded up to a power of two: per_token_group_quant_8bit_v2.cu:77-78 with scale_ue8m0
@@ -1474,9 +1521,17 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
 }
 
 extern "C" int mi355_fp8_blockwise_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len) {
-  return describe_route(true, M, N, K, aligned, buf, buf_len, "mi355_fp8_blockwise_mm_plan");
+  return describe_route(GK_F32, M, N, K, aligned, buf, buf_len, "mi355_fp8_blockwise_mm_plan");
+}
+
+extern "C" int mi355_fp8_blockwise_mm_ue8m0_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len) {
+  return describe_route(GK_UE8M0, M, N, K, aligned, buf, buf_len, "mi355_fp8_blockwise_mm_ue8m0_plan");
+}
+
+extern "C" int mi355_fp8_scaled_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len) {
+  return describe_route(GK_UNIT, M, N, K, aligned, buf, buf_len, "mi355_fp8_scaled_mm_plan");
 }
 
 extern "C" int mi355_int8_scaled_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len) {
-  return describe_route(false, M, N, K, aligned, buf, buf_len, "mi355_int8_scaled_mm_plan");
+  return describe_route(GK_INT8, M, N, K, aligned, buf, buf_len, "mi355_int8_scaled_mm_plan");
 }

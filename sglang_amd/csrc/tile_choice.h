@@ -12,15 +12,6 @@
 #include "gemm_common.h"
 
 namespace mi355 {
-namespace {
-
-enum GemmKind { GK_F32, GK_UE8M0, GK_UNIT, GK_INT8 };  // FP8 with block scales, with exponents, with epilogue scales; INT8
-enum TileFamily { TF_NONE, TF_DMA, TF_WAVESPLIT, TF_TWO_PHASE };
-
-struct TileChoice {
-  int family, bm, bn, splits;
-  double us;
-};
 
 struct TileTimes {
   // mid-M tile: launch + rounds of one workgroup per CU (64 x 128: two where there are more workgroups than CUs, each then
@@ -33,13 +24,13 @@ struct TileTimes {
   // together with the weight stream (ws_norm: how far the two overlap)
   double ws_launch, ws_tile, ws_kb, ws_kb_busy, ws_stream, ws_stream_us, ws_result, ws_norm;
 };
-constexpr TileTimes SCALED_TIMES = {
+constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     1.93, 0.586, 4.31, 0.217, 4.18, -4.54, 1.808, 0.421,
     {2.33, 2.83, 3.02, 3.40, 3.53, 4.64, 2.57, 3.31, 3.96, 4.32, 2.64, 3.53, 4.44},
     {0.219, 0.277, 0.317, 0.385, 0.419, 0.533, 0.288, 0.363, 0.441, 0.532, 0.334, 0.445, 0.535},
     7.88, 0.567, 1.70, 12.5,
     2.74, 1.041, 0.00591, 0.00334, 5.49, -3.81, 0.253, 1.511};
-constexpr TileTimes PLAIN_TIMES = {
+constexpr TileTimes PLAIN_TIMES = {  // FP8 with epilogue scales, INT8
     1.77, 0.777, 3.81, 0.251, 4.55, -2.24, 1.871, 0.402,
     {2.21, 2.72, 3.03, 3.17, 3.76, 4.72, 2.48, 3.12, 3.83, 4.14, 2.81, 3.80, 4.64},
     {0.165, 0.205, 0.240, 0.295, 0.333, 0.432, 0.224, 0.271, 0.339, 0.420, 0.278, 0.347, 0.431},
@@ -47,8 +38,35 @@ constexpr TileTimes PLAIN_TIMES = {
     2.71, 1.017, 0.00609, 0.00343, 5.07, -4.41, 0.282, 1.673};
 static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above follow MID_TILES");
 
+// Where the model is not asked or not trusted; both sides of each line stand beside the function that uses it.
+struct TileLimits {
+  double margin = 0.95, two_phase_margin = 0.90, large_weight_margin = 0.85, large_weight_max_tokens = 64.0;
+  double mid_wavesplit_max_weight = 100e6, ragged_max_weight = 100e6, ragged_max_factor = 2.0;
+  double decode_min_kblocks = 16.0, decode_padded_max_weight = 400e6, decode_max_weight = 140e6, decode_few_tokens_max_weight = 100e6;
+  double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
+  double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
+};
+struct TileModel {
+  TileTimes scaled = SCALED_TIMES, plain = PLAIN_TIMES;
+  TileLimits limits;
+};
+constexpr int TILE_CONSTANT_COUNT = sizeof(TileModel) / sizeof(double);
+// What the calling thread's dispatcher uses: the defaults above, or the perturbed copy a plan query installed.
+const TileModel& tile_model();
+
+namespace {
+
+enum GemmKind { GK_F32, GK_UE8M0, GK_UNIT, GK_INT8 };  // FP8 with block scales, with exponents, with epilogue scales; INT8
+enum TileFamily { TF_NONE, TF_DMA, TF_WAVESPLIT, TF_TWO_PHASE };
+
+struct TileChoice {
+  int family, bm, bn, splits;
+  double us;
+};
+
+const TileTimes& tile_times(GemmKind kind) { return kind == GK_F32 || kind == GK_UE8M0 ? tile_model().scaled : tile_model().plain; }
+
 double norm_of(double a, double b, double n) { return b <= 0.1 ? a : std::pow(std::pow(a, n) + std::pow(b, n), 1.0 / n); }
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // full rounds of `slots` workgroups and a partly filled one
 template <class Round>
 double rounds_of(int64_t workgroups, int64_t slots, Round round) {
@@ -113,9 +131,10 @@ TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
 // More than 16 tokens, K % 128 == 0, aligned operands: the fastest tile, or TF_NONE where `base`, what the route names (a mid-M
 // tile or the two-phase tile), models within 5 % of it (the two-phase tile 10 %): below that the model does not order two tiles.
 TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base) {
-  const TileTimes& t = kind == GK_F32 || kind == GK_UE8M0 ? SCALED_TIMES : PLAIN_TIMES;
+  const TileTimes& t = tile_times(kind);
   TileChoice best = best_dma_tile(t, M, N, K);
-  if (N * K <= 100000000) {  // (a larger weight streams better through the wide tiles: K = 4096 -> N = 28672 at 48 tokens 27.2 against 33.6 us)
+  const TileLimits& l = tile_model().limits;
+  if ((double)(N * K) <= l.mid_wavesplit_max_weight) {  // (a larger weight streams better through the wide tiles: K = 4096 -> N = 28672 at 48 tokens 27.2 against 33.6 us)
     const TileChoice ws = best_wavesplit_tile(t, M, N, K);
     if (ws.us < best.us) best = ws;
   }
@@ -130,7 +149,8 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
       if (MID_TILES[i].bm == base.bm && MID_TILES[i].bn == base.bn) base_us = dma_tile_us(t, i, M, N, K, base.splits);
   // (bound by a large weight's stream, the model knows little of how many CUs it takes: K = 10880 -> N = 16896 at 36 tokens, 132
   // unsplit tiles instead of 198 split ones, 54.8 against 48.3 us)
-  const double margin = base.family == TF_TWO_PHASE ? 0.90 : M <= 64 && N * K > 100000000 ? 0.85 : 0.95;
+  const bool large = (double)M <= l.large_weight_max_tokens && (double)(N * K) > l.mid_wavesplit_max_weight;
+  const double margin = base.family == TF_TWO_PHASE ? l.two_phase_margin : large ? l.large_weight_margin : l.margin;
   return best.us < margin * base_us ? best : TileChoice{TF_NONE, 0, 0, 1, 0.0};
 }
 
@@ -138,8 +158,10 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
 // twice as long as the mid-M tile would (K = 5920 -> N = 8320 at 90 tokens INT8: 42 against 18 us); not for the largest weights,
 // which the tile fetches once per 64 tokens (K = 16016 -> N = 26880 at 256 tokens 320 against 260 us).
 TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
-  const TileChoice ws = best_wavesplit_tile(PLAIN_TIMES, M, N, K);
-  return N * K <= 100000000 && ws.us < 2.0 * best_dma_tile(PLAIN_TIMES, M, N, K).us ? ws : TileChoice{TF_NONE, 0, 0, 1, 0.0};
+  const TileTimes& t = tile_model().plain;
+  const TileLimits& l = tile_model().limits;
+  const TileChoice ws = best_wavesplit_tile(t, M, N, K);
+  return (double)(N * K) <= l.ragged_max_weight && ws.us < l.ragged_max_factor * best_dma_tile(t, M, N, K).us ? ws : TileChoice{TF_NONE, 0, 0, 1, 0.0};
 }
 
 // Up to 16 tokens: the wave-split tile against the streaming and the register wave-split kernel.  It wins wherever K has more
@@ -151,14 +173,19 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
 // With fewer K blocks both are bound by the launch (K = 2048 -> N = 2048 4.3 / 4.4) except where there are many channels
 // (K = 1024 -> N = 12288 5.8/4.8, 8.0/4.9; but 512 -> 32768 5.9/6.8, 1536 -> 24576 9.3/9.6).
 TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K) {
-  const int64_t kb = ceil_div(K, KSTEP), weight = N * K;
+  const TileLimits& l = tile_model().limits;
+  const int64_t kb = ceil_div(K, KSTEP);
+  const double weight = (double)(N * K);
   // (the largest weights: the register kernel's single-tile stream is as fast for few tokens, unless it pads K to whole turns of 32 blocks:
   // K = 5152 -> N = 31936 INT8 at 5 tokens 50.3 us, 39.3 with the tile)
   const bool padded = kb <= 64 && (kb + 31) / 32 * 32 * 4 > kb * 5;
-  const int64_t most = padded ? 400000000 : M > (kind == GK_F32 ? 6 : 8) || kb > 64 ? 140000000 : 100000000;
-  const bool take = kb > 16 ? weight <= most : kb >= 8 && N >= 7168 && weight <= 20000000 && M > 8;
+  const bool few = (double)M <= (kind == GK_F32 ? l.decode_few_tokens_f32 : l.decode_few_tokens) && (double)kb <= l.decode_long_kblocks;
+  const double most = padded ? l.decode_padded_max_weight : few ? l.decode_few_tokens_max_weight : l.decode_max_weight;
+  const bool take = (double)kb > l.decode_min_kblocks ? weight <= most
+                                                      : (double)kb >= l.decode_short_min_kblocks && (double)N >= l.decode_short_min_channels &&
+                                                            weight <= l.decode_short_max_weight && (double)M > l.decode_short_min_tokens;
   if (!take) return TileChoice{TF_NONE, 0, 0, 1, 0.0};
-  const TileTimes& t = kind == GK_F32 || kind == GK_UE8M0 ? SCALED_TIMES : PLAIN_TIMES;
+  const TileTimes& t = tile_times(kind);
   TileChoice best{TF_NONE, 0, 0, 1, 1e30};
   for (int i = 0; i < 3; ++i) {
     static_assert(WAVESPLIT_TILES[2].bm == 16, "the 16-token tiles come first");

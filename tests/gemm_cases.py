@@ -4,7 +4,7 @@ parity tests, plus the full-size shapes of the benchmark configurations.
 A *variant* is one compiled code path: the kernel, its token-tile height, whether it writes split-K partial sums,
 for the decode kernel how many 128-channel groups a workgroup walks, for the wave-split decode kernel how many waves
 share a workgroup's K, whether a wave's share takes one turn of its four-slot register ring ("one_round") or several and
-whether the workgroup owns one 16-channel tile or two, for the large-M kernels whether K ends on a
+whether the workgroup owns one 16-channel tile or two, for the wave-split tile and the large-M kernels whether K ends on a
 128-byte block.  `variant_of` maps a plan (sglang_amd._lib.gemm_plan) to such a key.
 """
 
@@ -52,28 +52,6 @@ FP8_ROUTE_SHAPES = [
     (50, 3000, 4224), (40, 8, 1024), (100, 16, 4096), (1000, 8, 128),
 ]
 
-FP8_REQUIRED_VARIANTS = {
-    ("decode", "whole", "gpw1"), ("decode", "whole", "gpw2"), ("decode", "whole", "gpw3+"),
-    ("decode", "split", "gpw1"), ("decode", "split", "gpw2"), ("decode", "split", "gpw3+"),
-    ("decode_wavesplit", "w4", "one_round"), ("decode_wavesplit", "w4", "rounds"), ("decode_wavesplit", "w8", "one_round"),
-    ("decode_wavesplit", "w8", "rounds"),
-    ("decode_wavesplit", "w4", "one_round", "two_tiles"), ("decode_wavesplit", "w4", "rounds", "two_tiles"),
-    ("decode_wavesplit", "w8", "one_round", "two_tiles"), ("decode_wavesplit", "w8", "rounds", "two_tiles"),
-    ("dma3", 64, "whole"), ("dma3", 64, "split"), ("dma3", 128, "whole"), ("dma3", 128, "split"),
-    # "deep" = more than three LDS stages: always for 64 x 192 and 128 x 128 tiles; for 64 x 128 tiles where the launch has at
-    # most one workgroup per CU, which is the only place the plan puts them
-    ("dma3", 64, "whole", "bn128", "deep"), ("dma3", 64, "split", "bn128", "deep"),
-    ("dma3", 128, "whole", "bn128", "deep"), ("dma3", 128, "split", "bn128", "deep"),
-    ("dma3", 64, "whole", "bn192", "deep"), ("dma3", 64, "split", "bn192", "deep"),
-    ("dma3", 128, "whole", "bn192"), ("dma3", 128, "split", "bn192"),
-    ("pingpong", "kfull"), ("pingpong", "ktail"), ("pipelined", "kfull"), ("pipelined", "ktail"),
-    ("generic", 16, "aligned", "whole"), ("generic", 16, "aligned", "split"), ("generic", 16, "bytes", "split"),
-    ("generic", 32, "aligned", "split"), ("generic", 32, "bytes", "whole"),
-    ("generic", 64, "aligned", "whole"), ("generic", 64, "bytes", "whole"), ("generic", 64, "bytes", "split"),
-    ("generic", 128, "aligned", "whole"), ("generic", 128, "aligned", "split"), ("generic", 128, "bytes", "whole"),
-    ("generic", 128, "bytes", "split"), ("generic", 256, "bytes", "whole"),
-}
-
 # ---- INT8 (M, N, K): the operator requires K % 16 == 0 and N % 8 == 0
 INT8_ROUTE_SHAPES = [
     (16, 128, 512), (1, 6144, 4096), (1, 16640, 4480), (9, 33280, 2176), (16, 7168, 18432), (7, 33280, 4096),
@@ -95,19 +73,178 @@ INT8_ROUTE_SHAPES = [
     (20, 256, 2064), (33, 256, 272), (100, 256, 400), (100, 640, 2064),
 ]
 
-# (INT8 decode with a K split does not exist: from 8 K blocks on every INT8 decode shape takes the wave-split kernel)
-INT8_REQUIRED_VARIANTS = {
-    ("decode", "whole", "gpw1"), ("decode", "whole", "gpw2"), ("decode", "whole", "gpw3+"),
-    ("decode_wavesplit", "w4", "one_round"), ("decode_wavesplit", "w4", "rounds"), ("decode_wavesplit", "w8", "one_round"),
-    ("decode_wavesplit", "w8", "rounds"),
-    ("dma3", 64, "whole"), ("dma3", 64, "split"), ("pingpong128", "whole"), ("pingpong128", "split"),
-    # (the 128-channel tiles always run more than three stages: 128 x 128 four, 64 x 128 six - the plan puts 64 x 128 tiles only
-    # where the launch has at most one workgroup per CU)
-    ("dma3", 64, "whole", "bn128", "deep"), ("dma3", 64, "split", "bn128", "deep"), ("dma3", 128, "whole", "bn128", "deep"), ("dma3", 128, "split", "bn128", "deep"),
-    ("pingpong", "kfull"),
-    ("generic", 16, "aligned", "whole"), ("generic", 32, "aligned", "split"), ("generic", 64, "aligned", "whole"),
-    ("generic", 128, "aligned", "whole"), ("generic", 128, "aligned", "split"), ("generic", 256, "aligned", "whole"),
+# ---- every variant that each of the four GEMMs runs, with a small shape that reaches it ("fp8": block scales, "fp8_ue8m0": packed
+# exponents, "fp8_scaled": one scale per token and channel).  Found by asking the plan queries for 5.6 million random shapes
+# of 1 .. 5000 tokens, N up to 320000 and K up to 19000; tests/test_gemm_routes_cpu.py checks that other random shapes add none.
+VARIANT_SHAPES = {
+    "fp8": {
+        ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
+        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
+        ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
+        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 25216, 3968),
+        ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (68, 4256, 13696),
+        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (69, 8272, 17536),
+        ("dma3", 128, "whole", "bn128", "deep"): (4238, 584, 512), ("dma3", 128, "whole", "bn192"): (97, 32896, 128),
+        ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (130, 5736, 7936),
+        ("dma3", 160, "split", "bn192"): (129, 11264, 11648), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
+        ("dma3", 160, "whole", "bn192"): (129, 32896, 128), ("dma3", 192, "split", "bn128"): (3695, 272, 9728),
+        ("dma3", 192, "whole", "bn128"): (484, 8344, 128), ("dma3", 256, "split", "bn128"): (4112, 264, 12800),
+        ("dma3", 256, "whole", "bn128"): (641, 10760, 128), ("dma3", 64, "split", "bn128", "deep"): (33, 2936, 14592),
+        ("dma3", 64, "split", "bn192", "deep"): (17, 11168, 9216), ("dma3", 64, "split"): (97, 2752, 15488),
+        ("dma3", 64, "whole", "bn128", "deep"): (49, 4112, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
+        ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128), ("dma3", 64, "whole"): (129, 12832, 128),
+        ("dma3", 96, "split", "bn128", "deep"): (70, 2176, 18816), ("dma3", 96, "split", "bn192", "deep"): (266, 3656, 8576),
+        ("dma3", 96, "split"): (258, 4096, 10240), ("dma3", 96, "whole", "bn128", "deep"): (66, 25216, 384),
+        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (194, 16518, 128),
+        ("generic", 128, "aligned", "split"): (68, 8, 960), ("generic", 128, "aligned", "whole"): (66, 8, 16),
+        ("generic", 128, "bytes", "split"): (68, 8, 1038), ("generic", 128, "bytes", "whole"): (65, 8, 26),
+        ("generic", 16, "aligned", "split"): (1, 8, 912), ("generic", 16, "aligned", "whole"): (1, 8, 16),
+        ("generic", 16, "bytes", "split"): (1, 8, 907), ("generic", 16, "bytes", "whole"): (1, 8, 17),
+        ("generic", 256, "aligned", "split"): (1052, 6688, 928), ("generic", 256, "bytes", "split"): (1114, 7024, 922),
+        ("generic", 256, "bytes", "whole"): (1025, 6792, 17), ("generic", 32, "aligned", "split"): (17, 8, 960),
+        ("generic", 32, "aligned", "whole"): (17, 8, 32), ("generic", 32, "bytes", "split"): (20, 8, 983),
+        ("generic", 32, "bytes", "whole"): (17, 8, 18), ("generic", 64, "aligned", "split"): (33, 8, 912),
+        ("generic", 64, "aligned", "whole"): (33, 8, 32), ("generic", 64, "bytes", "split"): (39, 8, 941),
+        ("generic", 64, "bytes", "whole"): (33, 8, 18), ("pingpong", "kfull"): (223, 49272, 128),
+        ("pingpong", "ktail"): (1323, 11460, 16), ("pipelined", "ktail"): (1094, 6576, 16),
+        ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 32, "kfull"): (97, 579, 128),
+        ("wavesplit_tile", 16, 64, "kfull"): (65, 2728, 128), ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128),
+        ("wavesplit_tile", 32, 32, "kfull"): (49, 2064, 128), ("wavesplit_tile", 32, 64, "kfull"): (49, 4137, 128),
+        ("wavesplit_tile", 48, 16, "kfull"): (194, 616, 128), ("wavesplit_tile", 48, 32, "kfull"): (193, 1223, 128),
+        ("wavesplit_tile", 64, 32, "kfull"): (49, 4358, 128), ("wavesplit_tile", 64, 64, "kfull"): (1637, 291, 512),
+    },
+    "fp8_ue8m0": {
+        ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
+        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
+        ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
+        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 25216, 3968),
+        ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (68, 4256, 13696),
+        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (69, 8272, 17536),
+        ("dma3", 128, "whole", "bn128", "deep"): (4238, 584, 512), ("dma3", 128, "whole", "bn192"): (97, 32896, 128),
+        ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (130, 5736, 7936),
+        ("dma3", 160, "split", "bn192"): (129, 11264, 11648), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
+        ("dma3", 160, "whole", "bn192"): (129, 32896, 128), ("dma3", 192, "split", "bn128"): (3695, 272, 9728),
+        ("dma3", 192, "whole", "bn128"): (484, 8344, 128), ("dma3", 256, "split", "bn128"): (4112, 264, 12800),
+        ("dma3", 256, "whole", "bn128"): (641, 10760, 128), ("dma3", 64, "split", "bn128", "deep"): (33, 2936, 14592),
+        ("dma3", 64, "split", "bn192", "deep"): (17, 11168, 9216), ("dma3", 64, "split"): (97, 2752, 15488),
+        ("dma3", 64, "whole", "bn128", "deep"): (49, 4112, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
+        ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128), ("dma3", 64, "whole"): (129, 12832, 128),
+        ("dma3", 96, "split", "bn128", "deep"): (70, 2176, 18816), ("dma3", 96, "split", "bn192", "deep"): (266, 3656, 8576),
+        ("dma3", 96, "split"): (258, 4096, 10240), ("dma3", 96, "whole", "bn128", "deep"): (66, 25216, 384),
+        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (194, 16518, 128),
+        ("generic", 16, "aligned", "split", "unpacked"): (1, 8, 1024), ("generic", 16, "aligned", "whole", "unpacked"): (1, 8, 128),
+        ("pingpong", "kfull"): (223, 49272, 128), ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128),
+        ("wavesplit_tile", 16, 32, "kfull"): (97, 579, 128), ("wavesplit_tile", 16, 64, "kfull", "unpacked"): (7, 12824, 7808),
+        ("wavesplit_tile", 16, 64, "kfull"): (65, 2728, 128), ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128),
+        ("wavesplit_tile", 32, 32, "kfull"): (49, 2064, 128), ("wavesplit_tile", 32, 64, "kfull"): (49, 4137, 128),
+        ("wavesplit_tile", 48, 16, "kfull"): (194, 616, 128), ("wavesplit_tile", 48, 32, "kfull"): (193, 1223, 128),
+        ("wavesplit_tile", 64, 32, "kfull"): (49, 4358, 128), ("wavesplit_tile", 64, 64, "kfull"): (1637, 291, 512),
+    },
+    "fp8_scaled": {
+        ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
+        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
+        ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
+        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 25216, 3968),
+        ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (586, 432, 16640),
+        ("dma3", 128, "split", "bn192"): (65, 8544, 13312), ("dma3", 128, "split"): (321, 4272, 13824),
+        ("dma3", 128, "whole", "bn128", "deep"): (194, 12416, 640), ("dma3", 128, "whole", "bn192"): (194, 16528, 128),
+        ("dma3", 128, "whole"): (196, 24704, 128), ("dma3", 160, "split", "bn128", "deep"): (134, 3608, 12544),
+        ("dma3", 160, "split", "bn192"): (313, 5480, 18432), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
+        ("dma3", 160, "whole", "bn192"): (289, 16408, 128), ("dma3", 192, "split", "bn128"): (2794, 400, 14208),
+        ("dma3", 192, "whole", "bn128"): (161, 24608, 128), ("dma3", 256, "split", "bn128"): (211, 8312, 17664),
+        ("dma3", 256, "whole", "bn128"): (4677, 1544, 128), ("dma3", 64, "split", "bn128", "deep"): (290, 216, 17536),
+        ("dma3", 64, "split", "bn192", "deep"): (331, 576, 18048), ("dma3", 64, "split"): (17, 17024, 8320),
+        ("dma3", 64, "whole", "bn128", "deep"): (194, 616, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
+        ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128), ("dma3", 64, "whole"): (17, 57344, 512),
+        ("dma3", 96, "split", "bn128", "deep"): (69, 1920, 17408), ("dma3", 96, "split", "bn192", "deep"): (902, 544, 18432),
+        ("dma3", 96, "split"): (263, 4136, 16640), ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512),
+        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (261, 16488, 128),
+        ("generic", 128, "aligned", "split"): (65, 25352, 912), ("generic", 128, "aligned", "whole"): (708, 2816, 16),
+        ("generic", 16, "aligned", "split"): (1, 8, 1024), ("generic", 16, "aligned", "whole"): (1, 8, 128),
+        ("generic", 256, "aligned", "split"): (1052, 6688, 928), ("generic", 32, "aligned", "split"): (17, 9656, 10480),
+        ("generic", 32, "aligned", "whole"): (26, 50944, 16), ("generic", 64, "aligned", "split"): (33, 6016, 16688),
+        ("generic", 64, "aligned", "whole"): (34, 33648, 16), ("pingpong", "kfull"): (193, 49640, 128),
+        ("pingpong", "ktail"): (1555, 9984, 16), ("pipelined", "ktail"): (1094, 6576, 16),
+        ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 16, "ktail"): (1, 8, 16),
+        ("wavesplit_tile", 16, 32, "kfull"): (129, 456, 128), ("wavesplit_tile", 16, 32, "ktail"): (100, 592, 16),
+        ("wavesplit_tile", 16, 64, "kfull"): (33, 4104, 384), ("wavesplit_tile", 16, 64, "ktail"): (172, 1352, 16),
+        ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128), ("wavesplit_tile", 32, 16, "ktail"): (85, 712, 16),
+        ("wavesplit_tile", 32, 32, "kfull"): (50, 2104, 384), ("wavesplit_tile", 32, 32, "ktail"): (100, 1408, 16),
+        ("wavesplit_tile", 32, 64, "kfull"): (17, 8320, 768), ("wavesplit_tile", 32, 64, "ktail"): (195, 1664, 16),
+        ("wavesplit_tile", 48, 16, "kfull"): (193, 616, 256), ("wavesplit_tile", 48, 16, "ktail"): (162, 768, 16),
+        ("wavesplit_tile", 48, 32, "kfull"): (903, 272, 512), ("wavesplit_tile", 48, 32, "ktail"): (199, 1224, 16),
+        ("wavesplit_tile", 64, 32, "kfull"): (53, 4240, 896), ("wavesplit_tile", 64, 32, "ktail"): (248, 1432, 16),
+        ("wavesplit_tile", 64, 64, "kfull"): (1816, 264, 2176), ("wavesplit_tile", 64, 64, "ktail"): (323, 1536, 16),
+    },
+    "int8": {
+        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round"): (1, 16, 128),
+        ("decode_wavesplit", "w4", "rounds"): (1, 7936, 17664), ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (69, 2816, 15360),
+        ("dma3", 128, "split", "bn192"): (198, 5448, 12288), ("dma3", 128, "split"): (329, 4352, 18560),
+        ("dma3", 128, "whole", "bn128", "deep"): (194, 12416, 640), ("dma3", 128, "whole", "bn192"): (194, 16528, 128),
+        ("dma3", 128, "whole"): (1295, 10760, 128), ("dma3", 160, "split", "bn128", "deep"): (134, 3608, 12544),
+        ("dma3", 160, "split", "bn192"): (313, 5480, 18432), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
+        ("dma3", 160, "whole", "bn192"): (289, 16408, 128), ("dma3", 192, "split", "bn128"): (2794, 400, 14208),
+        ("dma3", 192, "whole", "bn128"): (484, 8344, 128), ("dma3", 256, "split", "bn128"): (208, 8568, 16512),
+        ("dma3", 256, "whole", "bn128"): (4677, 1544, 128), ("dma3", 64, "split", "bn128", "deep"): (290, 216, 17536),
+        ("dma3", 64, "split", "bn192", "deep"): (421, 912, 16128), ("dma3", 64, "split"): (17, 5848, 17408),
+        ("dma3", 64, "whole", "bn128", "deep"): (194, 616, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
+        ("dma3", 64, "whole", "bn192", "deep"): (17, 33280, 512), ("dma3", 64, "whole"): (12, 33096, 128),
+        ("dma3", 96, "split", "bn128", "deep"): (70, 1904, 17536), ("dma3", 96, "split", "bn192", "deep"): (902, 544, 18432),
+        ("dma3", 96, "split"): (263, 4136, 16640), ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512),
+        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (389, 10904, 128),
+        ("generic", 128, "aligned", "split"): (65, 25352, 912), ("generic", 128, "aligned", "whole"): (708, 2816, 16),
+        ("generic", 16, "aligned", "split"): (1, 8, 1024), ("generic", 16, "aligned", "whole"): (1, 8, 128),
+        ("generic", 256, "aligned", "split"): (1052, 6688, 928), ("generic", 256, "aligned", "whole"): (1094, 6576, 16),
+        ("generic", 32, "aligned", "split"): (17, 9656, 10480), ("generic", 32, "aligned", "whole"): (26, 50944, 16),
+        ("generic", 64, "aligned", "split"): (33, 6016, 16688), ("generic", 64, "aligned", "whole"): (34, 33648, 16),
+        ("pingpong", "kfull"): (223, 49272, 128), ("pingpong128", "whole"): (196, 24704, 128),
+        ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 16, "ktail"): (1, 8, 16),
+        ("wavesplit_tile", 16, 32, "kfull"): (129, 456, 128), ("wavesplit_tile", 16, 32, "ktail"): (100, 592, 16),
+        ("wavesplit_tile", 16, 64, "kfull"): (33, 4104, 384), ("wavesplit_tile", 16, 64, "ktail"): (172, 1352, 16),
+        ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128), ("wavesplit_tile", 32, 16, "ktail"): (85, 712, 16),
+        ("wavesplit_tile", 32, 32, "kfull"): (50, 2104, 384), ("wavesplit_tile", 32, 32, "ktail"): (100, 1408, 16),
+        ("wavesplit_tile", 32, 64, "kfull"): (17, 8320, 768), ("wavesplit_tile", 32, 64, "ktail"): (195, 1664, 16),
+        ("wavesplit_tile", 48, 16, "kfull"): (193, 616, 256), ("wavesplit_tile", 48, 16, "ktail"): (162, 768, 16),
+        ("wavesplit_tile", 48, 32, "kfull"): (903, 272, 512), ("wavesplit_tile", 48, 32, "ktail"): (199, 1224, 16),
+        ("wavesplit_tile", 64, 32, "kfull"): (53, 4240, 896), ("wavesplit_tile", 64, 32, "ktail"): (248, 1432, 16),
+        ("wavesplit_tile", 64, 64, "kfull"): (1816, 264, 2176), ("wavesplit_tile", 64, 64, "ktail"): (323, 1536, 16),
+    },
 }
+FP8_REQUIRED_VARIANTS = set(VARIANT_SHAPES["fp8"])
+INT8_REQUIRED_VARIANTS = set(VARIANT_SHAPES["int8"])
+
+# The mid-M tiles run a ring of LDS stages over the K blocks: (M, N) at which K alone does not move an unsplit tile away for every
+# remainder of the K blocks over its stages.  (tile, stages) -> (M, N)
+MID_TILE_SWEEPS = {
+    "fp8": {(64, 128, 3): (97, 24584), (64, 128, 6): (33, 8392), (64, 192, 4): (17, 32816), (64, 256, 3): (129, 13232), (96, 128, 5): (65, 24744), (96, 192, 4): (67, 32824), (96, 256, 3): (258, 16632), (128, 128, 4): (97, 24584), (128, 192, 3): (97, 33024), (128, 256, 3): (290, 16848), (160, 128, 4): (132, 25544), (160, 192, 3): (131, 33032), (192, 128, 3): (322, 12296), (256, 128, 3): (652, 10768)},
+    "fp8_scaled": {(64, 128, 3): (65, 16520), (64, 128, 6): (49, 4232), (64, 192, 4): (17, 32816), (64, 256, 3): (129, 18672), (96, 128, 5): (65, 18584), (96, 192, 4): (67, 32824), (96, 256, 3): (258, 16632), (128, 128, 4): (97, 24584), (128, 192, 3): (97, 33024), (128, 256, 3): (195, 25208), (160, 128, 4): (132, 25544), (160, 192, 3): (131, 33032), (192, 128, 3): (165, 24840), (256, 128, 3): (1163, 6432)},
+    "int8": {(64, 128, 3): (17, 32816), (64, 128, 6): (49, 4232), (64, 192, 4): (17, 32816), (64, 256, 3): (17, 36832), (96, 128, 5): (65, 18584), (96, 192, 4): (67, 32824), (96, 256, 3): (258, 16632), (128, 128, 4): (97, 24584), (128, 192, 3): (97, 33024), (128, 256, 3): (1312, 10760), (160, 128, 4): (132, 25544), (160, 192, 3): (131, 33032), (192, 128, 3): (322, 12296), (256, 128, 3): (1163, 6432)},
+}
+
+# ---- what the one-call linears do: (quantizer, kernel, channel tile of a fused or wave-split kernel, waves or channel groups, K split),
+# with a shape that reaches it; where a kind is not named, all of "block", "ue8m0", "token_fp8" and "int8" do it there
+LINEAR_SHAPES = [(1, 128, 128), (15, 128, 1408), (8, 34176, 1536), (2, 18432, 7424), (1, 16, 1024), (1, 29104, 3456), (3, 6400, 1024), (3, 28288, 3584),
+                 (13, 25728, 1280), (2, 22400, 6784), (13, 33024, 1152), (2, 33216, 7168), (13, 49536, 1152), (1, 16, 2176), (2, 4144, 2176),
+                 (9, 8320, 1024), (1, 16, 128), (4, 12528, 8064), (3, 6720, 128), (3, 13760, 7424), (16, 16, 2688), (16, 4336, 2688),
+                 (15, 8336, 2816), (1, 8320, 128), (15, 16, 1280), (12, 16896, 128), (5, 4864, 28800), (3, 14208, 7168), (9, 128, 1152), (17, 16, 128),
+                 (1, 8, 128), (1, 8, 1024), (1, 66304, 128)]
+
+
+def linear_variant_of(plan: dict, M: int):
+    if M > 16:
+        return (plan["quantizer"], "above decode sizes")
+    k, fused = plan["kernel"], plan["quantizer"] == "fused"
+    return (plan["quantizer"], k, plan["bn"] if fused or k in ("wavesplit_tile", "decode_wavesplit") else 0,
+            min(3, plan["groups_per_wg"]) if k == "decode" else plan["groups_per_wg"], plan["splits"] > 1)
+
 
 # ---- the benchmark configurations at full size: name -> (K, N)
 DSV3_MLP = {"gate_up": (7168, 36864), "down": (18432, 7168)}
@@ -120,6 +257,9 @@ INT8_CONFIG = [(M, N, K) for M in (1, 256, 4096) for (K, N) in LLAMA3_8B.values(
 
 
 def variant_of(plan: dict, K: int):
+    """What a plan runs, as a key; "unpacked": behind the launch that expands packed exponents to fp32 scales."""
+    if plan.get("exponents") == "unpacked":
+        return variant_of({**plan, "exponents": "mfma"}, K) + ("unpacked",)
     k = plan["kernel"]
     sp = "split" if plan["splits"] > 1 else "whole"
     if k == "decode":
@@ -129,6 +269,8 @@ def variant_of(plan: dict, K: int):
         waves = plan["groups_per_wg"]
         key = (k, f"w{waves}", "rounds" if -(-K // 128) > 4 * waves else "one_round")
         return key + ("two_tiles",) if plan["bn"] == 32 else key  # 32 channels per workgroup (FP8) or 16
+    if k == "wavesplit_tile":
+        return (k, plan["bm"], plan["bn"], "kfull" if K % 128 == 0 else "ktail")
     if k == "pingpong128":
         return (k, sp)
     if k == "dma3":  # "deep": more than three LDS stages (small tiles when every workgroup has a CU to itself, FP8)

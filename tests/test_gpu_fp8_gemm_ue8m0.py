@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from fp8_tolerance import check_fp8_gemm
+from gemm_cases import VARIANT_SHAPES, variant_of
 from sglang_amd.workloads import make_activation, make_fp8_weight
 
 pytestmark = pytest.mark.gpu
@@ -61,7 +62,7 @@ def test_ue8m0_gemm_against_oracle(gpu, oracle, M, N, K):
     from sglang_amd import _lib
     from sglang_amd.fp8_kernel import w8a8_block_fp8_matmul_deepgemm
 
-    print(f"case M={M} N={N} K={K} -> {_lib.gemm_plan('fp8', M, N, K)['kernel']}", flush=True)
+    print(f"case M={M} N={N} K={K} -> {_lib.gemm_plan('fp8_ue8m0', M, N, K)['kernel']}", flush=True)
     x_q, sa_words, w2, sb_words = _operands(M, N, K, gpu, 3 * M + N + K)
     out = w8a8_block_fp8_matmul_deepgemm(x_q, w2, sa_words, sb_words, [128, 128], torch.bfloat16)
     assert tuple(out.shape) == (M, N) and out.dtype == torch.bfloat16
@@ -100,12 +101,14 @@ def test_ue8m0_gemm_exact_integers(gpu, oracle, M, N, K):
     assert torch.equal(out.cpu().view(torch.int16), ref.view(torch.int16))
 
 
-# one shape per tile (64 / 128 tokens x 128 / 192 / 256 channels) and split of the mid-M kernel, which applies the exponents
-# in the MFMA too; 50 x 3000 has a ragged last channel tile, 33 x 16384 x 2176 a last exponent word with one byte used
+# every tile and split of the mid-M kernel, which applies the exponents in the MFMA too, and wave-split tiles at the same sizes; 50 x 3000 has a ragged last channel tile, 33 x 16384 x 2176 a last exponent word with one byte used
 MID_M = [(48, 16384, 2048), (33, 16384, 2176), (40, 4096, 7168), (50, 3000, 4224), (24, 36864, 14336), (130, 3072, 7168), (40, 65536, 512),
          (130, 4096, 7168), (100, 32768, 640), (65, 7168, 18432), (100, 36864, 640), (300, 3072, 14336), (100, 65536, 512),
          (400, 4096, 16384),
          (14, 36864, 1280), (16, 65536, 1152), (8, 36864, 7168), (16, 24576, 1536)]  # decode sizes on one round of unsplit 64-token tiles
+
+
+MID_M += [s for v, s in VARIANT_SHAPES["fp8_ue8m0"].items() if v[0] == "dma3" and s not in MID_M]
 
 
 def test_mid_m_shapes_reach_every_tile_and_split():
@@ -113,10 +116,10 @@ def test_mid_m_shapes_reach_every_tile_and_split():
 
     reached = set()
     for M, N, K in MID_M:
-        p = _lib.gemm_plan("fp8", M, N, K)
-        assert p["kernel"] == "dma3", (M, N, K, p)
-        reached.add((p["bm"], p["bn"], p["splits"] > 1))
-    assert reached == {(bm, bn, sp) for bm in (64, 128) for bn in (128, 192, 256) for sp in (False, True)}
+        p = _lib.gemm_plan("fp8_ue8m0", M, N, K)
+        assert p["kernel"] in ("dma3", "wavesplit_tile") and p["exponents"] == "mfma", (M, N, K, p)
+        reached.add(variant_of(p, K))
+    assert reached >= {v for v in VARIANT_SHAPES["fp8_ue8m0"] if v[0] == "dma3"}
 
 
 @pytest.mark.parametrize("M,N,K", MID_M)
@@ -133,14 +136,14 @@ def test_ue8m0_mid_m_kernel_against_oracle(gpu, oracle, M, N, K):
 
 # the streaming decode kernel: one K range and several, the last range short (K blocks not a multiple of 8), one to four
 # bytes used in the last exponent word, token counts below and at the 16 rows of the MFMA tile (rows past M repeat the last token)
-DECODE = [(8, 256, 512), (4, 4352, 512), (5, 4096, 36864), (16, 4096, 36864), (13, 18432, 7168), (15, 18432, 7168), (9, 3072, 1536),
-          (14, 70656, 1280), (14, 16384, 2304), (15, 65536, 640), (16, 66560, 1152), (13, 4096, 18432), (8, 4352, 128)]
+DECODE = [(8, 256, 512), (4, 4352, 512), (5, 4096, 36864), (16, 4096, 36864), (13, 19584, 7168), (12, 6016, 23296), (9, 3072, 1536),
+          (14, 70656, 1280), (15, 128, 1408), (15, 65536, 640), (16, 66560, 1152), (13, 3968, 35328), (8, 4352, 128)]
 
 
 def test_decode_shapes_reach_the_streaming_kernel():
     from sglang_amd import _lib
 
-    plans = [_lib.gemm_plan("fp8", M, N, K) for M, N, K in DECODE]
+    plans = [_lib.gemm_plan("fp8_ue8m0", M, N, K) for M, N, K in DECODE]
     assert all(p["kernel"] == "decode" for p in plans), plans
     assert {p["splits"] > 1 for p in plans} == {False, True}
 
@@ -187,11 +190,11 @@ def test_ue8m0_mid_m_exact_integers(gpu, oracle, M, N, K):
     _exact_integer_case(gpu, oracle, M, N, K)  # split and unsplit mid-M plans
 
 
-@pytest.mark.parametrize("M,N,K", [(8, 4352, 512), (13, 18432, 7168), (16, 2048, 7168), (14, 16384, 2304), (5, 4096, 36864)])
+@pytest.mark.parametrize("M,N,K", [(8, 4352, 512), (13, 19584, 7168), (16, 3072, 1536), (14, 128, 2048), (5, 4096, 36864)])
 def test_ue8m0_decode_exact_integers(gpu, oracle, M, N, K):
     from sglang_amd import _lib
 
-    assert _lib.gemm_plan("fp8", M, N, K)["kernel"] == "decode"
+    assert _lib.gemm_plan("fp8_ue8m0", M, N, K)["kernel"] == "decode"
     _exact_integer_case(gpu, oracle, M, N, K)
 
 

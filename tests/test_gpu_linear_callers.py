@@ -131,34 +131,39 @@ def test_fused_block_fp8_linear(gpu, oracle, shape, N, K, with_bias):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K", [(1, 2048, 7168), (12, 2048, 7168), (14, 16640, 4480), (8, 4096, 18432), (16, 512, 512), (5, 66048, 512),
-                                   (9, 256, 128), (4, 7168, 18432), (16, 7168, 2048),
-                                   (16, 24576, 1536), (5, 36864, 5760), (13, 53248, 1152), (16, 32768, 1152), (13, 45056, 1280),
-                                   (2, 36864, 5760), (3, 24576, 5120), (8, 36800, 5760)])
-def test_decode_linear_quantizes_in_the_gemm_kernel(gpu, oracle, M, N, K, dtype):
-    """At decode sizes the one-call linear has no quantizer launch: the streaming decode kernel quantizes the tokens of
-    each K range in its prologue.  Same arithmetic on the same codes and scales as quantizer + GEMM in two steps, so where
-    the two-step GEMM takes the same kernel the outputs must be identical bit for bit (split and unsplit plans, several
-    channel groups per workgroup, a short last K range, rows past M).  Where the two-step GEMM takes the wave-split decode
-    kernel instead (M = 1 here) the sums are added in another order and both are held to the oracle.  The last two shapes
-    (K of 144 blocks; K of 16 blocks with 16 tokens) are ones where the one-call linear itself launches the quantizer and
-    the wave-split kernel, being faster there: identical to the two steps again.  The five after them take the mid-M kernel on
-    one round of unsplit 64-token tiles (128-, 192- and 256-channel tiles: six, four and three stages; K of 12, 45, 9, 9 and
-    10 blocks), whose producer waves quantize the tokens: identical to quantizer + that kernel; the last two take it for the linear only
-    (fewer tokens than the GEMM's own threshold; K of five ranges for the streaming kernel)."""
+@pytest.mark.parametrize("M,N,K,quantizer,kernel,gemm", [
+    # the streaming kernel's prologue: K whole and split, one, two and more channel groups per workgroup, a short last K range
+    (16, 512, 512, "fused", "decode", "decode"), (5, 66048, 512, "fused", "decode", "decode"), (9, 256, 128, "fused", "decode", "decode"),
+    (15, 128, 1408, "fused", "decode", "decode"), (8, 34176, 1536, "fused", "decode", "decode_wavesplit"),
+    (2, 18432, 7424, "fused", "decode", "decode_wavesplit"),
+    # a quantizer launch in front of the wave-split kernels
+    (3, 13760, 7424, "launch", "decode_wavesplit", "decode_wavesplit"), (4, 7168, 18432, "launch", "wavesplit_tile", "wavesplit_tile"),
+    (12, 2048, 7168, "launch", "wavesplit_tile", "wavesplit_tile"),
+    # the wave-split kernels' own quantizers
+    (1, 2048, 7168, "fused", "wavesplit_tile", "wavesplit_tile"), (16, 7168, 2048, "fused", "wavesplit_tile", "wavesplit_tile"),
+    (1, 36864, 7168, "fused", "decode_wavesplit", "decode_wavesplit"),
+    # the mid-M kernel's producer waves: 128-, 192- and 256-channel tiles (six, four and three stages), K of 12, 9, 9, 10 and 56 blocks,
+    # the last with a ragged last channel tile
+    (16, 24576, 1536, "fused", "dma3", "dma3"), (13, 53248, 1152, "fused", "dma3", "dma3"), (16, 32768, 1152, "fused", "dma3", "dma3"),
+    (13, 45056, 1280, "fused", "dma3", "dma3"), (8, 36800, 7168, "fused", "dma3", "dma3"),
+    # ... for the linear only: fewer tokens than the GEMM's own threshold; K of many ranges for the streaming kernel
+    (2, 36864, 7168, "fused", "dma3", "decode_wavesplit"), (3, 22400, 6784, "fused", "dma3", "decode_wavesplit")])
+def test_decode_linear_quantizes_in_the_gemm_kernel(gpu, oracle, M, N, K, quantizer, kernel, gemm, dtype):
+    """At decode sizes the one-call linear has no quantizer launch where that is the faster way: the streaming and the
+    wave-split kernels quantize the tokens in their prologues, the mid-M kernel by producer waves.  Same arithmetic on the same
+    codes and scales as quantizer + GEMM in two steps, so where the two-step GEMM takes the same kernel the outputs must be
+    identical bit for bit (split and unsplit plans, several channel groups per workgroup, a short last K range, rows past M); where
+    it takes another one the sums are added in another order and both are held to the oracle."""
     from sglang_amd import _lib
     from sglang_amd.fp8_kernel import per_token_group_quant_fp8
+    from sglang_amd.fp8_utils import _one_call_takes_the_same_gemm
     from sglang_amd.fp8_utils import fused_w8a8_block_fp8_linear as w8a8_block_fp8_linear
     from sglang_amd.sgl_kernel import fp8_blockwise_scaled_mm
 
-    kernel = _lib.gemm_plan("fp8", M, N, K)["kernel"]
-    two_launches = (M, N, K) in ((4, 7168, 18432), (16, 7168, 2048))
-    producer = (M, N, K) in ((16, 24576, 1536), (5, 36864, 5760), (13, 53248, 1152), (16, 32768, 1152), (13, 45056, 1280),
-                            (8, 36800, 5760))  # (the last with a ragged last channel tile: 128 of 192 channels)
-    linear_only = (M, N, K) in ((2, 36864, 5760), (3, 24576, 5120))  # the GEMM alone takes the wave-split kernel, the linear the producers
-    assert kernel == ("dma3" if producer else "decode_wavesplit" if M == 1 or two_launches or linear_only else "decode")
     lin = _lib.block_linear_plan(M, N, K)
-    assert (lin["quantizer"], lin["kernel"]) == (("fused", "dma3") if producer or linear_only else ("launch", "decode_wavesplit") if two_launches else ("fused", "decode"))
+    print(f"case M={M} N={N} K={K} {dtype} {lin}", flush=True)
+    assert (lin["quantizer"], lin["kernel"], _lib.gemm_plan("fp8", M, N, K)["kernel"]) == (quantizer, kernel, gemm)
+    assert _one_call_takes_the_same_gemm(M, N, K) == (kernel == gemm)
     x = make_activation(M, K, seed=M + N, dtype=dtype)
     x[0, :128] = 0  # a group of zeros: scale 1e-10 / 448, codes 0
     w_q, w_s = make_fp8_weight(N, K, seed=K)
@@ -172,7 +177,7 @@ def test_decode_linear_quantizes_in_the_gemm_kernel(gpu, oracle, M, N, K, dtype)
 
         two_step = w8a8_block_fp8_matmul(q, wg, s, sg, [128, 128], dtype)
     assert fused.dtype == dtype
-    if kernel in ("decode", "dma3") or two_launches:
+    if kernel == gemm:
         assert torch.equal(fused.view(torch.int16), two_step.view(torch.int16))
     xq, xs = oracle.group_quant(x, 128, mode="div")
     ref, mag = oracle.fp8_blockwise_mm(xq, w_q, xs, w_s, torch.float32, want_abs=True)
@@ -181,7 +186,7 @@ def test_decode_linear_quantizes_in_the_gemm_kernel(gpu, oracle, M, N, K, dtype)
 
 
 @pytest.mark.parametrize("M,N,K", [(16, 53248, 1280), (16, 53248, 1408), (16, 45056, 1408), (16, 32768, 1664), (16, 32768, 1792),
-                                   (16, 32768, 2176)])
+                                   (16, 32768, 1408)])
 def test_producer_wave_linear_every_tail_length(gpu, M, N, K):
     """The producer waves and the other waves of the mid-M kernel must meet at the same number of barriers whatever is left of K
     after whole trips over the stages: three stages with 1 and 2 blocks left, four with 3, six with 1, 2 and 5 (0 and the other

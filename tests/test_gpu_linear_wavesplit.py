@@ -1,10 +1,11 @@
-"""One-call linears whose wave-split decode kernel quantizes the tokens itself: at the steps of the pieces a thread quantizes
+"""One-call linears whose wave-split kernels quantize the tokens themselves: at the steps of the pieces a thread quantizes
 (2, 4, 10), four and eight waves, one and two channel tiles, K blocks that do not fill the waves' turns, and just past the
-limit, where a quantizer launch stands in front of the GEMM again."""
+limit, where a quantizer launch stands in front of the GEMM again; and every other thing the four linears do (gemm_cases)."""
 import pytest
 import torch
 
 from fp8_tolerance import check_fp8_gemm
+from gemm_cases import LINEAR_SHAPES
 from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
 
 pytestmark = pytest.mark.gpu
@@ -14,16 +15,15 @@ SHAPES = [(1, 4096, 1152), (8, 144, 2048), (16, 4096, 1152), (2, 576, 4096), (3,
           (10, 6144, 4096), (11, 512, 4096), (1, 512, 8320), (1, 272, 20480), (2, 40960, 4096), (5, 576, 7168)]
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("M,N,K", SHAPES + [s for s in LINEAR_SHAPES if s not in SHAPES])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fused_quantizer_of_the_wavesplit_kernel(gpu, oracle, M, N, K, dtype):
     from sglang_amd import _lib, ops
     from sglang_amd.fp8_kernel import per_token_group_quant_fp8, sglang_per_token_group_quant_fp8, sglang_per_token_quant_fp8, w8a8_block_fp8_matmul
-    from sglang_amd.fp8_utils import requant_weight_ue8m0
+    from sglang_amd.fp8_utils import _one_call_takes_the_same_gemm, requant_weight_ue8m0
     from sglang_amd.int8_kernel import per_token_quant_int8
 
-    plan = _lib.block_linear_plan(M, N, K)
-    print(f"case M={M} N={N} K={K} {plan}", flush=True)
+    print(f"case M={M} N={N} K={K} {[_lib.linear_plan(k, M, N, K) for k in ('block', 'ue8m0', 'token_fp8', 'int8')]}", flush=True)
     bits = lambda t: t.view(torch.int16)
     x = make_activation(M, K, seed=M + N, dtype=dtype)
     x[0, :128] = 0
@@ -37,7 +37,7 @@ def test_fused_quantizer_of_the_wavesplit_kernel(gpu, oracle, M, N, K, dtype):
         out = ops.block_fp8_linear(xg, wg, sg, None, dtype, by_reciprocal=by_reciprocal)
         q, s = per_token_group_quant_fp8(xg, 128, column_major_scales=not by_reciprocal)
         two = w8a8_block_fp8_matmul(q, wg, s, sg, [128, 128], dtype)
-        if "wavesplit_waves" in plan and _lib.gemm_plan("fp8", M, N, K)["kernel"] == "decode_wavesplit":
+        if _one_call_takes_the_same_gemm(M, N, K):
             assert torch.equal(bits(out), bits(two))
         if N <= 1040:
             xq, xs = oracle.group_quant(x, 128, mode="rcp" if by_reciprocal else "div")

@@ -44,7 +44,7 @@ def test_every_tile_exact(gpu, shape, fp8_tile, int8_tile):
         plan = _lib.gemm_plan(kind, M, N, K)
         print(f"case {kind} {shape} {plan}", flush=True)
         if tile is not None:
-            assert (plan["run_bm"], plan["run_bn"]) == tile
+            assert (plan["bm"], plan["bn"]) == tile
     g = torch.Generator().manual_seed(M + N + K)
     a, w = torch.randint(-2, 3, (M, K), generator=g), torch.randint(-2, 3, (N, K), generator=g)
     a8, w8 = a.float().to(FP8).to(gpu), w.float().to(FP8).to(gpu)
