@@ -557,7 +557,7 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
   if (K % KSTEP != 0) {
     if (kind == GK_UNIT || kind == GK_INT8) c = choose_ragged_tile(M, N, K);
   } else if (M <= 16) {
-    c = choose_decode_tile(kind, M, N, K);
+    c = choose_decode_tile(kind, M, N, K, r.kernel == RK_DMA3, r.kernel == RK_WAVESPLIT);
   } else {
     TileChoice base{TF_NONE, r.bm, r.bn, r.splits, 0.0};
     if (r.kernel == RK_DMA3 || (r.kernel == RK_PP128 && r.splits == 1)) base.family = TF_DMA;
@@ -764,8 +764,9 @@ std::vector<std::string> tile_constant_names() {
                 "ws_result", "ws_norm"});
   }
   add("limits.", {"margin", "two_phase_margin", "large_weight_margin", "large_weight_max_tokens", "mid_wavesplit_max_weight", "ragged_max_weight",
-                  "ragged_max_factor", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
-                  "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
+                  "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
+                  "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
+                  "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
                   "decode_short_max_weight", "decode_short_min_tokens"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;

@@ -42,7 +42,9 @@ static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above 
 struct TileLimits {
   double margin = 0.95, two_phase_margin = 0.90, large_weight_margin = 0.85, large_weight_max_tokens = 64.0;
   double mid_wavesplit_max_weight = 100e6, ragged_max_weight = 100e6, ragged_max_factor = 2.0;
+  double wavesplit_max_tokens_bytes = 16e6, wavesplit_long_k = 9216.0, wavesplit_long_k_max_tokens_bytes = 10e6, few_workgroups_max_tokens = 128.0;
   double decode_min_kblocks = 16.0, decode_padded_max_weight = 400e6, decode_max_weight = 140e6, decode_few_tokens_max_weight = 100e6;
+  double decode_one_turn_min_kblocks = 30.0, decode_one_turn_kblocks = 32.0, decode_one_turn_max_channels = 16384.0, decode_one_turn_max_tokens = 10.0;
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
 };
@@ -134,7 +136,13 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
   const TileTimes& t = tile_times(kind);
   TileChoice best = best_dma_tile(t, M, N, K);
   const TileLimits& l = tile_model().limits;
-  if ((double)(N * K) <= l.mid_wavesplit_max_weight) {  // (a larger weight streams better through the wide tiles: K = 4096 -> N = 28672 at 48 tokens 27.2 against 33.6 us)
+  // The wave-split tile: a large weight streams better through the wide tiles (K = 4096 -> N = 28672 at 48 tokens 27.2 against
+  // 33.6 us), and so does a large token matrix, which leaves the XCDs' L2s and is fetched again by every channel tile (mid-M / wave-split:
+  // K = 10368 -> N = 704 at 2616 tokens 37.4 / 53.2, 10496 -> 960 at 1610 34.7 / 44.7, per-token FP8 7168 -> 384 at 2595 19.3 / 22.3;
+  // but 7168 -> 576 at 1608 23.1 / 20.3).
+  const double token_bytes = (double)(M * K);
+  const bool tokens_fit = token_bytes <= l.wavesplit_max_tokens_bytes && ((double)K <= l.wavesplit_long_k || token_bytes <= l.wavesplit_long_k_max_tokens_bytes);
+  if ((double)(N * K) <= l.mid_wavesplit_max_weight && tokens_fit) {
     const TileChoice ws = best_wavesplit_tile(t, M, N, K);
     if (ws.us < best.us) best = ws;
   }
@@ -147,9 +155,14 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
   if (base.family == TF_DMA)
     for (int i = 0; i < 13; ++i)
       if (MID_TILES[i].bm == base.bm && MID_TILES[i].bn == base.bn) base_us = dma_tile_us(t, i, M, N, K, base.splits);
-  // (bound by a large weight's stream, the model knows little of how many CUs it takes: K = 10880 -> N = 16896 at 36 tokens, 132
-  // unsplit tiles instead of 198 split ones, 54.8 against 48.3 us)
-  const bool large = (double)M <= l.large_weight_max_tokens && (double)(N * K) > l.mid_wavesplit_max_weight;
+  // Bound by a large weight's stream, the model knows little of how many CUs it takes: K = 10880 -> N = 16896 at 36 tokens, 132
+  // unsplit tiles instead of 198 split ones, 54.8 against 48.3 us.  From 65 tokens on the tile with more workgroups wins (14592 ->
+  // 17920 at 71 tokens, 140 / 210 workgroups 81.0 / 62.6; per-token FP8 17664 -> 19072 at 103, 149 / 225, 96 / 77; but 10624 -> 9792 at
+  // 65, 231 / 154, 28.7 / 39.2): of 24 shapes 22 by 4 to 30 %.
+  const bool large_weight = (double)(N * K) > l.mid_wavesplit_max_weight, large = (double)M <= l.large_weight_max_tokens && large_weight;
+  if (large_weight && !large && (double)M <= l.few_workgroups_max_tokens && base.family == TF_DMA &&
+      ceil_div(M, best.bm) * ceil_div(N, best.bn) * best.splits <= ceil_div(M, base.bm) * ceil_div(N, base.bn) * base.splits)
+    return TileChoice{TF_NONE, 0, 0, 1, 0.0};
   const double margin = base.family == TF_TWO_PHASE ? l.two_phase_margin : large ? l.large_weight_margin : l.margin;
   return best.us < margin * base_us ? best : TileChoice{TF_NONE, 0, 0, 1, 0.0};
 }
@@ -164,21 +177,36 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
   return (double)(N * K) <= l.ragged_max_weight && ws.us < l.ragged_max_factor * best_dma_tile(t, M, N, K).us ? ws : TileChoice{TF_NONE, 0, 0, 1, 0.0};
 }
 
-// Up to 16 tokens: the wave-split tile against the streaming and the register wave-split kernel.  It wins wherever K has more
-// than 16 blocks and the weight is not one of the largest (us, the other / the tile, one token and 16; FP8):
+// Up to 16 tokens: the wave-split tile against the kernel the constants table names.  It wins over the streaming and the register
+// wave-split kernel wherever K has more than 16 blocks and the weight is not one of the largest (us, the other / the tile, one
+// token and 16; FP8):
 //   K = 7168: N = 576 6.8/5.1, 9.4/5.6;  2048 6.9/5.2, 8.8/6.5;  K = 14336: N = 512 9.9/6.8, 8.0/6.8;  K = 5120: N = 10240 16.0/10.2, 13.9/10.5
 //   K = 18432: N = 896 12.4/7.7, 11.6/9.4;  7168 23.3/23.1, 28.1/25.0;  K = 4096: N = 6144 7.5/6.3, 9.7/6.2;  28672 22.9/24.7, 26.1/25.5
 // because its operands come in whole 128-byte lines: 16 rows x 64 bytes per instruction, which is what the MFMA's layout asks
 // for when loaded straight into registers, pass through a CU's cache at 16 bytes a cycle, whole lines at 61.
 // With fewer K blocks both are bound by the launch (K = 2048 -> N = 2048 4.3 / 4.4) except where there are many channels
 // (K = 1024 -> N = 12288 5.8/4.8, 8.0/4.9; but 512 -> 32768 5.9/6.8, 1536 -> 24576 9.3/9.6).
-TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+// It does not take over from
+//   * the mid-M kernel, which the table names where one round of unsplit tiles fills the chip (K = 2304 -> N = 36864 at 16 tokens
+//     19.3/22.9, 5120 -> 50688 51.3/57.3, INT8 1024 -> 17408 at 12 tokens 7.1/9.0; over 91 shapes 6 % faster), unless the rows of the weight lie
+//     a multiple of 4096 bytes apart, where that kernel's loads of eight rows collide (4096 -> 30464 31.7/29.5, per-token FP8 32.2/28.4);
+//   * the register wave-split kernel where K fills its one turn of 32 blocks and the channels are more than one round of the widest tile,
+//     up to 10 tokens: 4096 -> 20736 at 1 and 8 19.0/24.4, 21.3/24.4; 3840 -> 24576 at 1 20.0/23.0 (4096 -> 16384 at 1, 8 14.8/16.3,
+//     16.3/16.3; 3584 -> 27392 at 6 23.6/21.8; INT8 4096 -> 28672 at 11 29.8/26.2).
+// The weight limits were drawn at the shapes named beside them.  Measured around them since (K = 2304 .. 18432, 85 to 260 million weights,
+// 1 .. 16 tokens): also beyond them the tile is up to 25 % faster than the streaming and the two-turn register kernel, and slower than
+// the one-turn one; but a linear that leaves those loses their fused quantizers, so the limits stay where the linears were measured.
+TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_mid, bool from_wavesplit) {
   const TileLimits& l = tile_model().limits;
   const int64_t kb = ceil_div(K, KSTEP);
   const double weight = (double)(N * K);
   // (the largest weights: the register kernel's single-tile stream is as fast for few tokens, unless it pads K to whole turns of 32 blocks:
   // K = 5152 -> N = 31936 INT8 at 5 tokens 50.3 us, 39.3 with the tile)
   const bool padded = kb <= 64 && (kb + 31) / 32 * 32 * 4 > kb * 5;
+  if (from_mid && K % 4096 != 0) return TileChoice{TF_NONE, 0, 0, 1, 0.0};
+  const bool one_turn = (double)kb >= l.decode_one_turn_min_kblocks && (double)kb <= l.decode_one_turn_kblocks;
+  if (from_wavesplit && one_turn && (double)M <= l.decode_one_turn_max_tokens && (double)N > l.decode_one_turn_max_channels)
+    return TileChoice{TF_NONE, 0, 0, 1, 0.0};
   const bool few = (double)M <= (kind == GK_F32 ? l.decode_few_tokens_f32 : l.decode_few_tokens) && (double)kb <= l.decode_long_kblocks;
   const double most = padded ? l.decode_padded_max_weight : few ? l.decode_few_tokens_max_weight : l.decode_max_weight;
   const bool take = (double)kb > l.decode_min_kblocks ? weight <= most

@@ -82,33 +82,33 @@ VARIANT_SHAPES = {
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
         ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
-        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 25216, 3968),
-        ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (68, 4256, 13696),
-        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (69, 8272, 17536),
+        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
+        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (2761, 8, 7424),
+        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (67, 8280, 13056),
         ("dma3", 128, "whole", "bn128", "deep"): (4238, 584, 512), ("dma3", 128, "whole", "bn192"): (97, 32896, 128),
-        ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (130, 5736, 7936),
+        ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (2456, 8, 14080),
         ("dma3", 160, "split", "bn192"): (129, 11264, 11648), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
-        ("dma3", 160, "whole", "bn192"): (129, 32896, 128), ("dma3", 192, "split", "bn128"): (3695, 272, 9728),
+        ("dma3", 160, "whole", "bn192"): (129, 32896, 128), ("dma3", 192, "split", "bn128"): (4210, 8, 5504),
         ("dma3", 192, "whole", "bn128"): (484, 8344, 128), ("dma3", 256, "split", "bn128"): (4112, 264, 12800),
-        ("dma3", 256, "whole", "bn128"): (641, 10760, 128), ("dma3", 64, "split", "bn128", "deep"): (33, 2936, 14592),
-        ("dma3", 64, "split", "bn192", "deep"): (17, 11168, 9216), ("dma3", 64, "split"): (97, 2752, 15488),
-        ("dma3", 64, "whole", "bn128", "deep"): (49, 4112, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
-        ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128), ("dma3", 64, "whole"): (129, 12832, 128),
-        ("dma3", 96, "split", "bn128", "deep"): (70, 2176, 18816), ("dma3", 96, "split", "bn192", "deep"): (266, 3656, 8576),
-        ("dma3", 96, "split"): (258, 4096, 10240), ("dma3", 96, "whole", "bn128", "deep"): (66, 25216, 384),
-        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (194, 16518, 128),
-        ("generic", 128, "aligned", "split"): (68, 8, 960), ("generic", 128, "aligned", "whole"): (66, 8, 16),
-        ("generic", 128, "bytes", "split"): (68, 8, 1038), ("generic", 128, "bytes", "whole"): (65, 8, 26),
-        ("generic", 16, "aligned", "split"): (1, 8, 912), ("generic", 16, "aligned", "whole"): (1, 8, 16),
-        ("generic", 16, "bytes", "split"): (1, 8, 907), ("generic", 16, "bytes", "whole"): (1, 8, 17),
-        ("generic", 256, "aligned", "split"): (1052, 6688, 928), ("generic", 256, "bytes", "split"): (1114, 7024, 922),
-        ("generic", 256, "bytes", "whole"): (1025, 6792, 17), ("generic", 32, "aligned", "split"): (17, 8, 960),
-        ("generic", 32, "aligned", "whole"): (17, 8, 32), ("generic", 32, "bytes", "split"): (20, 8, 983),
-        ("generic", 32, "bytes", "whole"): (17, 8, 18), ("generic", 64, "aligned", "split"): (33, 8, 912),
-        ("generic", 64, "aligned", "whole"): (33, 8, 32), ("generic", 64, "bytes", "split"): (39, 8, 941),
-        ("generic", 64, "bytes", "whole"): (33, 8, 18), ("pingpong", "kfull"): (223, 49272, 128),
-        ("pingpong", "ktail"): (1323, 11460, 16), ("pipelined", "ktail"): (1094, 6576, 16),
+        ("dma3", 256, "whole", "bn128"): (641, 10760, 128), ("dma3", 64, "split", "bn128", "deep"): (674, 8, 14848),
+        ("dma3", 64, "split", "bn128"): (1874, 8, 8576), ("dma3", 64, "split", "bn192", "deep"): (722, 264, 14208),
+        ("dma3", 64, "split"): (1832, 200, 10240), ("dma3", 64, "whole", "bn128", "deep"): (49, 4112, 128),
+        ("dma3", 64, "whole", "bn128"): (65, 16472, 128), ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128),
+        ("dma3", 64, "whole"): (129, 12832, 128), ("dma3", 96, "split", "bn128", "deep"): (1618, 8, 9472),
+        ("dma3", 96, "split", "bn192", "deep"): (2893, 272, 8192), ("dma3", 96, "split"): (258, 4096, 10240),
+        ("dma3", 96, "whole", "bn128", "deep"): (66, 25216, 384), ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128),
+        ("dma3", 96, "whole"): (194, 16518, 128), ("generic", 128, "aligned", "split"): (68, 8, 960),
+        ("generic", 128, "aligned", "whole"): (66, 8, 16), ("generic", 128, "bytes", "split"): (68, 8, 1038),
+        ("generic", 128, "bytes", "whole"): (65, 8, 26), ("generic", 16, "aligned", "split"): (1, 8, 912),
+        ("generic", 16, "aligned", "whole"): (1, 8, 16), ("generic", 16, "bytes", "split"): (1, 8, 907),
+        ("generic", 16, "bytes", "whole"): (1, 8, 17), ("generic", 256, "aligned", "split"): (1052, 6688, 928),
+        ("generic", 256, "bytes", "split"): (1114, 7024, 922), ("generic", 256, "bytes", "whole"): (1025, 6792, 17),
+        ("generic", 32, "aligned", "split"): (17, 8, 960), ("generic", 32, "aligned", "whole"): (17, 8, 32),
+        ("generic", 32, "bytes", "split"): (20, 8, 983), ("generic", 32, "bytes", "whole"): (17, 8, 18),
+        ("generic", 64, "aligned", "split"): (33, 8, 912), ("generic", 64, "aligned", "whole"): (33, 8, 32),
+        ("generic", 64, "bytes", "split"): (39, 8, 941), ("generic", 64, "bytes", "whole"): (33, 8, 18),
+        ("pingpong", "kfull"): (223, 49272, 128), ("pingpong", "ktail"): (1323, 11460, 16), ("pipelined", "ktail"): (1094, 6576, 16),
         ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 32, "kfull"): (97, 579, 128),
         ("wavesplit_tile", 16, 64, "kfull"): (65, 2728, 128), ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128),
         ("wavesplit_tile", 32, 32, "kfull"): (49, 2064, 128), ("wavesplit_tile", 32, 64, "kfull"): (49, 4137, 128),
@@ -120,57 +120,58 @@ VARIANT_SHAPES = {
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
         ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
-        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 25216, 3968),
-        ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (68, 4256, 13696),
-        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (69, 8272, 17536),
+        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
+        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (2761, 8, 7424),
+        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (67, 8280, 13056),
         ("dma3", 128, "whole", "bn128", "deep"): (4238, 584, 512), ("dma3", 128, "whole", "bn192"): (97, 32896, 128),
-        ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (130, 5736, 7936),
+        ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (2456, 8, 14080),
         ("dma3", 160, "split", "bn192"): (129, 11264, 11648), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
-        ("dma3", 160, "whole", "bn192"): (129, 32896, 128), ("dma3", 192, "split", "bn128"): (3695, 272, 9728),
+        ("dma3", 160, "whole", "bn192"): (129, 32896, 128), ("dma3", 192, "split", "bn128"): (4210, 8, 5504),
         ("dma3", 192, "whole", "bn128"): (484, 8344, 128), ("dma3", 256, "split", "bn128"): (4112, 264, 12800),
-        ("dma3", 256, "whole", "bn128"): (641, 10760, 128), ("dma3", 64, "split", "bn128", "deep"): (33, 2936, 14592),
-        ("dma3", 64, "split", "bn192", "deep"): (17, 11168, 9216), ("dma3", 64, "split"): (97, 2752, 15488),
-        ("dma3", 64, "whole", "bn128", "deep"): (49, 4112, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
-        ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128), ("dma3", 64, "whole"): (129, 12832, 128),
-        ("dma3", 96, "split", "bn128", "deep"): (70, 2176, 18816), ("dma3", 96, "split", "bn192", "deep"): (266, 3656, 8576),
-        ("dma3", 96, "split"): (258, 4096, 10240), ("dma3", 96, "whole", "bn128", "deep"): (66, 25216, 384),
-        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (194, 16518, 128),
-        ("generic", 16, "aligned", "split", "unpacked"): (1, 8, 1024), ("generic", 16, "aligned", "whole", "unpacked"): (1, 8, 128),
-        ("pingpong", "kfull"): (223, 49272, 128), ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128),
-        ("wavesplit_tile", 16, 32, "kfull"): (97, 579, 128), ("wavesplit_tile", 16, 64, "kfull", "unpacked"): (7, 12824, 7808),
-        ("wavesplit_tile", 16, 64, "kfull"): (65, 2728, 128), ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128),
-        ("wavesplit_tile", 32, 32, "kfull"): (49, 2064, 128), ("wavesplit_tile", 32, 64, "kfull"): (49, 4137, 128),
-        ("wavesplit_tile", 48, 16, "kfull"): (194, 616, 128), ("wavesplit_tile", 48, 32, "kfull"): (193, 1223, 128),
-        ("wavesplit_tile", 64, 32, "kfull"): (49, 4358, 128), ("wavesplit_tile", 64, 64, "kfull"): (1637, 291, 512),
+        ("dma3", 256, "whole", "bn128"): (641, 10760, 128), ("dma3", 64, "split", "bn128", "deep"): (674, 8, 14848),
+        ("dma3", 64, "split", "bn128"): (1874, 8, 8576), ("dma3", 64, "split", "bn192", "deep"): (722, 264, 14208),
+        ("dma3", 64, "split"): (1832, 200, 10240), ("dma3", 64, "whole", "bn128", "deep"): (49, 4112, 128),
+        ("dma3", 64, "whole", "bn128"): (65, 16472, 128), ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128),
+        ("dma3", 64, "whole"): (129, 12832, 128), ("dma3", 96, "split", "bn128", "deep"): (1618, 8, 9472),
+        ("dma3", 96, "split", "bn192", "deep"): (2893, 272, 8192), ("dma3", 96, "split"): (258, 4096, 10240),
+        ("dma3", 96, "whole", "bn128", "deep"): (66, 25216, 384), ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128),
+        ("dma3", 96, "whole"): (194, 16518, 128), ("generic", 16, "aligned", "split", "unpacked"): (1, 8, 1024),
+        ("generic", 16, "aligned", "whole", "unpacked"): (1, 8, 128), ("pingpong", "kfull"): (223, 49272, 128),
+        ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 32, "kfull"): (97, 579, 128),
+        ("wavesplit_tile", 16, 64, "kfull", "unpacked"): (7, 12824, 7808), ("wavesplit_tile", 16, 64, "kfull"): (65, 2728, 128),
+        ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128), ("wavesplit_tile", 32, 32, "kfull"): (49, 2064, 128),
+        ("wavesplit_tile", 32, 64, "kfull"): (49, 4137, 128), ("wavesplit_tile", 48, 16, "kfull"): (194, 616, 128),
+        ("wavesplit_tile", 48, 32, "kfull"): (193, 1223, 128), ("wavesplit_tile", 64, 32, "kfull"): (49, 4358, 128),
+        ("wavesplit_tile", 64, 64, "kfull"): (1637, 291, 512),
     },
     "fp8_scaled": {
         ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
         ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
-        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 25216, 3968),
-        ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (586, 432, 16640),
-        ("dma3", 128, "split", "bn192"): (65, 8544, 13312), ("dma3", 128, "split"): (321, 4272, 13824),
+        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
+        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (3348, 8, 6272),
+        ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (67, 8280, 13056),
         ("dma3", 128, "whole", "bn128", "deep"): (194, 12416, 640), ("dma3", 128, "whole", "bn192"): (194, 16528, 128),
-        ("dma3", 128, "whole"): (196, 24704, 128), ("dma3", 160, "split", "bn128", "deep"): (134, 3608, 12544),
+        ("dma3", 128, "whole"): (196, 24704, 128), ("dma3", 160, "split", "bn128", "deep"): (2716, 8, 10752),
         ("dma3", 160, "split", "bn192"): (313, 5480, 18432), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
-        ("dma3", 160, "whole", "bn192"): (289, 16408, 128), ("dma3", 192, "split", "bn128"): (2794, 400, 14208),
+        ("dma3", 160, "whole", "bn192"): (289, 16408, 128), ("dma3", 192, "split", "bn128"): (4174, 8, 15488),
         ("dma3", 192, "whole", "bn128"): (161, 24608, 128), ("dma3", 256, "split", "bn128"): (211, 8312, 17664),
-        ("dma3", 256, "whole", "bn128"): (4677, 1544, 128), ("dma3", 64, "split", "bn128", "deep"): (290, 216, 17536),
-        ("dma3", 64, "split", "bn192", "deep"): (331, 576, 18048), ("dma3", 64, "split"): (17, 17024, 8320),
-        ("dma3", 64, "whole", "bn128", "deep"): (194, 616, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
-        ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128), ("dma3", 64, "whole"): (17, 57344, 512),
-        ("dma3", 96, "split", "bn128", "deep"): (69, 1920, 17408), ("dma3", 96, "split", "bn192", "deep"): (902, 544, 18432),
-        ("dma3", 96, "split"): (263, 4136, 16640), ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512),
-        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (261, 16488, 128),
-        ("generic", 128, "aligned", "split"): (65, 25352, 912), ("generic", 128, "aligned", "whole"): (708, 2816, 16),
-        ("generic", 16, "aligned", "split"): (1, 8, 1024), ("generic", 16, "aligned", "whole"): (1, 8, 128),
-        ("generic", 256, "aligned", "split"): (1052, 6688, 928), ("generic", 32, "aligned", "split"): (17, 9656, 10480),
-        ("generic", 32, "aligned", "whole"): (26, 50944, 16), ("generic", 64, "aligned", "split"): (33, 6016, 16688),
-        ("generic", 64, "aligned", "whole"): (34, 33648, 16), ("pingpong", "kfull"): (193, 49640, 128),
-        ("pingpong", "ktail"): (1555, 9984, 16), ("pipelined", "ktail"): (1094, 6576, 16),
+        ("dma3", 256, "whole", "bn128"): (4677, 1544, 128), ("dma3", 64, "split", "bn128", "deep"): (674, 8, 14848),
+        ("dma3", 64, "split", "bn128"): (2462, 8, 6528), ("dma3", 64, "split", "bn192", "deep"): (871, 280, 11648),
+        ("dma3", 64, "split"): (17, 17024, 8320), ("dma3", 64, "whole", "bn128", "deep"): (194, 616, 128),
+        ("dma3", 64, "whole", "bn128"): (65, 16472, 128), ("dma3", 64, "whole", "bn192", "deep"): (17, 32880, 128),
+        ("dma3", 64, "whole"): (17, 57344, 512), ("dma3", 96, "split", "bn128", "deep"): (3334, 8, 5248),
+        ("dma3", 96, "split", "bn192", "deep"): (2958, 264, 9344), ("dma3", 96, "split"): (263, 4136, 16640),
+        ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512), ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128),
+        ("dma3", 96, "whole"): (261, 16488, 128), ("generic", 128, "aligned", "split"): (65, 25352, 912),
+        ("generic", 128, "aligned", "whole"): (708, 2816, 16), ("generic", 16, "aligned", "split"): (1, 8, 1024),
+        ("generic", 16, "aligned", "whole"): (1, 8, 128), ("generic", 256, "aligned", "split"): (1052, 6688, 928),
+        ("generic", 32, "aligned", "split"): (17, 9656, 10480), ("generic", 32, "aligned", "whole"): (26, 50944, 16),
+        ("generic", 64, "aligned", "split"): (33, 6016, 16688), ("generic", 64, "aligned", "whole"): (34, 33648, 16),
+        ("pingpong", "kfull"): (193, 49640, 128), ("pingpong", "ktail"): (1555, 9984, 16), ("pipelined", "ktail"): (1094, 6576, 16),
         ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 16, "ktail"): (1, 8, 16),
         ("wavesplit_tile", 16, 32, "kfull"): (129, 456, 128), ("wavesplit_tile", 16, 32, "ktail"): (100, 592, 16),
         ("wavesplit_tile", 16, 64, "kfull"): (33, 4104, 384), ("wavesplit_tile", 16, 64, "ktail"): (172, 1352, 16),
@@ -185,37 +186,38 @@ VARIANT_SHAPES = {
     "int8": {
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round"): (1, 16, 128),
-        ("decode_wavesplit", "w4", "rounds"): (1, 7936, 17664), ("decode_wavesplit", "w8", "one_round"): (1, 25216, 3968),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (69, 2816, 15360),
+        ("decode_wavesplit", "w4", "rounds"): (1, 7936, 17664), ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840),
+        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (2796, 8, 5760),
         ("dma3", 128, "split", "bn192"): (198, 5448, 12288), ("dma3", 128, "split"): (329, 4352, 18560),
         ("dma3", 128, "whole", "bn128", "deep"): (194, 12416, 640), ("dma3", 128, "whole", "bn192"): (194, 16528, 128),
-        ("dma3", 128, "whole"): (1295, 10760, 128), ("dma3", 160, "split", "bn128", "deep"): (134, 3608, 12544),
+        ("dma3", 128, "whole"): (1295, 10760, 128), ("dma3", 160, "split", "bn128", "deep"): (2456, 8, 14080),
         ("dma3", 160, "split", "bn192"): (313, 5480, 18432), ("dma3", 160, "whole", "bn128", "deep"): (130, 24696, 128),
-        ("dma3", 160, "whole", "bn192"): (289, 16408, 128), ("dma3", 192, "split", "bn128"): (2794, 400, 14208),
+        ("dma3", 160, "whole", "bn192"): (289, 16408, 128), ("dma3", 192, "split", "bn128"): (3076, 264, 16640),
         ("dma3", 192, "whole", "bn128"): (484, 8344, 128), ("dma3", 256, "split", "bn128"): (208, 8568, 16512),
-        ("dma3", 256, "whole", "bn128"): (4677, 1544, 128), ("dma3", 64, "split", "bn128", "deep"): (290, 216, 17536),
-        ("dma3", 64, "split", "bn192", "deep"): (421, 912, 16128), ("dma3", 64, "split"): (17, 5848, 17408),
-        ("dma3", 64, "whole", "bn128", "deep"): (194, 616, 128), ("dma3", 64, "whole", "bn128"): (65, 16472, 128),
-        ("dma3", 64, "whole", "bn192", "deep"): (17, 33280, 512), ("dma3", 64, "whole"): (12, 33096, 128),
-        ("dma3", 96, "split", "bn128", "deep"): (70, 1904, 17536), ("dma3", 96, "split", "bn192", "deep"): (902, 544, 18432),
-        ("dma3", 96, "split"): (263, 4136, 16640), ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512),
-        ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128), ("dma3", 96, "whole"): (389, 10904, 128),
-        ("generic", 128, "aligned", "split"): (65, 25352, 912), ("generic", 128, "aligned", "whole"): (708, 2816, 16),
-        ("generic", 16, "aligned", "split"): (1, 8, 1024), ("generic", 16, "aligned", "whole"): (1, 8, 128),
-        ("generic", 256, "aligned", "split"): (1052, 6688, 928), ("generic", 256, "aligned", "whole"): (1094, 6576, 16),
-        ("generic", 32, "aligned", "split"): (17, 9656, 10480), ("generic", 32, "aligned", "whole"): (26, 50944, 16),
-        ("generic", 64, "aligned", "split"): (33, 6016, 16688), ("generic", 64, "aligned", "whole"): (34, 33648, 16),
-        ("pingpong", "kfull"): (223, 49272, 128), ("pingpong128", "whole"): (196, 24704, 128),
-        ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128), ("wavesplit_tile", 16, 16, "ktail"): (1, 8, 16),
-        ("wavesplit_tile", 16, 32, "kfull"): (129, 456, 128), ("wavesplit_tile", 16, 32, "ktail"): (100, 592, 16),
-        ("wavesplit_tile", 16, 64, "kfull"): (33, 4104, 384), ("wavesplit_tile", 16, 64, "ktail"): (172, 1352, 16),
-        ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128), ("wavesplit_tile", 32, 16, "ktail"): (85, 712, 16),
-        ("wavesplit_tile", 32, 32, "kfull"): (50, 2104, 384), ("wavesplit_tile", 32, 32, "ktail"): (100, 1408, 16),
-        ("wavesplit_tile", 32, 64, "kfull"): (17, 8320, 768), ("wavesplit_tile", 32, 64, "ktail"): (195, 1664, 16),
-        ("wavesplit_tile", 48, 16, "kfull"): (193, 616, 256), ("wavesplit_tile", 48, 16, "ktail"): (162, 768, 16),
-        ("wavesplit_tile", 48, 32, "kfull"): (903, 272, 512), ("wavesplit_tile", 48, 32, "ktail"): (199, 1224, 16),
-        ("wavesplit_tile", 64, 32, "kfull"): (53, 4240, 896), ("wavesplit_tile", 64, 32, "ktail"): (248, 1432, 16),
-        ("wavesplit_tile", 64, 64, "kfull"): (1816, 264, 2176), ("wavesplit_tile", 64, 64, "ktail"): (323, 1536, 16),
+        ("dma3", 256, "whole", "bn128"): (4677, 1544, 128), ("dma3", 64, "split", "bn128", "deep"): (674, 8, 14848),
+        ("dma3", 64, "split", "bn128"): (2462, 8, 6528), ("dma3", 64, "split", "bn192", "deep"): (792, 136, 17280),
+        ("dma3", 64, "split"): (17, 5848, 17408), ("dma3", 64, "whole", "bn128", "deep"): (194, 616, 128),
+        ("dma3", 64, "whole", "bn128"): (65, 16472, 128), ("dma3", 64, "whole", "bn192", "deep"): (17, 33280, 512),
+        ("dma3", 64, "whole"): (12, 33096, 128), ("dma3", 96, "split", "bn128", "deep"): (1606, 8, 12928),
+        ("dma3", 96, "split", "bn192", "deep"): (2958, 264, 9344), ("dma3", 96, "split"): (263, 4136, 16640),
+        ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512), ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128),
+        ("dma3", 96, "whole"): (389, 10904, 128), ("generic", 128, "aligned", "split"): (65, 25352, 912),
+        ("generic", 128, "aligned", "whole"): (708, 2816, 16), ("generic", 16, "aligned", "split"): (1, 8, 1024),
+        ("generic", 16, "aligned", "whole"): (1, 8, 128), ("generic", 256, "aligned", "split"): (1052, 6688, 928),
+        ("generic", 256, "aligned", "whole"): (1094, 6576, 16), ("generic", 32, "aligned", "split"): (17, 9656, 10480),
+        ("generic", 32, "aligned", "whole"): (26, 50944, 16), ("generic", 64, "aligned", "split"): (33, 6016, 16688),
+        ("generic", 64, "aligned", "whole"): (34, 33648, 16), ("pingpong", "kfull"): (223, 49272, 128),
+        ("pingpong128", "whole"): (196, 24704, 128), ("wavesplit_tile", 16, 16, "kfull"): (17, 8, 128),
+        ("wavesplit_tile", 16, 16, "ktail"): (1, 8, 16), ("wavesplit_tile", 16, 32, "kfull"): (129, 456, 128),
+        ("wavesplit_tile", 16, 32, "ktail"): (100, 592, 16), ("wavesplit_tile", 16, 64, "kfull"): (33, 4104, 384),
+        ("wavesplit_tile", 16, 64, "ktail"): (172, 1352, 16), ("wavesplit_tile", 32, 16, "kfull"): (81, 680, 128),
+        ("wavesplit_tile", 32, 16, "ktail"): (85, 712, 16), ("wavesplit_tile", 32, 32, "kfull"): (50, 2104, 384),
+        ("wavesplit_tile", 32, 32, "ktail"): (100, 1408, 16), ("wavesplit_tile", 32, 64, "kfull"): (17, 8320, 768),
+        ("wavesplit_tile", 32, 64, "ktail"): (195, 1664, 16), ("wavesplit_tile", 48, 16, "kfull"): (193, 616, 256),
+        ("wavesplit_tile", 48, 16, "ktail"): (162, 768, 16), ("wavesplit_tile", 48, 32, "kfull"): (903, 272, 512),
+        ("wavesplit_tile", 48, 32, "ktail"): (199, 1224, 16), ("wavesplit_tile", 64, 32, "kfull"): (53, 4240, 896),
+        ("wavesplit_tile", 64, 32, "ktail"): (248, 1432, 16), ("wavesplit_tile", 64, 64, "kfull"): (1816, 264, 2176),
+        ("wavesplit_tile", 64, 64, "ktail"): (323, 1536, 16),
     },
 }
 FP8_REQUIRED_VARIANTS = set(VARIANT_SHAPES["fp8"])

@@ -135,6 +135,26 @@ def test_benchmark_shapes_hold_their_kernels_when_a_constant_moves():
             assert (kind, shape, t) in moved, f"{kind} {shape}: recorded alternative {t} is no longer reached"
 
 
+# (kind, shape, kernel that has to run, its time, the other's: wave-split tile against the kernel the constants table names,
+# few workgroups against many), in microseconds as for RECORDED_BOUNDARIES; both sides of each line that tile_choice.h draws
+MEASURED_CHOICES = [
+    ("fp8", (16, 36864, 2304), "dma3", 19.3, 22.9), ("fp8", (16, 50688, 5120), "dma3", 51.3, 57.3), ("int8", (12, 17408, 1024), "dma3", 7.1, 9.0),
+    ("fp8", (16, 30464, 4096), "wavesplit_tile", 29.5, 31.7), ("fp8_scaled", (16, 30464, 4096), "wavesplit_tile", 28.4, 32.2),
+    ("fp8", (1, 20736, 4096), "decode_wavesplit", 19.0, 24.4), ("fp8", (8, 20736, 4096), "decode_wavesplit", 21.3, 24.4),
+    ("fp8", (6, 27392, 3584), "wavesplit_tile", 21.8, 23.6), ("int8", (11, 28672, 4096), "wavesplit_tile", 26.2, 29.8),
+    ("fp8", (2616, 704, 10368), "dma3", 37.4, 53.2), ("fp8", (1610, 960, 10496), "dma3", 34.7, 44.7), ("fp8_scaled", (2595, 384, 7168), "dma3", 19.3, 22.3),
+    ("fp8", (1608, 576, 7168), "wavesplit_tile", 20.3, 23.1),
+    ("fp8", (71, 17920, 14592), ("dma3", 128, 256, 3), 62.6, 81.0), ("fp8_scaled", (103, 19072, 17664), ("dma3", 128, 256, 3), 77.2, 96.2),
+    ("fp8_ue8m0", (65, 9792, 10624), ("dma3", 96, 128, 3), 28.7, 39.2),
+]
+
+
+@pytest.mark.parametrize("kind,shape,want,us,other", MEASURED_CHOICES)
+def test_the_faster_kernel_runs(kind, shape, want, us, other):
+    p = plan_for(kind, *shape)
+    assert us < other and want in (p["kernel"], (p["kernel"], p["bm"], p["bn"], p["splits"])), p
+
+
 def test_perturbed_plan_query():
     import ctypes
 
