@@ -11,8 +11,9 @@
 //         scale = max(absmax, eps) / 448 and either q = e4m3fn(clamp(x * (1 / scale))), the arithmetic of the Triton kernel
 //         python/sglang/srt/layers/quantization/fp8_kernel.py:122-161, or q = e4m3fn(clamp(x / scale)) with a true
 //         division, the arithmetic of sgl-kernel/csrc/gemm/per_token_group_quant_8bit.cu:25-114.
-// Two-byte inputs: rows of up to 24576 elements stay in registers between the two phases (per_token_quant_row_kernel; thousands of
-// short rows, and the mode with row sums up to 8192 elements, one WAVE per row, four rows per workgroup, no LDS and no barrier).
+// Two-byte inputs: rows of up to 24576 elements stay in registers between the two phases (per_token_quant_row_kernel; more than a
+// thousand rows of up to 4096 elements, rows of up to 512, and the mode with row sums up to 8192 elements, one WAVE per row, four rows per
+// workgroup, no LDS and no barrier).
 // Other rows take per_token_quant_kernel, which reads again (from L2) what its registers do not hold.
 #include "common.h"
 
@@ -296,8 +297,10 @@ int per_token_quant(const char* what, const void* x, int x_dtype, void* q, float
     // Rows in the registers of one workgroup: with few rows as many threads as a row has vectors (latency), with many rows more
     // vectors per thread (fewer barriers).  us before / now, FP8 and INT8:  160 x 7168 4.6 / 2.9, 5.6 / 3.1;  512 x 4096 3.9 / 3.0,
     // 4.5 / 3.1;  2048 x 14336 16.7 / 15.9, 18.2 / 16.5;  4096 x 18432 55 / 37 (rows beyond 8192 elements used to be read twice).
-    // Thousands of rows of up to 4096 elements stay with the wave per row (4096 x 4096 INT8 10.6 against 10.8).
-    if (x_dtype != MI355_F32 && K <= 8 * 512 * 6 && !(M > 3072 && K <= 4096)) {
+    // Rows of up to 4096 elements stay with the wave per row where a thousand of them fill the chip (wave / row, FP8: 1024 x 1024 3.0 / 2.8,
+    // 1024 x 4096 4.8 / 5.0, 1536 x 4096 5.8 / 6.2, 3072 x 2048 5.2 / 5.8;  INT8: 1024 x 2048 4.0 / 3.7, 1536 x 3072 5.6 / 5.8, 2048 x 4096
+    // 7.2 / 7.7), and rows of up to 512 elements always (FP8 8 x 512 2.5 / 2.6, 2048 x 128 2.7 / 3.0;  INT8 within 3 % either way).
+    if (x_dtype != MI355_F32 && K <= 8 * 512 * 6 && !(K <= 4096 && (M > 1024 || K <= 512))) {
 #define MI355_ROWS(T, NV)                                                                                                              \
   {                                                                                                                                    \
     if (x_dtype == MI355_BF16) hipLaunchKernelGGL((per_token_quant_row_kernel<MI355_BF16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K); \

@@ -8,8 +8,8 @@ from sglang_amd.workloads import make_activation
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M", [1, 640, 641])
-@pytest.mark.parametrize("K", [8, 2048, 2056, 4096, 4104, 8192, 8200, 16384, 16392, 24576, 24584])
+@pytest.mark.parametrize("M", [1, 640, 641, 1025])
+@pytest.mark.parametrize("K", [8, 512, 520, 2048, 2056, 4096, 4104, 8192, 8200, 16384, 16392, 24576, 24584])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_per_token(gpu, oracle, M, K, dtype):
     from sglang_amd.fp8_kernel import sglang_per_token_quant_fp8
