@@ -315,6 +315,17 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmParams p) 
   }
 }
 
+// Both tables, an array of doubles as far as the queries of single constants go.
+struct DispatchConstants {
+  RouteConstants route;
+  TileModel tiles;
+};
+constexpr int CONSTANT_COUNT = ROUTE_CONSTANT_COUNT + TILE_CONSTANT_COUNT;
+static_assert(sizeof(DispatchConstants) == CONSTANT_COUNT * sizeof(double), "the tables are read as an array of doubles");
+const DispatchConstants g_defaults{};
+thread_local const DispatchConstants* g_override = nullptr;  // set while a perturbed plan is queried
+bool dispatch_perturbed() { return g_override != nullptr; }
+
 // ---------------------------------------------------------------------------------------------
 struct Plan {
   int bm, bn, splits, kb_per_split;
@@ -350,14 +361,61 @@ Plan make_plan(int64_t M, int64_t N, int64_t K) {
 size_t scale_relayout_bytes(int64_t M, int64_t K);
 int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K);
 
+// What the dispatcher works out for a shape takes microseconds, and a call asks several times (the workspace query of the caller,
+// the entry point's check of it, the launch), so each thread keeps the answers for the shapes it met last.  Host time of a
+// workspace query, at a token count not met before and at a known one: K = 18432 to 7168 channels 15.6 and 2.4 us when every
+// query worked out the plans of all FP8 kinds and only routes were kept, 4.3 and below 0.1 now; 4096 to 6144 10.7 and 1.1, now
+// 2.8; 512 to 32768 3.3 and 0.2, now 1.1.
+template <class Key, class Value>
+class RecentShapes {
+  static constexpr int ENTRIES = 256;
+  struct Entry {
+    bool used;
+    Key key;
+    Value value;
+  };
+  Entry entries[ENTRIES] = {};
+
+ public:
+  template <class Compute>
+  const Value& get(const Key& key, Compute compute) {
+    uint64_t h = ((uint64_t)key.M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)key.N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)key.K * 0x165667b19e3779f9ull) ^
+                 (uint64_t)key.kind * 0x27d4eb2f165667c5ull;
+    Entry& e = entries[(h ^ (h >> 29)) >> 20 & (ENTRIES - 1)];
+    if (!e.used || !(e.key == key)) {
+      e.value = compute();
+      e.key = key, e.used = true;
+    }
+    return e.value;
+  }
+};
+struct ShapeKey {
+  int64_t M, N, K;
+  int kind;
+  bool operator==(const ShapeKey& o) const { return M == o.M && N == o.N && K == o.K && kind == o.kind; }
+};
+
+// The mid-M kernel's plan, which the route and the workspace bound of one shape both want.
+Dma3Plan mid_plan(int64_t M, int64_t N, int64_t K, bool is_int8) {
+  if (dispatch_perturbed()) return dma3_plan(M, N, K, is_int8);
+  struct Last {
+    ShapeKey key;
+    Dma3Plan plan;
+  };
+  static thread_local Last last{};  // (no shape has M = 0)
+  const ShapeKey key{M, N, K, (int)is_int8};
+  if (!(last.key == key)) last = Last{key, dma3_plan(M, N, K, is_int8)};
+  return last.plan;
+}
+
 // Upper bound over the kernels a shape may be routed to (the choice also depends on pointer alignment, which is not
 // known here).
-size_t workspace_bytes(int64_t M, int64_t N, int64_t K, bool is_fp8) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
+size_t workspace_bound(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+  const bool is_fp8 = kind != GK_INT8;
   const Plan pl = make_plan(M, N, K);
   size_t need = pl.splits > 1 ? (size_t)pl.splits * (size_t)M * (size_t)N * 4u : 0;
   if (M > 16 && K % KSTEP == 0) {
-    const Dma3Plan dp = dma3_plan(M, N, K, !is_fp8);  // (an upper bound: the dispatcher may still pick another kernel)
+    const Dma3Plan dp = mid_plan(M, N, K, !is_fp8);  // (an upper bound: the dispatcher may still pick another kernel)
     const size_t dneed = dp.splits > 1 ? (size_t)dp.splits * (size_t)M * (size_t)N * 4u : 0;
     if (dneed > need) need = dneed;
   }
@@ -367,12 +425,19 @@ size_t workspace_bytes(int64_t M, int64_t N, int64_t K, bool is_fp8) {
     if (dneed > need) need = dneed;
   }
   if (M > 16 && K % KSTEP == 0) {
-    const int splits = is_fp8 ? std::max(run_splits(GK_F32, M, N, K), run_splits(GK_UNIT, M, N, K)) : run_splits(GK_INT8, M, N, K);
+    const int splits = run_splits(kind, M, N, K);
     const size_t rneed = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * 4u : 0;
     if (rneed > need) need = rneed;
   }
   if (is_fp8 && (M > 16 || (double)M >= route_constants().decode_dma3_min_tokens)) need += scale_relayout_bytes(M, K);  // the direct-to-LDS kernels may have to re-lay the token scales out
   return need;
+}
+size_t workspace_bytes(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (kind == GK_UE8M0) kind = GK_F32;  // one model above decode sizes, and where the exponents are unpacked the fp32 kernels run
+  if (dispatch_perturbed()) return workspace_bound(kind, M, N, K);
+  static thread_local RecentShapes<ShapeKey, size_t> table;
+  return table.get(ShapeKey{M, N, K, (int)kind}, [&] { return workspace_bound(kind, M, N, K); });
 }
 
 template <bool IS_FP8, int BM, int BN, int WGM, int WGN, bool ALIGNED, bool SPLIT>
@@ -496,7 +561,7 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
     // 25 us for K=2048 -> N=7168 at 128 tokens, 23 against 68 us for K=7168 -> N=576 at 2048), its 64 x 128 tiles and K
     // splits filling the chip where the channels alone do not; without splits (N not a multiple of 4) the older
     // chip-filling score decides.
-    const Dma3Plan dp = dma3_plan(M, N, K, !is_fp8);
+    const Dma3Plan dp = mid_plan(M, N, K, !is_fp8);
     // Above 128 tokens the two-phase 256 x 256 kernel competes: a round of its tiles takes (K blocks) x 1.39 us + 11 us
     // (INT8: 1.46 us per block), whatever part of the tile is filled and however many CUs the round uses, so it wins
     // where the channels alone give it a round's worth of tiles (measured: K=7168 -> N=36864 at M=256: 89 against 141 us,
@@ -539,16 +604,6 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
   return r;
 }
 
-// Both tables, an array of doubles as far as the queries of single constants go.
-struct DispatchConstants {
-  RouteConstants route;
-  TileModel tiles;
-};
-constexpr int CONSTANT_COUNT = ROUTE_CONSTANT_COUNT + TILE_CONSTANT_COUNT;
-static_assert(sizeof(DispatchConstants) == CONSTANT_COUNT * sizeof(double), "the tables are read as an array of doubles");
-const DispatchConstants g_defaults{};
-thread_local const DispatchConstants* g_override = nullptr;  // set while a perturbed plan is queried
-
 // The route that runs: choose_route's, or the tile that models faster (tile_choice.h).
 Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
   Route r = choose_route(kind != GK_INT8, M, N, K, lda, ldb, aligned);
@@ -571,30 +626,16 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
   r.kb_per_split = (int)((kb + c.splits - 1) / c.splits);
   return r;
 }
-// A model evaluation takes some 10 us, so each thread keeps the routes of the shapes it met last.
 Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
-  struct Entry {
-    int64_t M, N, K, lda, ldb;
-    int kind;  // -1: empty
+  if (dispatch_perturbed()) return uncached_run_route(kind, M, N, K, lda, ldb, aligned);
+  struct Key : ShapeKey {
+    int64_t lda, ldb;
     bool aligned;
-    Route route;
+    bool operator==(const Key& o) const { return ShapeKey::operator==(o) && lda == o.lda && ldb == o.ldb && aligned == o.aligned; }
   };
-  constexpr int ENTRIES = 256;
-  struct Table {
-    Entry e[ENTRIES];
-    Table() {
-      for (Entry& x : e) x.kind = -1;
-    }
-  };
-  if (g_override != nullptr) return uncached_run_route(kind, M, N, K, lda, ldb, aligned);
-  static thread_local Table table;
-  uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull) ^ (uint64_t)kind * 0x27d4eb2f165667c5ull;
-  Entry& e = table.e[(h ^ (h >> 29)) >> 20 & (ENTRIES - 1)];
-  if (e.kind != (int)kind || e.M != M || e.N != N || e.K != K || e.lda != lda || e.ldb != ldb || e.aligned != aligned) {
-    e.route = uncached_run_route(kind, M, N, K, lda, ldb, aligned);
-    e.kind = (int)kind, e.M = M, e.N = N, e.K = K, e.lda = lda, e.ldb = ldb, e.aligned = aligned;
-  }
-  return e.route;
+  static thread_local RecentShapes<Key, Route> table;
+  if (kind == GK_UE8M0 && M > 16) kind = GK_F32;  // above decode sizes both kinds have one model
+  return table.get(Key{{M, N, K, (int)kind}, lda, ldb, aligned}, [&] { return uncached_run_route(kind, M, N, K, lda, ldb, aligned); });
 }
 int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K) { return run_route(kind, M, N, K, K, K, true).splits; }
 
@@ -838,7 +879,7 @@ extern "C" int mi355_gemm_plan_perturbed(int is_fp8, int64_t M, int64_t N, int64
 }
 
 extern "C" size_t mi355_fp8_blockwise_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return workspace_bytes(M, N, K, true);
+  return workspace_bytes(GK_F32, M, N, K);
 }
 
 namespace {
@@ -975,7 +1016,7 @@ size_t ue8m0_unpacked_bytes(int64_t M, int64_t N, int64_t K) {
 
 extern "C" size_t mi355_fp8_blockwise_mm_ue8m0_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return ue8m0_unpacked_bytes(M, N, K) + workspace_bytes(M, N, K, true);
+  return ue8m0_unpacked_bytes(M, N, K) + workspace_bytes(GK_UE8M0, M, N, K);
 }
 
 extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const void* sa_words, const void* sb_words,
@@ -1082,7 +1123,7 @@ extern "C" int mi355_qlinear_init(void) {
 }
 
 extern "C" size_t mi355_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return workspace_bytes(M, N, K, true);
+  return workspace_bytes(GK_UNIT, M, N, K);
 }
 
 extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const float* sb, const void* bias,
@@ -1245,7 +1286,7 @@ int run_wavesplit_quant(GemmParams& p, WavesplitQuant kind, const void* x, int x
 extern "C" size_t mi355_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const size_t kb = (size_t)((K + KSTEP - 1) / KSTEP);
-  return align256((size_t)M * (size_t)K) + align256((size_t)((M + 3) & ~3ll) * kb * 4u) + workspace_bytes(M, N, K, true);
+  return align256((size_t)M * (size_t)K) + align256((size_t)((M + 3) & ~3ll) * kb * 4u) + workspace_bytes(GK_F32, M, N, K);
 }
 
 namespace {
@@ -1348,7 +1389,7 @@ extern "C" int mi355_int8_linear_plan(int64_t M, int64_t N, int64_t K, char* buf
 }
 
 extern "C" size_t mi355_int8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return workspace_bytes(M, N, K, false);
+  return workspace_bytes(GK_INT8, M, N, K);
 }
 
 extern "C" int mi355_int8_scaled_mm(const void* a, const void* b, const float* sa, const float* sb, const void* bias,
@@ -1381,7 +1422,7 @@ extern "C" int mi355_int8_scaled_mm(const void* a, const void* b, const float* s
 
 extern "C" size_t mi355_int8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return align256((size_t)M * (size_t)K) + align256((size_t)M * 4u) + workspace_bytes(M, N, K, false);
+  return align256((size_t)M * (size_t)K) + align256((size_t)M * 4u) + workspace_bytes(GK_INT8, M, N, K);
 }
 
 extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, const float* w_scale, const void* bias, void* out,

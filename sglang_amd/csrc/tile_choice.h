@@ -7,6 +7,7 @@
 // mean over 2100 shapes), where the constants table alone was 16 to 25 % slower.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 
 #include "gemm_common.h"
@@ -76,7 +77,8 @@ double rounds_of(int64_t workgroups, int64_t slots, Round round) {
   return (double)full * round(1.0) + (rest ? round((double)rest / (double)slots) : 0.0);
 }
 
-double dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, int splits) {
+// (`most`: a time from which on the result does not matter; the powers are left out where the larger of the two bounds reaches it)
+double dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, int splits, double most = 1e30) {
   const int bm = MID_TILES[i].bm, bn = MID_TILES[i].bn;
   const int64_t kb = ceil_div(K, KSTEP), wg = ceil_div(M, bm) * ceil_div(N, bn) * splits;
   const double blocks = (double)ceil_div(kb, splits);
@@ -86,7 +88,8 @@ double dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, i
                     });
   const double mn = (double)M * (double)N * 1e-6;
   const double stream = ((double)N + (double)M) * (double)K * 1e-6 / t.stream + mn * 2.0 * t.result_us_per_mb + t.stream_us;
-  return norm_of(us, stream, 6.0) + (splits > 1 ? t.split_us + t.split_us_per_mb * splits * mn * 4.0 : 0.0);
+  const double split = splits > 1 ? t.split_us + t.split_us_per_mb * splits * mn * 4.0 : 0.0;
+  return std::max(us, stream) + split >= most ? most : norm_of(us, stream, 6.0) + split;
 }
 double two_phase_us(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
   const double blocks = (double)ceil_div(K, KSTEP);
@@ -94,20 +97,21 @@ double two_phase_us(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
            return norm_of(t.pp_tile + blocks * t.pp_block * (1.0 + t.pp_busy * fill), t.pp_store * fill, 6.0);
          });
 }
-double wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K) {
+double wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, double most = 1e30) {
   const int bm = WAVESPLIT_TILES[i].bm, bn = WAVESPLIT_TILES[i].bn;
   const double kbytes = (double)(bm + bn) * (double)K * 1e-3;
   const double us = t.ws_launch + rounds_of(ceil_div(M, bm) * ceil_div(N, bn), NUM_CUS, [&](double fill) {
                       return t.ws_tile + kbytes * (t.ws_kb + t.ws_kb_busy * fill) + (double)(bm * bn) / 1024.0 * t.ws_result;
                     });
-  return norm_of(us, (double)N * (double)K * 1e-6 / t.ws_stream + t.ws_stream_us, t.ws_norm);
+  const double stream = (double)N * (double)K * 1e-6 / t.ws_stream + t.ws_stream_us;
+  return std::max(us, stream) >= most ? most : norm_of(us, stream, t.ws_norm);
 }
 
 TileChoice best_wavesplit_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
   TileChoice best{TF_NONE, 0, 0, 1, 1e30};
   constexpr int COUNT = sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0]);
   for (int i = 0; i < COUNT; ++i) {
-    const double us = wavesplit_tile_us(t, i, M, N, K);
+    const double us = wavesplit_tile_us(t, i, M, N, K, best.us);
     if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
   }
   return best;
@@ -123,7 +127,7 @@ TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
       if (splits > 1 && (N % 4 != 0 || per < 4 || tiles * splits > 560 || tiles > 200)) break;
       if (splits == previous) continue;
       previous = splits;
-      const double us = dma_tile_us(t, i, M, N, K, splits);
+      const double us = dma_tile_us(t, i, M, N, K, splits, best.us);
       if (us < best.us) best = {TF_DMA, MID_TILES[i].bm, MID_TILES[i].bn, splits, us};
     }
   }
@@ -217,7 +221,7 @@ TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bo
   TileChoice best{TF_NONE, 0, 0, 1, 1e30};
   for (int i = 0; i < 3; ++i) {
     static_assert(WAVESPLIT_TILES[2].bm == 16, "the 16-token tiles come first");
-    const double us = wavesplit_tile_us(t, i, M, N, K);
+    const double us = wavesplit_tile_us(t, i, M, N, K, best.us);
     if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
   }
   return best;

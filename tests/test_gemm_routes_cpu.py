@@ -1,6 +1,9 @@
 """Which kernel variant the dispatcher picks is a host-side decision, so it is checked without a GPU: the shapes the
 GPU parity tests run (tests/gemm_cases.py) must between them reach every compiled variant, and the full-size benchmark
 configurations must only use variants that those tests (or the full-size tests themselves) exercise."""
+import random
+import time
+
 import pytest
 
 from gemm_cases import (FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, INT8_CONFIG,
@@ -241,6 +244,49 @@ def test_workspace_covers_the_plan(kind, M, N, K):
     p = plan_for(kind, M, N, K)
     ws = (L.mi355_fp8_blockwise_mm_workspace_bytes if kind == "fp8" else L.mi355_int8_scaled_mm_workspace_bytes)(M, N, K)
     assert ws >= (p["splits"] * M * N * 4 if p["splits"] > 1 else 0)
+
+
+GEMM_WORKSPACES = {"fp8": "mi355_fp8_blockwise_mm_workspace_bytes", "fp8_ue8m0": "mi355_fp8_blockwise_mm_ue8m0_workspace_bytes",
+                   "fp8_scaled": "mi355_fp8_scaled_mm_workspace_bytes", "int8": "mi355_int8_scaled_mm_workspace_bytes"}
+
+
+def test_workspace_covers_every_kind_asked_in_turn():
+    """The size is kept for the shapes met last: it is each shape's and kind's own, whatever was asked before."""
+    from sglang_amd import _lib
+
+    L = _lib.lib()
+    rng = random.Random(5)
+    shapes = [(rng.choice((3, 9, 16, 17, 33, 48, 96, 160, 387, 1100)), 8 * rng.randint(2, 4000), 128 * rng.randint(1, 160)) for _ in range(600)]
+    first = {}
+    for _ in range(2):  # the second turn meets some sizes kept and some replaced
+        for s in shapes:
+            for kind, name in GEMM_WORKSPACES.items():
+                size = getattr(L, name)(*s)
+                p = _lib.gemm_plan(kind, *s)
+                assert size >= (p["splits"] * s[0] * s[1] * 4 if p["splits"] > 1 else 0), (kind, s, p)
+                assert first.setdefault((kind, s), size) == size, (kind, s)
+
+
+def test_host_work_of_a_workspace_query():
+    """In units of a query that returns at once (M = 0; some 0.5 us): a known shape is a look at the table, and a token count not met
+    before works out the plans of the one kind asked for (measured 1 and 9 of these units; 6 and 35 where a query worked out
+    every FP8 kind's plans each time)."""
+    from sglang_amd import _lib
+
+    ask = _lib.lib().mi355_fp8_block_linear_workspace_bytes
+    K, N = 18432, 7168
+
+    def cost(tokens):
+        t = time.perf_counter()
+        for M in tokens:
+            ask(M, N, K)
+        return (time.perf_counter() - t) / len(tokens)
+
+    fresh = iter(range(20, 1420, 70))
+    trials = [(cost([0] * 400), cost([200] * 400), cost(range(m := next(fresh), m + 70))) for _ in range(20)]
+    nothing, known, new = (min(t) for t in zip(*trials))
+    assert known < 2 * nothing, (nothing, known)
+    assert new < 20 * nothing, (nothing, new)
 
 
 def test_grouped_plan_bounds_hold_for_any_routing():
