@@ -60,18 +60,13 @@ struct PipeState {
   uint32_t sc_off;                 // byte offset of this lane's first token scale inside a stage's scale row
 };
 
-// KFULL: K is a multiple of 128, so every chunk of every block is inside the row.
-template <bool KFULL, int SET>
+template <int SET>
 __device__ __forceinline__ void load_one(PipeState& s, int i, int kb) {
   kb = min(kb, s.kb_last);
   const uint8_t* base = (i < P_BM / 32 ? s.a_base : s.b_base) + (int64_t)kb * KSTEP;  // wave-uniform
-  if constexpr (KFULL) {
-    s.stage_regs[SET][i] = *reinterpret_cast<const u32x4*>(base + s.goff[i]);
-  } else {
-    const bool valid = kb * KSTEP + s.chunk_byte < s.K;  // past the end of the row: read chunk 0 instead, then zero
-    const u32x4 v = *reinterpret_cast<const u32x4*>(base + (valid ? s.goff[i] : s.goff[i] - (uint32_t)s.chunk_byte));
-    s.stage_regs[SET][i] = valid ? v : u32x4{0, 0, 0, 0};
-  }
+  const bool valid = kb * KSTEP + s.chunk_byte < s.K;  // past the end of the row: read chunk 0 instead, then zero
+  const u32x4 v = *reinterpret_cast<const u32x4*>(base + (valid ? s.goff[i] : s.goff[i] - (uint32_t)s.chunk_byte));
+  s.stage_regs[SET][i] = valid ? v : u32x4{0, 0, 0, 0};
 }
 
 template <int SET>
@@ -84,7 +79,7 @@ __device__ __forceinline__ void load_scale(PipeState& s, int kb) {
 // One K block.  wc: weight fragments of this block (already in registers); wn: receives the next block's.
 // tokb/scb: double-buffered token fragment and its scale; tokb[0]/scb[0] hold token tile 0 of this block on entry
 // and of the next block on exit.
-template <bool KFULL, int SET>
+template <int SET>
 __device__ __forceinline__ void k_block(PipeState& s, uint8_t* smem, float (&acc)[P_NT][P_MT][4], Frag (&wc)[P_NT],
                                         Frag (&wn)[P_NT], Frag (&tokb)[2], float (&scb)[2], int st_cur, int st_next,
                                         int st_write, int kb_load) {
@@ -112,7 +107,7 @@ __device__ __forceinline__ void k_block(PipeState& s, uint8_t* smem, float (&acc
       *reinterpret_cast<u32x4*>(wr + s.wr_off + t * 4096) = s.stage_regs[SET][t];
       if (t == 0) sc_wr[threadIdx.x] = s.stage_sa[SET] * s.stage_sb[SET];
     } else if (t < 2 * P_LOADS) {  // refill it with the block four ahead
-      load_one<KFULL, SET>(s, t - P_LOADS, kb_load);
+      load_one<SET>(s, t - P_LOADS, kb_load);
       if (t == P_LOADS) load_scale<SET>(s, kb_load);
     }
     if (i == 0 && j + 1 < P_MT) {  // next token tile of this block
@@ -142,7 +137,6 @@ __device__ __forceinline__ void k_block(PipeState& s, uint8_t* smem, float (&acc
   }
 }
 
-template <bool KFULL>
 __global__ __launch_bounds__(THREADS) void fp8_gemm_pipelined_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x;
@@ -199,7 +193,7 @@ __global__ __launch_bounds__(THREADS) void fp8_gemm_pipelined_kernel(const GemmP
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
 #pragma unroll
-    for (int i = 0; i < P_LOADS; ++i) load_one<KFULL, 0>(s, i, b);
+    for (int i = 0; i < P_LOADS; ++i) load_one<0>(s, i, b);
     load_scale<0>(s, b);
 #pragma unroll
     for (int i = 0; i < P_LOADS; ++i)
@@ -210,13 +204,13 @@ __global__ __launch_bounds__(THREADS) void fp8_gemm_pipelined_kernel(const GemmP
   // for the loop header from this path agree with those of the back edge
 #pragma unroll
   for (int i = 0; i < P_LOADS; ++i) {
-    load_one<KFULL, 0>(s, i, 2);
+    load_one<0>(s, i, 2);
     if (i == 0) load_scale<0>(s, 2);
   }
   __builtin_amdgcn_sched_barrier(0);  // keep the scheduler from interleaving the two groups
 #pragma unroll
   for (int i = 0; i < P_LOADS; ++i) {
-    load_one<KFULL, 1>(s, i, 3);
+    load_one<1>(s, i, 3);
     if (i == 0) load_scale<1>(s, 3);
   }
   __syncthreads();
@@ -235,15 +229,15 @@ __global__ __launch_bounds__(THREADS) void fp8_gemm_pipelined_kernel(const GemmP
   int st0 = 0, st1 = 1, st2 = 2;  // stage being multiplied, the next one, the one being overwritten
   int kb = 0;
   for (; kb + 1 < nkb; kb += 2) {  // two blocks per trip: the register sets and weight fragments ping-pong
-    k_block<KFULL, 0>(s, smem, acc, w0, w1, tokb, scb, st0, st1, st2, kb + 4);
+    k_block<0>(s, smem, acc, w0, w1, tokb, scb, st0, st1, st2, kb + 4);
     __syncthreads();
-    k_block<KFULL, 1>(s, smem, acc, w1, w0, tokb, scb, st1, st2, st0, kb + 5);
+    k_block<1>(s, smem, acc, w1, w0, tokb, scb, st1, st2, st0, kb + 5);
     __syncthreads();
     const int t = st0;
     st0 = st2, st2 = st1, st1 = t;  // rotate by two
   }
   if (kb < nkb) {  // odd number of blocks
-    k_block<KFULL, 0>(s, smem, acc, w0, w1, tokb, scb, st0, st1, st2, kb + 4);
+    k_block<0>(s, smem, acc, w0, w1, tokb, scb, st0, st1, st2, kb + 4);
   }
 
   // ---- epilogue: lane holds channels n .. n+3 of token m
@@ -269,21 +263,14 @@ int launch_fp8_pipelined(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_n = (p.N + P_BN - 1) / P_BN;
   static bool lds_reserved = false;
   if (!lds_reserved) {
-    for (const void* fn : {reinterpret_cast<const void*>(fp8_gemm_pipelined_kernel<true>),
-                           reinterpret_cast<const void*>(fp8_gemm_pipelined_kernel<false>)}) {
-      hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P_LDS);
-      if (e != hipSuccess) {
-        set_error("%s: cannot reserve %zu bytes of LDS: %s", what, P_LDS, hipGetErrorString(e));
-        return MI355_ERR_LAUNCH;
-      }
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fp8_gemm_pipelined_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)P_LDS);
+    if (e != hipSuccess) {
+      set_error("%s: cannot reserve %zu bytes of LDS: %s", what, P_LDS, hipGetErrorString(e));
+      return MI355_ERR_LAUNCH;
     }
     lds_reserved = true;
   }
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
-  if (p.K % KSTEP == 0)
-    hipLaunchKernelGGL(fp8_gemm_pipelined_kernel<true>, grid, dim3(THREADS), P_LDS, stream, p);
-  else
-    hipLaunchKernelGGL(fp8_gemm_pipelined_kernel<false>, grid, dim3(THREADS), P_LDS, stream, p);
+  hipLaunchKernelGGL(fp8_gemm_pipelined_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(THREADS), P_LDS, stream, p);
   return check_launch(what);
 }
 

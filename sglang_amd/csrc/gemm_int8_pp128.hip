@@ -11,8 +11,8 @@
 // 48 KB: the loads of step b + 2 go out in the memory phase of step b into the stage step b - 1 was read from (both groups
 // finished reading it a barrier ago) and have two K steps to land; each wave waits for its own loads of step b + 1 at the
 // end of that phase (s_waitcnt vmcnt(6): the six just issued may be in flight) and the barriers make that hold for all.
-// Arithmetic, fragment layout and swizzle are those of gemm_int8_pp.hip.  Optional split along K (int32 partials to the
-// workspace, the ordered reduce applies the epilogue).  Requires K % 128 == 0, 16-byte aligned rows, row offsets below 4 GiB.
+// Arithmetic, fragment layout and swizzle are those of gemm_int8_pp.hip.  K is not split (gemm_int8_dma3.hip does that).
+// Requires K % 128 == 0, 16-byte aligned rows, row offsets below 4 GiB.
 #include "gemm_common.h"
 
 namespace mi355 {
@@ -99,7 +99,6 @@ __device__ __forceinline__ void compute(const v4i (&w)[J_NT][2], const v4i (&t)[
       for (int i = 0; i < J_NT; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[i][h], t[j][h], acc[i][j], 0, 0, 0);
 }
 
-template <bool SPLIT>
 __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmParams p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -110,13 +109,11 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmPa
 
   const TileCoord tc = tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n);
   const int m0 = tc.tile_m * J_BM, n0 = tc.tile_n * J_BN;
-  const int kb_begin = tc.split * p.kb_per_split;
-  const int kb_end = min(p.kb_total, kb_begin + p.kb_per_split);
-  const int nkb = kb_end - kb_begin;
+  const int nkb = p.kb_total;
 
   JState s;
   s.wave = wave;
-  s.kb_last = kb_end - 1;
+  s.kb_last = nkb - 1;
   s.a_base = p.a;
   s.b_base = p.b;
   {
@@ -149,8 +146,8 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmPa
   v4i w[J_NT][2], t[J_MT][2];
 
   // ---- prologue: steps 0 and 1
-  issue_step(s, j_stage0, kb_begin);
-  issue_step(s, j_stage1, kb_begin + 1);
+  issue_step(s, j_stage0, 0);
+  issue_step(s, j_stage1, 1);
   asm volatile("s_waitcnt vmcnt(6)\n\ts_barrier" ::: "memory");  // step 0 is in LDS (step 1 may be in flight)
   if (grp == 1) compute_end();  // group 1 runs one phase behind group 0
 
@@ -165,38 +162,19 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmPa
 
   int k = 0;
   for (; k + 2 < nkb; k += 3) {
-    k_step(j_stage0, j_stage2, kb_begin + k);
-    k_step(j_stage1, j_stage0, kb_begin + k + 1);
-    k_step(j_stage2, j_stage1, kb_begin + k + 2);
+    k_step(j_stage0, j_stage2, k);
+    k_step(j_stage1, j_stage0, k + 1);
+    k_step(j_stage2, j_stage1, k + 2);
   }
   if (k < nkb) {
-    k_step(j_stage0, j_stage2, kb_begin + k);
-    if (k + 1 < nkb) k_step(j_stage1, j_stage0, kb_begin + k + 1);
+    k_step(j_stage0, j_stage2, k);
+    if (k + 1 < nkb) k_step(j_stage1, j_stage0, k + 1);
   }
   if (grp == 0) compute_end();  // as many barriers as group 1
   // the last requests refetch the last step into rows nobody reads any more: they must not outlive the workgroup's LDS
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- epilogue: lane holds, for token m = 16 j + l16 of the wave's rows, channels 16 i + 4 q + (0..3) of its columns
-  if constexpr (SPLIT) {
-#pragma unroll
-    for (int j = 0; j < J_MT; ++j) {
-      const int m = m0 + grp * J_WM + j * 16 + l16;
-      if (m >= p.M) continue;
-#pragma unroll
-      for (int i = 0; i < J_NT; ++i)
-        {
-          const int n = n0 + wave_n * J_WN + i * 16 + 4 * q;
-          if (n >= p.N) continue;
-          const int nvalid = min(4, p.N - n);
-          int* wsp = reinterpret_cast<int*>(p.ws) + ((int64_t)tc.split * p.M + m) * p.N + n;
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            if (v < nvalid) wsp[v] = acc[i][j][v];
-        }
-    }
-    return;
-  }
   const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
   const bool raw = p.out_dtype == MI355_I32;
   if (out_tile_ok<OUT_INT8>(p)) {
@@ -243,15 +221,12 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp128_kernel(const GemmPa
 
 }  // namespace
 
-// Needs 16-byte aligned rows, K % 128 == 0 and row offsets below 4 GiB.  The caller sets p.splits, p.kb_per_split and p.ws.
+// Needs 16-byte aligned rows, K % 128 == 0 and row offsets below 4 GiB.  K is not split.
 int launch_int8_pp128(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + J_BM - 1) / J_BM;
   p.tiles_n = (p.N + J_BN - 1) / J_BN;
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
-  if (p.splits > 1)
-    hipLaunchKernelGGL(int8_gemm_pp128_kernel<true>, grid, dim3(J_THREADS), 0, stream, p);
-  else
-    hipLaunchKernelGGL(int8_gemm_pp128_kernel<false>, grid, dim3(J_THREADS), 0, stream, p);
+  p.splits = 1, p.kb_per_split = p.kb_total;
+  hipLaunchKernelGGL(int8_gemm_pp128_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(J_THREADS), 0, stream, p);
   return check_launch(what);
 }
 

@@ -575,8 +575,8 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
       }
     }
     if (N % 4 == 0 || dp.efficiency >= route_constants().dma3_min_efficiency) {
-      // INT8: the 128 x 256 tile of this family is the two-phase 128-token kernel (gemm_int8_pp128.hip)
-      r.kernel = (!is_fp8 && dp.bm == 128 && dp.bn == 256) ? RK_PP128 : RK_DMA3;
+      // INT8: the 128 x 256 tile of this family is the two-phase 128-token kernel (gemm_int8_pp128.hip), where K is not split
+      r.kernel = (!is_fp8 && dp.bm == 128 && dp.bn == 256 && dp.splits == 1) ? RK_PP128 : RK_DMA3;
       r.bm = dp.bm, r.bn = dp.bn, r.splits = dp.splits, r.kb_per_split = dp.kb_per_split;
       return r;
     }
@@ -615,7 +615,9 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
     c = choose_decode_tile(kind, M, N, K, r.kernel == RK_DMA3, r.kernel == RK_WAVESPLIT);
   } else {
     TileChoice base{TF_NONE, r.bm, r.bn, r.splits, 0.0};
-    if (r.kernel == RK_DMA3 || (r.kernel == RK_PP128 && r.splits == 1)) base.family = TF_DMA;
+    // (the table's INT8 time of the 128 x 256 tile is the two-phase kernel's, which does not split K: no base where the plan splits it)
+    const bool split_128x256 = kind == GK_INT8 && r.bm == 128 && r.bn == 256 && r.splits > 1;
+    if (r.kernel == RK_PP128 || (r.kernel == RK_DMA3 && !split_128x256)) base.family = TF_DMA;
     if (r.kernel == RK_PINGPONG) base.family = TF_TWO_PHASE;
     c = choose_mid_tile(kind, M, N, K, base);
   }
@@ -731,9 +733,8 @@ int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_giv
         set_error("%s: the 128-token two-phase kernel is built for INT8", what);
         return MI355_ERR_UNSUPPORTED;
       } else {
-        rc = launch_int8_pp128(p, stream, what);
+        return launch_int8_pp128(p, stream, what);
       }
-      break;
     case RK_DMA3:
       if constexpr (IS_FP8) rc = p.ue8m0 ? launch_fp8_dma3_ue8m0(p, r.bm, r.bn, stream, what) : p.row_scale ? launch_fp8_dma3_unit(p, r.bm, r.bn, stream, what) : launch_fp8_dma3(p, r.bm, r.bn, stream, what);
       else rc = launch_int8_dma3(p, r.bm, r.bn, stream, what);

@@ -41,7 +41,7 @@ FP8_ROUTE_SHAPES = [
     # 192-channel tiles (a wave's three channel tiles are 64 channels apart): whole-K and split, a ragged last tile
     (100, 36864, 512), (20, 36864, 1024), (130, 3072, 7168), (300, 3072, 14336), (130, 1000, 896),
     # 256 x 256 two-phase and 256 x 128 pipelined kernels, K a multiple of 128 and not
-    # (the pipelined kernel takes whole-K shapes only where N % 4 != 0 rules the mid-M kernel's split reduce out)
+    # (the pipelined kernel is left K that is no multiple of 128: the mid-M and two-phase kernels take the rest)
     (4096, 4352, 512), (4000, 4300, 400), (4096, 2178, 256), (4000, 2100, 272), (4096, 2176, 256),
     # generic kernel: every token-tile height, aligned and byte-granular loads, whole-K and split
     (7, 1088, 512), (16, 576, 7168), (7, 1096, 512), (16, 584, 7168), (1, 1088, 3884), (17, 384, 2304), (20, 256, 264), (33, 512, 512), (64, 128, 3884),
