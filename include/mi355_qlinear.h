@@ -368,8 +368,10 @@ int mi355_per_tensor_quant_fp8(const void* x, int x_dtype, void* q, float* scale
  *          python/sglang/srt/layers/quantization/fp8_utils.py:565-853).
  *   a [M, K] e4m3fn row stride lda;  b [N, K] e4m3fn row stride ldb (the reference's column-major mat_b [K, N]);
  *   sa [M], sb [N] fp32 contiguous; bias NULL or [N] in the output dtype; out [M, N] BF16/F16 row stride ldo.
- *   It runs on the blockwise kernels (token scale applied when a 128-wide K block is promoted, channel scale and bias
- *   in the epilogue); workspace as for mi355_fp8_blockwise_mm.
+ *   The two-phase, mid-M and wave-split tiles accumulate without scales and apply both, and the bias, in the epilogue (or
+ *   in the ordered reduce of a split K); the streaming, register wave-split, pipelined and generic kernels run as for the
+ *   blockwise GEMM: token scale applied when a 128-wide K block is promoted, channel scale and bias in the epilogue.
+ *   mi355_fp8_scaled_mm_plan names the kernel.
  */
 size_t mi355_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const float* sb, const void* bias, void* out,

@@ -1,10 +1,13 @@
-// Every measured constant of the dispatcher's time models, in one place.
+// The measured constants of choose_route (gemm_w8a8.hip), of dma3_plan (gemm_fp8_dma3.hip) and of the one-call linears' choice
+// of a fused quantizer.  What choose_route names is the base; the tile that models faster by tile_choice.h, which has constants
+// of its own, replaces it.
 //
-// choose_route (gemm_w8a8.hip) and dma3_plan (gemm_fp8_dma3.hip) pick a kernel, a tile and a K split by comparing
-// modelled times.  The models' coefficients were fitted to timings on MI355X; they are data, not logic, so they live in
-// this table, each with the measurement it comes from (the rocprofv3 summaries of the same shapes are under profiles/).
-// Run-to-run and box-to-box spread of these timings is +-3 %; tests/test_gemm_routes_cpu.py perturbs every entry by
-// +-10 % through mi355_gemm_plan_perturbed and holds the benchmark shapes on their kernels, or names the measured times
+// Both pick a kernel, a tile and a K split by comparing modelled times.  The coefficients were fitted to timings on MI355X; they
+// are data, not logic, each with the measurement it comes from (rocprofv3 summaries of many of the shapes are under profiles/).
+// Figures of "the mid-M kernel" here are those of the kernel before gemm_dma_tile.h, which these constants were fitted to; they
+// decide where the two lines cross, and tile_choice.h corrects the choice with the present kernel's times.
+// Run-to-run and box-to-box spread of these timings is +-3 %; tests/test_gemm_routes_cpu.py perturbs every entry of both tables
+// by +-10 % through mi355_gemm_plan_perturbed and holds the benchmark shapes on their kernels, or names the measured times
 // of both candidates where a shape sits on a boundary.
 #pragma once
 

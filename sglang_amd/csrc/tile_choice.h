@@ -3,8 +3,10 @@
 //
 // The model was fitted to 60 000 timings of forced tiles (14 to 37 layers of K = 256 .. 18432 by N = 192 .. 36864, 1 to 4096
 // tokens, all tiles and splits, weights rotated out of the caches, and results too where they are large): 4 % root mean square for
-// the mid-M tiles, 6 % for the wave-split ones; its choice is 1.5 to 2 % slower than the best measured tile on average (geometric
-// mean over 2100 shapes), where the constants table alone was 16 to 25 % slower.
+// the mid-M tiles, 6 % for the wave-split ones.  With larger operands than those shapes had, the wave-split tiles take 1.1 to 1.5
+// times the modelled time: the limits below lie where they stop being the faster ones.
+// The route that runs against the constants table alone, 720 random shapes (profiles/tile_choice_random_shapes.txt): 16 % faster for
+// FP8, 18 % with packed exponents, 13 % per token, 19 % for INT8 (geometric means); more than 5 % slower at 34 shapes, by up to 15 %.
 #pragma once
 
 #include <algorithm>

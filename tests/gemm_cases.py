@@ -34,7 +34,7 @@ FP8_ROUTE_SHAPES = [
     # 192-channel tiles, instead of the split streaming kernel with 128- and 256-channel tiles
     (4, 36864, 7168), (13, 36864, 7168), (16, 24576, 1536), (14, 32768, 2048), (16, 49152, 2048),
     # K blocks left over after whole trips over the stages that no shape above has: 64 x 192 (four stages) 3; 128 x 128 (four) 2 and
-    # 3; 128 x 192 and 128 x 256 (three; loader waves) 0
+    # 3; 128 x 192 and 128 x 256 (three) 0
     (20, 36864, 896), (100, 32768, 768), (100, 32768, 896), (100, 36864, 768), (300, 16384, 768),
     # small tiles with more workgroups than CUs: 64 x 192 and 128 x 128
     (135, 49152, 1024), (198, 36864, 1024),
