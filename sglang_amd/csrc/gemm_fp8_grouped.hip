@@ -15,7 +15,7 @@
 //   2. fp8_grouped_pp_kernel (gemm_fp8_pp.hip), the two-phase 256 x 256 tile kernel, over the first table, then
 //      fp8_grouped_dma_kernel (gemm_fp8_dma3.hip), the mid-M tile of 64 or 128 tokens x 128 or 256 channels, over the second:
 //      one workgroup per (token tile, channel tile).  The first launch is left out when no expert can have more than
-//      128 rows, and where small tiles alone model faster (grouped_run): then every row goes to the second table.
+//      128 rows, and where small tiles alone model faster (choose_grouped_run): then every row goes to the second table.
 // Where the reference takes device arrays of per-expert pointers, strides and scale layouts as scratch that its own
 // set-up kernel fills, this interface takes the base pointers and strides and keeps its scratch in the workspace.
 #include <cmath>
