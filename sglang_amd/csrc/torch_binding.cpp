@@ -900,22 +900,22 @@ bool is_pair_of_128(PyObject* o) {
   return true;
 }
 
-// Whether an operator called on `t` here and now would end in the CUDA kernel itself.  A fast path launches kernels without
+// Whether an operator called on tensors with these keys here and now would end in the CUDA kernel itself.  A fast path launches kernels without
 // the dispatcher, so whoever listens there would see its allocations and not what fills them: modes, tracers and functional
-// wrappers (vmap, grad) announce themselves in the thread's or the tensor's key set, function modes in a state of their own.
+// wrappers (vmap, grad) announce themselves in the thread's or a tensor's key set, function modes in a state of their own.
 // Autograd and autocast keys may be set: the operators have no formula for either, and the calls record nothing with them.
-bool plain_dispatch(const Tensor& t) {
+bool plain_dispatch(c10::DispatchKeySet of_tensors) {
   using c10::DispatchKey;
   constexpr c10::DispatchKeySet direct({DispatchKey::Dense, DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView,
                                         DispatchKey::AutogradFunctionality, DispatchKey::AutocastCUDA, DispatchKey::AutocastCPU});
   const auto tls = c10::impl::tls_local_dispatch_key_set();
-  const c10::DispatchKeySet keys = ((t.key_set() | tls.included_) - tls.excluded_) - direct;
+  const c10::DispatchKeySet keys = ((of_tensors | tls.included_) - tls.excluded_) - direct;
   return (keys.raw_repr() & ~c10::full_backend_mask) == 0 && !at::impl::torch_function_mode_enabled();
 }
 
 PyObject* plain_dispatch_py(PyObject*, PyObject* t) {
   HANDLE_TH_ERRORS
-  return PyBool_FromLong(plain_dispatch(as_tensor(t)));
+  return PyBool_FromLong(plain_dispatch(as_tensor(t).key_set()));
   END_HANDLE_TH_ERRORS
 }
 
@@ -929,14 +929,19 @@ template <class R, class... A, R (*FN)(A...), int BLOCK> struct Try<FN, BLOCK> {
     TORCH_CHECK_TYPE(n == COUNT, COUNT, " arguments are expected, got ", n);
     PyObject* rest[sizeof...(A)];
     int at = 0;
+    c10::DispatchKeySet keys;  // of all tensors together: the thread's state is looked up once a call
     for (int i = 0; i < COUNT; ++i) {
       if (i == BLOCK) {
         if (!is_pair_of_128(args[i])) Py_RETURN_NONE;
         continue;
       }
-      if (THPVariable_Check(args[i]) && !(THPVariable_CheckExact(args[i]) && plain_dispatch(THPVariable_Unpack(args[i])))) Py_RETURN_NONE;
+      if (THPVariable_Check(args[i])) {
+        if (!THPVariable_CheckExact(args[i])) Py_RETURN_NONE;
+        keys = keys | THPVariable_Unpack(args[i]).key_set();
+      }
       rest[at++] = args[i];
     }
+    if (!plain_dispatch(keys)) Py_RETURN_NONE;
     return Call<FN>::py(self, rest, (Py_ssize_t)sizeof...(A));
     END_HANDLE_TH_ERRORS
   }

@@ -10,7 +10,7 @@ from __future__ import annotations
 from typing import List, Optional, Tuple
 
 import torch
-from torch.compiler import is_compiling
+from torch.compiler import is_dynamo_compiling
 
 from . import _lib, _native, ops
 from .sgl_kernel import _v2_by_environment, sgl_per_token_group_quant_8bit
@@ -75,7 +75,7 @@ def _per_token_group_quant_8bit_raw(
     ``s`` up to a power of two and repacks the fp32 scales with DeepGEMM's
     ``transform_sf_into_required_layout``; here the kernel writes that packed int32 layout
     directly (four exponent bytes per word, words column-major and padded to 4 rows)."""
-    if not is_compiling():
+    if not is_dynamo_compiling():
         out = _native.try_group_quant(x, group_size, eps, dtype, column_major_scales, scale_tma_aligned or scale_ue8m0, scale_ue8m0,
                                       True, False)
         if out is not None:
@@ -148,7 +148,7 @@ def _per_token_group_quant_8bit_fuse_silu_and_mul(
     assert scale_tma_aligned
     assert scale_ue8m0
     assert group_size == 128
-    if dst_dtype == fp8_dtype and not is_compiling():
+    if dst_dtype == fp8_dtype and not is_dynamo_compiling():
         out = _native.try_silu_quant(x, masked_m)
         if out is not None:
             return out
@@ -210,7 +210,7 @@ def sglang_per_token_group_quant_fp8(
     """fp8_kernel.py:477-527: allocate outputs, then ``sgl_per_token_group_quant_8bit``."""
     if enable_v2 is None:
         enable_v2 = _v2_by_environment()
-    if is_compiling():
+    if is_dynamo_compiling():
         pass
     elif fuse_silu_and_mul:
         if (enable_v2 and group_size == 128 and abs(1e-10 - eps) < 1e-13 and column_major_scales and scale_tma_aligned and scale_ue8m0):

@@ -26,7 +26,7 @@ import functools
 from typing import Callable, List, Optional
 
 import torch
-from torch.compiler import is_compiling
+from torch.compiler import is_dynamo_compiling
 
 from . import _lib, _native, ops
 from .fp8_kernel import (
@@ -79,7 +79,7 @@ def triton_w8a8_block_fp8_linear(
 ) -> torch.Tensor:
     """fp8_utils.py:281-301: row-major-scale quantizer (`x * (1 / s)`), the ragged-shape matmul, bias on the rounded output."""
     assert input_scale is None
-    if not is_compiling():
+    if not is_dynamo_compiling():
         output = _native.try_block_linear(input, weight, block_size, weight_scale, bias, True)
         if output is not None:
             return output
@@ -106,7 +106,7 @@ def cutlass_w8a8_block_fp8_linear_with_fallback(
     """fp8_utils.py:184-214: M-major-scale quantizer (`x / s`), `fp8_blockwise_scaled_mm` on the transposed views, bias on
     the rounded output; shapes with N or K not a multiple of 128 go to the Triton wrapper."""
     assert input_scale is None
-    if not is_compiling():
+    if not is_dynamo_compiling():
         output = _native.try_block_linear(input, weight, block_size, weight_scale, bias, False)
         if output is not None:
             return output
@@ -180,7 +180,7 @@ def deepgemm_w8a8_block_fp8_linear_with_fallback(
     assert input_scale is None
     if weight_scale.dtype != torch.int32 or input.dtype != torch.bfloat16 or weight.shape[1] % 128 != 0:
         return triton_w8a8_block_fp8_linear(input, weight, block_size, weight_scale, input_scale, bias)
-    if not is_compiling():
+    if not is_dynamo_compiling():
         out = _native.try_block_linear_ue8m0(input, weight, block_size, weight_scale, bias)
         if out is not None:
             return out
@@ -223,7 +223,7 @@ def apply_fp8_linear(
     default; a static per-tensor `input_scale` is repeated per token (:748-753); with `compressed_tensor_quant` the
     quantizer is `scaled_fp8_quant` (:598-603), whose per-tensor scale is repeated likewise for the GEMM.
     `input_scale_ub` is accepted and unused, as in the reference (:570 is its only mention there)."""
-    if not compressed_tensor_quant and not is_compiling():
+    if not compressed_tensor_quant and not is_dynamo_compiling():
         out = _native.try_token_linear(input, weight, weight_scale, input_scale, bias)
         if out is not None:
             return out

@@ -7,7 +7,7 @@ import os
 from typing import Optional
 
 import torch
-from torch.compiler import is_compiling
+from torch.compiler import is_dynamo_compiling
 
 from . import _native, ops
 
@@ -16,7 +16,7 @@ ops.register()
 
 def _v2_by_environment() -> bool:
     """SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2 with the truth values of sglang.srt.utils.get_bool_env_var."""
-    if is_compiling():  # (the tracer can follow this, and not a C function)
+    if is_dynamo_compiling():  # (the tracer can follow this, and not a C function)
         return os.getenv("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2", "false").lower() in ("true", "1")
     return _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
 

@@ -6,7 +6,7 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
-from torch.compiler import is_compiling
+from torch.compiler import is_dynamo_compiling
 
 from . import _native, ops
 from .int8_kernel import per_token_quant_int8
@@ -18,7 +18,7 @@ def apply_w8a8_int8_linear(
 ) -> torch.Tensor:
     """`weight` [K, N] int8, column-major (the checkpoint's [N, K] tensor transposed once at load time,
     w8a8_int8.py:353); `weight_scale` N fp32 values; `x` [..., K]."""
-    if not is_compiling():
+    if not is_dynamo_compiling():
         out = _native.try_int8_linear(x, weight, weight_scale, bias)  # the operands a served model meets, in one native call
         if out is not None:
             return out
