@@ -208,9 +208,10 @@ def sglang_per_token_group_quant_fp8(
     enable_v2: Optional[bool] = None,
 ):
     """fp8_kernel.py:477-527: allocate outputs, then ``sgl_per_token_group_quant_8bit``."""
+    traced = is_dynamo_compiling()
     if enable_v2 is None:
-        enable_v2 = _v2_by_environment()
-    if is_dynamo_compiling():
+        enable_v2 = _v2_by_environment() if traced else _native.env_flag("SGLANG_PER_TOKEN_GROUP_QUANT_8BIT_V2")
+    if traced:
         pass
     elif fuse_silu_and_mul:
         if (enable_v2 and group_size == 128 and abs(1e-10 - eps) < 1e-13 and column_major_scales and scale_tma_aligned and scale_ue8m0):
