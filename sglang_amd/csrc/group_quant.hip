@@ -26,6 +26,8 @@ struct QuantParams {
   uint8_t* q;
   void* s;
   uint32_t num_groups;     // M * K / group
+  uint32_t rows;           // M
+  FastDiv tiles_per_row;   // GM_COLS: workgroups along a row
   FastDiv groups_per_row;  // K / group
   float eps, qmin, qmax, inv_qmax, pow2_floor;
   int64_t s_stride_row, s_stride_col;
@@ -111,13 +113,22 @@ __device__ __forceinline__ float div_shared(float x, float s, float r) {
   return q;
 }
 
-// T: element tag; LPG lanes per group; ITERS 16-byte vectors per lane and group.
-// QUAD (UNROLL == 4 only): the four groups of a thread are four CONSECUTIVE groups of one row, so their scales leave as
-// one 16-byte store (fp32, row-major) or one 32-bit word (packed UE8M0) instead of four 4-byte or 1-byte stores; the host
-// selects it when groups per row and the group count are multiples of four and the scale layout is one of those two.
-template <typename T, int LPG, int ITERS, int MODE, bool UE8M0, bool FP8_OUT, int UNROLL, bool QUAD>
+// Which groups a thread takes, and how its scales leave.  Token scales of a GEMM lie M-major (or as packed words, M-major): with
+// groups dealt out along the rows, every scale of a column comes from another workgroup, mostly on another XCD, so each 128-byte line
+// of scales is written in pieces from several L2s.  GM_COLS gives a workgroup sixteen (or 32) neighbouring rows instead.
+//   us, 16-bit input, groups of 128, GM_FLAT or GM_QUAD with four groups a thread / this file's choice below:
+//   M-major fp32 scales: 904 x 7168 6.8 / 5.8, 4096 x 7168 21.4 / 18.5, 16384 x 7168 64.3 / 60.0;  packed words: 5103 x 18048 48.2 / 46.0
+enum GroupMap {
+  GM_FLAT,  // groups of the flat index, GROUPS_PER_PASS apart
+  GM_QUAD,  // four consecutive groups of a row, whose scales leave as one 16-byte store (fp32, row-major) or one 32-bit word
+  GM_COLS,  // a workgroup takes GROUPS_PER_PASS * RU rows x UNROLL / RU groups; four consecutive exponents leave as one word
+};
+
+// T: element tag; LPG lanes per group; ITERS 16-byte vectors per lane and group; UNROLL groups per thread.
+template <typename T, int LPG, int ITERS, int MODE, bool UE8M0, bool FP8_OUT, int UNROLL, GroupMap MAP, int RU = 1>
 __global__ __launch_bounds__(256) void group_quant_kernel(const QuantParams p) {
-  static_assert(!QUAD || UNROLL == 4, "a quad is four groups");
+  static_assert((MAP != GM_QUAD || UNROLL == 4) && UNROLL % RU == 0, "a quad is four groups");
+  constexpr bool QUAD = MAP == GM_QUAD, COLS = MAP == GM_COLS, WORD = COLS && UE8M0 && UNROLL == 4 && RU == 1;
   constexpr int VEC = Elem<T>::VEC;
   constexpr int GROUP = LPG * ITERS * VEC;
   constexpr int GROUPS_PER_PASS = 256 / LPG;
@@ -126,14 +137,20 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const QuantParams p) {
   // QUAD: quads past the end redo the last quad (same values to the same addresses), like single groups do below
   const uint32_t g_first = QUAD ? min(blockIdx.x * GROUPS_PER_PASS + threadIdx.x / LPG, p.num_groups / 4 - 1) * 4
                                 : blockIdx.x * (GROUPS_PER_PASS * UNROLL) + threadIdx.x / LPG;
-  float quad_scale[QUAD ? 4 : 1];
+  const uint32_t gpr = p.groups_per_row.div;
+  uint32_t tile_m = 0, tile_k = 0;
+  if constexpr (COLS) tile_m = fastdiv(blockIdx.x, p.tiles_per_row), tile_k = blockIdx.x - tile_m * p.tiles_per_row.div;
+  auto row_of = [&](int u) { return min(tile_m * (GROUPS_PER_PASS * RU) + (u % RU) * GROUPS_PER_PASS + threadIdx.x / LPG, p.rows - 1); };
+  auto kg_of = [&](int u) { return min(tile_k * (UNROLL / RU) + u / RU, gpr - 1); };
+  auto group_of = [&](int u) { return COLS ? row_of(u) * gpr + kg_of(u) : min(g_first + u * G_STEP, p.num_groups - 1); };
+  float quad_scale[QUAD || WORD ? 4 : 1];
 
   u32x4 raw[UNROLL][ITERS];
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
     // Past the last group the lanes redo the last group (same values to the same addresses): the body stays free of
     // branches, which keeps the stores nontemporal and the loop fully unrolled.
-    const uint32_t g = min(g_first + u * G_STEP, p.num_groups - 1);
+    const uint32_t g = group_of(u);
     const u32x4* src = reinterpret_cast<const u32x4*>(p.x) + (size_t)g * (LPG * ITERS) + lane;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -143,7 +160,7 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const QuantParams p) {
 
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
-    const uint32_t g = min(g_first + u * G_STEP, p.num_groups - 1);
+    const uint32_t g = group_of(u);
     float v[ITERS][VEC];
     float amax = p.eps;
 #pragma unroll
@@ -206,11 +223,11 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const QuantParams p) {
         else
           store_nt(d, w[0]);
       }
-      if constexpr (QUAD) {
+      if constexpr (QUAD || WORD) {
         quad_scale[u] = s_val;
       } else if (lane == 0) {
-        const uint32_t row = fastdiv(g, p.groups_per_row);
-        const uint32_t kg = g - row * p.groups_per_row.div;
+        const uint32_t row = COLS ? row_of(u) : fastdiv(g, p.groups_per_row);
+        const uint32_t kg = COLS ? kg_of(u) : g - row * p.groups_per_row.div;
         if constexpr (UE8M0) {
           uint8_t* sb = reinterpret_cast<uint8_t*>(p.s) + (size_t)(kg >> 2) * (size_t)p.s_stride_col * 4u +
                         (size_t)row * 4u + (kg & 3u);
@@ -223,51 +240,78 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const QuantParams p) {
       }
     }
   }
-  if constexpr (QUAD) {
+  if constexpr (WORD || (QUAD && UE8M0)) {
     if (lane == 0) {
-      if constexpr (UE8M0) {
-        const uint32_t row = fastdiv(g_first, p.groups_per_row);
-        const uint32_t kg = g_first - row * p.groups_per_row.div;  // a multiple of four
-        uint32_t word = 0;
+      // QUAD: whole words; WORD: groups past the end of the row are the word's padding, zero
+      const uint32_t row = WORD ? row_of(0) : fastdiv(g_first, p.groups_per_row);
+      const uint32_t kw = WORD ? tile_k : (g_first - row * gpr) >> 2;
+      uint32_t word = 0;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) word |= (__float_as_uint(quad_scale[u]) >> 23) << (8 * u);
-        *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(p.s) + (size_t)(kg >> 2) * (size_t)p.s_stride_col * 4u +
-                                     (size_t)row * 4u) = word;
-      } else {
-        typedef float f32x4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.s) + g_first) =
-            f32x4{quad_scale[0], quad_scale[1], quad_scale[2], quad_scale[3]};
-      }
+      for (int u = 0; u < 4; ++u) word |= QUAD || kw * 4 + u < gpr ? (__float_as_uint(quad_scale[u]) >> 23) << (8 * u) : 0u;
+      *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(p.s) + (size_t)kw * (size_t)p.s_stride_col * 4u + (size_t)row * 4u) = word;
+    }
+  } else if constexpr (QUAD) {
+    if (lane == 0) {
+      typedef float f32x4 __attribute__((ext_vector_type(4)));
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.s) + g_first) =
+          f32x4{quad_scale[0], quad_scale[1], quad_scale[2], quad_scale[3]};
     }
   }
 }
 
-template <typename T, int LPG, int ITERS, int MODE, bool UE8M0, bool FP8_OUT>
-int launch(const QuantParams& p, hipStream_t stream) {
-  // Fewer groups per thread when each group already spans several vectors per lane.
-  constexpr int UNROLL = (ITERS >= 4) ? 1 : (ITERS == 2 ? 2 : 4);
-  constexpr int GROUPS_PER_BLOCK = (256 / LPG) * UNROLL;
-  const uint32_t blocks = (p.num_groups + GROUPS_PER_BLOCK - 1) / GROUPS_PER_BLOCK;
-  if constexpr (UNROLL == 4) {
-    // four consecutive groups of a row per thread when their scales are adjacent in memory: fp32 scales indexed by the
-    // flat group number, or packed exponents (four k-groups per word)
-    const uint32_t gpr = p.groups_per_row.div;
-    const bool flat_f32 = !UE8M0 && p.s_stride_col == 1 && p.s_stride_row == (int64_t)gpr &&
-                          (reinterpret_cast<uintptr_t>(p.s) & 15) == 0;
-    const bool packed = UE8M0 && (reinterpret_cast<uintptr_t>(p.s) & 3) == 0;
-    if (gpr % 4 == 0 && p.num_groups % 4 == 0 && (flat_f32 || packed)) {
-      hipLaunchKernelGGL((group_quant_kernel<T, LPG, ITERS, MODE, UE8M0, FP8_OUT, UNROLL, true>), dim3(blocks), dim3(256), 0,
-                         stream, p);
-      return check_launch("mi355_group_quant_8bit");
-    }
+// How many groups a thread takes, for groups of 128 16-bit values (us on both sides of each line; 16 lanes and one load a group).
+// One, where there are too few groups to fill the chip several times over: the kernel is one chain of latencies then.
+//   row-major fp32: 387 x 1536 four 3.0 / one 2.2, 200 x 18432 4.15 / 4.01, 1024 x 4096 4.17 / 4.17, 4096 x 1536 5.3 / 5.5;
+//   rows that are not whole quads of groups: 14768 x 768 9.7 / 8.6, 6000 x 3968 16.4 / 15.9, 5103 x 18048 48.5 / 53.8
+constexpr uint32_t FLAT_ONE_MAX_GROUPS = 32768, FLAT_ONE_MAX_GROUPS_NO_QUADS = 200000;
+//   M-major fp32, one flat / one of a column: 387 x 1536 2.22 / 2.41, 3001 x 512 2.82 / 2.80, 200 x 18432 4.36 / 4.02;
+//   packed words: 200 x 18432 3.56 / 3.51, 904 x 7168 5.5 / 5.3
+constexpr uint32_t COLS_MIN_GROUPS_F32 = 12288, COLS_MIN_GROUPS_WORDS = 32768;
+//   a column's one / two rows x two: 1000 x 16384 11.2 / 11.5, 6000 x 3968 15.8 / 15.2, 5103 x 18048 51.7 / 48.6;
+//   two x two / one row x four: 5103 x 18048 48.6 / 49.2, 16384 x 7168 62.2 / 60.0;
+//   packed words, one / four: 1000 x 16384 10.2 / 10.3, 6000 x 3968 14.6 / 14.2, 16384 x 7168 61.6 / 57.7
+constexpr uint32_t COLS_ONE_MAX_GROUPS = 160000, COLS_TWO_MAX_GROUPS = 800000;
+
+template <typename T, int LPG, int ITERS, int MODE, bool UE8M0, bool FP8_OUT, int UNROLL, GroupMap MAP, int RU = 1>
+int launch_map(QuantParams& p, hipStream_t stream) {
+  constexpr uint32_t PASS = 256 / LPG;
+  uint32_t blocks = (p.num_groups + PASS * UNROLL - 1) / (PASS * UNROLL);
+  if constexpr (MAP == GM_COLS) {
+    p.tiles_per_row = make_fastdiv((p.groups_per_row.div + UNROLL / RU - 1) / (UNROLL / RU));
+    blocks = p.tiles_per_row.div * ((p.rows + PASS * RU - 1) / (PASS * RU));
   }
-  hipLaunchKernelGGL((group_quant_kernel<T, LPG, ITERS, MODE, UE8M0, FP8_OUT, UNROLL, false>), dim3(blocks), dim3(256), 0,
-                     stream, p);
+  hipLaunchKernelGGL((group_quant_kernel<T, LPG, ITERS, MODE, UE8M0, FP8_OUT, UNROLL, MAP, RU>), dim3(blocks), dim3(256), 0, stream, p);
   return check_launch("mi355_group_quant_8bit");
 }
 
+template <typename T, int LPG, int ITERS, int MODE, bool UE8M0, bool FP8_OUT>
+int launch(QuantParams& p, hipStream_t stream) {
+#define MI355_LAUNCH(...) launch_map<T, LPG, ITERS, MODE, UE8M0, FP8_OUT, __VA_ARGS__>(p, stream)
+  // Fewer groups per thread when each group already spans several vectors per lane.
+  constexpr int UNROLL = (ITERS >= 4) ? 1 : (ITERS == 2 ? 2 : 4);
+  const uint32_t groups = p.num_groups, gpr = p.groups_per_row.div;
+  const bool quads = gpr % 4 == 0 && groups % 4 == 0 &&
+                     (UE8M0 ? (reinterpret_cast<uintptr_t>(p.s) & 3) == 0
+                            : p.s_stride_col == 1 && p.s_stride_row == (int64_t)gpr && (reinterpret_cast<uintptr_t>(p.s) & 15) == 0);
+  if constexpr (LPG == 16 && ITERS == 1 && Elem<T>::VEC == 8) {
+    const bool columns = p.rows >= 16 && (UE8M0 ? (reinterpret_cast<uintptr_t>(p.s) & 3) == 0 && groups >= COLS_MIN_GROUPS_WORDS
+                                                : p.s_stride_row < p.s_stride_col && groups >= COLS_MIN_GROUPS_F32);
+    if (columns) {
+      if (groups < COLS_ONE_MAX_GROUPS) return MI355_LAUNCH(1, GM_COLS);
+      if constexpr (!UE8M0)
+        if (groups < COLS_TWO_MAX_GROUPS) return MI355_LAUNCH(4, GM_COLS, 2);
+      return MI355_LAUNCH(4, GM_COLS);
+    }
+    if (groups < (quads ? FLAT_ONE_MAX_GROUPS : FLAT_ONE_MAX_GROUPS_NO_QUADS)) return MI355_LAUNCH(1, GM_FLAT);
+  }
+  if constexpr (UNROLL == 4)
+    if (quads) return MI355_LAUNCH(4, GM_QUAD);
+  return MI355_LAUNCH(UNROLL, GM_FLAT);
+#undef MI355_LAUNCH
+}
+
 template <typename T, int LPG, int ITERS>
-int dispatch_mode(const QuantParams& p, int mode, bool ue8m0, bool fp8_out, hipStream_t stream) {
+int dispatch_mode(QuantParams& p, int mode, bool ue8m0, bool fp8_out, hipStream_t stream) {
 #define MI355_CASE(MODE_, UE_, FP8_)                                     \
   if (mode == MODE_ && ue8m0 == UE_ && fp8_out == FP8_) {                \
     return launch<T, LPG, ITERS, MODE_, UE_, FP8_>(p, stream);           \
@@ -288,7 +332,7 @@ int dispatch_mode(const QuantParams& p, int mode, bool ue8m0, bool fp8_out, hipS
 }
 
 template <typename T>
-int dispatch_shape(const QuantParams& p, int nvec, int mode, bool ue8m0, bool fp8_out, hipStream_t stream) {
+int dispatch_shape(QuantParams& p, int nvec, int mode, bool ue8m0, bool fp8_out, hipStream_t stream) {
   switch (nvec) {
     case 1: return dispatch_mode<T, 1, 1>(p, mode, ue8m0, fp8_out, stream);
     case 2: return dispatch_mode<T, 2, 1>(p, mode, ue8m0, fp8_out, stream);
@@ -339,6 +383,7 @@ extern "C" int mi355_group_quant_8bit(const void* x, int x_dtype, void* q, int q
   p.q = static_cast<uint8_t*>(q);
   p.s = s;
   p.num_groups = (uint32_t)num_groups;
+  p.rows = (uint32_t)M;
   p.groups_per_row = make_fastdiv((uint32_t)(K / group));
   p.eps = eps;
   p.qmin = qmin;

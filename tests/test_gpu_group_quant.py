@@ -76,6 +76,14 @@ def test_sgl_kernel_api(gpu, oracle, M, K, enable_v2, layout):
     assert _same_bits(q, q_o), _diff_report(q, q_o)
 
 
+# one shape for every way the groups are dealt out (group_quant.hip, GroupMap and the limits beside it): one group a thread along
+# the rows and by columns, two rows x two groups, one row x four; rows and groups per row that fill no workgroup or word
+@pytest.mark.parametrize("M,K", [(15, 2304), (1001, 1664), (2051, 2176), (2048, 2048), (5001, 4224), (6007, 17280)])
+@pytest.mark.parametrize("layout", ["row", "col", "col_aligned", "ue8m0"])
+def test_group_maps(gpu, oracle, M, K, layout):
+    test_sgl_kernel_api(gpu, oracle, M, K, False, layout)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("group", [16, 32, 64, 128, 256, 512])
 def test_group_sizes_and_input_dtypes(gpu, oracle, dtype, group):
