@@ -58,49 +58,75 @@ __device__ __forceinline__ int in_vgpr(int x) {
 
 // ---- 1 x 128 group quantization inside a GEMM kernel (the one-call linear at decode sizes): 16 lanes hold a group, 8
 // elements each, with the arithmetic of the group quantizer's reference path (amax floored at 1e-10, s = amax / 448,
-// q = e4m3fn(clamp(x / s)), group_quant.hip).
-// max over the 16 lanes of a DPP row
-__device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true)));
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true)));
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true)));
-  return v;
-}
-// x / s, correctly rounded, given r = RN(1 / s): two Markstein steps, as in the group quantizer (group_quant.hip), where
-// the conditions under which this equals the `/` operator are stated and checked.
-__device__ __forceinline__ float div_by_shared(float x, float s, float r) {
-  float q = x * r;
-  q = fmaf(fmaf(-q, s, x), r, q);
-  q = fmaf(fmaf(-q, s, x), r, q);
-  return q;
-}
-// The lane's eight 16-bit elements (raw) of a group spread over its DPP row -> their eight e4m3fn codes and the group's scale
-// (the same value in all 16 lanes).  Every lane of the row must be active.  by_reciprocal: q = x * (1 / s) as the
-// reference's row-major-scale quantizer computes it (fp8_kernel.py:156-158), else the true division of its M-major one.
-__device__ __forceinline__ u32x2 quantize_group_lane(const u32x4& raw, int x_dtype, bool by_reciprocal, float& scale) {
+// q = e4m3fn(clamp(x / s)), group_quant.hip).  A few waves do this for a whole workgroup before (or beside) its K loop, bound by
+// their vector instructions: 66 for the eight elements of a lane.  With compiler-made divisions, the type looked at per element
+// and two refinement steps per quotient it was 128; us, before / now: 7168 -> 384 at 4 tokens 8.2 / 7.5, 4864 -> 704 at 8 9.8 / 8.3,
+// INT8 3584 -> 1536 at 9 9.9 / 7.9, per-token FP8 2048 -> 2048 at 8 7.3 / 6.4.
+template <bool BF16>
+__device__ __forceinline__ void unpack8(const u32x4& raw, float (&v)[8]) {
   const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-  float v[8];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    v[2 * i] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu);
-    v[2 * i + 1] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16);
+    v[2 * i] = BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu);
+    v[2 * i + 1] = BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16);
   }
+}
+// max over the 16 lanes of a DPP row, of results of earlier max instructions (which are no signalling NaNs: the compiler, which cannot
+// know, would quiet every operand first)
+__device__ __forceinline__ float row16_max(float v) {
+#define MI355_ROW_MAX(PERM) asm("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 " PERM " row_mask:0xf bank_mask:0xf bound_ctrl:1" : "+v"(v))
+  MI355_ROW_MAX("quad_perm:[1,0,3,2]");
+  MI355_ROW_MAX("quad_perm:[2,3,0,1]");
+  MI355_ROW_MAX("row_half_mirror");
+  MI355_ROW_MAX("row_mirror");
+#undef MI355_ROW_MAX
+  return v;
+}
+// One Markstein step on q = RN(x * r), r = RN(1 / s): the correctly rounded x / s.  Exhaustively the same as the `/` operator for
+// every significand of a 16-bit x and of s (2^33 pairs), and for s = 448 for every significand of x; the exponents scale both
+// sides alike (no intermediate leaves the normal range; quotients below 2^-11 convert to zero, group_quant.hip).
+__device__ __forceinline__ float div_by_shared(float x, float s, float r) {
+  const float q = x * r;
+  return fmaf(fmaf(-q, s, x), r, q);
+}
+// The lane's eight 16-bit elements (raw) of a group spread over its DPP row -> their eight e4m3fn codes and the group's scale
+// (the same value in all 16 lanes).  Every lane of the row must be active.  by_reciprocal (wave-uniform): q = x * (1 / s) as the
+// reference's row-major-scale quantizer computes it (fp8_kernel.py:156-158), else the true division of its M-major one.
+template <bool BF16>
+__device__ __forceinline__ u32x2 quantize_group_lane(const u32x4& raw, bool by_reciprocal, float& scale) {
+  float v[8];
+  unpack8<BF16>(raw, v);
   float amax = 1e-10f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
   amax = row16_max(amax);
-  const float sc = amax / 448.0f;
-  const float rcp = 1.0f / sc;
+  // (a group with an infinity: scale infinity, reciprocal zero, as the `/` operator has them; the refinements would make NaN of them)
+  const bool finite = __float_as_uint(amax) < 0x7f800000u;
+  const float sc = finite ? div_by_shared(amax, 448.0f, 1.0f / 448.0f) : amax;
+  // RN(1 / s): the hardware's reciprocal and one Newton step, checked against the `/` operator for every significand of s
+  const float r0 = __builtin_amdgcn_rcpf(sc);
+  const float rcp = finite ? fmaf(fmaf(-sc, r0, 1.0f), r0, r0) : r0;
   float t[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) t[e] = fminf(fmaxf(by_reciprocal ? v[e] * rcp : div_by_shared(v[e], sc, rcp), -448.0f), 448.0f);
+  for (int e = 0; e < 8; ++e) t[e] = v[e] * rcp;
+  if (!by_reciprocal) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      t[e] = fmaf(fmaf(-t[e], sc, v[e]), rcp, t[e]);
+      asm volatile("" : "+v"(t[e]));  // a branch, not a selection: the other case does not compute this
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) t[e] = fminf(fmaxf(t[e], -448.0f), 448.0f);
   int c0 = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
   c0 = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c0, true);
   int c1 = __builtin_amdgcn_cvt_pk_fp8_f32(t[4], t[5], 0, false);
   c1 = __builtin_amdgcn_cvt_pk_fp8_f32(t[6], t[7], c1, true);
   scale = sc;
   return u32x2{(uint32_t)c0, (uint32_t)c1};
+}
+__device__ __forceinline__ u32x2 quantize_group_lane(const u32x4& raw, int x_dtype, bool by_reciprocal, float& scale) {
+  return x_dtype == MI355_BF16 ? quantize_group_lane<true>(raw, by_reciprocal, scale) : quantize_group_lane<false>(raw, by_reciprocal, scale);
 }
 
 __device__ __forceinline__ void store_out4(void* out, int out_dtype, int64_t off, const float* r, int nvalid,

@@ -20,15 +20,10 @@ constexpr int WS_QUANT_VECTORS = 10;
 
 __host__ __device__ constexpr int ws_scale_bytes(bool per_group, int M, int kb_total) { return ((per_group ? M * kb_total * 4 : 64) + 15) & ~15; }
 
-template <bool F8>
-__device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, int x_dtype, float mul) {  // per_token_quant.hip, emit_vector
-  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+template <bool F8, bool BF16>
+__device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, float mul) {  // per_token_quant.hip, emit_vector
   float f[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu);
-    f[2 * i + 1] = x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16);
-  }
+  unpack8<BF16>(raw, f);
   uint32_t out[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -39,24 +34,28 @@ __device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, int x_dtype, flo
       int c = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
       out[j] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c, true);
     } else {
-      out[j] = 0;
+      // round half away from zero: 0.5 less one unit keeps the sum's own rounding from lifting values just below a half, and for
+      // every float of magnitude up to 128 the truncated sum is roundf
+      uint32_t c[4];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) out[j] |= ((uint32_t)(int)roundf(f[4 * j + b] * mul) & 0xffu) << (8 * b);
+      for (int b = 0; b < 4; ++b) {
+        const float q = f[4 * j + b] * mul;
+        c[b] = (uint32_t)(int)add_rn(q, copysignf(0.49999997f, q));
+      }
+      const uint32_t lo = __builtin_amdgcn_perm(c[1], c[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(c[3], c[2], 0x04000c0cu);
+      out[j] = lo | hi;
     }
   }
   return u32x2{out[0], out[1]};
 }
-__device__ __forceinline__ float amax8(const u32x4& raw, int x_dtype) {
-  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-  float m = 0.f;
+template <bool BF16>
+__device__ __forceinline__ float amax8(const u32x4& raw) {
+  float f[8], m = 0.f;
+  unpack8<BF16>(raw, f);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m = fmaxf(m, fabsf(x_dtype == MI355_BF16 ? __uint_as_float(w[i] << 16) : f16_bits_to_f32(w[i] & 0xffffu)));
-    m = fmaxf(m, fabsf(x_dtype == MI355_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32(w[i] >> 16)));
-  }
+  for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(f[i]));
   return m;
 }
-
 
 // Piece c (16 bytes of input, 8 values) of the M x K / 8 goes to thread c % NT; 16 consecutive pieces are a group, in the 16 lanes
 // of a DPP row.  Codes go to codes[row * (K + 16) + k] (rows 16 bytes longer than K, so that a fragment's rows do not share banks),
@@ -91,50 +90,55 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, uint8_t* co
   request();
 #pragma unroll
   for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));  // landed
+  // the input's type is looked at once, not per element
+  auto by_type = [&](auto body) {
+    if (p.x_dtype == MI355_BF16) body(std::true_type{});
+    else body(std::false_type{});
+  };
   if constexpr (TQ == TQ_ROW) {
+    by_type([&](auto bf16_c) {
+      constexpr bool BF16 = decltype(bf16_c)::value;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      if (i * NT + wave * 64 < total) {
-        const float m = row16_max(amax8(raw[i], p.x_dtype));
-        if ((lane & 15) == 0 && row_of(i) < p.M) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
+      for (int i = 0; i < NV; ++i) {
+        if (i * NT + wave * 64 < total) {
+          const float m = row16_max(amax8<BF16>(raw[i]));
+          if ((lane & 15) == 0 && row_of(i) < p.M) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
+        }
       }
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (threadIdx.x < 16) {  // the row's scale, and the factor its values are multiplied with in the place of its maximum
+      const float m = row_max[threadIdx.x], sc = IS_FP8 ? m / 448.0f : m / 127.0f;
+      token_scale[threadIdx.x] = sc;
+      row_max[threadIdx.x] = !IS_FP8 ? 127.0f / m : sc == 0.f ? 0.f : 1.0f / sc;
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (threadIdx.x < 16) {
-      const float m = row_max[threadIdx.x];
-      token_scale[threadIdx.x] = IS_FP8 ? m / 448.0f : m / 127.0f;
-    }
   }
+  by_type([&](auto bf16_c) {
+    constexpr bool BF16 = decltype(bf16_c)::value;
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    __builtin_amdgcn_sched_barrier(0);  // one piece's arithmetic at a time: no register may be spilled while loads are in flight
-    if (i * NT + wave * 64 < total) {
-      u32x2 q8;
-      if constexpr (TQ == TQ_ROW) {
-        const float m = row_max[min(row_of(i), 15)];
-        float mul;
-        if constexpr (IS_FP8) {
-          const float sc = m / 448.0f;
-          mul = sc == 0.f ? 0.f : 1.0f / sc;
+    for (int i = 0; i < NV; ++i) {
+      __builtin_amdgcn_sched_barrier(0);  // one piece's arithmetic at a time: no register may be spilled while loads are in flight
+      if (i * NT + wave * 64 < total) {
+        u32x2 q8;
+        if constexpr (TQ == TQ_ROW) {
+          q8 = codes_of_row<IS_FP8, BF16>(raw[i], row_max[min(row_of(i), 15)]);
+        } else if constexpr (UE8M0) {
+          // q = x * 2^-e with e = ceil(log2(max(amax, 1e-10) / 448)): group_quant.hip, MUL with packed exponents
+          const float m = row16_max(fmaxf(amax8<BF16>(raw[i]), 1e-10f));
+          const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
+          const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
+          q8 = codes_of_row<true, BF16>(raw[i], __uint_as_float((uint32_t)(127 - e) << 23));
+          if ((lane & 15) == 0 && row_of(i) < p.M) reinterpret_cast<uint32_t*>(token_scale)[row_of(i) * p.kb_total + (col_of(i) >> 4)] = (uint32_t)(e + 127);
         } else {
-          mul = 127.0f / m;
+          float sc;
+          q8 = quantize_group_lane<BF16>(raw[i], p.x_by_reciprocal != 0, sc);
+          if ((lane & 15) == 0 && row_of(i) < p.M) token_scale[row_of(i) * p.kb_total + (col_of(i) >> 4)] = sc;
         }
-        q8 = codes_of_row<IS_FP8>(raw[i], p.x_dtype, mul);
-      } else if constexpr (UE8M0) {
-        // q = x * 2^-e with e = ceil(log2(max(amax, 1e-10) / 448)): group_quant.hip, MUL with packed exponents
-        const float m = row16_max(fmaxf(amax8(raw[i], p.x_dtype), 1e-10f));
-        const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
-        const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
-        q8 = codes_of_row<true>(raw[i], p.x_dtype, __uint_as_float((uint32_t)(127 - e) << 23));
-        if ((lane & 15) == 0 && row_of(i) < p.M) reinterpret_cast<uint32_t*>(token_scale)[row_of(i) * p.kb_total + (col_of(i) >> 4)] = (uint32_t)(e + 127);
-      } else {
-        float sc;
-        q8 = quantize_group_lane(raw[i], p.x_dtype, p.x_by_reciprocal != 0, sc);
-        if ((lane & 15) == 0 && row_of(i) < p.M) token_scale[row_of(i) * p.kb_total + (col_of(i) >> 4)] = sc;
+        if (row_of(i) < p.M) *reinterpret_cast<u32x2*>(codes + row_of(i) * code_pitch + col_of(i) * 8) = q8;
       }
-      if (row_of(i) < p.M) *reinterpret_cast<u32x2*>(codes + row_of(i) * code_pitch + col_of(i) * 8) = q8;
     }
-  }
+  });
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 

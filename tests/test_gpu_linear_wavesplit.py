@@ -53,3 +53,47 @@ def test_fused_quantizer_of_the_wavesplit_kernel(gpu, oracle, M, N, K, dtype):
     q, s = per_token_quant_int8(xg)
     iw, isc = i_q.to(gpu).t(), i_s.to(gpu)
     assert torch.equal(bits(ops.int8_linear(xg, iw, isc, bias, dtype)), bits(ops.int8_scaled_mm(q, iw, s, isc, dtype, bias)))
+
+
+@pytest.mark.parametrize("kind", ["block", "block_rcp", "ue8m0", "token_fp8", "int8"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fused_quantizer_on_every_16_bit_value(gpu, kind, dtype):
+    """Every bit pattern (infinities and NaN among them) through a one-hot weight: a channel's result is one code times its scales,
+    so the quantizer inside the GEMM has to write the codes and scales of the quantizer kernels."""
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import per_token_group_quant_fp8, sglang_per_token_group_quant_fp8, sglang_per_token_quant_fp8, w8a8_block_fp8_matmul
+    from sglang_amd.fp8_utils import requant_weight_ue8m0
+    from sglang_amd.int8_kernel import per_token_quant_int8
+
+    M, N, K = 16, 2176, 2176
+    assert _lib.linear_plan(kind.split("_rcp")[0], M, N, K)["quantizer"] == "fused"
+    patterns = torch.randperm(65536, generator=torch.Generator().manual_seed(3))
+    patterns = torch.cat([patterns, torch.zeros(2 * M * K - 65536, dtype=torch.int64)]).to(torch.int32).to(torch.int16).view(2, M, K)
+    # a second pair of inputs, all finite and sorted: groups of one magnitude, where the rounding of every quotient shows
+    finite = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
+    finite = finite[torch.isfinite(finite)].float().sort().values.to(dtype)
+    finite = torch.cat([finite, torch.zeros(2 * M * K - finite.numel(), dtype=dtype)]).view(2, M, K)
+    w = torch.eye(N, device=gpu)
+    one, ones = torch.ones(N, device=gpu), torch.ones(N // 128, K // 128, device=gpu)
+    for x in [*patterns.view(dtype), *finite]:
+        if kind == "ue8m0":  # (the two quantizers of this kind clamp a NaN to different ends)
+            x = torch.nan_to_num(x, nan=0.0, posinf=float("inf"), neginf=float("-inf"))
+        xg = x.contiguous().to(gpu)
+        if kind == "int8":
+            wi = w.to(torch.int8).t()
+            q, s = per_token_quant_int8(xg)
+            out, two = ops.int8_linear(xg, wi, one, None, dtype), ops.int8_scaled_mm(q, wi, s, one, dtype, None)
+        elif kind == "token_fp8":
+            wf = w.to(torch.float8_e4m3fn).t()
+            q, s = sglang_per_token_quant_fp8(xg)
+            out, two = ops.fp8_per_token_linear(xg, wf, one, None, dtype), ops.fp8_scaled_mm(q, wf, s, one, dtype, None)
+        elif kind == "ue8m0":
+            w2, words = requant_weight_ue8m0(w.to(torch.float8_e4m3fn), ones, [128, 128])
+            q, s = sglang_per_token_group_quant_fp8(xg, 128, column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=True, enable_v2=True)
+            out, two = ops.block_fp8_linear_ue8m0(xg, w2, words, None, dtype), ops.fp8_blockwise_mm_ue8m0(q, w2, s, words, dtype, None)
+        else:
+            wf, rcp = w.to(torch.float8_e4m3fn), kind == "block_rcp"
+            q, s = per_token_group_quant_fp8(xg, 128, column_major_scales=not rcp)
+            out, two = ops.block_fp8_linear(xg, wf, ones, None, dtype, by_reciprocal=rcp), w8a8_block_fp8_matmul(q, wf, s, ones, [128, 128], dtype)
+        same = (out.view(torch.int16) == two.view(torch.int16)) | (out.isnan() & two.isnan())
+        assert bool(same.all()), (~same).sum().item()
