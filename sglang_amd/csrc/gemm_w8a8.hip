@@ -475,14 +475,14 @@ int launch_tile(GemmParams& p, bool aligned, hipStream_t stream, const char* wha
 
 // Which kernel serves a problem, with which tiling.  run_route decides for the launchers and for the plan queries (choose_linear
 // for the one-call linears), so what a query reports is what runs.
-enum RouteKernel { RK_DECODE = 0, RK_DMA3, RK_PINGPONG, RK_PIPELINED, RK_GENERIC, RK_WAVESPLIT, RK_PP128, RK_WAVESPLIT_TILE };
-const char* const ROUTE_NAMES[] = {"decode", "dma3", "pingpong", "pipelined", "generic", "decode_wavesplit", "pingpong128", "wavesplit_tile"};
+enum RouteKernel { RK_DECODE = 0, RK_DMA3, RK_PINGPONG, RK_PIPELINED, RK_GENERIC, RK_WAVESPLIT, RK_PP128, RK_WAVESPLIT_TILE, RK_RESIDENT };
+const char* const ROUTE_NAMES[] = {"decode", "dma3", "pingpong", "pipelined", "generic", "decode_wavesplit", "pingpong128", "wavesplit_tile", "resident"};
 
 struct Route {
   int kernel;
   int bm, bn;
   int splits, kb_per_split;
-  int groups_per_wg;  // decode only
+  int groups_per_wg;  // decode: channel groups; register wave-split: waves; resident: token ranges
   bool aligned;
 };
 
@@ -605,7 +605,7 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
 }
 
 // The route that runs: choose_route's, or the tile that models faster (tile_choice.h).
-Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
+Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned, bool resident) {
   Route r = choose_route(kind != GK_INT8, M, N, K, lda, ldb, aligned);
   if (!aligned || M * lda >= (1ll << 32) || N * ldb >= (1ll << 32)) return r;
   TileChoice c{TF_NONE, 0, 0, 1, 0.0};
@@ -619,27 +619,41 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
     const bool split_128x256 = kind == GK_INT8 && r.bm == 128 && r.bn == 256 && r.splits > 1;
     if (r.kernel == RK_PP128 || (r.kernel == RK_DMA3 && !split_128x256)) base.family = TF_DMA;
     if (r.kernel == RK_PINGPONG) base.family = TF_TWO_PHASE;
-    c = choose_mid_tile(kind, M, N, K, base);
+    c = choose_mid_tile(kind, M, N, K, base, resident);
   }
   if (c.family == TF_NONE) return r;
-  r.kernel = c.family == TF_DMA ? RK_DMA3 : c.family == TF_WAVESPLIT ? RK_WAVESPLIT_TILE : RK_PINGPONG;
-  r.bm = c.bm, r.bn = c.bn, r.splits = c.splits, r.groups_per_wg = 0;
+  r.kernel = c.family == TF_DMA ? RK_DMA3 : c.family == TF_WAVESPLIT ? RK_WAVESPLIT_TILE : c.family == TF_RESIDENT ? RK_RESIDENT : RK_PINGPONG;
+  r.bm = c.bm, r.bn = c.bn, r.splits = c.splits, r.groups_per_wg = c.ranges;
   const int64_t kb = (K + KSTEP - 1) / KSTEP;
   r.kb_per_split = (int)((kb + c.splits - 1) / c.splits);
   return r;
 }
-Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned) {
-  if (dispatch_perturbed()) return uncached_run_route(kind, M, N, K, lda, ldb, aligned);
+// `resident`: the output and what the epilogue reads are such that the resident-weight kernel can store it (resident_operands_ok).
+Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned, bool resident = true) {
+  if (dispatch_perturbed()) return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident);
   struct Key : ShapeKey {
     int64_t lda, ldb;
-    bool aligned;
-    bool operator==(const Key& o) const { return ShapeKey::operator==(o) && lda == o.lda && ldb == o.ldb && aligned == o.aligned; }
+    bool aligned, resident;
+    bool operator==(const Key& o) const {
+      return ShapeKey::operator==(o) && lda == o.lda && ldb == o.ldb && aligned == o.aligned && resident == o.resident;
+    }
   };
   static thread_local RecentShapes<Key, Route> table;
   if (kind == GK_UE8M0 && M > 16) kind = GK_F32;  // above decode sizes both kinds have one model
-  return table.get(Key{{M, N, K, (int)kind}, lda, ldb, aligned}, [&] { return uncached_run_route(kind, M, N, K, lda, ldb, aligned); });
+  if (M <= 16 || K > RESIDENT_MAX_KBLOCKS * KSTEP) resident = true;  // (does not matter: one entry)
+  return table.get(Key{{M, N, K, (int)kind}, lda, ldb, aligned, resident}, [&] { return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident); });
 }
-int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K) { return run_route(kind, M, N, K, K, K, true).splits; }
+// K splits of the plan, whichever way the output decides
+int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+  const Route r = run_route(kind, M, N, K, K, K, true);
+  return r.kernel == RK_RESIDENT ? run_route(kind, M, N, K, K, K, true, false).splits : r.splits;
+}
+// The resident-weight kernel stores 16 bytes at a time and reads four channel scales (eight bytes of bias) at once.
+bool resident_operands_ok(GemmKind kind, const GemmParams& p) {
+  const float* channel_scales = kind == GK_INT8 ? p.sb : p.col_scale;
+  return (p.out_dtype == MI355_BF16 || p.out_dtype == MI355_F16) && p.ldo % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 &&
+         (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0 && ((kind != GK_UNIT && kind != GK_INT8) || (reinterpret_cast<uintptr_t>(channel_scales) & 15) == 0);
+}
 
 // out[kb * ld_out + m] = sa[m * sa_sm + kb * sa_sk]: token scales re-laid out M-major with a row pitch that is a multiple
 // of four floats.  One 32 x 32 tile per workgroup through LDS, so that reads and writes are both contiguous for either
@@ -675,7 +689,7 @@ bool fp8_scales_conform(const GemmParams& p) {
   return p.sa_sm == 1 && (p.sa_sk & 3) == 0 && p.sa_sk >= ((p.M + 3) & ~3) && (reinterpret_cast<uintptr_t>(p.sa) & 15) == 0;
 }
 bool route_wants_m_major_scales(bool is_fp8, const Route& r) {
-  return is_fp8 && (r.kernel == RK_PINGPONG || r.kernel == RK_DMA3);
+  return is_fp8 && (r.kernel == RK_PINGPONG || r.kernel == RK_DMA3 || r.kernel == RK_RESIDENT);
 }
 
 // Workspace bytes the chosen route needs for this call: a re-laid-out copy of the token scales (first) and split-K
@@ -689,6 +703,11 @@ size_t route_workspace_need(bool is_fp8, const Route& r, const GemmParams& p) {
 bool operands_aligned(const GemmParams& p) {
   return (p.K % 16 == 0) && (p.lda % 16 == 0) && (p.ldb % 16 == 0) && ((reinterpret_cast<uintptr_t>(p.a) & 15) == 0) &&
          ((reinterpret_cast<uintptr_t>(p.b) & 15) == 0);
+}
+
+// The route of a call, once its operands (bias and channel scales too) are in p.
+Route call_route(GemmKind kind, const GemmParams& p) {
+  return run_route(kind, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p), resident_operands_ok(kind, p));
 }
 
 template <bool IS_FP8>
@@ -728,6 +747,10 @@ int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_giv
       if constexpr (IS_FP8)
         return p.ue8m0 ? launch_fp8_wavesplit_tile_ue8m0(p, r.bm, r.bn, stream, what) : p.row_scale ? launch_fp8_wavesplit_tile_unit(p, r.bm, r.bn, stream, what) : launch_fp8_wavesplit_tile(p, r.bm, r.bn, stream, what);
       else return launch_int8_wavesplit_tile(p, r.bm, r.bn, stream, what);
+    case RK_RESIDENT:
+      if constexpr (IS_FP8)
+        return p.ue8m0 ? launch_fp8_resident_ue8m0(p, r.groups_per_wg, stream, what) : p.row_scale ? launch_fp8_resident_unit(p, r.groups_per_wg, stream, what) : launch_fp8_resident(p, r.groups_per_wg, stream, what);
+      else return launch_int8_resident(p, r.groups_per_wg, stream, what);
     case RK_PP128:
       if constexpr (IS_FP8) {
         set_error("%s: the 128-token two-phase kernel is built for INT8", what);
@@ -762,7 +785,7 @@ int run_gemm(GemmParams& p, void* workspace, size_t workspace_bytes_given, hipSt
   const bool aligned = operands_aligned(p);
   const GemmKind kind = !IS_FP8 ? GK_INT8 : p.ue8m0 ? GK_UE8M0 : p.row_scale ? GK_UNIT : GK_F32;
   const Route r = p.x16 != nullptr ? choose_route(IS_FP8, p.M, p.N, p.K, p.lda, p.ldb, aligned, true)
-                                   : run_route(kind, p.M, p.N, p.K, p.lda, p.ldb, aligned);
+                                   : call_route(kind, p);
   return run_gemm<IS_FP8>(p, r, workspace, workspace_bytes_given, stream, what);
 }
 
@@ -789,7 +812,7 @@ const char* const ROUTE_CONSTANT_NAMES[ROUTE_CONSTANT_COUNT] = {
 // UE8M0: the kernels in which the MFMA applies the exponents; the others take them as fp32 scales, unpacked by a launch in front.
 bool applies_exponents(const Route& r, int64_t K) {
   return ((r.kernel == RK_PINGPONG || r.kernel == RK_DMA3 || r.kernel == RK_WAVESPLIT) && K % KSTEP == 0) || r.kernel == RK_DECODE ||
-         r.kernel == RK_WAVESPLIT_TILE;
+         r.kernel == RK_WAVESPLIT_TILE || r.kernel == RK_RESIDENT;
 }
 
 // in the order of TileModel
@@ -803,13 +826,13 @@ std::vector<std::string> tile_constant_names() {
     for (const char* what : {"tile", "block"})
       for (const TileSize& t : MID_TILES) names.push_back(std::string(times) + what + "[" + std::to_string(t.bm) + "x" + std::to_string(t.bn) + "]");
     add(times, {"pp_tile", "pp_block", "pp_busy", "pp_store", "ws_launch", "ws_tile", "ws_kb", "ws_kb_busy", "ws_stream", "ws_stream_us",
-                "ws_result", "ws_norm"});
+                "ws_result", "ws_norm", "rs_launch", "rs_tile", "rs_tile_block", "rs_step", "rs_step_block", "rs_busy"});
   }
   add("limits.", {"margin", "two_phase_margin", "large_weight_margin", "large_weight_max_tokens", "mid_wavesplit_max_weight", "ragged_max_weight",
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
 }
@@ -1040,9 +1063,9 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
   p.bias = bias, p.bias_rounded = bias_rounded;
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
-  const Route r = run_route(GK_UE8M0, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  const Route r = call_route(GK_UE8M0, p);
   const bool words_conform = (sa_sk & 3) == 0 && sa_sk >= ((M + 3) & ~3ll) && (reinterpret_cast<uintptr_t>(sa_words) & 15) == 0;
-  const bool wants_conforming = r.kernel == RK_PINGPONG || r.kernel == RK_DMA3;  // (the decode kernels read the words with ordinary loads: any pitch will do)
+  const bool wants_conforming = r.kernel == RK_PINGPONG || r.kernel == RK_DMA3 || r.kernel == RK_RESIDENT;  // (the decode kernels read the words with ordinary loads: any pitch will do)
   if (applies_exponents(r, K) && (words_conform || !wants_conforming)) {
     // the MFMA applies both exponents itself: no scale arithmetic at all, and the workspace only holds split-K partial sums
     if (r.kernel == RK_PINGPONG) {
@@ -1102,7 +1125,7 @@ extern "C" int mi355_fp8_blockwise_mm_noalloc(const void* a, const void* b, cons
   int rc = fp8_mm_params(what, a, b, sa, sb, out, out_dtype, M, N, K, lda, ldb, sa_sm, sa_sk, sb_sn, sb_sk, ldo, p, empty);
   if (rc != MI355_OK || empty) return rc;
   // the same plan the launcher will make: how many partial-sum bytes it needs
-  Route r = run_route(GK_F32, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
+  Route r = call_route(GK_F32, p);
   if (route_workspace_need(true, r, p) > NOALLOC_SCRATCH_BYTES) r = choose_route(true, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
   const size_t need = route_workspace_need(true, r, p);
   MI355_REQUIRE(need <= NOALLOC_SCRATCH_BYTES, MI355_ERR_WORKSPACE,
@@ -1148,8 +1171,8 @@ extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa
   p.col_scale = sb;
   p.bias = bias;
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
-  const Route r = run_route(GK_UNIT, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p));
-  if (r.kernel == RK_DMA3 || r.kernel == RK_WAVESPLIT_TILE) p.row_scale = sa;  // no scales in the K loop, both in the epilogue (or the reduce)
+  const Route r = call_route(GK_UNIT, p);
+  if (r.kernel == RK_DMA3 || r.kernel == RK_WAVESPLIT_TILE || r.kernel == RK_RESIDENT) p.row_scale = sa;  // no scales in the K loop, both in the epilogue (or the reduce)
   if (r.kernel == RK_PINGPONG && K % KSTEP == 0) {
     // large M: accumulate in the MFMA with unit scales, apply both scales once in the epilogue (the reference's order)
     p.row_scale = sa;

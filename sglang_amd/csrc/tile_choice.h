@@ -26,19 +26,24 @@ struct TileTimes {
   // wave-split tile: rounds of ws_tile + KB of operands * (ws_kb + ws_kb_busy * fill) + kilo-elements of the tile * ws_result,
   // together with the weight stream (ws_norm: how far the two overlap)
   double ws_launch, ws_tile, ws_kb, ws_kb_busy, ws_stream, ws_stream_us, ws_result, ws_norm;
+  // weight in registers (gemm_resident.h): rounds of rs_tile + K blocks * rs_tile_block + steps * (rs_step + K blocks * rs_step_block) *
+  // (1 + rs_busy * fill), a step being 64 tokens (steps of 32 count half)
+  double rs_launch, rs_tile, rs_tile_block, rs_step, rs_step_block, rs_busy;
 };
 constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     1.93, 0.586, 4.31, 0.217, 4.18, -4.54, 1.808, 0.421,
     {2.33, 2.83, 3.02, 3.40, 3.53, 4.64, 2.57, 3.31, 3.96, 4.32, 2.64, 3.53, 4.44},
     {0.219, 0.277, 0.317, 0.385, 0.419, 0.533, 0.288, 0.363, 0.441, 0.532, 0.334, 0.445, 0.535},
     7.88, 0.567, 1.70, 12.5,
-    2.74, 1.041, 0.00591, 0.00334, 5.49, -3.81, 0.253, 1.511};
+    2.74, 1.041, 0.00591, 0.00334, 5.49, -3.81, 0.253, 1.511,
+    3.63, 0.11, 0.406, 0.596, 0.186, 0.733};
 constexpr TileTimes PLAIN_TIMES = {  // FP8 with epilogue scales, INT8
     1.77, 0.777, 3.81, 0.251, 4.55, -2.24, 1.871, 0.402,
     {2.21, 2.72, 3.03, 3.17, 3.76, 4.72, 2.48, 3.12, 3.83, 4.14, 2.81, 3.80, 4.64},
     {0.165, 0.205, 0.240, 0.295, 0.333, 0.432, 0.224, 0.271, 0.339, 0.420, 0.278, 0.347, 0.431},
     8.48, 0.511, 1.70, 10.8,
-    2.71, 1.017, 0.00609, 0.00343, 5.07, -4.41, 0.282, 1.673};
+    2.71, 1.017, 0.00609, 0.00343, 5.07, -4.41, 0.282, 1.673,
+    3.64, 0.01, 0.435, 0.760, 0.217, 0.531};
 static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above follow MID_TILES");
 
 // Where the model is not asked or not trusted; both sides of each line stand beside the function that uses it.
@@ -50,6 +55,7 @@ struct TileLimits {
   double decode_one_turn_min_kblocks = 30.0, decode_one_turn_kblocks = 32.0, decode_one_turn_max_channels = 16384.0, decode_one_turn_max_tokens = 10.0;
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
+  double resident_margin = 0.93;
 };
 struct TileModel {
   TileTimes scaled = SCALED_TIMES, plain = PLAIN_TIMES;
@@ -62,11 +68,12 @@ const TileModel& tile_model();
 namespace {
 
 enum GemmKind { GK_F32, GK_UE8M0, GK_UNIT, GK_INT8 };  // FP8 with block scales, with exponents, with epilogue scales; INT8
-enum TileFamily { TF_NONE, TF_DMA, TF_WAVESPLIT, TF_TWO_PHASE };
+enum TileFamily { TF_NONE, TF_DMA, TF_WAVESPLIT, TF_TWO_PHASE, TF_RESIDENT };
 
 struct TileChoice {
   int family, bm, bn, splits;
   double us;
+  int ranges = 0;  // TF_RESIDENT: workgroups that share a slice of channels
 };
 
 const TileTimes& tile_times(GemmKind kind) { return kind == GK_F32 || kind == GK_UE8M0 ? tile_model().scaled : tile_model().plain; }
@@ -136,9 +143,29 @@ TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+double resident_us(const TileTimes& t, int64_t M, int64_t N, int64_t K, int64_t ranges) {
+  const int64_t kb = K / KSTEP, step = 2 * resident_half_step(false, (int)kb), all = ceil_div(M, step), steps = ceil_div(all, ranges);
+  const double halves = (double)(steps * step) / 64.0;
+  return t.rs_launch + rounds_of(ceil_div(N, RESIDENT_CHANNELS) * ceil_div(all, steps), NUM_CUS, [&](double fill) {
+           return t.rs_tile + (double)kb * t.rs_tile_block + halves * (t.rs_step + (double)kb * t.rs_step_block) * (1.0 + t.rs_busy * fill);
+         });
+}
+// As many ranges of tokens as fill one, two or three rounds of workgroups, whichever models fastest.
+TileChoice best_resident(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+  if (K % KSTEP != 0 || K < 2 * KSTEP || K > RESIDENT_MAX_KBLOCKS * KSTEP || N % 8 != 0) return best;
+  const int64_t slices = ceil_div(N, RESIDENT_CHANNELS), most = ceil_div(M, 2 * resident_half_step(false, (int)(K / KSTEP)));
+  for (int rounds = 1; rounds <= 3; ++rounds) {
+    const int64_t ranges = std::min(std::max<int64_t>(rounds * NUM_CUS / slices, 1), most);
+    const double us = resident_us(t, M, N, K, ranges);
+    if (us < best.us) best = {TF_RESIDENT, 2 * resident_half_step(false, (int)(K / KSTEP)), RESIDENT_CHANNELS, 1, us, (int)ranges};
+  }
+  return best;
+}
+
 // More than 16 tokens, K % 128 == 0, aligned operands: the fastest tile, or TF_NONE where `base`, what the route names (a mid-M
 // tile or the two-phase tile), models within 5 % of it (the two-phase tile 10 %): below that the model does not order two tiles.
-TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base) {
+TileChoice choose_swept_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, double& base_us) {
   const TileTimes& t = tile_times(kind);
   TileChoice best = best_dma_tile(t, M, N, K);
   const TileLimits& l = tile_model().limits;
@@ -156,7 +183,7 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
     const double us = two_phase_us(t, M, N, K);
     if (us < best.us) best = {TF_TWO_PHASE, 256, 256, 1, us};
   }
-  double base_us = 1e30;
+  base_us = 1e30;
   if (base.family == TF_TWO_PHASE) base_us = two_phase_us(t, M, N, K);
   if (base.family == TF_DMA)
     for (int i = 0; i < 13; ++i)
@@ -171,6 +198,18 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
     return TileChoice{TF_NONE, 0, 0, 1, 0.0};
   const double margin = base.family == TF_TWO_PHASE ? l.two_phase_margin : large ? l.large_weight_margin : l.margin;
   return best.us < margin * base_us ? best : TileChoice{TF_NONE, 0, 0, 1, 0.0};
+}
+
+// The same, or the kernel that keeps the weight in registers where the call allows it and it models 7 % faster than what would run.
+// The linears on both sides of the line, us, other / this: block FP8 368 tokens 512 -> 32768 17.4 / 15.5, 430 tokens 512 -> 24576
+// 16.5 / 15.6, 243 tokens 512 -> 6144 8.3 / 8.4, 1340 tokens 512 -> 4096 11.3 / 12.2; 849 tokens 512 -> 6144 10.6 / 11.5;
+// per-token FP8 180 tokens 512 -> 24576 10.2 / 12.0, 624 tokens 640 -> 16384 17.2 / 15.7.
+TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool resident_allowed) {
+  double base_us;
+  const TileChoice c = choose_swept_tile(kind, M, N, K, base, base_us);
+  if (!resident_allowed) return c;
+  const TileChoice r = best_resident(tile_times(kind), M, N, K);
+  return r.us < tile_model().limits.resident_margin * (c.family != TF_NONE ? c.us : base_us) ? r : c;
 }
 
 // K not a multiple of 128 (scales in the epilogue only): the wave-split tile against the generic kernel, which takes at least

@@ -78,6 +78,7 @@ INT8_ROUTE_SHAPES = [
 # of 1 .. 5000 tokens, N up to 320000 and K up to 19000; tests/test_gemm_routes_cpu.py checks that other random shapes add none.
 VARIANT_SHAPES = {
     "fp8": {
+        ("resident", "kb2"): (450, 16472, 256), ("resident", "kb3"): (452, 16528, 384), ("resident", "kb4"): (449, 16424, 512), ("resident", "kb5"): (450, 16504, 640),
         ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
@@ -116,6 +117,7 @@ VARIANT_SHAPES = {
         ("wavesplit_tile", 64, 32, "kfull"): (49, 4358, 128), ("wavesplit_tile", 64, 64, "kfull"): (1637, 291, 512),
     },
     "fp8_ue8m0": {
+        ("resident", "kb2"): (450, 16472, 256), ("resident", "kb3"): (452, 16528, 384), ("resident", "kb4"): (449, 16424, 512), ("resident", "kb5"): (450, 16504, 640),
         ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
@@ -146,6 +148,7 @@ VARIANT_SHAPES = {
         ("wavesplit_tile", 64, 64, "kfull"): (1637, 291, 512),
     },
     "fp8_scaled": {
+        ("resident", "kb2"): (481, 16904, 256), ("resident", "kb3"): (484, 16496, 384), ("resident", "kb4"): (486, 16760, 512), ("resident", "kb5"): (486, 16584, 640),
         ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
@@ -184,6 +187,7 @@ VARIANT_SHAPES = {
         ("wavesplit_tile", 64, 64, "kfull"): (1816, 264, 2176), ("wavesplit_tile", 64, 64, "ktail"): (323, 1536, 16),
     },
     "int8": {
+        ("resident", "kb2"): (481, 16904, 256), ("resident", "kb3"): (484, 16496, 384), ("resident", "kb4"): (486, 16760, 512), ("resident", "kb5"): (542, 16592, 640),
         ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
         ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round"): (1, 16, 128),
         ("decode_wavesplit", "w4", "rounds"): (1, 7936, 17664), ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840),
@@ -275,6 +279,8 @@ def variant_of(plan: dict, K: int):
         return (k, plan["bm"], plan["bn"], "kfull" if K % 128 == 0 else "ktail")
     if k == "pingpong128":
         return (k, sp)
+    if k == "resident":  # a kernel for each number of K blocks
+        return (k, f"kb{K // 128}")
     if k == "dma3":  # "deep": more than three LDS stages (small tiles when every workgroup has a CU to itself, FP8)
         key = (k, plan["bm"], sp) if plan["bn"] == 256 else (k, plan["bm"], sp, f"bn{plan['bn']}")
         return key + ("deep",) if plan["stages"] > 3 else key

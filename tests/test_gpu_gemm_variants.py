@@ -74,3 +74,63 @@ def test_mid_tile_every_remainder(gpu, kind, tile):
             if kind == "fp8":  # (the same plan)
                 assert plan_for("fp8_ue8m0", M, N, 128 * kb)["bm"] == bm
                 check_exact(gpu, "fp8_ue8m0", M, N, 128 * kb)
+
+
+# weight in registers: more steps of tokens than the LDS has stages, a last range with fewer, channels that end inside a slice, and fewer
+# tokens than a step
+@pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
+@pytest.mark.parametrize("kb", [2, 3, 4, 5])
+def test_resident_many_steps(gpu, kind, kb):
+    for M, N in ((1237, 30008), (2049, 16392), (3000, 7176)):
+        print(f"case {kind} {(M, N, 128 * kb)}", flush=True)
+        assert plan_for(kind, M, N, 128 * kb)["kernel"] == "resident"
+        check_exact(gpu, kind, M, N, 128 * kb)
+
+
+def test_resident_hands_over_outputs_it_cannot_store(gpu):
+    """16-byte stores of 16-bit results: a base or a row pitch that does not allow them, and fp32 results, take another kernel."""
+    import ctypes
+
+    from sglang_amd import _lib
+
+    M, N, K = 600, 16384, 512
+    assert plan_for("fp8", M, N, K)["kernel"] == "resident"
+    g = torch.Generator(device=gpu).manual_seed(1)
+    a, w = (torch.randint(-2, 3, s, generator=g, device=gpu).float().to(FP8) for s in ((M, K), (N, K)))
+    sa, sb = torch.ones(K // 128, M, device=gpu), torch.ones(N // 128, K // 128, device=gpu)
+    want = a.double() @ w.double().t()
+    ws = torch.empty(_lib.lib().mi355_fp8_blockwise_mm_workspace_bytes(M, N, K), dtype=torch.uint8, device=gpu)
+    for code, dtype, pitch, shift in ((2, torch.bfloat16, N, 0), (2, torch.bfloat16, N, 4), (2, torch.bfloat16, N + 4, 0), (1, torch.float16, N + 8, 0), (0, torch.float32, N, 0)):
+        out = torch.zeros(M * pitch + 64, dtype=dtype, device=gpu)
+        ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+        rc = _lib.lib().mi355_fp8_blockwise_mm(ptr(a), ptr(w), ptr(sa), ptr(sb), ctypes.c_void_p(out.data_ptr() + shift * out.element_size()), code, M, N, K, K, K,
+                                               1, M, K // 128, 1, pitch, ptr(ws), ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, (dtype, pitch, shift, _lib.lib().mi355_last_error())
+        rows = out[shift:shift + M * pitch].view(M, pitch)
+        assert torch.equal(rows[:, :N].double(), want.to(dtype).double()), (dtype, pitch, shift)
+        assert not out[:shift].any() and not out[shift + M * pitch:].any() and not rows[:, N:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_resident_bias_and_rows(gpu, dtype):
+    """The four linears with a bias: the rows that a smaller call, on another kernel with the same order of sums, computes."""
+    from sglang_amd import _lib, fp8_utils, w8a8_int8
+    from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
+
+    M, N, K = 900, 24576, 512
+    x = make_activation(M, K, dtype=dtype).to(gpu)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2)).to(dtype).to(gpu)
+    w, s = (t.to(gpu) for t in make_fp8_weight(N, K))
+    w2, words = fp8_utils.requant_weight_ue8m0(w, s, [128, 128])
+    wi, si = (t.to(gpu) for t in make_int8_weight(N, K))
+    scale = torch.rand(N, 1, generator=torch.Generator().manual_seed(3)).to(gpu) * 0.01 + 1e-3
+    linear = fp8_utils.dispatch_w8a8_block_fp8_linear()
+    calls = {"block": lambda x: linear(x, w, [128, 128], s, None, bias), "token_fp8": lambda x: fp8_utils.apply_fp8_linear(x, w.t(), scale, None, bias=bias, use_per_token_if_dynamic=True),
+             "int8": lambda x: w8a8_int8.apply_w8a8_int8_linear(x, wi.t(), si, bias)}
+    if dtype == torch.bfloat16:
+        calls["ue8m0"] = lambda x: fp8_utils.deepgemm_w8a8_block_fp8_linear_with_fallback(x, w2, [128, 128], words, None, bias)
+    for kind, call in calls.items():
+        few = 200
+        assert _lib.linear_plan(kind, M, N, K)["kernel"] == "resident" and _lib.linear_plan(kind, few, N, K)["kernel"] == "dma3"
+        assert _lib.linear_plan(kind, few, N, K)["splits"] == 1
+        assert torch.equal(call(x)[:few].view(torch.int16), call(x[:few].contiguous()).view(torch.int16)), kind
