@@ -42,6 +42,7 @@ struct GemmParams {
   int64_t sa_sm, sa_sk, sb_sn, sb_sk;
   int kb_total, kb_per_split, splits;
   int tiles_m, tiles_n;
+  int rotate_k;  // mid-M tile: the K loops of different channel tiles start at different blocks
   int out_dtype;
   int ue8m0;  // FP8 only: sa / sb are packed exponent words and the route's kernel applies them in the MFMA (set by the UE8M0 entry point)
 };

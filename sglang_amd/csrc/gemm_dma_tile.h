@@ -117,11 +117,18 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
   const uint8_t* mixed_base = mixed_tokens ? p.a : p.b;
   // every wave fetches BM / 8 token scales per K block, four per lane; quads past M refetch the last valid one
   const uint32_t sa_off = (uint32_t)min(m0 + wave * (BM / 8) + min(lane, BM / 32 - 1) * 4, (p.M - 1) & ~3) * 4u;
+  // The K loop may start in the middle (the sum is the same products in another order): block k of the loop is block
+  // (k + rotation) % nkb of the range.  See rotates_k.
+  const int rotation = p.rotate_k ? __builtin_amdgcn_readfirstlane((n0 / BN) % nkb) : 0;
+  auto block_of = [&](int kb) {
+    kb = min(kb, kb_last) + rotation;
+    return kb > kb_last ? kb - nkb : kb;
+  };
   // Load number i of K block kb (< ROW_LOADS: tile rows; then the token scales) into stage `st`.  The statements write m0; it
   // cannot be listed as a clobber (the compiler reserves the register), and no compiler-managed use of m0 lies between them
   // and the next statement that sets it.
   auto issue = [&](int i, int st, int kb) {
-    kb = min(kb, kb_last);
+    kb = block_of(kb);
     if (i < T::ROW_LOADS) {
       // wave-uniform: the row group (the last load's may be one another wave fetches too) and its matrix
       const int group = i * 8 + 8 <= T::GROUPS ? i * 8 + wave : last_group;
@@ -164,7 +171,7 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
   float sbv[SB];  // scales (words) of the block to be multiplied next
   auto load_sb = [&](int kb) {
     if constexpr (T::SCALED) {
-      kb = min(kb, kb_last);
+      kb = block_of(kb);
 #pragma unroll
       for (int b = 0; b < SB; ++b) sbv[b] = sb_ptr[b][(int64_t)(AR == AR_UE8M0 ? kb >> 2 : kb) * p.sb_sk];
     }
@@ -223,7 +230,7 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
 #pragma unroll
         for (int b = 0; b < SB; ++b) sc[j][b] = tsc[CUR][j] * sbv[b];
     } else if constexpr (AR == AR_UE8M0) {
-      const int shift = (kb & 3) * 8;
+      const int shift = (block_of(kb) & 3) * 8;
 #pragma unroll
       for (int b = 0; b < SB; ++b) w_exp[b] = in_vgpr((int)(__float_as_uint(sbv[b]) >> shift));
 #pragma unroll
@@ -404,10 +411,19 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + 
   dma_tile<AR, BM, BN, SPLIT, S>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
 }
 
+// Weight rows a multiple of 4096 bytes apart: with every workgroup at the same K block, all rows being fetched lie at the same place of
+// that period, which is a few of the memory's channels.  Each channel tile then starts its K loop one block further on.  us, all from
+// block 0 / rotated (whole linears): 4096 -> 28672 at 32 tokens INT8 33.3 / 28.7, per-token FP8 at 100 35.5 / 32.2; 8192 -> 28672 at 32
+// 57.5 / 47.2; 12288 -> 28672 at 200 118.5 / 106.5; 16384 -> 4096 at 101 29.5 / 28.3.  Weights below 64 million values come out of the caches
+// often enough (14 shapes: 1.00, 0.98 to 1.03), and other pitches spread by themselves (K = 7168 -> 36864 0.99 to 1.00, 18432 -> 7168 at 40 1.01,
+// 4608 -> 7168 at 242 22.5 / 23.4: the token rows of concurrent tiles are no longer the same).
+inline bool rotates_k(const GemmParams& p) { return p.ldb % 4096 == 0 && (int64_t)p.N * p.ldb >= 64000000; }
+
 template <Arith AR, int BM, int BN>
 int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
+  p.rotate_k = rotates_k(p);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
   constexpr int OWN = stages_of(BM, BN, true), SHARED = stages_of(BM, BN, false);
   if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) {
