@@ -826,13 +826,15 @@ std::vector<std::string> tile_constant_names() {
     for (const char* what : {"tile", "block"})
       for (const TileSize& t : MID_TILES) names.push_back(std::string(times) + what + "[" + std::to_string(t.bm) + "x" + std::to_string(t.bn) + "]");
     add(times, {"pp_tile", "pp_block", "pp_busy", "pp_store", "ws_launch", "ws_tile", "ws_kb", "ws_kb_busy", "ws_stream", "ws_stream_us",
-                "ws_result", "ws_norm", "rs_launch", "rs_tile", "rs_tile_block", "rs_step", "rs_step_block", "rs_busy"});
+                "ws_result", "ws_norm", "rs_launch", "rs_tile", "rs_tile_block", "rs_step", "rs_step_block", "rs_busy",
+                "cold", "cold_channel", "cold_token", "cold_shared", "cold_stream", "cold_stream_us", "cold_again", "cold_split_us", "cold_split_us_per_mb",
+                "cold_ws_channel", "cold_ws_token", "cold_ws_stream", "cold_ws_stream_us", "cold_ws_norm", "cold_pp_tile", "cold_pp_block", "cold_pp_busy"});
   }
   add("limits.", {"margin", "two_phase_margin", "large_weight_margin", "large_weight_max_tokens", "mid_wavesplit_max_weight", "ragged_max_weight",
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "cold_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
 }

@@ -29,6 +29,13 @@ struct TileTimes {
   // weight in registers (gemm_resident.h): rounds of rs_tile + K blocks * rs_tile_block + steps * (rs_step + K blocks * rs_step_block) *
   // (1 + rs_busy * fill), a step being 64 tokens (steps of 32 count half)
   double rs_launch, rs_tile, rs_tile_block, rs_step, rs_step_block, rs_busy;
+  // a weight that comes from memory (choose_cold_tile): a K block of a mid-M tile takes no less than cold + channels * cold_channel +
+  // tokens * cold_token (64 x 128, two workgroups per CU: times cold_shared); its stream, of which every further token tile fetches
+  // the share cold_again once more; K / 1000 * (channels * cold_ws_channel + tokens * cold_ws_token) for a wave-split tile and its stream
+  // at cold_ws_stream times the rate above; 256 x 256: factors and busy of pp_block
+  double cold, cold_channel, cold_token, cold_shared, cold_stream, cold_stream_us, cold_again, cold_split_us, cold_split_us_per_mb;
+  double cold_ws_channel, cold_ws_token, cold_ws_stream, cold_ws_stream_us, cold_ws_norm;
+  double cold_pp_tile, cold_pp_block, cold_pp_busy;
 };
 constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     1.93, 0.586, 4.31, 0.217, 4.18, -4.54, 1.808, 0.421,
@@ -36,14 +43,20 @@ constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     {0.219, 0.277, 0.317, 0.385, 0.419, 0.533, 0.288, 0.363, 0.441, 0.532, 0.334, 0.445, 0.535},
     7.88, 0.567, 1.70, 12.5,
     2.74, 1.041, 0.00591, 0.00334, 5.49, -3.81, 0.253, 1.511,
-    3.63, 0.11, 0.406, 0.596, 0.186, 0.733};
+    3.63, 0.11, 0.406, 0.596, 0.186, 0.733,
+    0.101, 0.0019, 0.0020, 1.42, 4.88, -0.45, 0.202, 3.27, 0.320,
+    0.01269, 0.01362, 1.434, -1.44, 1.283,
+    6.52, 1.774, 0.55};
 constexpr TileTimes PLAIN_TIMES = {  // FP8 with epilogue scales, INT8
     1.77, 0.777, 3.81, 0.251, 4.55, -2.24, 1.871, 0.402,
     {2.21, 2.72, 3.03, 3.17, 3.76, 4.72, 2.48, 3.12, 3.83, 4.14, 2.81, 3.80, 4.64},
     {0.165, 0.205, 0.240, 0.295, 0.333, 0.432, 0.224, 0.271, 0.339, 0.420, 0.278, 0.347, 0.431},
     8.48, 0.511, 1.70, 10.8,
     2.71, 1.017, 0.00609, 0.00343, 5.07, -4.41, 0.282, 1.673,
-    3.64, 0.01, 0.435, 0.760, 0.217, 0.531};
+    3.64, 0.01, 0.435, 0.760, 0.217, 0.531,
+    0.092, 0.0020, 0.0018, 1.37, 5.02, 1.55, 0.230, 3.16, 0.331,
+    0.01247, 0.01387, 1.394, -1.13, 1.215,
+    6.35, 1.730, 0.681};
 static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above follow MID_TILES");
 
 // Where the model is not asked or not trusted; both sides of each line stand beside the function that uses it.
@@ -56,6 +69,7 @@ struct TileLimits {
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
   double resident_margin = 0.93;
+  double cold_min_weight = 40e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
 struct TileModel {
   TileTimes scaled = SCALED_TIMES, plain = PLAIN_TIMES;
@@ -116,16 +130,19 @@ double wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_
   return std::max(us, stream) >= most ? most : norm_of(us, stream, t.ws_norm);
 }
 
-TileChoice best_wavesplit_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+// The tile of least time; us(i, most) and us(i, splits, most) time the i-th one.
+template <class Time>
+TileChoice fastest_wavesplit_tile(Time us) {
   TileChoice best{TF_NONE, 0, 0, 1, 1e30};
   constexpr int COUNT = sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0]);
   for (int i = 0; i < COUNT; ++i) {
-    const double us = wavesplit_tile_us(t, i, M, N, K, best.us);
-    if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
+    const double u = us(i, best.us);
+    if (u < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, u};
   }
   return best;
 }
-TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+template <class Time>
+TileChoice fastest_dma_tile(int64_t M, int64_t N, int64_t K, Time us) {
   TileChoice best{TF_NONE, 0, 0, 1, 1e30};
   const int64_t kb = ceil_div(K, KSTEP);
   for (int i = 0; i < 13; ++i) {
@@ -136,11 +153,48 @@ TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
       if (splits > 1 && (N % 4 != 0 || per < 4 || tiles * splits > 560 || tiles > 200)) break;
       if (splits == previous) continue;
       previous = splits;
-      const double us = dma_tile_us(t, i, M, N, K, splits, best.us);
-      if (us < best.us) best = {TF_DMA, MID_TILES[i].bm, MID_TILES[i].bn, splits, us};
+      const double u = us(i, splits, best.us);
+      if (u < best.us) best = {TF_DMA, MID_TILES[i].bm, MID_TILES[i].bn, splits, u};
     }
   }
   return best;
+}
+TileChoice best_wavesplit_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  return fastest_wavesplit_tile([&](int i, double most) { return wavesplit_tile_us(t, i, M, N, K, most); });
+}
+TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  return fastest_dma_tile(M, N, K, [&](int i, int splits, double most) { return dma_tile_us(t, i, M, N, K, splits, most); });
+}
+
+// The same tiles with a weight that comes from memory.
+double cold_dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, int splits, double most = 1e30) {
+  const int bm = MID_TILES[i].bm, bn = MID_TILES[i].bn;
+  const int64_t tiles_m = ceil_div(M, bm), wg = tiles_m * ceil_div(N, bn) * splits;
+  const double blocks = (double)ceil_div(ceil_div(K, KSTEP), splits);
+  const bool two = bm + bn == 192 && wg > NUM_CUS;
+  const double fetch = (t.cold + t.cold_channel * bn + t.cold_token * (double)M / (double)tiles_m) * (two ? t.cold_shared : 1.0);
+  const double us = t.launch + rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) {
+                      return t.tile[i] + blocks * norm_of(t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill), fetch, 6.0);
+                    });
+  const double mn = (double)M * (double)N * 1e-6, fetches = 1.0 + t.cold_again * (double)(tiles_m - 1);
+  const double stream = ((double)N * fetches + (double)M) * (double)K * 1e-6 / t.cold_stream + mn * 2.0 * t.result_us_per_mb + t.cold_stream_us;
+  const double split = splits > 1 ? t.cold_split_us + t.cold_split_us_per_mb * splits * mn * 4.0 : 0.0;
+  return std::max(us, stream) + split >= most ? most : norm_of(us, stream, 6.0) + split;
+}
+double cold_wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, double most = 1e30) {
+  const int bm = WAVESPLIT_TILES[i].bm, bn = WAVESPLIT_TILES[i].bn;
+  const int64_t tiles_m = ceil_div(M, bm);
+  const double us = t.ws_launch + (double)ceil_div(tiles_m * ceil_div(N, bn), NUM_CUS) *
+                                      (t.ws_tile + (double)K * 1e-3 * (t.cold_ws_channel * bn + t.cold_ws_token * (double)M / (double)tiles_m) +
+                                       (double)(bm * bn) / 1024.0 * t.ws_result);
+  const double stream = (double)N * (double)K * 1e-6 / (t.cold_stream * t.cold_ws_stream) + t.cold_ws_stream_us;
+  return std::max(us, stream) >= most ? most : norm_of(us, stream, t.cold_ws_norm);
+}
+double cold_two_phase_us(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
+  const double blocks = (double)ceil_div(K, KSTEP);
+  return t.launch + rounds_of(ceil_div(M, 256) * ceil_div(N, 256), NUM_CUS, [&](double fill) {
+           return norm_of(t.cold_pp_tile + blocks * t.pp_block * t.cold_pp_block * (1.0 + t.cold_pp_busy * fill), t.pp_store * fill, 6.0);
+         });
 }
 
 double resident_us(const TileTimes& t, int64_t M, int64_t N, int64_t K, int64_t ranges) {
@@ -163,19 +217,24 @@ TileChoice best_resident(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+// The wave-split tile: a large weight streams better through the wide tiles (K = 4096 -> N = 28672 at 48 tokens 27.2 against
+// 33.6 us), and so does a large token matrix, which leaves the XCDs' L2s and is fetched again by every channel tile (mid-M / wave-split:
+// K = 10368 -> N = 704 at 2616 tokens 37.4 / 53.2, 10496 -> 960 at 1610 34.7 / 44.7, per-token FP8 7168 -> 384 at 2595 19.3 / 22.3;
+// but 7168 -> 576 at 1608 23.1 / 20.3).
+bool wavesplit_allowed(int64_t M, int64_t N, int64_t K) {
+  const TileLimits& l = tile_model().limits;
+  const double token_bytes = (double)(M * K);
+  return (double)(N * K) <= l.mid_wavesplit_max_weight && token_bytes <= l.wavesplit_max_tokens_bytes &&
+         ((double)K <= l.wavesplit_long_k || token_bytes <= l.wavesplit_long_k_max_tokens_bytes);
+}
+
 // More than 16 tokens, K % 128 == 0, aligned operands: the fastest tile, or TF_NONE where `base`, what the route names (a mid-M
 // tile or the two-phase tile), models within 5 % of it (the two-phase tile 10 %): below that the model does not order two tiles.
 TileChoice choose_swept_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, double& base_us) {
   const TileTimes& t = tile_times(kind);
   TileChoice best = best_dma_tile(t, M, N, K);
   const TileLimits& l = tile_model().limits;
-  // The wave-split tile: a large weight streams better through the wide tiles (K = 4096 -> N = 28672 at 48 tokens 27.2 against
-  // 33.6 us), and so does a large token matrix, which leaves the XCDs' L2s and is fetched again by every channel tile (mid-M / wave-split:
-  // K = 10368 -> N = 704 at 2616 tokens 37.4 / 53.2, 10496 -> 960 at 1610 34.7 / 44.7, per-token FP8 7168 -> 384 at 2595 19.3 / 22.3;
-  // but 7168 -> 576 at 1608 23.1 / 20.3).
-  const double token_bytes = (double)(M * K);
-  const bool tokens_fit = token_bytes <= l.wavesplit_max_tokens_bytes && ((double)K <= l.wavesplit_long_k || token_bytes <= l.wavesplit_long_k_max_tokens_bytes);
-  if ((double)(N * K) <= l.mid_wavesplit_max_weight && tokens_fit) {
+  if (wavesplit_allowed(M, N, K)) {
     const TileChoice ws = best_wavesplit_tile(t, M, N, K);
     if (ws.us < best.us) best = ws;
   }
@@ -200,13 +259,50 @@ TileChoice choose_swept_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, con
   return best.us < margin * base_us ? best : TileChoice{TF_NONE, 0, 0, 1, 0.0};
 }
 
+// A second look at what was chosen (the swept tile, or `base` where that stays) where the weight is large enough to come from
+// memory: 64 x 128 tiles on one CU in two read it at 33 KB a microsecond and CU, whatever their MFMAs could take, so what counts is
+// how many CUs read and how often each row is fetched, which the times above know little of.  Fitted to 19 000 timings of 330
+// shapes with 40 to 400 million weights, 17 to 1500 tokens: 3 to 4 % root mean square, where the times above are off by 5 to 7.
+// At 102 random shapes where it changes the tile (one in nine of 17 to 6000 tokens by 40 to 600 million weights) linears take 0.895 times
+// as long, 0.82 up to 64 tokens, at worst 1.05.  us, before / after: block FP8 139 tokens 18432 -> 7168 52.5 / 45.9, 158 tokens 16640 ->
+// 16384 104.6 / 77.7, 115 tokens 7680 -> 9600 37.0 / 30.0; per-token FP8 510 tokens 3456 -> 16512 51.9 / 44.2; INT8 169 tokens 7168 ->
+// 36864 98.4 / 83.4, but 216 tokens 9216 -> 7168 37.1 / 39.0.  Within 8 % it does not order two tiles.
+// Not judged: the 256 x 256 tile where it was chosen (2556 tokens 7168 -> 7168 155.3, 128 x 192 tiles 159.0), the INT8 kernel of 128 x 256 tiles in two phases, which has no time of its own here, and up to 128 tokens a split plan that
+// fills seven eighths of the chip, where two token tiles cost less than `cold_again` has it (128 tokens 18432 -> 7168: 64 x 128 tiles
+// in two splits 49.8 us measured, 128 x 128 in four 44.2; modelled 48 and 39; 72 tokens 8320 -> 21120 44.8 against 46.3).
+TileChoice choose_cold_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, const TileChoice& swept) {
+  const TileTimes& t = tile_times(kind);
+  const TileLimits& l = tile_model().limits;
+  const TileChoice& c = swept.family != TF_NONE ? swept : base;
+  if ((double)(N * K) < l.cold_min_weight || c.family == TF_NONE || c.family == TF_TWO_PHASE) return swept;
+  if (kind == GK_INT8 && swept.family == TF_NONE && c.bm == 128 && c.bn == 256) return swept;
+  if ((double)M <= l.cold_full_max_tokens && c.family == TF_DMA && c.splits > 1 &&
+      (double)(ceil_div(M, c.bm) * ceil_div(N, c.bn) * c.splits) >= l.cold_full_workgroups)
+    return swept;
+  double us = 1e30;
+  if (c.family == TF_DMA)
+    for (int i = 0; i < 13; ++i)
+      if (MID_TILES[i].bm == c.bm && MID_TILES[i].bn == c.bn) us = cold_dma_tile_us(t, i, M, N, K, c.splits);
+  if (c.family == TF_WAVESPLIT)
+    for (int i = 0; i < (int)(sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0])); ++i)
+      if (WAVESPLIT_TILES[i].bm == c.bm && WAVESPLIT_TILES[i].bn == c.bn) us = cold_wavesplit_tile_us(t, i, M, N, K);
+  TileChoice best = fastest_dma_tile(M, N, K, [&](int i, int splits, double most) { return cold_dma_tile_us(t, i, M, N, K, splits, most); });
+  if (wavesplit_allowed(M, N, K)) {
+    const TileChoice ws = fastest_wavesplit_tile([&](int i, double most) { return cold_wavesplit_tile_us(t, i, M, N, K, most); });
+    if (ws.us < best.us) best = ws;
+  }
+  const double two_phase = M > 128 ? cold_two_phase_us(t, M, N, K) : 1e30;
+  if (two_phase < best.us) best = {TF_TWO_PHASE, 256, 256, 1, two_phase};
+  return best.us < l.cold_margin * us ? best : swept;
+}
+
 // The same, or the kernel that keeps the weight in registers where the call allows it and it models 7 % faster than what would run.
 // The linears on both sides of the line, us, other / this: block FP8 368 tokens 512 -> 32768 17.4 / 15.5, 430 tokens 512 -> 24576
 // 16.5 / 15.6, 243 tokens 512 -> 6144 8.3 / 8.4, 1340 tokens 512 -> 4096 11.3 / 12.2; 849 tokens 512 -> 6144 10.6 / 11.5;
 // per-token FP8 180 tokens 512 -> 24576 10.2 / 12.0, 624 tokens 640 -> 16384 17.2 / 15.7.
 TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool resident_allowed) {
   double base_us;
-  const TileChoice c = choose_swept_tile(kind, M, N, K, base, base_us);
+  const TileChoice c = choose_cold_tile(kind, M, N, K, base, choose_swept_tile(kind, M, N, K, base, base_us));
   if (!resident_allowed) return c;
   const TileChoice r = best_resident(tile_times(kind), M, N, K);
   return r.us < tile_model().limits.resident_margin * (c.family != TF_NONE ? c.us : base_us) ? r : c;

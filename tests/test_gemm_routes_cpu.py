@@ -158,6 +158,23 @@ def test_the_faster_kernel_runs(kind, shape, want, us, other):
     assert us < other and want in (p["kernel"], (p["kernel"], p["bm"], p["bn"], p["splits"])), p
 
 
+# A large weight comes from memory: (kind, shape, tile and splits that have to run, linear's us, the tile's that the other times name)
+COLD_CHOICES = [
+    ("fp8", (139, 7168, 18432), ("dma3", 160, 128, 4), 45.9, 52.5), ("fp8", (158, 16384, 16640), ("dma3", 160, 128, 2), 77.7, 104.6),
+    ("fp8_ue8m0", (254, 12288, 12416), ("dma3", 128, 192, 2), 58.9, 68.9), ("fp8_scaled", (510, 16512, 3456), ("pingpong", 256, 256, 1), 44.2, 51.9),
+    ("int8", (63, 29184, 2816), ("dma3", 64, 128, 1), 20.6, 27.2), ("fp8", (44, 14336, 4096), ("wavesplit_tile", 64, 64, 1), 17.7, 21.3),
+    # what it leaves alone: two token tiles in a split plan that fills the chip, the 256 x 256 tile, smaller weights
+    ("fp8_ue8m0", (72, 21120, 8320), ("dma3", 128, 256, 3), 44.8, 46.3), ("fp8_ue8m0", (2556, 7168, 7168), ("pingpong", 256, 256, 1), 155.3, 159.0),
+    ("fp8", (1608, 576, 7168), ("wavesplit_tile", 64, 64, 1), 20.3, 23.1),
+]
+
+
+@pytest.mark.parametrize("kind,shape,want,us,other", COLD_CHOICES)
+def test_large_weights_run_the_faster_tile(kind, shape, want, us, other):
+    p = plan_for(kind, *shape)
+    assert us < other and (p["kernel"], p["bm"], p["bn"], p["splits"]) == want, p
+
+
 def test_perturbed_plan_query():
     import ctypes
 

@@ -79,7 +79,7 @@ def test_mid_tile_every_remainder(gpu, kind, tile):
 # weight rows a multiple of 4096 bytes apart: every channel tile starts its K loop at another block (whole K and split, one and several
 # token tiles, more channel tiles than K blocks and fewer, a ragged last tile)
 @pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
-@pytest.mark.parametrize("M,N,K", [(40, 16384, 4096), (100, 15688, 4096), (100, 4096, 16384), (300, 8192, 8192), (23, 2184, 32768)])
+@pytest.mark.parametrize("M,N,K", [(40, 20480, 4096), (100, 15688, 4096), (100, 4096, 16384), (300, 8192, 8192), (23, 2184, 32768)])
 def test_rotated_k(gpu, kind, M, N, K):
     assert N * K >= 64e6 and plan_for(kind, M, N, K)["kernel"] == "dma3"
     check_exact(gpu, kind, M, N, K)
