@@ -426,6 +426,19 @@ int launch_fp8_dma3_unit(GemmParams& p, int bm, int bn, hipStream_t stream, cons
 // One-call linear at decode sizes on this kernel: a producer wave quantizes the unquantized tokens (p.x16, M <= 16) block by block.
 int launch_fp8_dma3_quant(GemmParams& p, int bn, hipStream_t stream, const char* what);
 
+// Whether a launch loads its weight with nontemporal loads: a large one that every workgroup reads a part of its own of.  Such loads leave
+// nothing behind in the 256 MB Infinity Cache, and what has to come from memory comes faster: 264 MB read by 256 workgroups at 6.2
+// instead of 5.65 TB/s.  Linears, us, without / with: block FP8 7168 -> 36864 at 8 tokens 48.6 / 43.6, 4096 -> 28672 at 32 and 128 30.2 / 26.7,
+// 36.9 / 33.6, 18432 -> 7168 at 8 and 32 28.6 / 26.2, 34.2 / 32.2; INT8 7168 -> 24576 at 64 43.6 / 39.0; 256 experts of four rows 157 / 139.
+// Not below 100 million bytes, where a caller's few layers may still lie in that cache: with three weights in turn 7168 -> 7168 at 8 and 48
+// tokens 12.3 / 13.2 and 14.3 / 19.8, 7168 -> 12288 at 8 and 128 18.7 / 19.3, 33.3 / 36.7 (from memory, 16 to 96 in turn, 0.92 to 0.97 for one
+// tile of 64 tokens).  Not where several token tiles fetch the weight (18432 -> 7168 at 256 62.8 / 65.1, 4096 -> 28672 at 256 46.1 / 47.2),
+// and from 65 tokens on not where K is split (18432 -> 7168 at 96 and 112, four ways, INT8 43.1 / 43.9, 45.3 / 46.7).
+constexpr int64_t STREAMED_WEIGHT_BYTES = 100000000;
+inline bool streams_weight(const GemmParams& p) {
+  return p.tiles_m == 1 && (p.M <= 64 || p.splits == 1) && (int64_t)p.N * p.ldb >= STREAMED_WEIGHT_BYTES;
+}
+
 // Grouped problems on the tile bodies of the dense kernels: token rows of all experts stacked in one matrix, one weight
 // matrix per expert.  `g` describes expert 0 (a, out, b, sb, and sa = the re-laid-out token scales: M-major, every
 // expert's first row moved to column ((row0 + 3) & ~3) + 4 * expert so that each expert starts on a whole quad); N, K,
@@ -471,7 +484,7 @@ __device__ __forceinline__ bool grouped_tile_of_block(const GroupedParams& gp, G
   p.M = __builtin_amdgcn_readfirstlane(rec.z);
   return true;
 }
-int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, hipStream_t stream, const char* what);  // gemm_fp8_dma3.hip; 64 or 128 x 128 or 256
+int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, bool streamed, hipStream_t stream, const char* what);  // gemm_fp8_dma3.hip; 64 or 128 x 128 or 256
 int launch_fp8_grouped_pp(GroupedParams& gp, hipStream_t stream, const char* what);            // gemm_fp8_pp.hip: 256-row tiles
 int launch_int8_dma3(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);  // gemm_int8_dma3.hip: same tiling, int8 MFMA, int32 partials
 

@@ -79,7 +79,7 @@ struct TileShape {
 // One BM x BN output tile at (m0, n0), K blocks of split `split`, by the whole workgroup.
 // AR_UE8M0: p.sa / p.sb point to packed exponent words: token word (m, kw) at sa[kw * sa_sk + m], channel word (n, kw) at
 // sb[kw * sb_sk + n * sb_sn], byte kb & 3 of word kb >> 2 belongs to K block kb.
-template <Arith AR, int BM, int BN, bool SPLIT, int S>
+template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM = false>
 __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, int split) {
   using T = TileShape<AR, BM, BN>;
   static_assert(S >= 3 && S * (T::STAGE_BYTES + BM * 4) <= 160 * 1024, "the stages must fit the CU's LDS");
@@ -135,7 +135,10 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
       const uint8_t* base = (i * 8 + 8 <= BM / 8 ? p.a : i * 8 >= BM / 8 ? p.b : mixed_base) + (uint64_t)kb * KSTEP;
       asm volatile("" : "+s"(base));
       const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_stage + (uint32_t)(st * T::STAGE_BYTES + group * 8 * KSTEP);
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
+      if (STREAM && i * 8 >= BM / 8)  // (weight rows only)
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
+      else
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
     } else if constexpr (T::SCALED) {
       // BM / 32 lanes fetch 16 bytes each (a 4-byte-per-lane load in this stream costs far more than its size).  exec is
       // narrowed and restored inside the statement.  Packed exponents: one row of words per four K blocks, fetched again for
@@ -405,10 +408,10 @@ constexpr int stages_of(int bm, int bn, bool own_cu) {
   return bm + bn == 192 ? (own_cu ? 6 : 3) : bm + bn == 224 ? 5 : bm + bn <= 288 ? 4 : 3;
 }
 
-template <Arith AR, int BM, int BN, bool SPLIT, int S>
+template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM>
 __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + BN == 192 && S == 3 ? 4 : 2))) void gemm_dma_kernel(const GemmParams p) {
   const TileCoord tc = tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n);
-  dma_tile<AR, BM, BN, SPLIT, S>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
+  dma_tile<AR, BM, BN, SPLIT, S, STREAM>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
 }
 
 // Weight rows a multiple of 4096 bytes apart: with every workgroup at the same K block, all rows being fetched lie at the same place of
@@ -426,12 +429,20 @@ int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   p.rotate_k = rotates_k(p);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
   constexpr int OWN = stages_of(BM, BN, true), SHARED = stages_of(BM, BN, false);
-  if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) {
-    if (p.splits > 1) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, true, SHARED>), grid, dim3(T_THREADS), 0, stream, p);
-    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, false, SHARED>), grid, dim3(T_THREADS), 0, stream, p);
+  const auto launch = [&](auto split, auto streamed) {
+    constexpr bool SPLIT = decltype(split)::value, STREAM = decltype(streamed)::value;
+    if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, SHARED, STREAM>), grid, dim3(T_THREADS), 0, stream, p);
+    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, OWN, STREAM>), grid, dim3(T_THREADS), 0, stream, p);
+  };
+  const std::false_type no;
+  const std::integral_constant<bool, BM == 64> split_streams;
+  if (p.splits > 1) {
+    if (split_streams && streams_weight(p)) launch(std::true_type{}, split_streams);
+    else launch(std::true_type{}, no);
+  } else if (streams_weight(p)) {
+    launch(no, std::true_type{});
   } else {
-    if (p.splits > 1) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, true, OWN>), grid, dim3(T_THREADS), 0, stream, p);
-    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, false, OWN>), grid, dim3(T_THREADS), 0, stream, p);
+    launch(no, no);
   }
   return check_launch(what);
 }

@@ -37,18 +37,21 @@ struct Dma3State {
 // Load number i (a tile-row load) of K block kb, written as instructions.
 // The statements write m0; it cannot be listed as a clobber (the compiler reserves the register and rejects the entry), and
 // no compiler-managed use of m0 lies between them and the next statement that sets it.
-template <int BM, int BN>
+template <int BM, int BN, bool STREAM>
 __device__ __forceinline__ void issue_one(const Dma3State<BM, BN>& s, int i, uint8_t* stage, int kb) {
   kb = min(kb, s.kb_last);
   const uint8_t* base = s.b_base + (uint64_t)kb * KSTEP;  // wave-uniform
   asm volatile("" : "+s"(base));
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)(stage + (i * 64 + s.wave * 8) * KSTEP);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(s.goff[i]), "s"(base), "s"(lds_addr) : "memory");
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(s.goff[i]), "s"(base), "s"(lds_addr) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(s.goff[i]), "s"(base), "s"(lds_addr) : "memory");
 }
 
 // One K block out of `cur`; the weight-row loads of block kb_next go out in between, into `nxt` (a producer wave writes the
 // token rows).
-template <int BM, int BN>
+template <int BM, int BN, bool STREAM>
 __device__ __forceinline__ void k_block(const Dma3State<BM, BN>& s, const uint8_t* cur, const float* sc_cur,
                                         const float (&sbv)[Dma3State<BM, BN>::SB], float (&acc)[BN / 64][BM / 32][4], uint8_t* nxt,
                                         int kb_next) {
@@ -92,7 +95,7 @@ __device__ __forceinline__ void k_block(const Dma3State<BM, BN>& s, const uint8_
 #pragma unroll
       for (int b = 0; b < SB; ++b) scb[(j + 1) & 1][b] = scp[(j + 1) * 16] * sbv[b];
     }
-    if (t >= BM / 64 && t < LOADS) issue_one<BM, BN>(s, t, nxt, kb_next);
+    if (t >= BM / 64 && t < LOADS) issue_one<BM, BN, STREAM>(s, t, nxt, kb_next);
     __builtin_amdgcn_sched_barrier(0);
   }
   constexpr int t = MT * T_NT - 1;
@@ -138,7 +141,7 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, float (&acc)[BN 
 // the one being multiplied, and meets the others at every block's barrier.  Token rows 16..63 of a stage are never written:
 // what they hold only reaches accumulators of rows that are not stored.
 constexpr int T_PW = 4;  // producer waves of the fused quantizer
-template <int BN, int S>
+template <int BN, int S, bool STREAM>
 __device__ __forceinline__ void dma3_tile_q(const GemmParams& p, int n0) {
   constexpr int BM = 64;
   static_assert(S >= 3 && S * ((BM + BN) * KSTEP + BM * 4) <= 160 * 1024, "the stages must fit the CU's LDS");
@@ -247,7 +250,7 @@ __device__ __forceinline__ void dma3_tile_q(const GemmParams& p, int n0) {
 #pragma unroll
   for (int b = 0; b < S - 1; ++b)
 #pragma unroll
-    for (int i = BM / 64; i < LOADS; ++i) issue_one<BM, BN>(s, i, t_stage[b], b);
+    for (int i = BM / 64; i < LOADS; ++i) issue_one<BM, BN, STREAM>(s, i, t_stage[b], b);
   wait_and_barrier<YOUNGER>();  // the weight rows of block 0 have landed; the producer has written blocks 0 .. S-2
 
   auto sb_of = [&](int kb, float (&v)[SB]) {
@@ -261,7 +264,7 @@ __device__ __forceinline__ void dma3_tile_q(const GemmParams& p, int n0) {
     for (int u = 0; u < S; ++u) sb_of(k + u, sbv[u]);
 #pragma unroll
     for (int u = 0; u < S; ++u) {
-      k_block<BM, BN>(s, t_stage[u], t_scale[u], sbv[u], acc, t_stage[(u + S - 1) % S], k + u + S - 1);
+      k_block<BM, BN, STREAM>(s, t_stage[u], t_scale[u], sbv[u], acc, t_stage[(u + S - 1) % S], k + u + S - 1);
       wait_and_barrier<YOUNGER>();  // unconditional (a condition here makes the compiler sink arithmetic across blocks): when K
                                     // is a whole number of trips this is one barrier past the last block, which the producers match
     }
@@ -271,7 +274,7 @@ __device__ __forceinline__ void dma3_tile_q(const GemmParams& p, int n0) {
     if (k + u < nkb) {
       float sbl[SB];
       sb_of(k + u, sbl);
-      k_block<BM, BN>(s, t_stage[u], t_scale[u], sbl, acc, t_stage[(u + S - 1) % S], k + u + S - 1);
+      k_block<BM, BN, STREAM>(s, t_stage[u], t_scale[u], sbl, acc, t_stage[(u + S - 1) % S], k + u + S - 1);
       if (k + u + 1 < nkb) wait_and_barrier<YOUNGER>();
     }
   }
@@ -279,20 +282,20 @@ __device__ __forceinline__ void dma3_tile_q(const GemmParams& p, int n0) {
   store_tile<BM, BN>(p, acc, 0, n0, wave_m, wave_n, l16, q);
 }
 
-template <int BN, int S>
+template <int BN, int S, bool STREAM>
 __global__ __launch_bounds__(T_THREADS + 64 * T_PW) void fp8_gemm_dma3_q_kernel(const GemmParams p) {
   const TileCoord tc = tile_of_block(blockIdx.x, gridDim.x, 1, p.tiles_n);
-  dma3_tile_q<BN, S>(p, tc.tile_n * BN);
+  dma3_tile_q<BN, S, STREAM>(p, tc.tile_n * BN);
 }
 
 // Grouped problems (see GroupedParams): the workgroup's token tile comes from the table the plan kernel wrote, the
 // operand bases move to that tile's expert, and the ordinary tile runs.
-template <int BM, int BN, int S>
+template <int BM, int BN, int S, bool STREAM>
 __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + BN == 192 && S == 3 ? 4 : 2))) void fp8_grouped_dma_kernel(const GroupedParams gp) {
   GemmParams p;
   int m0, tile_n;
   if (!grouped_tile_of_block(gp, p, m0, tile_n)) return;  // the whole workgroup leaves before any barrier
-  dma_tile<AR_F32, BM, BN, false, S>(p, m0, tile_n * BN, 0);
+  dma_tile<AR_F32, BM, BN, false, S, STREAM>(p, m0, tile_n * BN, 0);
 }
 
 }  // namespace
@@ -385,16 +388,21 @@ Dma3Plan dma3_plan(int64_t M, int64_t N, int64_t K, bool is_int8) {
   return pl;
 }
 
-int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, hipStream_t stream, const char* what) {
+int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, bool streamed, hipStream_t stream, const char* what) {
   gp.g.tiles_n = (gp.g.N + bn - 1) / bn;
   gp.g.splits = 1, gp.g.kb_per_split = gp.g.kb_total;
   const dim3 grid((unsigned)(gp.max_tiles_m * gp.g.tiles_n));
   const dim3 block(T_THREADS);
-  if (bm == 64 && bn == 128 && few) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, true)>), grid, block, 0, stream, gp);
-  else if (bm == 64 && bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, false)>), grid, block, 0, stream, gp);
-  else if (bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 128, stages_of(128, 128, true)>), grid, block, 0, stream, gp);
-  else if (bm == 64) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 256, stages_of(64, 256, true)>), grid, block, 0, stream, gp);
-  else hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 256, stages_of(128, 256, true)>), grid, block, 0, stream, gp);
+  const auto launch = [&](auto streamed) {
+    constexpr bool STREAM = decltype(streamed)::value;
+    if (bm == 64 && bn == 128 && few) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, true), STREAM>), grid, block, 0, stream, gp);
+    else if (bm == 64 && bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, false), STREAM>), grid, block, 0, stream, gp);
+    else if (bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 128, stages_of(128, 128, true), STREAM>), grid, block, 0, stream, gp);
+    else if (bm == 64) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 256, stages_of(64, 256, true), STREAM>), grid, block, 0, stream, gp);
+    else hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 256, stages_of(128, 256, true), STREAM>), grid, block, 0, stream, gp);
+  };
+  if (streamed) launch(std::true_type{});
+  else launch(std::false_type{});
   return check_launch(what);
 }
 
@@ -412,9 +420,14 @@ int launch_fp8_dma3_quant(GemmParams& p, int bn, hipStream_t stream, const char*
   p.tiles_m = 1;
   p.tiles_n = (p.N + bn - 1) / bn;
   const dim3 grid((unsigned)p.tiles_n), block(T_THREADS + 64 * T_PW);
-  if (bn == 128) hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<128, 6>), grid, block, 0, stream, p);
-  else if (bn == 192) hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<192, 4>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<256, 3>), grid, block, 0, stream, p);
+  const auto launch = [&](auto streamed) {
+    constexpr bool STREAM = decltype(streamed)::value;
+    if (bn == 128) hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<128, 6, STREAM>), grid, block, 0, stream, p);
+    else if (bn == 192) hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<192, 4, STREAM>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<256, 3, STREAM>), grid, block, 0, stream, p);
+  };
+  if (streams_weight(p)) launch(std::true_type{});
+  else launch(std::false_type{});
   return check_launch(what);
 }
 

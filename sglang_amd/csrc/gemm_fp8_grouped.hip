@@ -352,5 +352,7 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
     if (rc != MI355_OK) return rc;
   }
   gp.tiles = small_tiles, gp.max_tiles_m = run.max_small;
-  return launch_fp8_grouped_dma3(gp, run.bm, run.bn, run.few, st, what);
+  const int64_t experts = std::min(num_experts, total_m);
+  const bool streamed = !run.use_big && total_m <= experts * run.bm && experts * N * K >= STREAMED_WEIGHT_BYTES;
+  return launch_fp8_grouped_dma3(gp, run.bm, run.bn, run.few, streamed, st, what);
 }

@@ -57,7 +57,7 @@ __device__ __forceinline__ void wait_blocks(int blocks) {
   else wait_loads<0>();
 }
 
-template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2>
+template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2, bool STREAM = false>
 __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void wavesplit_tile_kernel(const GemmParams p) {
   using T = WavesplitTile<AR, MT, CT, TQ>;
   static_assert(TQ == TQ_NONE || MT == 1, "the fused quantizer is for 16 tokens at most");
@@ -98,9 +98,13 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
     if constexpr (AR == AR_UNIT || AR == AR_INT8) back = kb == last ? (uint32_t)(max(chunk - (tail / 16 - 1), 0) * 16) : 0u;
     asm volatile("" : "+s"(wb), "+s"(tb), "+s"(lds));
 #pragma unroll
-    for (int i = 0; i < T::ROW_LOADS; ++i)
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i] - back), "s"(i * 8 < T::TOKENS ? tb : wb), "s"(lds + i * 1024)
-                   : "memory");
+    for (int i = 0; i < T::ROW_LOADS; ++i) {
+      if (STREAM && i * 8 >= T::TOKENS)
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(goff[i] - back), "s"(wb), "s"(lds + i * 1024) : "memory");
+      else
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i] - back), "s"(i * 8 < T::TOKENS ? tb : wb), "s"(lds + i * 1024)
+                     : "memory");
+    }
     if constexpr (T::SCALED) {
       const float* sbase = p.sa + (int64_t)(AR == AR_UE8M0 ? kb >> 2 : kb) * p.sa_sk;
       asm volatile("" : "+s"(sbase));
@@ -252,7 +256,10 @@ template <Arith AR, int MT, int CT>
 int launch_wavesplit_tile_inst(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + 16 * MT - 1) / (16 * MT), p.tiles_n = (p.N + 16 * CT - 1) / (16 * CT);
   p.splits = 1;
-  hipLaunchKernelGGL((wavesplit_tile_kernel<AR, MT, CT>), dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(64 * WST_WAVES), 0, stream, p);
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * WST_WAVES);
+  // (taller tiles are chosen for smaller weights only)
+  if (MT == 1 && streams_weight(p)) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, MT, CT, TQ_NONE, 2, MT == 1>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((wavesplit_tile_kernel<AR, MT, CT>), grid, block, 0, stream, p);
   return check_launch(what);
 }
 template <Arith AR, size_t... I>
@@ -276,9 +283,14 @@ int launch_wavesplit_tile_quant_inst(GemmParams& p, hipStream_t stream, const ch
   p.splits = 1;
   const dim3 grid((unsigned)p.tiles_n), block(64 * WST_WAVES);
   const int64_t pieces = (int64_t)p.M * p.K / 8;
-  if (pieces <= 2 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 2>), grid, block, 0, stream, p);
-  else if (pieces <= 4 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 4>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, WS_QUANT_VECTORS>), grid, block, 0, stream, p);
+  const auto launch = [&](auto streamed) {
+    constexpr bool STREAM = decltype(streamed)::value;
+    if (pieces <= 2 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 2, STREAM>), grid, block, 0, stream, p);
+    else if (pieces <= 4 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 4, STREAM>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, WS_QUANT_VECTORS, STREAM>), grid, block, 0, stream, p);
+  };
+  if (streams_weight(p)) launch(std::true_type{});
+  else launch(std::false_type{});
   return check_launch(what);
 }
 template <Arith AR, TokenQuant TQ>

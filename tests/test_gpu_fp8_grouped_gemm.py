@@ -72,6 +72,24 @@ def _verify(oracle, out, a, w, sa, sw, sizes, offsets, what):
         assert bool((out.float().cpu()[~owned] == 7.0).all()), f"{what}: rows outside every expert were written"
 
 
+@pytest.mark.parametrize("E,rows,N,K", [(16, 3, 1672, 3840), (8, 40, 3584, 3584), (64, 1, 768, 2048), (64, 50, 784, 2048)])
+def test_streamed_expert_weights(gpu, E, rows, N, K):
+    """Expert weights of 100 million bytes and more, a token tile each at most on average (uneven here: some experts have none, one has
+    several tiles).  Whole numbers: products and sums are exact."""
+    assert E * N * K >= 1e8
+    g = torch.Generator().manual_seed(rows)
+    sizes = [rows * (i % 3) for i in range(E)]
+    sizes[-1] = rows * E - sum(sizes[:-1])
+    offsets = [sum(sizes[:e]) for e in range(E)]
+    a = torch.randint(-2, 3, (rows * E, K), generator=g, dtype=torch.int8).float().to(FP8)
+    w = torch.randint(-2, 3, (E, N, K), generator=g, dtype=torch.int8).half().to(FP8)
+    one = lambda *s: torch.ones(*s)
+    out = _call(gpu, a, w, one(rows * E, K // 128), one(E, (N + 127) // 128, K // 128), sizes, offsets, torch.bfloat16)
+    for e, (m, r0) in enumerate(zip(sizes, offsets)):
+        want = a[r0:r0 + m].to(gpu).float() @ w[e].to(gpu).float().t()
+        assert torch.equal(out[r0:r0 + m], want.bfloat16()), e
+
+
 @pytest.mark.parametrize("num_experts", [8, 16, 32, 64, 128])
 @pytest.mark.parametrize("out_dtype", [torch.half, torch.bfloat16])
 def test_random_expert_sizes(gpu, oracle, num_experts, out_dtype):

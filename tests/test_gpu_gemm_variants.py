@@ -85,6 +85,33 @@ def test_rotated_k(gpu, kind, M, N, K):
     check_exact(gpu, kind, M, N, K)
 
 
+# weights of 100 million bytes and more are loaded as a stream where one token tile reads them: every height of the mid-M tile, K split and
+# whole, the 16-token tile, ragged last channel tiles
+@pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
+@pytest.mark.parametrize("M,N,K", [(13, 7176, 14336), (64, 7176, 18432), (33, 9224, 11264), (40, 36872, 2816), (90, 24584, 4224), (150, 24584, 4224),
+                                   (185, 28680, 3840)])
+def test_streamed_weights(gpu, kind, M, N, K):
+    p = plan_for(kind, M, N, K)
+    assert N * K >= 1e8 and p["kernel"] in ("dma3", "wavesplit_tile") and M <= p["bm"]
+    check_exact(gpu, kind, M, N, K)
+
+
+# the same below the kernels that quantize the tokens themselves: their results are those of a quantizer launch and the GEMM
+@pytest.mark.parametrize("M,N,K", [(2, 7184, 14336), (16, 24576, 7168), (7, 36880, 7168)])
+def test_streamed_weights_of_fused_linears(gpu, M, N, K):
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import per_token_group_quant_fp8, w8a8_block_fp8_matmul
+
+    assert _lib.linear_plan("block", M, N, K)["quantizer"] == "fused" and N * K >= 1e8
+    g = torch.Generator(device=gpu).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+    w = torch.randint(-8, 9, (N, K), generator=g, device=gpu, dtype=torch.int8).half().to(FP8)
+    s = torch.rand((N + 127) // 128, K // 128, generator=g, device=gpu) + 0.5
+    q, qs = per_token_group_quant_fp8(x, 128, column_major_scales=True)
+    two = w8a8_block_fp8_matmul(q, w, qs, s, [128, 128], torch.bfloat16)
+    assert torch.equal(ops.block_fp8_linear(x, w, s, None, torch.bfloat16).view(torch.int16), two.view(torch.int16))
+
+
 # weight in registers: more steps of tokens than the LDS has stages, a last range with fewer, channels that end inside a slice, and fewer
 # tokens than a step
 @pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
