@@ -79,7 +79,7 @@ struct TileShape {
 // One BM x BN output tile at (m0, n0), K blocks of split `split`, by the whole workgroup.
 // AR_UE8M0: p.sa / p.sb point to packed exponent words: token word (m, kw) at sa[kw * sa_sk + m], channel word (n, kw) at
 // sb[kw * sb_sk + n * sb_sn], byte kb & 3 of word kb >> 2 belongs to K block kb.
-template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM = false>
+template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM, bool ROTATES>
 __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, int split) {
   using T = TileShape<AR, BM, BN>;
   static_assert(S >= 3 && S * (T::STAGE_BYTES + BM * 4) <= 160 * 1024, "the stages must fit the CU's LDS");
@@ -119,9 +119,10 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
   const uint32_t sa_off = (uint32_t)min(m0 + wave * (BM / 8) + min(lane, BM / 32 - 1) * 4, (p.M - 1) & ~3) * 4u;
   // The K loop may start in the middle (the sum is the same products in another order): block k of the loop is block
   // (k + rotation) % nkb of the range.  See rotates_k.
-  const int rotation = p.rotate_k ? __builtin_amdgcn_readfirstlane((n0 / BN) % nkb) : 0;
+  const int rotation = ROTATES && p.rotate_k ? __builtin_amdgcn_readfirstlane((n0 / BN) % nkb) : 0;
   auto block_of = [&](int kb) {
     kb = min(kb, kb_last) + rotation;
+    if (!ROTATES) return kb;
     return kb > kb_last ? kb - nkb : kb;
   };
   // Load number i of K block kb (< ROW_LOADS: tile rows; then the token scales) into stage `st`.  The statements write m0; it
@@ -408,10 +409,10 @@ constexpr int stages_of(int bm, int bn, bool own_cu) {
   return bm + bn == 192 ? (own_cu ? 6 : 3) : bm + bn == 224 ? 5 : bm + bn <= 288 ? 4 : 3;
 }
 
-template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM>
+template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM, bool ROTATES>
 __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + BN == 192 && S == 3 ? 4 : 2))) void gemm_dma_kernel(const GemmParams p) {
   const TileCoord tc = tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n);
-  dma_tile<AR, BM, BN, SPLIT, S, STREAM>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
+  dma_tile<AR, BM, BN, SPLIT, S, STREAM, ROTATES>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
 }
 
 // Weight rows a multiple of 4096 bytes apart: with every workgroup at the same K block, all rows being fetched lie at the same place of
@@ -429,21 +430,23 @@ int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   p.rotate_k = rotates_k(p);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
   constexpr int OWN = stages_of(BM, BN, true), SHARED = stages_of(BM, BN, false);
-  const auto launch = [&](auto split, auto streamed) {
-    constexpr bool SPLIT = decltype(split)::value, STREAM = decltype(streamed)::value;
-    if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, SHARED, STREAM>), grid, dim3(T_THREADS), 0, stream, p);
-    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, OWN, STREAM>), grid, dim3(T_THREADS), 0, stream, p);
+  // (a kernel of its own for K loops that start in the middle: the few instructions more cost a chain of short K blocks 5 %, 16 experts of
+  // 36 rows, 3840 -> 256, 17.7 / 18.6 us; the streamed one has them, its blocks wait for memory)
+  const auto launch = [&](auto split, auto streamed, auto rotates) {
+    constexpr bool SPLIT = decltype(split)::value, STREAM = decltype(streamed)::value, ROTATES = decltype(rotates)::value;
+    if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, SHARED, STREAM, ROTATES>), grid, dim3(T_THREADS), 0, stream, p);
+    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, OWN, STREAM, ROTATES>), grid, dim3(T_THREADS), 0, stream, p);
   };
+  const std::true_type yes;
   const std::false_type no;
-  const std::integral_constant<bool, BM == 64> split_streams;
-  if (p.splits > 1) {
-    if (split_streams && streams_weight(p)) launch(std::true_type{}, split_streams);
-    else launch(std::true_type{}, no);
-  } else if (streams_weight(p)) {
-    launch(no, std::true_type{});
-  } else {
-    launch(no, no);
-  }
+  const auto launch_split = [&](auto split) {
+    const std::integral_constant<bool, !decltype(split)::value || BM == 64> may_stream;
+    if (may_stream && streams_weight(p)) launch(split, may_stream, yes);
+    else if (p.rotate_k) launch(split, no, yes);
+    else launch(split, no, no);
+  };
+  if (p.splits > 1) launch_split(yes);
+  else launch_split(no);
   return check_launch(what);
 }
 

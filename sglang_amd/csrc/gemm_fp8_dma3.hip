@@ -295,7 +295,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + 
   GemmParams p;
   int m0, tile_n;
   if (!grouped_tile_of_block(gp, p, m0, tile_n)) return;  // the whole workgroup leaves before any barrier
-  dma_tile<AR_F32, BM, BN, false, S, STREAM>(p, m0, tile_n * BN, 0);
+  dma_tile<AR_F32, BM, BN, false, S, STREAM, false>(p, m0, tile_n * BN, 0);
 }
 
 }  // namespace
