@@ -612,7 +612,7 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
   if (K % KSTEP != 0) {
     if (kind == GK_UNIT || kind == GK_INT8) c = choose_ragged_tile(M, N, K);
   } else if (M <= 16) {
-    c = choose_decode_tile(kind, M, N, K, r.kernel == RK_DMA3, r.kernel == RK_WAVESPLIT);
+    c = choose_decode_tile(kind, M, N, K, TileChoice{r.kernel == RK_DMA3 ? TF_DMA : TF_NONE, r.bm, r.bn, r.splits, 0.0}, r.kernel == RK_WAVESPLIT, r.kernel == RK_DECODE);
   } else {
     TileChoice base{TF_NONE, r.bm, r.bn, r.splits, 0.0};
     // (the table's INT8 time of the 128 x 256 tile is the two-phase kernel's, which does not split K: no base where the plan splits it)
@@ -834,7 +834,8 @@ std::vector<std::string> tile_constant_names() {
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "cold_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "streamed_apart", "streamed_apart_max_kblocks", "streamed_apart_min_tokens", "cold_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+  add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
 }
@@ -1229,7 +1230,7 @@ bool wavesplit_quant_preferred(WavesplitQuant kind, int64_t M, int64_t N, int64_
   const double kb = (double)(K / KSTEP), waves = wavesplit_shape(K).waves;
   const GemmKind gemm = kind == WavesplitQuant::BLOCK_F32 ? GK_F32 : kind == WavesplitQuant::BLOCK_UE8M0 ? GK_UE8M0 : is_fp8 ? GK_UNIT : GK_INT8;
   const int plain = run_route(gemm, M, N, K, K, ldw, true).kernel;
-  if (plain == RK_WAVESPLIT_TILE) return false;
+  if (plain == RK_WAVESPLIT_TILE || streamed_decode(gemm, M, N, K)) return false;
   const bool plain_wavesplit = plain == RK_WAVESPLIT;
   if ((kind == WavesplitQuant::BLOCK_UE8M0 || kind == WavesplitQuant::TOKEN_FP8) && !plain_wavesplit) return false;
   if (kb < route_constants().wavesplit_min_kblocks && (is_fp8 || N / 16 > 512)) return false;  // a block per wave: 512->32768 8.2 against 10.5
@@ -1264,7 +1265,7 @@ bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
 // What a one-call linear does: quantize inside the GEMM kernel, in one of four ways, or by a launch in front of the GEMM.  One
 // function decides for the entry points and for the plan queries.  `gemm` is the GEMM that runs; q_ok: the fused quantizers can
 // read the operands (wavesplit_quant_operands), w_aligned: the weight's base and row stride are multiples of 16 bytes.
-enum LinearMode { LM_LAUNCH, LM_TILE, LM_WAVESPLIT, LM_PRODUCER, LM_STREAMING };
+enum LinearMode { LM_LAUNCH, LM_LAUNCH_STREAMED, LM_TILE, LM_WAVESPLIT, LM_PRODUCER, LM_STREAMING };  // STREAMED: on `gemm`, also where the GEMM alone takes another kernel
 struct LinearRoute {
   LinearMode mode;
   Route gemm;
@@ -1274,6 +1275,19 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
   const Route run = run_route(kind, M, N, K, K, ldw, w_aligned && K % 16 == 0);
   if (!q_ok) return {LM_LAUNCH, run};
   if (tile_quant_preferred(run, M, N, K)) return {LM_TILE, run};
+  // the block linear on a large weight (its own choice, see choose_decode_tile), with the producer waves of the mid-M tile
+  if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && streamed_decode(kind, M, N, K)) {
+    const Route producer = linear_producer_route(M, N, K, ldw);
+    const TileChoice settled{run.kernel == RK_WAVESPLIT_TILE ? TF_WAVESPLIT : producer.kernel == RK_DMA3 ? TF_DMA : TF_NONE, 0,
+                             run.kernel == RK_WAVESPLIT_TILE ? run.bn : producer.bn, 1, 0.0};
+    const TileChoice c = choose_streamed_tile(M, N, K, settled);
+    Route r{};
+    r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
+    r.kernel = c.family == TF_DMA ? RK_DMA3 : RK_WAVESPLIT_TILE;
+    // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks)
+    if (c.family == TF_DMA) return {K % 4096 == 0 ? LM_LAUNCH_STREAMED : LM_PRODUCER, r};
+    return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_STREAMED, r};
+  }
   if (wavesplit_quant_preferred(quant, M, N, K, ldw)) {
     Route r{};
     r.kernel = RK_WAVESPLIT, r.bm = 16, r.bn = wavesplit_two_tiles(quant != WavesplitQuant::TOKEN_INT8, M, N, K) ? 32 : 16, r.splits = 1;
@@ -1346,7 +1360,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   // quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
   const bool w_aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
   const LinearRoute linear = choose_linear(WavesplitQuant::BLOCK_F32, M, N, K, ldw, wavesplit_quant_operands(x, x_dtype, w, ldw), w_aligned);
-  if (linear.mode != LM_LAUNCH) {
+  if (linear.mode != LM_LAUNCH && linear.mode != LM_LAUNCH_STREAMED) {
     GemmParams p;
     bool empty;
     // (a / sa are not read by the kernels in these modes; they only have to satisfy the checks)
@@ -1370,7 +1384,8 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   rc = fp8_mm_params(what, q, w, sa, w_scale, out, out_dtype, M, N, K, K, ldw, 1, pitch, ws_sn, ws_sk, ldo, p, empty);
   if (rc != MI355_OK || empty) return rc;
   p.bias = bias, p.bias_rounded = bias_rounded;
-  return run_gemm<true>(p, q + q_bytes + sa_bytes, workspace_bytes_given - q_bytes - sa_bytes, static_cast<hipStream_t>(stream), what);
+  p.kb_total = p.K / KSTEP;
+  return run_gemm<true>(p, linear.mode == LM_LAUNCH ? call_route(GK_F32, p) : linear.gemm, q + q_bytes + sa_bytes, workspace_bytes_given - q_bytes - sa_bytes, static_cast<hipStream_t>(stream), what);
 }
 }  // namespace
 
@@ -1397,7 +1412,7 @@ int describe_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K, char*
   const bool block = quant == WavesplitQuant::BLOCK_F32 || quant == WavesplitQuant::BLOCK_UE8M0;
   MI355_REQUIRE(K % (block ? KSTEP : 8) == 0, MI355_ERR_INVALID_ARGUMENT, "%s: K must be a multiple of %d", what, block ? KSTEP : 8);
   const LinearRoute r = choose_linear(quant, M, N, K, K, K % 16 == 0, K % 16 == 0);
-  return write_route(r.gemm, M, N, r.mode == LM_LAUNCH ? " quantizer=launch" : " quantizer=fused", buf, buf_len, what);
+  return write_route(r.gemm, M, N, r.mode == LM_LAUNCH || r.mode == LM_LAUNCH_STREAMED ? " quantizer=launch" : " quantizer=fused", buf, buf_len, what);
 }
 }  // namespace
 

@@ -37,6 +37,13 @@ struct TileTimes {
   double cold_ws_channel, cold_ws_token, cold_ws_stream, cold_ws_stream_us, cold_ws_norm;
   double cold_pp_tile, cold_pp_block, cold_pp_busy;
 };
+// Up to 16 tokens, a weight loaded as a stream (choose_streamed_tile): rounds of `tile` + K / 1000 * (channels * channel + tokens * token) and
+// the stream for the 16-token wave-split tiles; rounds of K blocks * (block + channels * block_channel + tokens * block_token), 64 x 128
+// in two workgroups per CU `shared` times, and the stream for the unsplit mid-M tiles of 64 tokens.
+struct StreamedTimes {
+  double tile = 1.55, channel = 0.0201, token = 0.0103, stream = 8.70, stream_us = 3.02, norm = 2.06;
+  double launch = 3.0, block = 0.098, block_channel = 0.00236, block_token = 0.00264, shared = 2.0, mid_stream = 7.06, mid_stream_us = 3.32;
+};
 constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     1.93, 0.586, 4.31, 0.217, 4.18, -4.54, 1.808, 0.421,
     {2.33, 2.83, 3.02, 3.40, 3.53, 4.64, 2.57, 3.31, 3.96, 4.32, 2.64, 3.53, 4.44},
@@ -69,11 +76,13 @@ struct TileLimits {
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
   double resident_margin = 0.93;
+  double streamed_min_weight = 105e6, streamed_min_channels = 8000.0, streamed_one_token_min_kblocks = 63.0, streamed_one_token_min_channels = 11000.0, streamed_one_token_min_weight = 150e6, streamed_two_tokens_min_kblocks = 36.0, streamed_apart = 1.1, streamed_apart_max_kblocks = 32.0, streamed_apart_min_tokens = 4.0;
   double cold_min_weight = 40e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
 struct TileModel {
   TileTimes scaled = SCALED_TIMES, plain = PLAIN_TIMES;
   TileLimits limits;
+  StreamedTimes streamed;
 };
 constexpr int TILE_CONSTANT_COUNT = sizeof(TileModel) / sizeof(double);
 // What the calling thread's dispatcher uses: the defaults above, or the perturbed copy a plan query installed.
@@ -318,6 +327,57 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
   return (double)(N * K) <= l.ragged_max_weight && ws.us < l.ragged_max_factor * best_dma_tile(t, M, N, K).us ? ws : TileChoice{TF_NONE, 0, 0, 1, 0.0};
 }
 
+// Up to 16 tokens on a weight large enough to be loaded as a stream (streams_weight): the wave-split and the mid-M tile have such loads, the
+// register wave-split kernel and the streaming kernel, whose instructions fetch parts of lines, lose by them.  Fitted to 290 linears
+// (100 to 480 million weights): 3 % root mean square; what it chooses takes 1.01 of the best one's time; 103 random ones take 0.86 of what ran before.
+// us, before / this: 18432 -> 14336 at 1 and 16 tokens block FP8 53.5 / 45.2, 64.1 / 47.9, INT8 55.7 / 44.4, 73.7 / 48.9; 8192 -> 14336 at 4 block
+// 36.8 / 23.4, packed exponents 29.3 / 23.4; 7168 -> 36864 at 4 INT8 53.2 / 44.2; 7168 -> 24576 at 8 per-token FP8 40.5 / 32.2; 12672 -> 14208 at 1
+// per-token FP8 40.2 / 30.1.
+// One and two tokens stay on the register kernel where its K is short, one token also on narrow weights up to where that kernel's limits end (at 1: 3584 -> 36864 23.3 / 24.8, 7168 -> 18432 INT8 25.6 / 27.3; 9344 ->
+// 31744 49.8 / 47.2; at 2: 4096 -> 28672 22.8 / 23.7, 7168 -> 36864 INT8 49.2 / 44.3;
+// block FP8 at 2 as at 1, it has the streaming kernel's
+// quantizer; at 4 INT8 4096 -> 28672, rows 4096 bytes apart, 25.2 / 26.0, at 9 per-token FP8 29.3 / 25.1).  Fewer than 8000 channels: the limits of
+// choose_limited_decode_tile hold.
+bool streamed_decode(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+  const TileLimits& l = tile_model().limits;
+  const double kb = (double)ceil_div(K, KSTEP), weight = (double)(N * K);
+  if (M > 16 || K % KSTEP != 0 || N % 16 != 0 || weight < l.streamed_min_weight || (double)N < l.streamed_min_channels) return false;
+  if (M == 1 || (M == 2 && kind == GK_F32))
+    return kb >= l.streamed_one_token_min_kblocks && ((double)N >= l.streamed_one_token_min_channels || weight >= l.streamed_one_token_min_weight);
+  if (M == 2) return kb >= l.streamed_two_tokens_min_kblocks;
+  return (double)M > l.streamed_apart_min_tokens || K % 4096 != 0 || kb > l.streamed_apart_max_kblocks;
+}
+double streamed_mid_us(int64_t M, int64_t N, int64_t K, int bn) {
+  const StreamedTimes& t = tile_model().streamed;
+  const int64_t wg = ceil_div(N, bn);
+  const bool two = bn == 128 && wg > NUM_CUS;
+  const double us = t.launch + (double)ceil_div(wg, two ? 2 * NUM_CUS : NUM_CUS) * (double)ceil_div(K, KSTEP) *
+                                   (t.block + bn * t.block_channel + (double)M * t.block_token) * (two ? t.shared : 1.0);
+  return norm_of(us, (double)(N * K) * 1e-6 / t.mid_stream + t.mid_stream_us, 6.0);
+}
+double streamed_wavesplit_us(int64_t M, int64_t N, int64_t K, int bn) {
+  const StreamedTimes& t = tile_model().streamed;
+  const double us = (double)ceil_div(N, (int64_t)bn * NUM_CUS) * (t.tile + (double)K * 1e-3 * (bn * t.channel + (double)M * t.token));
+  return norm_of(us, (double)(N * K) * 1e-6 / t.stream + t.stream_us, t.norm);
+}
+// `settled`: what runs without this rule where that is one of the two tiles; it stays unless another is 8 % faster (within that the model does
+// not order them: 12672 -> 9728 at 2 tokens 16 x 64 25.6, 16 x 16 27.9; 7168 -> 18432 at 16 64 x 128 29.4, 16 x 32 31.2).  Weight rows a
+// multiple of 4096 bytes apart are the wave-split tile's, up to the weights where choose_limited_decode_tile leaves them, unless the other is 10 %
+// faster (4096 -> 32832 at 7 tokens 31.8 on the register kernel, 34.2 / 26.0).
+TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoice& settled) {
+  const TileLimits& l = tile_model().limits;
+  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+  const auto consider = [&](int family, int bm, int bn, double us) {
+    if (family == settled.family && bn == settled.bn) us *= l.cold_margin;
+    if (us < best.us) best = {family, bm, bn, 1, us};
+  };
+  for (int i = 0; i < 3; ++i) consider(TF_WAVESPLIT, 16, WAVESPLIT_TILES[i].bn, streamed_wavesplit_us(M, N, K, WAVESPLIT_TILES[i].bn));
+  const double apart = K % 4096 == 0 && (double)(N * K) <= l.decode_max_weight ? l.streamed_apart : 1.0;
+  for (int bn = 128; bn <= 256; bn += 64)  // (in one round: 2048 -> 67232 at 13 in 351 workgroups 34.6, the register kernel 29.6)
+    if (ceil_div(N, bn) <= (bn == 128 ? 2 : 1) * NUM_CUS) consider(TF_DMA, 64, bn, apart * streamed_mid_us(M, N, K, bn));
+  return best;
+}
+
 // Up to 16 tokens: the wave-split tile against the kernel the constants table names.  It wins over the streaming and the register
 // wave-split kernel wherever K has more than 16 blocks and the weight is not one of the largest (us, the other / the tile, one
 // token and 16; FP8):
@@ -337,7 +397,7 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
 // The weight limits were drawn at the shapes named beside them.  Measured around them since (K = 2304 .. 18432, 85 to 260 million weights,
 // 1 .. 16 tokens): also beyond them the tile is up to 25 % faster than the streaming and the two-turn register kernel, and slower than
 // the one-turn one; but a linear that leaves those loses their fused quantizers, so the limits stay where the linears were measured.
-TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_mid, bool from_wavesplit) {
+TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_mid, bool from_wavesplit) {
   const TileLimits& l = tile_model().limits;
   const int64_t kb = ceil_div(K, KSTEP);
   const double weight = (double)(N * K);
@@ -362,6 +422,16 @@ TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bo
     if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
   }
   return best;
+}
+
+// `base`: what the constants table names.
+TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool from_wavesplit, bool from_streaming) {
+  const TileChoice c = choose_limited_decode_tile(kind, M, N, K, base.family == TF_DMA, from_wavesplit);
+  // (a bare GEMM with fp32 scales keeps its kernel: the mid-M tile may need a launch that lays the token scales out again.  The one-call
+  // linear of that kind lays them out as it likes: choose_linear.  Packed exponents stay on the streaming kernel where the table names it, 13 to 16
+  // tokens on K of up to 64 blocks that no single round of mid-M tiles covers: 7168 -> 19584 at 13 40.2, per-token FP8 there 40.3 / 33.1)
+  if (kind == GK_F32 || (kind == GK_UE8M0 && from_streaming) || !streamed_decode(kind, M, N, K)) return c;
+  return choose_streamed_tile(M, N, K, c.family != TF_NONE ? c : base);
 }
 
 }  // namespace

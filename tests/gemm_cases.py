@@ -241,7 +241,7 @@ LINEAR_SHAPES = [(1, 128, 128), (15, 128, 1408), (8, 34176, 1536), (2, 18432, 74
                  (13, 25728, 1280), (2, 22400, 6784), (13, 33024, 1152), (2, 33216, 7168), (13, 49536, 1152), (1, 16, 2176), (2, 4144, 2176),
                  (9, 8320, 1024), (1, 16, 128), (4, 12528, 8064), (3, 6720, 128), (3, 13760, 7424), (16, 16, 2688), (16, 4336, 2688),
                  (15, 8336, 2816), (1, 8320, 128), (15, 16, 1280), (12, 16896, 128), (5, 4864, 28800), (3, 14208, 7168), (9, 128, 1152), (17, 16, 128),
-                 (1, 8, 128), (1, 8, 1024), (1, 66304, 128)]
+                 (1, 8, 128), (1, 8, 1024), (1, 66304, 128), (5, 27904, 8192)]
 
 
 def linear_variant_of(plan: dict, M: int):

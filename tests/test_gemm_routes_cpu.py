@@ -175,6 +175,25 @@ def test_large_weights_run_the_faster_tile(kind, shape, want, us, other):
     assert us < other and (p["kernel"], p["bm"], p["bn"], p["splits"]) == want, p
 
 
+# Up to 16 tokens on weights that are loaded as a stream: (linear, shape, kernel and channel tile that have to run, us, what ran otherwise)
+STREAMED_CHOICES = [
+    ("block", (16, 14336, 18432), "wavesplit_tile", 64, 47.9, 64.1), ("block", (4, 14336, 8192), "wavesplit_tile", 64, 24.6, 36.7),
+    ("int8", (4, 36864, 7168), "dma3", 192, 44.2, 53.2), ("token_fp8", (8, 24576, 7168), "wavesplit_tile", 32, 33.4, 39.7),
+    ("ue8m0", (1, 12288, 13312), "wavesplit_tile", 16, 30.3, 38.2),
+    # what stays: short K at one and two tokens, rows 4096 bytes apart, few channels
+    ("block", (1, 36864, 3584), "decode_wavesplit", 16, 23.3, 24.8), ("int8", (2, 28672, 4096), "decode_wavesplit", 16, 22.9, 23.6),
+    ("int8", (4, 28672, 4096), "decode_wavesplit", 16, 25.2, 26.0), ("int8", (2, 9728, 12672), "wavesplit_tile", 64, 25.6, 27.9),
+]
+
+
+@pytest.mark.parametrize("kind,shape,kernel,bn,us,other", STREAMED_CHOICES)
+def test_streamed_weights_run_the_faster_kernel(kind, shape, kernel, bn, us, other):
+    from sglang_amd import _lib
+
+    p = _lib.linear_plan(kind, *shape)
+    assert us < other and (p["kernel"], p["bn"]) == (kernel, bn), p
+
+
 def test_perturbed_plan_query():
     import ctypes
 

@@ -112,6 +112,29 @@ def test_streamed_weights_of_fused_linears(gpu, M, N, K):
     assert torch.equal(ops.block_fp8_linear(x, w, s, None, torch.bfloat16).view(torch.int16), two.view(torch.int16))
 
 
+# the block linear's own choice on such weights, also where the GEMM alone takes another kernel: the wave-split tile quantizing and behind a
+# launch, producer waves, the mid-M tile where the rows lie 4096 bytes apart; the first and the last channels
+@pytest.mark.parametrize("M,N,K", [(2, 16400, 9088), (1, 14352, 12672), (9, 14352, 8320), (16, 18448, 13312), (3, 40960, 3584), (5, 27904, 8192)])
+def test_block_linear_on_streamed_weights(gpu, M, N, K):
+    from fp8_tolerance import check_fp8_gemm
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import per_token_group_quant_fp8
+
+    print(f"case {(M, N, K)} {_lib.block_linear_plan(M, N, K)}", flush=True)
+    assert _lib.block_linear_plan(M, N, K)["kernel"] in ("wavesplit_tile", "dma3")
+    g = torch.Generator(device=gpu).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+    w = torch.randint(-8, 9, (N, K), generator=g, device=gpu, dtype=torch.int8).half().to(FP8)
+    s = torch.rand((N + 127) // 128, K // 128, generator=g, device=gpu) + 0.5
+    out = ops.block_fp8_linear(x, w, s, None, torch.bfloat16)
+    q, qs = per_token_group_quant_fp8(x, 128, column_major_scales=True)  # (the linear's arithmetic: x / s)
+    a = q.double() * qs.double().repeat_interleave(128, 1)
+    for cols in (slice(0, 256), slice((N - 200) // 128 * 128, N)):
+        rows = s[cols.start // 128:(cols.stop + 127) // 128].double().repeat_interleave(128, 0)[:cols.stop - cols.start]
+        b = w[cols].double() * rows.repeat_interleave(128, 1)
+        check_fp8_gemm(out[:, cols], (a @ b.t()).float().cpu(), (a.abs() @ b.abs().t()).float().cpu(), f"{(M, N, K)}")
+
+
 # weight in registers: more steps of tokens than the LDS has stages, a last range with fewer, channels that end inside a slice, and fewer
 # tokens than a step
 @pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
