@@ -227,7 +227,7 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
     }
     const int m = m0 + t * 16 + l16;
     if (m < p.M && n < p.N)
-      *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.out) + (int64_t)m * p.ldo + n) = u32x4{word[0], word[1], word[2], word[3]};
+      store_result(p, reinterpret_cast<uint16_t*>(p.out) + (int64_t)m * p.ldo + n, u32x4{word[0], word[1], word[2], word[3]});
   };
   // fragments and scales of K block kb of half step h (in stage st) into set `set`
   auto read = [&](int set, int st, int h, int kb) __attribute__((always_inline)) {

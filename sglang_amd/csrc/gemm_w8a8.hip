@@ -713,6 +713,7 @@ Route call_route(GemmKind kind, const GemmParams& p) {
 template <bool IS_FP8>
 int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_given, hipStream_t stream, const char* what) {
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
+  p.write_through = writes_through(p);
   const bool aligned = operands_aligned(p);
   const bool wide_scales = (r.kernel == RK_WAVESPLIT_TILE) && p.sa_sm * (int64_t)p.M >= (1ll << 30);  // 32-bit byte offsets
   if (!p.ue8m0 && !p.row_scale && (wide_scales || route_workspace_need(IS_FP8, r, p) > workspace_bytes_given))  // (a workspace for the plan's own splits)
@@ -1182,6 +1183,7 @@ extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa
     p.sa = reinterpret_cast<const float*>(p.a);  // readable filler for the schedule's scale-load slots
     p.sa_sk = 0;
     p.splits = 1, p.kb_per_split = p.kb_total;
+    p.write_through = writes_through(p);
     return launch_fp8_pp_rowcol(p, static_cast<hipStream_t>(stream), what);
   }
   return run_gemm<true>(p, r, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);

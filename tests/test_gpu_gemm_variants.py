@@ -135,6 +135,14 @@ def test_block_linear_on_streamed_weights(gpu, M, N, K):
         check_fp8_gemm(out[:, cols], (a @ b.t()).float().cpu(), (a.abs() @ b.abs().t()).float().cpu(), f"{(M, N, K)}")
 
 
+# results on both sides of the size up to which they are written through the L2, out of every kernel that stores whole rows
+@pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
+@pytest.mark.parametrize("N,K", [(32768, 256), (24584, 896), (8200, 1024)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_results_written_through(gpu, kind, N, K, more):
+    check_exact(gpu, kind, 64000000 // N + more, N, K)
+
+
 # weight in registers: more steps of tokens than the LDS has stages, a last range with fewer, channels that end inside a slice, and fewer
 # tokens than a step
 @pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
