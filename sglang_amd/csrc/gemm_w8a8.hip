@@ -835,7 +835,7 @@ std::vector<std::string> tile_constant_names() {
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "streamed_apart", "streamed_apart_max_kblocks", "streamed_apart_min_tokens", "cold_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "streamed_apart", "streamed_apart_max_kblocks", "streamed_apart_min_tokens", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
@@ -1267,7 +1267,7 @@ bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
 // What a one-call linear does: quantize inside the GEMM kernel, in one of four ways, or by a launch in front of the GEMM.  One
 // function decides for the entry points and for the plan queries.  `gemm` is the GEMM that runs; q_ok: the fused quantizers can
 // read the operands (wavesplit_quant_operands), w_aligned: the weight's base and row stride are multiples of 16 bytes.
-enum LinearMode { LM_LAUNCH, LM_LAUNCH_STREAMED, LM_TILE, LM_WAVESPLIT, LM_PRODUCER, LM_STREAMING };  // STREAMED: on `gemm`, also where the GEMM alone takes another kernel
+enum LinearMode { LM_LAUNCH, LM_LAUNCH_OWN, LM_TILE, LM_WAVESPLIT, LM_PRODUCER, LM_STREAMING };  // OWN: a launch, and `gemm` also where the GEMM alone takes another kernel
 struct LinearRoute {
   LinearMode mode;
   Route gemm;
@@ -1287,8 +1287,14 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
     r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
     r.kernel = c.family == TF_DMA ? RK_DMA3 : RK_WAVESPLIT_TILE;
     // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks)
-    if (c.family == TF_DMA) return {K % 4096 == 0 ? LM_LAUNCH_STREAMED : LM_PRODUCER, r};
-    return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_STREAMED, r};
+    if (c.family == TF_DMA) return {K % 4096 == 0 ? LM_LAUNCH_OWN : LM_PRODUCER, r};
+    return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
+  }
+  if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && run.kernel == RK_DECODE && small_decode(kind, M, N, K, false, true)) {
+    const TileChoice c = best_decode_tile(kind, M, N, K);
+    Route r{};
+    r.kernel = RK_WAVESPLIT_TILE, r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
+    return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
   }
   if (wavesplit_quant_preferred(quant, M, N, K, ldw)) {
     Route r{};
@@ -1362,7 +1368,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   // quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
   const bool w_aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
   const LinearRoute linear = choose_linear(WavesplitQuant::BLOCK_F32, M, N, K, ldw, wavesplit_quant_operands(x, x_dtype, w, ldw), w_aligned);
-  if (linear.mode != LM_LAUNCH && linear.mode != LM_LAUNCH_STREAMED) {
+  if (linear.mode != LM_LAUNCH && linear.mode != LM_LAUNCH_OWN) {
     GemmParams p;
     bool empty;
     // (a / sa are not read by the kernels in these modes; they only have to satisfy the checks)
@@ -1414,7 +1420,7 @@ int describe_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K, char*
   const bool block = quant == WavesplitQuant::BLOCK_F32 || quant == WavesplitQuant::BLOCK_UE8M0;
   MI355_REQUIRE(K % (block ? KSTEP : 8) == 0, MI355_ERR_INVALID_ARGUMENT, "%s: K must be a multiple of %d", what, block ? KSTEP : 8);
   const LinearRoute r = choose_linear(quant, M, N, K, K, K % 16 == 0, K % 16 == 0);
-  return write_route(r.gemm, M, N, r.mode == LM_LAUNCH || r.mode == LM_LAUNCH_STREAMED ? " quantizer=launch" : " quantizer=fused", buf, buf_len, what);
+  return write_route(r.gemm, M, N, r.mode == LM_LAUNCH || r.mode == LM_LAUNCH_OWN ? " quantizer=launch" : " quantizer=fused", buf, buf_len, what);
 }
 }  // namespace
 

@@ -77,6 +77,7 @@ struct TileLimits {
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
   double resident_margin = 0.93;
   double streamed_min_weight = 105e6, streamed_min_channels = 8000.0, streamed_one_token_min_kblocks = 63.0, streamed_one_token_min_channels = 11000.0, streamed_one_token_min_weight = 150e6, streamed_two_tokens_min_kblocks = 36.0, streamed_apart = 1.1, streamed_apart_max_kblocks = 32.0, streamed_apart_min_tokens = 4.0;
+  double small_min_kblocks = 4.0, small_min_tokens = 4.0, small_min_channels = 192.0, small_max_tokens_values = 20800.0;
   double cold_min_weight = 40e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
 struct TileModel {
@@ -378,6 +379,33 @@ TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoic
   return best;
 }
 
+// K of 4 to 16 blocks on weights of up to 20 million values, which the launches bound: the tile quantizes the tokens in its one launch and takes
+// their scales as they lie.  260 linears of 1 to 16 tokens, K = 512 to 2176, the tile's time by what it takes over from (geometric mean):
+//   the register kernel: K below 8 blocks FP8 0.66, INT8 0.83 from 9 tokens on (below 1.04); from 8 blocks on 0.87 at 9 to 16 tokens, per-token
+//   kinds 0.88 at 5 to 8 (block FP8 0.92, at most 1.08, and packed exponents 0.99: left), 1.03 at fewer; with more than five pieces of eight
+//   values a thread (20800 in all) the quantizer in every workgroup takes longer than its launch (2048 -> 4096 at 16 tokens 5.8 / 8.2);
+//   the streaming kernel: per-token FP8 0.67; fp32 scales 0.81 from 8 blocks and 9 tokens on.  Packed exponents and shorter K with fp32 scales
+//   stay on it, 128 channels too, which are eight workgroups.
+bool small_decode(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_wavesplit, bool from_streaming) {
+  const TileLimits& l = tile_model().limits;
+  const int64_t kb = ceil_div(K, KSTEP);
+  if (M > 16 || K % KSTEP != 0 || (double)(N * K) > l.decode_short_max_weight || (double)kb < l.small_min_kblocks || (double)kb > l.decode_min_kblocks) return false;
+  const bool short_k = (double)kb < l.decode_short_min_kblocks, many = (double)M > l.decode_short_min_tokens;
+  if (from_wavesplit && !short_k && (double)(M * K) > l.small_max_tokens_values) return false;
+  if (from_wavesplit) return many || (short_k ? kind != GK_INT8 : (kind == GK_UNIT || kind == GK_INT8) && (double)M > l.small_min_tokens);
+  return from_streaming && (double)N >= l.small_min_channels && (kind == GK_UNIT || (kind == GK_F32 && many && !short_k));
+}
+TileChoice best_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+  const TileTimes& t = tile_times(kind);
+  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+  for (int i = 0; i < 3; ++i) {
+    static_assert(WAVESPLIT_TILES[2].bm == 16, "the 16-token tiles come first");
+    const double us = wavesplit_tile_us(t, i, M, N, K, best.us);
+    if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
+  }
+  return best;
+}
+
 // Up to 16 tokens: the wave-split tile against the kernel the constants table names.  It wins over the streaming and the register
 // wave-split kernel wherever K has more than 16 blocks and the weight is not one of the largest (us, the other / the tile, one
 // token and 16; FP8):
@@ -397,7 +425,7 @@ TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoic
 // The weight limits were drawn at the shapes named beside them.  Measured around them since (K = 2304 .. 18432, 85 to 260 million weights,
 // 1 .. 16 tokens): also beyond them the tile is up to 25 % faster than the streaming and the two-turn register kernel, and slower than
 // the one-turn one; but a linear that leaves those loses their fused quantizers, so the limits stay where the linears were measured.
-TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_mid, bool from_wavesplit) {
+TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_mid, bool from_wavesplit, bool from_streaming) {
   const TileLimits& l = tile_model().limits;
   const int64_t kb = ceil_div(K, KSTEP);
   const double weight = (double)(N * K);
@@ -410,23 +438,18 @@ TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64
     return TileChoice{TF_NONE, 0, 0, 1, 0.0};
   const bool few = (double)M <= (kind == GK_F32 ? l.decode_few_tokens_f32 : l.decode_few_tokens) && (double)kb <= l.decode_long_kblocks;
   const double most = padded ? l.decode_padded_max_weight : few ? l.decode_few_tokens_max_weight : l.decode_max_weight;
-  const bool take = (double)kb > l.decode_min_kblocks ? weight <= most
+  // (from the streaming kernel not a bare GEMM with fp32 scales: the one-call linear takes the tile for itself, choose_linear)
+  const bool small = small_decode(kind, M, N, K, from_wavesplit, from_streaming && kind != GK_F32);
+  const bool take = small || ((double)kb > l.decode_min_kblocks ? weight <= most
                                                       : (double)kb >= l.decode_short_min_kblocks && (double)N >= l.decode_short_min_channels &&
-                                                            weight <= l.decode_short_max_weight && (double)M > l.decode_short_min_tokens;
+                                                            weight <= l.decode_short_max_weight && (double)M > l.decode_short_min_tokens);
   if (!take) return TileChoice{TF_NONE, 0, 0, 1, 0.0};
-  const TileTimes& t = tile_times(kind);
-  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
-  for (int i = 0; i < 3; ++i) {
-    static_assert(WAVESPLIT_TILES[2].bm == 16, "the 16-token tiles come first");
-    const double us = wavesplit_tile_us(t, i, M, N, K, best.us);
-    if (us < best.us) best = {TF_WAVESPLIT, WAVESPLIT_TILES[i].bm, WAVESPLIT_TILES[i].bn, 1, us};
-  }
-  return best;
+  return best_decode_tile(kind, M, N, K);
 }
 
 // `base`: what the constants table names.
 TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool from_wavesplit, bool from_streaming) {
-  const TileChoice c = choose_limited_decode_tile(kind, M, N, K, base.family == TF_DMA, from_wavesplit);
+  const TileChoice c = choose_limited_decode_tile(kind, M, N, K, base.family == TF_DMA, from_wavesplit, from_streaming);
   // (a bare GEMM with fp32 scales keeps its kernel: the mid-M tile may need a launch that lays the token scales out again.  The one-call
   // linear of that kind lays them out as it likes: choose_linear.  Packed exponents stay on the streaming kernel where the table names it, 13 to 16
   // tokens on K of up to 64 blocks that no single round of mid-M tiles covers: 7168 -> 19584 at 13 40.2, per-token FP8 there 40.3 / 33.1)

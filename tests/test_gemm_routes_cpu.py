@@ -194,6 +194,22 @@ def test_streamed_weights_run_the_faster_kernel(kind, shape, kernel, bn, us, oth
     assert us < other and (p["kernel"], p["bn"]) == (kernel, bn), p
 
 
+# Small layers of short K at decode sizes: (linear, shape, kernel that has to run, us a call, what ran otherwise)
+SMALL_CHOICES = [
+    ("ue8m0", (13, 5888, 1536), "wavesplit_tile", 6.5, 8.1), ("int8", (7, 1088, 1024), "wavesplit_tile", 4.5, 5.3), ("ue8m0", (7, 1600, 640), "wavesplit_tile", 5.3, 8.4),
+    ("token_fp8", (16, 4288, 1280), "wavesplit_tile", 6.8, 8.7), ("block", (15, 1408, 1920), "wavesplit_tile", 7.4, 11.7),
+    # what stays: few tokens with K of 8 blocks and more (4.7, the tile no faster), many token values a workgroup
+    ("block", (2, 2688, 1280), "decode_wavesplit", 4.7, 4.8), ("block", (16, 4096, 2048), "decode_wavesplit", 5.8, 8.2),
+]
+
+
+@pytest.mark.parametrize("kind,shape,kernel,us,other", SMALL_CHOICES)
+def test_small_layers_run_the_faster_kernel(kind, shape, kernel, us, other):
+    from sglang_amd import _lib
+
+    assert us < other and _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
+
+
 def test_perturbed_plan_query():
     import ctypes
 
