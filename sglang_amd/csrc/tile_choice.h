@@ -334,10 +334,10 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
 // us, before / this: 18432 -> 14336 at 1 and 16 tokens block FP8 53.5 / 45.2, 64.1 / 47.9, INT8 55.7 / 44.4, 73.7 / 48.9; 8192 -> 14336 at 4 block
 // 36.8 / 23.4, packed exponents 29.3 / 23.4; 7168 -> 36864 at 4 INT8 53.2 / 44.2; 7168 -> 24576 at 8 per-token FP8 40.5 / 32.2; 12672 -> 14208 at 1
 // per-token FP8 40.2 / 30.1.
-// One and two tokens stay on the register kernel where its K is short, one token also on narrow weights up to where that kernel's limits end (at 1: 3584 -> 36864 23.3 / 24.8, 7168 -> 18432 INT8 25.6 / 27.3; 9344 ->
-// 31744 49.8 / 47.2; at 2: 4096 -> 28672 22.8 / 23.7, 7168 -> 36864 INT8 49.2 / 44.3;
-// block FP8 at 2 as at 1, it has the streaming kernel's
-// quantizer; at 4 INT8 4096 -> 28672, rows 4096 bytes apart, 25.2 / 26.0, at 9 per-token FP8 29.3 / 25.1).  Fewer than 8000 channels: the limits of
+// One and two tokens stay on the register kernel where its K is short, one token also on narrow weights up to where that kernel's limits end
+// (at 1: 3584 -> 36864 23.3 / 24.8, 7168 -> 18432 INT8 25.6 / 27.3, but 9344 -> 31744 49.8 / 47.2; at 2: 4096 -> 28672 22.8 / 23.7, but 7168 ->
+// 36864 INT8 49.2 / 44.3; block FP8 at 2 as at 1, it has the streaming kernel's quantizer); so do up to four on rows 4096 bytes apart with
+// one turn of K (at 4 INT8 4096 -> 28672 25.2 / 26.0, at 9 per-token FP8 29.3 / 25.1).  Fewer than 8000 channels: the limits of
 // choose_limited_decode_tile hold.
 bool streamed_decode(GemmKind kind, int64_t M, int64_t N, int64_t K) {
   const TileLimits& l = tile_model().limits;
