@@ -43,7 +43,7 @@ struct GemmParams {
   int kb_total, kb_per_split, splits;
   int tiles_m, tiles_n;
   int rotate_k;  // mid-M tile: the K loops of different channel tiles start at different blocks
-  int write_through;  // whole-row 16-bit results leave through the L2 (writes_through)
+  int write_through;  // whole-row 16-bit results leave through the L2 (writes_through; set where the shape is, so that no launch misses it)
   int out_dtype;
   int ue8m0;  // FP8 only: sa / sb are packed exponent words and the route's kernel applies them in the MFMA (set by the UE8M0 entry point)
 };
@@ -435,9 +435,10 @@ int launch_fp8_dma3_quant(GemmParams& p, int bn, hipStream_t stream, const char*
 // Whether whole-row results are written through the L2 (sc1 stores).  Left dirty there, up to 32 MB of them are written back at the end of the
 // kernel, when nothing else runs.  Linears, us, and the same with a quantizer that reads the result behind them, left / written through: block
 // FP8 512 -> 32768 at 200 tokens 12.8 / 12.0, 20.0 / 17.4, at 400 16.6 / 15.2, 25.7 / 22.4, at 1500 36.4 / 31.3, 58.4 / 53.6; 1536 -> 24576 at 387
-// 25.9 / 24.9, 31.8 / 30.6; 4096 -> 6144 at 2048 55.0 / 54.0, 61.6 / 61.0.  Not beyond 128 MB: 197 MB (3001 tokens) alone 65.9 / 59.1, but with
+// 25.9 / 24.9, 31.8 / 30.6; 4096 -> 6144 at 2048 55.0 / 54.0, 61.6 / 61.0; packed exponents 1536 -> 24576 at 387 28.2 / 27.5, 32.5 / 31.6, at 2048
+// 86.7 / 84.5, 106.8 / 105.7, 896 -> 24576 at 2603 96.9 / 93.7, 117.3 / 117.2.  Not beyond 128 MB: 197 MB (3001 tokens) alone 65.9 / 59.1, but with
 // the reader 107.9 / 112.6, which then finds less in the 256 MB Infinity Cache; nontemporal stores bypass that altogether (61.7, 119.6).
-inline bool writes_through(const GemmParams& p) { return (int64_t)p.M * p.N * 2 <= 128000000; }
+inline bool writes_through(int64_t rows, int64_t channels) { return rows * channels * 2 <= 128000000; }
 // Whether a launch loads its weight with nontemporal loads: a large one that every workgroup reads a part of its own of.  Such loads leave
 // nothing behind in the 256 MB Infinity Cache, and what has to come from memory comes faster: 264 MB read by 256 workgroups at 6.2
 // instead of 5.65 TB/s.  Linears, us, without / with: block FP8 7168 -> 36864 at 8 tokens 48.6 / 43.6, 4096 -> 28672 at 32 and 128 30.2 / 26.7,

@@ -713,7 +713,6 @@ Route call_route(GemmKind kind, const GemmParams& p) {
 template <bool IS_FP8>
 int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_given, hipStream_t stream, const char* what) {
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
-  p.write_through = writes_through(p);
   const bool aligned = operands_aligned(p);
   const bool wide_scales = (r.kernel == RK_WAVESPLIT_TILE) && p.sa_sm * (int64_t)p.M >= (1ll << 30);  // 32-bit byte offsets
   if (!p.ue8m0 && !p.row_scale && (wide_scales || route_workspace_need(IS_FP8, r, p) > workspace_bytes_given))  // (a workspace for the plan's own splits)
@@ -937,6 +936,7 @@ int fp8_mm_params(const char* what, const void* a, const void* b, const float* s
   p.b = static_cast<const uint8_t*>(b);
   p.sa = sa, p.sb = sb, p.bias = nullptr, p.out = out, p.ws = nullptr;
   p.M = (int)M, p.N = (int)N, p.K = (int)K;
+  p.write_through = writes_through(M, N);
   p.lda = lda, p.ldb = ldb, p.ldo = ldo;
   p.sa_sm = sa_sm, p.sa_sk = sa_sk, p.sb_sn = sb_sn, p.sb_sk = sb_sk;
   p.out_dtype = out_dtype;
@@ -1183,7 +1183,6 @@ extern "C" int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa
     p.sa = reinterpret_cast<const float*>(p.a);  // readable filler for the schedule's scale-load slots
     p.sa_sk = 0;
     p.splits = 1, p.kb_per_split = p.kb_total;
-    p.write_through = writes_through(p);
     return launch_fp8_pp_rowcol(p, static_cast<hipStream_t>(stream), what);
   }
   return run_gemm<true>(p, r, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
@@ -1464,6 +1463,7 @@ extern "C" int mi355_int8_scaled_mm(const void* a, const void* b, const float* s
   p.b = static_cast<const uint8_t*>(b);
   p.sa = sa, p.sb = sb, p.bias = bias, p.out = out, p.ws = nullptr;
   p.M = (int)M, p.N = (int)N, p.K = (int)K;
+  p.write_through = writes_through(M, N);
   p.lda = lda, p.ldb = ldb, p.ldo = ldo;
   p.out_dtype = out_dtype;
   return run_gemm<false>(p, workspace, workspace_bytes_given, static_cast<hipStream_t>(stream), what);
@@ -1502,6 +1502,7 @@ extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, cons
   p.b = static_cast<const uint8_t*>(w);
   p.sa = sa, p.sb = w_scale, p.bias = bias, p.out = out, p.ws = nullptr;
   p.M = (int)M, p.N = (int)N, p.K = (int)K;
+  p.write_through = writes_through(M, N);
   p.lda = K, p.ldb = ldw, p.ldo = ldo;
   p.out_dtype = out_dtype;
   const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);

@@ -135,12 +135,22 @@ def test_block_linear_on_streamed_weights(gpu, M, N, K):
         check_fp8_gemm(out[:, cols], (a @ b.t()).float().cpu(), (a.abs() @ b.abs().t()).float().cpu(), f"{(M, N, K)}")
 
 
-# results on both sides of the size up to which they are written through the L2, out of every kernel that stores whole rows
+# results on both sides of the size up to which they are written through the L2: the weight-in-registers and the two-phase kernels
 @pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
 @pytest.mark.parametrize("N,K", [(32768, 256), (24584, 896), (8200, 1024)])
 @pytest.mark.parametrize("more", [0, 1])
 def test_results_written_through(gpu, kind, N, K, more):
     check_exact(gpu, kind, 64000000 // N + more, N, K)
+
+
+# the same out of the mid-M and the 128-token kernel, and with the kernel named where packed exponents go straight to the two-phase one
+@pytest.mark.parametrize("kind,N,K,kernel", [("fp8", 13592, 128, "dma3"), ("fp8_ue8m0", 13592, 128, "dma3"), ("fp8_scaled", 65584, 128, "dma3"),
+                                             ("int8", 65584, 768, "pingpong128"), ("fp8_ue8m0", 24584, 1024, "pingpong")])
+@pytest.mark.parametrize("more", [0, 1])
+def test_results_written_through_by_kernel(gpu, kind, N, K, kernel, more):
+    M = 64000000 // N + more
+    assert plan_for(kind, M, N, K)["kernel"] == kernel
+    check_exact(gpu, kind, M, N, K)
 
 
 # weight in registers: more steps of tokens than the LDS has stages, a last range with fewer, channels that end inside a slice, and fewer
