@@ -436,7 +436,8 @@ int launch_fp8_dma3_quant(GemmParams& p, int bn, hipStream_t stream, const char*
 // kernel, when nothing else runs.  Linears, us, and the same with a quantizer that reads the result behind them, left / written through: block
 // FP8 512 -> 32768 at 200 tokens 12.8 / 12.0, 20.0 / 17.4, at 400 16.6 / 15.2, 25.7 / 22.4, at 1500 36.4 / 31.3, 58.4 / 53.6; 1536 -> 24576 at 387
 // 25.9 / 24.9, 31.8 / 30.6; 4096 -> 6144 at 2048 55.0 / 54.0, 61.6 / 61.0; packed exponents 1536 -> 24576 at 387 28.2 / 27.5, 32.5 / 31.6, at 2048
-// 86.7 / 84.5, 106.8 / 105.7, 896 -> 24576 at 2603 96.9 / 93.7, 117.3 / 117.2.  Not beyond 128 MB: 197 MB (3001 tokens) alone 65.9 / 59.1, but with
+// 86.7 / 84.5, 106.8 / 105.7, 896 -> 24576 at 2603 96.9 / 93.7, 117.3 / 117.2; grouped (of all experts' rows) 8 experts, 2048 rows, 512 -> 4096
+// 26.0 / 23.2, 28.1 / 27.9, 64 experts, 8192 rows, 512 -> 4096 72.6 / 69.1, 87.0 / 84.2.  Not beyond 128 MB: 197 MB (3001 tokens) alone 65.9 / 59.1, but with
 // the reader 107.9 / 112.6, which then finds less in the 256 MB Infinity Cache; nontemporal stores bypass that altogether (61.7, 119.6).
 inline bool writes_through(int64_t rows, int64_t channels) { return rows * channels * 2 <= 128000000; }
 // Whether a launch loads its weight with nontemporal loads: a large one that every workgroup reads a part of its own of.  Such loads leave

@@ -343,6 +343,7 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
   gp.g.sa_sm = 1, gp.g.sa_sk = pl.pitch, gp.g.sb_sn = sb_sn, gp.g.sb_sk = sb_sk;
   gp.g.kb_total = KB;
   gp.g.out_dtype = out_dtype;
+  gp.g.write_through = writes_through(total_m, N);
   gp.b_expert_stride = b_expert_stride;
   gp.sb_expert_stride = sb_expert_stride;
   gp.out_elem = 2;

@@ -90,6 +90,21 @@ def test_streamed_expert_weights(gpu, E, rows, N, K):
         assert torch.equal(out[r0:r0 + m], want.bfloat16()), e
 
 
+@pytest.mark.parametrize("rows", [15625, 15626])
+def test_results_written_through(gpu, rows):
+    """Results of all experts on both sides of the size (128 MB) up to which they are written through the L2.  Whole numbers, exact."""
+    E, N, K = 4, 4096, 256
+    g = torch.Generator().manual_seed(rows)
+    sizes = [1000, 70, 6500, rows - 7570]
+    offsets = [sum(sizes[:e]) for e in range(E)]
+    a = torch.randint(-2, 3, (rows, K), generator=g, dtype=torch.int8).float().to(FP8)
+    w = torch.randint(-2, 3, (E, N, K), generator=g, dtype=torch.int8).half().to(FP8)
+    out = _call(gpu, a, w, torch.ones(rows, K // 128), torch.ones(E, N // 128, K // 128), sizes, offsets, torch.bfloat16)
+    for e, (m, r0) in enumerate(zip(sizes, offsets)):
+        want = a[r0:r0 + m].to(gpu).float() @ w[e].to(gpu).float().t()
+        assert torch.equal(out[r0:r0 + m], want.bfloat16()), e
+
+
 @pytest.mark.parametrize("num_experts", [8, 16, 32, 64, 128])
 @pytest.mark.parametrize("out_dtype", [torch.half, torch.bfloat16])
 def test_random_expert_sizes(gpu, oracle, num_experts, out_dtype):
