@@ -166,9 +166,9 @@ int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* b, const fl
  *   bias      NULL or [N] in the output dtype, added in the epilogue
  * On gfx950 the matrix instruction applies such scales itself (v_mfma_scale_f32_16x16x128_f8f6f4), so for large M, for
  * the mid-M shapes on the three-stage kernel and for the decode sizes (M <= 16, both decode kernels) the K loop carries
- * no scale arithmetic at all and nothing runs in front of the GEMM (K % 128 == 0 and, above decode sizes, token words
- * with a 16-byte aligned base and a pitch that is a multiple of four words); other shapes (ragged K, the generic and
- * the two-stage kernels' shapes) expand the exponents to fp32 scales in the workspace and take the kernels of
+ * no scale arithmetic at all and nothing runs in front of the GEMM (K % 128 == 0 and, where no kernel that reads any pitch
+ * serves the shape, token words with a 16-byte aligned base and a pitch that is a multiple of four words); other shapes
+ * (ragged K, the generic and the two-stage kernels' shapes) expand the exponents to fp32 scales in the workspace and take the kernels of
  * mi355_fp8_blockwise_mm.  Replaces w8a8_block_fp8_matmul_deepgemm / deep_gemm gemm_nt_f8f8bf16
  * (python/sglang/srt/layers/quantization/fp8_kernel.py:1047-1065; caller deepgemm_w8a8_block_fp8_linear_with_fallback,
  * fp8_utils.py:217-255), whose kernel lives in the DeepGEMM package, not in the reference tree.
@@ -252,7 +252,7 @@ int mi355_int8_scaled_mm(const void* a, const void* b, const float* sa, const fl
  * here the choice is observable so that tests can prove every kernel variant is reached.
  *   aligned  nonzero if both operand base pointers and row strides are multiples of 16 bytes (rows are assumed dense)
  *   buf      receives a NUL-terminated "key=value ..." line:
- *            kernel=decode|decode_wavesplit|wavesplit_tile|dma3|pingpong|pingpong128|pipelined|generic bm= bn= splits=
+ *            kernel=decode|decode_wavesplit|wavesplit_tile|dma3|resident|pingpong|pingpong128|pipelined|generic bm= bn= splits=
  *            kb_per_split= groups_per_wg= aligned= stages=   (stages: LDS stages of the mid-M kernel's pipeline, 0 for the
  *            other kernels) and for UE8M0 exponents=mfma|unpacked (unpacked: a launch in front expands them to fp32 scales)
  * Launches nothing and touches no device state.

@@ -605,7 +605,10 @@ Route choose_route(bool is_fp8, int64_t M, int64_t N, int64_t K, int64_t lda, in
 }
 
 // The route that runs: choose_route's, or the tile that models faster (tile_choice.h).
-Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned, bool resident) {
+// `resident`: the output and what the epilogue reads are such that the resident-weight kernel can store it (resident_operands_ok).
+// `conforming`: the token scales lie as the direct-to-LDS kernels read them, or are laid out for them.  Packed exponents that do not
+// are expanded by a launch, so they stay on a kernel that reads any pitch wherever choose_limited_decode_tile or choose_swept_tile name one.
+Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned, bool resident, bool conforming) {
   Route r = choose_route(kind != GK_INT8, M, N, K, lda, ldb, aligned);
   if (!aligned || M * lda >= (1ll << 32) || N * ldb >= (1ll << 32)) return r;
   TileChoice c{TF_NONE, 0, 0, 1, 0.0};
@@ -613,6 +616,7 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
     if (kind == GK_UNIT || kind == GK_INT8) c = choose_ragged_tile(M, N, K);
   } else if (M <= 16) {
     c = choose_decode_tile(kind, M, N, K, TileChoice{r.kernel == RK_DMA3 ? TF_DMA : TF_NONE, r.bm, r.bn, r.splits, 0.0}, r.kernel == RK_WAVESPLIT, r.kernel == RK_DECODE);
+    if (!conforming && c.family == TF_DMA) c = choose_limited_decode_tile(kind, M, N, K, r.kernel == RK_DMA3, r.kernel == RK_WAVESPLIT, r.kernel == RK_DECODE);
   } else {
     TileChoice base{TF_NONE, r.bm, r.bn, r.splits, 0.0};
     // (the table's INT8 time of the 128 x 256 tile is the two-phase kernel's, which does not split K: no base where the plan splits it)
@@ -620,6 +624,11 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
     if (r.kernel == RK_PP128 || (r.kernel == RK_DMA3 && !split_128x256)) base.family = TF_DMA;
     if (r.kernel == RK_PINGPONG) base.family = TF_TWO_PHASE;
     c = choose_mid_tile(kind, M, N, K, base, resident);
+    if (!conforming && c.family != TF_WAVESPLIT) {
+      double base_us;
+      const TileChoice swept = choose_swept_tile(kind, M, N, K, base, base_us);
+      if (swept.family == TF_WAVESPLIT) c = swept;
+    }
   }
   if (c.family == TF_NONE) return r;
   r.kernel = c.family == TF_DMA ? RK_DMA3 : c.family == TF_WAVESPLIT ? RK_WAVESPLIT_TILE : c.family == TF_RESIDENT ? RK_RESIDENT : RK_PINGPONG;
@@ -628,20 +637,19 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
   r.kb_per_split = (int)((kb + c.splits - 1) / c.splits);
   return r;
 }
-// `resident`: the output and what the epilogue reads are such that the resident-weight kernel can store it (resident_operands_ok).
-Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned, bool resident = true) {
-  if (dispatch_perturbed()) return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident);
+Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool aligned, bool resident = true, bool conforming = true) {
+  if (dispatch_perturbed()) return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident, conforming);
   struct Key : ShapeKey {
     int64_t lda, ldb;
-    bool aligned, resident;
+    bool aligned, resident, conforming;
     bool operator==(const Key& o) const {
-      return ShapeKey::operator==(o) && lda == o.lda && ldb == o.ldb && aligned == o.aligned && resident == o.resident;
+      return ShapeKey::operator==(o) && lda == o.lda && ldb == o.ldb && aligned == o.aligned && resident == o.resident && conforming == o.conforming;
     }
   };
   static thread_local RecentShapes<Key, Route> table;
   if (kind == GK_UE8M0 && M > 16) kind = GK_F32;  // above decode sizes both kinds have one model
   if (M <= 16 || K > RESIDENT_MAX_KBLOCKS * KSTEP) resident = true;  // (does not matter: one entry)
-  return table.get(Key{{M, N, K, (int)kind}, lda, ldb, aligned, resident}, [&] { return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident); });
+  return table.get(Key{{M, N, K, (int)kind}, lda, ldb, aligned, resident, conforming}, [&] { return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident, conforming); });
 }
 // K splits of the plan, whichever way the output decides
 int run_splits(GemmKind kind, int64_t M, int64_t N, int64_t K) {
@@ -706,8 +714,8 @@ bool operands_aligned(const GemmParams& p) {
 }
 
 // The route of a call, once its operands (bias and channel scales too) are in p.
-Route call_route(GemmKind kind, const GemmParams& p) {
-  return run_route(kind, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p), resident_operands_ok(kind, p));
+Route call_route(GemmKind kind, const GemmParams& p, bool conforming = true) {
+  return run_route(kind, p.M, p.N, p.K, p.lda, p.ldb, operands_aligned(p), resident_operands_ok(kind, p), conforming);
 }
 
 template <bool IS_FP8>
@@ -1067,8 +1075,8 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
   p.bias = bias, p.bias_rounded = bias_rounded;
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
-  const Route r = call_route(GK_UE8M0, p);
   const bool words_conform = (sa_sk & 3) == 0 && sa_sk >= ((M + 3) & ~3ll) && (reinterpret_cast<uintptr_t>(sa_words) & 15) == 0;
+  const Route r = call_route(GK_UE8M0, p, words_conform);
   const bool wants_conforming = r.kernel == RK_PINGPONG || r.kernel == RK_DMA3 || r.kernel == RK_RESIDENT;  // (the decode kernels read the words with ordinary loads: any pitch will do)
   if (applies_exponents(r, K) && (words_conform || !wants_conforming)) {
     // the MFMA applies both exponents itself: no scale arithmetic at all, and the workspace only holds split-K partial sums

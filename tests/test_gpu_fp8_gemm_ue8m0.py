@@ -258,3 +258,32 @@ def test_w8a8_block_fp8_matmul_takes_packed_scales(gpu, oracle, M, N, K):
         check_fp8_gemm(mixed[rows.to(gpu)], ref, mag, f"mixed scales M={M} N={N} K={K}")
     with pytest.raises(AssertionError):
         w8a8_block_fp8_matmul(x_q, w2, sa_words[:, :0], sb_words, [128, 128], torch.bfloat16)
+
+
+# (kernel that the shape takes with conforming words, shape): decode sizes on a large weight, and a weight of medium size above them
+@pytest.mark.parametrize("conforming_kernel,M,N,K", [("dma3", 11, 25248, 11008), ("dma3", 3, 42496, 2560), ("dma3", 84, 5456, 10240), ("dma3", 79, 3600, 16128)])
+def test_token_words_of_any_pitch_without_a_launch_in_front(gpu, M, N, K, conforming_kernel):
+    """Token words whose pitch is no multiple of four: where a kernel that reads any pitch serves the shape, it takes the words as they
+    lie, with no workspace at all.  Whole numbers and powers of two: exact."""
+    import ctypes
+
+    from sglang_amd import _lib
+
+    assert _lib.gemm_plan("fp8_ue8m0", M, N, K)["kernel"] == conforming_kernel
+    g = torch.Generator(device=gpu).manual_seed(M)
+    a, w = (torch.randint(-2, 3, s, generator=g, device=gpu, dtype=torch.int8) for s in ((M, K), (N, K)))
+    kb, nb = K // 128, -(-N // 128)
+    ea, eb = (torch.randint(125, 130, s, generator=g, device=gpu, dtype=torch.int32).to(torch.uint8) for s in ((M, kb), (nb, kb)))
+    kw, pitch = -(-kb // 4), M + 1 if M % 4 != 3 else M + 2
+    words = torch.zeros(kw, pitch, 4, dtype=torch.uint8, device=gpu)
+    words[:, :M].view(kw, M, 4).copy_(torch.nn.functional.pad(ea, (0, 4 * kw - kb)).view(M, kw, 4).transpose(0, 1))
+    sb = torch.nn.functional.pad(eb, (0, 4 * kw - kb)).repeat_interleave(128, 0)[:N].contiguous()
+    a8, w8 = a.half().to(FP8), w.half().to(FP8)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = _lib.lib().mi355_fp8_blockwise_mm_ue8m0(ptr(a8), ptr(w8), ptr(words), ptr(sb), None, ptr(out), 2, M, N, K, K, K, pitch, kw, 1, N, None, 0,
+                                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, _lib.lib().mi355_last_error()
+    ta = torch.exp2(ea.double() - 127).repeat_interleave(128, 1) * a
+    tb = torch.exp2(eb.double() - 127).repeat_interleave(128, 1).repeat_interleave(128, 0)[:N] * w
+    assert torch.equal(out, (ta @ tb.t()).bfloat16())
