@@ -836,13 +836,13 @@ std::vector<std::string> tile_constant_names() {
     add(times, {"pp_tile", "pp_block", "pp_busy", "pp_store", "ws_launch", "ws_tile", "ws_kb", "ws_kb_busy", "ws_stream", "ws_stream_us",
                 "ws_result", "ws_norm", "rs_launch", "rs_tile", "rs_tile_block", "rs_step", "rs_step_block", "rs_busy",
                 "cold", "cold_channel", "cold_token", "cold_shared", "cold_stream", "cold_stream_us", "cold_again", "cold_split_us", "cold_split_us_per_mb",
-                "cold_ws_channel", "cold_ws_token", "cold_ws_stream", "cold_ws_stream_us", "cold_ws_norm", "cold_pp_tile", "cold_pp_block", "cold_pp_busy"});
+                "cold_ws_channel", "cold_ws_token", "cold_ws_stream", "cold_ws_stream_us", "cold_ws_norm", "cold_pp_tile", "cold_pp_block", "cold_pp_busy", "cold_cached"});
   }
   add("limits.", {"margin", "two_phase_margin", "large_weight_margin", "large_weight_max_tokens", "mid_wavesplit_max_weight", "ragged_max_weight",
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "streamed_apart", "streamed_apart_max_kblocks", "streamed_apart_min_tokens", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "streamed_apart", "streamed_apart_max_kblocks", "streamed_apart_min_tokens", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;

@@ -36,6 +36,7 @@ struct TileTimes {
   double cold, cold_channel, cold_token, cold_shared, cold_stream, cold_stream_us, cold_again, cold_split_us, cold_split_us_per_mb;
   double cold_ws_channel, cold_ws_token, cold_ws_stream, cold_ws_stream_us, cold_ws_norm;
   double cold_pp_tile, cold_pp_block, cold_pp_busy;
+  double cold_cached;  // how much slower a tile may model by the times above, on weights that the caches may hold
 };
 // Up to 16 tokens, a weight loaded as a stream (choose_streamed_tile): rounds of `tile` + K / 1000 * (channels * channel + tokens * token) and
 // the stream for the 16-token wave-split tiles; rounds of K blocks * (block + channels * block_channel + tokens * block_token), 64 x 128
@@ -53,7 +54,7 @@ constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     3.63, 0.11, 0.406, 0.596, 0.186, 0.733,
     0.101, 0.0019, 0.0020, 1.42, 4.88, -0.45, 0.202, 3.27, 0.320,
     0.01269, 0.01362, 1.434, -1.44, 1.283,
-    6.52, 1.774, 0.55};
+    6.52, 1.774, 0.55, 1.08};
 constexpr TileTimes PLAIN_TIMES = {  // FP8 with epilogue scales, INT8
     1.77, 0.777, 3.81, 0.251, 4.55, -2.24, 1.871, 0.402,
     {2.21, 2.72, 3.03, 3.17, 3.76, 4.72, 2.48, 3.12, 3.83, 4.14, 2.81, 3.80, 4.64},
@@ -63,7 +64,7 @@ constexpr TileTimes PLAIN_TIMES = {  // FP8 with epilogue scales, INT8
     3.64, 0.01, 0.435, 0.760, 0.217, 0.531,
     0.092, 0.0020, 0.0018, 1.37, 5.02, 1.55, 0.230, 3.16, 0.331,
     0.01247, 0.01387, 1.394, -1.13, 1.215,
-    6.35, 1.730, 0.681};
+    6.35, 1.730, 0.681, 1.03};
 static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above follow MID_TILES");
 
 // Where the model is not asked or not trusted; both sides of each line stand beside the function that uses it.
@@ -78,7 +79,7 @@ struct TileLimits {
   double resident_margin = 0.93;
   double streamed_min_weight = 105e6, streamed_min_channels = 8000.0, streamed_one_token_min_kblocks = 63.0, streamed_one_token_min_channels = 11000.0, streamed_one_token_min_weight = 150e6, streamed_two_tokens_min_kblocks = 36.0, streamed_apart = 1.1, streamed_apart_max_kblocks = 32.0, streamed_apart_min_tokens = 4.0;
   double small_min_kblocks = 4.0, small_min_tokens = 4.0, small_min_channels = 192.0, small_max_tokens_values = 20800.0;
-  double cold_min_weight = 40e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
+  double cold_min_weight = 40e6, cold_only_min_weight = 80e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
 struct TileModel {
   TileTimes scaled = SCALED_TIMES, plain = PLAIN_TIMES;
@@ -273,10 +274,17 @@ TileChoice choose_swept_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, con
 // memory: 64 x 128 tiles on one CU in two read it at 33 KB a microsecond and CU, whatever their MFMAs could take, so what counts is
 // how many CUs read and how often each row is fetched, which the times above know little of.  Fitted to 19 000 timings of 330
 // shapes with 40 to 400 million weights, 17 to 1500 tokens: 3 to 4 % root mean square, where the times above are off by 5 to 7.
-// At 102 random shapes where it changes the tile (one in nine of 17 to 6000 tokens by 40 to 600 million weights) linears take 0.895 times
-// as long, 0.82 up to 64 tokens, at worst 1.05.  us, before / after: block FP8 139 tokens 18432 -> 7168 52.5 / 45.9, 158 tokens 16640 ->
-// 16384 104.6 / 77.7, 115 tokens 7680 -> 9600 37.0 / 30.0; per-token FP8 510 tokens 3456 -> 16512 51.9 / 44.2; INT8 169 tokens 7168 ->
-// 36864 98.4 / 83.4, but 216 tokens 9216 -> 7168 37.1 / 39.0.  Within 8 % it does not order two tiles.
+// Within 8 % it does not order two tiles.
+// A weight below 80 million bytes may also lie in the 256 MB Infinity Cache (the few layers of a small model, or three in turn), where the
+// times above are the better ones: a tile is taken only if it models at most `cold_cached` times as long by those too.  That is where the
+// tiles measure the same with three weights in turn, 1.08 for the scaled kinds and 1.03 for the others, at 400 shapes of 40 to 100 million
+// weights: with it linears take 0.966 (scaled) and 0.992 as long with three in turn, 0.905 and 0.966 with weights from memory; without it
+// INT8 and epilogue scales take 1.044 with three in turn (143 tokens 7168 -> 9216 21.8 / 27.2 us in three K splits, and 30.2 / 34.1 from
+// memory; 191 tokens 9216 -> 7168 26.4 / 30.4, but 39.7 / 36.1).  From 80 million on three weights leave the cache: 0.93 and 0.91.
+// What it changes, 300 shapes with the layers of 64 to 66 million weights among them (profiles/tile_choice_large_weights.txt): 0.942 with three
+// in turn, at most 1.11, 0.899 from memory, at most 1.05.  us from memory, before / after: block FP8 139 tokens 18432 -> 7168 52.5 / 45.9,
+// 158 tokens 16640 -> 16384 104.6 / 77.7, 115 tokens 7680 -> 9600 37.0 / 30.0; per-token FP8 510 tokens 3456 -> 16512 51.9 / 44.2;
+// INT8 169 tokens 7168 -> 36864 98.4 / 83.4.
 // Not judged: the 256 x 256 tile where it was chosen (2556 tokens 7168 -> 7168 155.3, 128 x 192 tiles 159.0), the INT8 kernel of 128 x 256 tiles in two phases, which has no time of its own here, and up to 128 tokens a split plan that
 // fills seven eighths of the chip, where two token tiles cost less than `cold_again` has it (128 tokens 18432 -> 7168: 64 x 128 tiles
 // in two splits 49.8 us measured, 128 x 128 in four 44.2; modelled 48 and 39; 72 tokens 8320 -> 21120 44.8 against 46.3).
@@ -289,19 +297,32 @@ TileChoice choose_cold_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, cons
   if ((double)M <= l.cold_full_max_tokens && c.family == TF_DMA && c.splits > 1 &&
       (double)(ceil_div(M, c.bm) * ceil_div(N, c.bn) * c.splits) >= l.cold_full_workgroups)
     return swept;
-  double us = 1e30;
+  const auto cold = [&](int family, int i, int splits, double most) {
+    return family == TF_WAVESPLIT ? cold_wavesplit_tile_us(t, i, M, N, K, most) : cold_dma_tile_us(t, i, M, N, K, splits, most);
+  };
+  const auto cached = [&](int family, int i, int splits) {
+    return family == TF_WAVESPLIT ? wavesplit_tile_us(t, i, M, N, K) : dma_tile_us(t, i, M, N, K, splits);
+  };
+  int index = -1;  // of the tile to be beaten
   if (c.family == TF_DMA)
     for (int i = 0; i < 13; ++i)
-      if (MID_TILES[i].bm == c.bm && MID_TILES[i].bn == c.bn) us = cold_dma_tile_us(t, i, M, N, K, c.splits);
+      if (MID_TILES[i].bm == c.bm && MID_TILES[i].bn == c.bn) index = i;
   if (c.family == TF_WAVESPLIT)
     for (int i = 0; i < (int)(sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0])); ++i)
-      if (WAVESPLIT_TILES[i].bm == c.bm && WAVESPLIT_TILES[i].bn == c.bn) us = cold_wavesplit_tile_us(t, i, M, N, K);
-  TileChoice best = fastest_dma_tile(M, N, K, [&](int i, int splits, double most) { return cold_dma_tile_us(t, i, M, N, K, splits, most); });
+      if (WAVESPLIT_TILES[i].bm == c.bm && WAVESPLIT_TILES[i].bn == c.bn) index = i;
+  if (index < 0) return swept;
+  const double us = cold(c.family, index, c.splits, 1e30);
+  const double limit = (double)(N * K) >= l.cold_only_min_weight ? 1e30 : t.cold_cached * cached(c.family, index, c.splits);
+  const auto allowed_us = [&](int family, int i, int splits, double most) {
+    const double u = cold(family, i, splits, most);
+    return u < most && limit < 1e30 && cached(family, i, splits) > limit ? 1e30 : u;
+  };
+  TileChoice best = fastest_dma_tile(M, N, K, [&](int i, int splits, double most) { return allowed_us(TF_DMA, i, splits, most); });
   if (wavesplit_allowed(M, N, K)) {
-    const TileChoice ws = fastest_wavesplit_tile([&](int i, double most) { return cold_wavesplit_tile_us(t, i, M, N, K, most); });
+    const TileChoice ws = fastest_wavesplit_tile([&](int i, double most) { return allowed_us(TF_WAVESPLIT, i, 1, most); });
     if (ws.us < best.us) best = ws;
   }
-  const double two_phase = M > 128 ? cold_two_phase_us(t, M, N, K) : 1e30;
+  const double two_phase = M > 128 && two_phase_us(t, M, N, K) <= limit ? cold_two_phase_us(t, M, N, K) : 1e30;
   if (two_phase < best.us) best = {TF_TWO_PHASE, 256, 256, 1, two_phase};
   return best.us < l.cold_margin * us ? best : swept;
 }

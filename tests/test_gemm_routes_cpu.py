@@ -175,6 +175,22 @@ def test_large_weights_run_the_faster_tile(kind, shape, want, us, other):
     assert us < other and (p["kernel"], p["bm"], p["bn"], p["splits"]) == want, p
 
 
+# Weights that the caches may still hold, where a K split loses its reduce launch again, with three weights in turn (first pair of us:
+# unsplit, split) and from memory (second pair) or only with three in turn
+REDUCE_NOT_EARNED = [
+    ("int8", (143, 9216, 7168)),  # 21.8, 27.2; 30.2, 34.1
+    ("fp8_scaled", (218, 6144, 7168)),  # 21.8, 28.1; 29.9, 30.2
+    ("int8", (166, 8192, 8192)),  # 24.6, 30.0; 33.5, 34.9
+    ("int8", (216, 7168, 9216)),  # 37.1, 39.0 with eight weights in turn
+    ("fp8", (153, 9216, 7168)),  # 27.9, 29.4; 32.0, 34.0
+]
+
+
+@pytest.mark.parametrize("kind,shape", REDUCE_NOT_EARNED)
+def test_no_split_that_its_reduce_costs_more_than_it_gains(kind, shape):
+    assert plan_for(kind, *shape)["splits"] == 1, plan_for(kind, *shape)
+
+
 # Up to 16 tokens on weights that are loaded as a stream: (linear, shape, kernel and channel tile that have to run, us, what ran otherwise)
 STREAMED_CHOICES = [
     ("block", (16, 14336, 18432), "wavesplit_tile", 64, 47.9, 64.1), ("block", (4, 14336, 8192), "wavesplit_tile", 64, 24.6, 36.7),
