@@ -450,8 +450,16 @@ inline bool writes_through(int64_t rows, int64_t channels) { return rows * chann
 // and from 65 tokens on not where K is split (18432 -> 7168 at 96 and 112, four ways, INT8 43.1 / 43.9, 45.3 / 46.7).
 constexpr int64_t STREAMED_WEIGHT_BYTES = 100000000;
 inline bool streams_weight(const GemmParams& p) {
-  return p.tiles_m == 1 && (p.M <= 64 || p.splits == 1) && (int64_t)p.N * p.ldb >= STREAMED_WEIGHT_BYTES;
+  return p.tiles_m == 1 && (p.M <= 64 || p.splits == 1) && (int64_t)p.N * p.K >= STREAMED_WEIGHT_BYTES;
 }
+
+// Mid-M tile, weight rows a multiple of 4096 bytes apart: with every workgroup at the same K block, all rows being fetched lie at the same place of
+// that period, which is a few of the memory's channels.  Each channel tile then starts its K loop one block further on.  us, all from
+// block 0 / rotated (whole linears): 4096 -> 28672 at 32 tokens INT8 33.3 / 28.7, per-token FP8 at 100 35.5 / 32.2; 8192 -> 28672 at 32
+// 57.5 / 47.2; 12288 -> 28672 at 200 118.5 / 106.5; 16384 -> 4096 at 101 29.5 / 28.3.  Weights below 64 million values come out of the caches
+// often enough (14 shapes: 1.00, 0.98 to 1.03), and other pitches spread by themselves (K = 7168 -> 36864 0.99 to 1.00, 18432 -> 7168 at 40 1.01,
+// 4608 -> 7168 at 242 22.5 / 23.4: the token rows of concurrent tiles are no longer the same).
+inline bool rotates_k(int64_t N, int64_t K, int64_t ldb) { return ldb % 4096 == 0 && N * K >= 64000000; }
 
 // Grouped problems on the tile bodies of the dense kernels: token rows of all experts stacked in one matrix, one weight
 // matrix per expert.  `g` describes expert 0 (a, out, b, sb, and sa = the re-laid-out token scales: M-major, every

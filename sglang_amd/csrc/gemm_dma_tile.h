@@ -415,19 +415,11 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + 
   dma_tile<AR, BM, BN, SPLIT, S, STREAM, ROTATES>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
 }
 
-// Weight rows a multiple of 4096 bytes apart: with every workgroup at the same K block, all rows being fetched lie at the same place of
-// that period, which is a few of the memory's channels.  Each channel tile then starts its K loop one block further on.  us, all from
-// block 0 / rotated (whole linears): 4096 -> 28672 at 32 tokens INT8 33.3 / 28.7, per-token FP8 at 100 35.5 / 32.2; 8192 -> 28672 at 32
-// 57.5 / 47.2; 12288 -> 28672 at 200 118.5 / 106.5; 16384 -> 4096 at 101 29.5 / 28.3.  Weights below 64 million values come out of the caches
-// often enough (14 shapes: 1.00, 0.98 to 1.03), and other pitches spread by themselves (K = 7168 -> 36864 0.99 to 1.00, 18432 -> 7168 at 40 1.01,
-// 4608 -> 7168 at 242 22.5 / 23.4: the token rows of concurrent tiles are no longer the same).
-inline bool rotates_k(const GemmParams& p) { return p.ldb % 4096 == 0 && (int64_t)p.N * p.ldb >= 64000000; }
-
 template <Arith AR, int BM, int BN>
 int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
-  p.rotate_k = rotates_k(p);
+  p.rotate_k = rotates_k(p.N, p.K, p.ldb);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
   constexpr int OWN = stages_of(BM, BN, true), SHARED = stages_of(BM, BN, false);
   // (a kernel of its own for K loops that start in the middle: the few instructions more cost a chain of short K blocks 5 %, 16 experts of

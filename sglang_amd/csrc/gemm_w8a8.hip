@@ -842,7 +842,7 @@ std::vector<std::string> tile_constant_names() {
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "streamed_apart", "streamed_apart_max_kblocks", "streamed_apart_min_tokens", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
@@ -1284,6 +1284,8 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
   const Route run = run_route(kind, M, N, K, K, ldw, w_aligned && K % 16 == 0);
   if (!q_ok) return {LM_LAUNCH, run};
   if (tile_quant_preferred(run, M, N, K)) return {LM_TILE, run};
+  // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks; 4096 -> 24576 at 16 tokens 26.2 / 23.7)
+  const LinearMode producer_mode = rotates_k(N, K, ldw) ? LM_LAUNCH_OWN : LM_PRODUCER;
   // the block linear on a large weight (its own choice, see choose_decode_tile), with the producer waves of the mid-M tile
   if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && streamed_decode(kind, M, N, K)) {
     const Route producer = linear_producer_route(M, N, K, ldw);
@@ -1293,8 +1295,7 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
     Route r{};
     r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
     r.kernel = c.family == TF_DMA ? RK_DMA3 : RK_WAVESPLIT_TILE;
-    // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks)
-    if (c.family == TF_DMA) return {K % 4096 == 0 ? LM_LAUNCH_OWN : LM_PRODUCER, r};
+    if (c.family == TF_DMA) return {producer_mode, r};
     return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
   }
   if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && run.kernel == RK_DECODE && small_decode(kind, M, N, K, false, true)) {
@@ -1313,7 +1314,7 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
   if (quant != WavesplitQuant::BLOCK_F32 || (M <= 16 && run.kernel == RK_WAVESPLIT_TILE)) return {LM_LAUNCH, run};
   if (M <= 16) {
     const Route r = linear_producer_route(M, N, K, ldw);
-    if (r.kernel == RK_DMA3) return {LM_PRODUCER, r};  // one round of unsplit 64-token tiles: producer waves of that kernel quantize the tokens
+    if (r.kernel == RK_DMA3) return {producer_mode, r};  // one round of unsplit 64-token tiles: producer waves of that kernel quantize the tokens
   }
   const Route r = choose_route(true, M, N, K, K, ldw, true, true);
   if (r.kernel == RK_DECODE && fused_quant_preferred(M, N, K, ldw)) return {LM_STREAMING, r};

@@ -77,7 +77,7 @@ struct TileLimits {
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
   double resident_margin = 0.93;
-  double streamed_min_weight = 105e6, streamed_min_channels = 8000.0, streamed_one_token_min_kblocks = 63.0, streamed_one_token_min_channels = 11000.0, streamed_one_token_min_weight = 150e6, streamed_two_tokens_min_kblocks = 36.0, streamed_apart = 1.1, streamed_apart_max_kblocks = 32.0, streamed_apart_min_tokens = 4.0;
+  double streamed_min_weight = 105e6, streamed_min_channels = 8000.0, streamed_one_token_min_kblocks = 63.0, streamed_one_token_min_channels = 11000.0, streamed_one_token_min_weight = 150e6, streamed_two_tokens_min_kblocks = 36.0;
   double small_min_kblocks = 4.0, small_min_tokens = 4.0, small_min_channels = 192.0, small_max_tokens_values = 20800.0;
   double cold_min_weight = 40e6, cold_only_min_weight = 80e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
@@ -357,8 +357,7 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
 // per-token FP8 40.2 / 30.1.
 // One and two tokens stay on the register kernel where its K is short, one token also on narrow weights up to where that kernel's limits end
 // (at 1: 3584 -> 36864 23.3 / 24.8, 7168 -> 18432 INT8 25.6 / 27.3, but 9344 -> 31744 49.8 / 47.2; at 2: 4096 -> 28672 22.8 / 23.7, but 7168 ->
-// 36864 INT8 49.2 / 44.3; block FP8 at 2 as at 1, it has the streaming kernel's quantizer); so do up to four on rows 4096 bytes apart with
-// one turn of K (at 4 INT8 4096 -> 28672 25.2 / 26.0, at 9 per-token FP8 29.3 / 25.1).  Fewer than 8000 channels: the limits of
+// 36864 INT8 49.2 / 44.3; block FP8 at 2 as at 1, it has the streaming kernel's quantizer).  Fewer than 8000 channels: the limits of
 // choose_limited_decode_tile hold.
 bool streamed_decode(GemmKind kind, int64_t M, int64_t N, int64_t K) {
   const TileLimits& l = tile_model().limits;
@@ -366,8 +365,7 @@ bool streamed_decode(GemmKind kind, int64_t M, int64_t N, int64_t K) {
   if (M > 16 || K % KSTEP != 0 || N % 16 != 0 || weight < l.streamed_min_weight || (double)N < l.streamed_min_channels) return false;
   if (M == 1 || (M == 2 && kind == GK_F32))
     return kb >= l.streamed_one_token_min_kblocks && ((double)N >= l.streamed_one_token_min_channels || weight >= l.streamed_one_token_min_weight);
-  if (M == 2) return kb >= l.streamed_two_tokens_min_kblocks;
-  return (double)M > l.streamed_apart_min_tokens || K % 4096 != 0 || kb > l.streamed_apart_max_kblocks;
+  return M > 2 || kb >= l.streamed_two_tokens_min_kblocks;
 }
 double streamed_mid_us(int64_t M, int64_t N, int64_t K, int bn) {
   const StreamedTimes& t = tile_model().streamed;
@@ -383,9 +381,10 @@ double streamed_wavesplit_us(int64_t M, int64_t N, int64_t K, int bn) {
   return norm_of(us, (double)(N * K) * 1e-6 / t.stream + t.stream_us, t.norm);
 }
 // `settled`: what runs without this rule where that is one of the two tiles; it stays unless another is 8 % faster (within that the model does
-// not order them: 12672 -> 9728 at 2 tokens 16 x 64 25.6, 16 x 16 27.9; 7168 -> 18432 at 16 64 x 128 29.4, 16 x 32 31.2).  Weight rows a
-// multiple of 4096 bytes apart are the wave-split tile's, up to the weights where choose_limited_decode_tile leaves them, unless the other is 10 %
-// faster (4096 -> 32832 at 7 tokens 31.8 on the register kernel, 34.2 / 26.0).
+// not order them: 12672 -> 9728 at 2 tokens 16 x 64 25.6, 16 x 16 27.9; 7168 -> 18432 at 16 64 x 128 29.4, 16 x 32 31.2).
+// Weight rows a multiple of 4096 bytes apart have no rule of their own: the mid-M tile, whose K loops start at different blocks there, is the
+// faster one there too (wave-split or register kernel / mid-M tile at 4096 -> 28672, 3 to 10 tokens: per-token FP8 28.0 / 24.0, 28.8 / 24.2,
+// 27.8 / 24.6, 26.3 / 24.1, INT8 26.3 / 24.2 at 4, block FP8 26.2 / 24.6 at 4, 27.8 / 24.8 at 10; 112 such linears 0.913, at most 1.02).
 TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoice& settled) {
   const TileLimits& l = tile_model().limits;
   TileChoice best{TF_NONE, 0, 0, 1, 1e30};
@@ -394,9 +393,8 @@ TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoic
     if (us < best.us) best = {family, bm, bn, 1, us};
   };
   for (int i = 0; i < 3; ++i) consider(TF_WAVESPLIT, 16, WAVESPLIT_TILES[i].bn, streamed_wavesplit_us(M, N, K, WAVESPLIT_TILES[i].bn));
-  const double apart = K % 4096 == 0 && (double)(N * K) <= l.decode_max_weight ? l.streamed_apart : 1.0;
   for (int bn = 128; bn <= 256; bn += 64)  // (in one round: 2048 -> 67232 at 13 in 351 workgroups 34.6, the register kernel 29.6)
-    if (ceil_div(N, bn) <= (bn == 128 ? 2 : 1) * NUM_CUS) consider(TF_DMA, 64, bn, apart * streamed_mid_us(M, N, K, bn));
+    if (ceil_div(N, bn) <= (bn == 128 ? 2 : 1) * NUM_CUS) consider(TF_DMA, 64, bn, streamed_mid_us(M, N, K, bn));
   return best;
 }
 
@@ -438,11 +436,12 @@ TileChoice best_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K) {
 // (K = 1024 -> N = 12288 5.8/4.8, 8.0/4.9; but 512 -> 32768 5.9/6.8, 1536 -> 24576 9.3/9.6).
 // It does not take over from
 //   * the mid-M kernel, which the table names where one round of unsplit tiles fills the chip (K = 2304 -> N = 36864 at 16 tokens
-//     19.3/22.9, 5120 -> 50688 51.3/57.3, INT8 1024 -> 17408 at 12 tokens 7.1/9.0; over 91 shapes 6 % faster), unless the rows of the weight lie
-//     a multiple of 4096 bytes apart, where that kernel's loads of eight rows collide (4096 -> 30464 31.7/29.5, per-token FP8 32.2/28.4);
+//     19.3/22.9, 5120 -> 50688 51.3/57.3, INT8 1024 -> 17408 at 12 tokens 7.1/9.0; over 91 shapes 6 % faster), also where the rows of the weight
+//     lie a multiple of 4096 bytes apart: its K loops start at different blocks there (4096 -> 30464 23.5/25.7, per-token FP8 23.9/25.1;
+//     linears of 12 to 16 tokens, 4096 -> 18432 .. 32768, 95 of them: 0.90, at most 1.02);
 //   * the register wave-split kernel where K fills its one turn of 32 blocks and the channels are more than one round of the widest tile,
 //     up to 10 tokens: 4096 -> 20736 at 1 and 8 19.0/24.4, 21.3/24.4; 3840 -> 24576 at 1 20.0/23.0 (4096 -> 16384 at 1, 8 14.8/16.3,
-//     16.3/16.3; 3584 -> 27392 at 6 23.6/21.8; INT8 4096 -> 28672 at 11 29.8/26.2).
+//     16.3/16.3; 3584 -> 27392 at 6 23.6/21.8).
 // The weight limits were drawn at the shapes named beside them.  Measured around them since (K = 2304 .. 18432, 85 to 260 million weights,
 // 1 .. 16 tokens): also beyond them the tile is up to 25 % faster than the streaming and the two-turn register kernel, and slower than
 // the one-turn one; but a linear that leaves those loses their fused quantizers, so the limits stay where the linears were measured.
@@ -453,7 +452,7 @@ TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64
   // (the largest weights: the register kernel's single-tile stream is as fast for few tokens, unless it pads K to whole turns of 32 blocks:
   // K = 5152 -> N = 31936 INT8 at 5 tokens 50.3 us, 39.3 with the tile)
   const bool padded = kb <= 64 && (kb + 31) / 32 * 32 * 4 > kb * 5;
-  if (from_mid && K % 4096 != 0) return TileChoice{TF_NONE, 0, 0, 1, 0.0};
+  if (from_mid) return TileChoice{TF_NONE, 0, 0, 1, 0.0};
   const bool one_turn = (double)kb >= l.decode_one_turn_min_kblocks && (double)kb <= l.decode_one_turn_kblocks;
   if (from_wavesplit && one_turn && (double)M <= l.decode_one_turn_max_tokens && (double)N > l.decode_one_turn_max_channels)
     return TileChoice{TF_NONE, 0, 0, 1, 0.0};

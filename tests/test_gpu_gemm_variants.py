@@ -21,19 +21,21 @@ def _words(e):
     return buf.t()[:rows]
 
 
-def check_exact(gpu, kind, M, N, K):
+def check_exact(gpu, kind, M, N, K, pitch=None):
+    """`pitch`: elements between the weight's rows."""
     from sglang_amd import ops
 
     g = torch.Generator(device=gpu).manual_seed(M + 3 * N + 5 * K)
     draw = lambda low, high, *shape: torch.randint(low, high, shape, generator=g, device=gpu)
     a, w = draw(-2, 3, M, K), draw(-2, 3, N, K)
     kb, nb = -(-K // 128), -(-N // 128)
+    pad = lambda t: torch.nn.functional.pad(t, (0, pitch - K), value=1)[:, :K] if pitch else t
     if kind in ("fp8", "fp8_ue8m0"):
         ea, eb = draw(125, 130, M, kb), draw(125, 130, nb, kb)
         ta, tb = torch.exp2(ea.double() - 127), torch.exp2(eb.double() - 127)
         wide = lambda s: s.repeat_interleave(128, dim=1)[:, :K]
         want = (a * wide(ta)) @ (w * wide(tb.repeat_interleave(128, dim=0)[:N])).t()
-        a8, w8 = a.float().to(FP8), w.float().to(FP8)
+        a8, w8 = a.float().to(FP8), pad(w.float().to(FP8).view(torch.uint8)).view(FP8)
         if kind == "fp8":
             out = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
             ops.block_fp8_matmul(a8, w8, ta.float(), tb.float(), out)
@@ -45,9 +47,9 @@ def check_exact(gpu, kind, M, N, K):
         product = a.double() @ w.double().t()
         want = product * sa.double()[:, None] * sb.double() + bias.double()
         if kind == "fp8_scaled":
-            out = ops.fp8_scaled_mm(a.float().to(FP8), w.float().to(FP8).t(), sa, sb, torch.bfloat16, bias)
+            out = ops.fp8_scaled_mm(a.float().to(FP8), pad(w.float().to(FP8).view(torch.uint8)).view(FP8).t(), sa, sb, torch.bfloat16, bias)
         else:
-            a8, w8 = a.to(torch.int8), w.to(torch.int8)
+            a8, w8 = a.to(torch.int8), pad(w.to(torch.int8))
             assert torch.equal(ops.int8_mm_raw_accumulators(a8, w8.t()).double(), product), (kind, M, N, K)
             out = ops.int8_scaled_mm(a8, w8.t(), sa, sb, torch.bfloat16, bias)
     assert torch.equal(out, want.float().to(torch.bfloat16)), (kind, M, N, K)
@@ -85,6 +87,16 @@ def test_rotated_k(gpu, kind, M, N, K):
     check_exact(gpu, kind, M, N, K)
 
 
+# weight rows further apart than K bytes: 4096 bytes apart (K loops that start at different blocks, with streamed loads or without, decode
+# sizes), and K = 4096 where they are not; the weight-in-registers kernel and the two-phase kernels
+@pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
+@pytest.mark.parametrize("M,N,K,pitch", [(40, 20488, 3968, 4096), (300, 16392, 3968, 4096), (100, 28680, 3968, 4096), (8, 28688, 3968, 4096), (8, 28688, 4096, 4224),
+                                         (100, 15688, 4096, 4224), (900, 16392, 512, 640), (1, 1040, 2176, 4096), (2100, 8200, 1024, 1152)])
+def test_weight_rows_of_any_pitch(gpu, kind, M, N, K, pitch):
+    print(f"case {kind} {(M, N, K)} pitch {pitch}", flush=True)
+    check_exact(gpu, kind, M, N, K, pitch)
+
+
 # weights of 100 million bytes and more are loaded as a stream where one token tile reads them: every height of the mid-M tile, K split and
 # whole, the 16-token tile, ragged last channel tiles
 @pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
@@ -110,6 +122,25 @@ def test_streamed_weights_of_fused_linears(gpu, M, N, K):
     q, qs = per_token_group_quant_fp8(x, 128, column_major_scales=True)
     two = w8a8_block_fp8_matmul(q, w, qs, s, [128, 128], torch.bfloat16)
     assert torch.equal(ops.block_fp8_linear(x, w, s, None, torch.bfloat16).view(torch.int16), two.view(torch.int16))
+
+
+def test_block_linear_on_padded_rows(gpu):
+    """Rows 4096 bytes apart with K below that, and the other way round: what dense rows give, where the sums have one order, and the
+    same to the rounding of the result where the K loops start at other blocks."""
+    from fp8_tolerance import check_fp8_gemm
+    from sglang_amd import ops
+    from sglang_amd.fp8_kernel import per_token_group_quant_fp8
+
+    for M, N, K, pitch in ((4, 28672, 3968, 4096), (16, 28672, 3968, 4096), (4, 28672, 4096, 4224), (1, 1024, 2176, 4096)):
+        g = torch.Generator(device=gpu).manual_seed(M + K)
+        x = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+        w = torch.randint(-8, 9, (N, pitch), generator=g, device=gpu, dtype=torch.int8).half().to(FP8)[:, :K]
+        s = torch.rand(N // 128, K // 128, generator=g, device=gpu) + 0.5
+        out = ops.block_fp8_linear(x, w, s, None, torch.bfloat16)
+        q, qs = per_token_group_quant_fp8(x, 128, column_major_scales=True)
+        a = q.double() * qs.double().repeat_interleave(128, 1)
+        b = w[:1024].double() * s[:8].double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+        check_fp8_gemm(out[:, :1024], (a @ b.t()).float().cpu(), (a.abs() @ b.abs().t()).float().cpu(), f"{(M, N, K, pitch)}")
 
 
 # the block linear's own choice on such weights, also where the GEMM alone takes another kernel: the wave-split tile quantizing and behind a
