@@ -103,7 +103,12 @@ struct TileChoice {
 
 const TileTimes& tile_times(GemmKind kind) { return kind == GK_F32 || kind == GK_UE8M0 ? tile_model().scaled : tile_model().plain; }
 
-double norm_of(double a, double b, double n) { return b <= 0.1 ? a : std::pow(std::pow(a, n) + std::pow(b, n), 1.0 / n); }
+double norm_of(double a, double b, double n) {
+  if (b <= 0.1) return a;
+  if (n != 6.0) return std::pow(std::pow(a, n) + std::pow(b, n), 1.0 / n);
+  const double x = a * a * a, y = b * b * b;  // (most of a sweep's powers)
+  return std::cbrt(std::sqrt(x * x + y * y));
+}
 // full rounds of `slots` workgroups and a partly filled one
 template <class Round>
 double rounds_of(int64_t workgroups, int64_t slots, Round round) {
@@ -114,16 +119,17 @@ double rounds_of(int64_t workgroups, int64_t slots, Round round) {
 // (`most`: a time from which on the result does not matter; the powers are left out where the larger of the two bounds reaches it)
 double dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, int splits, double most = 1e30) {
   const int bm = MID_TILES[i].bm, bn = MID_TILES[i].bn;
+  const double mn = (double)M * (double)N * 1e-6;
+  const double stream = ((double)N + (double)M) * (double)K * 1e-6 / t.stream + mn * 2.0 * t.result_us_per_mb + t.stream_us;
+  const double split = splits > 1 ? t.split_us + t.split_us_per_mb * splits * mn * 4.0 : 0.0;
+  if (stream + split >= most) return most;
   const int64_t kb = ceil_div(K, KSTEP), wg = ceil_div(M, bm) * ceil_div(N, bn) * splits;
   const double blocks = (double)ceil_div(kb, splits);
   const bool two = bm + bn == 192 && wg > NUM_CUS;
   const double us = t.launch + rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) {
                       return t.tile[i] + blocks * t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill);
                     });
-  const double mn = (double)M * (double)N * 1e-6;
-  const double stream = ((double)N + (double)M) * (double)K * 1e-6 / t.stream + mn * 2.0 * t.result_us_per_mb + t.stream_us;
-  const double split = splits > 1 ? t.split_us + t.split_us_per_mb * splits * mn * 4.0 : 0.0;
-  return std::max(us, stream) + split >= most ? most : norm_of(us, stream, 6.0) + split;
+  return us + split >= most ? most : norm_of(us, stream, 6.0) + split;
 }
 double two_phase_us(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
   const double blocks = (double)ceil_div(K, KSTEP);
@@ -141,10 +147,10 @@ double wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_
   return std::max(us, stream) >= most ? most : norm_of(us, stream, t.ws_norm);
 }
 
-// The tile of least time; us(i, most) and us(i, splits, most) time the i-th one.
+// The tile of least time below `most`, or TF_NONE; us(i, most) and us(i, splits, most) time the i-th one.
 template <class Time>
-TileChoice fastest_wavesplit_tile(Time us) {
-  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+TileChoice fastest_wavesplit_tile(Time us, double most = 1e30) {
+  TileChoice best{TF_NONE, 0, 0, 1, most};
   constexpr int COUNT = sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0]);
   for (int i = 0; i < COUNT; ++i) {
     const double u = us(i, best.us);
@@ -153,8 +159,8 @@ TileChoice fastest_wavesplit_tile(Time us) {
   return best;
 }
 template <class Time>
-TileChoice fastest_dma_tile(int64_t M, int64_t N, int64_t K, Time us) {
-  TileChoice best{TF_NONE, 0, 0, 1, 1e30};
+TileChoice fastest_dma_tile(int64_t M, int64_t N, int64_t K, Time us, double most = 1e30) {
+  TileChoice best{TF_NONE, 0, 0, 1, most};
   const int64_t kb = ceil_div(K, KSTEP);
   for (int i = 0; i < 13; ++i) {
     const int64_t tiles = ceil_div(M, MID_TILES[i].bm) * ceil_div(N, MID_TILES[i].bn);
@@ -181,16 +187,20 @@ TileChoice best_dma_tile(const TileTimes& t, int64_t M, int64_t N, int64_t K) {
 double cold_dma_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, int splits, double most = 1e30) {
   const int bm = MID_TILES[i].bm, bn = MID_TILES[i].bn;
   const int64_t tiles_m = ceil_div(M, bm), wg = tiles_m * ceil_div(N, bn) * splits;
-  const double blocks = (double)ceil_div(ceil_div(K, KSTEP), splits);
-  const bool two = bm + bn == 192 && wg > NUM_CUS;
-  const double fetch = (t.cold + t.cold_channel * bn + t.cold_token * (double)M / (double)tiles_m) * (two ? t.cold_shared : 1.0);
-  const double us = t.launch + rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) {
-                      return t.tile[i] + blocks * norm_of(t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill), fetch, 6.0);
-                    });
   const double mn = (double)M * (double)N * 1e-6, fetches = 1.0 + t.cold_again * (double)(tiles_m - 1);
   const double stream = ((double)N * fetches + (double)M) * (double)K * 1e-6 / t.cold_stream + mn * 2.0 * t.result_us_per_mb + t.cold_stream_us;
   const double split = splits > 1 ? t.cold_split_us + t.cold_split_us_per_mb * splits * mn * 4.0 : 0.0;
-  return std::max(us, stream) + split >= most ? most : norm_of(us, stream, 6.0) + split;
+  if (stream + split >= most) return most;
+  const double blocks = (double)ceil_div(ceil_div(K, KSTEP), splits);
+  const bool two = bm + bn == 192 && wg > NUM_CUS;
+  const double fetch = (t.cold + t.cold_channel * bn + t.cold_token * (double)M / (double)tiles_m) * (two ? t.cold_shared : 1.0);
+  const auto rounds = [&](auto larger) {
+    return t.launch + rounds_of(wg, two ? 2 * NUM_CUS : NUM_CUS, [&](double fill) {
+             return t.tile[i] + blocks * larger(t.block[i] * (two ? t.shared : 1.0) * (1.0 + t.busy * fill), fetch);
+           });
+  };
+  if (rounds([](double x, double y) { return std::max(x, y); }) + split >= most) return most;
+  return norm_of(rounds([](double x, double y) { return norm_of(x, y, 6.0); }), stream, 6.0) + split;
 }
 double cold_wavesplit_tile_us(const TileTimes& t, int i, int64_t M, int64_t N, int64_t K, double most = 1e30) {
   const int bm = WAVESPLIT_TILES[i].bm, bn = WAVESPLIT_TILES[i].bn;
@@ -311,20 +321,20 @@ TileChoice choose_cold_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, cons
     for (int i = 0; i < (int)(sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0])); ++i)
       if (WAVESPLIT_TILES[i].bm == c.bm && WAVESPLIT_TILES[i].bn == c.bn) index = i;
   if (index < 0) return swept;
-  const double us = cold(c.family, index, c.splits, 1e30);
+  const double most = l.cold_margin * cold(c.family, index, c.splits, 1e30);  // (within that it does not order two tiles)
   const double limit = (double)(N * K) >= l.cold_only_min_weight ? 1e30 : t.cold_cached * cached(c.family, index, c.splits);
-  const auto allowed_us = [&](int family, int i, int splits, double most) {
-    const double u = cold(family, i, splits, most);
-    return u < most && limit < 1e30 && cached(family, i, splits) > limit ? 1e30 : u;
+  const auto allowed_us = [&](int family, int i, int splits, double least) {
+    const double u = cold(family, i, splits, least);
+    return u < least && limit < 1e30 && cached(family, i, splits) > limit ? 1e30 : u;
   };
-  TileChoice best = fastest_dma_tile(M, N, K, [&](int i, int splits, double most) { return allowed_us(TF_DMA, i, splits, most); });
+  TileChoice best = fastest_dma_tile(M, N, K, [&](int i, int splits, double least) { return allowed_us(TF_DMA, i, splits, least); }, most);
   if (wavesplit_allowed(M, N, K)) {
-    const TileChoice ws = fastest_wavesplit_tile([&](int i, double most) { return allowed_us(TF_WAVESPLIT, i, 1, most); });
-    if (ws.us < best.us) best = ws;
+    const TileChoice ws = fastest_wavesplit_tile([&](int i, double least) { return allowed_us(TF_WAVESPLIT, i, 1, least); }, best.us);
+    if (ws.family != TF_NONE) best = ws;
   }
   const double two_phase = M > 128 && two_phase_us(t, M, N, K) <= limit ? cold_two_phase_us(t, M, N, K) : 1e30;
   if (two_phase < best.us) best = {TF_TWO_PHASE, 256, 256, 1, two_phase};
-  return best.us < l.cold_margin * us ? best : swept;
+  return best.family != TF_NONE ? best : swept;
 }
 
 // The same, or the kernel that keeps the weight in registers where the call allows it and it models 7 % faster than what would run.

@@ -361,6 +361,26 @@ def test_host_work_of_a_workspace_query():
     assert new < 20 * nothing, (nothing, new)
 
 
+def test_host_work_of_a_known_linear():
+    """What a linear does is kept per shape: a query for a large weight at decode sizes, which takes the longest to work out, costs what
+    any other known one does (1.0; 1.5 where it was worked out on every call)."""
+    import ctypes
+
+    from sglang_amd import _lib
+
+    ask, buf = _lib.lib().mi355_fp8_block_linear_plan, ctypes.create_string_buffer(256)
+
+    def cost(M, N, K):
+        t = time.perf_counter()
+        for _ in range(400):
+            ask(M, N, K, buf, len(buf))
+        return time.perf_counter() - t
+
+    trials = [(cost(4096, 36864, 7168), cost(8, 36864, 7168), cost(16, 24576, 7168)) for _ in range(30)]
+    any_other, *large = (min(t) for t in zip(*trials))
+    assert max(large) < 1.25 * any_other, (any_other, large)
+
+
 def test_grouped_plan_bounds_hold_for_any_routing():
     """The grouped GEMM sizes its tile tables and grids on the host from (experts, stacked rows) alone, while the real
     tile counts come from row counts that only exist on the device.  Replay the device rule here (256-row tiles; a rest of
