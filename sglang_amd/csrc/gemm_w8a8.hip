@@ -647,7 +647,9 @@ Route run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t lda, int
     }
   };
   static thread_local RecentShapes<Key, Route> table;
-  if (kind == GK_UE8M0 && M > 16) kind = GK_F32;  // above decode sizes both kinds have one model
+  // above decode sizes both kinds have one model, but for the tokens of the resident kernel's steps
+  const int kb = (int)std::min<int64_t>(K / KSTEP, RESIDENT_MAX_KBLOCKS);
+  if (kind == GK_UE8M0 && M > 16 && resident_half_step(true, kb) == resident_half_step(false, kb)) kind = GK_F32;
   if (M <= 16 || K > RESIDENT_MAX_KBLOCKS * KSTEP) resident = true;  // (does not matter: one entry)
   return table.get(Key{{M, N, K, (int)kind}, lda, ldb, aligned, resident, conforming}, [&] { return uncached_run_route(kind, M, N, K, lda, ldb, aligned, resident, conforming); });
 }
@@ -842,7 +844,7 @@ std::vector<std::string> tile_constant_names() {
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_rounds_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;

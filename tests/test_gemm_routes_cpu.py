@@ -23,6 +23,17 @@ def test_variant_shapes_run_what_they_are_named_after(kind):
         assert variant_of(plan_for(kind, *shape), shape[2]) == variant, (kind, shape)
 
 
+@pytest.mark.parametrize("kind", VARIANT_SHAPES)
+@pytest.mark.parametrize("kb", [2, 3, 4, 5])
+def test_resident_plan_names_the_tokens_of_a_step(kind, kb):
+    """64 tokens a step of the weight-in-registers kernel, 32 where the registers hold no more beside the weight: from five K blocks on,
+    with packed exponents from four on (whatever the other kinds' plan for the same shape was before)."""
+    M, N, K = VARIANT_SHAPES[kind]["resident", f"kb{kb}"]
+    for other in VARIANT_SHAPES:
+        plan_for(other, M, N, K)
+    assert plan_for(kind, M, N, K)["bm"] == (64 if kb <= (3 if kind == "fp8_ue8m0" else 4) else 32)
+
+
 def _random_shapes(count, seed):
     """Token counts, channels and K over the whole range, half of the channels and three quarters of K in whole 128s."""
     import random
