@@ -117,7 +117,7 @@ __device__ __forceinline__ float div_shared(float x, float s, float r) {
 // groups dealt out along the rows, every scale of a column comes from another workgroup, mostly on another XCD, so each 128-byte line
 // of scales is written in pieces from several L2s.  GM_COLS gives a workgroup sixteen (or 32) neighbouring rows instead.
 //   us, 16-bit input, groups of 128, GM_FLAT or GM_QUAD with four groups a thread / this file's choice below:
-//   M-major fp32 scales: 904 x 7168 6.8 / 5.8, 4096 x 7168 21.4 / 18.5, 16384 x 7168 64.3 / 60.0;  packed words: 5103 x 18048 48.2 / 46.0
+//   M-major fp32 scales: 904 x 7168 6.8 / 5.8, 4096 x 7168 21.4 / 17.8, 16384 x 7168 64.3 / 60.0;  packed words: 5103 x 18048 48.2 / 46.0
 enum GroupMap {
   GM_FLAT,  // groups of the flat index, GROUPS_PER_PASS apart
   GM_QUAD,  // four consecutive groups of a row, whose scales leave as one 16-byte store (fp32, row-major) or one 32-bit word
@@ -267,10 +267,13 @@ constexpr uint32_t FLAT_ONE_MAX_GROUPS = 32768, FLAT_ONE_MAX_GROUPS_NO_QUADS = 2
 //   M-major fp32, one flat / one of a column: 387 x 1536 2.22 / 2.41, 3001 x 512 2.82 / 2.80, 200 x 18432 4.36 / 4.02;
 //   packed words: 200 x 18432 3.56 / 3.51, 904 x 7168 5.5 / 5.3
 constexpr uint32_t COLS_MIN_GROUPS_F32 = 12288, COLS_MIN_GROUPS_WORDS = 32768;
-//   a column's one / two rows x two: 1000 x 16384 11.2 / 11.5, 6000 x 3968 15.8 / 15.2, 5103 x 18048 51.7 / 48.6;
-//   two x two / one row x four: 5103 x 18048 48.6 / 49.2, 16384 x 7168 62.2 / 60.0;
-//   packed words, one / four: 1000 x 16384 10.2 / 10.3, 6000 x 3968 14.6 / 14.2, 16384 x 7168 61.6 / 57.7
-constexpr uint32_t COLS_ONE_MAX_GROUPS = 160000, COLS_TWO_MAX_GROUPS = 800000;
+//   one / two rows of a column: 2656 x 8192 13.3 / 13.4, 20000 x 1280 16.3 / 15.6, 10714 x 7168 45.1 / 41.6, 600000 x 128 44.2 / 41.4;
+//   two rows / one row x four: 20833 x 12288 144 / 143, 35714 x 7168 144 / 137, 62500 x 4096 158 / 148;
+//   packed words, one / one row x four: 1000 x 16384 10.2 / 10.3, 6000 x 3968 14.6 / 14.2, 16384 x 7168 61.6 / 57.7
+constexpr uint32_t COLS_ONE_MAX_GROUPS = 160000, COLS_FOUR_MIN_GROUPS_F32 = 800000;
+// Four of a row only where the rows hardly end inside a four, whose missing groups are done again: two rows / one row x four,
+//   1200000 x 128 87 / 263 (packed words 82 / 189), 240000 x 640 95 / 133 (76 / 90), 70588 x 2176 88 / 97 (75 / 77), but 109090 x 1408 packed 75 / 74
+constexpr bool fours_fill(uint32_t groups_per_row) { return (groups_per_row + 3) / 4 * 4 * 10 <= groups_per_row * 11; }
 
 template <typename T, int LPG, int ITERS, int MODE, bool UE8M0, bool FP8_OUT, int UNROLL, GroupMap MAP, int RU = 1>
 int launch_map(QuantParams& p, hipStream_t stream) {
@@ -298,9 +301,8 @@ int launch(QuantParams& p, hipStream_t stream) {
                                                 : p.s_stride_row < p.s_stride_col && groups >= COLS_MIN_GROUPS_F32);
     if (columns) {
       if (groups < COLS_ONE_MAX_GROUPS) return MI355_LAUNCH(1, GM_COLS);
-      if constexpr (!UE8M0)
-        if (groups < COLS_TWO_MAX_GROUPS) return MI355_LAUNCH(4, GM_COLS, 2);
-      return MI355_LAUNCH(4, GM_COLS);
+      if (fours_fill(gpr) && (UE8M0 || groups >= COLS_FOUR_MIN_GROUPS_F32)) return MI355_LAUNCH(4, GM_COLS);
+      return MI355_LAUNCH(2, GM_COLS, 2);
     }
     if (groups < (quads ? FLAT_ONE_MAX_GROUPS : FLAT_ONE_MAX_GROUPS_NO_QUADS)) return MI355_LAUNCH(1, GM_FLAT);
   }

@@ -77,8 +77,9 @@ def test_sgl_kernel_api(gpu, oracle, M, K, enable_v2, layout):
 
 
 # one shape for every way the groups are dealt out (group_quant.hip, GroupMap and the limits beside it): one group a thread along
-# the rows and by columns, two rows x two groups, one row x four; rows and groups per row that fill no workgroup or word
-@pytest.mark.parametrize("M,K", [(15, 2304), (1001, 1664), (2051, 2176), (2048, 2048), (5001, 4224), (6007, 17280)])
+# the rows and by columns, two rows of a column, one row x four; rows and groups per row that fill no workgroup or word, and
+# short rows (one, five, six groups) of which many thousands follow one another
+@pytest.mark.parametrize("M,K", [(15, 2304), (1001, 1664), (2051, 2176), (2048, 2048), (5001, 4224), (6007, 17280), (200003, 128), (160001, 640), (27001, 768)])
 @pytest.mark.parametrize("layout", ["row", "col", "col_aligned", "ue8m0"])
 def test_group_maps(gpu, oracle, M, K, layout):
     test_sgl_kernel_api(gpu, oracle, M, K, False, layout)
