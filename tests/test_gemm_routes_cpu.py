@@ -171,21 +171,25 @@ def test_the_faster_kernel_runs(kind, shape, want, us, other):
     assert us < other and want in (p["kernel"], (p["kernel"], p["bm"], p["bn"], p["splits"])), p
 
 
-# A large weight comes from memory: (kind, shape, tile and splits that have to run, linear's us, the tile's that the other times name)
+# A large weight comes from memory: (kind, shape, tile and splits that run).  us of the linear, and of the tile that the other times name:
 COLD_CHOICES = [
-    ("fp8", (139, 7168, 18432), ("dma3", 160, 128, 4), 45.9, 52.5), ("fp8", (158, 16384, 16640), ("dma3", 160, 128, 2), 77.7, 104.6),
-    ("fp8_ue8m0", (254, 12288, 12416), ("dma3", 128, 192, 2), 58.9, 68.9), ("fp8_scaled", (510, 16512, 3456), ("pingpong", 256, 256, 1), 44.2, 51.9),
-    ("int8", (63, 29184, 2816), ("dma3", 64, 128, 1), 20.6, 27.2), ("fp8", (44, 14336, 4096), ("wavesplit_tile", 64, 64, 1), 17.7, 21.3),
+    ("fp8", (139, 7168, 18432), ("dma3", 160, 128, 4)),  # 45.9, 52.5
+    ("fp8", (158, 16384, 16640), ("dma3", 160, 128, 2)),  # 77.7, 104.6
+    ("fp8_ue8m0", (254, 12288, 12416), ("dma3", 128, 192, 2)),  # 58.9, 68.9
+    ("fp8_scaled", (510, 16512, 3456), ("pingpong", 256, 256, 1)),  # 44.2, 51.9
+    ("int8", (63, 29184, 2816), ("dma3", 64, 128, 1)),  # 20.6, 27.2
+    ("fp8", (44, 14336, 4096), ("wavesplit_tile", 64, 64, 1)),  # 17.7, 21.3
     # what it leaves alone: two token tiles in a split plan that fills the chip, the 256 x 256 tile, smaller weights
-    ("fp8_ue8m0", (72, 21120, 8320), ("dma3", 128, 256, 3), 44.8, 46.3), ("fp8_ue8m0", (2556, 7168, 7168), ("pingpong", 256, 256, 1), 155.3, 159.0),
-    ("fp8", (1608, 576, 7168), ("wavesplit_tile", 64, 64, 1), 20.3, 23.1),
+    ("fp8_ue8m0", (72, 21120, 8320), ("dma3", 128, 256, 3)),  # 44.8, 46.3
+    ("fp8_ue8m0", (2556, 7168, 7168), ("pingpong", 256, 256, 1)),  # 155.3, 159.0
+    ("fp8", (1608, 576, 7168), ("wavesplit_tile", 64, 64, 1)),  # 20.3, 23.1
 ]
 
 
-@pytest.mark.parametrize("kind,shape,want,us,other", COLD_CHOICES)
-def test_large_weights_run_the_faster_tile(kind, shape, want, us, other):
+@pytest.mark.parametrize("kind,shape,want", COLD_CHOICES)
+def test_large_weights_run_the_measured_tile(kind, shape, want):
     p = plan_for(kind, *shape)
-    assert us < other and (p["kernel"], p["bm"], p["bn"], p["splits"]) == want, p
+    assert (p["kernel"], p["bm"], p["bn"], p["splits"]) == want, p
 
 
 # Weights that the caches may still hold, where a K split loses its reduce launch again, with three weights in turn (first pair of us:
@@ -204,41 +208,49 @@ def test_no_split_that_its_reduce_costs_more_than_it_gains(kind, shape):
     assert plan_for(kind, *shape)["splits"] == 1, plan_for(kind, *shape)
 
 
-# Up to 16 tokens on weights that are loaded as a stream: (linear, shape, kernel and channel tile that have to run, us, what ran otherwise)
+# Up to 16 tokens on weights that are loaded as a stream: (linear, shape, kernel and channel tile that run).  us, and what ran otherwise:
 STREAMED_CHOICES = [
-    ("block", (16, 14336, 18432), "wavesplit_tile", 64, 47.9, 64.1), ("block", (4, 14336, 8192), "wavesplit_tile", 64, 24.6, 36.7),
-    ("int8", (4, 36864, 7168), "dma3", 192, 44.2, 53.2), ("token_fp8", (8, 24576, 7168), "wavesplit_tile", 32, 33.4, 39.7),
-    ("ue8m0", (1, 12288, 13312), "wavesplit_tile", 16, 30.3, 38.2),
+    ("block", (16, 14336, 18432), "wavesplit_tile", 64),  # 47.9, 64.1
+    ("block", (4, 14336, 8192), "wavesplit_tile", 64),  # 24.6, 36.7
+    ("int8", (4, 36864, 7168), "dma3", 192),  # 44.2, 53.2
+    ("token_fp8", (8, 24576, 7168), "wavesplit_tile", 32),  # 33.4, 39.7
+    ("ue8m0", (1, 12288, 13312), "wavesplit_tile", 16),  # 30.3, 38.2
     # rows 4096 bytes apart too: the mid-M tile starts its K loops at different blocks there
-    ("int8", (4, 28672, 4096), "dma3", 128, 24.2, 26.3), ("token_fp8", (8, 28672, 4096), "dma3", 128, 24.1, 26.3),
+    ("int8", (4, 28672, 4096), "dma3", 128),  # 24.2, 26.3
+    ("token_fp8", (8, 28672, 4096), "dma3", 128),  # 24.1, 26.3
     # what stays: short K at one and two tokens, few channels
-    ("block", (1, 36864, 3584), "decode_wavesplit", 16, 23.3, 24.8), ("int8", (2, 28672, 4096), "decode_wavesplit", 16, 22.9, 23.6),
-    ("int8", (2, 9728, 12672), "wavesplit_tile", 64, 25.6, 27.9),
+    ("block", (1, 36864, 3584), "decode_wavesplit", 16),  # 23.3, 24.8
+    ("int8", (2, 28672, 4096), "decode_wavesplit", 16),  # 22.9, 23.6
+    ("int8", (2, 9728, 12672), "wavesplit_tile", 64),  # 25.6, 27.9
 ]
 
 
-@pytest.mark.parametrize("kind,shape,kernel,bn,us,other", STREAMED_CHOICES)
-def test_streamed_weights_run_the_faster_kernel(kind, shape, kernel, bn, us, other):
+@pytest.mark.parametrize("kind,shape,kernel,bn", STREAMED_CHOICES)
+def test_streamed_weights_run_the_measured_kernel(kind, shape, kernel, bn):
     from sglang_amd import _lib
 
     p = _lib.linear_plan(kind, *shape)
-    assert us < other and (p["kernel"], p["bn"]) == (kernel, bn), p
+    assert (p["kernel"], p["bn"]) == (kernel, bn), p
 
 
-# Small layers of short K at decode sizes: (linear, shape, kernel that has to run, us a call, what ran otherwise)
+# Small layers of short K at decode sizes: (linear, shape, kernel that runs).  us a call, and what ran otherwise:
 SMALL_CHOICES = [
-    ("ue8m0", (13, 5888, 1536), "wavesplit_tile", 6.5, 8.1), ("int8", (7, 1088, 1024), "wavesplit_tile", 4.5, 5.3), ("ue8m0", (7, 1600, 640), "wavesplit_tile", 5.3, 8.4),
-    ("token_fp8", (16, 4288, 1280), "wavesplit_tile", 6.8, 8.7), ("block", (15, 1408, 1920), "wavesplit_tile", 7.4, 11.7),
+    ("ue8m0", (13, 5888, 1536), "wavesplit_tile"),  # 6.5, 8.1
+    ("int8", (7, 1088, 1024), "wavesplit_tile"),  # 4.5, 5.3
+    ("ue8m0", (7, 1600, 640), "wavesplit_tile"),  # 5.3, 8.4
+    ("token_fp8", (16, 4288, 1280), "wavesplit_tile"),  # 6.8, 8.7
+    ("block", (15, 1408, 1920), "wavesplit_tile"),  # 7.4, 11.7
     # what stays: few tokens with K of 8 blocks and more (4.7, the tile no faster), many token values a workgroup
-    ("block", (2, 2688, 1280), "decode_wavesplit", 4.7, 4.8), ("block", (16, 4096, 2048), "decode_wavesplit", 5.8, 8.2),
+    ("block", (2, 2688, 1280), "decode_wavesplit"),  # 4.7, 4.8
+    ("block", (16, 4096, 2048), "decode_wavesplit"),  # 5.8, 8.2
 ]
 
 
-@pytest.mark.parametrize("kind,shape,kernel,us,other", SMALL_CHOICES)
-def test_small_layers_run_the_faster_kernel(kind, shape, kernel, us, other):
+@pytest.mark.parametrize("kind,shape,kernel", SMALL_CHOICES)
+def test_small_layers_run_the_measured_kernel(kind, shape, kernel):
     from sglang_amd import _lib
 
-    assert us < other and _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
+    assert _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
 
 
 def test_perturbed_plan_query():
