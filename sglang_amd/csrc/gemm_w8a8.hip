@@ -844,7 +844,7 @@ std::vector<std::string> tile_constant_names() {
                   "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_rounds_margin", "streamed_min_weight", "streamed_min_channels", "streamed_one_token_min_kblocks", "streamed_one_token_min_channels", "streamed_one_token_min_weight", "streamed_two_tokens_min_kblocks", "small_min_kblocks", "small_min_tokens", "small_min_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_rounds_margin", "streamed_min_weight", "streamed_two_tokens_min_kblocks", "small_min_tokens", "small_max_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
@@ -1241,7 +1241,7 @@ bool wavesplit_quant_preferred(WavesplitQuant kind, int64_t M, int64_t N, int64_
   const double kb = (double)(K / KSTEP), waves = wavesplit_shape(K).waves;
   const GemmKind gemm = kind == WavesplitQuant::BLOCK_F32 ? GK_F32 : kind == WavesplitQuant::BLOCK_UE8M0 ? GK_UE8M0 : is_fp8 ? GK_UNIT : GK_INT8;
   const int plain = run_route(gemm, M, N, K, K, ldw, true).kernel;
-  if (plain == RK_WAVESPLIT_TILE || streamed_decode(gemm, M, N, K)) return false;
+  if (plain == RK_WAVESPLIT_TILE || streamed_decode(M, N, K)) return false;
   const bool plain_wavesplit = plain == RK_WAVESPLIT;
   if ((kind == WavesplitQuant::BLOCK_UE8M0 || kind == WavesplitQuant::TOKEN_FP8) && !plain_wavesplit) return false;
   if (kb < route_constants().wavesplit_min_kblocks && (is_fp8 || N / 16 > 512)) return false;  // a block per wave: 512->32768 8.2 against 10.5
@@ -1289,7 +1289,7 @@ LinearRoute uncached_choose_linear(WavesplitQuant quant, int64_t M, int64_t N, i
   // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks; 4096 -> 24576 at 16 tokens 26.2 / 23.7)
   const LinearMode producer_mode = rotates_k(N, K, ldw) ? LM_LAUNCH_OWN : LM_PRODUCER;
   // the block linear on a large weight (its own choice, see choose_decode_tile), with the producer waves of the mid-M tile
-  if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && streamed_decode(kind, M, N, K)) {
+  if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && streamed_decode(M, N, K)) {
     const Route producer = linear_producer_route(M, N, K, ldw);
     const TileChoice settled{run.kernel == RK_WAVESPLIT_TILE ? TF_WAVESPLIT : producer.kernel == RK_DMA3 ? TF_DMA : TF_NONE, 0,
                              run.kernel == RK_WAVESPLIT_TILE ? run.bn : producer.bn, 1, 0.0};
@@ -1298,12 +1298,6 @@ LinearRoute uncached_choose_linear(WavesplitQuant quant, int64_t M, int64_t N, i
     r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
     r.kernel = c.family == TF_DMA ? RK_DMA3 : RK_WAVESPLIT_TILE;
     if (c.family == TF_DMA) return {producer_mode, r};
-    return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
-  }
-  if (quant == WavesplitQuant::BLOCK_F32 && w_aligned && N * ldw < (1ll << 32) && run.kernel == RK_DECODE && small_decode(kind, M, N, K, false, true)) {
-    const TileChoice c = best_decode_tile(kind, M, N, K);
-    Route r{};
-    r.kernel = RK_WAVESPLIT_TILE, r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
     return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
   }
   if (wavesplit_quant_preferred(quant, M, N, K, ldw)) {

@@ -77,8 +77,8 @@ struct TileLimits {
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
   double resident_margin = 0.93, resident_rounds_margin = 0.95;
-  double streamed_min_weight = 105e6, streamed_min_channels = 8000.0, streamed_one_token_min_kblocks = 63.0, streamed_one_token_min_channels = 11000.0, streamed_one_token_min_weight = 150e6, streamed_two_tokens_min_kblocks = 36.0;
-  double small_min_kblocks = 4.0, small_min_tokens = 4.0, small_min_channels = 192.0, small_max_tokens_values = 20800.0;
+  double streamed_min_weight = 100e6, streamed_two_tokens_min_kblocks = 33.0;
+  double small_min_tokens = 4.0, small_max_channels = 64.0 * NUM_CUS, small_max_tokens_values = 20800.0;
   double cold_min_weight = 40e6, cold_only_min_weight = 80e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
 struct TileModel {
@@ -372,17 +372,14 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
 // us, before / this: 18432 -> 14336 at 1 and 16 tokens block FP8 53.5 / 45.2, 64.1 / 47.9, INT8 55.7 / 44.4, 73.7 / 48.9; 8192 -> 14336 at 4 block
 // 36.8 / 23.4, packed exponents 29.3 / 23.4; 7168 -> 36864 at 4 INT8 53.2 / 44.2; 7168 -> 24576 at 8 per-token FP8 40.5 / 32.2; 12672 -> 14208 at 1
 // per-token FP8 40.2 / 30.1.
-// One and two tokens stay on the register kernel where its K is short, one token also on narrow weights up to where that kernel's limits end
-// (at 1: 3584 -> 36864 23.3 / 24.8, 7168 -> 18432 INT8 25.6 / 27.3, but 9344 -> 31744 49.8 / 47.2; at 2: 4096 -> 28672 22.8 / 23.7, but 7168 ->
-// 36864 INT8 49.2 / 44.3; block FP8 at 2 as at 1, it has the streaming kernel's quantizer).  Fewer than 8000 channels: the limits of
-// choose_limited_decode_tile hold.
-bool streamed_decode(GemmKind kind, int64_t M, int64_t N, int64_t K) {
+// One and two tokens stay on the register kernel where their K is one of its turns of 32 blocks and its quantizer saves the launch (at 1: 3584 -> 36864
+// 23.3 / 24.8; at 2: 4096 -> 28672 23.5 / 24.5; one token, 24 to 32 blocks, 64 linears 1.01).  From the second turn on they do not: 118 linears of
+// one token, 33 to 63 blocks, 0.92 (7552 -> 16384 24.2 / 21.9, 7168 -> 36864 48.9 / 47.0; at most 1.06, 16.5 to 20 thousand channels, which are a
+// second round of the tile), longer K on fewer than 11000 channels 0.81 (0.72 to 0.90), weights of 100 to 105 million 0.84 (0.70 to 0.95).
+bool streamed_decode(int64_t M, int64_t N, int64_t K) {
   const TileLimits& l = tile_model().limits;
-  const double kb = (double)ceil_div(K, KSTEP), weight = (double)(N * K);
-  if (M > 16 || K % KSTEP != 0 || N % 16 != 0 || weight < l.streamed_min_weight || (double)N < l.streamed_min_channels) return false;
-  if (M == 1 || (M == 2 && kind == GK_F32))
-    return kb >= l.streamed_one_token_min_kblocks && ((double)N >= l.streamed_one_token_min_channels || weight >= l.streamed_one_token_min_weight);
-  return M > 2 || kb >= l.streamed_two_tokens_min_kblocks;
+  if (M > 16 || K % KSTEP != 0 || N % 16 != 0 || (double)(N * K) < l.streamed_min_weight) return false;
+  return M > 2 || (double)ceil_div(K, KSTEP) >= l.streamed_two_tokens_min_kblocks;
 }
 double streamed_mid_us(int64_t M, int64_t N, int64_t K, int bn) {
   const StreamedTimes& t = tile_model().streamed;
@@ -415,21 +412,19 @@ TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoic
   return best;
 }
 
-// K of 4 to 16 blocks on weights of up to 20 million values, which the launches bound: the tile quantizes the tokens in its one launch and takes
-// their scales as they lie.  260 linears of 1 to 16 tokens, K = 512 to 2176, the tile's time by what it takes over from (geometric mean):
-//   the register kernel: K below 8 blocks FP8 0.66, INT8 0.83 from 9 tokens on (below 1.04); from 8 blocks on 0.87 at 9 to 16 tokens, per-token
-//   kinds 0.88 at 5 to 8 (block FP8 0.92, at most 1.08, and packed exponents 0.99: left), 1.03 at fewer; with more than five pieces of eight
-//   values a thread (20800 in all) the quantizer in every workgroup takes longer than its launch (2048 -> 4096 at 16 tokens 5.8 / 8.2);
-//   the streaming kernel: per-token FP8 0.67; fp32 scales 0.81 from 8 blocks and 9 tokens on.  Packed exponents and shorter K with fp32 scales
-//   stay on it, 128 channels too, which are eight workgroups.
-bool small_decode(GemmKind kind, int64_t M, int64_t N, int64_t K, bool from_wavesplit, bool from_streaming) {
+// K of up to 16 blocks on weights of up to 20 million values, which the launches bound: the tile quantizes the tokens in its one launch and takes
+// their scales as they lie.  600 linears of 1 to 16 tokens, the tile's time by what it takes over from (geometric mean, and range):
+//   the register kernel: K below 8 blocks FP8 0.61 (0.40 to 0.76), INT8 0.84 (0.41 to 0.99); from 8 blocks on 0.86 (0.73 to 1.00) from five tokens
+//   on, 1.01 (0.71 to 1.18) up to four; with more than five pieces of eight values a thread (20800 in all) the quantizer in every workgroup
+//   takes longer than its launch (2048 -> 4096 at 16 tokens 5.8 / 8.2);
+//   the streaming kernel: 0.61 (0.49 to 0.83) up to one round of its widest tile, 16384 channels; beyond, 1.19 (0.82 to 1.27; packed exponents
+//   640 -> 16896 at 16 tokens 8.3 / 10.0).
+bool small_decode(int64_t M, int64_t N, int64_t K, bool from_wavesplit, bool from_streaming) {
   const TileLimits& l = tile_model().limits;
   const int64_t kb = ceil_div(K, KSTEP);
-  if (M > 16 || K % KSTEP != 0 || (double)(N * K) > l.decode_short_max_weight || (double)kb < l.small_min_kblocks || (double)kb > l.decode_min_kblocks) return false;
-  const bool short_k = (double)kb < l.decode_short_min_kblocks, many = (double)M > l.decode_short_min_tokens;
-  if (from_wavesplit && !short_k && (double)(M * K) > l.small_max_tokens_values) return false;
-  if (from_wavesplit) return many || (short_k ? kind != GK_INT8 : (kind == GK_UNIT || kind == GK_INT8) && (double)M > l.small_min_tokens);
-  return from_streaming && (double)N >= l.small_min_channels && (kind == GK_UNIT || (kind == GK_F32 && many && !short_k));
+  if (M > 16 || K % KSTEP != 0 || (double)(N * K) > l.decode_short_max_weight || (double)kb > l.decode_min_kblocks) return false;
+  if (from_streaming) return (double)N <= l.small_max_channels;
+  return from_wavesplit && ((double)kb < l.decode_short_min_kblocks || ((double)M > l.small_min_tokens && (double)(M * K) <= l.small_max_tokens_values));
 }
 TileChoice best_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K) {
   const TileTimes& t = tile_times(kind);
@@ -475,8 +470,7 @@ TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64
     return TileChoice{TF_NONE, 0, 0, 1, 0.0};
   const bool few = (double)M <= (kind == GK_F32 ? l.decode_few_tokens_f32 : l.decode_few_tokens) && (double)kb <= l.decode_long_kblocks;
   const double most = padded ? l.decode_padded_max_weight : few ? l.decode_few_tokens_max_weight : l.decode_max_weight;
-  // (from the streaming kernel not a bare GEMM with fp32 scales: the one-call linear takes the tile for itself, choose_linear)
-  const bool small = small_decode(kind, M, N, K, from_wavesplit, from_streaming && kind != GK_F32);
+  const bool small = small_decode(M, N, K, from_wavesplit, from_streaming);
   const bool take = small || ((double)kb > l.decode_min_kblocks ? weight <= most
                                                       : (double)kb >= l.decode_short_min_kblocks && (double)N >= l.decode_short_min_channels &&
                                                             weight <= l.decode_short_max_weight && (double)M > l.decode_short_min_tokens);
@@ -488,9 +482,8 @@ TileChoice choose_limited_decode_tile(GemmKind kind, int64_t M, int64_t N, int64
 TileChoice choose_decode_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool from_wavesplit, bool from_streaming) {
   const TileChoice c = choose_limited_decode_tile(kind, M, N, K, base.family == TF_DMA, from_wavesplit, from_streaming);
   // (a bare GEMM with fp32 scales keeps its kernel: the mid-M tile may need a launch that lays the token scales out again.  The one-call
-  // linear of that kind lays them out as it likes: choose_linear.  Packed exponents stay on the streaming kernel where the table names it, 13 to 16
-  // tokens on K of up to 64 blocks that no single round of mid-M tiles covers: 7168 -> 19584 at 13 40.2, per-token FP8 there 40.3 / 33.1)
-  if (kind == GK_F32 || (kind == GK_UE8M0 && from_streaming) || !streamed_decode(kind, M, N, K)) return c;
+  // linear of that kind lays them out as it likes: choose_linear.)
+  if (kind == GK_F32 || !streamed_decode(M, N, K)) return c;
   return choose_streamed_tile(M, N, K, c.family != TF_NONE ? c : base);
 }
 

@@ -79,10 +79,10 @@ INT8_ROUTE_SHAPES = [
 VARIANT_SHAPES = {
     "fp8": {
         ("resident", "kb2"): (450, 16472, 256), ("resident", "kb3"): (452, 16528, 384), ("resident", "kb4"): (449, 16424, 512), ("resident", "kb5"): (450, 16504, 640),
-        ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
-        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
-        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
-        ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
+        ("decode", "split", "gpw1"): (13, 20864, 1536), ("decode", "split", "gpw3+"): (13, 66176, 1152),
+        ("decode", "whole", "gpw1"): (1, 16512, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6400, 1024),
+        ("decode_wavesplit", "w4", "one_round"): (1, 16, 1024), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
         ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
         ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
         ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (2761, 8, 7424),
@@ -118,13 +118,13 @@ VARIANT_SHAPES = {
     },
     "fp8_ue8m0": {
         ("resident", "kb2"): (450, 16472, 256), ("resident", "kb3"): (452, 16528, 384), ("resident", "kb4"): (449, 16424, 512), ("resident", "kb5"): (450, 16504, 640),
-        ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
-        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
-        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
-        ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
-        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
-        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (2761, 8, 7424),
+        ("decode", "split", "gpw1"): (13, 20864, 1536), ("decode", "split", "gpw3+"): (13, 66176, 1152),
+        ("decode", "whole", "gpw1"): (1, 16512, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6400, 1024),
+        ("decode_wavesplit", "w4", "one_round"): (1, 16, 1024),
+         ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
+        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840),
+         ("dma3", 128, "split", "bn128", "deep"): (2761, 8, 7424),
         ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (67, 8280, 13056),
         ("dma3", 128, "whole", "bn128", "deep"): (4238, 584, 512), ("dma3", 128, "whole", "bn192"): (97, 32896, 128),
         ("dma3", 128, "whole"): (289, 16408, 128), ("dma3", 160, "split", "bn128", "deep"): (2456, 8, 14080),
@@ -149,13 +149,13 @@ VARIANT_SHAPES = {
     },
     "fp8_scaled": {
         ("resident", "kb2"): (481, 16904, 256), ("resident", "kb3"): (484, 16496, 384), ("resident", "kb4"): (486, 16760, 512), ("resident", "kb5"): (486, 16584, 640),
-        ("decode", "split", "gpw1"): (9, 128, 1152), ("decode", "split", "gpw3+"): (13, 66176, 1152),
-        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
-        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6432, 128),
-        ("decode_wavesplit", "w4", "one_round"): (1, 16, 128), ("decode_wavesplit", "w4", "rounds", "two_tiles"): (1, 7936, 17664),
-        ("decode_wavesplit", "w4", "rounds"): (1, 10544, 13312), ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
-        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840), ("decode_wavesplit", "w8", "rounds", "two_tiles"): (3, 12416, 8064),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (3348, 8, 6272),
+        ("decode", "split", "gpw1"): (13, 20864, 1536), ("decode", "split", "gpw3+"): (13, 66176, 1152),
+        ("decode", "whole", "gpw1"): (1, 16512, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round", "two_tiles"): (3, 6400, 1024),
+        ("decode_wavesplit", "w4", "one_round"): (1, 16, 1024),
+         ("decode_wavesplit", "w8", "one_round", "two_tiles"): (3, 16512, 3840),
+        ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840),
+         ("dma3", 128, "split", "bn128", "deep"): (3348, 8, 6272),
         ("dma3", 128, "split", "bn192"): (71, 8272, 12160), ("dma3", 128, "split"): (67, 8280, 13056),
         ("dma3", 128, "whole", "bn128", "deep"): (194, 12416, 640), ("dma3", 128, "whole", "bn192"): (194, 16528, 128),
         ("dma3", 128, "whole"): (196, 24704, 128), ("dma3", 160, "split", "bn128", "deep"): (2716, 8, 10752),
@@ -188,10 +188,10 @@ VARIANT_SHAPES = {
     },
     "int8": {
         ("resident", "kb2"): (481, 16904, 256), ("resident", "kb3"): (484, 16496, 384), ("resident", "kb4"): (486, 16760, 512), ("resident", "kb5"): (542, 16592, 640),
-        ("decode", "whole", "gpw1"): (1, 128, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
-        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round"): (1, 16, 128),
-        ("decode_wavesplit", "w4", "rounds"): (1, 7936, 17664), ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840),
-        ("decode_wavesplit", "w8", "rounds"): (1, 13312, 7552), ("dma3", 128, "split", "bn128", "deep"): (2796, 8, 5760),
+        ("decode", "whole", "gpw1"): (1, 16512, 128), ("decode", "whole", "gpw2"): (1, 65664, 128),
+        ("decode", "whole", "gpw3+"): (2, 133376, 128), ("decode_wavesplit", "w4", "one_round"): (1, 16, 1024),
+         ("decode_wavesplit", "w8", "one_round"): (1, 16512, 3840),
+         ("dma3", 128, "split", "bn128", "deep"): (2796, 8, 5760),
         ("dma3", 128, "split", "bn192"): (198, 5448, 12288), ("dma3", 128, "split"): (329, 4352, 18560),
         ("dma3", 128, "whole", "bn128", "deep"): (194, 12416, 640), ("dma3", 128, "whole", "bn192"): (194, 16528, 128),
         ("dma3", 128, "whole"): (1295, 10760, 128), ("dma3", 160, "split", "bn128", "deep"): (2456, 8, 14080),
@@ -224,6 +224,10 @@ VARIANT_SHAPES = {
         ("wavesplit_tile", 64, 64, "ktail"): (323, 1536, 16),
     },
 }
+# Shapes that ran the register wave-split kernel in several turns or the streaming kernel before the wave-split tile took them over: one to
+# three K blocks for its eight waves, 16 and 128 channels, and the weights from 100 million on
+TAKEN_OVER_SHAPES = [(1, 16, 128), (1, 128, 128), (3, 6432, 128), (2, 48, 256), (16, 272, 384), (9, 128, 1152), (1, 7936, 17664), (1, 10544, 13312),
+                     (3, 12416, 8064), (1, 13312, 7552)]
 FP8_REQUIRED_VARIANTS = set(VARIANT_SHAPES["fp8"])
 INT8_REQUIRED_VARIANTS = set(VARIANT_SHAPES["int8"])
 
@@ -241,7 +245,9 @@ LINEAR_SHAPES = [(1, 128, 128), (15, 128, 1408), (8, 34176, 1536), (2, 18432, 74
                  (13, 25728, 1280), (2, 22400, 6784), (13, 33024, 1152), (2, 33216, 7168), (13, 49536, 1152), (1, 16, 2176), (2, 4144, 2176),
                  (9, 8320, 1024), (1, 16, 128), (4, 12528, 8064), (3, 6720, 128), (3, 13760, 7424), (16, 16, 2688), (16, 4336, 2688),
                  (15, 8336, 2816), (1, 8320, 128), (15, 16, 1280), (12, 16896, 128), (5, 4864, 28800), (3, 14208, 7168), (9, 128, 1152), (17, 16, 128),
-                 (1, 8, 128), (1, 8, 1024), (1, 66304, 128), (5, 27904, 8192)]
+                 (1, 8, 128), (1, 8, 1024), (1, 66304, 128), (5, 27904, 8192), (3, 78208, 256), (1, 131328, 128), (11, 16, 1920), (2, 23872, 3840),
+                 (2, 33472, 4096), (1, 80768, 3328), (3, 17408, 3840), (5, 17920, 3840), (13, 20864, 1536), (13, 65664, 1152), (1, 16512, 128),
+                 (7, 32512, 1792), (15, 28160, 1024), (5, 19392, 4096)]
 
 
 def linear_variant_of(plan: dict, M: int):

@@ -108,6 +108,7 @@ RECORDED_BOUNDARIES = {
     ("fp8", (8, 7168, 18432)): {("wavesplit_tile", 16, 32, 1): 25.6, ("decode_wavesplit", 16, 32, 1): 28.0},
     ("fp8", (128, 7168, 18432)): {("dma3", 128, 128, 4): 44.2, ("dma3", 64, 128, 2): 49.8, ("dma3", 128, 192, 6): 43.1},
     ("fp8", (4096, 576, 7168)): {("dma3", 64, 192, 1): 31.2, ("dma3", 96, 128, 1): 31.3},
+    ("int8", (1, 28672, 4096)): {("decode_wavesplit", 16, 16, 1): 23.2, ("dma3", 64, 128, 1): 21.8},
     ("int8", (256, 28672, 4096)): {("pingpong128", 128, 256, 1): 44.9, ("dma3", 128, 256, 1): 43.7},
     ("int8", (256, 4096, 14336)): {("dma3", 128, 128, 4): 32.6, ("wavesplit_tile", 64, 64, 1): 34.2},
     ("int8", (4096, 6144, 4096)): {("pingpong", 256, 256, 1): 100.7, ("dma3", 256, 128, 1): 97.6, ("dma3", 128, 256, 1): 101.2},
@@ -218,9 +219,11 @@ STREAMED_CHOICES = [
     # rows 4096 bytes apart too: the mid-M tile starts its K loops at different blocks there
     ("int8", (4, 28672, 4096), "dma3", 128),  # 24.2, 26.3
     ("token_fp8", (8, 28672, 4096), "dma3", 128),  # 24.1, 26.3
-    # what stays: short K at one and two tokens, few channels
+    # one and two tokens from the second turn of the register kernel on
+    ("ue8m0", (1, 16384, 7552), "wavesplit_tile", 64),  # 21.9, 24.2
+    # what stays: one turn of that kernel at one and two tokens, a tile that another models within 8 % of
     ("block", (1, 36864, 3584), "decode_wavesplit", 16),  # 23.3, 24.8
-    ("int8", (2, 28672, 4096), "decode_wavesplit", 16),  # 22.9, 23.6
+    ("int8", (2, 28672, 4096), "decode_wavesplit", 16),  # 23.5, 24.2
     ("int8", (2, 9728, 12672), "wavesplit_tile", 64),  # 25.6, 27.9
 ]
 
@@ -240,9 +243,13 @@ SMALL_CHOICES = [
     ("ue8m0", (7, 1600, 640), "wavesplit_tile"),  # 5.3, 8.4
     ("token_fp8", (16, 4288, 1280), "wavesplit_tile"),  # 6.8, 8.7
     ("block", (15, 1408, 1920), "wavesplit_tile"),  # 7.4, 11.7
-    # what stays: few tokens with K of 8 blocks and more (4.7, the tile no faster), many token values a workgroup
+    ("block", (16, 512, 512), "wavesplit_tile"),  # 4.2, 8.1
+    ("ue8m0", (9, 128, 1024), "wavesplit_tile"),  # 4.1, 6.1
+    ("token_fp8", (1, 2048, 128), "wavesplit_tile"),  # 3.3, 6.2
+    # what stays: up to four tokens with K of 8 blocks and more (4.7, the tile no faster), many token values a workgroup, many channels
     ("block", (2, 2688, 1280), "decode_wavesplit"),  # 4.7, 4.8
     ("block", (16, 4096, 2048), "decode_wavesplit"),  # 5.8, 8.2
+    ("ue8m0", (16, 16896, 640), "decode"),  # 8.3, 10.0
 ]
 
 
@@ -304,9 +311,9 @@ def test_block_linear_plan():
 
     from sglang_amd import _lib
 
-    for shape, want in (((1, 36864, 7168), ("fused", "decode_wavesplit")), ((3, 36864, 7168), ("fused", "dma3")), ((8, 36864, 7168), ("fused", "dma3")),
-                        ((1, 28672, 4096), ("fused", "decode_wavesplit")), ((8, 24576, 7168), ("fused", "dma3")), ((16, 512, 512), ("fused", "decode")),
-                        ((16, 2048, 7168), ("launch", "wavesplit_tile")), ((8, 7168, 2048), ("fused", "decode_wavesplit")),
+    for shape, want in (((1, 36864, 7168), ("fused", "dma3")), ((3, 36864, 7168), ("fused", "dma3")), ((8, 36864, 7168), ("fused", "dma3")),
+                        ((1, 28672, 4096), ("fused", "decode_wavesplit")), ((8, 24576, 7168), ("fused", "dma3")), ((16, 512, 512), ("fused", "wavesplit_tile")), ((16, 16896, 512), ("fused", "decode")),
+                        ((16, 2048, 7168), ("launch", "wavesplit_tile")), ((8, 7168, 2048), ("fused", "wavesplit_tile")), ((4, 7168, 2048), ("fused", "decode_wavesplit")),
                         ((4, 7168, 18432), ("launch", "wavesplit_tile")), ((16, 7168, 2048), ("fused", "wavesplit_tile")),
                         ((128, 7168, 2048), ("launch", "wavesplit_tile")), ((4, 1000, 1024), ("launch", "generic"))):
         p = _lib.block_linear_plan(*shape)
@@ -318,7 +325,7 @@ def test_block_linear_plan():
     from sglang_amd.fp8_utils import _one_call_takes_the_same_gemm
 
     for shape, want in (((8, 36864, 7168), True), ((16, 2048, 7168), True), ((4, 7168, 18432), True), ((4100, 1024, 256), True),
-                        ((40, 200, 384), True), ((1, 36864, 7168), True), ((3, 36864, 7168), False), ((8, 24576, 7168), False)):
+                        ((40, 200, 384), True), ((1, 28672, 4096), True), ((1, 36864, 7168), False), ((3, 36864, 7168), False), ((8, 24576, 7168), False)):
         assert _one_call_takes_the_same_gemm(*shape) == want, shape
     # the other linears promise that wherever they are: their GEMM is the one the entry point alone takes
     gemm = {"ue8m0": "fp8_ue8m0", "token_fp8": "fp8_scaled", "int8": "int8"}

@@ -136,8 +136,10 @@ def test_ue8m0_mid_m_kernel_against_oracle(gpu, oracle, M, N, K):
 
 # the streaming decode kernel: one K range and several, the last range short (K blocks not a multiple of 8), one to four
 # bytes used in the last exponent word, token counts below and at the 16 rows of the MFMA tile (rows past M repeat the last token)
-DECODE = [(8, 256, 512), (4, 4352, 512), (5, 4096, 36864), (16, 4096, 36864), (13, 19584, 7168), (12, 6016, 23296), (9, 3072, 1536),
-          (14, 70656, 1280), (15, 128, 1408), (15, 65536, 640), (16, 66560, 1152), (13, 3968, 35328), (8, 4352, 128)]
+DECODE = [(8, 16640, 512), (4, 20608, 512), (13, 20864, 1536), (14, 70656, 1280), (15, 65536, 640), (16, 66560, 1152), (8, 17408, 128), (16, 16512, 640)]
+# shapes that the wave-split tile took over from it
+DECODE_ON_THE_TILE = [(8, 256, 512), (4, 4352, 512), (5, 4096, 36864), (16, 4096, 36864), (13, 19584, 7168), (12, 6016, 23296), (9, 3072, 1536),
+                      (15, 128, 1408), (13, 3968, 35328), (8, 4352, 128)]
 
 
 def test_decode_shapes_reach_the_streaming_kernel():
@@ -146,9 +148,11 @@ def test_decode_shapes_reach_the_streaming_kernel():
     plans = [_lib.gemm_plan("fp8_ue8m0", M, N, K) for M, N, K in DECODE]
     assert all(p["kernel"] == "decode" for p in plans), plans
     assert {p["splits"] > 1 for p in plans} == {False, True}
+    plans = [_lib.gemm_plan("fp8_ue8m0", M, N, K) for M, N, K in DECODE_ON_THE_TILE]
+    assert all(p["kernel"] == "wavesplit_tile" for p in plans), plans
 
 
-@pytest.mark.parametrize("M,N,K", DECODE)
+@pytest.mark.parametrize("M,N,K", DECODE + DECODE_ON_THE_TILE)
 def test_ue8m0_decode_kernel_against_oracle(gpu, oracle, M, N, K):
     from sglang_amd.fp8_kernel import w8a8_block_fp8_matmul_deepgemm
 
@@ -190,11 +194,13 @@ def test_ue8m0_mid_m_exact_integers(gpu, oracle, M, N, K):
     _exact_integer_case(gpu, oracle, M, N, K)  # split and unsplit mid-M plans
 
 
-@pytest.mark.parametrize("M,N,K", [(8, 4352, 512), (13, 19584, 7168), (16, 3072, 1536), (14, 128, 2048), (5, 4096, 36864)])
-def test_ue8m0_decode_exact_integers(gpu, oracle, M, N, K):
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (8, 16640, 512, "decode"), (13, 20864, 1536, "decode"), (14, 66176, 1152, "decode"), (8, 4352, 512, "wavesplit_tile"), (13, 19584, 7168, "wavesplit_tile"),
+    (16, 3072, 1536, "wavesplit_tile"), (14, 128, 2048, "wavesplit_tile"), (5, 4096, 36864, "wavesplit_tile")])
+def test_ue8m0_decode_exact_integers(gpu, oracle, M, N, K, kernel):
     from sglang_amd import _lib
 
-    assert _lib.gemm_plan("fp8_ue8m0", M, N, K)["kernel"] == "decode"
+    assert _lib.gemm_plan("fp8_ue8m0", M, N, K)["kernel"] == kernel
     _exact_integer_case(gpu, oracle, M, N, K)
 
 

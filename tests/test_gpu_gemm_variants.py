@@ -5,7 +5,7 @@ multiplied twice or skipped, a wrong scale or a wrong row shows as a wrong numbe
 import pytest
 import torch
 
-from gemm_cases import MID_TILE_SWEEPS, VARIANT_SHAPES, plan_for, variant_of
+from gemm_cases import MID_TILE_SWEEPS, TAKEN_OVER_SHAPES, VARIANT_SHAPES, plan_for, variant_of
 
 pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
@@ -53,6 +53,13 @@ def check_exact(gpu, kind, M, N, K, pitch=None):
             assert torch.equal(ops.int8_mm_raw_accumulators(a8, w8.t()).double(), product), (kind, M, N, K)
             out = ops.int8_scaled_mm(a8, w8.t(), sa, sb, torch.bfloat16, bias)
     assert torch.equal(out, want.float().to(torch.bfloat16)), (kind, M, N, K)
+
+
+@pytest.mark.parametrize("kind", ["fp8", "fp8_ue8m0", "fp8_scaled", "int8"])
+@pytest.mark.parametrize("M,N,K", TAKEN_OVER_SHAPES)
+def test_taken_over_exact(gpu, kind, M, N, K):
+    print(f"case {kind} {(M, N, K)} {plan_for(kind, M, N, K)['kernel']}", flush=True)
+    check_exact(gpu, kind, M, N, K)
 
 
 @pytest.mark.parametrize("kind,variant", [(kind, v) for kind, shapes in VARIANT_SHAPES.items() for v in shapes],

@@ -133,21 +133,24 @@ def test_fused_block_fp8_linear(gpu, oracle, shape, N, K, with_bias):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K,quantizer,kernel,gemm", [
     # the streaming kernel's prologue: K whole and split, one, two and more channel groups per workgroup, a short last K range
-    (16, 512, 512, "fused", "decode", "decode"), (5, 66048, 512, "fused", "decode", "decode"), (9, 256, 128, "fused", "decode", "decode"),
-    (15, 128, 1408, "fused", "decode", "decode"), (8, 34176, 1536, "fused", "decode", "decode_wavesplit"),
-    (2, 18432, 7424, "fused", "decode", "decode_wavesplit"),
+    (16, 16896, 512, "fused", "decode", "decode"), (5, 66048, 512, "fused", "decode", "decode"), (9, 20480, 128, "fused", "decode", "decode"),
+    (13, 20864, 1536, "fused", "decode", "decode"), (13, 65664, 1152, "fused", "decode", "decode"), (8, 34176, 1536, "fused", "decode", "decode_wavesplit"),
     # a quantizer launch in front of the wave-split kernels
-    (3, 13760, 7424, "launch", "decode_wavesplit", "decode_wavesplit"), (4, 7168, 18432, "launch", "wavesplit_tile", "wavesplit_tile"),
+    (15, 17408, 1408, "launch", "decode_wavesplit", "decode_wavesplit"), (4, 7168, 18432, "launch", "wavesplit_tile", "wavesplit_tile"),
     (12, 2048, 7168, "launch", "wavesplit_tile", "wavesplit_tile"),
     # the wave-split kernels' own quantizers
     (1, 2048, 7168, "fused", "wavesplit_tile", "wavesplit_tile"), (16, 7168, 2048, "fused", "wavesplit_tile", "wavesplit_tile"),
-    (1, 36864, 7168, "fused", "decode_wavesplit", "decode_wavesplit"),
+    (16, 512, 512, "fused", "wavesplit_tile", "wavesplit_tile"), (9, 256, 128, "fused", "wavesplit_tile", "wavesplit_tile"),
+    (15, 128, 1408, "fused", "wavesplit_tile", "wavesplit_tile"),
+    (1, 28672, 4096, "fused", "decode_wavesplit", "decode_wavesplit"), (4, 7168, 2048, "fused", "decode_wavesplit", "decode_wavesplit"),
+    # ... for the linear only, with the weight as a stream
+    (3, 13760, 7424, "fused", "wavesplit_tile", "decode_wavesplit"), (2, 18432, 7424, "launch", "wavesplit_tile", "decode_wavesplit"),
     # the mid-M kernel's producer waves: 128-, 192- and 256-channel tiles (six, four and three stages), K of 12, 9, 9, 10 and 56 blocks,
     # the last with a ragged last channel tile
     (16, 24576, 1536, "fused", "dma3", "dma3"), (13, 53248, 1152, "fused", "dma3", "dma3"), (16, 32768, 1152, "fused", "dma3", "dma3"),
     (13, 45056, 1280, "fused", "dma3", "dma3"), (8, 36800, 7168, "fused", "dma3", "dma3"),
     # ... for the linear only: fewer tokens than the GEMM's own threshold; K of many ranges for the streaming kernel
-    (2, 36864, 7168, "fused", "dma3", "decode_wavesplit"), (3, 22400, 6784, "fused", "dma3", "decode_wavesplit")])
+    (1, 36864, 7168, "fused", "dma3", "decode_wavesplit"), (2, 36864, 7168, "fused", "dma3", "decode_wavesplit"), (3, 22400, 6784, "fused", "dma3", "decode_wavesplit")])
 def test_decode_linear_quantizes_in_the_gemm_kernel(gpu, oracle, M, N, K, quantizer, kernel, gemm, dtype):
     """At decode sizes the one-call linear has no quantizer launch where that is the faster way: the streaming and the
     wave-split kernels quantize the tokens in their prologues, the mid-M kernel by producer waves.  Same arithmetic on the same

@@ -41,7 +41,7 @@ def test_noalloc_matches_workspace_entry_point_twice_in_a_row(gpu, oracle):
 
     L = _lib.lib()
     # split-K decode (36 splits, 4.7 MB of partials), then a smaller split problem, then mid-M split, then one without split
-    shapes = [(8, 4096, 36864), (12, 3072, 1536), (48, 7168, 18432), (300, 1024, 512)]
+    shapes = [(8, 4096, 36864), (13, 20864, 1536), (48, 7168, 18432), (300, 1024, 512)]
     plans = [_lib.gemm_plan("fp8", *s) for s in shapes]
     assert plans[0]["splits"] > 1 and plans[1]["splits"] > 1 and plans[2]["splits"] > 1 and plans[3]["splits"] == 1
     problems = [_problem(*s, seed=i + 1, gpu=gpu) for i, s in enumerate(shapes)]
