@@ -229,6 +229,13 @@ int mi355_probe_fp8_mfma_stream(int mode, int workgroups, int iters, const void*
 int mi355_probe_int8_mfma_stream(int mode, int workgroups, int iters, const void* a, const void* b, void* out, void* stream);
 
 /*
+ * Checking aid, not an operator (no counterpart in the reference): counts the significands of s = 1.x * 2^exponent for which the
+ * arithmetic of the quantizers inside the decode GEMMs differs from the `/` operator.  Adds to mismatches[0] those of 1 / s, to
+ * mismatches[1] those of s / 448 (two 64-bit counters in device memory).  exponent -100 .. 120.
+ */
+int mi355_probe_reciprocal(int exponent, void* mismatches, void* stream);
+
+/*
  * Per-token x per-channel INT8 GEMM:  acc = sum_k a[m,k] * b[n,k] exactly in int32;
  *   out[m,n] = cast( f32(acc) * (sb[n] * sa[m]) + f32(bias[n]) ).
  * Replaces int8_scaled_mm (sgl-kernel/csrc/gemm/int8_gemm_kernel.cu:663-747; epilogue order of

@@ -91,6 +91,12 @@ __device__ __forceinline__ float div_by_shared(float x, float s, float r) {
   const float q = x * r;
   return fmaf(fmaf(-q, s, x), r, q);
 }
+// RN(1 / s), s and 1 / s normal: the hardware's reciprocal and one Newton step.  The same as the `/` operator for every significand and every
+// exponent that a scale can have (mi355_probe_reciprocal).
+__device__ __forceinline__ float refined_reciprocal(float s) {
+  const float r = __builtin_amdgcn_rcpf(s);
+  return fmaf(fmaf(-s, r, 1.0f), r, r);
+}
 // The lane's eight 16-bit elements (raw) of a group spread over its DPP row -> their eight e4m3fn codes and the group's scale
 // (the same value in all 16 lanes).  Every lane of the row must be active.  by_reciprocal (wave-uniform): q = x * (1 / s) as the
 // reference's row-major-scale quantizer computes it (fp8_kernel.py:156-158), else the true division of its M-major one.
@@ -105,9 +111,7 @@ __device__ __forceinline__ u32x2 quantize_group_lane(const u32x4& raw, bool by_r
   // (a group with an infinity: scale infinity, reciprocal zero, as the `/` operator has them; the refinements would make NaN of them)
   const bool finite = __float_as_uint(amax) < 0x7f800000u;
   const float sc = finite ? div_by_shared(amax, 448.0f, 1.0f / 448.0f) : amax;
-  // RN(1 / s): the hardware's reciprocal and one Newton step, checked against the `/` operator for every significand of s
-  const float r0 = __builtin_amdgcn_rcpf(sc);
-  const float rcp = finite ? fmaf(fmaf(-sc, r0, 1.0f), r0, r0) : r0;
+  const float rcp = finite ? refined_reciprocal(sc) : __builtin_amdgcn_rcpf(sc);
   float t[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) t[e] = v[e] * rcp;

@@ -12,7 +12,7 @@
 //   mode 1  v_mfma_i32_32x32x32_i8 accumulating in place (16 per round)
 // Each of the 8 waves of a workgroup (two per SIMD, as in the kernels) holds four weight and four token fragments and
 // runs `iters` rounds of their 16 products.
-#include "common.h"
+#include "gemm_common.h"
 
 namespace mi355 {
 namespace {
@@ -158,10 +158,27 @@ __global__ __launch_bounds__(512) void int8_mfma_stream_kernel(const uint8_t* a,
   out[blockIdx.x * 512 + threadIdx.x] = sum;
 }
 
+// mismatches[0]: refined_reciprocal against 1 / s, [1]: div_by_shared by 448 against s / 448; every significand, one a thread
+__global__ __launch_bounds__(256) void reciprocal_kernel(int exponent, unsigned long long* mismatches) {
+  const float s = __uint_as_float(((uint32_t)(127 + exponent) << 23) | (blockIdx.x * 256 + threadIdx.x));
+  if (refined_reciprocal(s) != 1.0f / s) atomicAdd(&mismatches[0], 1ull);
+  if (div_by_shared(s, 448.0f, 1.0f / 448.0f) != s / 448.0f) atomicAdd(&mismatches[1], 1ull);
+}
+
 }  // namespace
 }  // namespace mi355
 
 using namespace mi355;
+
+extern "C" int mi355_probe_reciprocal(int exponent, void* mismatches, void* stream) {
+  const char* what = "mi355_probe_reciprocal";
+  clear_error();
+  MI355_REQUIRE(exponent >= -100 && exponent <= 120, MI355_ERR_INVALID_ARGUMENT, "%s: exponent -100..120", what);
+  MI355_REQUIRE(mismatches, MI355_ERR_INVALID_ARGUMENT, "%s: null pointer", what);
+  hipLaunchKernelGGL(reciprocal_kernel, dim3((1u << 23) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), exponent,
+                     static_cast<unsigned long long*>(mismatches));
+  return check_launch(what);
+}
 
 extern "C" int mi355_probe_fp8_mfma_stream(int mode, int workgroups, int iters, const void* a, const void* b, void* out,
                                            void* stream) {

@@ -55,9 +55,33 @@ def test_fused_quantizer_of_the_wavesplit_kernel(gpu, oracle, M, N, K, dtype):
     assert torch.equal(bits(ops.int8_linear(xg, iw, isc, bias, dtype)), bits(ops.int8_scaled_mm(q, iw, s, isc, dtype, bias)))
 
 
-@pytest.mark.parametrize("kind", ["block", "block_rcp", "ue8m0", "token_fp8", "int8"])
+def test_reciprocal_on_every_significand(gpu):
+    """RN(1 / s) and RN(s / 448) of the quantizers inside the GEMMs, for every float of the exponents that a scale (or, for the second, a
+    group's maximum) can have: 1e-10 / 448 and up to the largest bfloat16."""
+    import ctypes
+
+    from sglang_amd import _lib
+
+    counts = torch.zeros(2, dtype=torch.int64, device=gpu)
+    for e in range(-43, 120):
+        _lib.check(_lib.lib().mi355_probe_reciprocal(e, ctypes.c_void_p(counts.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert counts.tolist() == [0, 0]
+    assert _lib.lib().mi355_probe_reciprocal(121, ctypes.c_void_p(counts.data_ptr()), None) == 1
+
+
+# every kernel that quantizes tokens itself: (kinds, kernel, channel tile or waves, shape)
+FUSED_KERNELS = [(("block", "block_rcp", "ue8m0", "token_fp8", "int8"), "wavesplit_tile", 0, (16, 2176, 2176)),
+                 (("block", "block_rcp", "ue8m0", "token_fp8", "int8"), "wavesplit_tile", 0, (16, 1024, 512)),
+                 (("block", "block_rcp", "ue8m0", "token_fp8", "int8"), "decode_wavesplit", 4, (4, 7168, 2048)),
+                 (("block", "block_rcp", "ue8m0", "token_fp8", "int8"), "decode_wavesplit", 8, (1, 16512, 3840)),
+                 (("block", "block_rcp"), "decode", 1, (16, 16896, 512)), (("block", "block_rcp"), "decode", 1, (13, 20864, 1536)),
+                 (("block", "block_rcp"), "dma3", 128, (16, 24576, 1536)), (("block", "block_rcp"), "dma3", 192, (13, 45056, 1280)),
+                 (("block", "block_rcp"), "dma3", 256, (13, 53248, 1152))]
+
+
+@pytest.mark.parametrize("kind,kernel,detail,M,N,K", [(kind, k, d, *s) for kinds, k, d, s in FUSED_KERNELS for kind in kinds])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_fused_quantizer_on_every_16_bit_value(gpu, kind, dtype):
+def test_fused_quantizer_on_every_16_bit_value(gpu, kind, dtype, kernel, detail, M, N, K):
     """Every bit pattern (infinities and NaN among them) through a one-hot weight: a channel's result is one code times its scales,
     so the quantizer inside the GEMM has to write the codes and scales of the quantizer kernels."""
     from sglang_amd import _lib, ops
@@ -65,15 +89,17 @@ def test_fused_quantizer_on_every_16_bit_value(gpu, kind, dtype):
     from sglang_amd.fp8_utils import requant_weight_ue8m0
     from sglang_amd.int8_kernel import per_token_quant_int8
 
-    M, N, K = 16, 2176, 2176
-    assert _lib.linear_plan(kind.split("_rcp")[0], M, N, K)["quantizer"] == "fused"
+    plan = _lib.linear_plan(kind.split("_rcp")[0], M, N, K)
+    assert plan["quantizer"] == "fused" and plan["kernel"] == kernel and detail in (0, plan["bn" if kernel == "dma3" else "groups_per_wg"]), plan
+    calls = -(-65536 // (M * K))
     patterns = torch.randperm(65536, generator=torch.Generator().manual_seed(3))
-    patterns = torch.cat([patterns, torch.zeros(2 * M * K - 65536, dtype=torch.int64)]).to(torch.int32).to(torch.int16).view(2, M, K)
+    patterns = torch.cat([patterns, torch.zeros(calls * M * K - 65536, dtype=torch.int64)]).to(torch.int32).to(torch.int16).view(calls, M, K)
     # a second pair of inputs, all finite and sorted: groups of one magnitude, where the rounding of every quotient shows
     finite = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
     finite = finite[torch.isfinite(finite)].float().sort().values.to(dtype)
-    finite = torch.cat([finite, torch.zeros(2 * M * K - finite.numel(), dtype=dtype)]).view(2, M, K)
-    w = torch.eye(N, device=gpu)
+    finite = torch.cat([finite, torch.zeros(calls * M * K - finite.numel(), dtype=dtype)]).view(calls, M, K)
+    w = torch.zeros(N, K, device=gpu, dtype=torch.float16)
+    w[torch.arange(N), torch.arange(N) % K] = 1
     one, ones = torch.ones(N, device=gpu), torch.ones(N // 128, K // 128, device=gpu)
     for x in [*patterns.view(dtype), *finite]:
         if kind == "ue8m0":  # (the two quantizers of this kind clamp a NaN to different ends)
