@@ -5,8 +5,8 @@
 // tokens, all tiles and splits, weights rotated out of the caches, and results too where they are large): 4 % root mean square for
 // the mid-M tiles, 6 % for the wave-split ones.  With larger operands than those shapes had, the wave-split tiles take 1.1 to 1.5
 // times the modelled time: the limits below lie where they stop being the faster ones.
-// The route that runs against the constants table alone, 720 random shapes (profiles/tile_choice_random_shapes.txt): 16 % faster for
-// FP8, 18 % with packed exponents, 13 % per token, 19 % for INT8 (geometric means); more than 5 % slower at 34 shapes, by up to 15 %.
+// The route that runs against the constants table alone, 720 random shapes (profiles/tile_choice_random_shapes.txt): 19 % faster for
+// FP8, 21 % with packed exponents, 17 % per token, 22 % for INT8 (geometric means); more than 5 % slower at 13 shapes, by up to 17 %.
 #pragma once
 
 #include <algorithm>
@@ -368,7 +368,7 @@ TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
 
 // Up to 16 tokens on a weight large enough to be loaded as a stream (streams_weight): the wave-split and the mid-M tile have such loads, the
 // register wave-split kernel and the streaming kernel, whose instructions fetch parts of lines, lose by them.  Fitted to 290 linears
-// (100 to 480 million weights): 3 % root mean square; what it chooses takes 1.01 of the best one's time; 103 random ones take 0.86 of what ran before.
+// (100 to 480 million weights): 3 % root mean square; what it chooses takes 1.01 of the best one's time.
 // us, before / this: 18432 -> 14336 at 1 and 16 tokens block FP8 53.5 / 45.2, 64.1 / 47.9, INT8 55.7 / 44.4, 73.7 / 48.9; 8192 -> 14336 at 4 block
 // 36.8 / 23.4, packed exponents 29.3 / 23.4; 7168 -> 36864 at 4 INT8 53.2 / 44.2; 7168 -> 24576 at 8 per-token FP8 40.5 / 32.2; 12672 -> 14208 at 1
 // per-token FP8 40.2 / 30.1.
