@@ -343,7 +343,9 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
   gp.g.sa_sm = 1, gp.g.sa_sk = pl.pitch, gp.g.sb_sn = sb_sn, gp.g.sb_sk = sb_sk;
   gp.g.kb_total = KB;
   gp.g.out_dtype = out_dtype;
-  gp.g.write_through = writes_through(total_m, N);
+  // (not results below 4 MB, which lie beside the stream of the experts' weights: 256 experts, 94 rows, 1664 -> 1664 46.6 us, 47.4 written through,
+  // 32 experts, 64 rows, 2048 -> 4096 44.9, 45.6)
+  gp.g.write_through = writes_through(total_m, N) && total_m * N * 2 >= 4000000;
   gp.b_expert_stride = b_expert_stride;
   gp.sb_expert_stride = sb_expert_stride;
   gp.out_elem = 2;

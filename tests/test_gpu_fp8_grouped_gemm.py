@@ -90,12 +90,12 @@ def test_streamed_expert_weights(gpu, E, rows, N, K):
         assert torch.equal(out[r0:r0 + m], want.bfloat16()), e
 
 
-@pytest.mark.parametrize("rows", [15625, 15626])
+@pytest.mark.parametrize("rows", [488, 489, 15625, 15626])
 def test_results_written_through(gpu, rows):
-    """Results of all experts on both sides of the size (128 MB) up to which they are written through the L2.  Whole numbers, exact."""
+    """Results of all experts on both sides of the sizes (4 and 128 MB) between which they are written through the L2.  Whole numbers, exact."""
     E, N, K = 4, 4096, 256
     g = torch.Generator().manual_seed(rows)
-    sizes = [1000, 70, 6500, rows - 7570]
+    sizes = [rows // 16, 70, rows // 16 * 6, rows - rows // 16 * 7 - 70]
     offsets = [sum(sizes[:e]) for e in range(E)]
     a = torch.randint(-2, 3, (rows, K), generator=g, dtype=torch.int8).float().to(FP8)
     w = torch.randint(-2, 3, (E, N, K), generator=g, dtype=torch.int8).half().to(FP8)
