@@ -181,9 +181,9 @@ extern "C" int mi355_block_cast_to_fp8(const void* x, int x_dtype, void* q, floa
 #define MI355_LAUNCH_CAST(DT_)                                                                                      \
   do {                                                                                                              \
     if (vec)                                                                                                        \
-      hipLaunchKernelGGL((block_cast_kernel<DT_, true>), grid, dim3(256), 0, st, x, qq, s, m, n, blocks_n);         \
+      launch_kernel((block_cast_kernel<DT_, true>), grid, dim3(256), 0, st, x, qq, s, m, n, blocks_n);         \
     else                                                                                                            \
-      hipLaunchKernelGGL((block_cast_kernel<DT_, false>), grid, dim3(256), 0, st, x, qq, s, m, n, blocks_n);        \
+      launch_kernel((block_cast_kernel<DT_, false>), grid, dim3(256), 0, st, x, qq, s, m, n, blocks_n);        \
   } while (0)
   switch (x_dtype) {
     case MI355_F32: MI355_LAUNCH_CAST(MI355_F32); break;
@@ -209,9 +209,9 @@ extern "C" int mi355_block_dequant_fp8(const void* q, const float* s, void* out,
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint8_t* qq = static_cast<const uint8_t*>(q);
   switch (out_dtype) {
-    case MI355_F32: hipLaunchKernelGGL(block_dequant_kernel<MI355_F32>, grid, dim3(256), 0, st, qq, s, out, n, k, blocks_k); break;
-    case MI355_F16: hipLaunchKernelGGL(block_dequant_kernel<MI355_F16>, grid, dim3(256), 0, st, qq, s, out, n, k, blocks_k); break;
-    default: hipLaunchKernelGGL(block_dequant_kernel<MI355_BF16>, grid, dim3(256), 0, st, qq, s, out, n, k, blocks_k);
+    case MI355_F32: launch_kernel(block_dequant_kernel<MI355_F32>, grid, dim3(256), 0, st, qq, s, out, n, k, blocks_k); break;
+    case MI355_F16: launch_kernel(block_dequant_kernel<MI355_F16>, grid, dim3(256), 0, st, qq, s, out, n, k, blocks_k); break;
+    default: launch_kernel(block_dequant_kernel<MI355_BF16>, grid, dim3(256), 0, st, qq, s, out, n, k, blocks_k);
   }
   return check_launch(what);
 }

@@ -284,13 +284,13 @@ template <bool IS_FP8, int W, int KBW, bool UE8M0 = false, int CT = 1, TokenQuan
 int launch_variant(const GemmParams& p, hipStream_t stream, const char* what) {
   const dim3 grid((unsigned)(p.N / (16 * CT))), block(64 * W);
   if constexpr (TQ == TQ_NONE) {
-    hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT>), grid, block, 0, stream, p);
+    launch_kernel((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT>), grid, block, 0, stream, p);
   } else {
     const size_t lds = (size_t)ws_scale_bytes(TQ == TQ_GROUP, p.M, p.kb_total) + (size_t)p.M * (p.K + 16);
     const int64_t pieces = (int64_t)p.M * p.K / 8;  // over 64 W threads, 2, 4 or WS_QUANT_VECTORS each
-    if (pieces <= 2 * 64 * W) hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, 2>), grid, block, lds, stream, p);
-    else if (pieces <= 4 * 64 * W) hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, 4>), grid, block, lds, stream, p);
-    else hipLaunchKernelGGL((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, WS_QUANT_VECTORS>), grid, block, lds, stream, p);
+    if (pieces <= 2 * 64 * W) launch_kernel((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, 2>), grid, block, lds, stream, p);
+    else if (pieces <= 4 * 64 * W) launch_kernel((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, 4>), grid, block, lds, stream, p);
+    else launch_kernel((decode_wavesplit_kernel<IS_FP8, W, KBW, UE8M0, CT, TQ, WS_QUANT_VECTORS>), grid, block, lds, stream, p);
   }
   return check_launch(what);
 }

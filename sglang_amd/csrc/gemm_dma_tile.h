@@ -426,8 +426,8 @@ int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   // 36 rows, 3840 -> 256, 17.7 / 18.6 us; the streamed one has them, its blocks wait for memory)
   const auto launch = [&](auto split, auto streamed, auto rotates) {
     constexpr bool SPLIT = decltype(split)::value, STREAM = decltype(streamed)::value, ROTATES = decltype(rotates)::value;
-    if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, SHARED, STREAM, ROTATES>), grid, dim3(T_THREADS), 0, stream, p);
-    else hipLaunchKernelGGL((gemm_dma_kernel<AR, BM, BN, SPLIT, OWN, STREAM, ROTATES>), grid, dim3(T_THREADS), 0, stream, p);
+    if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n * p.splits > NUM_CUS) launch_kernel((gemm_dma_kernel<AR, BM, BN, SPLIT, SHARED, STREAM, ROTATES>), grid, dim3(T_THREADS), 0, stream, p);
+    else launch_kernel((gemm_dma_kernel<AR, BM, BN, SPLIT, OWN, STREAM, ROTATES>), grid, dim3(T_THREADS), 0, stream, p);
   };
   const std::true_type yes;
   const std::false_type no;

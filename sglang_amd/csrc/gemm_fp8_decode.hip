@@ -402,22 +402,22 @@ static int launch_decode(GemmParams& p, int gpw, hipStream_t stream, const char*
   if constexpr (IS_FP8) {
     if (p.x16 != nullptr) {  // tokens arrive unquantized
       if (p.splits > 1)
-        hipLaunchKernelGGL((decode_kernel<true, true, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
+        launch_kernel((decode_kernel<true, true, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
       else
-        hipLaunchKernelGGL((decode_kernel<true, false, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
+        launch_kernel((decode_kernel<true, false, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
       return check_launch(what);
     }
   }
   if (p.splits > 1) {
     if constexpr (IS_FP8) {
-      hipLaunchKernelGGL((decode_kernel<true, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
+      launch_kernel((decode_kernel<true, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
     } else {
       // INT8 shapes with more than one K range (8 blocks) all go to the wave-split kernel: this variant is not built
       set_error("%s: the INT8 streaming decode kernel has no K split", what);
       return MI355_ERR_UNSUPPORTED;
     }
   } else {
-    hipLaunchKernelGGL((decode_kernel<IS_FP8, false>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
+    launch_kernel((decode_kernel<IS_FP8, false>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
   }
   return check_launch(what);
 }
@@ -430,9 +430,9 @@ int launch_fp8_decode(GemmParams& p, int gpw, hipStream_t stream, const char* wh
     p.tiles_n = groups_n;
     const dim3 grid((unsigned)(wg_per_split * p.splits));
     if (p.splits > 1)
-      hipLaunchKernelGGL((decode_kernel<true, true, false, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
+      launch_kernel((decode_kernel<true, true, false, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
     else
-      hipLaunchKernelGGL((decode_kernel<true, false, false, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
+      launch_kernel((decode_kernel<true, false, false, true>), grid, dim3(64 * WAVES), 0, stream, p, gpw, wg_per_split);
     return check_launch(what);
   }
   return launch_decode<true>(p, gpw, stream, what);

@@ -395,11 +395,11 @@ int launch_fp8_grouped_dma3(GroupedParams& gp, int bm, int bn, bool few, bool st
   const dim3 block(T_THREADS);
   const auto launch = [&](auto streamed) {
     constexpr bool STREAM = decltype(streamed)::value;
-    if (bm == 64 && bn == 128 && few) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, true), STREAM>), grid, block, 0, stream, gp);
-    else if (bm == 64 && bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, false), STREAM>), grid, block, 0, stream, gp);
-    else if (bn == 128) hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 128, stages_of(128, 128, true), STREAM>), grid, block, 0, stream, gp);
-    else if (bm == 64) hipLaunchKernelGGL((fp8_grouped_dma_kernel<64, 256, stages_of(64, 256, true), STREAM>), grid, block, 0, stream, gp);
-    else hipLaunchKernelGGL((fp8_grouped_dma_kernel<128, 256, stages_of(128, 256, true), STREAM>), grid, block, 0, stream, gp);
+    if (bm == 64 && bn == 128 && few) launch_kernel((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, true), STREAM>), grid, block, 0, stream, gp);
+    else if (bm == 64 && bn == 128) launch_kernel((fp8_grouped_dma_kernel<64, 128, stages_of(64, 128, false), STREAM>), grid, block, 0, stream, gp);
+    else if (bn == 128) launch_kernel((fp8_grouped_dma_kernel<128, 128, stages_of(128, 128, true), STREAM>), grid, block, 0, stream, gp);
+    else if (bm == 64) launch_kernel((fp8_grouped_dma_kernel<64, 256, stages_of(64, 256, true), STREAM>), grid, block, 0, stream, gp);
+    else launch_kernel((fp8_grouped_dma_kernel<128, 256, stages_of(128, 256, true), STREAM>), grid, block, 0, stream, gp);
   };
   if (streamed) launch(std::true_type{});
   else launch(std::false_type{});
@@ -422,9 +422,9 @@ int launch_fp8_dma3_quant(GemmParams& p, int bn, hipStream_t stream, const char*
   const dim3 grid((unsigned)p.tiles_n), block(T_THREADS + 64 * T_PW);
   const auto launch = [&](auto streamed) {
     constexpr bool STREAM = decltype(streamed)::value;
-    if (bn == 128) hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<128, 6, STREAM>), grid, block, 0, stream, p);
-    else if (bn == 192) hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<192, 4, STREAM>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((fp8_gemm_dma3_q_kernel<256, 3, STREAM>), grid, block, 0, stream, p);
+    if (bn == 128) launch_kernel((fp8_gemm_dma3_q_kernel<128, 6, STREAM>), grid, block, 0, stream, p);
+    else if (bn == 192) launch_kernel((fp8_gemm_dma3_q_kernel<192, 4, STREAM>), grid, block, 0, stream, p);
+    else launch_kernel((fp8_gemm_dma3_q_kernel<256, 3, STREAM>), grid, block, 0, stream, p);
   };
   if (streams_weight(p)) launch(std::true_type{});
   else launch(std::false_type{});

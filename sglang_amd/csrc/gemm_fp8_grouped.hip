@@ -329,7 +329,7 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
   float* sa_mm = reinterpret_cast<float*>(wsp + pl.big_bytes + small_bytes);
   const int KB = (int)(K / KSTEP);
   const GroupedTables tables{(int)num_experts, (int)total_m, run.bm, (int)run.use_big, run.max_big, run.max_small, big_tiles, small_tiles};
-  hipLaunchKernelGGL(grouped_prepare_kernel, dim3((unsigned)((total_m + CHUNK - 1) / CHUNK + 1), (unsigned)((KB + 31) / 32)), dim3(256), 0, st,
+  launch_kernel(grouped_prepare_kernel, dim3((unsigned)((total_m + CHUNK - 1) / CHUNK + 1), (unsigned)((KB + 31) / 32)), dim3(256), 0, st,
                      problem_sizes, expert_offsets, tables, scales_a, sa_sm, sa_sk, sa_mm, pl.pitch, KB);
   int rc = check_launch(what);
   if (rc != MI355_OK) return rc;

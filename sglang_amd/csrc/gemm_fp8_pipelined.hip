@@ -270,7 +270,7 @@ int launch_fp8_pipelined(GemmParams& p, hipStream_t stream, const char* what) {
     }
     lds_reserved = true;
   }
-  hipLaunchKernelGGL(fp8_gemm_pipelined_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(THREADS), P_LDS, stream, p);
+  launch_kernel(fp8_gemm_pipelined_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(THREADS), P_LDS, stream, p);
   return check_launch(what);
 }
 

@@ -417,7 +417,7 @@ int launch_fp8_grouped_pp(GroupedParams& gp, hipStream_t stream, const char* wha
   gp.g.tiles_n = (gp.g.N + G_BN - 1) / G_BN;
   gp.g.splits = 1, gp.g.kb_per_split = gp.g.kb_total;
   const dim3 grid((unsigned)(gp.max_tiles_m * gp.g.tiles_n));
-  hipLaunchKernelGGL(fp8_grouped_pp_kernel, grid, dim3(G_THREADS), 0, stream, gp);
+  launch_kernel(fp8_grouped_pp_kernel, grid, dim3(G_THREADS), 0, stream, gp);
   return check_launch(what);
 }
 
@@ -427,9 +427,9 @@ int launch_fp8_pp(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_n = (p.N + G_BN - 1) / G_BN;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
   if (p.K % KSTEP == 0)
-    hipLaunchKernelGGL((fp8_gemm_pp_kernel<true, SM_BLOCK_F32>), grid, dim3(G_THREADS), 0, stream, p);
+    launch_kernel((fp8_gemm_pp_kernel<true, SM_BLOCK_F32>), grid, dim3(G_THREADS), 0, stream, p);
   else
-    hipLaunchKernelGGL((fp8_gemm_pp_kernel<false, SM_BLOCK_F32>), grid, dim3(G_THREADS), 0, stream, p);
+    launch_kernel((fp8_gemm_pp_kernel<false, SM_BLOCK_F32>), grid, dim3(G_THREADS), 0, stream, p);
   return check_launch(what);
 }
 
@@ -438,7 +438,7 @@ int launch_fp8_pp_noload(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + G_BM - 1) / G_BM;
   p.tiles_n = (p.N + G_BN - 1) / G_BN;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
-  hipLaunchKernelGGL((fp8_gemm_pp_kernel<true, SM_BLOCK_F32, true>), grid, dim3(G_THREADS), 0, stream, p);
+  launch_kernel((fp8_gemm_pp_kernel<true, SM_BLOCK_F32, true>), grid, dim3(G_THREADS), 0, stream, p);
   return check_launch(what);
 }
 
@@ -448,7 +448,7 @@ int launch_fp8_pp_ue8m0(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + G_BM - 1) / G_BM;
   p.tiles_n = (p.N + G_BN - 1) / G_BN;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
-  hipLaunchKernelGGL((fp8_gemm_pp_kernel<true, SM_UE8M0>), grid, dim3(G_THREADS), 0, stream, p);
+  launch_kernel((fp8_gemm_pp_kernel<true, SM_UE8M0>), grid, dim3(G_THREADS), 0, stream, p);
   return check_launch(what);
 }
 
@@ -460,7 +460,7 @@ int launch_fp8_pp_rowcol(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + G_BM - 1) / G_BM;
   p.tiles_n = (p.N + G_BN - 1) / G_BN;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
-  hipLaunchKernelGGL((fp8_gemm_pp_kernel<true, SM_EPILOGUE>), grid, dim3(G_THREADS), 0, stream, p);
+  launch_kernel((fp8_gemm_pp_kernel<true, SM_EPILOGUE>), grid, dim3(G_THREADS), 0, stream, p);
   return check_launch(what);
 }
 

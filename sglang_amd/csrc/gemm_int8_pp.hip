@@ -243,7 +243,7 @@ __global__ __launch_bounds__(J_THREADS) void int8_gemm_pp_kernel(const GemmParam
 int launch_int8_pp(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + J_BM - 1) / J_BM;
   p.tiles_n = (p.N + J_BN - 1) / J_BN;
-  hipLaunchKernelGGL(int8_gemm_pp_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(J_THREADS), 0, stream, p);
+  launch_kernel(int8_gemm_pp_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(J_THREADS), 0, stream, p);
   return check_launch(what);
 }
 

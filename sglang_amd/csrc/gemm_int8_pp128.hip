@@ -226,7 +226,7 @@ int launch_int8_pp128(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + J_BM - 1) / J_BM;
   p.tiles_n = (p.N + J_BN - 1) / J_BN;
   p.splits = 1, p.kb_per_split = p.kb_total;
-  hipLaunchKernelGGL(int8_gemm_pp128_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(J_THREADS), 0, stream, p);
+  launch_kernel(int8_gemm_pp128_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(J_THREADS), 0, stream, p);
   return check_launch(what);
 }
 

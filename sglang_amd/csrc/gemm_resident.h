@@ -308,7 +308,7 @@ int launch_resident_inst(const GemmParams& p, int ranges, hipStream_t stream, co
   const int per_step = 2 * resident_half_step(AR == AR_UE8M0, KB), all = (p.M + per_step - 1) / per_step, steps = (all + ranges - 1) / ranges;
   ranges = (all + steps - 1) / steps;  // none without tokens
   const int slices = (p.N + RS_BN - 1) / RS_BN;
-  hipLaunchKernelGGL((resident_kernel<AR, KB>), dim3((unsigned)(slices * ranges)), dim3(RS_THREADS), 0, stream, p, ranges, steps);
+  launch_kernel((resident_kernel<AR, KB>), dim3((unsigned)(slices * ranges)), dim3(RS_THREADS), 0, stream, p, ranges, steps);
   return check_launch(what);
 }
 // `ranges`: workgroups that share a slice of 256 channels, each with its own tokens (the last may have fewer).

@@ -455,7 +455,7 @@ int launch_tile_inst(const GemmParams& p, unsigned grid, size_t lds, hipStream_t
       return MI355_ERR_LAUNCH;
     }
   }
-  hipLaunchKernelGGL(kfn, dim3(grid), dim3(THREADS), lds, stream, p);
+  launch_kernel(kfn, dim3(grid), dim3(THREADS), lds, stream, p);
   return check_launch(what);
 }
 
@@ -740,7 +740,7 @@ int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_giv
   if (!p.ue8m0 && !p.row_scale && route_wants_m_major_scales(IS_FP8, r) && !fp8_scales_conform(p)) {
     float* dst = static_cast<float*>(workspace);
     const int64_t ld = (p.M + 3) & ~3;
-    hipLaunchKernelGGL(relayout_scales_kernel, dim3((unsigned)((p.M + 31) / 32), (unsigned)((p.kb_total + 31) / 32)), dim3(256), 0,
+    launch_kernel(relayout_scales_kernel, dim3((unsigned)((p.M + 31) / 32), (unsigned)((p.kb_total + 31) / 32)), dim3(256), 0,
                        stream, p.sa, p.sa_sm, p.sa_sk, dst, ld, p.M, p.kb_total);
     const int rc0 = check_launch(what);
     if (rc0 != MI355_OK) return rc0;
@@ -786,7 +786,7 @@ int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_giv
   }
   if (rc != MI355_OK || p.splits == 1) return rc;
   const int64_t quads = ((int64_t)p.M * p.N + 3) / 4;
-  hipLaunchKernelGGL(splitk_reduce_kernel<IS_FP8>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, p);
+  launch_kernel(splitk_reduce_kernel<IS_FP8>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, p);
   return check_launch(what);
 }
 
@@ -1101,7 +1101,7 @@ extern "C" int mi355_fp8_blockwise_mm_ue8m0(const void* a, const void* b, const 
   const int NB = (int)((N + 127) / 128);
   float* sa_f = static_cast<float*>(workspace);
   float* sb_f = sa_f + ldm * KB;
-  hipLaunchKernelGGL(unpack_ue8m0_kernel, dim3((unsigned)(((int64_t)(M + NB) * KB + 255) / 256)), dim3(256), 0, st,
+  launch_kernel(unpack_ue8m0_kernel, dim3((unsigned)(((int64_t)(M + NB) * KB + 255) / 256)), dim3(256), 0, st,
                      static_cast<const uint32_t*>(sa_words), sa_sk, sa_f, ldm, (int)M, static_cast<const uint32_t*>(sb_words), sb_sn,
                      sb_sk, sb_f, NB, KB);
   rc = check_launch(what);

@@ -258,8 +258,8 @@ int launch_wavesplit_tile_inst(GemmParams& p, hipStream_t stream, const char* wh
   p.splits = 1;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * WST_WAVES);
   // (taller tiles are chosen for smaller weights only)
-  if (MT == 1 && streams_weight(p)) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, MT, CT, TQ_NONE, 2, MT == 1>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((wavesplit_tile_kernel<AR, MT, CT>), grid, block, 0, stream, p);
+  if (MT == 1 && streams_weight(p)) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ_NONE, 2, MT == 1>), grid, block, 0, stream, p);
+  else launch_kernel((wavesplit_tile_kernel<AR, MT, CT>), grid, block, 0, stream, p);
   return check_launch(what);
 }
 template <Arith AR, size_t... I>
@@ -285,9 +285,9 @@ int launch_wavesplit_tile_quant_inst(GemmParams& p, hipStream_t stream, const ch
   const int64_t pieces = (int64_t)p.M * p.K / 8;
   const auto launch = [&](auto streamed) {
     constexpr bool STREAM = decltype(streamed)::value;
-    if (pieces <= 2 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 2, STREAM>), grid, block, 0, stream, p);
-    else if (pieces <= 4 * 64 * WST_WAVES) hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, 4, STREAM>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((wavesplit_tile_kernel<AR, 1, CT, TQ, WS_QUANT_VECTORS, STREAM>), grid, block, 0, stream, p);
+    if (pieces <= 2 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, 1, CT, TQ, 2, STREAM>), grid, block, 0, stream, p);
+    else if (pieces <= 4 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, 1, CT, TQ, 4, STREAM>), grid, block, 0, stream, p);
+    else launch_kernel((wavesplit_tile_kernel<AR, 1, CT, TQ, WS_QUANT_VECTORS, STREAM>), grid, block, 0, stream, p);
   };
   if (streams_weight(p)) launch(std::true_type{});
   else launch(std::false_type{});

@@ -283,7 +283,7 @@ int launch_map(QuantParams& p, hipStream_t stream) {
     p.tiles_per_row = make_fastdiv((p.groups_per_row.div + UNROLL / RU - 1) / (UNROLL / RU));
     blocks = p.tiles_per_row.div * ((p.rows + PASS * RU - 1) / (PASS * RU));
   }
-  hipLaunchKernelGGL((group_quant_kernel<T, LPG, ITERS, MODE, UE8M0, FP8_OUT, UNROLL, MAP, RU>), dim3(blocks), dim3(256), 0, stream, p);
+  launch_kernel((group_quant_kernel<T, LPG, ITERS, MODE, UE8M0, FP8_OUT, UNROLL, MAP, RU>), dim3(blocks), dim3(256), 0, stream, p);
   return check_launch("mi355_group_quant_8bit");
 }
 

@@ -175,7 +175,7 @@ extern "C" int mi355_probe_reciprocal(int exponent, void* mismatches, void* stre
   clear_error();
   MI355_REQUIRE(exponent >= -100 && exponent <= 120, MI355_ERR_INVALID_ARGUMENT, "%s: exponent -100..120", what);
   MI355_REQUIRE(mismatches, MI355_ERR_INVALID_ARGUMENT, "%s: null pointer", what);
-  hipLaunchKernelGGL(reciprocal_kernel, dim3((1u << 23) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), exponent,
+  launch_kernel(reciprocal_kernel, dim3((1u << 23) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), exponent,
                      static_cast<unsigned long long*>(mismatches));
   return check_launch(what);
 }
@@ -192,10 +192,10 @@ extern "C" int mi355_probe_fp8_mfma_stream(int mode, int workgroups, int iters, 
   const uint8_t* pb = static_cast<const uint8_t*>(b);
   float* po = static_cast<float*>(out);
   switch (mode) {
-    case 0: hipLaunchKernelGGL(mfma_stream_kernel<0>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
-    case 1: hipLaunchKernelGGL(mfma_stream_kernel<1>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
-    case 2: hipLaunchKernelGGL(mfma_stream_kernel<2>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
-    default: hipLaunchKernelGGL(mfma_stream_kernel<3>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
+    case 0: launch_kernel(mfma_stream_kernel<0>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
+    case 1: launch_kernel(mfma_stream_kernel<1>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
+    case 2: launch_kernel(mfma_stream_kernel<2>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
+    default: launch_kernel(mfma_stream_kernel<3>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters); break;
   }
   return check_launch(what);
 }
@@ -211,7 +211,7 @@ extern "C" int mi355_probe_int8_mfma_stream(int mode, int workgroups, int iters,
   const uint8_t* pa = static_cast<const uint8_t*>(a);
   const uint8_t* pb = static_cast<const uint8_t*>(b);
   int* po = static_cast<int*>(out);
-  if (mode == 0) hipLaunchKernelGGL(int8_mfma_stream_kernel<0>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters);
-  else hipLaunchKernelGGL(int8_mfma_stream_kernel<1>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters);
+  if (mode == 0) launch_kernel(int8_mfma_stream_kernel<0>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters);
+  else launch_kernel(int8_mfma_stream_kernel<1>, dim3(workgroups), dim3(512), 0, st, pa, pb, po, iters);
   return check_launch(what);
 }

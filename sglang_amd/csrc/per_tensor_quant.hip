@@ -156,9 +156,9 @@ template <int DT>
 void launch_static(const void* x, uint8_t* q, float* scale, int64_t n, float* scale_rows, int64_t rows, hipStream_t st) {
   const int64_t nvec = n / ((DT == MI355_F32) ? 4 : 8);
   if (nvec <= 256 * 2048)
-    hipLaunchKernelGGL((per_tensor_quant_kernel<DT, 256, 1, false>), dim3((unsigned)std::max<int64_t>(1, (nvec + 255) / 256)), dim3(256), 0, st, x, q, scale, n, scale_rows, rows);
+    launch_kernel((per_tensor_quant_kernel<DT, 256, 1, false>), dim3((unsigned)std::max<int64_t>(1, (nvec + 255) / 256)), dim3(256), 0, st, x, q, scale, n, scale_rows, rows);
   else
-    hipLaunchKernelGGL((per_tensor_quant_kernel<DT, 256, 4, true>), dim3((unsigned)std::min<int64_t>((nvec + 1023) / 1024, 1 << 20)), dim3(256), 0, st, x, q, scale, n, scale_rows, rows);
+    launch_kernel((per_tensor_quant_kernel<DT, 256, 4, true>), dim3((unsigned)std::min<int64_t>((nvec + 1023) / 1024, 1 << 20)), dim3(256), 0, st, x, q, scale, n, scale_rows, rows);
 }
 
 template <int DT>
@@ -168,8 +168,8 @@ void launch_both(const void* x, uint8_t* q, float* scale, int64_t n, bool is_sta
   if (is_static) return launch_static<DT>(x, q, scale, n, scale_rows, rows, st);
   const int64_t per_wg = (int64_t)ABSMAX_THREADS * ABSMAX_UNROLL * ((DT == MI355_F32) ? 4 : 8);
   const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + per_wg - 1) / per_wg, ABSMAX_MAX_WGS));
-  hipLaunchKernelGGL(per_tensor_absmax_kernel<DT>, dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, scale, n);
-  hipLaunchKernelGGL((per_tensor_quant_kernel<DT, ABSMAX_THREADS, ABSMAX_UNROLL, true>), dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, q, scale, n, scale_rows, rows);
+  launch_kernel(per_tensor_absmax_kernel<DT>, dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, scale, n);
+  launch_kernel((per_tensor_quant_kernel<DT, ABSMAX_THREADS, ABSMAX_UNROLL, true>), dim3(grid), dim3(ABSMAX_THREADS), 0, st, x, q, scale, n, scale_rows, rows);
 }
 
 }  // namespace

@@ -303,8 +303,8 @@ int per_token_quant(const char* what, const void* x, int x_dtype, void* q, float
     if (x_dtype != MI355_F32 && K <= 8 * 512 * 6 && !(K <= 4096 && (M > 1024 || K <= 512))) {
 #define MI355_ROWS(T, NV)                                                                                                              \
   {                                                                                                                                    \
-    if (x_dtype == MI355_BF16) hipLaunchKernelGGL((per_token_quant_row_kernel<MI355_BF16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K); \
-    else hipLaunchKernelGGL((per_token_quant_row_kernel<MI355_F16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K);  \
+    if (x_dtype == MI355_BF16) launch_kernel((per_token_quant_row_kernel<MI355_BF16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K); \
+    else launch_kernel((per_token_quant_row_kernel<MI355_F16, FP8_OUT, T, NV>), dim3((unsigned)M), dim3(T), 0, st, x, qq, s, K);  \
   }
       const bool few = M <= 640;
       if (K <= 2048) {
@@ -326,7 +326,7 @@ int per_token_quant(const char* what, const void* x, int x_dtype, void* q, float
     const dim3 grid((unsigned)((M + 3) / 4));
     const int nv = (int)((K / 8 + 63) / 64);
 #define MI355_WAVE_ROWS(DT, NV) \
-  hipLaunchKernelGGL((per_token_quant_wave_kernel<DT, FP8_OUT, NV, SUM>), grid, dim3(256), 0, st, x, qq, s, M, K, x_sum)
+  launch_kernel((per_token_quant_wave_kernel<DT, FP8_OUT, NV, SUM>), grid, dim3(256), 0, st, x, qq, s, M, K, x_sum)
     if (x_dtype == MI355_BF16) {
       if (nv <= 4) MI355_WAVE_ROWS(MI355_BF16, 4);
       else if (nv <= 8) MI355_WAVE_ROWS(MI355_BF16, 8);
@@ -341,13 +341,13 @@ int per_token_quant(const char* what, const void* x, int x_dtype, void* q, float
   }
   switch (x_dtype) {
     case MI355_F32:
-      hipLaunchKernelGGL((per_token_quant_kernel<MI355_F32, FP8_OUT, ROW_GROUP, DIVIDE, SUM>), dim3((unsigned)M), dim3(256), 0, st, x, qq, s, K, eps, x_sum);
+      launch_kernel((per_token_quant_kernel<MI355_F32, FP8_OUT, ROW_GROUP, DIVIDE, SUM>), dim3((unsigned)M), dim3(256), 0, st, x, qq, s, K, eps, x_sum);
       break;
     case MI355_F16:
-      hipLaunchKernelGGL((per_token_quant_kernel<MI355_F16, FP8_OUT, ROW_GROUP, DIVIDE, SUM>), dim3((unsigned)M), dim3(256), 0, st, x, qq, s, K, eps, x_sum);
+      launch_kernel((per_token_quant_kernel<MI355_F16, FP8_OUT, ROW_GROUP, DIVIDE, SUM>), dim3((unsigned)M), dim3(256), 0, st, x, qq, s, K, eps, x_sum);
       break;
     default:
-      hipLaunchKernelGGL((per_token_quant_kernel<MI355_BF16, FP8_OUT, ROW_GROUP, DIVIDE, SUM>), dim3((unsigned)M), dim3(256), 0, st, x, qq, s, K, eps, x_sum);
+      launch_kernel((per_token_quant_kernel<MI355_BF16, FP8_OUT, ROW_GROUP, DIVIDE, SUM>), dim3((unsigned)M), dim3(256), 0, st, x, qq, s, K, eps, x_sum);
   }
   return check_launch(what);
 }

@@ -311,13 +311,13 @@ int silu_mul_group_quant(const char* what, const void* x, int x_dtype, void* q, 
     const bool bf16 = x_dtype == MI355_BF16;
     if (bf16 && groups <= (masked_m ? SQ_NEAR_GROUPS_MASKED : SQ_NEAR_GROUPS)) {
       const dim3 grid((unsigned)std::min<int64_t>((groups + 15) / 16, SQ_NEAR_WORKGROUPS));
-      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_BF16, ST_NEAR>), grid, dim3(256), 0, st, p);
+      launch_kernel((silu_mul_quant_kernel<MI355_BF16, ST_NEAR>), grid, dim3(256), 0, st, p);
     } else if (bf16) {
-      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_BF16, ST_WHOLE>), dim3(256), dim3(1024), 0, st, p);
+      launch_kernel((silu_mul_quant_kernel<MI355_BF16, ST_WHOLE>), dim3(256), dim3(1024), 0, st, p);
     } else if (groups <= (masked_m ? SQ_IN_PLACE_GROUPS_MASKED : SQ_IN_PLACE_GROUPS)) {
-      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_F16, ST_IN_PLACE>), dim3((unsigned)((groups + 15) / 16)), dim3(256), 0, st, p);
+      launch_kernel((silu_mul_quant_kernel<MI355_F16, ST_IN_PLACE>), dim3((unsigned)((groups + 15) / 16)), dim3(256), 0, st, p);
     } else {
-      hipLaunchKernelGGL((silu_mul_quant_kernel<MI355_F16, ST_WHOLE>), dim3(256), dim3(1024), 0, st, p);
+      launch_kernel((silu_mul_quant_kernel<MI355_F16, ST_WHOLE>), dim3(256), dim3(1024), 0, st, p);
     }
     const int rc = check_launch(what);
     if (rc != MI355_OK) return rc;
