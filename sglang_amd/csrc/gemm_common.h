@@ -61,7 +61,7 @@ __device__ __forceinline__ int in_vgpr(int x) {
 // ---- 1 x 128 group quantization inside a GEMM kernel (the one-call linear at decode sizes): 16 lanes hold a group, 8
 // elements each, with the arithmetic of the group quantizer's reference path (amax floored at 1e-10, s = amax / 448,
 // q = e4m3fn(clamp(x / s)), group_quant.hip).  A few waves do this for a whole workgroup before (or beside) its K loop, bound by
-// their vector instructions: 66 for the eight elements of a lane.  With compiler-made divisions, the type looked at per element
+// their vector instructions: 58 for the eight elements of a lane.  With compiler-made divisions, the type looked at per element
 // and two refinement steps per quotient it was 128; us, before / now: 7168 -> 384 at 4 tokens 8.2 / 7.5, 4864 -> 704 at 8 9.8 / 8.3,
 // INT8 3584 -> 1536 at 9 9.9 / 7.9, per-token FP8 2048 -> 2048 at 8 7.3 / 6.4.
 template <bool BF16>
@@ -123,7 +123,7 @@ __device__ __forceinline__ u32x2 quantize_group_lane(const u32x4& raw, bool by_r
     }
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) t[e] = fminf(fmaxf(t[e], -448.0f), 448.0f);
+  for (int e = 0; e < 8; ++e) t[e] = __builtin_amdgcn_fmed3f(t[e], -448.0f, 448.0f);  // (NaN: -448, as the quantizer kernel has it)
   int c0 = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
   c0 = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c0, true);
   int c1 = __builtin_amdgcn_cvt_pk_fp8_f32(t[4], t[5], 0, false);
@@ -554,12 +554,13 @@ int launch_fp8_wavesplit_tile(GemmParams& p, int bm, int bn, hipStream_t stream,
 int launch_fp8_wavesplit_tile_ue8m0(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
 int launch_fp8_wavesplit_tile_unit(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
 int launch_int8_wavesplit_tile(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
-// The same for 16-token tiles with a quantizer for the tokens inside (p.x16 / p.ldx / p.x_dtype, p.x_by_reciprocal; p.a and p.sa
-// are not read): per 1 x 128 group, or per token for the unit-scale FP8 and the INT8 kernel.  K % 128 == 0, few tokens.
-int launch_fp8_wavesplit_tile_quant(GemmParams& p, int bn, hipStream_t stream, const char* what);
-int launch_fp8_wavesplit_tile_ue8m0_quant(GemmParams& p, int bn, hipStream_t stream, const char* what);
-int launch_fp8_wavesplit_tile_unit_quant(GemmParams& p, int bn, hipStream_t stream, const char* what);
-int launch_int8_wavesplit_tile_quant(GemmParams& p, int bn, hipStream_t stream, const char* what);
+// The same with a quantizer for the tokens inside (p.x16 / p.ldx / p.x_dtype, p.x_by_reciprocal; p.a and p.sa are not read): per 1 x 128
+// group, or per token for the unit-scale FP8 and the INT8 kernel.  K % 128 == 0, few values in a tile's tokens.
+constexpr TileSize WAVESPLIT_QUANT_TILES[] = {{16, 16}, {16, 32}, {16, 64}};
+int launch_fp8_wavesplit_tile_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
+int launch_fp8_wavesplit_tile_ue8m0_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
+int launch_fp8_wavesplit_tile_unit_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
+int launch_int8_wavesplit_tile_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
 
 // Short K, many tokens: the weight in registers (gemm_resident.h).  `ranges` workgroups share 256 channels, each with its own tokens.
 // K of 2 .. RESIDENT_MAX_KBLOCKS whole blocks, 16-byte aligned rows, row offsets below 4 GiB, conforming token scales, and an output that

@@ -198,7 +198,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu((CT == 2
     for (int j = 0; j < KBW; ++j) request(j, j);
   } else {
     // the raw values are requested first, then the first weight blocks, so that these are in flight while the tokens are quantized
-    quantize_tokens<IS_FP8, UE8M0, TQ, NV, 64 * W>(p, codes, token_scale, row_max, [&] {
+    quantize_tokens<IS_FP8, UE8M0, TQ, NV, 64 * W, 16>(p, 0, p.M, codes, token_scale, row_max, [&] {
 #pragma unroll
       for (int j = 0; j < KBW; ++j) request(j, j);
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KBW * LOADS) : "memory");
@@ -336,7 +336,7 @@ int launch_fp8_wavesplit_ue8m0(GemmParams& p, hipStream_t stream, const char* wh
 // Unquantized tokens (p.x16, p.ldx, p.x_dtype; 16-byte aligned rows): quantized in the kernel.
 bool wavesplit_quant_fits(int64_t M, int64_t K) { return M * K <= (int64_t)wavesplit_shape(K).waves * 64 * WS_QUANT_VECTORS * 8; }
 int launch_wavesplit_quant(GemmParams& p, WavesplitQuant kind, hipStream_t stream, const char* what) {
-  if (p.x16 == nullptr || p.M > 16 || !wavesplit_quant_fits(p.M, p.K)) {
+  if (p.x16 == nullptr || p.ldx != p.K || p.M > 16 || !wavesplit_quant_fits(p.M, p.K)) {
     set_error("%s: the fused quantizer of the wave-split kernel takes few unquantized tokens", what);
     return MI355_ERR_UNSUPPORTED;
   }

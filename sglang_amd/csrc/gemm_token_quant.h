@@ -1,5 +1,5 @@
-// Tokens quantized inside a GEMM kernel at decode sizes: the whole workgroup quantizes ALL of the M x K tokens into LDS before
-// its K loop, with the arithmetic of the quantizer kernels, and takes its token fragments from there.
+// Tokens quantized inside a GEMM kernel: the whole workgroup quantizes all K values of its tile's tokens into LDS before its K
+// loop, with the arithmetic of the quantizer kernels, and takes its token fragments from there.
 #pragma once
 
 #include "gemm_common.h"
@@ -30,7 +30,7 @@ __device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, float mul) {  //
     if constexpr (F8) {
       float t[4];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) t[b] = fmaxf(fminf(f[4 * j + b] * mul, 448.0f), -448.0f);
+      for (int b = 0; b < 4; ++b) t[b] = -__builtin_amdgcn_fmed3f(-(f[4 * j + b] * mul), -448.0f, 448.0f);  // (NaN: 448, as the quantizer kernel has it)
       int c = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
       out[j] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c, true);
     } else {
@@ -57,34 +57,35 @@ __device__ __forceinline__ float amax8(const u32x4& raw) {
   return m;
 }
 
-// Piece c (16 bytes of input, 8 values) of the M x K / 8 goes to thread c % NT; 16 consecutive pieces are a group, in the 16 lanes
-// of a DPP row.  Codes go to codes[row * (K + 16) + k] (rows 16 bytes longer than K, so that a fragment's rows do not share banks),
-// scales to token_scale (one per token, or per token and K block: row * kb_total + kb; exponents for UE8M0).  `request` is called
-// behind the loads of the raw values: it requests the first weight blocks and waits until only those are outstanding.  Ends with
-// a barrier that does not wait for them.
-template <bool IS_FP8, bool UE8M0, TokenQuant TQ, int NV, int NT, class Request>
-__device__ __forceinline__ void quantize_tokens(const GemmParams& p, uint8_t* codes, float* token_scale, float* row_max, Request request) {
-  const int lane = threadIdx.x & 63, code_pitch = p.K + 16;
+// The tokens m0 .. m0 + rows - 1, at most BM, whose rows lie one behind the other.  Piece c (16 bytes of input, 8 values) of them goes to
+// thread c % NT; 16 consecutive pieces are a group, in the 16 lanes of a DPP row.  Codes go to codes[row * (K + 16) + k] (rows 16 bytes
+// longer than K, so that a fragment's rows do not share banks), scales to token_scale (one per token, or per token and K block: row *
+// kb_total + kb, which is c / 16; exponents for UE8M0).  `request` is called behind the loads of the raw values: it requests the first weight
+// blocks and waits until only those are outstanding.  Ends with a barrier that does not wait for them.
+// Bound by its vector instructions, about 70 a piece and lane: flat addresses, one multiplication for the row, one median for the clamp.  With
+// row and column of a piece found by a loop and clamps behind a quieting maximum it was 130; whole linears, us, before / now: block FP8
+// 1152 -> 256 at 16 tokens 6.1 / 4.7, 1536 -> 24576 at 8 11.9 / 10.8; packed exponents 1280 -> 1920 at 15 5.8 / 4.8; INT8 1408 -> 704 at 12
+// 5.8 / 4.9; per-token FP8 1152 -> 17280 at 10 11.8 / 10.75.
+template <bool IS_FP8, bool UE8M0, TokenQuant TQ, int NV, int NT, int BM, class Request>
+__device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int rows, uint8_t* codes, float* token_scale, float* row_max, Request request) {
+  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int per_row = p.K >> 3, total = p.M * per_row;
-  const uint16_t* x = reinterpret_cast<const uint16_t*>(p.x16);
+  const int total = __builtin_amdgcn_readfirstlane(rows * (p.K >> 3));
+  const uint8_t* x = reinterpret_cast<const uint8_t*>(p.x16) + (int64_t)m0 * p.K * 2;
+  static_assert(NV * NT / 16 <= 512, "row_of: groups below 2^9 and a 20-bit inverse");
+  // the row of piece c, exact for c / 16 * kb_total < 2^20; any row past the last one for pieces past the end
+  const uint32_t inverse = __builtin_amdgcn_readfirstlane(((1u << 20) + (uint32_t)p.kb_total - 1u) / (uint32_t)p.kb_total);
+  auto piece = [&](int i) { return (int)threadIdx.x + i * NT; };
+  auto row_of = [&](int i) { return (int)(__umul24((uint32_t)piece(i) >> 4, inverse) >> 20); };
   // (NV pieces per thread, all of them always requested: a load under a condition could leave the compiler a copy to make
   // while it is in flight; pieces past the end repeat the last one and are dropped)
   u32x4 raw[NV];
-  int at[NV];  // the piece's row in the high half, its place in the row in the low one
-  auto row_of = [&](int i) { return at[i] >> 16; };
-  auto col_of = [&](int i) { return at[i] & 0xffff; };
-  int r = 0, c = threadIdx.x;
+  asm volatile("" : "+s"(x));
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    while (c >= per_row && r < p.M) c -= per_row, ++r;
-    at[i] = (r << 16) | (c & 0xffff);
-    const uint16_t* src = x + (int64_t)min(r, p.M - 1) * p.ldx + (r < p.M ? c : per_row - 1) * 8;
-    asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(raw[i]) : "v"(src) : "memory");
-    c += NT;
-  }
+  for (int i = 0; i < NV; ++i)
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(raw[i]) : "v"((uint32_t)min(piece(i), total - 1) * 16u), "s"(x) : "memory");
   if constexpr (TQ == TQ_ROW) {
-    if (threadIdx.x < 16) reinterpret_cast<uint32_t*>(row_max)[threadIdx.x] = __float_as_uint(IS_FP8 ? 0.f : 1e-10f);
+    if (threadIdx.x < BM) reinterpret_cast<uint32_t*>(row_max)[threadIdx.x] = __float_as_uint(IS_FP8 ? 0.f : 1e-10f);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
   request();
@@ -102,12 +103,12 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, uint8_t* co
       for (int i = 0; i < NV; ++i) {
         if (i * NT + wave * 64 < total) {
           const float m = row16_max(amax8<BF16>(raw[i]));
-          if ((lane & 15) == 0 && row_of(i) < p.M) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
+          if ((lane & 15) == 0 && piece(i) < total) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
         }
       }
     });
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (threadIdx.x < 16) {  // the row's scale, and the factor its values are multiplied with in the place of its maximum
+    if (threadIdx.x < BM) {  // the row's scale, and the factor its values are multiplied with in the place of its maximum
       const float m = row_max[threadIdx.x], sc = IS_FP8 ? m / 448.0f : m / 127.0f;
       token_scale[threadIdx.x] = sc;
       row_max[threadIdx.x] = !IS_FP8 ? 127.0f / m : sc == 0.f ? 0.f : 1.0f / sc;
@@ -121,21 +122,24 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, uint8_t* co
       __builtin_amdgcn_sched_barrier(0);  // one piece's arithmetic at a time: no register may be spilled while loads are in flight
       if (i * NT + wave * 64 < total) {
         u32x2 q8;
+        const int row = row_of(i);
         if constexpr (TQ == TQ_ROW) {
-          q8 = codes_of_row<IS_FP8, BF16>(raw[i], row_max[min(row_of(i), 15)]);
-        } else if constexpr (UE8M0) {
-          // q = x * 2^-e with e = ceil(log2(max(amax, 1e-10) / 448)): group_quant.hip, MUL with packed exponents
-          const float m = row16_max(fmaxf(amax8<BF16>(raw[i]), 1e-10f));
-          const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
-          const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
-          q8 = codes_of_row<true, BF16>(raw[i], __uint_as_float((uint32_t)(127 - e) << 23));
-          if ((lane & 15) == 0 && row_of(i) < p.M) reinterpret_cast<uint32_t*>(token_scale)[row_of(i) * p.kb_total + (col_of(i) >> 4)] = (uint32_t)(e + 127);
+          q8 = codes_of_row<IS_FP8, BF16>(raw[i], row_max[min(row, BM - 1)]);
         } else {
           float sc;
-          q8 = quantize_group_lane<BF16>(raw[i], p.x_by_reciprocal != 0, sc);
-          if ((lane & 15) == 0 && row_of(i) < p.M) token_scale[row_of(i) * p.kb_total + (col_of(i) >> 4)] = sc;
+          if constexpr (UE8M0) {
+            // q = x * 2^-e with e = ceil(log2(max(amax, 1e-10) / 448)): group_quant.hip, MUL with packed exponents
+            const float m = row16_max(fmaxf(amax8<BF16>(raw[i]), 1e-10f));
+            const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
+            const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
+            q8 = codes_of_row<true, BF16>(raw[i], __uint_as_float((uint32_t)(127 - e) << 23));
+            sc = __uint_as_float((uint32_t)(e + 127));
+          } else {
+            q8 = quantize_group_lane<BF16>(raw[i], p.x_by_reciprocal != 0, sc);
+          }
+          if ((lane & 15) == 0 && piece(i) < total) token_scale[piece(i) >> 4] = sc;
         }
-        if (row_of(i) < p.M) *reinterpret_cast<u32x2*>(codes + row_of(i) * code_pitch + col_of(i) * 8) = q8;
+        if (piece(i) < total) *reinterpret_cast<u32x2*>(codes + piece(i) * 8 + row * 16) = q8;
       }
     }
   });

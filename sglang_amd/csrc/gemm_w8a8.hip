@@ -1332,10 +1332,10 @@ int run_tile_quant(GemmParams& p, WavesplitQuant kind, const Route& run, const v
   p.kb_total = p.K / KSTEP;
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (kind) {
-    case WavesplitQuant::BLOCK_F32: return launch_fp8_wavesplit_tile_quant(p, run.bn, st, what);
-    case WavesplitQuant::BLOCK_UE8M0: return launch_fp8_wavesplit_tile_ue8m0_quant(p, run.bn, st, what);
-    case WavesplitQuant::TOKEN_FP8: return launch_fp8_wavesplit_tile_unit_quant(p, run.bn, st, what);
-    default: return launch_int8_wavesplit_tile_quant(p, run.bn, st, what);
+    case WavesplitQuant::BLOCK_F32: return launch_fp8_wavesplit_tile_quant(p, run.bm, run.bn, st, what);
+    case WavesplitQuant::BLOCK_UE8M0: return launch_fp8_wavesplit_tile_ue8m0_quant(p, run.bm, run.bn, st, what);
+    case WavesplitQuant::TOKEN_FP8: return launch_fp8_wavesplit_tile_unit_quant(p, run.bm, run.bn, st, what);
+    default: return launch_int8_wavesplit_tile_quant(p, run.bm, run.bn, st, what);
   }
 }
 int run_wavesplit_quant(GemmParams& p, WavesplitQuant kind, const void* x, int x_dtype, void* stream, const char* what) {

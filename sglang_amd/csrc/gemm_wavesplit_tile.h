@@ -30,15 +30,16 @@ namespace {
 // Eight waves: with four, K = 7168 takes twice the steps; sixteen would halve the slots.
 constexpr int WST_WAVES = 8;
 
-// TQ: the tokens arrive unquantized (MT = 1 only); their codes take WST_CODE_BYTES of the LDS and the slots hold weight rows only.
-constexpr int WST_CODE_BYTES = 64 * WST_WAVES * WS_QUANT_VECTORS * 8 + 16 * 16;  // M (K + 16) for as many pieces as there may be
-constexpr int WST_SCALE_BYTES = WST_CODE_BYTES / KSTEP * 4;
+// TQ: the tokens arrive unquantized; their codes take code_bytes of the LDS and the slots hold weight rows only.
+constexpr int WST_QUANT_VALUES = 64 * WST_WAVES * WS_QUANT_VECTORS * 8;  // of a tile's tokens: as many pieces as there may be
+constexpr int WST_SCALE_BYTES = (WST_QUANT_VALUES / KSTEP + 2) * 4;
+constexpr int wst_code_bytes(int bm) { return WST_QUANT_VALUES + bm * 16; }  // rows are 16 bytes longer than K
 template <Arith AR, int MT, int CT, TokenQuant TQ>
 struct WavesplitTile {
   static constexpr bool SCALED = (AR == AR_F32 || AR == AR_UE8M0) && TQ == TQ_NONE;  // token scales in the slots
   static constexpr int BM = 16 * MT, BN = 16 * CT, TOKENS = TQ == TQ_NONE ? BM : 0;
   static constexpr int SLOT_BYTES = (TOKENS + BN) * KSTEP + (SCALED ? BM * 4 : 0);
-  static constexpr int RING_LIMIT = 160 * 1024 - (TQ == TQ_NONE ? 0 : WST_CODE_BYTES + WST_SCALE_BYTES + 64);
+  static constexpr int RING_LIMIT = 160 * 1024 - (TQ == TQ_NONE ? 0 : wst_code_bytes(BM) + WST_SCALE_BYTES + BM * 4);
   static constexpr int FIT = RING_LIMIT / (WST_WAVES * SLOT_BYTES), R = FIT > 4 ? 4 : FIT;
   static_assert(R >= 1, "a slot per wave");
   static constexpr int ROW_LOADS = (TOKENS + BN) / 8, LOADS = ROW_LOADS + (SCALED ? 1 : 0);
@@ -60,15 +61,16 @@ __device__ __forceinline__ void wait_blocks(int blocks) {
 template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2, bool STREAM = false>
 __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void wavesplit_tile_kernel(const GemmParams p) {
   using T = WavesplitTile<AR, MT, CT, TQ>;
-  static_assert(TQ == TQ_NONE || MT == 1, "the fused quantizer is for 16 tokens at most");
   constexpr int R = T::R, LOADS = T::LOADS, BM = T::BM, BN = T::BN, W = WST_WAVES;
   using AccT = typename std::conditional<AR == AR_INT8, int, float>::type;
   typedef AccT acc4 __attribute__((ext_vector_type(4)));
+  // the slots and, with unquantized tokens, their codes; the partial tiles lie over both
   constexpr int RING_BYTES = W * R * T::SLOT_BYTES, RED_BYTES = W * MT * CT * 64 * 16;
-  __shared__ __attribute__((aligned(1024))) uint8_t ring[RING_BYTES > RED_BYTES ? RING_BYTES : RED_BYTES];
-  __shared__ __attribute__((aligned(16))) uint8_t codes[TQ == TQ_NONE ? 16 : WST_CODE_BYTES];
+  constexpr int LOOP_BYTES = RING_BYTES + (TQ == TQ_NONE ? 0 : wst_code_bytes(BM));
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[LOOP_BYTES > RED_BYTES ? LOOP_BYTES : RED_BYTES];
+  uint8_t* const codes = ring + RING_BYTES;
   __shared__ float token_scale[TQ == TQ_NONE ? 1 : WST_SCALE_BYTES / 4];
-  __shared__ float row_max[TQ == TQ_ROW ? 16 : 1];
+  __shared__ float row_max[TQ == TQ_ROW ? BM : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, q = lane >> 4;
@@ -77,6 +79,7 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
   const int per_xcd = (int)gridDim.x >> 3;
   if (bid < per_xcd * 8) bid = (bid & 7) * per_xcd + (bid >> 3);
   const int m0 = (bid % p.tiles_m) * BM, n0 = (bid / p.tiles_m) * BN;
+  const int rows = min(p.M - m0, BM);  // tokens of the tile
 
   // loader: a load fills 8 rows of a slot, lane = row lane >> 3, 16-byte chunk lane & 7; chunks land swizzled by (row & 7)
   uint32_t goff[T::ROW_LOADS];
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
   if constexpr (TQ == TQ_NONE) {
     request_first();
   } else {
-    quantize_tokens<AR != AR_INT8, AR == AR_UE8M0, TQ, NV, 64 * W>(p, codes, token_scale, row_max, [&] {
+    quantize_tokens<AR != AR_INT8, AR == AR_UE8M0, TQ, NV, 64 * W, BM>(p, m0, rows, codes, token_scale, row_max, [&] {
       request_first();
       wait_blocks<LOADS>(min(blocks, R));
     });
@@ -151,9 +154,10 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
       if constexpr (TQ == TQ_NONE) {
         tf[t].lo = lds16(st + lo, t * 2048), tf[t].hi = lds16(st + hi, t * 2048);
       } else {
-        const uint8_t* src = codes + min(l16, p.M - 1) * (p.K + 16) + kb * KSTEP + q * 16;
+        const int row = min(16 * t + l16, rows - 1);  // (past the last token: results that are not stored)
+        const uint8_t* src = codes + row * (p.K + 16) + kb * KSTEP + q * 16;
         tf[t].lo = *reinterpret_cast<const u32x4*>(src), tf[t].hi = *reinterpret_cast<const u32x4*>(src + 64);
-        if constexpr (TQ == TQ_GROUP) ts[t] = token_scale[min(l16, p.M - 1) * p.kb_total + kb];
+        if constexpr (TQ == TQ_GROUP) ts[t] = token_scale[row * p.kb_total + kb];
       }
       if constexpr (T::SCALED) ts[t] = lds_f32(st + (T::ROW_LOADS * 1024) + l16 * 4, t * 64);
     }
@@ -243,10 +247,10 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
     float r[4];
     if constexpr (AR == AR_INT8) {
       const int a4[4] = {s[0], s[1], s[2], s[3]};
-      int8_apply_terms(p, ct, TQ == TQ_NONE ? p.sa[m] : token_scale[m], a4, r);
+      int8_apply_terms(p, ct, TQ == TQ_NONE ? p.sa[m] : token_scale[m - m0], a4, r);
     } else {
       r[0] = s[0], r[1] = s[1], r[2] = s[2], r[3] = s[3];
-      fp8_apply_terms(p, ct, TQ == TQ_ROW ? token_scale[m] : p.row_scale ? p.row_scale[m] : 1.f, r);
+      fp8_apply_terms(p, ct, TQ == TQ_ROW ? token_scale[m - m0] : p.row_scale ? p.row_scale[m] : 1.f, r);
     }
     store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, min(4, p.N - n), vec_ok);
   }
@@ -277,32 +281,39 @@ int launch_wavesplit_tile_of(GemmParams& p, int bm, int bn, hipStream_t stream, 
 }
 
 // The same with the tokens quantized in the kernel (p.x16 / p.ldx / p.x_dtype; p.a and p.sa are not read).
-template <Arith AR, TokenQuant TQ, int CT>
+template <Arith AR, TokenQuant TQ, int MT, int CT>
 int launch_wavesplit_tile_quant_inst(GemmParams& p, hipStream_t stream, const char* what) {
-  p.tiles_m = 1, p.tiles_n = (p.N + 16 * CT - 1) / (16 * CT);
+  p.tiles_m = (p.M + 16 * MT - 1) / (16 * MT), p.tiles_n = (p.N + 16 * CT - 1) / (16 * CT);
   p.splits = 1;
-  const dim3 grid((unsigned)p.tiles_n), block(64 * WST_WAVES);
-  const int64_t pieces = (int64_t)p.M * p.K / 8;
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * WST_WAVES);
+  const int64_t pieces = (int64_t)min(p.M, 16 * MT) * p.K / 8;
   const auto launch = [&](auto streamed) {
     constexpr bool STREAM = decltype(streamed)::value;
-    if (pieces <= 2 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, 1, CT, TQ, 2, STREAM>), grid, block, 0, stream, p);
-    else if (pieces <= 4 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, 1, CT, TQ, 4, STREAM>), grid, block, 0, stream, p);
-    else launch_kernel((wavesplit_tile_kernel<AR, 1, CT, TQ, WS_QUANT_VECTORS, STREAM>), grid, block, 0, stream, p);
+    if (MT == 1 && pieces <= 2 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, MT == 1 ? 2 : 5, STREAM>), grid, block, 0, stream, p);
+    else if (pieces <= (MT == 1 ? 4 : 5) * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, MT == 1 ? 4 : 5, STREAM>), grid, block, 0, stream, p);
+    else launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, WS_QUANT_VECTORS, STREAM>), grid, block, 0, stream, p);
   };
-  if (streams_weight(p)) launch(std::true_type{});
+  if (MT == 1 && streams_weight(p)) launch(std::integral_constant<bool, MT == 1>{});
   else launch(std::false_type{});
   return check_launch(what);
 }
+template <Arith AR, TokenQuant TQ, size_t... I>
+int launch_wavesplit_tile_quant_of(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what, std::index_sequence<I...>) {
+  int rc = MI355_ERR_UNSUPPORTED;
+  bool found = false;
+  ((found = found || (bm == WAVESPLIT_QUANT_TILES[I].bm && bn == WAVESPLIT_QUANT_TILES[I].bn &&
+                      (rc = launch_wavesplit_tile_quant_inst<AR, TQ, WAVESPLIT_QUANT_TILES[I].bm / 16, WAVESPLIT_QUANT_TILES[I].bn / 16>(p, stream, what), true))), ...);
+  if (!found) set_error("%s: no wave-split %d x %d tile that quantizes is built", what, bm, bn);
+  return rc;
+}
 template <Arith AR, TokenQuant TQ>
-int launch_wavesplit_tile_quant(GemmParams& p, int bn, hipStream_t stream, const char* what) {
-  if (p.x16 == nullptr || p.M > 16 || p.K % KSTEP != 0 || (int64_t)p.M * p.K > 64 * WST_WAVES * WS_QUANT_VECTORS * 8) {
+int launch_wavesplit_tile_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what) {
+  if (p.x16 == nullptr || p.ldx != p.K || p.K % KSTEP != 0 || (int64_t)min(p.M, bm) * p.K > WST_QUANT_VALUES) {
     set_error("%s: the fused quantizer of the wave-split tile takes few unquantized tokens", what);
     return MI355_ERR_UNSUPPORTED;
   }
   if (TQ == TQ_ROW && AR != AR_INT8) p.row_scale = p.col_scale;  // (there is one: it lies in LDS)
-  return bn == 16 ? launch_wavesplit_tile_quant_inst<AR, TQ, 1>(p, stream, what)
-       : bn == 32 ? launch_wavesplit_tile_quant_inst<AR, TQ, 2>(p, stream, what)
-                  : launch_wavesplit_tile_quant_inst<AR, TQ, 4>(p, stream, what);
+  return launch_wavesplit_tile_quant_of<AR, TQ>(p, bm, bn, stream, what, std::make_index_sequence<sizeof(WAVESPLIT_QUANT_TILES) / sizeof(WAVESPLIT_QUANT_TILES[0])>{});
 }
 
 }  // namespace
