@@ -395,7 +395,9 @@ int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const flo
  *          is no quantizer launch where that is the faster way: the GEMM kernel quantizes the tokens itself (the wave-split
  *          kernel, the wave-split tile and the streaming kernel in their prologues, the mid-M kernel by producer waves), with
  *          the same arithmetic; the result is bit-identical to the two-step sequence where the GEMM alone takes the same
- *          kernel, that is where mi355_fp8_block_linear_plan without its last key equals mi355_fp8_blockwise_mm_plan.
+ *          kernel, that is where mi355_fp8_block_linear_plan without its last key equals mi355_fp8_blockwise_mm_plan, and
+ *          wherever both name the wave-split tile: tiles of any size add the same products in the same order.  Above 16 tokens
+ *          that tile quantizes too where its tokens hold few values (layers of short K), in any of the four linears.
  *          mi355_fp8_block_linear_plan (host only, dense 16-byte aligned operands and 16-bit x assumed) writes the GEMM that
  *          runs in the format of mi355_fp8_blockwise_mm_plan followed by quantizer=fused|launch.
  *   x [M, K] contiguous F32/F16/BF16, K % 128 == 0; w [N, K] e4m3fn row stride ldw; w_scale element (nb, kb) at

@@ -13,15 +13,16 @@ enum TokenQuant {
   TQ_GROUP,  // unquantized (p.x16): quantized here per 1 x 128 group, fp32 scales, or exponents where UE8M0
   TQ_ROW,    // unquantized: quantized here per token
 };
-// Every workgroup repeats the quantizer's work, so it pays for few tokens only: at most WS_QUANT_VECTORS 16-byte pieces per
-// thread (K = 7168 with eight waves: five tokens), about 1 us, most of it under the latency of the weight blocks requested just
-// before; the launch it replaces costs 2.4 us on the GPU and 2.7 us on the host.
+// Every workgroup repeats the quantizer's work, so it pays for few values only: at most WS_QUANT_VECTORS 16-byte pieces per
+// thread (K = 7168 with eight waves: five tokens), 0.3 us each, the first of it under the latency of the weight blocks requested just
+// before; the launch it replaces costs 2.1 us on the GPU and 2.4 us on the host.
 constexpr int WS_QUANT_VECTORS = 10;
 
 __host__ __device__ constexpr int ws_scale_bytes(bool per_group, int M, int kb_total) { return ((per_group ? M * kb_total * 4 : 64) + 15) & ~15; }
 
-template <bool F8, bool BF16>
-__device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, float mul) {  // per_token_quant.hip, emit_vector
+// NAN_LOW: a NaN becomes -448, as group_quant.hip clamps; else 448 (per_token_quant.hip, emit_vector)
+template <bool F8, bool BF16, bool NAN_LOW = false>
+__device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, float mul) {
   float f[8];
   unpack8<BF16>(raw, f);
   uint32_t out[2];
@@ -30,7 +31,10 @@ __device__ __forceinline__ u32x2 codes_of_row(const u32x4& raw, float mul) {  //
     if constexpr (F8) {
       float t[4];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) t[b] = -__builtin_amdgcn_fmed3f(-(f[4 * j + b] * mul), -448.0f, 448.0f);  // (NaN: 448, as the quantizer kernel has it)
+      for (int b = 0; b < 4; ++b) {
+        const float v = f[4 * j + b] * mul;
+        t[b] = NAN_LOW ? __builtin_amdgcn_fmed3f(v, -448.0f, 448.0f) : -__builtin_amdgcn_fmed3f(-v, -448.0f, 448.0f);
+      }
       int c = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
       out[j] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], c, true);
     } else {
@@ -132,7 +136,7 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int
             const float m = row16_max(fmaxf(amax8<BF16>(raw[i]), 1e-10f));
             const uint32_t bits = __float_as_uint(m * (1.0f / 448.0f));
             const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0u);
-            q8 = codes_of_row<true, BF16>(raw[i], __uint_as_float((uint32_t)(127 - e) << 23));
+            q8 = codes_of_row<true, BF16, true>(raw[i], __uint_as_float((uint32_t)(127 - e) << 23));
             sc = __uint_as_float((uint32_t)(e + 127));
           } else {
             q8 = quantize_group_lane<BF16>(raw[i], p.x_by_reciprocal != 0, sc);

@@ -846,6 +846,7 @@ std::vector<std::string> tile_constant_names() {
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
                   "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_rounds_margin", "streamed_min_weight", "streamed_two_tokens_min_kblocks", "small_min_tokens", "small_max_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
+  add("quant.", {"launch", "tile", "piece[block]", "piece[ue8m0]", "piece[token_fp8]", "piece[int8]", "kb", "kb_busy", "result", "saved"});
   names.resize(TILE_CONSTANT_COUNT);
   return names;
 }
@@ -1286,6 +1287,12 @@ LinearRoute uncached_choose_linear(WavesplitQuant quant, int64_t M, int64_t N, i
   const Route run = run_route(kind, M, N, K, K, ldw, w_aligned && K % 16 == 0);
   if (!q_ok) return {LM_LAUNCH, run};
   if (tile_quant_preferred(run, M, N, K)) return {LM_TILE, run};
+  if (M > 16 && run.kernel == RK_WAVESPLIT_TILE && K % KSTEP == 0) {
+    const TileChoice c = choose_quant_tile(kind, M, N, K, run.bm, run.bn);
+    Route r = run;
+    r.bm = c.bm, r.bn = c.bn;
+    if (c.family != TF_NONE) return {LM_TILE, r};
+  }
   // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks; 4096 -> 24576 at 16 tokens 26.2 / 23.7)
   const LinearMode producer_mode = rotates_k(N, K, ldw) ? LM_LAUNCH_OWN : LM_PRODUCER;
   // the block linear on a large weight (its own choice, see choose_decode_tile), with the producer waves of the mid-M tile

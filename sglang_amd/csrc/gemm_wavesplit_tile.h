@@ -32,6 +32,7 @@ constexpr int WST_WAVES = 8;
 
 // TQ: the tokens arrive unquantized; their codes take code_bytes of the LDS and the slots hold weight rows only.
 constexpr int WST_QUANT_VALUES = 64 * WST_WAVES * WS_QUANT_VECTORS * 8;  // of a tile's tokens: as many pieces as there may be
+static_assert(WST_QUANT_VALUES == WAVESPLIT_QUANT_VALUES, "what the choice of a tile goes by");
 constexpr int WST_SCALE_BYTES = (WST_QUANT_VALUES / KSTEP + 2) * 4;
 constexpr int wst_code_bytes(int bm) { return WST_QUANT_VALUES + bm * 16; }  // rows are 16 bytes longer than K
 template <Arith AR, int MT, int CT, TokenQuant TQ>

@@ -45,6 +45,12 @@ struct StreamedTimes {
   double tile = 1.55, channel = 0.0201, token = 0.0103, stream = 8.70, stream_us = 3.02, norm = 2.06;
   double launch = 3.0, block = 0.098, block_channel = 0.00236, block_token = 0.00264, shared = 2.0, mid_stream = 7.06, mid_stream_us = 3.32;
 };
+// More than 16 tokens quantized inside the wave-split tile (choose_quant_tile), one round of workgroups: launch + tile + pieces of eight values a
+// thread * piece (by GemmKind) + KB of weight * kb * (1 + kb_busy * fill) + kilo-elements of the tile * result.  `saved`: what the quantizer's
+// launch takes beside the wave-split tile's modelled time.
+struct QuantTimes {
+  double launch = 1.29, tile = 1.32, piece[4] = {0.310, 0.295, 0.370, 0.377}, kb = 0.0051, kb_busy = 2.54, result = 0.488, saved = 1.4;
+};
 constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     1.93, 0.586, 4.31, 0.217, 4.18, -4.54, 1.808, 0.421,
     {2.33, 2.83, 3.02, 3.40, 3.53, 4.64, 2.57, 3.31, 3.96, 4.32, 2.64, 3.53, 4.44},
@@ -85,6 +91,7 @@ struct TileModel {
   TileTimes scaled = SCALED_TIMES, plain = PLAIN_TIMES;
   TileLimits limits;
   StreamedTimes streamed;
+  QuantTimes quant;
 };
 constexpr int TILE_CONSTANT_COUNT = sizeof(TileModel) / sizeof(double);
 // What the calling thread's dispatcher uses: the defaults above, or the perturbed copy a plan query installed.
@@ -242,6 +249,31 @@ TileChoice best_resident(GemmKind kind, int64_t M, int64_t N, int64_t K) {
     if (us < (rounds > 1 ? tile_model().limits.resident_rounds_margin : 1.0) * best.us) best = {TF_RESIDENT, step, RESIDENT_CHANNELS, 1, us, (int)ranges};
   }
   if (best.family != TF_NONE) best.us = least;
+  return best;
+}
+
+// A linear of more than 16 tokens whose GEMM runs on the wave-split tile: the tile, of any size (all of them add the same products in the same
+// order), that quantizes its tokens itself in the one launch, or TF_NONE.  Every channel tile repeats the quantizer's work, so it pays
+// for layers of short K, as long as one round of workgroups does it (a second one never: 42 tokens 1536 -> 12288 16.3 us, two launches
+// 10.3), and where the tile's tokens are at most ten pieces of eight values a thread.
+// Fitted to 1600 timings of 320 linears: 6 % root mean square, the tile it names within 0.2 % of the best on average.  130 linears on this side
+// of the line, one launch / two: 0.845 of the time in a graph (0.53 to 1.05), 0.72 eager (0.5 to 0.9); us in a graph, two launches / this:
+// 18 tokens 512 -> 896 5.0 / 3.5, 669 tokens packed exponents 640 -> 384 6.8 / 4.3, 69 tokens per-token FP8 768 -> 384 5.3 / 4.2, INT8 103 tokens
+// 768 -> 768 5.6 / 4.35, 82 tokens 1664 -> 512 5.6 / 5.4; on the other side 23 tokens per-token FP8 1792 -> 4096 5.8 / 6.4, 41 tokens
+// 2432 -> 2176 5.9 / 6.8.
+TileChoice choose_quant_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, int plain_bm, int plain_bn) {
+  const QuantTimes& q = tile_model().quant;
+  double two_launches = 0.0;
+  for (int i = 0; i < (int)(sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0])); ++i)
+    if (WAVESPLIT_TILES[i].bm == plain_bm && WAVESPLIT_TILES[i].bn == plain_bn) two_launches = wavesplit_tile_us(tile_times(kind), i, M, N, K) + q.saved;
+  TileChoice best{TF_NONE, 0, 0, 1, two_launches};
+  for (const TileSize& t : WAVESPLIT_QUANT_TILES) {
+    const int64_t values = std::min<int64_t>(M, t.bm) * K, wg = ceil_div(M, t.bm) * ceil_div(N, t.bn);
+    if (values > WAVESPLIT_QUANT_VALUES || wg > NUM_CUS) continue;
+    const double us = q.launch + q.tile + (double)ceil_div(values, WAVESPLIT_QUANT_VALUES / 10) * q.piece[kind] +
+                      (double)(t.bn * K) * 1e-3 * q.kb * (1.0 + q.kb_busy * (double)wg / NUM_CUS) + (double)(t.bm * t.bn) / 1024.0 * q.result;
+    if (us < best.us) best = {TF_WAVESPLIT, t.bm, t.bn, 1, us};
+  }
   return best;
 }
 

@@ -247,7 +247,14 @@ LINEAR_SHAPES = [(1, 128, 128), (15, 128, 1408), (8, 34176, 1536), (2, 18432, 74
                  (15, 8336, 2816), (1, 8320, 128), (15, 16, 1280), (12, 16896, 128), (5, 4864, 28800), (3, 14208, 7168), (9, 128, 1152), (17, 16, 128),
                  (1, 8, 128), (1, 8, 1024), (1, 66304, 128), (5, 27904, 8192), (3, 78208, 256), (1, 131328, 128), (11, 16, 1920), (2, 23872, 3840),
                  (2, 33472, 4096), (1, 80768, 3328), (3, 17408, 3840), (5, 17920, 3840), (13, 20864, 1536), (13, 65664, 1152), (1, 16512, 128),
-                 (7, 32512, 1792), (15, 28160, 1024), (5, 19392, 4096)]
+                 (7, 32512, 1792), (15, 28160, 1024), (5, 19392, 4096),
+                 (17, 2816, 7168)]
+# Above decode sizes, the wave-split tiles that quantize their tokens: (tokens x channels, whether a thread has more than five pieces of eight values),
+# each with a last tile of a few tokens or channels
+QUANT_TILE_SHAPES = {((16, 16), False): (143, 24, 640), ((16, 16), True): (49, 16, 1664), ((16, 32), False): (168, 400, 1280),
+                     ((16, 32), True): (76, 968, 1408), ((16, 64), False): (54, 2656, 384), ((16, 64), True): (171, 896, 1408),
+                     ((32, 32), False): (21, 5200, 896), ((32, 32), True): (18, 7064, 1152), ((32, 64), False): (139, 2304, 640),
+                     ((32, 64), True): (23, 9392, 896)}
 
 
 def linear_variant_of(plan: dict, M: int):

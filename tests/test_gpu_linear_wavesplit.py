@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from fp8_tolerance import check_fp8_gemm
-from gemm_cases import LINEAR_SHAPES
+from gemm_cases import LINEAR_SHAPES, QUANT_TILE_SHAPES
 from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +67,46 @@ def test_reciprocal_on_every_significand(gpu):
         _lib.check(_lib.lib().mi355_probe_reciprocal(e, ctypes.c_void_p(counts.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
     assert counts.tolist() == [0, 0]
     assert _lib.lib().mi355_probe_reciprocal(121, ctypes.c_void_p(counts.data_ptr()), None) == 1
+
+
+@pytest.mark.parametrize("tile,many", QUANT_TILE_SHAPES)
+def test_fused_quantizer_above_decode_sizes(gpu, tile, many):
+    """One launch against quantizer and GEMM entry point, which runs on a wave-split tile of its own size: the same codes, scales and sums,
+    so the same results bit for bit, with rows that are all zero, infinite or partly NaN."""
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import per_token_group_quant_fp8, sglang_per_token_group_quant_fp8, sglang_per_token_quant_fp8, w8a8_block_fp8_matmul
+    from sglang_amd.fp8_utils import requant_weight_ue8m0
+    from sglang_amd.int8_kernel import per_token_quant_int8
+
+    M, N, K = QUANT_TILE_SHAPES[tile, many]
+    plans = {k: _lib.linear_plan(k, M, N, K) for k in ("block", "ue8m0", "token_fp8", "int8")}
+    print(f"case M={M} N={N} K={K} {plans}", flush=True)
+    assert any((p["quantizer"], p["bm"], p["bn"]) == ("fused", *tile) for p in plans.values()) and (min(M, tile[0]) * K > 20480) == many
+    for dtype in (torch.bfloat16, torch.float16):
+        bits = lambda t: torch.where(t.isnan(), torch.zeros_like(t), t).view(torch.int16)
+        x = make_activation(M, K, seed=M + N, dtype=dtype)
+        x[0], x[M - 1], x[M // 2, 5], x[1, 7] = 0, 0, float("inf"), float("nan")
+        xg = x.to(gpu)
+        bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).to(dtype).to(gpu)
+        w_q, w_s = make_fp8_weight(N, K, seed=K)
+        wg, sg = w_q.to(gpu), w_s.to(gpu)
+        for by_reciprocal in (False, True):
+            q, s = per_token_group_quant_fp8(xg, 128, column_major_scales=not by_reciprocal)
+            out, two = ops.block_fp8_linear(xg, wg, sg, None, dtype, by_reciprocal=by_reciprocal), w8a8_block_fp8_matmul(q, wg, s, sg, [128, 128], dtype)
+            assert torch.equal(bits(out), bits(two)) and torch.equal(out.isnan(), two.isnan())
+        w2, words = requant_weight_ue8m0(wg, sg, [128, 128])
+        q, s = sglang_per_token_group_quant_fp8(xg, 128, column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=True, enable_v2=True)
+        out, two = ops.block_fp8_linear_ue8m0(xg, w2, words, bias, dtype), ops.fp8_blockwise_mm_ue8m0(q, w2, s, words, dtype, bias)
+        assert torch.equal(bits(out), bits(two)) and torch.equal(out.isnan(), two.isnan())
+        scale = torch.rand(N, generator=torch.Generator().manual_seed(K)).to(gpu) * 0.01 + 1e-3
+        q, s = sglang_per_token_quant_fp8(xg)
+        out, two = ops.fp8_per_token_linear(xg, wg.t(), scale, bias, dtype), ops.fp8_scaled_mm(q, wg.t(), s, scale, dtype, bias)
+        assert torch.equal(bits(out), bits(two)) and torch.equal(out.isnan(), two.isnan())
+        xg[M // 2, 5] = xg[1, 7] = 1  # (a row with an infinity has no INT8 codes)
+        i_q, i_s = make_int8_weight(N, K, seed=K)
+        q, s = per_token_quant_int8(xg)
+        iw, isc = i_q.to(gpu).t(), i_s.to(gpu)
+        assert torch.equal(bits(ops.int8_linear(xg, iw, isc, bias, dtype)), bits(ops.int8_scaled_mm(q, iw, s, isc, dtype, bias)))
 
 
 # every kernel that quantizes tokens itself: (kinds, kernel, channel tile or waves, shape)
