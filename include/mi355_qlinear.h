@@ -446,6 +446,12 @@ int mi355_fp8_per_token_linear_plan(int64_t M, int64_t N, int64_t K, char* buf, 
 int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void* w, const float* w_scale, const void* bias, void* out,
                                int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo, void* workspace,
                                size_t workspace_bytes, void* stream);
+/* The same with one static scale for all tokens, x_scale[0] on the device (apply_fp8_linear's input_scale, fp8_utils.py:748-753): the
+ * result is that of mi355_per_tensor_quant_fp8 (static, scale copied per row) followed by mi355_fp8_scaled_mm, bit for bit; what runs is
+ * mi355_fp8_per_token_linear_plan's, same workspace. */
+int mi355_fp8_static_linear(const void* x, int x_dtype, const float* x_scale, const void* w, const float* w_scale, const void* bias,
+                            void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo, void* workspace,
+                            size_t workspace_bytes, void* stream);
 
 /*
  * One block-FP8 linear layer with packed power-of-two scales in one call:

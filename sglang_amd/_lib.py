@@ -68,6 +68,7 @@ EXPORTS = (
     "mi355_int8_linear",
     "mi355_fp8_per_token_linear_workspace_bytes",
     "mi355_fp8_per_token_linear",
+    "mi355_fp8_static_linear",
     "mi355_fp8_block_linear_ue8m0_workspace_bytes",
     "mi355_fp8_block_linear_ue8m0",
 )
@@ -177,6 +178,8 @@ def lib() -> ctypes.CDLL:
     L.mi355_fp8_per_token_linear_workspace_bytes.restype = sz
     L.mi355_fp8_per_token_linear.argtypes = [vp, i32, vp, vp, vp, vp, i32] + [i64] * 5 + [vp, sz, vp]
     L.mi355_fp8_per_token_linear.restype = i32
+    L.mi355_fp8_static_linear.argtypes = [vp, i32, vp, vp, vp, vp, vp, i32] + [i64] * 5 + [vp, sz, vp]
+    L.mi355_fp8_static_linear.restype = i32
     L.mi355_fp8_block_linear_ue8m0_workspace_bytes.argtypes = [i64, i64, i64]
     L.mi355_fp8_block_linear_ue8m0_workspace_bytes.restype = sz
     L.mi355_fp8_block_linear_ue8m0.argtypes = [vp, i32, vp, vp, i64, i64, vp, vp, i32] + [i64] * 5 + [vp, sz, vp]

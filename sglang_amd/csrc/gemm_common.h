@@ -34,6 +34,7 @@ struct GemmParams {
   const void* x16;         // FP8 decode kernel only, optional: unquantized tokens [M, K] (x_dtype, row stride ldx elements);
   int64_t ldx;             // when set, the kernel quantizes them per 1 x 128 group itself and ignores a / sa
   int x_dtype;
+  const float* x_scale;    // per-token FP8 only, optional: one scale for all unquantized tokens in the place of theirs
   int x_by_reciprocal;     // the fused quantizer computes q = x * (1 / s) instead of q = x / s
   void* out;
   void* ws;  // split-K partial tiles: [splits][M][N] fp32 or int32

@@ -88,9 +88,12 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int
 #pragma unroll
   for (int i = 0; i < NV; ++i)
     asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(raw[i]) : "v"((uint32_t)min(piece(i), total - 1) * 16u), "s"(x) : "memory");
+  const bool given = TQ == TQ_ROW && IS_FP8 && p.x_scale != nullptr;  // one scale for all tokens: per_tensor_quant.hip's arithmetic
+  float given_scale = 1.0f;
   if constexpr (TQ == TQ_ROW) {
-    if (threadIdx.x < BM) reinterpret_cast<uint32_t*>(row_max)[threadIdx.x] = __float_as_uint(IS_FP8 ? 0.f : 1e-10f);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (given) given_scale = *(const __attribute__((address_space(4))) float*)p.x_scale;
+    else if (threadIdx.x < BM) reinterpret_cast<uint32_t*>(row_max)[threadIdx.x] = __float_as_uint(IS_FP8 ? 0.f : 1e-10f);
+    if (!given) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
   request();
 #pragma unroll
@@ -100,7 +103,10 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int
     if (p.x_dtype == MI355_BF16) body(std::true_type{});
     else body(std::false_type{});
   };
-  if constexpr (TQ == TQ_ROW) {
+  if (given) {
+    if (threadIdx.x < BM) token_scale[threadIdx.x] = given_scale, row_max[threadIdx.x] = 1.0f / given_scale;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  } else if constexpr (TQ == TQ_ROW) {
     by_type([&](auto bf16_c) {
       constexpr bool BF16 = decltype(bf16_c)::value;
 #pragma unroll

@@ -1542,10 +1542,11 @@ extern "C" size_t mi355_fp8_per_token_linear_workspace_bytes(int64_t M, int64_t 
   return align256((size_t)M * (size_t)K) + align256((size_t)M * 4u) + mi355_fp8_scaled_mm_workspace_bytes(M, N, K);
 }
 
-extern "C" int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void* w, const float* w_scale, const void* bias,
-                                          void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo,
-                                          void* workspace, size_t workspace_bytes_given, void* stream) {
-  const char* what = "mi355_fp8_per_token_linear";
+namespace {
+// x_scale: one scale for all tokens, or null (each token's own)
+int per_token_linear(const char* what, const void* x, int x_dtype, const float* x_scale, const void* w, const float* w_scale, const void* bias,
+                     void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo, void* workspace,
+                     size_t workspace_bytes_given, void* stream) {
   clear_error();
   MI355_REQUIRE(M >= 0 && N >= 0 && K >= 0, MI355_ERR_INVALID_ARGUMENT, "%s: negative shape", what);
   MI355_REQUIRE(out_dtype == MI355_BF16 || out_dtype == MI355_F16, MI355_ERR_INVALID_ARGUMENT,
@@ -1572,14 +1573,30 @@ extern "C" int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void
     // (the block scales are not read in this mode; they only have to satisfy the checks)
     const int rc = fp8_mm_params(what, x, w, w_scale, w_scale, out, out_dtype, M, N, K, K, ldw, 1, 0, 0, 0, ldo, p, empty);
     if (rc != MI355_OK || empty) return rc;
-    p.col_scale = w_scale, p.bias = bias;
+    p.col_scale = w_scale, p.bias = bias, p.x_scale = x_scale;
     if (linear.mode == LM_TILE) return run_tile_quant(p, WavesplitQuant::TOKEN_FP8, linear.gemm, x, x_dtype, stream, what);
     return run_wavesplit_quant(p, WavesplitQuant::TOKEN_FP8, x, x_dtype, stream, what);
   }
-  const int rc = mi355_per_token_quant_fp8(x, x_dtype, q, sa, M, K, stream);
+  const int rc = x_scale ? mi355_per_tensor_quant_fp8(x, x_dtype, q, const_cast<float*>(x_scale), M * K, 1, sa, M, stream)
+                         : mi355_per_token_quant_fp8(x, x_dtype, q, sa, M, K, stream);
   if (rc != MI355_OK) return rc;
   return mi355_fp8_scaled_mm(q, w, sa, w_scale, bias, out, out_dtype, M, N, K, K, ldw, ldo, q + q_bytes + sa_bytes,
                              workspace_bytes_given - q_bytes - sa_bytes, stream);
+}
+}  // namespace
+
+extern "C" int mi355_fp8_per_token_linear(const void* x, int x_dtype, const void* w, const float* w_scale, const void* bias,
+                                          void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo,
+                                          void* workspace, size_t workspace_bytes_given, void* stream) {
+  return per_token_linear("mi355_fp8_per_token_linear", x, x_dtype, nullptr, w, w_scale, bias, out, out_dtype, M, N, K, ldw, ldo, workspace,
+                          workspace_bytes_given, stream);
+}
+extern "C" int mi355_fp8_static_linear(const void* x, int x_dtype, const float* x_scale, const void* w, const float* w_scale, const void* bias,
+                                       void* out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldo, void* workspace,
+                                       size_t workspace_bytes_given, void* stream) {
+  const char* what = "mi355_fp8_static_linear";
+  MI355_REQUIRE(x_scale != nullptr || M == 0 || N == 0, MI355_ERR_INVALID_ARGUMENT, "%s: null pointer", what);
+  return per_token_linear(what, x, x_dtype, x_scale, w, w_scale, bias, out, out_dtype, M, N, K, ldw, ldo, workspace, workspace_bytes_given, stream);
 }
 
 extern "C" size_t mi355_fp8_block_linear_ue8m0_workspace_bytes(int64_t M, int64_t N, int64_t K) {

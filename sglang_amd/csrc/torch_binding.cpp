@@ -710,18 +710,10 @@ std::optional<Tensor> try_token_linear(const Tensor& x, const Tensor& w, const T
   }
   if (!(input_scale->numel() == 1 && input_scale->is_cuda() && input_scale->scalar_type() == ScalarType::Float)) return std::nullopt;
   Tensor out = new_output(x, N);
-  // codes, then the scale once per row, then the GEMM's own workspace
-  const auto align256 = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t q_bytes = align256((size_t)M * (size_t)K), s_bytes = align256((size_t)M * 4);
-  const Workspace mem(q_bytes + s_bytes + mi355_fp8_scaled_mm_workspace_bytes(M, N, K));
-  uint8_t* q = static_cast<uint8_t*>(mem.ptr());
-  float* s = reinterpret_cast<float*>(q + q_bytes);
-  void* stream = current_stream();
-  check(mi355_per_tensor_quant_fp8(x.const_data_ptr(), dtype_code(x.scalar_type()), q, static_cast<float*>(input_scale->data_ptr()), M * K, 1,
-                                   s, M, stream));
-  check(mi355_fp8_scaled_mm(q, w.const_data_ptr(), s, static_cast<const float*>(ws.const_data_ptr()), data_or_null(bias), out.data_ptr(),
-                            dtype_code(out.scalar_type()), M, N, K, K, w.stride(1), N, q + q_bytes + s_bytes,
-                            mem.bytes - q_bytes - s_bytes, stream));
+  const Workspace mem(mi355_fp8_per_token_linear_workspace_bytes(M, N, K));
+  check(mi355_fp8_static_linear(x.const_data_ptr(), dtype_code(x.scalar_type()), static_cast<const float*>(input_scale->const_data_ptr()),
+                                w.const_data_ptr(), static_cast<const float*>(ws.const_data_ptr()), data_or_null(bias), out.data_ptr(),
+                                dtype_code(out.scalar_type()), M, N, K, w.stride(1), N, mem.ptr(), mem.bytes, current_stream()));
   return out;
 }
 

@@ -105,6 +105,11 @@ def test_newer_entry_points_validate_before_any_device_work():
     assert I(p, _lib.BF16, p, p, None, p, _lib.BF16, 4, 128, 1024, 1024, 128, None, 0, None) == 4
     assert I(None, _lib.BF16, None, None, None, None, _lib.BF16, 0, 128, 1024, 1024, 128, None, 0, None) == 0
     assert L.mi355_int8_linear_workspace_bytes(0, 128, 1024) == 0 and L.mi355_int8_linear_workspace_bytes(4, 128, 1024) % 256 == 0
+    # the same with a static scale: the scale, workspace, empty problem
+    S = L.mi355_fp8_static_linear
+    assert S(p, _lib.BF16, None, p, p, None, p, _lib.BF16, 4, 128, 1024, 1024, 128, p, 1 << 20, None) == 1 and b"null" in L.mi355_last_error()
+    assert S(p, _lib.BF16, p, p, p, None, p, _lib.BF16, 4, 128, 1024, 1024, 128, None, 0, None) == 4
+    assert S(None, _lib.BF16, None, None, None, None, None, _lib.BF16, 0, 128, 1024, 1024, 128, None, 0, None) == 0
     # one-call per-token FP8 linear: output dtype, workspace, empty problem
     T = L.mi355_fp8_per_token_linear
     assert T(p, _lib.BF16, p, p, None, p, _lib.F32, 4, 128, 1024, 1024, 128, p, 1 << 20, None) == 1

@@ -111,3 +111,35 @@ def test_apply_fp8_linear_paths(gpu, oracle, path):
     ref, mag = oracle.fp8_scaled_mm(q_o, w, sa.contiguous(), ws, torch.float32, None, want_abs=True)
     ref = ref + bias.float()[None, :]
     check_fp8_gemm(out.reshape(M, N), ref, mag, path)
+
+
+# one launch on the wave-split tile at decode sizes and above, on the register kernel, and a launch in front of the GEMM
+@pytest.mark.parametrize("M,N,K,quantizer,kernel", [(16, 2176, 2176, "fused", "wavesplit_tile"), (1, 576, 7168, "fused", "wavesplit_tile"),
+                                                    (143, 24, 640, "fused", "wavesplit_tile"), (40, 3712, 640, "fused", "wavesplit_tile"),
+                                                    (1, 16512, 3840, "fused", "decode_wavesplit"), (4, 7168, 2048, "fused", "decode_wavesplit"),
+                                                    (17, 2816, 7168, "launch", "wavesplit_tile"), (40, 1032, 1040, "launch", "wavesplit_tile")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_static_scale_inside_the_gemm(gpu, M, N, K, quantizer, kernel, dtype):
+    """apply_fp8_linear with a static scale against quantizer and GEMM: the same codes and sums, so the same bits; values beyond the scale's
+    range, infinities and NaN among them."""
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import static_quant_fp8
+    from sglang_amd.fp8_utils import apply_fp8_linear
+    from sglang_amd.workloads import make_activation, make_fp8_weight
+
+    plan = _lib.linear_plan("token_fp8", M, N, K)
+    print(f"case M={M} N={N} K={K} {plan}", flush=True)
+    assert (plan["quantizer"], plan["kernel"]) == (quantizer, kernel)
+    x = make_activation(M, K, seed=M + N, dtype=dtype)
+    x[0, 3], x[M // 2, 5], x[M - 1, K - 1] = float("inf"), float("nan"), 3e4
+    xg = x.to(gpu)
+    w = make_fp8_weight(N, (K + 127) // 128 * 128, seed=K)[0][:, :K].contiguous().to(gpu)
+    scale = torch.rand(N, generator=torch.Generator().manual_seed(K)).to(gpu) * 0.01 + 1e-3
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).to(dtype).to(gpu)
+    bits = lambda t: torch.where(t.isnan(), torch.zeros_like(t), t).view(torch.int16)
+    for given in (0.02, 0.5):
+        s = torch.tensor([given], device=gpu)
+        out = apply_fp8_linear(xg, w.t(), scale, s, bias=bias)
+        q, rows = static_quant_fp8(xg, s, repeat_scale=True)
+        two = ops.fp8_scaled_mm(q, w.t(), rows, scale, dtype, bias)
+        assert torch.equal(bits(out), bits(two)) and torch.equal(out.isnan(), two.isnan())
