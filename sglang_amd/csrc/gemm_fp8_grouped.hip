@@ -16,11 +16,12 @@
 //      fp8_grouped_dma_kernel (gemm_fp8_dma3.hip), the mid-M tile of 64 or 128 tokens x 128 or 256 channels, over the second:
 //      one workgroup per (token tile, channel tile).  The first launch is left out when no expert can have more than
 //      128 rows, and where small tiles alone model faster (choose_grouped_run): then every row goes to the second table.
+// Few rows on small weights take one launch instead, fp8_grouped_wavesplit_kernel, whose workgroups find their tile themselves.
 // Where the reference takes device arrays of per-expert pointers, strides and scale layouts as scratch that its own
 // set-up kernel fills, this interface takes the base pointers and strides and keeps its scratch in the workspace.
 #include <cmath>
 
-#include "gemm_common.h"
+#include "gemm_wavesplit_tile.h"
 
 namespace mi355 {
 namespace {
@@ -132,6 +133,81 @@ __global__ __launch_bounds__(256) void grouped_prepare_kernel(const int32_t* pro
   }
 }
 
+// ---- few rows an expert on small weights: the wave-split tile, in one launch.  Every workgroup finds its token tile itself, by the prefix sums of
+// the tile counts over the experts, 512 experts (or runs of experts) at a time, and the tile reads the token scales as they lie.
+struct GroupedRouting {
+  const int32_t *problem_sizes, *expert_offsets;
+  int E, total_m;
+};
+// The workgroup's token tile as the parameters of its expert's problem; false for a workgroup without one (all of it leaves).
+template <int BM>
+__device__ __forceinline__ bool find_tile(const GroupedParams& gp, const GroupedRouting& r, GemmParams& p, int& m0, int& tile_n) {
+  constexpr int W = WST_WAVES;
+  __shared__ int wave_tiles[W];
+  __shared__ v4i record;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int run = (r.E + 64 * W - 1) / (64 * W), first = (int)threadIdx.x * run;  // a thread's experts
+  const auto tiles_of = [&](int e) { return expert_tiles(r.problem_sizes, r.expert_offsets, e, r.E, r.total_m, BM, false); };
+  int mine = 0;
+  for (int i = 0; i < run; ++i) mine += tiles_of(first + i).small;
+  int sum = mine;  // inclusive, within the wave
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(sum, d);
+    if (lane >= d) sum += v;
+  }
+  if (lane == 63) wave_tiles[wave] = sum;
+  __syncthreads();
+  int before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    const int n = wave_tiles[w];
+    all += n;
+    if (w < wave) before += n;
+  }
+  const int count = min(__builtin_amdgcn_readfirstlane(all), gp.max_tiles_m), total = count * gp.g.tiles_n;
+  int bid = blockIdx.x;
+  if (bid >= total) return false;
+  // the XCDs take contiguous ranges; inside one the token tiles of a channel tile follow each other
+  const int per = total >> 3;
+  if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
+  const int span = GROUPED_GM * gp.g.tiles_n, group = bid / span, at = bid - group * span, gm = min(GROUPED_GM, count - group * GROUPED_GM);
+  tile_n = at / gm;
+  int t = group * GROUPED_GM + at % gm - (before + sum - mine);  // counted from the thread's first tile
+  if (t >= 0 && t < mine) {
+    for (int i = 0; i < run; ++i) {
+      const ExpertTiles x = tiles_of(first + i);
+      if (t >= 0 && t < x.small) record = v4i{first + i, x.row0, x.rows, t * BM};
+      t -= x.small;
+    }
+  }
+  __syncthreads();
+  const int e = __builtin_amdgcn_readfirstlane(record.x), row0 = __builtin_amdgcn_readfirstlane(record.y);
+  m0 = __builtin_amdgcn_readfirstlane(record.w);
+  p = gp.g;
+  p.a += (int64_t)row0 * p.lda;
+  p.b += (int64_t)e * gp.b_expert_stride;
+  p.sa += (int64_t)row0 * p.sa_sm;
+  p.sb += (int64_t)e * gp.sb_expert_stride;
+  p.out = reinterpret_cast<uint8_t*>(p.out) + (int64_t)row0 * p.ldo * gp.out_elem;
+  p.M = __builtin_amdgcn_readfirstlane(record.z);
+  return true;
+}
+template <int MT, int CT>
+__global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp8_grouped_wavesplit_kernel(const GroupedParams gp, const GroupedRouting r) {
+  GemmParams p;
+  int m0, tile_n;
+  if (find_tile<16 * MT>(gp, r, p, m0, tile_n)) wavesplit_tile<AR_F32, MT, CT, TQ_NONE, 2, false>(p, m0, tile_n * 16 * CT);
+}
+constexpr TileSize GROUPED_WAVESPLIT_TILES[] = {{16, 16}, {16, 32}, {16, 64}, {32, 32}, {32, 64}, {64, 64}};
+template <size_t... I>
+void launch_grouped_wavesplit(const GroupedParams& gp, const GroupedRouting& r, int bm, int bn, hipStream_t stream, std::index_sequence<I...>) {
+  const dim3 grid((unsigned)(gp.max_tiles_m * gp.g.tiles_n)), block(64 * WST_WAVES);
+  ((bm == GROUPED_WAVESPLIT_TILES[I].bm && bn == GROUPED_WAVESPLIT_TILES[I].bn
+        ? launch_kernel((fp8_grouped_wavesplit_kernel<GROUPED_WAVESPLIT_TILES[I].bm / 16, GROUPED_WAVESPLIT_TILES[I].bn / 16>), grid, block, 0, stream, gp, r)
+        : (void)0), ...);
+}
+
 struct GroupedPlan {
   int max_big;             // upper bound on the number of 256-row tiles
   int64_t pitch;           // floats per K block in the re-laid-out token scales
@@ -154,6 +230,10 @@ struct GroupedRun {
   bool use_big;
   int bm, bn, max_big, max_small;
   bool few;  // at most a workgroup per CU is expected
+  // where split.bm > 0: one launch on the wave-split tile of this size, at most split_tiles token tiles; the above where the token scales' rows lie
+  // too far apart for it, and for the workspace
+  TileSize split{0, 0};
+  int split_tiles = 0;
 };
 
 size_t grouped_small_bytes(const GroupedRun& r) { return align256((size_t)(r.max_small + 1) * sizeof(v4i)); }
@@ -229,6 +309,37 @@ struct GroupedTimes {
   }
 };
 
+// The wave-split tile in one launch, us: LAUNCH + rounds of TILE + KB of operands * KB_US * (1 + BUSY * fill) + kilo-elements of the tile * RESULT,
+// joined with the stream of the weights that are used.  Rows fall on experts at random, so some of few get none.  Fitted to 770 timings of
+// 190 problems with up to 220 million active weights (their routing uneven by 0.25 .. 1.25): 7 % root mean square.  It saves the preparation and
+// splits K over eight waves where the mid-M tile has a chain of K blocks on a few CUs, but every further round of workgroups starts with
+// the search and the first loads again: taken up to one and a half rounds, where it models 10 % faster.  74 of the 190, this / tables and
+// mid-M tile: 0.595 of the time in a graph (at most 1.12), 0.65 eager; us in a graph 16 experts 22 rows 1152 -> 256 9.6 / 4.2, 32 of 136
+// 3840 -> 256 17.1 / 9.0, 64 of 59 6528 -> 384 31.6 / 18.6, 8 of 662 3456 -> 384 17.4 / 9.3; beyond, 128 of 61 1664 -> 768 17.0 / 18.6, 256 of 271
+// 1408 -> 640 31.9 / 44.4.
+struct GroupedWavesplitTimes {
+  static constexpr double LAUNCH = 1.27, TILE = 2.26, KB_US = 0.0064, BUSY = 1.07, RESULT = 0.459, STREAM = 7.71, NORM = 1.364, MOST_ROUNDS = 1.5, MARGIN = 0.9;
+  double active;
+  int64_t total_m, N, K;
+  GroupedWavesplitTimes(int64_t E, int64_t total_m_, int64_t N_, int64_t K_)
+      : active((double)E * (1.0 - std::pow(1.0 - 1.0 / (double)E, (double)total_m_))), total_m(total_m_), N(N_), K(K_) {}
+  double us(const TileSize& t, double most) const {
+    double tiles = 0.0;
+    for (int j = 0; j < GroupedTimes::SPREAD; ++j) {
+      const double share = active <= 1.0 ? 1.0 : 0.25 + (j + 0.5) * 1.5 / GroupedTimes::SPREAD;
+      tiles += (double)ceil_div(std::max<int64_t>(1, (int64_t)std::ceil((double)total_m / active * share - 1e-9)), t.bm) * active / GroupedTimes::SPREAD;
+    }
+    const double workgroups = tiles * (double)ceil_div(N, t.bn);
+    if (workgroups > MOST_ROUNDS * NUM_CUS) return most;
+    const auto round = [&](double fill) {
+      return TILE + (double)((t.bm + t.bn) * K) * 1e-3 * KB_US * (1.0 + BUSY * fill) + (double)(t.bm * t.bn) / 1024.0 * RESULT;
+    };
+    const double full = std::floor(workgroups / NUM_CUS), rest = workgroups / NUM_CUS - full;
+    const double tile_us = full * round(1.0) + (rest > 1e-9 ? round(rest) : 0.0), stream = active * (double)N * (double)K * 1e-6 / STREAM;
+    return LAUNCH + std::pow(std::pow(tile_us, NORM) + std::pow(stream, NORM), 1.0 / NORM);
+  }
+};
+
 GroupedRun choose_grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, const GroupedPlan& pl) {
   const GroupedTimes times(E, total_m, N, K);
   const auto alone = [&](const GroupedTile& t) {
@@ -246,6 +357,12 @@ GroupedRun choose_grouped_run(int64_t E, int64_t total_m, int64_t N, int64_t K, 
   for (int i = 1; i < 4; ++i) {
     const double us = times.small(SMALL_TILES[i]);
     if (us < 0.95 * best) best = us, r = alone(SMALL_TILES[i]);
+  }
+  const GroupedWavesplitTimes split(E, total_m, N, K);
+  best *= GroupedWavesplitTimes::MARGIN;
+  for (const TileSize& t : GROUPED_WAVESPLIT_TILES) {
+    const double us = split.us(t, best);
+    if (us < best) best = us, r.split = t, r.split_tiles = (int)std::min<int64_t>(total_m, total_m / t.bm + E);
   }
   return r;
 }
@@ -280,9 +397,11 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm_plan(int64_t num_experts, i
   MI355_REQUIRE(buf && buf_len > 0, MI355_ERR_INVALID_ARGUMENT, "%s: no buffer", what);
   MI355_REQUIRE(num_experts > 0 && total_m > 0 && N > 0 && K > 0, MI355_ERR_INVALID_ARGUMENT, "%s: empty problem", what);
   const GroupedRun run = grouped_run(num_experts, total_m, N, K, grouped_plan(num_experts, total_m, K));
+  const bool split = run.split.bm > 0;
+  const TileSize tile = split ? run.split : TileSize{run.bm, run.bn};
   const int n = snprintf(buf, buf_len, "kernel=%s small_tile=%dx%d max_big_tiles=%d max_small_tiles=%d tiles_n=%lld",
-                         run.use_big ? "grouped_pingpong+grouped_dma3" : "grouped_dma3", run.bm, run.bn, run.max_big, run.max_small,
-                         (long long)ceil_div(N, run.bn));
+                         split ? "grouped_wavesplit" : run.use_big ? "grouped_pingpong+grouped_dma3" : "grouped_dma3", tile.bm, tile.bn,
+                         split ? 0 : run.max_big, split ? run.split_tiles : run.max_small, (long long)ceil_div(N, tile.bn));
   MI355_REQUIRE(n > 0 && (size_t)n < buf_len, MI355_ERR_INVALID_ARGUMENT, "%s: buffer of %zu bytes is too small", what, buf_len);
   return MI355_OK;
 }
@@ -314,7 +433,8 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
   const GroupedPlan pl = grouped_plan(num_experts, total_m, K);
   const GroupedRun run = grouped_run(num_experts, total_m, N, K, pl);
   const size_t small_bytes = grouped_small_bytes(run);
-  MI355_REQUIRE(((int64_t)run.max_big + run.max_small) * ((N + run.bn - 1) / run.bn) < (1ll << 31), MI355_ERR_INVALID_ARGUMENT,
+  MI355_REQUIRE(((int64_t)run.max_big + run.max_small) * ((N + run.bn - 1) / run.bn) < (1ll << 31) &&
+                    (run.split.bm == 0 || run.split_tiles * ceil_div(N, run.split.bn) < (1ll << 31)), MI355_ERR_INVALID_ARGUMENT,
                 "%s: too many tiles", what);
   const size_t need = pl.big_bytes + small_bytes + pl.scale_bytes;
   MI355_REQUIRE(workspace && workspace_bytes >= need, MI355_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", what,
@@ -323,6 +443,20 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
                 "%s: workspace must be 256-byte aligned", what);
 
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (run.split.bm > 0 && total_m * std::max<int64_t>(sa_sm, 1) < (1ll << 30)) {  // (32-bit offsets of the token scales)
+    GroupedParams gp{};
+    gp.g.a = static_cast<const uint8_t*>(a), gp.g.b = static_cast<const uint8_t*>(b);
+    gp.g.sa = scales_a, gp.g.sb = scales_b, gp.g.out = out;
+    gp.g.N = (int)N, gp.g.K = (int)K, gp.g.kb_total = (int)(K / KSTEP), gp.g.splits = 1;
+    gp.g.lda = lda, gp.g.ldb = ldb, gp.g.ldo = ldo;
+    gp.g.sa_sm = sa_sm, gp.g.sa_sk = sa_sk, gp.g.sb_sn = sb_sn, gp.g.sb_sk = sb_sk;
+    gp.g.out_dtype = out_dtype;
+    gp.b_expert_stride = b_expert_stride, gp.sb_expert_stride = sb_expert_stride, gp.out_elem = 2;
+    gp.g.tiles_n = (int)ceil_div(N, run.split.bn), gp.max_tiles_m = run.split_tiles;
+    launch_grouped_wavesplit(gp, GroupedRouting{problem_sizes, expert_offsets, (int)num_experts, (int)total_m}, run.split.bm, run.split.bn, st,
+                             std::make_index_sequence<sizeof(GROUPED_WAVESPLIT_TILES) / sizeof(GROUPED_WAVESPLIT_TILES[0])>{});
+    return check_launch(what);
+  }
   uint8_t* wsp = static_cast<uint8_t*>(workspace);
   v4i* big_tiles = reinterpret_cast<v4i*>(wsp);
   v4i* small_tiles = reinterpret_cast<v4i*>(wsp + pl.big_bytes);

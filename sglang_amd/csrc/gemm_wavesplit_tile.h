@@ -59,10 +59,11 @@ __device__ __forceinline__ void wait_blocks(int blocks) {
   else wait_loads<0>();
 }
 
-template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2, bool STREAM = false>
-__global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void wavesplit_tile_kernel(const GemmParams p) {
+// The 16 MT x 16 CT tile at (m0, n0), by the whole workgroup.
+template <Arith AR, int MT, int CT, TokenQuant TQ, int NV, bool STREAM>
+__device__ __forceinline__ void wavesplit_tile(const GemmParams& p, int m0, int n0) {
   using T = WavesplitTile<AR, MT, CT, TQ>;
-  constexpr int R = T::R, LOADS = T::LOADS, BM = T::BM, BN = T::BN, W = WST_WAVES;
+  constexpr int R = T::R, LOADS = T::LOADS, BM = T::BM, W = WST_WAVES;
   using AccT = typename std::conditional<AR == AR_INT8, int, float>::type;
   typedef AccT acc4 __attribute__((ext_vector_type(4)));
   // the slots and, with unquantized tokens, their codes; the partial tiles lie over both
@@ -75,11 +76,6 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, q = lane >> 4;
-  // consecutive workgroups of an XCD take the token tiles of the same channels
-  int bid = blockIdx.x;
-  const int per_xcd = (int)gridDim.x >> 3;
-  if (bid < per_xcd * 8) bid = (bid & 7) * per_xcd + (bid >> 3);
-  const int m0 = (bid % p.tiles_m) * BM, n0 = (bid / p.tiles_m) * BN;
   const int rows = min(p.M - m0, BM);  // tokens of the tile
 
   // loader: a load fills 8 rows of a slot, lane = row lane >> 3, 16-byte chunk lane & 7; chunks land swizzled by (row & 7)
@@ -255,6 +251,15 @@ __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(
     }
     store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, min(4, p.N - n), vec_ok);
   }
+}
+
+template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2, bool STREAM = false>
+__global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void wavesplit_tile_kernel(const GemmParams p) {
+  // consecutive workgroups of an XCD take the token tiles of the same channels
+  int bid = blockIdx.x;
+  const int per_xcd = (int)gridDim.x >> 3;
+  if (bid < per_xcd * 8) bid = (bid & 7) * per_xcd + (bid >> 3);
+  wavesplit_tile<AR, MT, CT, TQ, NV, STREAM>(p, (bid % p.tiles_m) * (16 * MT), (bid / p.tiles_m) * (16 * CT));
 }
 
 template <Arith AR, int MT, int CT>

@@ -17,6 +17,12 @@ pytestmark = pytest.mark.gpu
     ("wide", [40] * 16, 2056, 256),
     ("tall_and_wide", [160] * 8, 3000, 128),
     ("big_tiles", [700, 300, 129, 128, 1025], 2048, 4224),
+    # the same edges with more channels, where tables are prepared
+    ("chunk_edges_prepared", [31, 1, 32, 33, 0, 0, 63, 1, 1, 64, 5], 2056, 4480),
+    ("two_scans_prepared", [1, 0, 2] * 110, 1032, 128),
+    ("one_row_each_prepared", [1] * 70, 1040, 4224),
+    # more experts than threads: runs of two a thread
+    ("runs_of_experts", [0, 0, 0, 1, 2, 0] * 7 + [0] * 555 + [17, 3, 2], 24, 256),
 ])
 @pytest.mark.parametrize("m_major", [False, True])
 def test_grouped(gpu, oracle, name, sizes, N, K, m_major):
@@ -28,7 +34,9 @@ def test_grouped(gpu, oracle, name, sizes, N, K, m_major):
 
 
 # experts (uneven: some without a row, one with many), stacked rows, N, K -> what has to run
-FORMS = [(40, 1240, 2056, 128, "grouped_dma3", "64x256"), (16, 16, 64, 384, "grouped_dma3", "64x128"),
+FORMS = [(40, 1240, 2056, 128, "grouped_dma3", "64x256"), (2, 3254, 328, 384, "grouped_dma3", "64x128"),
+         (16, 16, 64, 384, "grouped_wavesplit", "16x16"), (8, 209, 416, 128, "grouped_wavesplit", "16x32"), (40, 29, 392, 1152, "grouped_wavesplit", "16x64"),
+         (24, 1574, 128, 128, "grouped_wavesplit", "32x32"), (16, 1613, 224, 128, "grouped_wavesplit", "32x64"), (3, 545, 1544, 1152, "grouped_wavesplit", "64x64"),
          (40, 29, 2056, 128, "grouped_dma3", "64x128"),  # (more workgroups than CUs: two share one)
          (24, 1233, 2056, 384, "grouped_dma3", "128x256"), (16, 2075, 2056, 384, "grouped_dma3", "128x256"),
          (1, 1695, 2056, 640, "grouped_dma3", "128x128"), (24, 3078, 768, 2048, "grouped_dma3", "128x128"),
