@@ -413,7 +413,7 @@ int launch_fp8_pp_rowcol(GemmParams& p, hipStream_t stream, const char* what);
 
 
 // Mid-M blockwise FP8 GEMM (64/128 x 256 tile, 8 waves, three LDS stages, hand-issued direct-to-LDS loads);
-// gemm_fp8_dma3.hip.  Needs 16-byte aligned rows, K % 128 == 0, row offsets below 4 GiB.  dma3_plan() gives the split it
+// gemm_fp8_dma3.hip.  Needs 16-byte aligned rows, K % 128 == 0 (K % 16 == 0 unsplit where only the epilogue scales), row offsets below 4 GiB.  dma3_plan() gives the split it
 // wants; the caller sets p.splits, p.kb_per_split and p.ws accordingly.
 // The tile shapes it is built with, tokens x channels.
 struct TileSize {
@@ -453,9 +453,11 @@ inline bool writes_through(int64_t rows, int64_t channels) { return rows * chann
 // tokens 12.3 / 13.2 and 14.3 / 19.8, 7168 -> 12288 at 8 and 128 18.7 / 19.3, 33.3 / 36.7 (from memory, 16 to 96 in turn, 0.92 to 0.97 for one
 // tile of 64 tokens).  Not where several token tiles fetch the weight (18432 -> 7168 at 256 62.8 / 65.1, 4096 -> 28672 at 256 46.1 / 47.2),
 // and from 65 tokens on not where K is split (18432 -> 7168 at 96 and 112, four ways, INT8 43.1 / 43.9, 45.3 / 46.7).
+// Not where the rows' pitch is no multiple of 128 bytes: consecutive K blocks then share lines, which such loads fetch twice (per-token FP8 8464 ->
+// 22208 at 1 token 47.3 with / 42.8 without, 14304 -> 19776 at 4 68.0 / 62.8, 11280 -> 30080 at 46 97.7 / 90.8; 16 linears 0.94).
 constexpr int64_t STREAMED_WEIGHT_BYTES = 100000000;
 inline bool streams_weight(const GemmParams& p) {
-  return p.tiles_m == 1 && (p.M <= 64 || p.splits == 1) && (int64_t)p.N * p.K >= STREAMED_WEIGHT_BYTES;
+  return p.tiles_m == 1 && (p.M <= 64 || p.splits == 1) && (int64_t)p.N * p.K >= STREAMED_WEIGHT_BYTES && p.ldb % KSTEP == 0;
 }
 
 // Mid-M tile, weight rows a multiple of 4096 bytes apart: with every workgroup at the same K block, all rows being fetched lie at the same place of

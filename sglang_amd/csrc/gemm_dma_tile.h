@@ -15,8 +15,11 @@
 //     nothing and count down;
 //   * s_waitcnt lgkmcnt(0) in front of the barrier: the fragments of block k have left its stage;
 //   * nothing else in the loop counts in vmcnt (weight-block scales come by scalar loads).
-// Requires K % 128 == 0, 16-byte aligned rows and row offsets below 4 GiB; AR_F32 / AR_UE8M0 also token scales laid out
-// M-major with a pitch that is a multiple of four words.
+// Requires 16-byte aligned rows and row offsets below 4 GiB; AR_F32 / AR_UE8M0 also K % 128 == 0 and token scales laid out M-major
+// with a pitch that is a multiple of four words; AR_UNIT / AR_INT8 K % 128 == 0, or K % 16 == 0 in a kernel of its own (RAGGED, K not
+// split): chunks past a row's end repeat its last one, and the last block's token fragments are cleared there before they are
+// multiplied, so a weight row meets nothing but its own values.  One subtraction a load; what it costs is lines: rows no multiple of
+// 128 bytes apart share them between K blocks (per-token FP8 94 tokens 5440 -> 36352 60, 5504 -> 36352 51 us; 102 on the generic kernel).
 #pragma once
 
 #include <utility>
@@ -79,9 +82,10 @@ struct TileShape {
 // One BM x BN output tile at (m0, n0), K blocks of split `split`, by the whole workgroup.
 // AR_UE8M0: p.sa / p.sb point to packed exponent words: token word (m, kw) at sa[kw * sa_sk + m], channel word (n, kw) at
 // sb[kw * sb_sk + n * sb_sn], byte kb & 3 of word kb >> 2 belongs to K block kb.
-template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM, bool ROTATES>
+template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM, bool ROTATES, bool RAGGED = false>
 __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, int split) {
   using T = TileShape<AR, BM, BN>;
+  static_assert(!RAGGED || ((AR == AR_UNIT || AR == AR_INT8) && !SPLIT && !ROTATES), "the last K block is multiplied last");
   static_assert(S >= 3 && S * (T::STAGE_BYTES + BM * 4) <= 160 * 1024, "the stages must fit the CU's LDS");
   constexpr int MT = T::MT, NT = T::NT, SB = T::SB, LOADS = T::LOADS, WM = T::WM;
   using AccT = typename std::conditional<AR == AR_INT8, int, float>::type;
@@ -111,6 +115,8 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
                          : (uint32_t)((int64_t)min(n0 + row - BM, p.N - 1) * p.ldb + chunk_byte);
     }
   }
+  const int tail = p.K - (p.kb_total - 1) * KSTEP;  // bytes of the last K block
+  const uint32_t past_end = RAGGED ? (uint32_t)max((((lane & 7) ^ (lane >> 3)) - (tail / 16 - 1)) * 16, 0) : 0u;  // of it, where its row ends
   const int last_group = __builtin_amdgcn_readfirstlane(min((T::ROW_LOADS - 1) * 8 + wave, T::GROUPS - 1));
   // matrix of the wave's row group in the load that covers both kinds of rows (BM not a multiple of 64)
   const bool mixed_tokens = __builtin_amdgcn_readfirstlane(BM / 64 * 8 + wave < BM / 8);
@@ -135,11 +141,12 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
       const int group = i * 8 + 8 <= T::GROUPS ? i * 8 + wave : last_group;
       const uint8_t* base = (i * 8 + 8 <= BM / 8 ? p.a : i * 8 >= BM / 8 ? p.b : mixed_base) + (uint64_t)kb * KSTEP;
       asm volatile("" : "+s"(base));
+      const uint32_t off = RAGGED ? goff[i] - (kb == kb_last ? past_end : 0u) : goff[i];
       const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)t_stage + (uint32_t)(st * T::STAGE_BYTES + group * 8 * KSTEP);
       if (STREAM && i * 8 >= BM / 8)  // (weight rows only)
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds_addr) : "memory");
       else
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(base), "s"(lds_addr) : "memory");
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory");
     } else if constexpr (T::SCALED) {
       // BM / 32 lanes fetch 16 bytes each (a 4-byte-per-lane load in this stream costs far more than its size).  exec is
       // narrowed and restored inside the statement.  Packed exponents: one row of words per four K blocks, fetched again for
@@ -239,6 +246,15 @@ __device__ __forceinline__ void dma_tile(const GemmParams& p, int m0, int n0, in
       for (int b = 0; b < SB; ++b) w_exp[b] = in_vgpr((int)(__float_as_uint(sbv[b]) >> shift));
 #pragma unroll
       for (int j = 0; j < MT; ++j) sc[j][0] = __uint_as_float(__float_as_uint(tsc[CUR][j]) >> shift);
+    }
+    if constexpr (RAGGED && !FILL) {  // (the last block is among those that request nothing any more)
+      const int valid = kb == kb_last ? tail : KSTEP;
+      const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        if (16 * q >= valid) tok[CUR][j].lo = z;
+        if (64 + 16 * q >= valid) tok[CUR][j].hi = z;
+      }
     }
     __builtin_amdgcn_sched_barrier(0);  // the waits for this block's scales come before the scalar load of the next one's
     load_sb(kb + 1);
@@ -409,17 +425,17 @@ constexpr int stages_of(int bm, int bn, bool own_cu) {
   return bm + bn == 192 ? (own_cu ? 6 : 3) : bm + bn == 224 ? 5 : bm + bn <= 288 ? 4 : 3;
 }
 
-template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM, bool ROTATES>
+template <Arith AR, int BM, int BN, bool SPLIT, int S, bool STREAM, bool ROTATES, bool RAGGED = false>
 __global__ __launch_bounds__(T_THREADS) __attribute__((amdgpu_waves_per_eu(BM + BN == 192 && S == 3 ? 4 : 2))) void gemm_dma_kernel(const GemmParams p) {
   const TileCoord tc = tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n);
-  dma_tile<AR, BM, BN, SPLIT, S, STREAM, ROTATES>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
+  dma_tile<AR, BM, BN, SPLIT, S, STREAM, ROTATES, RAGGED>(p, tc.tile_m * BM, tc.tile_n * BN, tc.split);
 }
 
 template <Arith AR, int BM, int BN>
 int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
-  p.rotate_k = rotates_k(p.N, p.K, p.ldb);
+  p.rotate_k = p.K % KSTEP == 0 && rotates_k(p.N, p.K, p.ldb);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
   constexpr int OWN = stages_of(BM, BN, true), SHARED = stages_of(BM, BN, false);
   // (a kernel of its own for K loops that start in the middle: the few instructions more cost a chain of short K blocks 5 %, 16 experts of
@@ -431,6 +447,22 @@ int launch_dma_tile(GemmParams& p, hipStream_t stream, const char* what) {
   };
   const std::true_type yes;
   const std::false_type no;
+  if constexpr (AR == AR_UNIT || AR == AR_INT8) {
+    if (p.K % KSTEP != 0) {
+      const auto launch_ragged = [&](auto streamed) {
+        constexpr bool STREAM = decltype(streamed)::value;
+        if (OWN != SHARED && (int64_t)p.tiles_m * p.tiles_n > NUM_CUS) launch_kernel((gemm_dma_kernel<AR, BM, BN, false, SHARED, STREAM, false, true>), grid, dim3(T_THREADS), 0, stream, p);
+        else launch_kernel((gemm_dma_kernel<AR, BM, BN, false, OWN, STREAM, false, true>), grid, dim3(T_THREADS), 0, stream, p);
+      };
+      if (p.splits != 1) {
+        set_error("%s: the mid-M tile does not split a K of parts of blocks", what);
+        return MI355_ERR_UNSUPPORTED;
+      }
+      if (BM == 64 && streams_weight(p)) launch_ragged(std::integral_constant<bool, BM == 64>{});
+      else launch_ragged(no);
+      return check_launch(what);
+    }
+  }
   const auto launch_split = [&](auto split) {
     const std::integral_constant<bool, !decltype(split)::value || BM == 64> may_stream;
     if (may_stream && streams_weight(p)) launch(split, may_stream, yes);

@@ -613,7 +613,7 @@ Route uncached_run_route(GemmKind kind, int64_t M, int64_t N, int64_t K, int64_t
   if (!aligned || M * lda >= (1ll << 32) || N * ldb >= (1ll << 32)) return r;
   TileChoice c{TF_NONE, 0, 0, 1, 0.0};
   if (K % KSTEP != 0) {
-    if (kind == GK_UNIT || kind == GK_INT8) c = choose_ragged_tile(M, N, K);
+    if (kind == GK_UNIT || kind == GK_INT8) c = choose_ragged_tile(M, N, K, r.kernel == RK_PINGPONG);
   } else if (M <= 16) {
     c = choose_decode_tile(kind, M, N, K, TileChoice{r.kernel == RK_DMA3 ? TF_DMA : TF_NONE, r.bm, r.bn, r.splits, 0.0}, r.kernel == RK_WAVESPLIT, r.kernel == RK_DECODE);
     if (!conforming && c.family == TF_DMA) c = choose_limited_decode_tile(kind, M, N, K, r.kernel == RK_DMA3, r.kernel == RK_WAVESPLIT, r.kernel == RK_DECODE);
@@ -841,7 +841,7 @@ std::vector<std::string> tile_constant_names() {
                 "cold_ws_channel", "cold_ws_token", "cold_ws_stream", "cold_ws_stream_us", "cold_ws_norm", "cold_pp_tile", "cold_pp_block", "cold_pp_busy", "cold_cached"});
   }
   add("limits.", {"margin", "two_phase_margin", "large_weight_margin", "large_weight_max_tokens", "mid_wavesplit_max_weight", "ragged_max_weight",
-                  "ragged_max_factor", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
+                  "ragged_max_factor", "ragged_min_kblocks", "ragged_two_phase_kblocks", "ragged_min_workgroups", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
                   "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_rounds_margin", "streamed_min_weight", "streamed_two_tokens_min_kblocks", "small_min_tokens", "small_max_channels", "small_max_tokens_values", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});

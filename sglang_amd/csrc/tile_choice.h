@@ -77,6 +77,7 @@ static_assert(sizeof(MID_TILES) / sizeof(MID_TILES[0]) == 13, "the tables above 
 struct TileLimits {
   double margin = 0.95, two_phase_margin = 0.90, large_weight_margin = 0.85, large_weight_max_tokens = 64.0;
   double mid_wavesplit_max_weight = 100e6, ragged_max_weight = 100e6, ragged_max_factor = 2.0;
+  double ragged_min_kblocks = 2.0, ragged_two_phase_kblocks = 32.0, ragged_min_workgroups = 0.5 * NUM_CUS;
   double wavesplit_max_tokens_bytes = 16e6, wavesplit_long_k = 9216.0, wavesplit_long_k_max_tokens_bytes = 10e6, few_workgroups_max_tokens = 128.0;
   double decode_min_kblocks = 16.0, decode_padded_max_weight = 400e6, decode_max_weight = 140e6, decode_few_tokens_max_weight = 100e6;
   double decode_one_turn_min_kblocks = 30.0, decode_one_turn_kblocks = 32.0, decode_one_turn_max_channels = 16384.0, decode_one_turn_max_tokens = 10.0;
@@ -388,16 +389,6 @@ TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const
   return r.us < tile_model().limits.resident_margin * (c.family != TF_NONE ? c.us : base_us) ? r : c;
 }
 
-// K not a multiple of 128 (scales in the epilogue only): the wave-split tile against the generic kernel, which takes at least
-// twice as long as the mid-M tile would (K = 5920 -> N = 8320 at 90 tokens INT8: 42 against 18 us); not for the largest weights,
-// which the tile fetches once per 64 tokens (K = 16016 -> N = 26880 at 256 tokens 320 against 260 us).
-TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K) {
-  const TileTimes& t = tile_model().plain;
-  const TileLimits& l = tile_model().limits;
-  const TileChoice ws = best_wavesplit_tile(t, M, N, K);
-  return (double)(N * K) <= l.ragged_max_weight && ws.us < l.ragged_max_factor * best_dma_tile(t, M, N, K).us ? ws : TileChoice{TF_NONE, 0, 0, 1, 0.0};
-}
-
 // Up to 16 tokens on a weight large enough to be loaded as a stream (streams_weight): the wave-split and the mid-M tile have such loads, the
 // register wave-split kernel and the streaming kernel, whose instructions fetch parts of lines, lose by them.  Fitted to 290 linears
 // (100 to 480 million weights): 3 % root mean square; what it chooses takes 1.01 of the best one's time.
@@ -442,6 +433,40 @@ TileChoice choose_streamed_tile(int64_t M, int64_t N, int64_t K, const TileChoic
   for (int bn = 128; bn <= 256; bn += 64)  // (in one round: 2048 -> 67232 at 13 in 351 workgroups 34.6, the register kernel 29.6)
     if (ceil_div(N, bn) <= (bn == 128 ? 2 : 1) * NUM_CUS) consider(TF_DMA, 64, bn, streamed_mid_us(M, N, K, bn));
   return best;
+}
+
+// K not a multiple of 128 (scales in the epilogue only), us before / after where it says no more (the generic kernel, or the wave-split
+// tile wherever it modelled below twice the mid-M tile, before).
+// Above 16 tokens the wave-split tile, or the mid-M tile with K unsplit where it models 5 % faster: per-token FP8 149 tokens 832 -> 8832
+// 12.9 / 8.9, 94 tokens 5440 -> 36352 102 / 60, 236 tokens 5216 -> 15360 54 / 38, 2000 tokens 4112 -> 2048 65 / 34; INT8 426 tokens 1504 -> 27200
+// 77 / 35, 173 tokens 608 -> 18816 22.7 / 10.3, 4096 tokens 4176 -> 4096 230 / 87.  The mid-M tile only from half a chip of workgroups on: with fewer
+// the generic kernel's K split wins (generic / mid-M tile: 94 workgroups 16688 -> 6016 at 65 64.7 / 79.8, 102 8016 -> 13000 at 33
+// 46.6 / 50.0, 76 10480 -> 9656 at 17 40.0 / 57.2; 157 10000 -> 10016 at 200 102.5 / 58.6).  `two_phase`: FP8 where the 256 x 256 tile with a
+// promotion per block runs otherwise; it stays for long K (that / mid-M tile: 4096 tokens 7184 -> 18432 596 / 679, 2048 tokens 7184 ->
+// 36864 618 / 676, 4112 -> 28672 315 / 319; 4096 tokens 2064 -> 18432 258 / 229, 1040 -> 16384 152 / 120, 3000 tokens 720 -> 12288 86 / 57).  K
+// below two blocks is no layer's and stays where it was.
+// Up to 16 tokens the wave-split tile; from `streamed_min_weight` on what the weight's stream chooses: 14304 -> 19776 at 4 76.3 / 62.8, 8464 ->
+// 22208 at 1 57.6 / 42.8, 7776 -> 18688 at 9 46.8 / 39.4.
+TileChoice choose_ragged_tile(int64_t M, int64_t N, int64_t K, bool two_phase) {
+  const TileTimes& t = tile_model().plain;
+  const TileLimits& l = tile_model().limits;
+  const TileChoice none{TF_NONE, 0, 0, 1, 0.0};
+  const double weights = (double)(N * K);
+  if (M <= 16 && weights >= l.streamed_min_weight) return choose_streamed_tile(M, N, K, none);
+  const TileChoice ws = best_wavesplit_tile(t, M, N, K);
+  const bool ws_allowed = weights <= l.ragged_max_weight && ws.us < l.ragged_max_factor * best_dma_tile(t, M, N, K).us;
+  if (M > 16 && (double)ceil_div(K, KSTEP) >= l.ragged_min_kblocks) {
+    TileChoice d{TF_NONE, 0, 0, 1, ws_allowed ? l.margin * ws.us : 1e30};
+    if (two_phase && weights > l.ragged_max_weight && (double)ceil_div(K, KSTEP) > l.ragged_two_phase_kblocks) return none;
+    for (int i = 0; i < 13; ++i) {
+      const int bm = MID_TILES[i].bm, bn = MID_TILES[i].bn;
+      if ((double)(ceil_div(M, bm) * ceil_div(N, bn)) < l.ragged_min_workgroups) continue;
+      const double us = dma_tile_us(t, i, M, N, K, 1, d.us);
+      if (us < d.us) d = {TF_DMA, bm, bn, 1, us};
+    }
+    if (d.family == TF_DMA) return d;
+  }
+  return ws_allowed ? ws : none;
 }
 
 // K of up to 16 blocks on weights of up to 20 million values, which the launches bound: the tile quantizes the tokens in its one launch and takes

@@ -169,9 +169,9 @@ VARIANT_SHAPES = {
         ("dma3", 64, "whole"): (17, 57344, 512), ("dma3", 96, "split", "bn128", "deep"): (3334, 8, 5248),
         ("dma3", 96, "split", "bn192", "deep"): (2958, 264, 9344), ("dma3", 96, "split"): (263, 4136, 16640),
         ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512), ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128),
-        ("dma3", 96, "whole"): (261, 16488, 128), ("generic", 128, "aligned", "split"): (65, 25352, 912),
+        ("dma3", 96, "whole"): (261, 16488, 128), ("generic", 128, "aligned", "split"): (65, 6016, 16688),
         ("generic", 128, "aligned", "whole"): (708, 2816, 16), ("generic", 16, "aligned", "split"): (1, 8, 1024),
-        ("generic", 16, "aligned", "whole"): (1, 8, 128), ("generic", 256, "aligned", "split"): (1052, 6688, 928),
+        ("generic", 16, "aligned", "whole"): (1, 8, 128),
         ("generic", 32, "aligned", "split"): (17, 9656, 10480), ("generic", 32, "aligned", "whole"): (26, 50944, 16),
         ("generic", 64, "aligned", "split"): (33, 6016, 16688), ("generic", 64, "aligned", "whole"): (34, 33648, 16),
         ("pingpong", "kfull"): (193, 49640, 128), ("pingpong", "ktail"): (1555, 9984, 16), ("pipelined", "ktail"): (1094, 6576, 16),
@@ -205,9 +205,9 @@ VARIANT_SHAPES = {
         ("dma3", 64, "whole"): (12, 33096, 128), ("dma3", 96, "split", "bn128", "deep"): (1606, 8, 12928),
         ("dma3", 96, "split", "bn192", "deep"): (2958, 264, 9344), ("dma3", 96, "split"): (263, 4136, 16640),
         ("dma3", 96, "whole", "bn128", "deep"): (65, 18944, 512), ("dma3", 96, "whole", "bn192", "deep"): (65, 32896, 128),
-        ("dma3", 96, "whole"): (389, 10904, 128), ("generic", 128, "aligned", "split"): (65, 25352, 912),
+        ("dma3", 96, "whole"): (389, 10904, 128), ("generic", 128, "aligned", "split"): (65, 6016, 16688),
         ("generic", 128, "aligned", "whole"): (708, 2816, 16), ("generic", 16, "aligned", "split"): (1, 8, 1024),
-        ("generic", 16, "aligned", "whole"): (1, 8, 128), ("generic", 256, "aligned", "split"): (1052, 6688, 928),
+        ("generic", 16, "aligned", "whole"): (1, 8, 128),
         ("generic", 256, "aligned", "whole"): (1094, 6576, 16), ("generic", 32, "aligned", "split"): (17, 9656, 10480),
         ("generic", 32, "aligned", "whole"): (26, 50944, 16), ("generic", 64, "aligned", "split"): (33, 6016, 16688),
         ("generic", 64, "aligned", "whole"): (34, 33648, 16), ("pingpong", "kfull"): (223, 49272, 128),
