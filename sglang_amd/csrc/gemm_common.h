@@ -558,7 +558,7 @@ int launch_fp8_wavesplit_tile_ue8m0(GemmParams& p, int bm, int bn, hipStream_t s
 int launch_fp8_wavesplit_tile_unit(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
 int launch_int8_wavesplit_tile(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);
 // The same with a quantizer for the tokens inside (p.x16 / p.ldx / p.x_dtype, p.x_by_reciprocal; p.a and p.sa are not read): per 1 x 128
-// group, or per token for the unit-scale FP8 and the INT8 kernel.  K % 128 == 0, few values in a tile's tokens.
+// group (K % 128 == 0), or per token for the unit-scale FP8 and the INT8 kernel (K % 16 == 0).  Few values in a tile's tokens.
 constexpr int WAVESPLIT_QUANT_VALUES = 8 * 64 * 10 * 8;  // of the tokens of one tile
 constexpr TileSize WAVESPLIT_QUANT_TILES[] = {{16, 16}, {16, 32}, {16, 64}, {32, 32}, {32, 64}};
 int launch_fp8_wavesplit_tile_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what);

@@ -63,31 +63,42 @@ __device__ __forceinline__ float amax8(const u32x4& raw) {
 
 // The tokens m0 .. m0 + rows - 1, at most BM, whose rows lie one behind the other.  Piece c (16 bytes of input, 8 values) of them goes to
 // thread c % NT; 16 consecutive pieces are a group, in the 16 lanes of a DPP row.  Codes go to codes[row * (K + 16) + k] (rows 16 bytes
-// longer than K, so that a fragment's rows do not share banks), scales to token_scale (one per token, or per token and K block: row *
+// longer than K in whole blocks, so that a fragment's rows do not share banks), scales to token_scale (one per token, or per token and K block: row *
 // kb_total + kb, which is c / 16; exponents for UE8M0).  `request` is called behind the loads of the raw values: it requests the first weight
 // blocks and waits until only those are outstanding.  Ends with a barrier that does not wait for them.
 // Bound by its vector instructions, about 70 a piece and lane: flat addresses, one multiplication for the row, one median for the clamp.  With
 // row and column of a piece found by a loop and clamps behind a quieting maximum it was 130; whole linears, us, before / now: block FP8
 // 1152 -> 256 at 16 tokens 6.1 / 4.7, 1536 -> 24576 at 8 11.9 / 10.8; packed exponents 1280 -> 1920 at 15 5.8 / 4.8; INT8 1408 -> 704 at 12
 // 5.8 / 4.9; per-token FP8 1152 -> 17280 at 10 11.8 / 10.75.
-template <bool IS_FP8, bool UE8M0, TokenQuant TQ, int NV, int NT, int BM, class Request>
+// PARTS: K is a multiple of 16 only (TQ_ROW).  Rows then take whole blocks of pieces all the same; those past a row's end, loaded from where the
+// next row begins or the last one ends, stay out of its maximum and become zeros, which the weight's repeated bytes meet (6 instructions a piece;
+// graphs, us, a quantizer launch in front / this: INT8 928 -> 2304 at 8 tokens 5.0 / 4.0, 960 -> 320 at 406 6.4 / 5.4; per-token FP8 576 -> 896 at 13
+// 5.0 / 4.2, 1440 -> 4544 at 6 5.45 / 4.8; eager 8.3 / 5.6, 7.9 / 5.7, 8.4 / 5.2, 7.9 / 5.5).
+template <bool IS_FP8, bool UE8M0, TokenQuant TQ, int NV, int NT, int BM, bool PARTS = false, class Request>
 __device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int rows, uint8_t* codes, float* token_scale, float* row_max, Request request) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int total = __builtin_amdgcn_readfirstlane(rows * (p.K >> 3));
+  static_assert(!PARTS || TQ == TQ_ROW, "groups are whole");
+  const int total = __builtin_amdgcn_readfirstlane(PARTS ? rows * p.kb_total * 16 : rows * (p.K >> 3));
   const uint8_t* x = reinterpret_cast<const uint8_t*>(p.x16) + (int64_t)m0 * p.K * 2;
   static_assert(NV * NT / 16 <= 512, "row_of: groups below 2^9 and a 20-bit inverse");
   // the row of piece c, exact for c / 16 * kb_total < 2^20; any row past the last one for pieces past the end
   const uint32_t inverse = __builtin_amdgcn_readfirstlane(((1u << 20) + (uint32_t)p.kb_total - 1u) / (uint32_t)p.kb_total);
   auto piece = [&](int i) { return (int)threadIdx.x + i * NT; };
   auto row_of = [&](int i) { return (int)(__umul24((uint32_t)piece(i) >> 4, inverse) >> 20); };
+  const uint32_t missing = PARTS ? (uint32_t)(p.kb_total * KSTEP - p.K) * 2u : 0u, last_piece = (uint32_t)(rows * p.K) * 2u - 16u;  // bytes
+  auto offset = [&](int i) {
+    if constexpr (PARTS) return min((uint32_t)piece(i) * 16u - __umul24((uint32_t)row_of(i), missing), last_piece);
+    else return (uint32_t)min(piece(i), total - 1) * 16u;
+  };
+  auto in_row = [&](int i) { return !PARTS || piece(i) - row_of(i) * p.kb_total * 16 < p.K >> 3; };
   // (NV pieces per thread, all of them always requested: a load under a condition could leave the compiler a copy to make
   // while it is in flight; pieces past the end repeat the last one and are dropped)
   u32x4 raw[NV];
   asm volatile("" : "+s"(x));
 #pragma unroll
   for (int i = 0; i < NV; ++i)
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(raw[i]) : "v"((uint32_t)min(piece(i), total - 1) * 16u), "s"(x) : "memory");
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(raw[i]) : "v"(offset(i)), "s"(x) : "memory");
   const bool given = TQ == TQ_ROW && IS_FP8 && p.x_scale != nullptr;  // one scale for all tokens: per_tensor_quant.hip's arithmetic
   float given_scale = 1.0f;
   if constexpr (TQ == TQ_ROW) {
@@ -112,7 +123,7 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
         if (i * NT + wave * 64 < total) {
-          const float m = row16_max(amax8<BF16>(raw[i]));
+          const float m = row16_max(in_row(i) ? amax8<BF16>(raw[i]) : 0.f);
           if ((lane & 15) == 0 && piece(i) < total) atomicMax(reinterpret_cast<uint32_t*>(row_max) + row_of(i), __float_as_uint(m));  // (m >= 0: ordered as bits)
         }
       }
@@ -135,6 +146,7 @@ __device__ __forceinline__ void quantize_tokens(const GemmParams& p, int m0, int
         const int row = row_of(i);
         if constexpr (TQ == TQ_ROW) {
           q8 = codes_of_row<IS_FP8, BF16>(raw[i], row_max[min(row, BM - 1)]);
+          if (!in_row(i)) q8 = u32x2{0u, 0u};
         } else {
           float sc;
           if constexpr (UE8M0) {

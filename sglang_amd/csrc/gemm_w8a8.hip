@@ -1257,11 +1257,15 @@ bool wavesplit_quant_preferred(WavesplitQuant kind, int64_t M, int64_t N, int64_
 bool wavesplit_quant_operands(const void* x, int x_dtype, const void* w, int64_t ldw) {
   return x_dtype != MI355_F32 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
 }
+// The quantizer per token also takes a K in parts of blocks; 1 x 128 groups are whole.
+bool tile_quant_takes(WavesplitQuant quant, int64_t K) {
+  return K % (quant == WavesplitQuant::TOKEN_FP8 || quant == WavesplitQuant::TOKEN_INT8 ? 16 : KSTEP) == 0;
+}
 // The wave-split tile quantizing the tokens itself, where the GEMM takes that tile (same sums, bit for bit): the launch saved
 // against the quantizer's work in every workgroup, v pieces per thread and round.
-bool tile_quant_preferred(const Route& run, int64_t M, int64_t N, int64_t K) {
-  if (run.kernel != RK_WAVESPLIT_TILE || M > 16 || K % KSTEP != 0) return false;
-  const int64_t pieces = M * K / 8, threads = 512, rounds = (N + (int64_t)run.bn * NUM_CUS - 1) / ((int64_t)run.bn * NUM_CUS);
+bool tile_quant_preferred(WavesplitQuant quant, const Route& run, int64_t M, int64_t N, int64_t K) {
+  if (run.kernel != RK_WAVESPLIT_TILE || M > 16 || !tile_quant_takes(quant, K)) return false;
+  const int64_t pieces = M * ((K + KSTEP - 1) / KSTEP) * (KSTEP / 8), threads = 512, rounds = (N + (int64_t)run.bn * NUM_CUS - 1) / ((int64_t)run.bn * NUM_CUS);
   return pieces <= 10 * threads && pieces * rounds <= 10 * threads;
 }
 bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
@@ -1286,9 +1290,9 @@ LinearRoute uncached_choose_linear(WavesplitQuant quant, int64_t M, int64_t N, i
   const GemmKind kind = quant == WavesplitQuant::BLOCK_F32 ? GK_F32 : quant == WavesplitQuant::BLOCK_UE8M0 ? GK_UE8M0 : quant == WavesplitQuant::TOKEN_FP8 ? GK_UNIT : GK_INT8;
   const Route run = run_route(kind, M, N, K, K, ldw, w_aligned && K % 16 == 0);
   if (!q_ok) return {LM_LAUNCH, run};
-  if (tile_quant_preferred(run, M, N, K)) return {LM_TILE, run};
-  if (M > 16 && run.kernel == RK_WAVESPLIT_TILE && K % KSTEP == 0) {
-    const TileChoice c = choose_quant_tile(kind, M, N, K, run.bm, run.bn);
+  if (tile_quant_preferred(quant, run, M, N, K)) return {LM_TILE, run};
+  if (M > 16 && run.kernel == RK_WAVESPLIT_TILE && tile_quant_takes(quant, K)) {
+    const TileChoice c = choose_quant_tile(kind, M, N, (K + KSTEP - 1) / KSTEP * KSTEP, run.bm, run.bn);
     Route r = run;
     r.bm = c.bm, r.bn = c.bn;
     if (c.family != TF_NONE) return {LM_TILE, r};
@@ -1305,7 +1309,7 @@ LinearRoute uncached_choose_linear(WavesplitQuant quant, int64_t M, int64_t N, i
     r.bm = c.bm, r.bn = c.bn, r.splits = 1, r.kb_per_split = (int)(K / KSTEP), r.aligned = true;
     r.kernel = c.family == TF_DMA ? RK_DMA3 : RK_WAVESPLIT_TILE;
     if (c.family == TF_DMA) return {producer_mode, r};
-    return {tile_quant_preferred(r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
+    return {tile_quant_preferred(quant, r, M, N, K) ? LM_TILE : LM_LAUNCH_OWN, r};
   }
   if (wavesplit_quant_preferred(quant, M, N, K, ldw)) {
     Route r{};
@@ -1336,7 +1340,7 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
 }
 int run_tile_quant(GemmParams& p, WavesplitQuant kind, const Route& run, const void* x, int x_dtype, void* stream, const char* what) {
   p.x16 = x, p.ldx = p.K, p.x_dtype = x_dtype;
-  p.kb_total = p.K / KSTEP;
+  p.kb_total = (p.K + KSTEP - 1) / KSTEP;
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (kind) {
     case WavesplitQuant::BLOCK_F32: return launch_fp8_wavesplit_tile_quant(p, run.bm, run.bn, st, what);

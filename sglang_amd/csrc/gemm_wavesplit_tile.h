@@ -60,7 +60,7 @@ __device__ __forceinline__ void wait_blocks(int blocks) {
 }
 
 // The 16 MT x 16 CT tile at (m0, n0), by the whole workgroup.
-template <Arith AR, int MT, int CT, TokenQuant TQ, int NV, bool STREAM>
+template <Arith AR, int MT, int CT, TokenQuant TQ, int NV, bool STREAM, bool PARTS = false>
 __device__ __forceinline__ void wavesplit_tile(const GemmParams& p, int m0, int n0) {
   using T = WavesplitTile<AR, MT, CT, TQ>;
   constexpr int R = T::R, LOADS = T::LOADS, BM = T::BM, W = WST_WAVES;
@@ -132,7 +132,7 @@ __device__ __forceinline__ void wavesplit_tile(const GemmParams& p, int m0, int 
   if constexpr (TQ == TQ_NONE) {
     request_first();
   } else {
-    quantize_tokens<AR != AR_INT8, AR == AR_UE8M0, TQ, NV, 64 * W, BM>(p, m0, rows, codes, token_scale, row_max, [&] {
+    quantize_tokens<AR != AR_INT8, AR == AR_UE8M0, TQ, NV, 64 * W, BM, PARTS>(p, m0, rows, codes, token_scale, row_max, [&] {
       request_first();
       wait_blocks<LOADS>(min(blocks, R));
     });
@@ -152,7 +152,7 @@ __device__ __forceinline__ void wavesplit_tile(const GemmParams& p, int m0, int 
         tf[t].lo = lds16(st + lo, t * 2048), tf[t].hi = lds16(st + hi, t * 2048);
       } else {
         const int row = min(16 * t + l16, rows - 1);  // (past the last token: results that are not stored)
-        const uint8_t* src = codes + row * (p.K + 16) + kb * KSTEP + q * 16;
+        const uint8_t* src = codes + row * ((PARTS ? p.kb_total * KSTEP : p.K) + 16) + kb * KSTEP + q * 16;
         tf[t].lo = *reinterpret_cast<const u32x4*>(src), tf[t].hi = *reinterpret_cast<const u32x4*>(src + 64);
         if constexpr (TQ == TQ_GROUP) ts[t] = token_scale[row * p.kb_total + kb];
       }
@@ -253,13 +253,13 @@ __device__ __forceinline__ void wavesplit_tile(const GemmParams& p, int m0, int 
   }
 }
 
-template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2, bool STREAM = false>
+template <Arith AR, int MT, int CT, TokenQuant TQ = TQ_NONE, int NV = 2, bool STREAM = false, bool PARTS = false>
 __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void wavesplit_tile_kernel(const GemmParams p) {
   // consecutive workgroups of an XCD take the token tiles of the same channels
   int bid = blockIdx.x;
   const int per_xcd = (int)gridDim.x >> 3;
   if (bid < per_xcd * 8) bid = (bid & 7) * per_xcd + (bid >> 3);
-  wavesplit_tile<AR, MT, CT, TQ, NV, STREAM>(p, (bid % p.tiles_m) * (16 * MT), (bid / p.tiles_m) * (16 * CT));
+  wavesplit_tile<AR, MT, CT, TQ, NV, STREAM, PARTS>(p, (bid % p.tiles_m) * (16 * MT), (bid / p.tiles_m) * (16 * CT));
 }
 
 template <Arith AR, int MT, int CT>
@@ -292,15 +292,19 @@ int launch_wavesplit_tile_quant_inst(GemmParams& p, hipStream_t stream, const ch
   p.tiles_m = (p.M + 16 * MT - 1) / (16 * MT), p.tiles_n = (p.N + 16 * CT - 1) / (16 * CT);
   p.splits = 1;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * WST_WAVES);
-  const int64_t pieces = (int64_t)min(p.M, 16 * MT) * p.K / 8;
-  const auto launch = [&](auto streamed) {
-    constexpr bool STREAM = decltype(streamed)::value;
-    if (MT == 1 && pieces <= 2 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, MT == 1 ? 2 : 5, STREAM>), grid, block, 0, stream, p);
-    else if (pieces <= (MT == 1 ? 4 : 5) * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, MT == 1 ? 4 : 5, STREAM>), grid, block, 0, stream, p);
-    else launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, WS_QUANT_VECTORS, STREAM>), grid, block, 0, stream, p);
+  const int64_t pieces = (int64_t)min(p.M, 16 * MT) * p.kb_total * (KSTEP / 8);
+  const auto launch = [&](auto streamed, auto parts) {
+    constexpr bool STREAM = decltype(streamed)::value, PARTS = decltype(parts)::value;
+    if (MT == 1 && pieces <= 2 * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, MT == 1 ? 2 : 5, STREAM, PARTS>), grid, block, 0, stream, p);
+    else if (pieces <= (MT == 1 ? 4 : 5) * 64 * WST_WAVES) launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, MT == 1 ? 4 : 5, STREAM, PARTS>), grid, block, 0, stream, p);
+    else launch_kernel((wavesplit_tile_kernel<AR, MT, CT, TQ, WS_QUANT_VECTORS, STREAM, PARTS>), grid, block, 0, stream, p);
   };
-  if (MT == 1 && streams_weight(p)) launch(std::integral_constant<bool, MT == 1>{});
-  else launch(std::false_type{});
+  const auto launch_parts = [&](auto streamed) {
+    if (p.K % KSTEP != 0) launch(streamed, std::integral_constant<bool, TQ == TQ_ROW>{});
+    else launch(streamed, std::false_type{});
+  };
+  if (MT == 1 && streams_weight(p)) launch_parts(std::integral_constant<bool, MT == 1>{});
+  else launch_parts(std::false_type{});
   return check_launch(what);
 }
 template <Arith AR, TokenQuant TQ, size_t... I>
@@ -314,7 +318,8 @@ int launch_wavesplit_tile_quant_of(GemmParams& p, int bm, int bn, hipStream_t st
 }
 template <Arith AR, TokenQuant TQ>
 int launch_wavesplit_tile_quant(GemmParams& p, int bm, int bn, hipStream_t stream, const char* what) {
-  if (p.x16 == nullptr || p.ldx != p.K || p.K % KSTEP != 0 || (int64_t)min(p.M, bm) * p.K > WST_QUANT_VALUES) {
+  if (p.x16 == nullptr || p.ldx != p.K || p.K % (TQ == TQ_ROW ? 16 : KSTEP) != 0 || p.kb_total != (p.K + KSTEP - 1) / KSTEP ||
+      (int64_t)min(p.M, bm) * p.kb_total * KSTEP > WST_QUANT_VALUES) {
     set_error("%s: the fused quantizer of the wave-split tile takes few unquantized tokens", what);
     return MI355_ERR_UNSUPPORTED;
   }

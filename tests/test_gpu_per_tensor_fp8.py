@@ -117,7 +117,7 @@ def test_apply_fp8_linear_paths(gpu, oracle, path):
 @pytest.mark.parametrize("M,N,K,quantizer,kernel", [(16, 2176, 2176, "fused", "wavesplit_tile"), (1, 576, 7168, "fused", "wavesplit_tile"),
                                                     (143, 24, 640, "fused", "wavesplit_tile"), (40, 3712, 640, "fused", "wavesplit_tile"),
                                                     (1, 16512, 3840, "fused", "decode_wavesplit"), (4, 7168, 2048, "fused", "decode_wavesplit"),
-                                                    (17, 2816, 7168, "launch", "wavesplit_tile"), (40, 1032, 1040, "launch", "wavesplit_tile")])
+                                                    (17, 2816, 7168, "launch", "wavesplit_tile"), (40, 1032, 1040, "fused", "wavesplit_tile")])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_static_scale_inside_the_gemm(gpu, M, N, K, quantizer, kernel, dtype):
     """apply_fp8_linear with a static scale against quantizer and GEMM: the same codes and sums, so the same bits; values beyond the scale's

@@ -41,3 +41,50 @@ def test_parts_of_blocks_exact(gpu, shape, tile):
     assert out[:, 5].isnan().all()
     keep = torch.arange(N, device=gpu) != 5
     assert torch.equal(out[:, keep], want[:, keep])
+
+
+# last blocks of 16 to 112 values, one block, rows that share a DPP row of sixteen pieces with no other, several token tiles, the most values a
+# tile quantizes (40960), every tile height
+QUANTIZED = [(1, 136, 16), (3, 264, 112), (16, 576, 144), (5, 1032, 4112), (16, 2056, 2416), (16, 16400, 304), (45, 264, 272), (72, 640, 1472), (33, 4104, 1008), (16, 520, 2544),
+             (700, 320, 368), (100, 4000, 272)]
+
+
+@pytest.mark.parametrize("M,N,K", QUANTIZED)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_quantizer_inside_parts_of_blocks(gpu, M, N, K, dtype):
+    """One launch against quantizer and GEMM entry point: the same codes, scales and sums, so the same bits, with zeros, infinities and NaN
+    in some rows and at their ends; a static scale of zero too, whose codes are all at the limit."""
+    from sglang_amd import _lib, ops
+    from sglang_amd.fp8_kernel import sglang_per_token_quant_fp8, static_quant_fp8
+    from sglang_amd.fp8_utils import apply_fp8_linear
+    from sglang_amd.int8_kernel import per_token_quant_int8
+    from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
+
+    for kind in ("token_fp8", "int8"):
+        plan = _lib.linear_plan(kind, M, N, K)
+        print(f"case {kind} {(M, N, K)} {plan}", flush=True)
+        assert plan["quantizer"] == "fused"
+    bits = lambda t: torch.where(t.isnan(), torch.zeros_like(t), t).view(torch.int16)
+    whole = (K + 127) // 128 * 128
+    x = make_activation(M, whole, seed=M + N, dtype=dtype)[:, :K].contiguous()
+    if M > 2:
+        x[0], x[M // 2, 5], x[1, K - 1] = 0, float("inf"), float("nan")
+    x[M - 1, K - 1] = 300  # the row's maximum where it ends
+    xg = x.to(gpu)
+    w = make_fp8_weight(N, whole, seed=K)[0][:, :K].contiguous().to(gpu)
+    scale = torch.rand(N, generator=torch.Generator().manual_seed(K)).to(gpu) * 0.01 + 1e-3
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).to(dtype).to(gpu)
+    q, s = sglang_per_token_quant_fp8(xg)
+    out, two = ops.fp8_per_token_linear(xg, w.t(), scale, bias, dtype), ops.fp8_scaled_mm(q, w.t(), s, scale, dtype, bias)
+    assert torch.equal(bits(out), bits(two)) and torch.equal(out.isnan(), two.isnan())
+    for given in (0.5, 0.0):
+        s = torch.tensor([given], device=gpu)
+        q, rows = static_quant_fp8(xg, s, repeat_scale=True)
+        out, two = apply_fp8_linear(xg, w.t(), scale, s, bias=bias), ops.fp8_scaled_mm(q, w.t(), rows, scale, dtype, bias)
+        assert torch.equal(bits(out), bits(two)) and torch.equal(out.isnan(), two.isnan())
+    if M > 2:
+        xg[M // 2, 5] = xg[1, K - 1] = 1  # (a row with an infinity has no INT8 codes)
+    q, s = per_token_quant_int8(xg)
+    w8, ws = make_int8_weight(N, whole, seed=K)
+    w8, ws = w8[:, :K].contiguous().to(gpu).t(), ws.to(gpu)
+    assert torch.equal(bits(ops.int8_linear(xg, w8, ws, bias, dtype)), bits(ops.int8_scaled_mm(q, w8, s, ws, dtype, bias)))
