@@ -11,7 +11,7 @@
 //      its number of records; sizes are clamped into the stacked matrix, so inconsistent routing data cannot make a later kernel read
 //      or write out of bounds.  The other workgroups re-lay the token scales out M-major (what the direct-to-LDS GEMMs read with
 //      16-byte loads), every expert padded to start on a whole quad of rows; they find the experts of their 32 rows themselves and
-//      wait for nobody (two launches, one after the other, took 9.6 us with the gap between them, this one 5);
+//      wait for nobody (two launches, one after the other, took 9.6 us with the gap between them, this one 4);
 //   2. fp8_grouped_pp_kernel (gemm_fp8_pp.hip), the two-phase 256 x 256 tile kernel, over the first table, then
 //      fp8_grouped_dma_kernel (gemm_fp8_dma3.hip), the mid-M tile of 64 or 128 tokens x 128 or 256 channels, over the second:
 //      one workgroup per (token tile, channel tile).  The first launch is left out when no expert can have more than
@@ -59,26 +59,31 @@ struct GroupedTables {
 __device__ void grouped_plan(const int32_t* problem_sizes, const int32_t* expert_offsets, const GroupedTables& g) {
   const int E = g.E, bm = g.bm, max_big = g.max_big, max_small = g.max_small;
   v4i *big_tiles = g.big_tiles, *small_tiles = g.small_tiles;
-  __shared__ int scan_b[256], scan_s[256];
+  __shared__ int wave_b[4], wave_s[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int base_b = 0, base_s = 0;
   for (int c = 0; c < E; c += 256) {
     const int e = c + (int)threadIdx.x;
     const ExpertTiles t = expert_tiles(problem_sizes, expert_offsets, e, E, g.total_m, bm, g.use_big);
-    scan_b[threadIdx.x] = t.big, scan_s[threadIdx.x] = t.small;
-    __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {  // inclusive prefix sums
-      const int vb = (int)threadIdx.x >= d ? scan_b[threadIdx.x - d] : 0;
-      const int vs = (int)threadIdx.x >= d ? scan_s[threadIdx.x - d] : 0;
-      __syncthreads();
-      scan_b[threadIdx.x] += vb, scan_s[threadIdx.x] += vs;
-      __syncthreads();
+    int sum_b = t.big, sum_s = t.small;  // inclusive, within the wave
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int vb = __shfl_up(sum_b, d), vs = __shfl_up(sum_s, d);
+      if (lane >= d) sum_b += vb, sum_s += vs;
     }
-    const int first_b = base_b + scan_b[threadIdx.x] - t.big, first_s = base_s + scan_s[threadIdx.x] - t.small;
+    if (lane == 63) wave_b[wave] = sum_b, wave_s[wave] = sum_s;
+    __syncthreads();
+    int first_b = base_b + sum_b - t.big, first_s = base_s + sum_s - t.small;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int nb = wave_b[w], ns = wave_s[w];
+      base_b += nb, base_s += ns;
+      if (w < wave) first_b += nb, first_s += ns;
+    }
     for (int j = 0; j < t.big; ++j)
       if (first_b + j < max_big) big_tiles[1 + first_b + j] = v4i{e, t.row0, t.rows, j * BIG};
     for (int j = 0; j < t.small; ++j)
       if (first_s + j < max_small) small_tiles[1 + first_s + j] = v4i{e, t.row0, t.rows, t.small_first + j * bm};
-    base_b += scan_b[255], base_s += scan_s[255];
     __syncthreads();
   }
   // record 0 of each table: how many follow (consistent routing data never exceeds the bounds)
@@ -90,6 +95,10 @@ __device__ void grouped_plan(const int32_t* problem_sizes, const int32_t* expert
 
 // Workgroup (x, y) < (chunks, K blocks / 32): out[kb * pitch + col(e) + m] = sa[(row0 + m) * sa_sm + kb * sa_sk] for 32 stacked rows x 32
 // K blocks, col(e) = ((row0 + 3) & ~3) + 4 * e, through LDS so that both sides are contiguous.  The last x: the tables.
+// Bound by its chain of latencies: routing data and scales are requested together, an expert leaves two edges in LDS however many rows it
+// has, and sums run over lanes.  With the scales waited for first, an atomic a row and expert, and sums over barriers, whole calls took, us, that /
+// this: 64 experts, 1575 rows, 512 -> 512 12.2 / 9.9; 32, 7721 rows, 1664 -> 384 17.0 / 14.6; 128, 5206 rows, 1408 -> 640 34.6 / 32.6; 256, 1024 rows,
+// 7168 -> 512 147.5 / 147.1.  (One mask of owned rows instead of the edges is 0.3 us slower with few rows: its atomics meet in one word.)
 constexpr int CHUNK = 32;
 __global__ __launch_bounds__(256) void grouped_prepare_kernel(const int32_t* problem_sizes, const int32_t* expert_offsets, GroupedTables g,
                                                               const float* sa, int64_t sa_sm, int64_t sa_sk, float* out, int64_t pitch, int KB) {
@@ -98,30 +107,46 @@ __global__ __launch_bounds__(256) void grouped_prepare_kernel(const int32_t* pro
     return;
   }
   __shared__ float tile[32][CHUNK + 1];
-  __shared__ int owners[CHUNK], column[CHUNK];  // per row of the chunk: how many experts of the batch own it, and the row's column
+  // an expert's rows in the chunk: +1 where they begin, -1 behind their end; and, where they begin, from a row to its column
+  __shared__ int edges[CHUNK + 1], begins[CHUNK], shift_at[CHUNK];
   const int r0 = blockIdx.x * CHUNK, r1 = min(r0 + CHUNK, g.total_m), k0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const bool k_fast = sa_sk < sa_sm;
+  ExpertTiles t = expert_tiles(problem_sizes, expert_offsets, threadIdx.x, g.E, g.total_m, g.bm, false);
+  float scale[4];
 #pragma unroll
-  for (int i = ty; i < 32; i += 8) {
-    const int m = k_fast ? i : tx, kb = k_fast ? tx : i;
-    if (r0 + m < r1 && k0 + kb < KB) tile[kb][m] = sa[(int64_t)(r0 + m) * sa_sm + (int64_t)(k0 + kb) * sa_sk];
+  for (int i = 0; i < 4; ++i) {
+    const int m = k_fast ? ty + 8 * i : tx, kb = k_fast ? tx : ty + 8 * i;
+    scale[i] = sa[(int64_t)min(r0 + m, r1 - 1) * sa_sm + (int64_t)min(k0 + kb, KB - 1) * sa_sk];
   }
   auto store = [&](int m, int col) {
     for (int kb = ty; kb < 32; kb += 8)
       if (k0 + kb < KB) out[(int64_t)(k0 + kb) * pitch + col] = tile[kb][m];
   };
   for (int c = 0; c < g.E; c += 256) {
-    if (threadIdx.x < CHUNK) owners[threadIdx.x] = 0;
+    if (threadIdx.x <= CHUNK) edges[threadIdx.x] = 0;
+    if (threadIdx.x < CHUNK) begins[threadIdx.x] = 0;
     __syncthreads();
     const int e = c + (int)threadIdx.x;
-    const ExpertTiles t = expert_tiles(problem_sizes, expert_offsets, e, g.E, g.total_m, g.bm, false);
-    const int lo = max(t.row0, r0), hi = min(t.row0 + t.rows, r1), shift = ((t.row0 + 3) & ~3) + 4 * e - t.row0;
-    int shared_rows = 0;
-    if (e < g.E)
-      for (int m = lo; m < hi; ++m) shared_rows |= atomicAdd(&owners[m - r0], 1), column[m - r0] = shift + m;
-    if (__syncthreads_or(shared_rows) == 0) {  // every row has one owner at most: all rows at once
-      if (owners[tx]) store(tx, column[tx]);
+    if (c > 0) t = expert_tiles(problem_sizes, expert_offsets, e, g.E, g.total_m, g.bm, false);
+    const int lo = max(t.row0, r0) - r0, hi = min(t.row0 + t.rows, r1) - r0;
+    if (e < g.E && lo < hi) {
+      atomicAdd(&edges[lo], 1), atomicAdd(&edges[hi], -1);
+      begins[lo] = 1, shift_at[lo] = ((t.row0 + 3) & ~3) + 4 * e - t.row0;
+    }
+    if (c == 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) (k_fast ? tile[tx][ty + 8 * i] : tile[ty + 8 * i][tx]) = scale[i];
+    __syncthreads();
+    int owners = edges[tx];  // of row tx: the sum of the edges up to it
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+      const int v = __shfl_up(owners, d, 32);
+      if (tx >= d) owners += v;
+    }
+    const uint32_t starts = (uint32_t)__ballot(begins[tx] != 0);
+    if (__all(owners <= 1)) {  // every row has one owner at most: all rows at once
+      if (owners) store(tx, shift_at[31 - __clz((int)(starts & (0xffffffffu >> (31 - tx))))] + r0 + tx);
     } else {  // inconsistent offsets: expert by expert
       for (int i = 0; i < 256 && c + i < g.E; ++i) {
         const ExpertTiles o = expert_tiles(problem_sizes, expert_offsets, c + i, g.E, g.total_m, g.bm, false);
