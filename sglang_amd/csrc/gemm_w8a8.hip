@@ -255,64 +255,54 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(const GemmParams p) {
   }
 }
 
-// Sums the split-K partial tiles in ascending split order and applies the epilogue.  The partial tiles are fetched eight at
-// a time before they are added: with one load per addition the kernel is a chain of memory latencies (4.6 us for 7 splits).
-constexpr int REDUCE_BATCH = 8;
-template <bool IS_FP8>
+// Sums the split-K partial tiles in ascending split order and applies the epilogue.  A chain of latencies for the few megabytes it reads: up to
+// BATCH partial tiles are fetched before the first is added (with one load per addition 4.6 us for 7 splits), the epilogue's terms with
+// them, and rows are found by a 32-bit division.  With batches of eight whatever the splits, 64-bit divisions and the terms fetched behind
+// the sum, whole linears took, us, that / this: packed exponents 18432 -> 7168 at 48 tokens, four splits, 33.5 / 32.6; INT8 14336 -> 1024 at 825
+// 31.4 / 30.5, 14336 -> 512 at 2176 43.0 / 42.1; block FP8 14208 -> 12800 at 45, two splits, 43.7 / 43.0; 22 such 0.99, none slower.
+template <bool IS_FP8, int BATCH>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmParams p) {
+  using Sum = typename std::conditional<IS_FP8, float, int>::type;
+  typedef Sum sum4 __attribute__((ext_vector_type(4)));
   const int64_t total = (int64_t)p.M * p.N;
   const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (idx >= total) return;
+  const Sum* w = reinterpret_cast<const Sum*>(p.ws) + idx;
+  sum4 t[BATCH];
+  const auto fetch = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) t[j] = *reinterpret_cast<const sum4*>(w + (int64_t)min(k0 + j, p.splits - 1) * total);
+  };
+  fetch(0);
   // N % 4 == 0 is required for the split path, so the four elements share a row
-  const int m = (int)(idx / p.N);
+  const int m = total < (1ll << 32) ? (int)((uint32_t)idx / (uint32_t)p.N) : (int)(idx / p.N);
   const int n = (int)(idx - (int64_t)m * p.N);
+  const ChannelTerms terms = load_channel_terms(p, IS_FP8 ? p.col_scale : p.sb, n);  // (unread where raw INT8 sums are asked for)
+  const float token_scale = IS_FP8 ? (p.row_scale ? p.row_scale[m] : 1.f) : p.out_dtype == MI355_I32 ? 1.f : p.sa[m];
+  sum4 s = {0, 0, 0, 0};  // 0 + first partial is exact, so the sum is the one that starts from the first partial
+  for (int k0 = 0;;) {
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j)
+      if (k0 + j < p.splits) s[0] += t[j][0], s[1] += t[j][1], s[2] += t[j][2], s[3] += t[j][3];
+    if ((k0 += BATCH) >= p.splits) break;
+    fetch(k0);
+  }
+  const Sum sum[4] = {s[0], s[1], s[2], s[3]};
+  float r[4];
   if constexpr (IS_FP8) {
-    const float* w = reinterpret_cast<const float*>(p.ws) + idx;
-    v4f s = {0.f, 0.f, 0.f, 0.f};  // 0 + first partial is exact, so the sum is the one that starts from the first partial
-    for (int k0 = 0; k0 < p.splits; k0 += REDUCE_BATCH) {
-      v4f t[REDUCE_BATCH];
 #pragma unroll
-      for (int j = 0; j < REDUCE_BATCH; ++j)
-        t[j] = *reinterpret_cast<const v4f*>(w + (int64_t)min(k0 + j, p.splits - 1) * total);
-#pragma unroll
-      for (int j = 0; j < REDUCE_BATCH; ++j)
-        if (k0 + j < p.splits) s[0] += t[j][0], s[1] += t[j][1], s[2] += t[j][2], s[3] += t[j][3];
-    }
-    float r[4] = {s[0], s[1], s[2], s[3]};
-    fp8_apply_terms(p, load_channel_terms(p, p.col_scale, n), p.row_scale ? p.row_scale[m] : 1.f, r);
-    const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
-    store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, 4, vec_ok);
+    for (int v = 0; v < 4; ++v) r[v] = sum[v];
+    fp8_apply_terms(p, terms, token_scale, r);
   } else {
-    const int* w = reinterpret_cast<const int*>(p.ws) + idx;
-    v4i s = {0, 0, 0, 0};
-    for (int k0 = 0; k0 < p.splits; k0 += REDUCE_BATCH) {
-      v4i t[REDUCE_BATCH];
-#pragma unroll
-      for (int j = 0; j < REDUCE_BATCH; ++j)
-        t[j] = *reinterpret_cast<const v4i*>(w + (int64_t)min(k0 + j, p.splits - 1) * total);
-#pragma unroll
-      for (int j = 0; j < REDUCE_BATCH; ++j)
-        if (k0 + j < p.splits) s[0] += t[j][0], s[1] += t[j][1], s[2] += t[j][2], s[3] += t[j][3];
-    }
     if (p.out_dtype == MI355_I32) {
       int* o = reinterpret_cast<int*>(p.out) + (int64_t)m * p.ldo + n;
-      for (int v = 0; v < 4; ++v) o[v] = s[v];
+      for (int v = 0; v < 4; ++v) o[v] = sum[v];
       return;
     }
-    const float sa_m = p.sa[m];
-    float r[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      float t = mul_rn((float)s[v], mul_rn(p.sb[n + v], sa_m));
-      if (p.bias) {
-        const uint32_t hb = reinterpret_cast<const uint16_t*>(p.bias)[n + v];
-        t = add_rn(t, (p.out_dtype == MI355_BF16) ? bf16_bits_to_f32(hb) : f16_bits_to_f32(hb));
-      }
-      r[v] = t;
-    }
-    const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
-    store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, 4, vec_ok);
+    int8_apply_terms(p, terms, token_scale, sum, r);
   }
+  const bool vec_ok = ((p.ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
+  store_out4(p.out, p.out_dtype, (int64_t)m * p.ldo + n, r, 4, vec_ok);
 }
 
 // Both tables, an array of doubles as far as the queries of single constants go.
@@ -786,7 +776,10 @@ int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_giv
   }
   if (rc != MI355_OK || p.splits == 1) return rc;
   const int64_t quads = ((int64_t)p.M * p.N + 3) / 4;
-  launch_kernel(splitk_reduce_kernel<IS_FP8>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, p);
+  const dim3 grid((unsigned)((quads + 255) / 256)), block(256);
+  if (p.splits <= 2) launch_kernel((splitk_reduce_kernel<IS_FP8, 2>), grid, block, 0, stream, p);
+  else if (p.splits <= 4) launch_kernel((splitk_reduce_kernel<IS_FP8, 4>), grid, block, 0, stream, p);
+  else launch_kernel((splitk_reduce_kernel<IS_FP8, 8>), grid, block, 0, stream, p);
   return check_launch(what);
 }
 
