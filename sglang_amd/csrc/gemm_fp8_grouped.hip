@@ -338,12 +338,13 @@ struct GroupedTimes {
 // joined with the stream of the weights that are used.  Rows fall on experts at random, so some of few get none.  Fitted to 770 timings of
 // 190 problems with up to 220 million active weights (their routing uneven by 0.25 .. 1.25): 7 % root mean square.  It saves the preparation and
 // splits K over eight waves where the mid-M tile has a chain of K blocks on a few CUs, but every further round of workgroups starts with
-// the search and the first loads again: taken up to one and a half rounds, where it models 10 % faster.  74 of the 190, this / tables and
-// mid-M tile: 0.595 of the time in a graph (at most 1.12), 0.65 eager; us in a graph 16 experts 22 rows 1152 -> 256 9.6 / 4.2, 32 of 136
-// 3840 -> 256 17.1 / 9.0, 64 of 59 6528 -> 384 31.6 / 18.6, 8 of 662 3456 -> 384 17.4 / 9.3; beyond, 128 of 61 1664 -> 768 17.0 / 18.6, 256 of 271
-// 1408 -> 640 31.9 / 44.4.
+// the search and the first loads again: taken up to 1.12 rounds, with 0, 5 and 10 % more workgroups than expected on average, where it models
+// 17 % faster than the mid-M tile (whose model has a preparation 1 to 2 us longer than it is).  58 of the 190, this / tables and mid-M tile: 0.56 of
+// the time in a graph (at most 1.03), 0.63 eager; us in a graph 16 experts 22 rows 1152 -> 256 9.1 / 4.2, 32 of 136 3840 -> 256 16.7 / 9.0,
+// 64 of 59 6528 -> 384 31.2 / 18.6, 8 of 662 3456 -> 384 15.4 / 9.3, 16 of 67 6784 -> 1024 34.0 / 21.4 (0.99 rounds), 256 of 50 5888 -> 384 30.7 / 25.3
+// (1.07); beyond, 128 of 9 3200 -> 2176 (1.16) 15.5 / 16.6, 256 of 117 6272 -> 256 (1.47) 32.5 / 36.1, 16 of 244 4096 -> 1536 (1.5) 26.9 / 28.9.
 struct GroupedWavesplitTimes {
-  static constexpr double LAUNCH = 1.27, TILE = 2.26, KB_US = 0.0064, BUSY = 1.07, RESULT = 0.459, STREAM = 7.71, NORM = 1.364, MOST_ROUNDS = 1.5, MARGIN = 0.9;
+  static constexpr double LAUNCH = 1.27, TILE = 2.26, KB_US = 0.0064, BUSY = 1.07, RESULT = 0.459, STREAM = 7.71, NORM = 1.364, MOST_ROUNDS = 1.12, MARGIN = 0.83;
   double active;
   int64_t total_m, N, K;
   GroupedWavesplitTimes(int64_t E, int64_t total_m_, int64_t N_, int64_t K_)
@@ -359,8 +360,12 @@ struct GroupedWavesplitTimes {
     const auto round = [&](double fill) {
       return TILE + (double)((t.bm + t.bn) * K) * 1e-3 * KB_US * (1.0 + BUSY * fill) + (double)(t.bm * t.bn) / 1024.0 * RESULT;
     };
-    const double full = std::floor(workgroups / NUM_CUS), rest = workgroups / NUM_CUS - full;
-    const double tile_us = full * round(1.0) + (rest > 1e-9 ? round(rest) : 0.0), stream = active * (double)N * (double)K * 1e-6 / STREAM;
+    double tile_us = 0.0;
+    for (const double more : {1.0, 1.05, 1.1}) {
+      const double all = more * workgroups / NUM_CUS, full = std::floor(all), rest = all - full;
+      tile_us += (full * round(1.0) + (rest > 1e-9 ? round(rest) : 0.0)) / 3.0;
+    }
+    const double stream = active * (double)N * (double)K * 1e-6 / STREAM;
     return LAUNCH + std::pow(std::pow(tile_us, NORM) + std::pow(stream, NORM), 1.0 / NORM);
   }
 };

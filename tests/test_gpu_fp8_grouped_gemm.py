@@ -122,13 +122,13 @@ def test_random_expert_sizes(gpu, oracle, num_experts, out_dtype):
 
 
 @pytest.mark.parametrize("name,sizes,N,K,tile", [
-    ("decode_like", [1, 0, 3, 1, 0, 0, 2, 8, 1, 1, 0, 5, 16, 1, 2, 1], 512, 7168, "16x32"),
+    ("decode_like", [1, 0, 3, 1, 0, 0, 2, 8, 1, 1, 0, 5, 16, 1, 2, 1], 512, 7168, "16x64"),
     ("one_token", [1], 256, 128, "16x16"),
     ("empty_experts_around_a_big_one", [0, 0, 700, 0, 1, 0], 384, 512, "32x64"),
     ("prefill_like", [130, 257, 128, 64, 511, 129, 300, 200], 768, 1024, "64x128"),
-    ("tile_edges", [64, 65, 63, 128, 127, 129, 1, 256], 256, 256, "32x32"),
+    ("tile_edges", [64, 65, 63, 128, 127, 129, 1, 256], 256, 256, "16x64"),
     ("many_small", [3] * 300, 128, 256, "64x128"),
-    ("large_experts", [1000, 513, 384, 2], 512, 512, "64x64"),
+    ("large_experts", [1000, 513, 384, 2], 512, 512, "64x128"),
     ("ragged_channels", [40, 90, 17], 200, 384, "16x16"),
     ("decode_like_wide", [1, 0, 3, 1, 0, 0, 2, 8, 1, 1, 0, 5, 16, 1, 2, 1], 1664, 7168, "64x128"),
     ("empty_experts_around_a_big_one_wide", [0, 0, 700, 0, 1, 0], 1280, 512, "64x128"),

@@ -36,7 +36,8 @@ def test_grouped(gpu, oracle, name, sizes, N, K, m_major):
 # experts (uneven: some without a row, one with many), stacked rows, N, K -> what has to run
 FORMS = [(40, 1240, 2056, 128, "grouped_dma3", "64x256"), (2, 3254, 328, 384, "grouped_dma3", "64x128"),
          (16, 16, 64, 384, "grouped_wavesplit", "16x16"), (8, 209, 416, 128, "grouped_wavesplit", "16x32"), (40, 29, 392, 1152, "grouped_wavesplit", "16x64"),
-         (24, 1574, 128, 128, "grouped_wavesplit", "32x32"), (16, 1613, 224, 128, "grouped_wavesplit", "32x64"), (3, 545, 1544, 1152, "grouped_wavesplit", "64x64"),
+         (5, 56, 1240, 128, "grouped_wavesplit", "32x32"), (40, 492, 272, 128, "grouped_wavesplit", "32x64"), (40, 1798, 136, 128, "grouped_wavesplit", "64x64"),
+         (24, 1574, 128, 128, "grouped_wavesplit", "16x64"), (16, 1613, 224, 128, "grouped_wavesplit", "64x64"), (3, 545, 1544, 1152, "grouped_dma3", "64x128"),
          (40, 29, 2056, 128, "grouped_dma3", "64x128"),  # (more workgroups than CUs: two share one)
          (24, 1233, 2056, 384, "grouped_dma3", "128x256"), (16, 2075, 2056, 384, "grouped_dma3", "128x256"),
          (1, 1695, 2056, 640, "grouped_dma3", "128x128"), (24, 3078, 768, 2048, "grouped_dma3", "128x128"),
