@@ -277,8 +277,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmParams p) 
   // N % 4 == 0 is required for the split path, so the four elements share a row
   const int m = total < (1ll << 32) ? (int)((uint32_t)idx / (uint32_t)p.N) : (int)(idx / p.N);
   const int n = (int)(idx - (int64_t)m * p.N);
-  const ChannelTerms terms = load_channel_terms(p, IS_FP8 ? p.col_scale : p.sb, n);  // (unread where raw INT8 sums are asked for)
-  const float token_scale = IS_FP8 ? (p.row_scale ? p.row_scale[m] : 1.f) : p.out_dtype == MI355_I32 ? 1.f : p.sa[m];
+  ChannelTerms terms{};
+  float token_scale = 1.f;
+  const bool raw = !IS_FP8 && p.out_dtype == MI355_I32;  // (of raw sums the caller's scales and bias may be anything: not to be read)
+  if (!raw) {
+    terms = load_channel_terms(p, IS_FP8 ? p.col_scale : p.sb, n);
+    if constexpr (IS_FP8) token_scale = p.row_scale ? p.row_scale[m] : 1.f;
+    else token_scale = p.sa[m];
+  }
   sum4 s = {0, 0, 0, 0};  // 0 + first partial is exact, so the sum is the one that starts from the first partial
   for (int k0 = 0;;) {
 #pragma unroll
@@ -294,7 +300,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmParams p) 
     for (int v = 0; v < 4; ++v) r[v] = sum[v];
     fp8_apply_terms(p, terms, token_scale, r);
   } else {
-    if (p.out_dtype == MI355_I32) {
+    if (raw) {
       int* o = reinterpret_cast<int*>(p.out) + (int64_t)m * p.ldo + n;
       for (int v = 0; v < 4; ++v) o[v] = sum[v];
       return;

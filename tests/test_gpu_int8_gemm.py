@@ -49,6 +49,30 @@ def test_int32_accumulator_extremes(gpu):
     assert acc[0, 0] == 128 * 128 * K and acc[2, 1] == -128 * 127 * K
 
 
+# partial tiles that the reduce kernel fetches at a time: 2, 4, 8, each a kernel of its own
+@pytest.mark.parametrize("M,N,K,batch", [(474, 2912, 11392, 2), (300, 4096, 14336, 4), (1606, 8, 12928, 8)])
+def test_raw_accumulators_ignore_scales_and_bias(gpu, M, N, K, batch):
+    """int32 results of a split K: scales and bias, of any length, are not read (the buffers here hold one value, which is NaN)."""
+    from sglang_amd import _lib, ops
+
+    plan = _lib.gemm_plan("int8", M, N, K)
+    print(f"case M={M} N={N} K={K} {plan}", flush=True)
+    assert plan["splits"] > 1 and (2 if plan["splits"] <= 2 else 4 if plan["splits"] <= 4 else 8) == batch
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a, w = (torch.randint(-128, 128, (rows, K), generator=g, device=gpu, dtype=torch.int8) for rows in (M, N))
+    one, half = torch.full((1,), float("nan"), device=gpu), torch.full((1,), float("nan"), device=gpu, dtype=torch.bfloat16)
+    out = torch.empty((M, N), device=gpu, dtype=torch.int32)
+    L = _lib.lib()
+    need = L.mi355_int8_scaled_mm_workspace_bytes(M, N, K)
+    ws = torch.empty(need, device=gpu, dtype=torch.uint8)
+    _lib.check(L.mi355_int8_scaled_mm(a.data_ptr(), w.data_ptr(), one.data_ptr(), one.data_ptr(), half.data_ptr(), out.data_ptr(), _lib.I32,
+                                      M, N, K, K, K, N, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out, ops.int8_mm_raw_accumulators(a, w.t()))
+    rows = torch.arange(0, M, max(1, M // 7), device=gpu)
+    exact = (a[rows].double() @ w.double().t()).to(torch.int32)  # (below 2^53)
+    assert torch.equal(out[rows], exact)
+
+
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("with_bias", [False, True])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
