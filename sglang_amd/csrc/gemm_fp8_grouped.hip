@@ -222,7 +222,7 @@ template <int MT, int CT>
 __global__ __launch_bounds__(64 * WST_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp8_grouped_wavesplit_kernel(const GroupedParams gp, const GroupedRouting r) {
   GemmParams p;
   int m0, tile_n;
-  if (find_tile<16 * MT>(gp, r, p, m0, tile_n)) wavesplit_tile<AR_F32, MT, CT, TQ_NONE, 2, false>(p, m0, tile_n * 16 * CT);
+  if (find_tile<16 * MT>(gp, r, p, m0, tile_n)) wavesplit_tile<AR_F32, MT, CT, TQ_NONE, 2, false, false, true>(p, m0, tile_n * 16 * CT);
 }
 constexpr TileSize GROUPED_WAVESPLIT_TILES[] = {{16, 16}, {16, 32}, {16, 64}, {32, 32}, {32, 64}, {64, 64}};
 template <size_t... I>
@@ -255,8 +255,7 @@ struct GroupedRun {
   bool use_big;
   int bm, bn, max_big, max_small;
   bool few;  // at most a workgroup per CU is expected
-  // where split.bm > 0: one launch on the wave-split tile of this size, at most split_tiles token tiles; the above where the token scales' rows lie
-  // too far apart for it, and for the workspace
+  // where split.bm > 0: one launch on the wave-split tile of this size, at most split_tiles token tiles; the above is the workspace's then
   TileSize split{0, 0};
   int split_tiles = 0;
 };
@@ -473,7 +472,7 @@ extern "C" int mi355_fp8_blockwise_scaled_grouped_mm(const void* a, const void* 
                 "%s: workspace must be 256-byte aligned", what);
 
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (run.split.bm > 0 && total_m * std::max<int64_t>(sa_sm, 1) < (1ll << 30)) {  // (32-bit offsets of the token scales)
+  if (run.split.bm > 0) {
     GroupedParams gp{};
     gp.g.a = static_cast<const uint8_t*>(a), gp.g.b = static_cast<const uint8_t*>(b);
     gp.g.sa = scales_a, gp.g.sb = scales_b, gp.g.out = out;

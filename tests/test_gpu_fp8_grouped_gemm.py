@@ -177,6 +177,42 @@ def test_token_scales_in_either_layout(gpu, oracle):
     assert torch.equal(out_row, out_col)
 
 
+@pytest.mark.parametrize("N,kernel", [(256, "grouped_wavesplit"), (6400, "grouped_dma3")])
+def test_token_scales_any_distance_apart(gpu, oracle, N, kernel):
+    """Rows of scales more than 4 GiB apart, and both strides negative: the same result as from dense scales, on the kernel the plan names (it
+    knows nothing of the strides)."""
+    from sglang_amd import _lib
+
+    sizes, K = [3, 0, 12, 1], 256
+    a, w, sa, sw, offsets, T = _problem(sizes, N, K, 17)
+    E, KB, NB = len(sizes), K // 128, (N + 127) // 128
+    assert _lib.grouped_gemm_plan(E, T, N, K)["kernel"] == kernel
+    ag, wg, sg = a.to(gpu), w.to(gpu), sw.to(gpu)
+    problem_sizes = torch.tensor([[m, N, K] for m in sizes], dtype=torch.int32, device=gpu)
+    expert_offsets = torch.tensor(offsets, dtype=torch.int32, device=gpu)
+    L = _lib.lib()
+    need = L.mi355_fp8_blockwise_scaled_grouped_mm_workspace_bytes(E, T, N, K)
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu)
+
+    def call(scales_ptr, sa_sm, sa_sk):
+        out = torch.full((T, N), 7.0, dtype=torch.bfloat16, device=gpu)
+        _lib.check(L.mi355_fp8_blockwise_scaled_grouped_mm(
+            ag.data_ptr(), wg.data_ptr(), scales_ptr, sg.data_ptr(), out.data_ptr(), _lib.BF16, problem_sizes.data_ptr(),
+            expert_offsets.data_ptr(), E, T, N, K, K, K, N * K, sa_sm, sa_sk, NB * KB, KB, 1, N, ws.data_ptr(), need,
+            torch.cuda.current_stream().cuda_stream))
+        return out
+
+    dense = sa.to(gpu)
+    want = call(dense.data_ptr(), KB, 1)
+    _verify(oracle, want, a, w, sa, sw, sizes, offsets, kernel)
+    pitch = (1 << 27) + 2  # floats: sixteen rows over 8 GiB
+    far = torch.empty((T - 1) * pitch + KB, dtype=torch.float32, device=gpu)
+    far.as_strided((T, KB), (pitch, 1)).copy_(dense)
+    assert torch.equal(call(far.data_ptr(), pitch, 1), want)
+    back = dense.flip(0, 1).contiguous()  # element (0, 0) lies last
+    assert torch.equal(call(back.data_ptr() + 4 * (T * KB - 1), -KB, -1), want)
+
+
 def test_expert_specialised_entry_point(gpu, oracle):
     """es_fp8_blockwise_scaled_grouped_mm (sgl-kernel/tests/test_es_fp8_blockwise_moe.py:103-196): same layouts, no
     scratch tensors in the argument list; same result as the other entry point, bit for bit."""
