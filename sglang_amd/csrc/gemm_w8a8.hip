@@ -720,7 +720,7 @@ template <bool IS_FP8>
 int run_gemm(GemmParams& p, Route r, void* workspace, size_t workspace_bytes_given, hipStream_t stream, const char* what) {
   p.kb_total = (p.K + KSTEP - 1) / KSTEP;
   const bool aligned = operands_aligned(p);
-  const bool wide_scales = (r.kernel == RK_WAVESPLIT_TILE) && p.sa_sm * (int64_t)p.M >= (1ll << 30);  // 32-bit byte offsets
+  const bool wide_scales = (r.kernel == RK_WAVESPLIT_TILE) && (p.sa_sm < 0 || p.sa_sm * (int64_t)p.M >= (1ll << 30));  // 32-bit byte offsets
   if (!p.ue8m0 && !p.row_scale && (wide_scales || route_workspace_need(IS_FP8, r, p) > workspace_bytes_given))  // (a workspace for the plan's own splits)
     r = choose_route(IS_FP8, p.M, p.N, p.K, p.lda, p.ldb, aligned, p.x16 != nullptr);
   p.splits = r.splits;

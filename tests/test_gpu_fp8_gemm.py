@@ -61,6 +61,37 @@ def test_sgl_kernel_fp8_blockwise_scaled_mm(gpu, oracle, M, N, K, out_dtype):
     _check(out, ref, mag, f"M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 2176, 2176), (40, 512, 1024)])
+def test_token_scales_any_distance_apart(gpu, oracle, M, N, K):
+    """Rows of scales more than 4 GiB apart and both strides negative, where dense scales run on the wave-split tile."""
+    from sglang_amd import _lib
+
+    assert _lib.gemm_plan("fp8", M, N, K)["kernel"] == "wavesplit_tile"
+    g = torch.Generator().manual_seed(M)
+    a, w = _rand_fp8((M, K), g), _rand_fp8((N, K), g)
+    KB, NB = K // 128, N // 128
+    sa, sb = torch.randn(M, KB, generator=g) * 1e-3, torch.randn(NB, KB, generator=g) * 1e-3
+    ag, wg, sg, dense = a.to(gpu), w.to(gpu), sb.to(gpu), sa.to(gpu)
+    L = _lib.lib()
+    need = L.mi355_fp8_blockwise_mm_workspace_bytes(M, N, K)
+    ws = torch.empty(need + 256, dtype=torch.uint8, device=gpu)
+    ref, mag = oracle.fp8_blockwise_mm(a, w, sa, sb, torch.float32, want_abs=True)
+
+    def check(what, scales_ptr, sa_sm, sa_sk):
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=gpu)
+        _lib.check(L.mi355_fp8_blockwise_mm(ag.data_ptr(), wg.data_ptr(), scales_ptr, sg.data_ptr(), out.data_ptr(), _lib.BF16, M, N, K, K, K,
+                                            sa_sm, sa_sk, KB, 1, N, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+        _check(out, ref, mag, what)
+
+    check("dense", dense.data_ptr(), KB, 1)
+    pitch = (1 << 30) // M + 2  # floats
+    far = torch.empty((M - 1) * pitch + KB, dtype=torch.float32, device=gpu)
+    far.as_strided((M, KB), (pitch, 1)).copy_(dense)
+    check("far", far.data_ptr(), pitch, 1)
+    back = dense.flip(0, 1).contiguous()  # element (0, 0) lies last
+    check("backwards", back.data_ptr() + 4 * (M * KB - 1), -KB, -1)
+
+
 RAGGED_SHAPES = [(7, 1088, 512), (83, 7748, 256), (16, 576, 7168), (64, 128, 3884), (130, 200, 300),
                  (1, 1088, 3884), (256, 576, 1024)]
 
