@@ -260,6 +260,28 @@ def test_small_layers_run_the_measured_kernel(kind, shape, kernel):
     assert _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
 
 
+# Above 16 tokens on small layers of short K: (linear, shape, whether the tile quantizes its tokens).  us in a graph, and what ran otherwise:
+SMALL_BATCH_CHOICES = [
+    ("ue8m0", (173, 256, 2048), "launch"),  # 5.5, 6.7
+    ("ue8m0", (185, 640, 1536), "launch"),  # 5.65, 6.6
+    ("int8", (121, 384, 1536), "launch"),  # 5.6, 6.5
+    ("block", (48, 768, 2048), "launch"),  # 5.8, 6.6
+    ("token_fp8", (168, 768, 1280), "launch"),  # 6.0, 7.0
+    ("block", (46, 512, 1280), "fused"),  # 5.1, 5.3
+    ("ue8m0", (669, 384, 640), "fused"),  # 4.3, 6.8
+    ("token_fp8", (69, 384, 768), "fused"),  # 4.2, 5.3
+    ("int8", (103, 768, 768), "fused"),  # 4.35, 5.6
+    ("block", (89, 2560, 1024), "fused"),  # 5.5, 5.7
+]
+
+
+@pytest.mark.parametrize("kind,shape,quantizer", SMALL_BATCH_CHOICES)
+def test_small_batches_take_the_measured_number_of_launches(kind, shape, quantizer):
+    from sglang_amd import _lib
+
+    assert _lib.linear_plan(kind, *shape)["quantizer"] == quantizer, _lib.linear_plan(kind, *shape)
+
+
 def test_perturbed_plan_query():
     import ctypes
 
