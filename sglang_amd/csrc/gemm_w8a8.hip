@@ -1261,11 +1261,15 @@ bool tile_quant_takes(WavesplitQuant quant, int64_t K) {
   return K % (quant == WavesplitQuant::TOKEN_FP8 || quant == WavesplitQuant::TOKEN_INT8 ? 16 : KSTEP) == 0;
 }
 // The wave-split tile quantizing the tokens itself, where the GEMM takes that tile (same sums, bit for bit): the launch saved
-// against the quantizer's work in every workgroup, v pieces per thread and round.
+// against the quantizer's work in every workgroup, v pieces per thread and round.  K in parts of blocks, where a piece takes more: beyond
+// six pieces only up to six tokens, whose launch has a long row for each workgroup (120 linears in a graph, launch in front / this: INT8 3 tokens
+// 9664 -> 14080 41.1 / 31.4, 3 tokens 10432 -> 768 9.4 / 8.8, 4 tokens per-token FP8 8352 -> 6016 17.1 / 16.3; 27 of seven tokens and more 1.08,
+// INT8 13 tokens 2784 -> 1152 6.3 / 7.6, per-token FP8 15 tokens 2016 -> 640 5.6 / 6.25).
 bool tile_quant_preferred(WavesplitQuant quant, const Route& run, int64_t M, int64_t N, int64_t K) {
   if (run.kernel != RK_WAVESPLIT_TILE || M > 16 || !tile_quant_takes(quant, K)) return false;
   const int64_t pieces = M * ((K + KSTEP - 1) / KSTEP) * (KSTEP / 8), threads = 512, rounds = (N + (int64_t)run.bn * NUM_CUS - 1) / ((int64_t)run.bn * NUM_CUS);
-  return pieces <= 10 * threads && pieces * rounds <= 10 * threads;
+  const int64_t most = K % KSTEP == 0 || M <= 6 ? 10 : 6;
+  return pieces <= most * threads && pieces * rounds <= 10 * threads;
 }
 bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
   const int plain = choose_route(true, M, N, K, K, ldw, true).kernel;

@@ -260,7 +260,7 @@ def test_small_layers_run_the_measured_kernel(kind, shape, kernel):
     assert _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
 
 
-# Above 16 tokens on small layers of short K: (linear, shape, whether the tile quantizes its tokens).  us in a graph, and what ran otherwise:
+# Small layers of short K above 16 tokens: (linear, shape, whether the tile quantizes its tokens).  us in a graph, and what ran otherwise:
 SMALL_BATCH_CHOICES = [
     ("ue8m0", (173, 256, 2048), "launch"),  # 5.5, 6.7
     ("ue8m0", (185, 640, 1536), "launch"),  # 5.65, 6.6
@@ -272,11 +272,18 @@ SMALL_BATCH_CHOICES = [
     ("token_fp8", (69, 384, 768), "fused"),  # 4.2, 5.3
     ("int8", (103, 768, 768), "fused"),  # 4.35, 5.6
     ("block", (89, 2560, 1024), "fused"),  # 5.5, 5.7
+    # K in parts of blocks at decode sizes
+    ("int8", (13, 1152, 2784), "launch"),  # 6.3, 7.6
+    ("int8", (9, 640, 4384), "launch"),  # 6.7, 7.9
+    ("token_fp8", (15, 640, 2016), "launch"),  # 5.6, 6.25
+    ("int8", (3, 768, 10432), "fused"),  # 8.8, 9.4
+    ("token_fp8", (4, 6016, 8352), "fused"),  # 16.3, 17.1
+    ("int8", (14, 8320, 1504), "fused"),  # 7.8, 7.8
 ]
 
 
 @pytest.mark.parametrize("kind,shape,quantizer", SMALL_BATCH_CHOICES)
-def test_small_batches_take_the_measured_number_of_launches(kind, shape, quantizer):
+def test_tokens_are_quantized_where_it_measured_faster(kind, shape, quantizer):
     from sglang_amd import _lib
 
     assert _lib.linear_plan(kind, *shape)["quantizer"] == quantizer, _lib.linear_plan(kind, *shape)
