@@ -62,14 +62,81 @@ def test_every_tiling(gpu, oracle, E, rows, N, K, kernel, tile):
     _verify(oracle, out, a, w, sa, sw, sizes, offsets, f"{E} {rows}")
 
 
-def test_experts_that_share_rows(gpu, oracle):
-    """Overlapping offsets: every expert still multiplies the rows it names with its own weight; rows named twice hold the result of
-    one of them."""
-    sizes = [40, 40, 24]
-    a, w, sa, sw, _, T = _problem(sizes, 256, 256, 5)
-    out = _call(gpu, a, w, sa, sw, sizes, [0, 20, 80], torch.bfloat16).float().cpu()
-    for e, (m, r0) in enumerate(zip(sizes, (0, 20, 80))):
-        ref, mag = oracle.fp8_blockwise_mm(a[r0:r0 + m], w[e], sa[r0:r0 + m], sw[e], torch.float32, want_abs=True)
-        alone = [r for r in range(r0, r0 + m) if not 20 <= r < 40]
-        index = torch.tensor(alone) - r0
-        assert bool(((out[alone] - ref[index]).abs() <= 1e-2 * ref[index].abs() + 1e-4 * mag[index]).all())
+# routing that is not dense and in order, on the one-launch tile and where tables are prepared: (sizes, offsets, stacked rows, N, K, what runs)
+SHARED = [([40, 40, 24], [0, 20, 80], 104, 256, 256, "grouped_wavesplit"), ([40, 40, 24], [0, 20, 80], 104, 6152, 256, "grouped_dma3"),
+          # out of order, one inside another, one outside every 32-row chunk of the others, a gap inside a chunk
+          ([30, 7, 50, 3], [60, 64, 5, 200], 237, 264, 384, "grouped_wavesplit"), ([30, 7, 50, 3], [60, 64, 5, 200], 237, 5128, 384, "grouped_dma3")]
+# more experts than a scan takes at a time: rows shared inside the second 256 experts, and with one of the first
+MANY = [1] * 300
+MANY_OFFSETS = [e + (e > 100) * 3 for e in range(300)]
+MANY[280], MANY[281], MANY_OFFSETS[290] = 5, 3, 10
+SHARED += [(MANY, MANY_OFFSETS, 310, 24, 128, "grouped_wavesplit"), (MANY, MANY_OFFSETS, 310, 1032, 128, "grouped_dma3")]
+
+
+@pytest.mark.parametrize("sizes,offsets,T,N,K,kernel", SHARED, ids=lambda v: str(v) if isinstance(v, (int, str)) else str(len(v)))
+def test_experts_that_share_rows(gpu, oracle, sizes, offsets, T, N, K, kernel):
+    """Overlapping offsets: every expert still multiplies the rows it names with its own weight; rows named by several hold results of
+    theirs, and rows named by none stay as they were.  Prepared scales have a column for each row of an expert, which two that share rows
+    may share too: wrong results there are what such routing gets, and nowhere else."""
+    from sglang_amd import _lib
+
+    print(f"case {T} {N} {K} {_lib.grouped_gemm_plan(len(sizes), T, N, K)}", flush=True)
+    assert _lib.grouped_gemm_plan(len(sizes), T, N, K)["kernel"] == kernel
+    a, w, sa, sw, _, _ = _problem([T] + [0] * (len(sizes) - 1), N, K, 5)
+    out = _call(gpu, a, w, sa, sw, sizes, offsets, torch.bfloat16).float().cpu()
+    right, owners = torch.zeros(T, N, dtype=torch.bool), torch.zeros(T, dtype=torch.int32)
+    column = lambda e, r0: (r0 + 3) // 4 * 4 + 4 * e
+    taken = torch.zeros(2 * T + 4 * len(sizes), dtype=torch.int32)
+    for e, (m, r0) in enumerate(zip(sizes, offsets)):
+        taken[column(e, r0):column(e, r0) + m] += 1
+    own_scales = torch.ones(T, dtype=torch.bool)
+    for e, (m, r0) in enumerate(zip(sizes, offsets)):
+        rows = slice(r0, r0 + m)
+        own_scales[rows] &= taken[column(e, r0):column(e, r0) + m] == 1
+        ref, mag = oracle.fp8_blockwise_mm(a[rows], w[e], sa[rows], sw[e], torch.float32, want_abs=True)
+        right[rows] |= (out[rows] - ref).abs() <= 1e-2 * ref.abs() + 1e-4 * mag
+        owners[rows] += 1
+    assert bool((owners > 1).any()) and bool((owners == 0).any())
+    if kernel == "grouped_wavesplit":
+        own_scales[:] = True
+    assert 2 * int((own_scales & (owners > 0)).sum()) > int((owners > 0).sum())
+    assert bool(right[own_scales & (owners > 0)].all()) and bool((out[owners == 0] == 7.0).all())
+
+
+@pytest.mark.parametrize("N,kernel", [(256, "grouped_wavesplit"), (5128, "grouped_dma3")])
+def test_gaps_and_sizes_beyond_the_matrix(gpu, oracle, N, kernel):
+    """Unused rows between experts, some of them in the same 32 as used ones, and a last expert that claims more rows than there are."""
+    from sglang_amd import _lib
+
+    sizes = [5, 100, 0, 33, 64]
+    a, w, sa, sw, offsets, T = _problem(sizes, N, 512, 9, gap=7)
+    assert _lib.grouped_gemm_plan(5, T, N, 512)["kernel"] == kernel
+    _verify(oracle, _call(gpu, a, w, sa, sw, sizes, offsets, torch.float16), a, w, sa, sw, sizes, offsets, "gaps")
+    claimed, there = sizes[:4] + [1 << 20], sizes[:4] + [T - offsets[4]]
+    _verify(oracle, _call(gpu, a, w, sa, sw, claimed, offsets, torch.float16), a, w, sa, sw, there, offsets, "claimed")
+    # offsets outside the matrix: nothing of those experts is written
+    beyond = offsets[:3] + [-4, T + 9]
+    out = _call(gpu, a, w, sa, sw, sizes[:3] + [0, 64], beyond, torch.float16)
+    _verify(oracle, out, a, w, sa, sw, sizes[:3] + [0, 0], offsets, "beyond")
+
+
+@pytest.mark.parametrize("sizes,N,K,kernel", [([70, 9, 140], 512, 640, "grouped_wavesplit"), ([70, 9, 140], 4104, 640, "grouped_dma3"),
+                                              ([200, 1, 77, 300, 0, 129], 384, 768, "grouped_wavesplit"),
+                                              ([200, 1, 77, 300, 0, 129], 2056, 768, "grouped_dma3")])
+def test_entry_points_and_scale_layouts_agree(gpu, sizes, N, K, kernel):
+    """Both entry points, and token scales row-major and column-major: the same bits."""
+    from sglang_amd import _lib
+    from sglang_amd.sgl_kernel import es_fp8_blockwise_scaled_grouped_mm
+
+    a, w, sa, sw, offsets, T = _problem(sizes, N, K, 21)
+    E = len(sizes)
+    assert _lib.grouped_gemm_plan(E, T, N, K)["kernel"] == kernel
+    want = _call(gpu, a, w, sa, sw, sizes, offsets, torch.bfloat16)
+    assert torch.equal(want, _call(gpu, a, w, sa.to(gpu).t().contiguous().t(), sw, sizes, offsets, torch.bfloat16))
+    out = torch.full((T, N), 7.0, dtype=torch.bfloat16, device=gpu)
+    i64 = lambda v: torch.full((E,), v, dtype=torch.int64, device=gpu)
+    es_fp8_blockwise_scaled_grouped_mm(
+        out, a.to(gpu), w.to(gpu).transpose(1, 2), sa.to(gpu), sw.to(gpu).transpose(1, 2), i64(K), i64(K), i64(N),
+        torch.tensor([[m, N, K] for m in sizes], dtype=torch.int32, device=gpu),
+        torch.tensor(offsets, dtype=torch.int32, device=gpu), torch.empty(16 << 20, dtype=torch.uint8, device=gpu))
+    assert torch.equal(want, out)
