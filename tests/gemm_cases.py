@@ -255,6 +255,61 @@ QUANT_TILE_SHAPES = {((16, 16), False): (143, 24, 640), ((16, 16), True): (49, 1
                      ((16, 32), True): (76, 968, 1408), ((16, 64), False): (54, 2656, 384), ((16, 64), True): (110, 1168, 1152),
                      ((32, 32), False): (21, 5200, 896), ((32, 32), True): (18, 7064, 1152), ((32, 64), False): (139, 2304, 640),
                      ((32, 64), True): (23, 9392, 896)}
+# Every kernel of the wave-split tile that quantizes its tokens: (kinds, tokens x channels of the tile, at most so many pieces of eight values a
+# thread, K in whole blocks or in parts, weights cached or of 100 million bytes and more, which are loaded as a stream), and a shape.
+# (K in parts streams where the rows' pitch is a multiple of 128 all the same.)
+QUANT_TILE_KERNELS = [
+    ("token_fp8 int8", 16, 16, 2, "parts", "cached", (17, 40, 48)),
+    ("token_fp8 int8", 16, 16, 4, "parts", "cached", (18, 40, 528)),
+    ("token_fp8 int8", 16, 16, 10, "parts", "cached", (18, 40, 1088)),
+    ("token_fp8 int8", 16, 32, 2, "parts", "cached", (50, 1032, 48)),
+    ("token_fp8 int8", 16, 32, 4, "parts", "cached", (173, 392, 544)),
+    ("token_fp8 int8", 16, 32, 10, "parts", "cached", (15, 4112, 1072)),
+    ("token_fp8 int8", 16, 64, 2, "parts", "cached", (162, 760, 144)),
+    ("token_fp8 int8", 16, 64, 4, "parts", "cached", (199, 656, 528)),
+    ("token_fp8 int8", 16, 64, 10, "parts", "cached", (11, 8232, 1472)),
+    ("token_fp8 int8", 32, 32, 5, "parts", "cached", (17, 176, 1136)),
+    ("token_fp8 int8", 32, 32, 10, "parts", "cached", (401, 600, 656)),
+    ("token_fp8 int8", 32, 64, 5, "parts", "cached", (98, 2312, 48)),
+    ("block ue8m0 token_fp8 int8", 16, 16, 2, "whole", "cached", (17, 40, 128)),
+    ("block ue8m0 token_fp8 int8", 16, 16, 4, "whole", "cached", (17, 40, 640)),
+    ("block ue8m0 token_fp8 int8", 16, 16, 10, "whole", "cached", (18, 40, 1152)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 2, "whole", "cached", (114, 520, 128)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 4, "whole", "cached", (133, 456, 640)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 10, "whole", "cached", (15, 5648, 1152)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 2, "whole", "cached", (194, 624, 256)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 4, "whole", "cached", (227, 552, 640)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 10, "whole", "cached", (12, 8352, 1408)),
+    ("block ue8m0 token_fp8 int8", 32, 32, 5, "whole", "cached", (17, 56, 1152)),
+    ("block ue8m0 token_fp8 int8", 32, 32, 10, "whole", "cached", (371, 664, 768)),
+    ("block ue8m0 token_fp8 int8", 32, 64, 5, "whole", "cached", (194, 1256, 640)),
+    ("block ue8m0", 32, 64, 10, "whole", "cached", (300, 840, 768)),
+    ("token_fp8 int8", 16, 16, 4, "parts", "streamed", (1, 9640, 10864)),
+    ("token_fp8 int8", 16, 32, 2, "parts", "streamed", (1, 17040, 5920)),
+    ("token_fp8 int8", 16, 32, 4, "parts", "streamed", (1, 7192, 13936)),
+    ("token_fp8 int8", 16, 32, 10, "parts", "streamed", (2, 6920, 14624)),
+    ("token_fp8 int8", 16, 64, 2, "parts", "streamed", (3, 69552, 1440)),
+    ("token_fp8 int8", 16, 64, 4, "parts", "streamed", (1, 11160, 9072)),
+    ("token_fp8 int8", 16, 64, 10, "parts", "streamed", (2, 11312, 8880)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 2, "whole", "streamed", (1, 16848, 6912)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 4, "whole", "streamed", (1, 7600, 13312)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 10, "whole", "streamed", (2, 7448, 13440)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 2, "whole", "streamed", (3, 39064, 2560)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 4, "whole", "streamed", (3, 20616, 4864)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 10, "whole", "streamed", (2, 8592, 11648)),
+    ("block ue8m0 token_fp8 int8", 16, 16, 4, "whole", "streamed", (1, 11184, 13312)),
+]
+QUANT_PIECES = {16: (2, 4, 10), 32: (5, 10)}  # by the tile's tokens
+
+
+def quant_tile_kernel(plan: dict, M: int, N: int, K: int, padded: bool = True):
+    """The kernel of QUANT_TILE_KERNELS that a linear with this plan runs, None where its tokens are quantized elsewhere."""
+    if plan["quantizer"] != "fused" or plan["kernel"] != "wavesplit_tile":
+        return None
+    pieces = -(-min(M, plan["bm"]) * -(-K // 128) * 16 // 512)
+    streams = plan["bm"] >= M and M <= 16 and N * K >= 1e8 and (padded or K % 128 == 0)
+    return (plan["bm"], plan["bn"], next(p for p in QUANT_PIECES[plan["bm"]] if pieces <= p), "parts" if K % 128 else "whole",
+            "streamed" if streams else "cached")
 
 
 def linear_variant_of(plan: dict, M: int):

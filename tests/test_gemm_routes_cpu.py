@@ -7,8 +7,8 @@ import time
 import pytest
 
 from gemm_cases import (FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, INT8_CONFIG,
-                        INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, VARIANT_SHAPES, linear_variant_of, plan_for,
-                        variant_of)
+                        INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, VARIANT_SHAPES,
+                        linear_variant_of, plan_for, quant_tile_kernel, variant_of)
 
 LINEARS = ("block", "ue8m0", "token_fp8", "int8")
 
@@ -68,6 +68,26 @@ def test_random_linears_run_only_listed_variants():
         for kind in LINEARS:
             v = linear_variant_of(_lib.linear_plan(kind, M, N, K), M)
             assert v in listed[kind], f"{kind} {(M, N, K)} runs {v}"
+
+
+def test_quantizing_tiles_are_named_and_listed():
+    """QUANT_TILE_KERNELS: each shape runs the kernel it stands for, and random linears run no other."""
+    from sglang_amd import _lib
+
+    listed = {kind: set() for kind in LINEARS}
+    for kinds, *kernel, shape in QUANT_TILE_KERNELS:
+        for kind in kinds.split():
+            assert quant_tile_kernel(_lib.linear_plan(kind, *shape), *shape) == tuple(kernel), (kind, shape)
+            listed[kind].add(tuple(kernel))
+    rng = random.Random(31)
+    spread = lambda low, high: int(low * (high / low) ** rng.random())
+    for _ in range(20000):
+        M, N, K = (spread(1, 16) if rng.random() < 0.5 else spread(17, 1200)), 8 * spread(1, 9000), 16 * spread(1, 1200)
+        K = (K + 127) // 128 * 128 if rng.random() < 0.5 else K
+        for kind in LINEARS if K % 128 == 0 else LINEARS[2:]:
+            if N * K < 2e8:
+                kernel = quant_tile_kernel(_lib.linear_plan(kind, M, N, K), M, N, K)
+                assert kernel is None or kernel in listed[kind], f"{kind} {(M, N, K)} runs {kernel}"
 
 
 def test_mid_tile_sweeps_meet_every_remainder():

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from fp8_tolerance import check_fp8_gemm
-from gemm_cases import LINEAR_SHAPES, QUANT_TILE_SHAPES
+from gemm_cases import LINEAR_SHAPES, QUANT_TILE_KERNELS, QUANT_TILE_SHAPES
 from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
 
 pytestmark = pytest.mark.gpu
@@ -72,7 +72,8 @@ def test_reciprocal_on_every_significand(gpu):
 @pytest.mark.parametrize("tile,many", QUANT_TILE_SHAPES)
 def test_fused_quantizer_above_decode_sizes(gpu, tile, many):
     """One launch against quantizer and GEMM entry point, which runs on a wave-split tile of its own size: the same codes, scales and sums,
-    so the same results bit for bit, with rows that are all zero, infinite or partly NaN."""
+    so the same results bit for bit, with rows that are all zero, infinite or partly NaN.  (Some of the four linears take the named tile; each
+    tile by each linear is QUANT_TILE_KERNELS.)"""
     from sglang_amd import _lib, ops
     from sglang_amd.fp8_kernel import per_token_group_quant_fp8, sglang_per_token_group_quant_fp8, sglang_per_token_quant_fp8, w8a8_block_fp8_matmul
     from sglang_amd.fp8_utils import requant_weight_ue8m0
@@ -107,6 +108,50 @@ def test_fused_quantizer_above_decode_sizes(gpu, tile, many):
         q, s = per_token_quant_int8(xg)
         iw, isc = i_q.to(gpu).t(), i_s.to(gpu)
         assert torch.equal(bits(ops.int8_linear(xg, iw, isc, bias, dtype)), bits(ops.int8_scaled_mm(q, iw, s, isc, dtype, bias)))
+
+
+@pytest.mark.parametrize("kind,kernel,shape", [(kind, kernel, shape) for kinds, *kernel, shape in QUANT_TILE_KERNELS for kind in kinds.split()],
+                         ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_kernel_that_quantizes_in_its_tile(gpu, kind, kernel, shape, dtype):
+    """Small integers whose groups (rows) have a maximum of 448 (127) times a power of two: scales are powers of two, codes the values, and sums
+    exact in any order.  Padded weight rows hold NaN bytes (127) behind K; a row's last value is its maximum.  The kernel that a shape
+    runs is held by the CPU tests."""
+    from sglang_amd import ops
+    from test_gpu_gemm_variants import _words
+
+    M, N, K = shape
+    print(f"case {kind} {kernel} {shape} {dtype}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(M + 3 * N + 5 * K)
+    draw = lambda low, high, *s: torch.randint(low, high, s, generator=g, device=gpu)
+    most, kb, nb = 127 if kind == "int8" else 448, -(-K // 128), -(-N // 128)
+    v = draw(-3, 4, M, K).double()
+    if kind in ("block", "ue8m0"):
+        v.view(M, kb, 128)[:, :, 127] = most * (1 - 2 * draw(0, 2, M, kb))
+        v = (v.view(M, kb, 128) * torch.exp2(draw(-2, 3, M, kb).double())[:, :, None]).reshape(M, K)
+    else:
+        v[:, K - 1] = most * (1 - 2 * draw(0, 2, M))
+        v = v * torch.exp2(draw(-2, 3, M).double())[:, None]
+    x = v.to(dtype)
+    assert torch.equal(x.double(), v)
+    pitch = (K + 127) // 128 * 128
+    codes = torch.full((N, pitch), 127, dtype=torch.uint8, device=gpu)  # (NaN as FP8)
+    wv = draw(-2, 3, N, K)
+    codes[:, :K] = (wv.to(torch.int8) if kind == "int8" else wv.half().to(torch.float8_e4m3fn)).view(torch.uint8)
+    w = codes.view(torch.int8 if kind == "int8" else torch.float8_e4m3fn)[:, :K]
+    if kernel[4] == "cached" and K % 128:  # dense rows: the next row's bytes lie behind K
+        w = w.contiguous()
+    if kind in ("block", "ue8m0"):
+        eb = draw(125, 130, nb, kb)
+        full = torch.exp2(eb.double() - 127).repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)[:, :K]
+        want = v @ (wv * full).t()
+        out = ops.block_fp8_linear(x, w, torch.exp2(eb.float() - 127), None, dtype) if kind == "block" else \
+            ops.block_fp8_linear_ue8m0(x, w, _words(eb.repeat_interleave(128, dim=0)[:N]), None, dtype)
+    else:
+        sb = torch.exp2(draw(-3, 4, N).float())
+        want = (v @ wv.double().t()) * sb.double()
+        out = (ops.int8_linear if kind == "int8" else ops.fp8_per_token_linear)(x, w.t(), sb, None, dtype)
+    assert torch.equal(out, want.float().to(dtype))
 
 
 # every kernel that quantizes tokens itself: (kinds, kernel, channel tile or waves, shape)

@@ -44,7 +44,7 @@ def test_parts_of_blocks_exact(gpu, shape, tile):
 
 
 # last blocks of 16 to 112 values, one block, rows that share a DPP row of sixteen pieces with no other, several token tiles, the most values a
-# tile quantizes (40960), every tile height
+# tile quantizes (40960); every kernel that does it: QUANT_TILE_KERNELS in gemm_cases.py
 QUANTIZED = [(1, 136, 16), (3, 264, 112), (16, 576, 144), (5, 1032, 4112), (6, 2056, 6768), (16, 16400, 304), (45, 264, 272), (66, 264, 1200), (33, 4104, 1008), (2, 520, 20464), (16, 520, 1520),
              (700, 320, 368), (100, 4000, 272)]
 
