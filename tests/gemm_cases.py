@@ -255,6 +255,26 @@ QUANT_TILE_SHAPES = {((16, 16), False): (143, 24, 640), ((16, 16), True): (49, 1
                      ((16, 32), True): (76, 968, 1408), ((16, 64), False): (54, 2656, 384), ((16, 64), True): (110, 1168, 1152),
                      ((32, 32), False): (21, 5200, 896), ((32, 32), True): (18, 7064, 1152), ((32, 64), False): (139, 2304, 640),
                      ((32, 64), True): (23, 9392, 896)}
+# K in parts of blocks (one scale per token and channel, INT8): (shape, mid-M tile and LDS stages that run), every tile from three blocks on,
+# fewer blocks than stages among them; and K of two blocks
+RAGGED_TILE_SHAPES = [
+    ((17, 17208, 272), (64, 128, 6)), ((17, 36192, 272), (64, 128, 3)), ((17, 36192, 400), (64, 192, 4)), ((33, 17208, 656), (64, 128, 6)),
+    ((20, 16392, 6160), (64, 128, 6)), ((17, 45656, 304), (64, 192, 4)), ((396, 8888, 1456), (64, 256, 3)), ((71, 18736, 400), (96, 128, 5)),
+    ((70, 33408, 272), (96, 192, 4)), ((272, 16456, 288), (96, 256, 3)), ((97, 24888, 928), (128, 128, 4)), ((207, 17048, 288), (128, 192, 3)),
+    ((215, 25152, 272), (128, 256, 3)), ((133, 24744, 352), (160, 128, 4)), ((136, 35040, 272), (160, 192, 3)), ((331, 12432, 368), (192, 128, 3)),
+    ((667, 10824, 272), (256, 128, 3)),
+    ((3275, 528, 240), (64, 128, 3)), ((2002, 400, 176), (64, 128, 6)), ((1802, 2192, 144), (96, 192, 4)), ((389, 10920, 208), (96, 256, 3)),
+    ((193, 16752, 240), (128, 192, 3)), ((3051, 2344, 192), (128, 256, 3)), ((3471, 1168, 160), (160, 128, 4)), ((3703, 1560, 160), (160, 192, 3)),
+    ((490, 8408, 224), (192, 128, 3)), ((3279, 2336, 144), (256, 128, 3)),
+]
+# The same on weights of 100 million bytes and more whose rows lie a multiple of 128 bytes apart all the same: loaded as a stream.  (shape,
+# kernel and its tile)
+STREAMED_RAGGED_SHAPES = [
+    ((14, 23168, 4320), ("dma3", 64, 128)), ((25, 32224, 3104), ("dma3", 64, 128)), ((10, 46304, 2160), ("dma3", 64, 192)),
+    ((33, 35752, 2800), ("dma3", 64, 192)), ((2, 57024, 1760), ("dma3", 64, 256)), ((50, 53480, 1872), ("dma3", 64, 256)),
+    ((2, 9080, 11088), ("wavesplit_tile", 16, 16)), ((6, 18664, 5360), ("wavesplit_tile", 16, 32)), ((2, 16032, 6240), ("wavesplit_tile", 16, 64)),
+]
+
 # Every kernel of the wave-split tile that quantizes its tokens: (kinds, tokens x channels of the tile, at most so many pieces of eight values a
 # thread, K in whole blocks or in parts, weights cached or of 100 million bytes and more, which are loaded as a stream), and a shape.
 # (K in parts streams where the rows' pitch is a multiple of 128 all the same.)

@@ -7,8 +7,8 @@ import time
 import pytest
 
 from gemm_cases import (FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, INT8_CONFIG,
-                        INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, VARIANT_SHAPES,
-                        linear_variant_of, plan_for, quant_tile_kernel, variant_of)
+                        INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, RAGGED_TILE_SHAPES,
+                        STREAMED_RAGGED_SHAPES, VARIANT_SHAPES, linear_variant_of, plan_for, quant_tile_kernel, variant_of)
 
 LINEARS = ("block", "ue8m0", "token_fp8", "int8")
 
@@ -68,6 +68,16 @@ def test_random_linears_run_only_listed_variants():
         for kind in LINEARS:
             v = linear_variant_of(_lib.linear_plan(kind, M, N, K), M)
             assert v in listed[kind], f"{kind} {(M, N, K)} runs {v}"
+
+
+@pytest.mark.parametrize("kind", ["fp8_scaled", "int8"])
+def test_parts_of_blocks_run_the_named_tiles(kind):
+    for shape, tile in RAGGED_TILE_SHAPES:
+        p = plan_for(kind, *shape)
+        assert ("dma3", 1, *tile) == (p["kernel"], p["splits"], p["bm"], p["bn"], p["stages"]), (shape, p)
+    for shape, kernel in STREAMED_RAGGED_SHAPES:
+        p = plan_for(kind, *shape)
+        assert kernel == (p["kernel"], p["bm"], p["bn"]) and p["splits"] == 1 and shape[0] <= p["bm"] and shape[1] * shape[2] >= 1e8, (shape, p)
 
 
 def test_quantizing_tiles_are_named_and_listed():

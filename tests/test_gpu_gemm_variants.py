@@ -21,15 +21,22 @@ def _words(e):
     return buf.t()[:rows]
 
 
-def check_exact(gpu, kind, M, N, K, pitch=None):
-    """`pitch`: elements between the weight's rows."""
+def check_exact(gpu, kind, M, N, K, pitch=None, behind=1, token_pitch=None):
+    """`pitch`: elements between the weight's rows, with the bytes `behind` after each (127 is a NaN as FP8); `token_pitch`: between the tokens'."""
     from sglang_amd import ops
 
     g = torch.Generator(device=gpu).manual_seed(M + 3 * N + 5 * K)
     draw = lambda low, high, *shape: torch.randint(low, high, shape, generator=g, device=gpu)
     a, w = draw(-2, 3, M, K), draw(-2, 3, N, K)
     kb, nb = -(-K // 128), -(-N // 128)
-    pad = lambda t: torch.nn.functional.pad(t, (0, pitch - K), value=1)[:, :K] if pitch else t
+    pad = lambda t: torch.nn.functional.pad(t, (0, pitch - K), value=behind)[:, :K] if pitch else t
+
+    def apart(t):
+        if token_pitch is None:
+            return t
+        rows = torch.empty((M - 1) * token_pitch + K, dtype=torch.uint8, device=gpu).as_strided((M, K), (token_pitch, 1))
+        return rows.copy_(t.view(torch.uint8)).view(t.dtype)
+
     if kind in ("fp8", "fp8_ue8m0"):
         ea, eb = draw(125, 130, M, kb), draw(125, 130, nb, kb)
         ta, tb = torch.exp2(ea.double() - 127), torch.exp2(eb.double() - 127)
@@ -47,9 +54,9 @@ def check_exact(gpu, kind, M, N, K, pitch=None):
         product = a.double() @ w.double().t()
         want = product * sa.double()[:, None] * sb.double() + bias.double()
         if kind == "fp8_scaled":
-            out = ops.fp8_scaled_mm(a.float().to(FP8), pad(w.float().to(FP8).view(torch.uint8)).view(FP8).t(), sa, sb, torch.bfloat16, bias)
+            out = ops.fp8_scaled_mm(apart(a.float().to(FP8)), pad(w.float().to(FP8).view(torch.uint8)).view(FP8).t(), sa, sb, torch.bfloat16, bias)
         else:
-            a8, w8 = a.to(torch.int8), pad(w.to(torch.int8))
+            a8, w8 = apart(a.to(torch.int8)), pad(w.to(torch.int8))
             assert torch.equal(ops.int8_mm_raw_accumulators(a8, w8.t()).double(), product), (kind, M, N, K)
             out = ops.int8_scaled_mm(a8, w8.t(), sa, sb, torch.bfloat16, bias)
     assert torch.equal(out, want.float().to(torch.bfloat16)), (kind, M, N, K)
@@ -102,6 +109,13 @@ def test_rotated_k(gpu, kind, M, N, K):
 def test_weight_rows_of_any_pitch(gpu, kind, M, N, K, pitch):
     print(f"case {kind} {(M, N, K)} pitch {pitch}", flush=True)
     check_exact(gpu, kind, M, N, K, pitch)
+
+
+# tokens whose rows span more than 4 GiB stay on the kernel of 64-bit offsets, in tiles of 256 tokens with K split and whole
+@pytest.mark.parametrize("kind", ["fp8_scaled", "int8"])
+@pytest.mark.parametrize("M,N,K", [(1052, 6688, 928), (1052, 6688, 128), (70, 520, 1040)])
+def test_token_rows_over_four_gigabytes(gpu, kind, M, N, K):
+    check_exact(gpu, kind, M, N, K, token_pitch=(1 << 32) // M // 16 * 16 + 32)
 
 
 # weights of 100 million bytes and more are loaded as a stream where one token tile reads them: every height of the mid-M tile, K split and
