@@ -255,6 +255,33 @@ QUANT_TILE_SHAPES = {((16, 16), False): (143, 24, 640), ((16, 16), True): (49, 1
                      ((16, 32), True): (76, 968, 1408), ((16, 64), False): (54, 2656, 384), ((16, 64), True): (110, 1168, 1152),
                      ((32, 32), False): (21, 5200, 896), ((32, 32), True): (18, 7064, 1152), ((32, 64), False): (139, 2304, 640),
                      ((32, 64), True): (23, 9392, 896)}
+# Grouped calls by the rows of each expert: (name, rows, N, K, small tile that runs)
+GROUPED_SHAPES = [
+    ("decode_like", [1, 0, 3, 1, 0, 0, 2, 8, 1, 1, 0, 5, 16, 1, 2, 1], 512, 7168, "16x64"),
+    ("one_token", [1], 256, 128, "16x16"),
+    ("empty_experts_around_a_big_one", [0, 0, 700, 0, 1, 0], 384, 512, "32x64"),
+    ("prefill_like", [130, 257, 128, 64, 511, 129, 300, 200], 768, 1024, "64x128"),
+    ("tile_edges", [64, 65, 63, 128, 127, 129, 1, 256], 256, 256, "16x64"),
+    ("many_small", [3] * 300, 128, 256, "64x128"),
+    ("large_experts", [1000, 513, 384, 2], 512, 512, "64x128"),
+    ("ragged_channels", [40, 90, 17], 200, 384, "16x16"),
+    ("decode_like_wide", [1, 0, 3, 1, 0, 0, 2, 8, 1, 1, 0, 5, 16, 1, 2, 1], 1664, 7168, "64x128"),
+    ("empty_experts_around_a_big_one_wide", [0, 0, 700, 0, 1, 0], 1280, 512, "64x128"),
+    ("tile_edges_wide", [64, 65, 63, 128, 127, 129, 1, 256], 1024, 256, "64x256"),
+    ("large_experts_wide", [1000, 513, 384, 2], 640, 512, "64x128"),
+    ("ragged_channels_wide", [40, 90, 17], 4424, 384, "64x128"),
+]
+# Grouped calls: experts (uneven: some without a row, one with many), stacked rows, N, K, and the kernel and small tile that run
+GROUPED_FORMS = [
+    (40, 1240, 2056, 128, "grouped_dma3", "64x256"), (2, 3254, 328, 384, "grouped_dma3", "64x128"),
+    (16, 16, 64, 384, "grouped_wavesplit", "16x16"), (8, 209, 416, 128, "grouped_wavesplit", "16x32"), (40, 29, 392, 1152, "grouped_wavesplit", "16x64"),
+    (5, 56, 1240, 128, "grouped_wavesplit", "32x32"), (40, 492, 272, 128, "grouped_wavesplit", "32x64"), (40, 1798, 136, 128, "grouped_wavesplit", "64x64"),
+    (24, 1574, 128, 128, "grouped_wavesplit", "16x64"), (16, 1613, 224, 128, "grouped_wavesplit", "64x64"), (3, 545, 1544, 1152, "grouped_dma3", "64x128"),
+    (40, 29, 2056, 128, "grouped_dma3", "64x128"),  # (more workgroups than CUs: two share one)
+    (24, 1233, 2056, 384, "grouped_dma3", "128x256"), (16, 2075, 2056, 384, "grouped_dma3", "128x256"),
+    (1, 1695, 2056, 640, "grouped_dma3", "128x128"), (24, 3078, 768, 2048, "grouped_dma3", "128x128"),
+    (2, 5548, 2056, 384, "grouped_pingpong+grouped_dma3", "128x256")]
+
 # K in parts of blocks (one scale per token and channel, INT8): (shape, mid-M tile and LDS stages that run), every tile from three blocks on,
 # fewer blocks than stages among them; and K of two blocks
 RAGGED_TILE_SHAPES = [

@@ -6,7 +6,7 @@ import time
 
 import pytest
 
-from gemm_cases import (FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, INT8_CONFIG,
+from gemm_cases import (FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, GROUPED_FORMS, GROUPED_SHAPES, INT8_CONFIG,
                         INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, RAGGED_TILE_SHAPES,
                         STREAMED_RAGGED_SHAPES, VARIANT_SHAPES, linear_variant_of, plan_for, quant_tile_kernel, variant_of)
 
@@ -68,6 +68,16 @@ def test_random_linears_run_only_listed_variants():
         for kind in LINEARS:
             v = linear_variant_of(_lib.linear_plan(kind, M, N, K), M)
             assert v in listed[kind], f"{kind} {(M, N, K)} runs {v}"
+
+
+def test_grouped_shapes_run_the_named_tiles():
+    from sglang_amd import _lib
+
+    for name, sizes, N, K, tile in GROUPED_SHAPES:
+        assert _lib.grouped_gemm_plan(len(sizes), sum(sizes), N, K)["small_tile"] == tile, name
+    for E, rows, N, K, kernel, tile in GROUPED_FORMS:
+        plan = _lib.grouped_gemm_plan(E, rows, N, K)
+        assert (plan["kernel"], plan["small_tile"]) == (kernel, tile), (E, rows, N, K)
 
 
 @pytest.mark.parametrize("kind", ["fp8_scaled", "int8"])

@@ -4,6 +4,7 @@ chunk, several experts and none in one, more experts than one scan takes, K of a
 import pytest
 import torch
 
+from gemm_cases import GROUPED_FORMS
 from test_gpu_fp8_grouped_gemm import _call, _problem, _verify
 
 pytestmark = pytest.mark.gpu
@@ -33,24 +34,9 @@ def test_grouped(gpu, oracle, name, sizes, N, K, m_major):
     _verify(oracle, out, a, w, sa, sw, sizes, offsets, name)
 
 
-# experts (uneven: some without a row, one with many), stacked rows, N, K -> what has to run
-FORMS = [(40, 1240, 2056, 128, "grouped_dma3", "64x256"), (2, 3254, 328, 384, "grouped_dma3", "64x128"),
-         (16, 16, 64, 384, "grouped_wavesplit", "16x16"), (8, 209, 416, 128, "grouped_wavesplit", "16x32"), (40, 29, 392, 1152, "grouped_wavesplit", "16x64"),
-         (5, 56, 1240, 128, "grouped_wavesplit", "32x32"), (40, 492, 272, 128, "grouped_wavesplit", "32x64"), (40, 1798, 136, 128, "grouped_wavesplit", "64x64"),
-         (24, 1574, 128, 128, "grouped_wavesplit", "16x64"), (16, 1613, 224, 128, "grouped_wavesplit", "64x64"), (3, 545, 1544, 1152, "grouped_dma3", "64x128"),
-         (40, 29, 2056, 128, "grouped_dma3", "64x128"),  # (more workgroups than CUs: two share one)
-         (24, 1233, 2056, 384, "grouped_dma3", "128x256"), (16, 2075, 2056, 384, "grouped_dma3", "128x256"),
-         (1, 1695, 2056, 640, "grouped_dma3", "128x128"), (24, 3078, 768, 2048, "grouped_dma3", "128x128"),
-         (2, 5548, 2056, 384, "grouped_pingpong+grouped_dma3", "128x256")]
-
-
-@pytest.mark.parametrize("E,rows,N,K,kernel,tile", FORMS)
-def test_every_tiling(gpu, oracle, E, rows, N, K, kernel, tile):
-    from sglang_amd import _lib
-
-    plan = _lib.grouped_gemm_plan(E, rows, N, K)
-    print(f"case {E} {rows} {N} {K} {plan}", flush=True)
-    assert (plan["kernel"], plan["small_tile"]) == (kernel, tile)
+@pytest.mark.parametrize("E,rows,N,K", [form[:4] for form in GROUPED_FORMS])
+def test_every_tiling(gpu, oracle, E, rows, N, K):
+    print(f"case {E} {rows} {N} {K}", flush=True)
     g = torch.Generator().manual_seed(E + rows)
     weight = torch.rand(E, generator=g) + 0.1
     weight[E // 2] += E / 4

@@ -10,7 +10,7 @@ from gemm_cases import RAGGED_TILE_SHAPES, STREAMED_RAGGED_SHAPES
 pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
 
-SHAPES = [shape for shape, _ in RAGGED_TILE_SHAPES] + [(3, 15000, 6704)]
+SHAPES = [shape for shape, _ in RAGGED_TILE_SHAPES] + [(3, 15000, 6704), (65, 25352, 912), (1052, 6688, 928)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=str)
