@@ -345,6 +345,7 @@ QUANT_TILE_KERNELS = [
     ("block ue8m0 token_fp8 int8", 16, 64, 4, "whole", "streamed", (3, 20616, 4864)),
     ("block ue8m0 token_fp8 int8", 16, 64, 10, "whole", "streamed", (2, 8592, 11648)),
     ("block ue8m0 token_fp8 int8", 16, 16, 4, "whole", "streamed", (1, 11184, 13312)),
+    ("block ue8m0 token_fp8 int8", 16, 16, 10, "whole", "streamed", (1, 2504, 40576)), ("token_fp8 int8", 16, 16, 10, "parts", "streamed", (1, 3760, 27040)),
 ]
 QUANT_PIECES = {16: (2, 4, 10), 32: (5, 10)}  # by the tile's tokens
 
