@@ -398,6 +398,8 @@ int mi355_fp8_scaled_mm(const void* a, const void* b, const float* sa, const flo
  *          kernel, that is where mi355_fp8_block_linear_plan without its last key equals mi355_fp8_blockwise_mm_plan, and
  *          wherever both name the wave-split tile: tiles of any size add the same products in the same order.  Above 16 tokens
  *          that tile quantizes too where its tokens hold few values (layers of short K), in any of the four linears.
+ *          Where that one launch takes the GPU longer than two and only the host less, a call on a stream that is being captured
+ *          takes two (the same bits); the plan queries name what an eager call runs.
  *          mi355_fp8_block_linear_plan (host only, dense 16-byte aligned operands and 16-bit x assumed) writes the GEMM that
  *          runs in the format of mi355_fp8_blockwise_mm_plan followed by quantizer=fused|launch.
  *   x [M, K] contiguous F32/F16/BF16, K % 128 == 0; w [N, K] e4m3fn row stride ldw; w_scale element (nb, kb) at

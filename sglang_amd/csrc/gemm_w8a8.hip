@@ -1261,15 +1261,18 @@ bool tile_quant_takes(WavesplitQuant quant, int64_t K) {
   return K % (quant == WavesplitQuant::TOKEN_FP8 || quant == WavesplitQuant::TOKEN_INT8 ? 16 : KSTEP) == 0;
 }
 // The wave-split tile quantizing the tokens itself, where the GEMM takes that tile (same sums, bit for bit): the launch saved
-// against the quantizer's work in every workgroup, v pieces per thread and round.  K in parts of blocks, where a piece takes more: beyond
-// six pieces only up to six tokens, whose launch has a long row for each workgroup (120 linears in a graph, launch in front / this: INT8 3 tokens
-// 9664 -> 14080 41.1 / 31.4, 3 tokens 10432 -> 768 9.4 / 8.8, 4 tokens per-token FP8 8352 -> 6016 17.1 / 16.3; 27 of seven tokens and more 1.08,
-// INT8 13 tokens 2784 -> 1152 6.3 / 7.6, per-token FP8 15 tokens 2016 -> 640 5.6 / 6.25).
+// against the quantizer's work in every workgroup, v pieces per thread and round.
 bool tile_quant_preferred(WavesplitQuant quant, const Route& run, int64_t M, int64_t N, int64_t K) {
   if (run.kernel != RK_WAVESPLIT_TILE || M > 16 || !tile_quant_takes(quant, K)) return false;
   const int64_t pieces = M * ((K + KSTEP - 1) / KSTEP) * (KSTEP / 8), threads = 512, rounds = (N + (int64_t)run.bn * NUM_CUS - 1) / ((int64_t)run.bn * NUM_CUS);
-  const int64_t most = K % KSTEP == 0 || M <= 6 ? 10 : 6;
-  return pieces <= most * threads && pieces * rounds <= 10 * threads;
+  return pieces <= 10 * threads && pieces * rounds <= 10 * threads;
+}
+// K in parts of blocks, where a piece takes more: beyond six pieces, from seven tokens on, the launch's host time is all that is saved (up to six
+// tokens it has a long row for each workgroup).  Launch in front / this, us in a graph: INT8 3 tokens 9664 -> 14080 41.1 / 31.4, 3 tokens
+// 10432 -> 768 9.4 / 8.8, 4 tokens per-token FP8 8352 -> 6016 17.1 / 16.3; 27 linears of seven tokens and more 1.08 in a graph, 0.94 eager: INT8
+// 13 tokens 2784 -> 1152 6.3 / 7.6, per-token FP8 15 tokens 2016 -> 640 5.6 / 6.25.
+bool tile_quant_eager_only(int64_t M, int64_t K) {
+  return K % KSTEP != 0 && M > 6 && M * ((K + KSTEP - 1) / KSTEP) * (KSTEP / 8) > 6 * 512;
 }
 bool fused_quant_preferred(int64_t M, int64_t N, int64_t K, int64_t ldw) {
   const int plain = choose_route(true, M, N, K, K, ldw, true).kernel;
@@ -1288,17 +1291,19 @@ enum LinearMode { LM_LAUNCH, LM_LAUNCH_OWN, LM_TILE, LM_WAVESPLIT, LM_PRODUCER, 
 struct LinearRoute {
   LinearMode mode;
   Route gemm;
+  bool eager_only = false;  // LM_TILE: in a capture the quantizer's launch and the GEMM's own route, for the same bits
 };
 LinearRoute uncached_choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K, int64_t ldw, bool q_ok, bool w_aligned) {
   const GemmKind kind = quant == WavesplitQuant::BLOCK_F32 ? GK_F32 : quant == WavesplitQuant::BLOCK_UE8M0 ? GK_UE8M0 : quant == WavesplitQuant::TOKEN_FP8 ? GK_UNIT : GK_INT8;
   const Route run = run_route(kind, M, N, K, K, ldw, w_aligned && K % 16 == 0);
   if (!q_ok) return {LM_LAUNCH, run};
-  if (tile_quant_preferred(quant, run, M, N, K)) return {LM_TILE, run};
+  if (tile_quant_preferred(quant, run, M, N, K)) return {LM_TILE, run, tile_quant_eager_only(M, K)};
   if (M > 16 && run.kernel == RK_WAVESPLIT_TILE && tile_quant_takes(quant, K)) {
-    const TileChoice c = choose_quant_tile(kind, M, N, (K + KSTEP - 1) / KSTEP * KSTEP, run.bm, run.bn);
+    bool eager_only;
+    const TileChoice c = choose_quant_tile(kind, M, N, (K + KSTEP - 1) / KSTEP * KSTEP, run.bm, run.bn, eager_only);
     Route r = run;
     r.bm = c.bm, r.bn = c.bn;
-    if (c.family != TF_NONE) return {LM_TILE, r};
+    if (c.family != TF_NONE) return {LM_TILE, r, eager_only};
   }
   // (rows 4096 bytes apart: the mid-M tile proper, which starts its K loops at different blocks; 4096 -> 24576 at 16 tokens 26.2 / 23.7)
   const LinearMode producer_mode = rotates_k(N, K, ldw) ? LM_LAUNCH_OWN : LM_PRODUCER;
@@ -1340,6 +1345,19 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
   };
   static thread_local RecentShapes<Key, LinearRoute> table;
   return table.get(Key{{M, N, K, (int)quant}, ldw, q_ok, w_aligned}, [&] { return uncached_choose_linear(quant, M, N, K, ldw, q_ok, w_aligned); });
+}
+bool being_captured(void* stream) {
+  if (stream == nullptr) return false;  // (the null stream never is; asked about while another stream is, it would end that capture)
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
+// What a call on `stream` does; the plan queries name what an eager one does.
+LinearRoute linear_route(WavesplitQuant quant, int64_t M, int64_t N, int64_t K, int64_t ldw, bool q_ok, bool w_aligned, void* stream) {
+  LinearRoute r = choose_linear(quant, M, N, K, ldw, q_ok, w_aligned);
+  if (r.eager_only && being_captured(stream)) r.mode = LM_LAUNCH;
+  return r;
 }
 int run_tile_quant(GemmParams& p, WavesplitQuant kind, const Route& run, const void* x, int x_dtype, void* stream, const char* what) {
   p.x16 = x, p.ldx = p.K, p.x_dtype = x_dtype;
@@ -1396,7 +1414,7 @@ int block_linear(const char* what, const void* x, int x_dtype, int quant_mode, c
   // Decode sizes: the GEMM kernel quantizes the tokens itself (same arithmetic), no quantizer launch - except where a
   // quantizer launch in front of the wave-split kernel is measured faster (route_constants.h).
   const bool w_aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 16 == 0;
-  const LinearRoute linear = choose_linear(WavesplitQuant::BLOCK_F32, M, N, K, ldw, wavesplit_quant_operands(x, x_dtype, w, ldw), w_aligned);
+  const LinearRoute linear = linear_route(WavesplitQuant::BLOCK_F32, M, N, K, ldw, wavesplit_quant_operands(x, x_dtype, w, ldw), w_aligned, stream);
   if (linear.mode != LM_LAUNCH && linear.mode != LM_LAUNCH_OWN) {
     GemmParams p;
     bool empty;
@@ -1536,7 +1554,7 @@ extern "C" int mi355_int8_linear(const void* x, int x_dtype, const void* w, cons
   p.lda = K, p.ldb = ldw, p.ldo = ldo;
   p.out_dtype = out_dtype;
   const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);
-  const LinearRoute linear = choose_linear(WavesplitQuant::TOKEN_INT8, M, N, K, ldw, q_ok, q_ok);
+  const LinearRoute linear = linear_route(WavesplitQuant::TOKEN_INT8, M, N, K, ldw, q_ok, q_ok, stream);
   if (linear.mode == LM_TILE) return run_tile_quant(p, WavesplitQuant::TOKEN_INT8, linear.gemm, x, x_dtype, stream, what);
   if (linear.mode == LM_WAVESPLIT) return run_wavesplit_quant(p, WavesplitQuant::TOKEN_INT8, x, x_dtype, stream, what);
   const int rc = mi355_per_token_quant_int8(x, x_dtype, q, sa, M, K, stream);
@@ -1573,7 +1591,7 @@ int per_token_linear(const char* what, const void* x, int x_dtype, const float* 
   float* sa = reinterpret_cast<float*>(q + q_bytes);
   const size_t sa_bytes = align256((size_t)M * 4u);
   const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);
-  const LinearRoute linear = choose_linear(WavesplitQuant::TOKEN_FP8, M, N, K, ldw, q_ok, q_ok);
+  const LinearRoute linear = linear_route(WavesplitQuant::TOKEN_FP8, M, N, K, ldw, q_ok, q_ok, stream);
   if (linear.mode != LM_LAUNCH) {
     GemmParams p;
     bool empty;
@@ -1640,7 +1658,7 @@ extern "C" int mi355_fp8_block_linear_ue8m0(const void* x, int x_dtype, const vo
   const int64_t pitch = (M + 3) & ~3ll;
   const size_t sa_bytes = align256((size_t)pitch * (size_t)((K / KSTEP + 3) / 4) * 4u);
   const bool q_ok = wavesplit_quant_operands(x, x_dtype, w, ldw);
-  const LinearRoute linear = choose_linear(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw, q_ok, q_ok);
+  const LinearRoute linear = linear_route(WavesplitQuant::BLOCK_UE8M0, M, N, K, ldw, q_ok, q_ok, stream);
   if (linear.mode != LM_LAUNCH) {
     GemmParams p;
     bool empty;

@@ -46,8 +46,8 @@ struct StreamedTimes {
   double launch = 3.0, block = 0.098, block_channel = 0.00236, block_token = 0.00264, shared = 2.0, mid_stream = 7.06, mid_stream_us = 3.32;
 };
 // More than 16 tokens quantized inside the wave-split tile (choose_quant_tile), one round of workgroups: launch + tile + pieces of eight values a
-// thread * piece (by GemmKind), `many` more for the kernel of ten + KB of weight * kb * (1 + kb_busy * fill) + kilo-elements of the tile * result.  `saved`: what the quantizer's
-// launch takes beside the wave-split tile's modelled time.
+// thread * piece (by GemmKind) + KB of weight * kb * (1 + kb_busy * fill) + kilo-elements of the tile * result.  `saved`: what the quantizer's
+// launch takes beside the wave-split tile's modelled time; `many`: see there.
 struct QuantTimes {
   double launch = 1.29, tile = 1.32, piece[4] = {0.310, 0.295, 0.370, 0.377}, many = 0.55, kb = 0.0051, kb_busy = 2.54, result = 0.488, saved = 1.4;
 };
@@ -258,24 +258,28 @@ TileChoice best_resident(GemmKind kind, int64_t M, int64_t N, int64_t K) {
 // for layers of short K, as long as one round of workgroups does it (a second one never: 42 tokens 1536 -> 12288 16.3 us, two launches
 // 10.3), and where the tile's tokens are at most ten pieces of eight values a thread.
 // Fitted to 1600 timings of 320 linears: 6 % root mean square, the tile it names within 0.2 % of the best on average; `many` is what 16-token tiles
-// take beyond four pieces, in the kernel of ten, by 160 more.  240 linears on this side of the line, one launch / two: 0.82 of the time in a graph
-// (at most 1.04, but for two of 1.06 and 1.18), 0.64 eager; us in a graph, two launches / this: 18 tokens 512 -> 896 5.0 / 3.5, 669 tokens packed
-// exponents 640 -> 384 6.8 / 4.3, 69 tokens per-token FP8 768 -> 384 5.3 / 4.2, INT8 103 tokens 768 -> 768 5.6 / 4.35; on the other side
-// 173 tokens packed exponents 2048 -> 256 5.5 / 6.7, 48 tokens 2048 -> 768 5.8 / 6.6, INT8 121 tokens 1536 -> 384 5.6 / 6.5, per-token FP8 23 tokens
-// 1792 -> 4096 5.8 / 6.4 (eager those 21 took 0.7 of the two launches' time: the line is drawn by what the GPU does).
-TileChoice choose_quant_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, int plain_bm, int plain_bn) {
+// take beyond four pieces, in the kernel of ten, by 160 more.  240 linears where one launch models no slower, one launch / two: 0.82 of the
+// time in a graph (at most 1.04, but for two of 1.06 and 1.18), 0.64 eager; us in a graph, two launches / this: 18 tokens 512 -> 896 5.0 / 3.5,
+// 669 tokens packed exponents 640 -> 384 6.8 / 4.3, 69 tokens per-token FP8 768 -> 384 5.3 / 4.2, INT8 103 tokens 768 -> 768 5.6 / 4.35.
+// `eager_only`: with `many` it takes more of the GPU's time than two launches, less than the 2.4 us that a launch takes on the host; not in a
+// capture, where they are not spent.  19 such linears 1.06 (0.94 to 1.23) of the two launches' time in a graph, 0.70 eager; graph, eager: 173 tokens packed exponents
+// 2048 -> 256 5.5 / 6.7, 9.5 / 6.7; 48 tokens 2048 -> 768 5.8 / 6.6, 8.8 / 6.6; INT8 121 tokens 1536 -> 384 5.6 / 6.5, 8.9 / 6.4.
+TileChoice choose_quant_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, int plain_bm, int plain_bn, bool& eager_only) {
   const QuantTimes& q = tile_model().quant;
   double two_launches = 0.0;
   for (int i = 0; i < (int)(sizeof(WAVESPLIT_TILES) / sizeof(WAVESPLIT_TILES[0])); ++i)
     if (WAVESPLIT_TILES[i].bm == plain_bm && WAVESPLIT_TILES[i].bn == plain_bn) two_launches = wavesplit_tile_us(tile_times(kind), i, M, N, K) + q.saved;
   TileChoice best{TF_NONE, 0, 0, 1, two_launches};
+  eager_only = false;
   for (const TileSize& t : WAVESPLIT_QUANT_TILES) {
     const int64_t values = std::min<int64_t>(M, t.bm) * K, wg = ceil_div(M, t.bm) * ceil_div(N, t.bn);
     if (values > WAVESPLIT_QUANT_VALUES || wg > NUM_CUS) continue;
     const int64_t pieces = ceil_div(values, WAVESPLIT_QUANT_VALUES / 10);
-    const double us = q.launch + q.tile + (double)pieces * q.piece[kind] + (t.bm == 16 && pieces > 4 ? q.many : 0.0) +
-                      (double)(t.bn * K) * 1e-3 * q.kb * (1.0 + q.kb_busy * (double)wg / NUM_CUS) + (double)(t.bm * t.bn) / 1024.0 * q.result;
-    if (us < best.us) best = {TF_WAVESPLIT, t.bm, t.bn, 1, us};
+    const double us = q.launch + q.tile + (double)pieces * q.piece[kind] + (double)(t.bn * K) * 1e-3 * q.kb * (1.0 + q.kb_busy * (double)wg / NUM_CUS) +
+                      (double)(t.bm * t.bn) / 1024.0 * q.result;
+    if (us >= best.us) continue;
+    best = {TF_WAVESPLIT, t.bm, t.bn, 1, us};
+    eager_only = t.bm == 16 && pieces > 4 && us + q.many >= two_launches;
   }
   return best;
 }

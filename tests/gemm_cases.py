@@ -311,11 +311,11 @@ QUANT_TILE_KERNELS = [
     ("token_fp8 int8", 16, 16, 10, "parts", "cached", (18, 40, 1088)),
     ("token_fp8 int8", 16, 32, 2, "parts", "cached", (50, 1032, 48)),
     ("token_fp8 int8", 16, 32, 4, "parts", "cached", (173, 392, 544)),
-    ("token_fp8 int8", 16, 32, 10, "parts", "cached", (15, 4112, 1072)),
+    ("token_fp8 int8", 16, 32, 10, "parts", "cached", (133, 464, 1104)),
     ("token_fp8 int8", 16, 64, 2, "parts", "cached", (162, 760, 144)),
     ("token_fp8 int8", 16, 64, 4, "parts", "cached", (199, 656, 528)),
-    ("token_fp8 int8", 16, 64, 10, "parts", "cached", (11, 8232, 1472)),
-    ("token_fp8 int8", 32, 32, 5, "parts", "cached", (17, 176, 1136)),
+    ("token_fp8 int8", 16, 64, 10, "parts", "cached", (257, 496, 1040)),
+    ("token_fp8 int8", 32, 32, 5, "parts", "cached", (66, 1688, 48)),
     ("token_fp8 int8", 32, 32, 10, "parts", "cached", (401, 600, 656)),
     ("token_fp8 int8", 32, 64, 5, "parts", "cached", (98, 2312, 48)),
     ("block ue8m0 token_fp8 int8", 16, 16, 2, "whole", "cached", (17, 40, 128)),
@@ -323,11 +323,11 @@ QUANT_TILE_KERNELS = [
     ("block ue8m0 token_fp8 int8", 16, 16, 10, "whole", "cached", (18, 40, 1152)),
     ("block ue8m0 token_fp8 int8", 16, 32, 2, "whole", "cached", (114, 520, 128)),
     ("block ue8m0 token_fp8 int8", 16, 32, 4, "whole", "cached", (133, 456, 640)),
-    ("block ue8m0 token_fp8 int8", 16, 32, 10, "whole", "cached", (15, 5648, 1152)),
+    ("block ue8m0 token_fp8 int8", 16, 32, 10, "whole", "cached", (131, 456, 1152)),
     ("block ue8m0 token_fp8 int8", 16, 64, 2, "whole", "cached", (194, 624, 256)),
     ("block ue8m0 token_fp8 int8", 16, 64, 4, "whole", "cached", (227, 552, 640)),
-    ("block ue8m0 token_fp8 int8", 16, 64, 10, "whole", "cached", (12, 8352, 1408)),
-    ("block ue8m0 token_fp8 int8", 32, 32, 5, "whole", "cached", (17, 56, 1152)),
+    ("block ue8m0 token_fp8 int8", 16, 64, 10, "whole", "cached", (217, 616, 1152)),
+    ("block ue8m0 token_fp8 int8", 32, 32, 5, "whole", "cached", (307, 400, 128)),
     ("block ue8m0 token_fp8 int8", 32, 32, 10, "whole", "cached", (371, 664, 768)),
     ("block ue8m0 token_fp8 int8", 32, 64, 5, "whole", "cached", (194, 1256, 640)),
     ("block ue8m0", 32, 64, 10, "whole", "cached", (300, 840, 768)),
@@ -346,6 +346,27 @@ QUANT_TILE_KERNELS = [
     ("block ue8m0 token_fp8 int8", 16, 64, 10, "whole", "streamed", (2, 8592, 11648)),
     ("block ue8m0 token_fp8 int8", 16, 16, 4, "whole", "streamed", (1, 11184, 13312)),
     ("block ue8m0 token_fp8 int8", 16, 16, 10, "whole", "streamed", (1, 2504, 40576)), ("token_fp8 int8", 16, 16, 10, "parts", "streamed", (1, 3760, 27040)),
+]
+# Linears that quantize their tokens in the one launch when they are called eagerly, and the launches of a captured call: (linear, shape, launches).
+# us in a graph with one launch and with two:
+CAPTURED_LINEARS = [
+    ("ue8m0", (173, 256, 2048), 2),  # 6.7, 5.5
+    ("ue8m0", (185, 640, 1536), 2),  # 6.6, 5.65
+    ("int8", (121, 384, 1536), 2),  # 6.5, 5.6
+    ("block", (48, 768, 2048), 2),  # 6.6, 5.8
+    ("token_fp8", (168, 768, 1280), 2),  # 7.0, 6.0
+    ("block", (46, 512, 1280), 1),  # 5.1, 5.3
+    ("ue8m0", (669, 384, 640), 1),  # 4.3, 6.8
+    ("token_fp8", (69, 384, 768), 1),  # 4.2, 5.3
+    ("int8", (103, 768, 768), 1),  # 4.35, 5.6
+    ("block", (89, 2560, 1024), 1),  # 5.5, 5.7
+    # K in parts of blocks at decode sizes
+    ("int8", (13, 1152, 2784), 2),  # 7.6, 6.3
+    ("int8", (9, 640, 4384), 2),  # 7.9, 6.7
+    ("token_fp8", (15, 640, 2016), 2),  # 6.25, 5.6
+    ("int8", (3, 768, 10432), 1),  # 8.8, 9.4
+    ("token_fp8", (4, 6016, 8352), 1),  # 16.3, 17.1
+    ("int8", (14, 8320, 1504), 1),  # 7.8, 7.8
 ]
 QUANT_PIECES = {16: (2, 4, 10), 32: (5, 10)}  # by the tile's tokens
 

@@ -6,8 +6,8 @@ import time
 
 import pytest
 
-from gemm_cases import (FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, GROUPED_FORMS, GROUPED_SHAPES, INT8_CONFIG,
-                        INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, RAGGED_TILE_SHAPES,
+from gemm_cases import (CAPTURED_LINEARS, FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, GROUPED_FORMS, GROUPED_SHAPES,
+                        INT8_CONFIG, INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, RAGGED_TILE_SHAPES,
                         STREAMED_RAGGED_SHAPES, VARIANT_SHAPES, linear_variant_of, plan_for, quant_tile_kernel, variant_of)
 
 LINEARS = ("block", "ue8m0", "token_fp8", "int8")
@@ -300,33 +300,11 @@ def test_small_layers_run_the_measured_kernel(kind, shape, kernel):
     assert _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
 
 
-# Small layers of short K above 16 tokens: (linear, shape, whether the tile quantizes its tokens).  us in a graph, and what ran otherwise:
-SMALL_BATCH_CHOICES = [
-    ("ue8m0", (173, 256, 2048), "launch"),  # 5.5, 6.7
-    ("ue8m0", (185, 640, 1536), "launch"),  # 5.65, 6.6
-    ("int8", (121, 384, 1536), "launch"),  # 5.6, 6.5
-    ("block", (48, 768, 2048), "launch"),  # 5.8, 6.6
-    ("token_fp8", (168, 768, 1280), "launch"),  # 6.0, 7.0
-    ("block", (46, 512, 1280), "fused"),  # 5.1, 5.3
-    ("ue8m0", (669, 384, 640), "fused"),  # 4.3, 6.8
-    ("token_fp8", (69, 384, 768), "fused"),  # 4.2, 5.3
-    ("int8", (103, 768, 768), "fused"),  # 4.35, 5.6
-    ("block", (89, 2560, 1024), "fused"),  # 5.5, 5.7
-    # K in parts of blocks at decode sizes
-    ("int8", (13, 1152, 2784), "launch"),  # 6.3, 7.6
-    ("int8", (9, 640, 4384), "launch"),  # 6.7, 7.9
-    ("token_fp8", (15, 640, 2016), "launch"),  # 5.6, 6.25
-    ("int8", (3, 768, 10432), "fused"),  # 8.8, 9.4
-    ("token_fp8", (4, 6016, 8352), "fused"),  # 16.3, 17.1
-    ("int8", (14, 8320, 1504), "fused"),  # 7.8, 7.8
-]
-
-
-@pytest.mark.parametrize("kind,shape,quantizer", SMALL_BATCH_CHOICES)
-def test_tokens_are_quantized_where_it_measured_faster(kind, shape, quantizer):
+def test_captured_linears_quantize_their_tokens_when_eager():
     from sglang_amd import _lib
 
-    assert _lib.linear_plan(kind, *shape)["quantizer"] == quantizer, _lib.linear_plan(kind, *shape)
+    for kind, shape, kernels in CAPTURED_LINEARS:
+        assert _lib.linear_plan(kind, *shape)["quantizer"] == "fused", (kind, shape, kernels)
 
 
 def test_perturbed_plan_query():

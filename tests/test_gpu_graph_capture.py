@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from fp8_tolerance import check_fp8_gemm
+from gemm_cases import CAPTURED_LINEARS
 from sglang_amd.workloads import make_activation, make_fp8_weight, make_int8_weight
 
 pytestmark = pytest.mark.gpu
@@ -220,3 +221,64 @@ def test_linear_methods_replay(gpu, M, N, K):
         for name, g_, w_ in zip(("cutlass-style", "triton-style", "per-token fp8", "int8"), got, want):
             assert torch.equal(g_.view(torch.int16), w_.view(torch.int16)), (i, name)
             assert bool(torch.isfinite(g_).all())
+
+
+def _kernel_nodes(graph):
+    """Kernels in a captured graph: all its nodes have to be kernels."""
+    import ctypes
+
+    with open("/proc/self/maps") as maps:
+        path = next(line.split()[-1] for line in maps if "libamdhip64.so" in line)
+    hip = ctypes.CDLL(path)  # the runtime that torch has loaded
+    handle, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(handle, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(handle, nodes, ctypes.byref(n)) == 0
+    for node in nodes:
+        kind = ctypes.c_int(-1)
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0 and kind.value == 0  # hipGraphNodeTypeKernel
+    return n.value
+
+
+@pytest.mark.parametrize("kind,shape,launches", CAPTURED_LINEARS)
+def test_captured_linear_takes_what_the_gpu_does_faster(gpu, kind, shape, launches):
+    """Outside a capture these quantize their tokens in the GEMM's launch for the host's sake; inside, where it takes longer than two launches,
+    they take two.  The same bits from either, on every replay."""
+    from sglang_amd import ops
+    from sglang_amd.fp8_utils import requant_weight_ue8m0
+
+    M, N, K = shape
+    print(f"case {kind} {shape} {launches}", flush=True)
+    whole = (K + 127) // 128 * 128
+    if kind == "int8":
+        w, s = make_int8_weight(N, whole, seed=K)
+        w, s = w[:, :K].contiguous().to(gpu), s.to(gpu)
+        call = lambda x: ops.int8_linear(x, w.t(), s, None, torch.bfloat16)
+    else:
+        w, s = make_fp8_weight(N, whole, seed=K)
+        w, s = w[:, :K].contiguous().to(gpu), s.to(gpu)
+        if kind == "ue8m0":
+            w, s = requant_weight_ue8m0(w, s, [128, 128])
+        if kind == "token_fp8":
+            s = torch.rand(N, generator=torch.Generator().manual_seed(K)).to(gpu) * 0.01 + 1e-3
+        call = {"block": lambda x: ops.block_fp8_linear(x, w, s, None, torch.bfloat16), "ue8m0": lambda x: ops.block_fp8_linear_ue8m0(x, w, s, None, torch.bfloat16),
+                "token_fp8": lambda x: ops.fp8_per_token_linear(x, w.t(), s, None, torch.bfloat16)}[kind]
+    inputs = [make_activation(M, whole, seed=i)[:, :K].contiguous().to(gpu) for i in range(4)]
+    x = inputs[0].clone()
+    stream = torch.cuda.Stream()  # default priority
+    with torch.cuda.stream(stream):
+        call(x)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=stream):
+            out = call(x)
+    torch.cuda.synchronize()
+    assert _kernel_nodes(graph) == launches
+    graph.instantiate()
+    for value in inputs[1:] + inputs[:1]:
+        x.copy_(value)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), call(x).view(torch.int16))
+        torch.cuda.synchronize()
