@@ -135,14 +135,17 @@ int mi355_fp8_blockwise_mm(const void* a, const void* b, const float* sa, const 
  * Row counts and offsets are clamped into [0, total_m] on the device, so inconsistent routing data gives wrong rows, not
  * out-of-bounds accesses.  K % 128 == 0 and 16-byte aligned operand rows are required (MI355_ERR_UNSUPPORTED otherwise).
  * The tile schedule and the re-laid-out token scales live in `workspace` (256-byte aligned,
- * >= ..._workspace_bytes(num_experts, total_m, N, K)); nothing is allocated, two or three launches on `stream`.
+ * >= ..._workspace_bytes(num_experts, total_m, N, K)); nothing is allocated, one to three launches on `stream`.  Experts that
+ * share rows may take each other's scales for them where the scales are re-laid out.  Scales may have any strides.
  * Replaces fp8_blockwise_scaled_grouped_mm (sgl-kernel/csrc/moe/fp8_blockwise_moe_kernel.cu:650-810, set-up kernel
  * sgl-kernel/csrc/moe/cutlass_moe_helper.cu:17-80, Python sgl-kernel/python/sgl_kernel/moe.py:96-135; caller
  * cutlass_fused_experts_fp8, python/sglang/srt/layers/moe/cutlass_moe.py:146-201).  The reference's pointer, stride and
  * scale-layout arrays are scratch its own set-up kernel fills; here that scratch is the workspace.
- * ..._plan writes what such a call runs (host only): "kernel=grouped_pingpong+grouped_dma3|grouped_dma3
- * small_tile=<64|128>x<128|256> max_big_tiles=<n> max_small_tiles=<n> tiles_n=<channel tiles of the small kernel>": experts
- * are cut into 256-row tiles plus, for a rest of at most 128 rows, small tiles, or (grouped_dma3) into small tiles alone.
+ * ..._plan writes what such a call runs (host only): "kernel=grouped_pingpong+grouped_dma3|grouped_dma3|grouped_wavesplit
+ * small_tile=<rows>x<channels> max_big_tiles=<n> max_small_tiles=<n> tiles_n=<channel tiles of the small kernel>": experts
+ * are cut into 256-row tiles plus, for a rest of at most 128 rows, small tiles, or (grouped_dma3) into small tiles alone, of
+ * 64 or 128 rows x 128 or 256 channels, or (grouped_wavesplit, few rows on small weights) into tiles of 16 x 16, 16 x 32,
+ * 16 x 64, 32 x 32, 32 x 64 or 64 x 64 by one launch that needs no schedule.
  */
 size_t mi355_fp8_blockwise_scaled_grouped_mm_workspace_bytes(int64_t num_experts, int64_t total_m, int64_t N, int64_t K);
 int mi355_fp8_blockwise_scaled_grouped_mm_plan(int64_t num_experts, int64_t total_m, int64_t N, int64_t K, char* buf,

@@ -247,7 +247,8 @@ def gemm_plan_perturbed(kind: str, M: int, N: int, K: int, constant: int, factor
 
 def grouped_gemm_plan(num_experts: int, total_m: int, N: int, K: int) -> dict:
     """What the grouped FP8 GEMM runs for this many experts and stacked rows: {"kernel": "grouped_pingpong+grouped_dma3" |
-    "grouped_dma3", "small_tile": "<64|128>x<128|256>", "max_big_tiles": int, "max_small_tiles": int, "tiles_n": int}."""
+    "grouped_dma3" | "grouped_wavesplit", "small_tile": "<rows>x<channels>" (64 or 128 x 128 or 256; 16x16 to 64x64 for
+    "grouped_wavesplit"), "max_big_tiles": int, "max_small_tiles": int, "tiles_n": int}."""
     buf = ctypes.create_string_buffer(256)
     check(lib().mi355_fp8_blockwise_scaled_grouped_mm_plan(num_experts, total_m, N, K, buf, len(buf)))
     return _parse(buf.value)
