@@ -1347,7 +1347,7 @@ LinearRoute choose_linear(WavesplitQuant quant, int64_t M, int64_t N, int64_t K,
   return table.get(Key{{M, N, K, (int)quant}, ldw, q_ok, w_aligned}, [&] { return uncached_choose_linear(quant, M, N, K, ldw, q_ok, w_aligned); });
 }
 bool being_captured(void* stream) {
-  if (stream == nullptr) return false;  // (the null stream never is; asked about while another stream is, it would end that capture)
+  if (stream == nullptr || stream == hipStreamLegacy) return false;  // (never is; asked about while another stream is, the runtime has an error)
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
   (void)hipGetLastError();
