@@ -262,8 +262,8 @@ TileChoice best_resident(GemmKind kind, int64_t M, int64_t N, int64_t K) {
 // time in a graph (at most 1.04, but for two of 1.06 and 1.18), 0.64 eager; us in a graph, two launches / this: 18 tokens 512 -> 896 5.0 / 3.5,
 // 669 tokens packed exponents 640 -> 384 6.8 / 4.3, 69 tokens per-token FP8 768 -> 384 5.3 / 4.2, INT8 103 tokens 768 -> 768 5.6 / 4.35.
 // `eager_only`: with `many` it takes more of the GPU's time than two launches, less than the 2.4 us that a launch takes on the host; not in a
-// capture, where they are not spent.  19 such linears 1.06 (0.94 to 1.23) of the two launches' time in a graph, 0.70 eager; graph, eager: 173 tokens packed exponents
-// 2048 -> 256 5.5 / 6.7, 9.5 / 6.7; 48 tokens 2048 -> 768 5.8 / 6.6, 8.8 / 6.6; INT8 121 tokens 1536 -> 384 5.6 / 6.5, 8.9 / 6.4.
+// capture, where they are not spent.  19 such linears 1.06 (0.94 to 1.23) of the two launches' time in a graph, 0.70 eager; graph, eager:
+// 173 tokens packed exponents 2048 -> 256 5.5 / 6.7, 9.5 / 6.7; 48 tokens 2048 -> 768 5.8 / 6.6, 8.8 / 6.6; INT8 121 tokens 1536 -> 384 5.6 / 6.5, 8.9 / 6.4.
 TileChoice choose_quant_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, int plain_bm, int plain_bn, bool& eager_only) {
   const QuantTimes& q = tile_model().quant;
   double two_launches = 0.0;

@@ -249,8 +249,8 @@ LINEAR_SHAPES = [(1, 128, 128), (15, 128, 1408), (8, 34176, 1536), (2, 18432, 74
                  (2, 33472, 4096), (1, 80768, 3328), (3, 17408, 3840), (5, 17920, 3840), (13, 20864, 1536), (13, 65664, 1152), (1, 16512, 128),
                  (7, 32512, 1792), (15, 28160, 1024), (5, 19392, 4096),
                  (17, 2816, 7168)]
-# Above decode sizes, the wave-split tiles that quantize their tokens: (tokens x channels, whether a thread has more than four pieces of eight values, five with 32 tokens),
-# each with a last tile of a few tokens or channels
+# Above decode sizes, the wave-split tiles that quantize their tokens: (tokens x channels, whether a thread has more than four pieces of eight
+# values, five with 32 tokens), each with a last tile of a few tokens or channels; some of the four linears run the tile named
 QUANT_TILE_SHAPES = {((16, 16), False): (143, 24, 640), ((16, 16), True): (49, 16, 1664), ((16, 32), False): (83, 688, 640),
                      ((16, 32), True): (76, 968, 1408), ((16, 64), False): (54, 2656, 384), ((16, 64), True): (110, 1168, 1152),
                      ((32, 32), False): (21, 5200, 896), ((32, 32), True): (18, 7064, 1152), ((32, 64), False): (139, 2304, 640),

@@ -7,7 +7,7 @@ import time
 import pytest
 
 from gemm_cases import (CAPTURED_LINEARS, FP8_DECODE_CONFIG, FP8_PREFILL_CONFIG, FP8_REQUIRED_VARIANTS, FP8_ROUTE_SHAPES, GROUPED_FORMS, GROUPED_SHAPES,
-                        INT8_CONFIG, INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, RAGGED_TILE_SHAPES,
+                        INT8_CONFIG, INT8_REQUIRED_VARIANTS, INT8_ROUTE_SHAPES, LINEAR_SHAPES, MID_TILE_SWEEPS, QUANT_TILE_KERNELS, QUANT_TILE_SHAPES, RAGGED_TILE_SHAPES,
                         STREAMED_RAGGED_SHAPES, VARIANT_SHAPES, linear_variant_of, plan_for, quant_tile_kernel, variant_of)
 
 LINEARS = ("block", "ue8m0", "token_fp8", "int8")
@@ -88,6 +88,16 @@ def test_parts_of_blocks_run_the_named_tiles(kind):
     for shape, kernel in STREAMED_RAGGED_SHAPES:
         p = plan_for(kind, *shape)
         assert kernel == (p["kernel"], p["bm"], p["bn"]) and p["splits"] == 1 and shape[0] <= p["bm"] and shape[1] * shape[2] >= 1e8, (shape, p)
+
+
+@pytest.mark.parametrize("tile,many", QUANT_TILE_SHAPES)
+def test_quantizing_tiles_above_decode_sizes(tile, many):
+    from sglang_amd import _lib
+
+    M, N, K = QUANT_TILE_SHAPES[tile, many]
+    plans = [_lib.linear_plan(kind, M, N, K) for kind in LINEARS]
+    assert any((p["quantizer"], p["bm"], p["bn"]) == ("fused", *tile) for p in plans), plans
+    assert (min(M, tile[0]) * K > (16384 if tile[0] == 16 else 20480)) == many
 
 
 def test_quantizing_tiles_are_named_and_listed():
