@@ -843,7 +843,7 @@ std::vector<std::string> tile_constant_names() {
                   "ragged_max_factor", "ragged_min_kblocks", "ragged_two_phase_kblocks", "ragged_min_workgroups", "wavesplit_max_tokens_bytes", "wavesplit_long_k", "wavesplit_long_k_max_tokens_bytes",
                   "few_workgroups_max_tokens", "decode_min_kblocks", "decode_padded_max_weight", "decode_max_weight", "decode_few_tokens_max_weight",
                   "decode_one_turn_min_kblocks", "decode_one_turn_kblocks", "decode_one_turn_max_channels", "decode_one_turn_max_tokens", "decode_few_tokens_f32", "decode_few_tokens", "decode_long_kblocks", "decode_short_min_kblocks", "decode_short_min_channels",
-                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_far_margin", "resident_min_channels", "resident_min_tokens", "resident_rounds_margin", "streamed_min_weight", "streamed_two_tokens_min_kblocks", "small_min_tokens", "small_max_channels", "small_max_tokens_values", "half_decode_min_kblocks", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
+                  "decode_short_max_weight", "decode_short_min_tokens", "resident_margin", "resident_rounds_margin", "streamed_min_weight", "streamed_two_tokens_min_kblocks", "small_min_tokens", "small_max_channels", "small_max_tokens_values", "half_decode_min_kblocks", "cold_min_weight", "cold_only_min_weight", "cold_margin", "cold_full_max_tokens", "cold_full_workgroups"});
   add("streamed.", {"tile", "channel", "token", "stream", "stream_us", "norm", "launch", "block", "block_channel", "block_token", "shared", "mid_stream", "mid_stream_us"});
   add("quant.", {"launch", "tile", "piece[block]", "piece[ue8m0]", "piece[token_fp8]", "piece[int8]", "many", "kb", "kb_busy", "result", "saved"});
   names.resize(TILE_CONSTANT_COUNT);

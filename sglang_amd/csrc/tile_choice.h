@@ -57,7 +57,7 @@ constexpr TileTimes SCALED_TIMES = {  // FP8 with scales in the K loop
     {0.219, 0.277, 0.317, 0.385, 0.419, 0.533, 0.288, 0.363, 0.441, 0.532, 0.334, 0.445, 0.535},
     7.88, 0.567, 1.70, 12.5,
     2.74, 1.041, 0.00591, 0.00334, 5.49, -3.81, 0.253, 1.511,
-    3, 0.0909, 0.335, 0.492, 0.154, 0.733,
+    3.63, 0.11, 0.406, 0.596, 0.186, 0.733,
     0.101, 0.0019, 0.0020, 1.42, 4.88, -0.45, 0.202, 3.27, 0.320,
     0.01269, 0.01362, 1.434, -1.44, 1.283,
     6.52, 1.774, 0.55, 1.08};
@@ -67,7 +67,7 @@ constexpr TileTimes PLAIN_TIMES = {  // FP8 with epilogue scales, INT8
     {0.165, 0.205, 0.240, 0.295, 0.333, 0.432, 0.224, 0.271, 0.339, 0.420, 0.278, 0.347, 0.431},
     8.48, 0.511, 1.70, 10.8,
     2.71, 1.017, 0.00609, 0.00343, 5.07, -4.41, 0.282, 1.673,
-    3.01, 0.00826, 0.359, 0.628, 0.179, 0.531,
+    3.64, 0.01, 0.435, 0.760, 0.217, 0.531,
     0.092, 0.0020, 0.0018, 1.37, 5.02, 1.55, 0.230, 3.16, 0.331,
     0.01247, 0.01387, 1.394, -1.13, 1.215,
     6.35, 1.730, 0.681, 1.03};
@@ -83,7 +83,7 @@ struct TileLimits {
   double decode_one_turn_min_kblocks = 30.0, decode_one_turn_kblocks = 32.0, decode_one_turn_max_channels = 16384.0, decode_one_turn_max_tokens = 10.0;
   double decode_few_tokens_f32 = 6.0, decode_few_tokens = 8.0, decode_long_kblocks = 64.0;
   double decode_short_min_kblocks = 8.0, decode_short_min_channels = 7168.0, decode_short_max_weight = 20e6, decode_short_min_tokens = 8.0;
-  double resident_margin = 0.87, resident_far_margin = 0.76, resident_min_channels = 8 * RESIDENT_CHANNELS, resident_min_tokens = 64.0, resident_rounds_margin = 0.95;
+  double resident_margin = 0.93, resident_rounds_margin = 0.95;
   double streamed_min_weight = 100e6, streamed_two_tokens_min_kblocks = 33.0;
   double small_min_tokens = 4.0, small_max_channels = 64.0 * NUM_CUS, small_max_tokens_values = 20800.0;
   double half_decode_min_kblocks = 18.0;
@@ -384,23 +384,16 @@ TileChoice choose_cold_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, cons
   return best.family != TF_NONE ? best : swept;
 }
 
-// The same, or the kernel that keeps the weight in registers where the call allows it and it models 13 % faster than what would run; 23 %
-// for up to 2048 channels, where an XCD reads all tokens for its few channels, for up to 64 tokens, one step, and against the two-phase kernels, on
-// which results beyond 128 MB cost no more than here.  Linears by modelled time of this over the other: 0.77 to 0.87 0.65 to 0.99 of the time, 0.87 to
-// 0.91 0.80 to 0.98, 0.95 to 1.0 0.90 to 1.07.  Us, other / this: block FP8 206 tokens 384 -> 24576 10.7 / 10.0, 458 tokens 512 -> 16384 12.8 / 10.6,
-// 1544 tokens 512 -> 4096 12.9 / 11.4; per-token FP8 553 tokens 512 -> 16384 15.6 / 11.7, 900 tokens 640 -> 13952 19.3 / 17.1; not taken: block FP8 301
-// tokens 384 -> 24576 12.4 / 12.2, 784 tokens 512 -> 5184 10.9 / 11.2, 61 tokens 512 -> 32768 9.5 / 9.7, 40 tokens 768 -> 34944 10.5 / 11.3, 1846 tokens
-// 768 -> 1216 10.8 / 11.6, INT8 4088 tokens 768 -> 1856 16.9 / 18.6, 1100 tokens 768 -> 65584 98.1 / 100.2.
+// The same, or the kernel that keeps the weight in registers where the call allows it and it models 7 % faster than what would run.
+// The linears on both sides of the line, us, other / this: block FP8 368 tokens 512 -> 32768 17.4 / 15.5, 430 tokens 512 -> 24576
+// 16.5 / 15.6, 243 tokens 512 -> 6144 8.3 / 8.4, 1340 tokens 512 -> 4096 11.3 / 12.2; 849 tokens 512 -> 6144 10.6 / 11.5;
+// per-token FP8 180 tokens 512 -> 24576 10.2 / 12.0, 624 tokens 640 -> 16384 17.2 / 15.7.
 TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool resident_allowed) {
   double base_us;
   const TileChoice c = choose_cold_tile(kind, M, N, K, base, choose_swept_tile(kind, M, N, K, base, base_us));
   if (!resident_allowed) return c;
   const TileChoice r = best_resident(kind, M, N, K);
-  const TileLimits& l = tile_model().limits;
-  const TileChoice& other = c.family != TF_NONE ? c : base;
-  const bool two_phase = other.family == TF_TWO_PHASE || (kind == GK_INT8 && other.bm == 128 && other.bn == 256);
-  const bool near = N > l.resident_min_channels && M > l.resident_min_tokens && !two_phase;
-  return r.us < (near ? l.resident_margin : l.resident_far_margin) * (c.family != TF_NONE ? c.us : base_us) ? r : c;
+  return r.us < tile_model().limits.resident_margin * (c.family != TF_NONE ? c.us : base_us) ? r : c;
 }
 
 // Up to 16 tokens on a weight large enough to be loaded as a stream (streams_weight): the wave-split and the mid-M tile have such loads, the
