@@ -384,10 +384,14 @@ TileChoice choose_cold_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, cons
   return best.family != TF_NONE ? best : swept;
 }
 
-// The same, or the kernel that keeps the weight in registers where the call allows it and it models 7 % faster than what would run.
-// The linears on both sides of the line, us, other / this: block FP8 368 tokens 512 -> 32768 17.4 / 15.5, 430 tokens 512 -> 24576
-// 16.5 / 15.6, 243 tokens 512 -> 6144 8.3 / 8.4, 1340 tokens 512 -> 4096 11.3 / 12.2; 849 tokens 512 -> 6144 10.6 / 11.5;
-// per-token FP8 180 tokens 512 -> 24576 10.2 / 12.0, 624 tokens 640 -> 16384 17.2 / 15.7.
+// The same, or the kernel that keeps the weight in registers where the call allows it and it models 7 % faster than what would run.  Its modelled
+// times are of the loop it had before its outputs became kernels of their own, and longer than it takes now: a call that is not taken may have gained by it,
+// one that is taken rarely loses (114 random linears of K = 768 that take it 0.85 of the time in a graph, seven slower, by up to 7 %).
+// Linears on both sides of the line, us in a graph, other / this, taken: block FP8 368 tokens 512 -> 32768 19.5 / 16.6; packed exponents 1493 tokens
+// 768 -> 7296 21.2 / 17.4; per-token FP8 827 tokens 768 -> 24576 38.0 / 28.9; INT8 577 tokens 768 -> 20496 25.0 / 22.7, 975 tokens 768 -> 65584 120 / 102,
+// 1100 tokens 108 / 102.  Not taken: block FP8 430 tokens 512 -> 24576 18.0 / 14.9, 458 tokens 512 -> 16384 13.3 / 11.6, 1544 tokens 512 -> 4096 13.5 / 11.8,
+// 849 tokens 512 -> 6144 11.1 / 11.0, 784 tokens 512 -> 5184 10.7 / 10.9, 40 tokens 768 -> 34944 10.6 / 11.3; per-token FP8 624 tokens 640 -> 16384
+// 18.3 / 14.6, 180 tokens 512 -> 24576 10.4 / 11.2; INT8 4088 tokens 768 -> 1856 17.1 / 18.7.
 TileChoice choose_mid_tile(GemmKind kind, int64_t M, int64_t N, int64_t K, const TileChoice& base, bool resident_allowed) {
   double base_us;
   const TileChoice c = choose_cold_tile(kind, M, N, K, base, choose_swept_tile(kind, M, N, K, base, base_us));

@@ -310,6 +310,22 @@ def test_small_layers_run_the_measured_kernel(kind, shape, kernel):
     assert _lib.linear_plan(kind, *shape)["kernel"] == kernel, _lib.linear_plan(kind, *shape)
 
 
+# (tokens, channels, K) on both sides of the line from which the weight-in-registers kernel is taken; the times stand at choose_mid_tile
+RESIDENT_CHOICES = [
+    ("block", (368, 32768, 512), True), ("ue8m0", (1493, 7296, 768), True), ("token_fp8", (827, 24576, 768), True), ("int8", (577, 20496, 768), True),
+    ("int8", (975, 65584, 768), True), ("int8", (1100, 65584, 768), True), ("block", (430, 24576, 512), False), ("block", (458, 16384, 512), False),
+    ("block", (1544, 4096, 512), False), ("block", (849, 6144, 512), False), ("block", (784, 5184, 512), False), ("block", (40, 34944, 768), False),
+    ("token_fp8", (624, 16384, 640), False), ("token_fp8", (180, 24576, 512), False), ("int8", (4088, 1856, 768), False),
+]
+
+
+@pytest.mark.parametrize("kind,shape,taken", RESIDENT_CHOICES)
+def test_resident_kernel_is_taken_where_the_rule_says(kind, shape, taken):
+    from sglang_amd import _lib
+
+    assert (_lib.linear_plan(kind, *shape)["kernel"] == "resident") == taken, _lib.linear_plan(kind, *shape)
+
+
 def test_captured_linears_quantize_their_tokens_when_eager():
     from sglang_amd import _lib
 

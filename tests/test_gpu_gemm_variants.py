@@ -5,7 +5,7 @@ multiplied twice or skipped, a wrong scale or a wrong row shows as a wrong numbe
 import pytest
 import torch
 
-from gemm_cases import MID_TILE_SWEEPS, TAKEN_OVER_SHAPES, VARIANT_SHAPES, plan_for
+from gemm_cases import MID_TILE_SWEEPS, TAKEN_OVER_SHAPES, VARIANT_SHAPES, plan_for, variant_of
 
 pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
@@ -74,6 +74,7 @@ def test_taken_over_exact(gpu, kind, M, N, K):
 def test_variant_exact(gpu, kind, variant):
     M, N, K = VARIANT_SHAPES[kind][variant]
     print(f"case {kind} {(M, N, K)} {variant}", flush=True)
+    assert variant_of(plan_for(kind, M, N, K), K) == variant
     check_exact(gpu, kind, M, N, K)
 
 
@@ -194,9 +195,11 @@ def test_results_written_through(gpu, kind, N, K, more):
     check_exact(gpu, kind, 64000000 // N + more, N, K)
 
 
-# the same out of the mid-M and the 128-token kernel, and with the kernel named where packed exponents go straight to the two-phase one
+# the same out of the mid-M, the 128-token and (K = 768) the weight-in-registers kernel, and with the kernel named where packed exponents go
+# straight to the two-phase one
 @pytest.mark.parametrize("kind,N,K,kernel", [("fp8", 13592, 128, "dma3"), ("fp8_ue8m0", 13592, 128, "dma3"), ("fp8_scaled", 65584, 128, "dma3"),
-                                             ("int8", 65584, 768, "pingpong128"), ("fp8_ue8m0", 24584, 1024, "pingpong")])
+                                             ("int8", 65584, 768, "resident"),
+                                             ("int8", 65584, 896, "pingpong128"), ("fp8_ue8m0", 24584, 1024, "pingpong")])
 @pytest.mark.parametrize("more", [0, 1])
 def test_results_written_through_by_kernel(gpu, kind, N, K, kernel, more):
     M = 64000000 // N + more
