@@ -78,17 +78,20 @@ __device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f) {
   return (t + n) >> f.shift;  // n < 2^31, so t + n cannot overflow
 }
 
-// Separately rounded fp32 multiply and add, written as instructions: the INT8 epilogue contract is mul, mul, add, and no
-// compiler setting or code motion may fuse two of them into an FMA (a fused result differs in the last bit of the 16-bit
-// output about once in 10^5 elements).
+// Separately rounded fp32 multiply and add: the INT8 epilogue contract is mul, mul, add, and no code motion may fuse two of them into an FMA (a fused
+// result differs in the last bit of the 16-bit output about once in 10^5 elements), nor one of them into a conversion (v_fma_mixlo_f16 rounds a product to
+// fp16 once).  So the result passes through an empty asm, and the pragma takes the leave to fuse off the operation itself, which -ffp-contract=fast would
+// pass over.  The operation is not asm: the compiler does not see what asm reads, and would not wait for an MFMA's result in front of it.
 __device__ __forceinline__ float mul_rn(float a, float b) {
-  float r;
-  asm("v_mul_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+#pragma clang fp contract(off)
+  float r = a * b;
+  asm("" : "+v"(r));
   return r;
 }
 __device__ __forceinline__ float add_rn(float a, float b) {
-  float r;
-  asm("v_add_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+#pragma clang fp contract(off)
+  float r = a + b;
+  asm("" : "+v"(r));
   return r;
 }
 

@@ -220,3 +220,18 @@ def test_bench_refuses_more_than_one_gpu():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert r.returncode != 0 and "ONE GPU" in (r.stdout + r.stderr)
+
+
+def test_asm_computes_nothing():
+    """Inline asm loads, stores, waits and moves scalars: the compiler does not see what asm reads, and would not wait for an MFMA's result in front of an
+    instruction that computes with it.  (The one exception reads a maximum of vector instructions, behind an s_nop of its own.)"""
+    from sglang_amd import _lib
+
+    csrc = os.path.dirname(_lib.LIB_PATH)
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".h", ".hip", ".cpp")):
+            with open(os.path.join(csrc, name)) as f:
+                text = re.sub(r"//[^\n]*", "", f.read())
+            for statement in re.findall(r"\basm\b(?:\s+volatile)?\s*\(((?:\s*\"[^\"]*\"|\s*[A-Z]+\b)+)", text):
+                instructions = re.findall(r"\bv_\w+", statement)
+                assert not instructions or (instructions == ["v_max_f32_dpp"] and "s_nop 1" in statement), (name, statement)
