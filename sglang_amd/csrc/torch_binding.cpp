@@ -14,6 +14,7 @@
 //     the Python function then goes its long way, which calls the operators and raises the errors.
 #include <Python.h>
 
+#include <ATen/Context.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
@@ -99,10 +100,13 @@ Tensor new_tensor(at::IntArrayRef sizes, ScalarType dtype, const Tensor& like) {
   return at::empty(sizes, like.options().dtype(dtype).layout(at::kStrided).requires_grad(false).memory_format(std::nullopt));
 }
 
-// The same for a fast path, which nobody listens to: the device's own function that at::empty ends in, without the dispatcher in front of it, half of the
-// 0.7 us that a tensor takes (one launch is about 3).  A profiler that records operators gets to see at::empty.
+// The same for a fast path, which nobody listens to: the device's own allocation that at::empty's kernel makes, without the dispatcher in front of it, half
+// of the 0.7 us that a tensor takes (one launch is about 3).  That kernel then fills the memory where deterministic algorithms are asked for (what no
+// kernel writes, the pitch of aligned scales, would differ from run to run), and a profiler that records operators gets to see at::empty: both go there.
 Tensor new_plain_tensor(at::IntArrayRef sizes, ScalarType dtype, const Tensor& like) {
-  if (at::getStepCallbacksUnlessEmpty(at::RecordScope::FUNCTION).has_value()) return new_tensor(sizes, dtype, like);
+  const at::Context& context = at::globalContext();
+  if (at::getStepCallbacksUnlessEmpty(at::RecordScope::FUNCTION).has_value() || (context.deterministicAlgorithms() && context.deterministicFillUninitializedMemory()))
+    return new_tensor(sizes, dtype, like);
   return Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }
 

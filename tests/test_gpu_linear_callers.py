@@ -287,3 +287,20 @@ def test_outputs_of_the_fast_paths_are_those_of_empty(gpu):
     assert sum(e.count for e in prof.key_averages() if e.key == "aten::empty") >= 3
     assert all(torch.equal(a.view(torch.uint8) if a.dtype.itemsize == 1 else a, b.view(torch.uint8) if b.dtype.itemsize == 1 else b) for a, b in zip(plain, profiled))
 
+
+def test_deterministic_algorithms_fill_what_no_kernel_writes(gpu):
+    """torch.use_deterministic_algorithms has new memory filled, on the fast paths too: three rows of scales with a pitch of four."""
+    from sglang_amd.fp8_kernel import sglang_per_token_group_quant_fp8
+    from sglang_amd.workloads import make_activation
+
+    x = make_activation(3, 256).to(gpu)
+    rest = lambda s: torch.empty(0, dtype=s.dtype, device=gpu).set_(s.untyped_storage()).view(-1, 4)[:, 3]
+    quant = lambda ue8m0: sglang_per_token_group_quant_fp8(x, 128, column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=ue8m0)
+    plain = quant(False)
+    torch.use_deterministic_algorithms(True)
+    try:
+        filled, words = quant(False), quant(True)[1]
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert rest(filled[1]).isnan().all() and (rest(words) == torch.iinfo(torch.int32).max).all()
+    assert torch.equal(filled[0].view(torch.uint8), plain[0].view(torch.uint8)) and torch.equal(filled[1], plain[1])
