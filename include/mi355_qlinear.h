@@ -264,7 +264,9 @@ int mi355_int8_scaled_mm(const void* a, const void* b, const float* sa, const fl
  *   buf      receives a NUL-terminated "key=value ..." line:
  *            kernel=decode|decode_wavesplit|wavesplit_tile|dma3|resident|pingpong|pingpong128|pipelined|generic bm= bn= splits=
  *            kb_per_split= groups_per_wg= aligned= stages=   (stages: LDS stages of the mid-M kernel's pipeline, 0 for the
- *            other kernels) and for UE8M0 exponents=mfma|unpacked (unpacked: a launch in front expands them to fp32 scales)
+ *            other kernels) and for UE8M0 exponents=mfma|unpacked (unpacked: a launch in front expands them to fp32 scales).
+ *            resident: bm is the tokens of a step without a bias; with one, K = 512 with epilogue scales (FP8, INT8) runs
+ *            steps of 32 tokens where bm is 64, in the same groups_per_wg ranges of tokens.
  * Launches nothing and touches no device state.
  */
 int mi355_fp8_blockwise_mm_plan(int64_t M, int64_t N, int64_t K, int aligned, char* buf, size_t buf_len);
