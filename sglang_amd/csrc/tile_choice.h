@@ -86,7 +86,7 @@ struct TileLimits {
   double resident_margin = 0.93, resident_rounds_margin = 0.95;
   double streamed_min_weight = 100e6, streamed_two_tokens_min_kblocks = 33.0;
   double small_min_tokens = 4.0, small_max_channels = 64.0 * NUM_CUS, small_max_tokens_values = 20800.0;
-  double half_decode_min_kblocks = 18.0;
+  double half_decode_min_kblocks = 24.0;
   double cold_min_weight = 40e6, cold_only_min_weight = 80e6, cold_margin = 0.92, cold_full_max_tokens = 128.0, cold_full_workgroups = 0.875 * NUM_CUS;
 };
 struct TileModel {
@@ -497,10 +497,11 @@ bool small_decode(int64_t M, int64_t N, int64_t K, bool from_wavesplit, bool fro
 // Up to 16 tokens, eight channels a workgroup instead of sixteen where twice the workgroups still make one round: each loads half the weight rows through
 // a CU that takes 100 KB a microsecond.  us in a graph, 16 / 8: block FP8 7168 -> 576 at 1 token 4.59 / 4.50, 7168 -> 896 at 2 5.49 / 5.20; per-token FP8 7680 -> 1792 at 2
 // 6.25 / 5.98; INT8 7168 -> 576 at 12 7.62 / 7.34; packed exponents 7168 -> 192 at 1 4.60 / 4.35; 45 linears 0.974, at most 1.01 (nine tokens and more, which the
-// quantizer in the tile bounds).  Up to 18 blocks a wave loads three at most: 2304 -> 64 to 256 at 1, 8 and 16 tokens 0.98, 2048 -> 512 1.00, 7168 0.955.
+// quantizer in the tile bounds).  From 24 blocks of K on, three for each wave: 96 linears of 64 to 2048 channels, graph, by blocks 4 to 16 1.006 (1.00 to 1.01),
+// 17 to 22 0.996 (0.98 to 1.00), 24 0.990, 25 0.986, 28 0.985.
 TileChoice half_decode_tile(int64_t M, int64_t N, int64_t K, TileChoice c) {
   const TileLimits& l = tile_model().limits;
-  if (c.family == TF_WAVESPLIT && c.bm == 16 && c.bn == 16 && M <= 16 && ceil_div(N, 8) <= NUM_CUS && (double)ceil_div(K, KSTEP) > l.half_decode_min_kblocks &&
+  if (c.family == TF_WAVESPLIT && c.bm == 16 && c.bn == 16 && M <= 16 && ceil_div(N, 8) <= NUM_CUS && (double)ceil_div(K, KSTEP) >= l.half_decode_min_kblocks &&
       (double)(N * K) < l.streamed_min_weight)
     c.bn = 8;
   return c;

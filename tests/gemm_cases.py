@@ -248,7 +248,7 @@ LINEAR_SHAPES = [(1, 128, 128), (15, 128, 1408), (8, 34176, 1536), (2, 18432, 74
                  (1, 8, 128), (1, 8, 1024), (1, 66304, 128), (5, 27904, 8192), (3, 78208, 256), (1, 131328, 128), (11, 16, 1920), (2, 23872, 3840),
                  (2, 33472, 4096), (1, 80768, 3328), (3, 17408, 3840), (5, 17920, 3840), (13, 20864, 1536), (13, 65664, 1152), (1, 16512, 128),
                  (7, 32512, 1792), (15, 28160, 1024), (5, 19392, 4096),
-                 (17, 2816, 7168), (15, 2104, 2816), (3, 256, 6400)]
+                 (17, 2816, 7168), (15, 2104, 2816), (3, 256, 6400), (12, 136, 15872)]
 # Above decode sizes, the wave-split tiles that quantize their tokens: (tokens x channels, whether a thread has more than four pieces of eight
 # values, five with 32 tokens), each with a last tile of a few tokens or channels; some of the four linears run the tile named
 QUANT_TILE_SHAPES = {((16, 16), False): (143, 24, 640), ((16, 16), True): (49, 16, 1664), ((16, 32), False): (83, 688, 640),
@@ -318,8 +318,8 @@ QUANT_TILE_KERNELS = [
     ("token_fp8 int8", 32, 32, 5, "parts", "cached", (66, 1688, 48)),
     ("token_fp8 int8", 32, 32, 10, "parts", "cached", (401, 600, 656)),
     ("token_fp8 int8", 32, 64, 5, "parts", "cached", (98, 2312, 48)),
-    ("block ue8m0 token_fp8 int8", 16, 8, 2, "whole", "cached", (2, 40, 2432)),
-    ("block ue8m0 token_fp8 int8", 16, 8, 4, "whole", "cached", (3, 2040, 2816)),
+    ("block ue8m0 token_fp8 int8", 16, 8, 2, "whole", "cached", (2, 40, 3072)),
+    ("block ue8m0 token_fp8 int8", 16, 8, 4, "whole", "cached", (3, 2040, 3200)),
     ("block ue8m0 token_fp8 int8", 16, 8, 10, "whole", "cached", (5, 200, 3328)),
     ("block ue8m0 token_fp8 int8", 16, 16, 2, "whole", "cached", (17, 40, 128)),
     ("block ue8m0 token_fp8 int8", 16, 16, 4, "whole", "cached", (17, 40, 640)),

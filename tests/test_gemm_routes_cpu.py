@@ -338,7 +338,7 @@ def test_every_route_constant_has_its_name():
     from sglang_amd import _lib
 
     constants = _lib.route_constants()
-    assert all(constants) and constants["limits.half_decode_min_kblocks"] == 18.0
+    assert all(constants) and constants["limits.half_decode_min_kblocks"] == 24.0
     assert constants["limits.cold_margin"] == 0.92 and constants["streamed.tile"] == 1.55 and constants["quant.saved"] == 1.4
 
 
