@@ -17,12 +17,12 @@
 // What bounds it: the products and their promotion, about as many cycles of the vector unit as of the matrix pipe, then the stores; results beyond
 // 128 MB, which are not written through, the stores (512 -> 32768 at 3001 tokens takes 62 us with the results of three calls in turn and 53 with
 // one call's, which the Infinity Cache holds).  A result costs a conversion and a sixteenth of a store: the loop is a kernel of its own for each output
-// type, with and without a bias, the stores are buffer stores whose range check drops what does not exist, and their addresses advance in scalar registers.  With
-// all these choices and checks in the loop every half step ran through a dozen branches and 50 vector instructions beside the promotion's 64, and the
-// compiler moved products across the branches; us of the GPU, before / now, 3001 tokens 512 -> 32768 in a loop on one set of buffers: FP8 56.5 / 53, packed
-// exponents 51 / 46, epilogue scales 58 / 50, INT8 63 / 51; 36 random linears 0.91.  (With results that go to memory that call did not gain: 71 to 72 us.)
-// Of 80 random linears, a branch in the loop for the bias 1.03 of the time of two kernels (packed exponents of K = 640 and 768 1.9 to 3.7, spilled; the others
-// 1.00), for writing through 0.998: that one is a branch.
+// type, with and without a bias, written through or not, the stores are buffer stores whose range check drops what does not exist, and their
+// addresses advance in scalar registers.  With these choices and checks in the loop every half step ran through a dozen branches and 50 vector
+// instructions beside the promotion's 64, and the compiler moved products across the branches; us of the GPU, before / now, 3001 tokens 512 -> 32768 in a loop on
+// one set of buffers: FP8 56.5 / 53, packed exponents 51 / 46, epilogue scales 58 / 50, INT8 63 / 51; 36 random linears 0.91.  One choice alone as a branch in the
+// loop: the bias 1.03 of the time of 80 random linears (packed exponents of K = 640 and 768 1.9 to 3.7, spilled); writing through 1.00, packed exponents
+// 1.015 (20 linears of 17 to 120 MB) and 1.02 (20 of more than 128 MB), whose products are sunk behind it.
 // Whole linears, us, two-phase tile / this:
 //   block FP8 3001 tokens 512 -> 32768 89.9 / 73.9, 2310 tokens 256 -> 32768 56.2 / 36.3, 1966 tokens 640 -> 16384 43.1 / 31.2;
 //   packed exponents 1609 tokens 512 -> 32768 63.6 / 36.6;  per token FP8 820 tokens 512 -> 32768 37.8 / 24.3;  INT8 952 tokens 640 -> 32768 38.6 / 29.1;
@@ -49,7 +49,7 @@ constexpr int RS_THREADS = 64 * (RS_COMPUTE + RS_LOAD);
 template <Arith AR, int KB, bool BIAS>
 constexpr int rs_half_step() { return BIAS && KB == 4 && (AR == AR_UNIT || AR == AR_INT8) ? 16 : resident_half_step(AR == AR_UE8M0, KB); }
 
-template <Arith AR, int KB, bool BF16, bool BIAS>
+template <Arith AR, int KB, bool BF16, bool BIAS, bool THROUGH>
 __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void resident_kernel(const GemmParams p, const int ranges, const int steps_per_range) {
   constexpr bool SCALED = AR == AR_F32 || AR == AR_UE8M0;
   constexpr int HALF = rs_half_step<AR, KB, BIAS>(), TS = 2 * HALF, TT = HALF / 16, CT = RS_CT;  // tokens of a half step, of a step
@@ -275,8 +275,7 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
       word[2 * c + 1] = BF16 ? pack_bf16x2(r[2], r[3]) : pack_f16x2(r[2], r[3]);
     }
     const u32x4 v = {word[0], word[1], word[2], word[3]};
-    if (p.write_through) __builtin_amdgcn_raw_buffer_store_b128(v, to, at[t], 0, 16);  // (sc1)
-    else __builtin_amdgcn_raw_buffer_store_b128(v, to, at[t], 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, to, at[t], 0, THROUGH ? 16 : 0);  // (16: sc1)
   };
   int st = 0;
   for (int i = 0; i < steps; ++i) {
@@ -339,12 +338,14 @@ int launch_resident_inst(const GemmParams& p, int ranges, hipStream_t stream, co
   const int per_step = 2 * (p.bias != nullptr ? rs_half_step<AR, KB, true>() : rs_half_step<AR, KB, false>()), all = (p.M + per_step - 1) / per_step, steps = (all + ranges - 1) / ranges;
   ranges = (all + steps - 1) / steps;  // none without tokens
   const int slices = (p.N + RS_BN - 1) / RS_BN;
-  const auto launch = [&](auto bf16, auto bias) {
-    launch_kernel((resident_kernel<AR, KB, decltype(bf16)::value, decltype(bias)::value>), dim3((unsigned)(slices * ranges)), dim3(RS_THREADS), 0, stream, p, ranges, steps);
+  const auto launch = [&](auto bf16, auto bias, auto through) {
+    launch_kernel((resident_kernel<AR, KB, decltype(bf16)::value, decltype(bias)::value, decltype(through)::value>), dim3((unsigned)(slices * ranges)),
+                  dim3(RS_THREADS), 0, stream, p, ranges, steps);
   };
   const std::true_type yes;
   const std::false_type no;
-  const auto launch_bias = [&](auto bf16) { p.bias != nullptr ? launch(bf16, yes) : launch(bf16, no); };
+  const auto launch_through = [&](auto bf16, auto bias) { p.write_through ? launch(bf16, bias, yes) : launch(bf16, bias, no); };
+  const auto launch_bias = [&](auto bf16) { p.bias != nullptr ? launch_through(bf16, yes) : launch_through(bf16, no); };
   p.out_dtype == MI355_BF16 ? launch_bias(yes) : launch_bias(no);
   return check_launch(what);
 }
