@@ -211,6 +211,11 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
   float ts[2][TT], sc[2][TT] = {};
   v4f part[4] = {};
   constexpr int LAST = KB * TT * CT;  // products of a half step
+  // Behind which product the half step before this one starts to leave: soon, or, where it has 32 tokens and its results are not written through, behind the
+  // last ones.  80 linears, graph, late / soon: results beyond 128 MB of K = 256 and 384 0.98, packed exponents 0.92, of K = 512 0.95 (3001 tokens -> 32768 block FP8
+  // 79 / 72 us, INT8 74 / 69); of half steps of 16 tokens 1.00; results that are written through 1.02.  Left soon, packed exponents of K = 256 and 384 took up to
+  // 1.10 of the time of the loop with all choices in it, whose stores its branches held up.
+  constexpr int EMIT = !THROUGH && TT == 2 ? LAST - TT : 2;
   static_assert(LAST % 2 == 0, "the ring of products continues from step to step");
   auto ring = [](int h, int s) { return (h * LAST + s) & 3; };
 
@@ -248,16 +253,16 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
   MI355_RS_BARRIER();  // steps 0 and 1 have landed
   read(0, 0, 0, 0);
 
-  // eight channels of token tile t of half step h converted and stored
-  const auto emit = [&](int h, int t, __amdgpu_buffer_rsrc_t to) __attribute__((always_inline)) {
+  // eight channels of token tile t of half step h, whose tokens have the scale `row`, converted and stored
+  const auto emit = [&](int h, int t, float row, __amdgpu_buffer_rsrc_t to) __attribute__((always_inline)) {
     uint32_t word[2 * CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       float r[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {  // separately rounded steps, as in out_tile_put
-        if constexpr (AR == AR_INT8) r[v] = mul_rn((float)acc[h][c][t][v], mul_rn(cs[c][v], row_ts[h][t]));
-        else if constexpr (AR == AR_UNIT) r[v] = mul_rn(row_ts[h][t], mul_rn(cs[c][v], acc[h][c][t][v]));
+        if constexpr (AR == AR_INT8) r[v] = mul_rn((float)acc[h][c][t][v], mul_rn(cs[c][v], row));
+        else if constexpr (AR == AR_UNIT) r[v] = mul_rn(row, mul_rn(cs[c][v], acc[h][c][t][v]));
         else r[v] = acc[h][c][t][v];
       }
       if constexpr (BIAS) {
@@ -284,6 +289,9 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const auto to = rows_of(h == 1 ? m0 : m0 - HALF, h == 1 || i > 0);  // (none before the first half step)
+      float row_before[TT];  // (the last block's read brings the scales of the half step after this one)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) row_before[t] = row_ts[h ^ 1][t];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
         const int set = (h * KB + kb) & 1;  // fragment sets alternate
@@ -314,7 +322,7 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
               acc[h][c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(as_v4i(w[kb][c].hi), as_v4i(tok[set][t].hi), acc[h][c][t], 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (s >= 2 && s < 2 + TT) emit(h ^ 1, s - 2, to);
+            if (s >= EMIT && s < EMIT + TT) emit(h ^ 1, s - EMIT, row_before[s - EMIT], to);
             __builtin_amdgcn_sched_barrier(0);
           }
       }
@@ -329,7 +337,7 @@ __global__ __launch_bounds__(RS_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
   if constexpr (AR == AR_F32) promote(1, LAST - 2), promote(1, LAST - 1);
   const auto last = rows_of(m_begin + steps * TS - HALF, true);
 #pragma unroll
-  for (int t = 0; t < TT; ++t) emit(1, t, last);
+  for (int t = 0; t < TT; ++t) emit(1, t, row_ts[1][t], last);
 #undef MI355_RS_BARRIER
 }
 

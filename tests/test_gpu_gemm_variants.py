@@ -277,7 +277,7 @@ def test_resident_bias_and_rows(gpu, dtype):
 
 
 @pytest.mark.parametrize("kind", ["block", "ue8m0", "token_fp8", "int8"])
-@pytest.mark.parametrize("kb", [2, 4, 5, 6])
+@pytest.mark.parametrize("kb", [2, 3, 4, 5, 6])
 def test_resident_kinds_of_output(gpu, kind, kb):
     """A kernel for each output type, with and without a bias, written through or not (beyond 128 MB): channels that end inside a slice and tokens
     inside a half step, against the first and last rows by a smaller call, on another kernel with the same order of sums."""
