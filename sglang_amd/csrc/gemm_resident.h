@@ -14,9 +14,8 @@
 // A lane's results are eight consecutive channels of a token, because the weight's rows are dealt to the two channel tiles of a wave in
 // fours (channel 8 q + 4 c + v is row 4 q + v of tile c): 16-byte stores without a pass through LDS.
 // Tokens are read from L2 once per 256 channels (16 bytes a cycle and CU).
-// What bounds it: the products and their promotion, about as many cycles of the vector unit as of the matrix pipe, then the stores; results beyond
-// 128 MB, which are not written through, the stores (512 -> 32768 at 3001 tokens takes 62 us with the results of three calls in turn and 53 with
-// one call's, which the Infinity Cache holds).  A result costs a conversion and a sixteenth of a store: the loop is a kernel of its own for each output
+// What bounds it: the products and their promotion, about as many cycles of the vector unit as of the matrix pipe, then the stores (512 -> 32768 at 3001
+// tokens takes 55 us, packed exponents 62, where the results go to memory).  A result costs a conversion and a sixteenth of a store: the loop is a kernel of its own for each output
 // type, with and without a bias, written through or not, the stores are buffer stores whose range check drops what does not exist, and their
 // addresses advance in scalar registers.  With these choices and checks in the loop every half step ran through a dozen branches and 50 vector
 // instructions beside the promotion's 64, and the compiler moved products across the branches; us of the GPU, before / now, 3001 tokens 512 -> 32768 in a loop on
@@ -44,7 +43,8 @@ constexpr int RS_BN = RESIDENT_CHANNELS, RS_COMPUTE = 8, RS_LOAD = 2, RS_WEIGHT_
 constexpr int RS_THREADS = 64 * (RS_COMPUTE + RS_LOAD);
 
 // Tokens of a half step.  With a bias the unscaled kinds' epilogue takes twelve registers more, which would be spilled beside K = 512 and 32 tokens (a
-// reload waits for every store in flight): 32 random linears, half steps of 32 / of 16: per-token FP8 1.10 in a graph and 1.11 eager, INT8 1.01 and 1.01.  The
+// reload waits for every store in flight): 32 random linears, half steps of 32 / of 16: per-token FP8 1.10 in a graph and 1.11 eager, INT8 1.01 and 1.01.  (INT8
+// of K = 512 spills a register or two, block FP8 of K = 512 with a bias and results beyond 128 MB four, outside the loop.)  The
 // choice of ranges and the plan go by the steps without a bias, which take 1 to 3 % less time.
 template <Arith AR, int KB, bool BIAS>
 constexpr int rs_half_step() { return BIAS && KB == 4 && (AR == AR_UNIT || AR == AR_INT8) ? 16 : resident_half_step(AR == AR_UE8M0, KB); }
