@@ -20,8 +20,8 @@
 // addresses advance in scalar registers.  With these choices and checks in the loop every half step ran through a dozen branches and 50 vector
 // instructions beside the promotion's 64, and the compiler moved products across the branches; us of the GPU, before / now, 3001 tokens 512 -> 32768 in a loop on
 // one set of buffers: FP8 56.5 / 53, packed exponents 51 / 46, epilogue scales 58 / 50, INT8 63 / 51; 36 random linears 0.91.  One choice alone as a branch in the
-// loop: the bias 1.03 of the time of 80 random linears (packed exponents of K = 640 and 768 1.9 to 3.7, spilled); writing through 1.00, packed exponents
-// 1.015 (20 linears of 17 to 120 MB) and 1.02 (20 of more than 128 MB), whose products are sunk behind it.
+// loop, 80 random linears: the bias packed exponents 1.13 (of K = 640 and 768 1.9 to 3.7, spilled), the others, which have one scheme with them, 1.00; writing
+// through packed exponents 1.015 (20 of 17 to 120 MB) and 1.02 (20 of more than 128 MB), whose products are sunk behind it, the others 1.00.
 // Whole linears, us, two-phase tile / this:
 //   block FP8 3001 tokens 512 -> 32768 89.9 / 73.9, 2310 tokens 256 -> 32768 56.2 / 36.3, 1966 tokens 640 -> 16384 43.1 / 31.2;
 //   packed exponents 1609 tokens 512 -> 32768 63.6 / 36.6;  per token FP8 820 tokens 512 -> 32768 37.8 / 24.3;  INT8 952 tokens 640 -> 32768 38.6 / 29.1;
